@@ -58,6 +58,9 @@ struct KeyedScanCall {
   float* carry;
   int decay_span;         // form 0: 0 a step size per head and key channel, 1 one per head
   const float* dt_bias;   // form 0: null, or [heads * dim] ([heads] with decay_span 1): g holds raw sums, dt = softplus(g + dt_bias)
+  // null, or room for what blocks of 16 tokens leave: (tokens / 16 + n_seqs + 1) * heads * (16 (3 dim + vdim) + dim) floats,
+  // aligned to 16 bytes; with it long sequences go in blocks on the matrix units (max_count as above)
+  float* blocks;
 };
 
 // One wave per (4 value channels of a head, sequence): sixteen lanes share a channel, each owns R key channels
@@ -355,6 +358,392 @@ static void launch_keyed_scan(hipStream_t stream, const KeyedScanCall& c) {
     hipLaunchKernelGGL((keyed_scan_kernel<R, 1, 0>), grid, block, lds, stream, c, chunk, tiles);
 }
 
+// --- blocks of sixteen tokens on the matrix units ----------------------------------------------
+//
+// A token of the walk above costs 0.25 to 0.5 us (delta rule) however idle the chip is.  What a block of B = 16 tokens does to the
+// state can be written down before the state is known.  With a_t the product of the block's decays up to and with
+// token t (per key channel), b_s that of the decays behind token s, kd = a k, qd = a q, ku = b k:
+//     A[t][s] = beta_t sum_d k_t k_s g_(s+1) .. g_t   (s < t),   P[t][s] the same with q_t, without beta, and s <= t
+//     T = (I + A)^-1 diag(beta),  M = P T
+//     u = T v - (T kd) S0,   o = M v + (qd - M kd) S0,   S = diag(a_B) S0 + ku^T u
+// so W = T kd, R = qd - M kd, T v and M v are left by one kernel, all blocks side by side, and a second one walks
+// the blocks in order with the state in registers: two products with S0 and one into it a block, on
+// v_mfma_f32_16x16x4_f32 (32-bit multiply and add throughout).  Decays are only ever multiplied with each other, never
+// divided and never taken to logarithms, so a decay of nearly nothing is as exact as in the walk.  The forget gate
+// writes plain values: T v is v and W is not there.
+//
+// Operands lie in the workspace as the lanes of a wave want them (a lane's four values of a 16 x 16 tile side by side,
+// lanes one after the other).  Of an instruction's four K values step i takes number 4 g + i in lane group g = lane / 16:
+// the registers in which a product's result lands are then the B operand of the next one, and nothing moves between
+// lanes.  Measured, token by token / in blocks (us; 8 heads of 128 x 128, 2 x 1,024 tokens): delta rule with one decay
+// a head 386 / 78, one a key channel 522 / 82, forget gate (there in spans) 139 / 57; 2 x 128 tokens 52 / 24, 69 / 26,
+// 45 / 18.  The operands take 25 us (18 without T) of the long ones; the walk takes 0.87 us a block (0.63), of which the
+// matrix units are busy for 0.32 (0.21): a wave is alone on its SIMD, and the chain from S0 through LDS and back into S
+// is what is left.
+#define KB_TOKENS 16
+
+// Floats of one block and head: W, R and ku [tiles of 16 channels][64 lanes][4], T v [tiles of 16 values][64][4], a_B [dim].
+__host__ __device__ __forceinline__ int64_t kb_floats(int dim, int vdim) { return (int64_t)KB_TOKENS * (3 * dim + vdim) + dim; }
+
+// Where block `block` of sequence `seq` and a head keeps them: ranges of different sequences do not meet.
+__device__ __forceinline__ float* kb_place(const KeyedScanCall& c, int seq, int block, int head) {
+  return c.blocks + ((int64_t)(c.seq_off[seq] / KB_TOKENS + seq + block) * c.heads + head) * kb_floats(c.dim, c.vdim);
+}
+
+template <int FORM, int DT>
+__global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
+  constexpr int DIM = 16 * DT, PITCH = DIM + 4;
+  __shared__ __attribute__((aligned(16))) float K[KB_TOKENS][PITCH], Q[KB_TOKENS][PITCH], G[KB_TOKENS][PITCH];
+  __shared__ __attribute__((aligned(16))) float A[KB_TOKENS][KB_TOKENS], P[KB_TOKENS][KB_TOKENS], T[KB_TOKENS][20], M[KB_TOKENS][20];
+  __shared__ float strength[KB_TOKENS], one[KB_TOKENS];                  // beta, and a decay the whole head shares
+  const int seq = blockIdx.z, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int first = c.seq_off[seq] + (int)blockIdx.x * KB_TOKENS;
+  const int count = min(KB_TOKENS, c.seq_off[seq + 1] - first);
+  if (count <= 0) return;                                                // (the whole work-group)
+  const int shared = FORM == 0 ? head / (c.heads / c.kv_heads) : head;
+  float* place = kb_place(c, seq, blockIdx.x, head);
+  const float rate = FORM == 0 ? -expf(c.A_log[head]) : 0.f;
+  const bool per_head = FORM == 0 && c.decay_span == 1;
+  if (FORM == 0 && tid < KB_TOKENS) {
+    const int64_t t = first + min(tid, count - 1);
+    strength[tid] = tid < count ? 1.0f / (1.0f + expf(-c.beta[t * c.ld_beta + head])) : 0.f;
+    if (per_head) {
+      const float raw = c.g[t * c.ld_g + head];
+      one[tid] = expf(rate * (c.dt_bias ? softplus_f(raw + c.dt_bias[head]) : raw));
+    }
+  }
+  if (per_head) __syncthreads();
+  // rows behind the sequence's end decay by one and hold zeros: they change nothing
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    const int i = (tid + 256 * j) / DIM, d = (tid + 256 * j) % DIM;
+    const int64_t t = first + min(i, count - 1);
+    const float raw = per_head ? 0.f : c.g[t * c.ld_g + head * DIM + d];
+    float q = c.q[t * c.ld_q + shared * DIM + d], k, decay;
+    if (FORM == 0) {
+      k = c.k[t * c.ld_k + shared * DIM + d];
+      decay = per_head ? one[i] : expf(rate * (c.dt_bias ? softplus_f(raw + c.dt_bias[head * DIM + d]) : raw));
+    } else {
+      const float low = c.lower[head * DIM + d];
+      decay = low + (1.0f - low) / (1.0f + expf(-(raw + (c.g_bias ? c.g_bias[head * DIM + d] : 0.f))));
+      k = 1.0f - decay;
+      q = silu_f(q);
+    }
+    const bool there = i < count;
+    K[i][d] = there ? k : 0.f;
+    Q[i][d] = there ? q : 0.f;
+    G[i][d] = there ? decay : 1.f;
+  }
+  __syncthreads();
+  const int sub = tid & 15, s = tid >> 4;
+  if (FORM == 0 && c.unit) {                                             // sixteen lanes make a token's vectors unit vectors
+    float sk = 0.f, sq = 0.f;
+#pragma unroll
+    for (int r = 0; r < DT; ++r) {
+      sk = fmaf(K[s][sub + 16 * r], K[s][sub + 16 * r], sk);
+      sq = fmaf(Q[s][sub + 16 * r], Q[s][sub + 16 * r], sq);
+    }
+    sk = 1.0f / sqrtf(sum_of_16_lanes(sk) + c.unit_eps);
+    sq = c.q_scale / sqrtf(sum_of_16_lanes(sq) + c.unit_eps);
+#pragma unroll
+    for (int r = 0; r < DT; ++r) {
+      K[s][sub + 16 * r] *= sk;
+      Q[s][sub + 16 * r] *= sq;
+    }
+    __syncthreads();
+  }
+  // pairs: sixteen lanes carry token s's key through the decays behind it and meet every later key and query; a lane
+  // owns channels 4 sub .. 4 sub + 3 of every 64, so that a row is read 16 bytes at a time
+  {
+    constexpr int R = (DT + 3) / 4;
+    floatx4 w[R];
+    auto row = [&](const float* at, int r) {
+      const int d = 64 * r + 4 * sub;
+      return DT % 4 == 0 || d < DIM ? *reinterpret_cast<const floatx4*>(at + d) : floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = row(K[s], r);
+    const int begin = __builtin_amdgcn_readfirstlane(tid >> 6) * 4;      // the first s of the wave
+#pragma unroll 2
+    for (int t = begin; t < KB_TOKENS; ++t) {
+      floatx4 ak = {0.f, 0.f, 0.f, 0.f}, aq = ak;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const floatx4 g = row(G[t], r), q = row(Q[t], r);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          w[r][i] = t > s ? w[r][i] * g[i] : w[r][i];
+          aq[i] = fmaf(w[r][i], q[i], aq[i]);
+        }
+        if (FORM == 0) {
+          const floatx4 k = row(K[t], r);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ak[i] = fmaf(w[r][i], k[i], ak[i]);
+        }
+      }
+      const float pair_q = sum_of_16_lanes((aq[0] + aq[1]) + (aq[2] + aq[3]));
+      if (FORM == 0) {
+        const float pair_k = sum_of_16_lanes((ak[0] + ak[1]) + (ak[2] + ak[3]));
+        if (sub == 0) {
+          P[t][s] = t >= s ? pair_q : 0.f;
+          A[t][s] = t > s ? strength[t] * pair_k : 0.f;
+        }
+      } else if (sub == 0) {
+        M[t][s] = t >= s ? pair_q : 0.f;
+      }
+    }
+    if (FORM == 1 && sub == 0)
+      for (int t = 0; t < begin; ++t) M[t][s] = 0.f;
+  }
+  __syncthreads();
+  if (FORM == 0 && wave == 0) {                                          // T, a column a lane (four lanes share one), and M
+    float col[KB_TOKENS];
+#pragma unroll
+    for (int t = 0; t < KB_TOKENS; ++t) {
+      floatx4 v = {t == sub ? 1.f : 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < t; ++e) v[e & 3] = fmaf(-A[t][e], col[e], v[e & 3]);
+      col[t] = (v[0] + v[1]) + (v[2] + v[3]);
+    }
+#pragma unroll
+    for (int t = 0; t < KB_TOKENS; ++t) col[t] *= strength[sub];
+#pragma unroll
+    for (int t = 0; t < KB_TOKENS; ++t)
+      if ((lane >> 4) == (t & 3)) T[t][sub] = col[t];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {                                        // rows 4 i + g; behind the diagonal P is zero or col is
+      const int t = 4 * i + (lane >> 4);
+      float m = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4 * i + 4; ++e) m = fmaf(e <= t ? P[t][e] : 0.f, col[e], m);
+      M[t][sub] = m;
+    }
+  }
+  if (wave >= 2) {                                                       // k -> kd, q -> qd, decays -> ku, a channel a thread
+    const int d = tid - 128;
+    if (d < DIM) {
+      float k[KB_TOKENS], g[KB_TOKENS], run = 1.f;
+#pragma unroll
+      for (int t = 0; t < KB_TOKENS; ++t) {
+        k[t] = K[t][d];
+        g[t] = G[t][d];
+        run *= g[t];
+        K[t][d] = k[t] * run;
+        Q[t][d] *= run;
+      }
+      place[KB_TOKENS * (3 * DIM + c.vdim) + d] = run;
+      run = 1.f;
+#pragma unroll
+      for (int t = KB_TOKENS - 1; t >= 0; --t) {
+        G[t][d] = k[t] * run;
+        run *= g[t];
+      }
+    }
+  }
+  __syncthreads();
+  const int g = lane >> 4, n = lane & 15;
+  floatx4 tb, mb = *reinterpret_cast<const floatx4*>(&M[n][4 * g]);
+  if (FORM == 0) tb = *reinterpret_cast<const floatx4*>(&T[n][4 * g]);
+  floatx4* frag = reinterpret_cast<floatx4*>(place);
+  for (int tile = wave; tile < DT; tile += 4) {
+    const int d = 16 * tile + n;
+    floatx4 r = *reinterpret_cast<const floatx4*>(&Q[n][16 * tile + 4 * g]), u;
+    if (FORM == 0) {
+      floatx4 w = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float kd = K[4 * g + i][d];
+        w = __builtin_amdgcn_mfma_f32_16x16x4f32(kd, tb[i], w, 0, 0, 0);
+        r = __builtin_amdgcn_mfma_f32_16x16x4f32(kd, -mb[i], r, 0, 0, 0);
+      }
+      frag[64 * tile + lane] = w;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = G[4 * g + i][d];
+    frag[64 * (DT + tile) + lane] = r;
+    frag[64 * (2 * DT + tile) + lane] = u;
+  }
+  const float* v_rows = c.v + (int64_t)first * c.ld_v + head * c.vdim;
+  float* out = c.out + (int64_t)first * c.ld_out + head * c.vdim;
+  for (int tile = wave; 16 * tile < c.vdim; tile += 4) {
+    floatx4 v, u = {0.f, 0.f, 0.f, 0.f}, o = u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float value = v_rows[(int64_t)min(4 * g + i, count - 1) * c.ld_v + 16 * tile + n];
+      v[i] = 4 * g + i < count ? value : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (FORM == 0) u = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[i], v[i], u, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_16x16x4f32(mb[i], v[i], o, 0, 0, 0);
+    }
+    frag[64 * (3 * DT + tile) + lane] = FORM == 0 ? u : v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * g + i < count) out[(int64_t)(4 * g + i) * c.ld_out + 16 * tile + n] = o[i];
+  }
+}
+
+// One work-group per 16 value channels of a head and sequence: four waves share the key channels (TW tiles of 16 each),
+// every wave's part of W S0 and R S0 meets in LDS.  The operands of the next KB_AHEAD - 1 blocks are on their way.
+#define KB_AHEAD 4
+
+// A barrier that waits for this wave's LDS traffic only: operands asked for blocks ahead stay on their way.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);                      // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int FORM, int TW>
+struct KbStage {
+  floatx4 w[FORM == 0 ? TW : 1], r[TW], ku[TW], a[TW], u;
+  float o;
+};
+
+template <int FORM, int DT>
+__global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall c) {
+  constexpr int TW = (DT + 3) / 4, DIM = 16 * DT;
+  __shared__ __attribute__((aligned(16))) floatx4 parts[2][2][4][64];   // [turn][W S0, R S0][wave][lane]
+  // the columns of a head and sequence read the same operands: they are numbered onto one XCD (work-groups are dealt to
+  // eight of them in turn), which reads them from memory once
+  const int columns = c.vdim / 16, pair = blockIdx.x / (8 * columns) * 8 + blockIdx.x % 8;
+  if (pair >= c.heads * c.n_seqs) return;
+  const int column = blockIdx.x / 8 % columns, head = pair % c.heads, seq = pair / c.heads;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
+  const int first = c.seq_off[seq], count = c.seq_off[seq + 1] - first;
+  if (count <= 0) return;
+  const int blocks = (count + KB_TOKENS - 1) / KB_TOKENS;
+  const int64_t stride = (int64_t)c.heads * kb_floats(DIM, c.vdim);
+  const float* place = kb_place(c, seq, 0, head);
+  const int vtiles = (c.vdim + 3) / 4, p = 16 * column + n;
+  float* slot = c.S + (int64_t)c.slots[seq] * c.state_stride + ((int64_t)head * vtiles + p / 4) * DIM * 4 + p % 4;
+  // tiles of key channels are dealt in turn; a wave has all its TW tiles unless DT is no multiple of four
+  auto mine = [&](int j) { return DT % 4 == 0 || wave * TW + j < DT; };
+  floatx4 S[TW];
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[j][i] = mine(j) ? slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] : 0.f;
+  KbStage<FORM, TW> stages[KB_AHEAD];
+  // a block's operands: one address that all lanes share, and every lane's distances from it
+  uint32_t from_tile[TW], from_decay[TW];
+#pragma unroll
+  for (int j = 0; j < TW; ++j) {
+    const int tile = min(wave * TW + j, DT - 1);
+    from_tile[j] = (256 * tile + 4 * lane) * 4;
+    from_decay[j] = (KB_TOKENS * (3 * DIM + c.vdim) + 16 * tile + 4 * g) * 4;
+  }
+  const uint32_t from_u = (KB_TOKENS * 3 * DIM + 256 * column + 4 * lane) * 4;
+  const char* at = reinterpret_cast<const char*>(place);
+  int row = 4 * g + wave, ahead = row, fetched = 0;        // a wave finishes every fourth token's read-out
+  float* out = c.out + (first + (int64_t)min(row, count - 1)) * c.ld_out + head * c.vdim + p;
+  const float* out_ahead = out;
+  const int64_t out_step = KB_TOKENS * c.ld_out;
+  auto load4 = [&](uint32_t from) { return *reinterpret_cast<const floatx4*>(at + from); };
+  auto fetch = [&](KbStage<FORM, TW>& st) {
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      if (FORM == 0) st.w[j] = load4(from_tile[j]);
+      st.r[j] = load4(from_tile[j] + KB_TOKENS * DIM * 4);
+      st.ku[j] = load4(from_tile[j] + 2 * KB_TOKENS * DIM * 4);
+      st.a[j] = load4(from_decay[j]);
+    }
+    st.u = load4(from_u);
+    st.o = *out_ahead;
+    // on to the next block; at the end the last one's operands are asked for again and not used
+    at += ++fetched < blocks ? stride * 4 : 0;
+    ahead += KB_TOKENS;
+    out_ahead += ahead < count ? out_step : 0;
+  };
+  auto walk = [&](KbStage<FORM, TW>& st, int turn) {
+    floatx4 ws = {0.f, 0.f, 0.f, 0.f}, rs = ws;
+    if (FORM == 0) {
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        if (mine(j))
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ws = __builtin_amdgcn_mfma_f32_16x16x4f32(st.w[j][i], S[j][i], ws, 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+      if (mine(j))
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rs = __builtin_amdgcn_mfma_f32_16x16x4f32(st.r[j][i], S[j][i], rs, 0, 0, 0);
+    if (FORM == 0) parts[turn][0][wave][lane] = ws;
+    parts[turn][1][wave][lane] = rs;
+#pragma unroll
+    for (int j = 0; j < TW; ++j) S[j] *= st.a[j];
+    lds_barrier();
+    floatx4 u = st.u;
+    if (FORM == 0)
+      u -= (parts[turn][0][0][lane] + parts[turn][0][1][lane]) + (parts[turn][0][2][lane] + parts[turn][0][3][lane]);
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+      if (mine(j))
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.ku[j][i], u[i], S[j], 0, 0, 0);
+    const float* r = reinterpret_cast<const float*>(&parts[turn][1][0][lane]) + wave;
+    const float o = st.o + ((r[0] + r[256]) + (r[512] + r[768]));
+    if (row < count) *out = o;
+    row += KB_TOKENS;
+    out += out_step;
+  };
+#pragma unroll
+  for (int i = 0; i < KB_AHEAD - 1; ++i) {
+    fetch(stages[i]);
+    __builtin_amdgcn_sched_barrier(0);                     // (in order: a stage is waited for by the loads behind it)
+  }
+  for (int block = 0; block < blocks; block += KB_AHEAD) {
+#pragma unroll
+    for (int i = 0; i < KB_AHEAD; ++i) {
+      if (block + i >= blocks) break;                      // (the same for all four waves)
+      fetch(stages[(i + KB_AHEAD - 1) % KB_AHEAD]);
+      walk(stages[i], i & 1);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+    if (mine(j))
+#pragma unroll
+      for (int i = 0; i < 4; ++i) slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] = S[j][i];
+}
+
+// Steps whose longest sequence brings at least this many tokens go in blocks.  Below, two launches cost what walking
+// does (us, token by token / in blocks; one decay a head, one a key channel, forget gate): 2 x 32 tokens 16.0 / 17.2,
+// 19.9 / 19.5, 13.8 / 13.0; 16 x 40 tokens 42.8 / 37.0, 56.3 / 39.3, 32.8 / 28.4; 4 x 48 tokens 22.9 / 19.6, 29.2 / 22.1, 20.0 / 15.0.
+#define KB_MIN_TOKENS 40
+
+template <int DT>
+static void launch_keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
+  dim3 side((c.max_count + KB_TOKENS - 1) / KB_TOKENS, c.heads, c.n_seqs), block(256);
+  dim3 walk((unsigned)((c.heads * c.n_seqs + 7) / 8 * 8 * (c.vdim / 16)));
+  if (c.form == 0) {
+    hipLaunchKernelGGL((keyed_blocks_kernel<0, DT>), side, block, 0, stream, c);
+    hipLaunchKernelGGL((keyed_blocks_walk_kernel<0, DT>), walk, block, 0, stream, c);
+  } else {
+    hipLaunchKernelGGL((keyed_blocks_kernel<1, DT>), side, block, 0, stream, c);
+    hipLaunchKernelGGL((keyed_blocks_walk_kernel<1, DT>), walk, block, 0, stream, c);
+  }
+}
+
+// True if the call went in blocks: it brings the room, tiles of 16 and enough tokens.
+static bool keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
+  if (!c.blocks || c.max_count < KB_MIN_TOKENS || c.dim % 16 != 0 || c.dim > 128 || c.vdim % 16 != 0) return false;
+  switch (c.dim / 16) {
+    case 1: launch_keyed_blocks<1>(stream, c); break;
+    case 2: launch_keyed_blocks<2>(stream, c); break;
+    case 3: launch_keyed_blocks<3>(stream, c); break;
+    case 4: launch_keyed_blocks<4>(stream, c); break;
+    case 5: launch_keyed_blocks<5>(stream, c); break;
+    case 6: launch_keyed_blocks<6>(stream, c); break;
+    case 7: launch_keyed_blocks<7>(stream, c); break;
+    default: launch_keyed_blocks<8>(stream, c); break;
+  }
+  return true;
+}
+
 BT_EXPORT int bt_keyed_scan_call(void* stream, const KeyedScanCall* c) {
   if (c->tokens <= 0 || c->n_seqs <= 0) return BT_OK;
   if (c->heads <= 0 || c->dim <= 0 || c->dim > 256 || c->vdim <= 0)
@@ -376,7 +765,9 @@ BT_EXPORT int bt_keyed_scan_call(void* stream, const KeyedScanCall* c) {
     BT_REFUSE("keyed_scan: a slot's state of %lld elements does not hold %d heads of %d x %d", (long long)c->state_stride,
               c->heads, c->dim, c->vdim);
   if (c->heads > 65535 || c->n_seqs > 65535) BT_REFUSE("keyed_scan: %d heads of %d sequences are too many", c->heads, c->n_seqs);
+  if ((uintptr_t)c->blocks % 16 != 0) BT_REFUSE("keyed_scan: the room for blocks is not aligned to 16 bytes");
   hipStream_t s = (hipStream_t)stream;
+  if (keyed_blocks(s, *c)) return bt_check_launch("keyed_scan");
   const int per = (c->dim + 15) / 16;
   if (per <= 1) launch_keyed_scan<1>(s, *c);
   else if (per <= 2) launch_keyed_scan<2>(s, *c);

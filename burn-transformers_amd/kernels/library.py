@@ -243,7 +243,7 @@ class KeyedScanCall(ctypes.Structure):
                 ("g", _c_ptr), ("ld_g", _c_i64), ("beta", _c_ptr), ("ld_beta", _c_i64), ("A_log", _c_ptr),
                 ("g_bias", _c_ptr), ("lower", _c_ptr), ("out", _c_ptr), ("ld_out", _c_i64), ("S", _c_ptr),
                 ("state_stride", _c_i64), ("seq_off", _c_ptr), ("slots", _c_ptr), ("span", _c_int), ("max_count", _c_int),
-                ("carry", _c_ptr), ("decay_span", _c_int), ("dt_bias", _c_ptr)]
+                ("carry", _c_ptr), ("decay_span", _c_int), ("dt_bias", _c_ptr), ("blocks", _c_ptr)]
     _step_fields_ = {"tokens": "tokens", "max_count": "max_count"}
 
 
@@ -1470,8 +1470,20 @@ def soft_cap(logits, cap):
 
 # --- linear attention with a matrix state -------------------------------------------------------
 
+SCAN_BLOCK = 16       # tokens of a block of the keyed scan (csrc/linear_attention.hip)
+
+
+def scan_blocks(step, heads, dim, vdim):
+    """Room for what the blocks of a step's long sequences leave to the kernel that walks them, for a step of any shape
+    of its class; None for steps that never go in blocks."""
+    if step.max_count <= 1 or step.token_capacity < 2 * SCAN_BLOCK or dim % 16 or dim > 128 or vdim % 16:
+        return None
+    blocks = step.token_capacity // SCAN_BLOCK + step.n_seqs + 1
+    return step.buffer("scan.blocks", blocks, heads * (SCAN_BLOCK * (3 * dim + vdim) + dim), "float32")
+
+
 def keyed_scan(q, k, v, g, out, state, step, heads, kv_heads, dim, vdim, form, beta=None, A_log=None, g_bias=None,
-               lower=None, unit=False, unit_eps=1e-6, q_scale=1.0, carry=None, decay_per_head=False, dt_bias=None):
+               lower=None, unit=False, unit_eps=1e-6, q_scale=1.0, carry=None, decay_per_head=False, dt_bias=None, blocks=None):
     """Per head S <- diag(decay) S; S <- S + key u^T; out = S^T query, token after token (csrc/linear_attention.hip).
     ``form`` "delta": u = sigmoid(beta) (v - S^T key), decay = exp(-exp(A_log) g) from step sizes ``g``, ``q`` and
     ``k`` rows of ``kv_heads`` heads (made unit vectors per head with ``unit``, q times ``q_scale``).  ``form``
@@ -1480,7 +1492,8 @@ def keyed_scan(q, k, v, g, out, state, step, heads, kv_heads, dim, vdim, form, b
     ``scan_carry`` (a slot's state floats, heads * dim extra); with it the "forget" form scans long sequences in
     spans side by side.  ``decay_per_head`` ("delta"): ``g`` has one step size per head, for all its key channels;
     ``dt_bias`` ("delta"; [heads * dim], or [heads] per head): ``g`` holds raw sums and the step size is
-    softplus(g + dt_bias)."""
+    softplus(g + dt_bias).  ``blocks``: room from ``scan_blocks``; with it long sequences go in blocks of tokens on the
+    matrix units."""
     _launch(_module("linear_attention"), "bt_keyed_scan_call",
             KeyedScanCall(tokens=v.shape[0], n_seqs=step.n_seqs, heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim,
                           form={"delta": 0, "forget": 1}[form], unit=1 if unit else 0, unit_eps=unit_eps, q_scale=q_scale,
@@ -1490,7 +1503,7 @@ def keyed_scan(q, k, v, g, out, state, step, heads, kv_heads, dim, vdim, form, b
                           lower=_ptr(lower), out=out.data_ptr(), ld_out=out.stride(0), S=state.data_ptr(),
                           state_stride=state.stride(0), seq_off=step.seq_off.data_ptr(), slots=step.slots.data_ptr(),
                           span=SCAN_SPAN if carry is not None else 0, max_count=step.max_count, carry=_ptr(carry),
-                          decay_span=1 if decay_per_head else 0, dt_bias=_ptr(dt_bias)))
+                          decay_span=1 if decay_per_head else 0, dt_bias=_ptr(dt_bias), blocks=_ptr(blocks)))
 
 
 def head_norm_gate(y, weight, heads, vdim, eps, out, gate=None, mult=1.0, gate_act="sigmoid"):

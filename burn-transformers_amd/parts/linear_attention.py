@@ -147,7 +147,8 @@ class GatedDeltaRule(_MatrixState):
         y = step.buffer("delta.y", tokens, self.inner, "float32")
         K.keyed_scan(qkv[:, :qk], qkv[:, qk:2 * qk], qkv[:, 2 * qk:], dt, y, scan_state, step, self.heads, self.kv_heads,
                      self.dim, self.vdim, "delta", beta=fused[:, self.at_beta:self.at_beta + self.heads], A_log=self.A_log,
-                     unit=True, unit_eps=self.unit_eps, q_scale=self.dim ** -0.5, decay_per_head=self.per_head, dt_bias=raw)
+                     unit=True, unit_eps=self.unit_eps, q_scale=self.dim ** -0.5, decay_per_head=self.per_head, dt_bias=raw,
+                     blocks=K.scan_blocks(step, self.heads, self.dim, self.vdim))
         gated = step.buffer("delta.gated", tokens, self.inner_cols, step.dtype)
         K.head_norm_gate(y, self.norm_weight, self.heads, self.vdim, self.eps, gated, gate=gate, gate_act=self.gate_act)
         stream.add_product(step, gated, self.out_weight, packed=self.out_packed)
@@ -173,7 +174,8 @@ class ForgetGateAttention(_MatrixState):
         y = step.buffer("forget.y", tokens, self.inner, "float32")
         K.keyed_scan(fused[:, :qk], None, fused[:, 2 * qk:], fused[:, qk:2 * qk], y, memory.state(), step, self.heads,
                      self.heads, self.dim, self.vdim, "forget", g_bias=self.f_bias, lower=self.lower,
-                     carry=K.scan_carry(step, self.scan_state, self.heads * self.dim))
+                     carry=K.scan_carry(step, self.scan_state, self.heads * self.dim),
+                     blocks=K.scan_blocks(step, self.heads, self.dim, self.vdim))
         normed = step.buffer("forget.normed", tokens, self.inner_cols, step.dtype)
         K.head_norm_gate(y, self.norm_weight, self.heads, self.vdim, self.eps, normed)
         stream.add_product(step, normed, self.out_weight, packed=self.out_packed)

@@ -1,0 +1,98 @@
+"""The keyed scan in blocks of sixteen tokens on the matrix units, against the recurrence token by token in 64 bits."""
+
+import pytest
+import torch
+
+from burn_transformers_amd.kernels import library as K
+
+from step_helpers import make_step
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rel_err(got, want):
+    return float((got.double() - want).abs().max() / want.abs().max())
+
+
+def recurrence(S, q, k, v, decay, beta):
+    """S [H, D, V]; rows [T, H, ...] in 64 bits: (read-outs [T, H, V], the state behind them)."""
+    out = []
+    for t in range(q.shape[0]):
+        S = decay[t][..., None] * S
+        u = v[t] if beta is None else beta[t][:, None] * (v[t] - (S * k[t][..., None]).sum(1))
+        S = S + k[t][..., None] * u[:, None]
+        out.append((S * q[t][..., None]).sum(1))
+    return torch.stack(out), S
+
+
+def state_rows(state, heads, dim, vdim):
+    """A slot's floats as [heads, dim, vdim]."""
+    return state[:, :heads * dim * vdim].view(-1, heads, vdim // 4, dim, 4).permute(0, 1, 3, 2, 4).reshape(-1, heads, dim, vdim)
+
+
+# lengths around a block's edges beside the shortest and sequences of one token; a second portion starts from a state
+# that is not zero; `strong`: decays down to nothing (products that underflow) beside decays of nearly one
+@pytest.mark.parametrize("form,heads,kv_heads,dim,vdim,lengths,strong", [
+    ("head", 4, 2, 128, 128, [33, 1, 16, 47], False), ("head", 2, 2, 16, 16, [100, 32, 5], True),
+    ("channel", 2, 1, 128, 32, [64, 17, 31], False), ("channel", 3, 3, 80, 48, [49, 2], True),
+    ("forget", 2, 2, 128, 128, [130, 15, 1], False), ("forget", 3, 3, 48, 80, [35, 64], True),
+    ("channel", 1, 1, 64, 16, [400], False), ("forget", 1, 1, 32, 64, [333], True)])
+def test_blocks_of_tokens(form, heads, kv_heads, dim, vdim, lengths, strong):
+    gen = torch.Generator().manual_seed(heads * 1000 + dim + len(lengths))
+    qk, inner = kv_heads * dim, heads * vdim
+    decays = heads if form == "head" else heads * dim
+    columns = 2 * qk + inner + decays + heads + 3                       # an odd pitch: rows are not aligned
+    portions = [lengths, [n % 40 + 32 for n in lengths]]
+    A_log, bias = torch.log(torch.rand(heads, generator=gen) * 3.0 + 0.5), torch.randn(decays, generator=gen)
+    lower = torch.rand(decays, generator=gen) * (0.0 if strong else 0.9)
+    slots = list(reversed(range(len(lengths))))
+    state = torch.zeros(len(lengths), heads * dim * vdim + 7, device=DEV)
+    walked = state.clone()
+    want_state = [torch.zeros(heads, dim, vdim, dtype=torch.float64) for _ in lengths]
+    spread = lambda x: x.repeat_interleave(heads // kv_heads, 1)
+    errors = {"blocks": [], "walk": []}
+    for part, counts in enumerate(portions):
+        rows = torch.randn(sum(counts), columns, generator=gen)
+        if strong:
+            rows[:, 2 * qk + inner:2 * qk + inner + decays] *= 20.0
+        r = rows.double()
+        q, k = r[:, :qk].view(-1, kv_heads, dim), r[:, qk:2 * qk].view(-1, kv_heads, dim)
+        v, raw = r[:, 2 * qk:2 * qk + inner].view(-1, heads, vdim), r[:, 2 * qk + inner:2 * qk + inner + decays]
+        beta = None
+        if form == "forget":
+            decay = (lower.double() + (1.0 - lower.double()) * torch.sigmoid(raw + bias.double())).view(-1, heads, dim)
+            q, k = (q * torch.sigmoid(q)), 1.0 - decay
+        else:
+            unit = lambda x: spread(x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6))
+            q, k, beta = unit(q) * dim ** -0.5, unit(k), torch.sigmoid(r[:, -3 - heads:-3])
+            dt = torch.nn.functional.softplus(raw + bias.double(), threshold=50.0).view(-1, heads, decays // heads)
+            decay = torch.exp(-torch.exp(A_log.double())[:, None] * dt).expand(-1, heads, dim)
+        step = make_step(torch.float32, counts, starts=[0 if part == 0 else n for n in lengths], slots=slots)
+        on = rows.to(DEV)
+        run = dict(blocks=(state, K.scan_blocks(step, heads, dim, vdim)), walk=(walked, None))
+        assert run["blocks"][1] is not None
+        want, at = [], 0
+        for s, n in enumerate(counts):
+            here = slice(at, at + n)
+            o, want_state[s] = recurrence(want_state[s], q[here], k[here], v[here], decay[here], None if beta is None else beta[here])
+            want.append(o.reshape(n, inner))
+            at += n
+        want = torch.cat(want)
+        for name, (held, room) in run.items():
+            y = torch.full((sum(counts), inner + 2), float("nan"), device=DEV)
+            if room is not None:
+                room.fill_(float("nan"))
+            extra = dict(g_bias=bias.to(DEV), lower=lower.to(DEV)) if form == "forget" else \
+                dict(beta=on[:, -3 - heads:-3], A_log=A_log.to(DEV), unit=True, unit_eps=1e-6, q_scale=dim ** -0.5,
+                     decay_per_head=form == "head", dt_bias=bias.to(DEV))
+            K.keyed_scan(on[:, :qk], None if form == "forget" else on[:, qk:2 * qk], on[:, 2 * qk:2 * qk + inner],
+                         on[:, 2 * qk + inner:2 * qk + inner + decays], y, held, step, heads, kv_heads, dim, vdim,
+                         "forget" if form == "forget" else "delta", blocks=room, **extra)
+            assert bool(torch.isnan(y[:, inner:]).all())
+            errors[name].append(rel_err(y[:, :inner].cpu(), want))
+            got = state_rows(held, heads, dim, vdim).cpu()
+            errors[name].append(max(rel_err(got[slot], w) for slot, w in zip(slots, want_state)))
+    # a sum of 128 products of 32-bit values and a few hundred decays multiplied one after the other: some 1e-6
+    assert max(errors["blocks"]) < 5e-6, errors
+    assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
