@@ -510,10 +510,11 @@ __device__ __forceinline__ void wait_for_all_but(int newer) {
   }
 }
 
-template <int BM, int BN, int STAGES>
+template <typename T, int BM, int BN, int STAGES>
 __global__ void __launch_bounds__(256)
-gemm_tile_deep_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int N,
+gemm_tile_deep_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
                       int K, Epilogue epi, int tiles_m, int tiles_n) {
+  constexpr int ELEMS = Mma<T>::ELEMS, ROW_K = 8 * ELEMS;       // K values in 16 bytes and in a stage's row
   constexpr int ROWS = BM + BN;                   // rows of a stage
   constexpr int STAGE_BYTES = ROWS * TILE_ROW_BYTES;
   constexpr int LOADS = ROWS / 32;                // global_load_lds instructions per wave and tile (8 rows each)
@@ -527,13 +528,13 @@ gemm_tile_deep_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* _
   const int tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
   const int m_base = (tile % tiles_m) * BM, n_base = (tile / tiles_m) * BN;
   const int split = blockIdx.z, splits = gridDim.z;
-  const int k_tiles = K / TILE_K;
+  const int k_tiles = K / ROW_K;
   const int kt_begin = (int)((int64_t)k_tiles * split / splits);
   const int count = (int)((int64_t)k_tiles * (split + 1) / splits) - kt_begin;
 
   // load j of wave w fills stage rows 8 (LOADS w + j) .. + 7: A's rows below BM, W's from there on
-  const unsigned char* a_bytes = reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * (TILE_K * 2);
-  const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * (TILE_K * 2);
+  const unsigned char* a_bytes = reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * TILE_ROW_BYTES;
+  const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * TILE_ROW_BYTES;
   unsigned off[LOADS];
   bool from_w[LOADS];
 #pragma unroll
@@ -545,7 +546,7 @@ gemm_tile_deep_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* _
     int row = from_w[j] ? n_base + stage_row - BM : m_base + stage_row;
     int limit = from_w[j] ? N : M;
     row = row < limit ? row : limit - 1;
-    off[j] = (unsigned)(((int64_t)row * (from_w[j] ? (int64_t)K : lda) + chunk * 8) * 2);
+    off[j] = (unsigned)(((int64_t)row * (from_w[j] ? (int64_t)K : lda) + chunk * ELEMS) * sizeof(T));
   }
   auto issue = [&](int stage) {   // the tile a_bytes / w_bytes point at, into `stage`; then advance
 #pragma unroll
@@ -554,8 +555,8 @@ gemm_tile_deep_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* _
           (const __attribute__((address_space(1))) void*)((from_w[j] ? w_bytes : a_bytes) + off[j]),
           (__attribute__((address_space(3))) void*)(lds + stage * STAGE_BYTES + 8 * (LOADS * wave + j) * TILE_ROW_BYTES),
           16, 0, 0);
-    a_bytes += TILE_K * 2;
-    w_bytes += TILE_K * 2;
+    a_bytes += TILE_ROW_BYTES;
+    w_bytes += TILE_ROW_BYTES;
   };
   int w_rd[4], a_rd[4];
 #pragma unroll
@@ -582,21 +583,20 @@ gemm_tile_deep_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* _
     asm volatile("" ::: "memory");
     if (i + STAGES - 1 < count) issue(next_stage);
     const unsigned char* base = lds + stage * STAGE_BYTES;
-    bf16x8 wop[4][TN], aop[4][TM];
+    int4v wop[4][TN], aop[4][TM];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
-      for (int b = 0; b < TN; ++b) wop[kk][b] = *reinterpret_cast<const bf16x8*>(base + w_rd[kk] + b * 4096);
+      for (int b = 0; b < TN; ++b) wop[kk][b] = *reinterpret_cast<const int4v*>(base + w_rd[kk] + b * 4096);
 #pragma unroll
-      for (int b = 0; b < TM; ++b) aop[kk][b] = *reinterpret_cast<const bf16x8*>(base + a_rd[kk] + b * 4096);
+      for (int b = 0; b < TM; ++b) aop[kk][b] = *reinterpret_cast<const int4v*>(base + a_rd[kk] + b * 4096);
     }
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
       for (int bn = 0; bn < TN; ++bn)
 #pragma unroll
-        for (int bm = 0; bm < TM; ++bm)
-          acc[bn][bm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wop[kk][bn], aop[kk][bm], acc[bn][bm], 0, 0, 0);
+        for (int bm = 0; bm < TM; ++bm) Mma<T>::block32(acc[bn][bm], wop[kk][bn], aop[kk][bm]);
     stage = stage + 1 == STAGES ? 0 : stage + 1;
     next_stage = next_stage + 1 == STAGES ? 0 : next_stage + 1;
   }
@@ -611,7 +611,7 @@ gemm_tile_deep_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* _
       for (int q = 0; q < 4; ++q) {
         float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
         int n0 = n_base + wn * (BN / 2) + bn * 32 + q * 8 + g * 4;
-        if (m < M) epilogue4<bf16_t>(epi, N, m, n0, v, split);
+        if (m < M) epilogue4<T>(epi, N, m, n0, v, split);
       }
     }
   }
@@ -879,10 +879,10 @@ static void launch_tile(hipStream_t stream, const T* A, int64_t lda, const T* W,
                      K, epi, tiles_m, tiles_n);
 }
 
-template <int BM, int BN, int STAGES>
-static int launch_deep_form(hipStream_t s, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K,
+template <int BM, int BN, int STAGES, typename T>
+static int launch_deep_form(hipStream_t s, const T* a, int64_t lda, const T* w, int M, int N, int K,
                             const Epilogue& epi, int splits) {
-  auto kernel = gemm_tile_deep_kernel<BM, BN, STAGES>;
+  auto kernel = gemm_tile_deep_kernel<T, BM, BN, STAGES>;
   const size_t lds = (size_t)STAGES * (BM + BN) * TILE_ROW_BYTES;
   static bool raised = false;
   if (!raised) {
@@ -896,7 +896,8 @@ static int launch_deep_form(hipStream_t s, const bf16_t* a, int64_t lda, const b
 }
 
 // variants 4 .. 7: the deep forms (64 x 64 with 8 or 4 stages, 128 x 64 with 6 or 3)
-static int launch_deep(hipStream_t s, int variant, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K,
+template <typename T>
+static int launch_deep(hipStream_t s, int variant, const T* a, int64_t lda, const T* w, int M, int N, int K,
                        const Epilogue& epi, int splits) {
   switch (variant) {
     case 4: return launch_deep_form<64, 64, 8>(s, a, lda, w, M, N, K, epi, splits);
@@ -911,7 +912,14 @@ static int launch_deep(hipStream_t s, int variant, const bf16_t* a, int64_t lda,
 // variant: 0 = the fastest form the operands allow; 1 = template, 2 = lean, 3 = direct to LDS,
 // 4 .. 7 = direct to LDS with smaller tiles and more stages (asked for by tests, by measurements
 // and, for steps of some tens to some hundreds of rows, by the caller; a form that cannot take
-// the operands is refused; float has the template only)
+// the operands is refused; float has the template and the forms 4 .. 7).
+// Float products take the deep forms wherever K is a multiple of 32: the template's tile of 128 x 128 takes a compute unit
+// 2.4 us for 32 values of K (0.44 GFLOP/us of the 0.61 its matrix units have) and leaves most units idle where there
+// are few tiles; 64 x 64 in four stages takes 0.65, 128 x 64 in three 1.2 (1.85 times as long for twice the work), two
+// work-groups to a unit.  A unit's share comes in whole tiles, so the busiest unit decides: 64 x 64 unless 1.85 times the
+// rounds of the taller tiles are fewer.  Measured (us, template / 64 x 64 / 128 x 64): 65 x 768 x 3072 230 / 63 / 114;
+// 400 x 3072 x 768 63 / 33 / 34; 800 x 4096 x 1024 88 / 81 / 75; 2298 x 768 x 3072 226 / 115 / 117; 2298 x 2304 x 768 113 / 92 / 86;
+// 2298 x 1600 x 6400 468 / 460 / 427; 4096 x 3072 x 768 170 / 178 / 170; 4096 x 1600 x 6400 876 / 793 / 847.
 BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, const void* W, int M, int N, int K,
                            const Epilogue* epi, int splits, int variant) {
   if (M <= 0) return BT_OK;
@@ -922,7 +930,15 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == 0) {
-    if (variant > 1) BT_REFUSE("gemm_tile: float products have the general form only, not variant %d", variant);
+    const float *a = (const float*)A, *w = (const float*)W;
+    const bool deep_ok = K % (TILE_ROW_BYTES / 4) == 0 && (int64_t)M * lda * 4 < ((int64_t)1 << 32) && (int64_t)N * K * 4 < ((int64_t)1 << 32);
+    if (variant == 2 || variant == 3) BT_REFUSE("gemm_tile: float products have the general form only, not variant %d", variant);
+    if (variant >= 4 && !deep_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 32 and operands below 4 GiB", K);
+    if (variant == 0 && deep_ok) {
+      const int64_t small = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits, tall = (int64_t)((M + 127) / 128) * ((N + 63) / 64) * splits;
+      variant = 20 * ((small + 255) / 256) <= 37 * ((tall + 255) / 256) ? 5 : 7;
+    }
+    if (variant >= 4) return launch_deep(s, variant, a, lda, w, M, N, K, *epi, splits);
     launch_tile<float, 128, 128, 2, 2, 1>(s, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits);
     return bt_check_launch("gemm_tile");
   }

@@ -948,6 +948,23 @@ def deep_split_count(rows, columns, k, units=256):
     return max(1, min(4, splits, (k // 64) // 4))
 
 
+def float_split_count(rows, columns, k, units=256):
+    """The same for float32 products of more than 64 rows, whose tiles of 64 x 64 (1) or 128 x 64 (1.85) take a
+    compute unit 0.65 us for 32 values of K: as many slices, at most four, each at least four tiles of K long, as leave the
+    busiest unit the least to do, the slices the norm reads in addition counted at 4.5 TB/s; none for a gain below a
+    tenth.  Measured (us, slices 1 / 2 / 4): 65 x 768 x 3072 63 / 34 / 19; 400 x 768 x 3072 64 / 35 / 34; 800 x 768 x 3072 63 /
+    60 / 48; 1200 x 768 x 3072 65 / 62 / 62; 65 x 768 x 768 18.9 / 11.5 / 7.8."""
+    if rows <= 64 or k % 32:
+        return 1
+
+    def cost(splits):
+        tiles = lambda m: (rows + m - 1) // m * ((columns + 63) // 64) * splits
+        rounds = min((tiles(64) + units - 1) // units, 1.85 * ((tiles(128) + units - 1) // units))
+        return rounds / splits * (k // 32) * 0.65 + (splits - 1) * rows * columns * 8 / 4.5e6
+    best = min((s for s in range(1, 5) if s == 1 or (k // 32) // s >= 4), key=cost)
+    return best if cost(best) < 0.9 * cost(1) else 1
+
+
 def prompt_products_in_library(m, n, k, lda, scatters=False):
     """Whether a bfloat16 product of a step of ``m`` rows goes to the vendor's library (which cannot
     scatter keys and values into the cache: the caller then copies them)."""
