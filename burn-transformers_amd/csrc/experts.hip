@@ -20,6 +20,7 @@
 //   * weighed experts, for small steps: the router's logits come from the product that makes the experts' units (rows of
 //     the same matrix, 32-bit results), and ONE kernel makes the choice and multiplies the units by their weights.
 #include "host.h"
+#include "tile.h"
 
 #define ROUTE_THREADS 1024
 #define ROUTE_MAX_EXPERTS 1024
@@ -386,6 +387,370 @@ BT_EXPORT int bt_gated_experts_call(void* stream, const GatedExpertsCall* c) {
   else
     hipLaunchKernelGGL(gated_experts_kernel<bf16_t>, grid, block, 0, (hipStream_t)stream, *c);
   return bt_check_launch("gated_experts");
+}
+
+// --- experts by rows -----------------------------------------------------------------------------
+//
+// In a step of many tokens every expert would multiply every token, though a token uses `top` of them.  Here the tokens
+// that chose an expert are listed (group_experts), one kernel makes the units of the listed rows only, the rows gathered
+// by the loads that bring them into LDS and the activation and the token's weight applied to the sums while they are in
+// registers, and one kernel multiplies them with the experts' down matrices and lays every (token, choice)'s output into
+// a plane of its own; the norm behind adds the planes as it adds any partial sums.  The expert that every token uses is
+// one more group whose list is all tokens.  Which expert and rows a work-group takes follows from the counts, which are
+// on the GPU: the grid is the most tiles there can be, and work-groups beyond the counted ones leave at once.
+// Of K the tiles hold 128-byte rows as the plain products' deep forms do (tile.h); 128 columns and BM rows of a tile on four
+// waves.  Where units have a gate, the two 32-wide blocks of a wave's columns are 32 gate rows and the up rows beside them.
+#define GROUP_PLACE_BITS 24        // a list's entry: the token, and behind it which of the token's choices the expert is
+#define GROUP_MAX_EXPERTS 64       // (a lane an expert)
+
+// Tiles of 128 rows (two stages, two work-groups to a compute unit) from this many rows an expert on average, tiles of 64
+// (three stages, two work-groups) below and for float.  Measured with the router (us, every expert on every row / tiles of 64 /
+// of 128; 8 experts of the width, two a token): width 1,024 with gates, 128 tokens 37 / 33 / 42, 512 61 / 40 / 48, 1,024 97 / 58 / 57, 2,048
+// 157 / 91 / 88, 4,096 289 / 154 / 142; width 2,048 without gates and a shared expert, 200 tokens 98 / 51 / 69, 773 250 / 102 / 101, 2,048
+// 378 / 221 / 192.  One work-group to a unit with more stages loses (128 rows in four: 106 us at 2,048 tokens).  Float: width
+// 1,024 with gates, 128 tokens 104 / 92 / 150, 2,048 908 / 310 / 353.  From 65 tokens on the rows win or draw (65 tokens of 1,024
+// without gates: 36.6 / 37.2).  What bounds them is what a compute unit pulls, as in the plain products' deep forms: 0.5 to 0.6 PFLOP/s.
+#define EXPERT_TALL_ROWS 192
+
+struct GroupExpertsCall {
+  int dtype;                // element type of `h`
+  int tokens;
+  int experts, identity;    // experts with tensors and identity experts, as in GatedExpertsCall
+  int top;
+  int width;
+  const float* weights;     // [tokens][experts + identity]
+  int* rows;                // [experts][pitch]: the tokens that use an expert, in order
+  int64_t pitch;
+  int* counts;              // [experts]
+  const void* h;            // [tokens][ldh]
+  int64_t ldh;
+  float* out;               // [top][..][ld_out]: rows of planes that no expert writes are written here: the identity experts'
+  int64_t plane;            // weights * h, or zeros
+  int64_t ld_out;
+};
+
+template <typename T>
+__global__ void __launch_bounds__(1024) group_experts_kernel(GroupExpertsCall c) {
+  __shared__ int found[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, outputs = c.experts + c.identity;
+  if ((int)blockIdx.x < c.experts) {
+    const int e = blockIdx.x;
+    int base = 0;
+    for (int t0 = 0; t0 < c.tokens; t0 += 1024) {
+      const int t = t0 + threadIdx.x;
+      const float* w = c.weights + (int64_t)(t < c.tokens ? t : 0) * outputs;
+      bool mine = false;
+      int place = 0;
+      if (t < c.tokens) {
+        mine = w[e] != 0.f;
+        for (int i = 0; i < e; ++i) place += w[i] != 0.f ? 1 : 0;
+      }
+      const unsigned long long all = __builtin_amdgcn_ballot_w64(mine);
+      if (lane == 0) found[wave] = __builtin_popcountll(all);
+      __syncthreads();
+      int before = base + __builtin_popcountll(all & ((1ull << lane) - 1)), total = 0;
+      for (int i = 0; i < 16; ++i) {
+        before += i < wave ? found[i] : 0;
+        total += found[i];
+      }
+      if (mine) c.rows[e * c.pitch + before] = (place << GROUP_PLACE_BITS) | t;
+      base += total;
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) c.counts[e] = base;
+    return;
+  }
+  const int t = ((int)blockIdx.x - c.experts) * 16 + wave;              // a wave a token
+  if (t >= c.tokens) return;
+  const float* w = c.weights + (int64_t)t * outputs;
+  const int used = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < c.experts && w[lane < c.experts ? lane : 0] != 0.f));
+  if (used >= c.top) return;
+  float own = 0.f;
+  for (int i = 0; i < c.identity; ++i) own += w[c.experts + i];
+  const T* h = static_cast<const T*>(c.h) + (int64_t)t * c.ldh;
+  for (int p = used; p < c.top; ++p) {
+    float* out = c.out + p * c.plane + (int64_t)t * c.ld_out;
+    for (int col = lane; col < c.width; col += 64) out[col] = p == used && own != 0.f ? own * to_float(h[col]) : 0.f;
+  }
+}
+
+BT_EXPORT int bt_group_experts_call(void* stream, const GroupExpertsCall* c) {
+  if (c->tokens <= 0) return BT_OK;
+  if (c->experts <= 0 || c->experts > GROUP_MAX_EXPERTS || c->identity < 0 || c->top <= 0 || c->top > 64 || c->width <= 0)
+    BT_REFUSE("group_experts: %d experts (1..%d), %d identity experts, %d a token", c->experts, GROUP_MAX_EXPERTS, c->identity, c->top);
+  if (c->tokens >= 1 << GROUP_PLACE_BITS) BT_REFUSE("group_experts: %d tokens are too many", c->tokens);
+  if (!c->weights || !c->rows || !c->counts || !c->h || !c->out || c->pitch < c->tokens || c->ldh < c->width || c->ld_out < c->width)
+    BT_REFUSE("group_experts: missing operand or rows too short");
+  dim3 grid(c->experts + (c->tokens + 15) / 16), block(1024);
+  if (c->dtype == 0)
+    hipLaunchKernelGGL(group_experts_kernel<float>, grid, block, 0, (hipStream_t)stream, *c);
+  else
+    hipLaunchKernelGGL(group_experts_kernel<bf16_t>, grid, block, 0, (hipStream_t)stream, *c);
+  return bt_check_launch("group_experts");
+}
+
+struct ExpertProductsCall {
+  int dtype;                // element type of `a`, `w` and, of the first product, `hidden`
+  int second;               // 0: units of the listed rows of `a` = h; 1: `a` = the units, outputs into planes
+  int tokens;
+  int experts, identity, top;
+  int ff, shared_ff, width; // shared_ff 0: no expert that every token uses
+  const int* rows;          // as group_experts leaves them
+  int64_t pitch;
+  const int* counts;
+  const void* h;            // [tokens][ldh]
+  int64_t ldh;
+  const void* w;            // first: [rows][ld_w], rows as `gu` of GatedExpertsCall has columns; second: [width][ld_w], an
+  int64_t ld_w;             // expert's ff columns behind the other's, the shared expert's behind them
+  const float* weights;     // [tokens][experts + identity]
+  const float* gate;        // [tokens] or null
+  void* hidden;             // [tokens * top][ff]: the listed rows one expert behind the other
+  void* shared_hidden;      // [tokens][shared_ff]
+  float* out;               // second: [top (+ 1: the shared expert's)][..][ld_out]
+  int64_t plane;
+  int64_t ld_out;
+  int act;                  // as in GatedExpertsCall
+  float limit, alpha;
+};
+
+// Which tile a work-group takes: of which expert (-1: the shared one), its first row in the expert's list and column tile.
+struct GroupTile {
+  int expert, first, count, column;
+  int slot;                 // where the expert's rows start in `hidden`
+};
+
+template <int BM>
+__device__ __forceinline__ bool group_tile(const ExpertProductsCall& c, int columns, int shared_columns, GroupTile& tile) {
+  const int lane = threadIdx.x & 63;
+  const int count = lane < c.experts ? c.counts[lane] : 0, tiles = (count + BM - 1) / BM;
+  int rows_to = count, tiles_to = tiles;                                // sums up to and with this lane's expert
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int r = __shfl_up(rows_to, o, 64), t = __shfl_up(tiles_to, o, 64);
+    if (lane >= o) { rows_to += r; tiles_to += t; }
+  }
+  const int routed = __builtin_amdgcn_readlane(tiles_to, 63) * columns;
+  const int all = routed + (c.tokens + BM - 1) / BM * shared_columns;
+  if ((int)blockIdx.x >= all) return false;
+  const int id = xcd_contiguous(blockIdx.x, all);
+  if (id >= routed) {
+    tile.expert = -1;
+    tile.first = (id - routed) / shared_columns * BM;
+    tile.column = (id - routed) % shared_columns;
+    tile.count = c.tokens;
+    tile.slot = 0;
+    return true;
+  }
+  const int row_tile = id / columns;
+  tile.column = id % columns;
+  tile.expert = __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles_to > row_tile));
+  tile.count = __builtin_amdgcn_readlane(count, tile.expert);
+  tile.first = (row_tile - (__builtin_amdgcn_readlane(tiles_to, tile.expert) - __builtin_amdgcn_readlane(tiles, tile.expert))) * BM;
+  tile.slot = __builtin_amdgcn_readlane(rows_to, tile.expert) - tile.count;
+  return true;
+}
+
+template <typename T, int BM, int STAGES, bool SECOND, bool GATED>
+__global__ void __launch_bounds__(256) expert_products_kernel(ExpertProductsCall c) {
+  constexpr int ELEMS = Mma<T>::ELEMS, ROW_K = 8 * ELEMS, BN = 128;
+  constexpr int STAGE_BYTES = (BM + BN) * TILE_ROW_BYTES;
+  constexpr int LOADS = (BM + BN) / 32;
+  constexpr int TM = BM / 64;
+  constexpr int HELD = !SECOND && GATED ? 64 : 128;                     // output columns of a tile
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // [STAGES][BM + BN][128 bytes]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave & 1, wn = wave >> 1, l32 = lane & 31, g = lane >> 5;
+  GroupTile tile;
+  const int columns = SECOND ? (c.width + HELD - 1) / HELD : (c.ff + HELD - 1) / HELD;
+  const int shared_columns = c.shared_ff == 0 ? 0 : SECOND ? columns : (c.shared_ff + HELD - 1) / HELD;
+  if (!group_tile<BM>(c, columns, shared_columns, tile)) return;        // (the whole work-group)
+  const bool shared = tile.expert < 0;
+  const int ff = shared ? c.shared_ff : c.ff, n_base = tile.column * HELD, n_end = SECOND ? c.width : ff;
+  const int* list = c.rows + (int64_t)(shared ? 0 : tile.expert) * c.pitch;
+  auto entry = [&](int m) { return shared ? m : list[m]; };
+  auto token = [&](int m) { return entry(m) & ((1 << GROUP_PLACE_BITS) - 1); };
+
+  // operands: a stage's rows are BM of A, then BN of W; the addresses' first parts are the same for the whole work-group
+  const T *a, *w;
+  if (SECOND) {
+    a = shared ? static_cast<const T*>(c.shared_hidden) : static_cast<const T*>(c.hidden) + (int64_t)tile.slot * c.ff;
+    w = static_cast<const T*>(c.w) + (int64_t)(shared ? c.experts : tile.expert) * c.ff;
+  } else {
+    a = static_cast<const T*>(c.h);
+    w = static_cast<const T*>(c.w) + (int64_t)(shared ? c.experts : tile.expert) * c.ff * (GATED ? 2 : 1) * c.ld_w;
+  }
+  const int64_t ld_a = SECOND ? ff : c.ldh;
+  const unsigned char* a_bytes = reinterpret_cast<const unsigned char*>(a);
+  const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(w);
+  const int count = (SECOND ? ff : c.width) / ROW_K;
+  int64_t off[LOADS];
+  bool from_w[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    const int first_row = __builtin_amdgcn_readfirstlane(8 * (LOADS * wave + j));
+    from_w[j] = first_row >= BM;                  // (eight rows never straddle BM)
+    const int stage_row = first_row + (lane >> 3), chunk = (lane & 7) ^ ((stage_row >> 1) & 7);
+    int64_t row;
+    if (from_w[j]) {
+      const int r = stage_row - BM;
+      int n = !SECOND && GATED ? n_base + (r >> 6) * 32 + (r & 31) : n_base + r;
+      n = n < n_end ? n : n_end - 1;
+      row = (!SECOND && GATED && (r & 32) ? ff : 0) + n;
+    } else {
+      int m = tile.first + stage_row;
+      m = m < tile.count ? m : tile.count - 1;
+      row = SECOND ? m : token(m);
+    }
+    off[j] = (row * (from_w[j] ? c.ld_w : ld_a) + chunk * ELEMS) * (int64_t)sizeof(T);
+  }
+  auto issue = [&](int stage) {
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)((from_w[j] ? w_bytes : a_bytes) + off[j]),
+          (__attribute__((address_space(3))) void*)(lds + stage * STAGE_BYTES + 8 * (LOADS * wave + j) * TILE_ROW_BYTES),
+          16, 0, 0);
+    a_bytes += TILE_ROW_BYTES;
+    w_bytes += TILE_ROW_BYTES;
+  };
+  // the rows' tokens and weights are asked for before the operands
+  int held[TM];
+  float weight[TM];
+#pragma unroll
+  for (int bm = 0; bm < TM; ++bm) {
+    const int m = tile.first + wm * (BM / 2) + bm * 32 + l32;
+    held[bm] = m < tile.count ? entry(m) : -1;
+    weight[bm] = 1.f;
+    if (!SECOND && held[bm] >= 0) {
+      const int t = held[bm] & ((1 << GROUP_PLACE_BITS) - 1);
+      if (!shared) weight[bm] = c.weights[(int64_t)t * (c.experts + c.identity) + tile.expert];
+      else if (c.gate) weight[bm] = c.gate[t];
+    }
+  }
+  int w_rd[4], a_rd[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    w_rd[kk] = BM * TILE_ROW_BYTES + swizzled(wn * 64 + l32, 2 * kk + g);
+    a_rd[kk] = swizzled(wm * (BM / 2) + l32, 2 * kk + g);
+  }
+  floatx16 acc[2][TM];
+#pragma unroll
+  for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0.f;
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < count) issue(t);
+  int stage = 0, next_stage = STAGES - 1;
+  for (int i = 0; i < count; ++i) {
+    wait_for_all_but<STAGES - 2, LOADS>(count - 1 - i);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (i + STAGES - 1 < count) issue(next_stage);
+    const unsigned char* base = lds + stage * STAGE_BYTES;
+    int4v wop[4][2], aop[4][TM];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) wop[kk][b] = *reinterpret_cast<const int4v*>(base + w_rd[kk] + b * 4096);
+#pragma unroll
+      for (int b = 0; b < TM; ++b) aop[kk][b] = *reinterpret_cast<const int4v*>(base + a_rd[kk] + b * 4096);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+        for (int bm = 0; bm < TM; ++bm) Mma<T>::block32(acc[bn][bm], wop[kk][bn], aop[kk][bm]);
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+    next_stage = next_stage + 1 == STAGES ? 0 : next_stage + 1;
+  }
+
+  // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m)
+  GatedExpertsCall unit;
+  unit.act = c.act;
+  unit.limit = c.limit;
+  unit.alpha = c.alpha;
+#pragma unroll
+  for (int bm = 0; bm < TM; ++bm) {
+    if (held[bm] < 0) continue;
+    const int m = tile.first + wm * (BM / 2) + bm * 32 + l32;
+    if (SECOND) {
+      const int t = held[bm] & ((1 << GROUP_PLACE_BITS) - 1), place = shared ? c.top : held[bm] >> GROUP_PLACE_BITS;
+      float* out = c.out + place * c.plane + (int64_t)t * c.ld_out;
+#pragma unroll
+      for (int bn = 0; bn < 2; ++bn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int n = n_base + wn * 64 + bn * 32 + q * 8 + g * 4;
+          if (n < n_end) *reinterpret_cast<floatx4*>(out + n) = floatx4{acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
+        }
+    } else {
+      T* out = shared ? static_cast<T*>(c.shared_hidden) + (int64_t)m * ff : static_cast<T*>(c.hidden) + (int64_t)(tile.slot + m) * ff;
+#pragma unroll
+      for (int bn = 0; bn < (GATED ? 1 : 2); ++bn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int n = n_base + (GATED ? wn * 32 : wn * 64 + bn * 32) + q * 8 + g * 4;
+          if (n >= n_end) continue;
+          typedef __attribute__((__vector_size__(4 * sizeof(T)))) T T4;
+          T4 v;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            v[i] = from_float<T>(weight[bm] * (GATED ? gated_unit(unit, acc[0][bm][4 * q + i], acc[1][bm][4 * q + i])
+                                                     : plain_unit(unit, acc[bn][bm][4 * q + i])));
+          *reinterpret_cast<T4*>(out + n) = v;
+        }
+    }
+  }
+}
+
+template <typename T, int BM, int STAGES, bool SECOND, bool GATED>
+static int launch_expert_products(hipStream_t s, const ExpertProductsCall& c) {
+  auto kernel = expert_products_kernel<T, BM, STAGES, SECOND, GATED>;
+  const size_t lds = (size_t)STAGES * (BM + 128) * TILE_ROW_BYTES;
+  static bool raised = false;
+  if (!raised) {
+    hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (err != hipSuccess) BT_REFUSE("expert_products: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));
+    raised = true;
+  }
+  const int held = !SECOND && GATED ? 64 : 128;
+  const int64_t columns = ((SECOND ? c.width : c.ff) + held - 1) / held;
+  const int64_t shared_columns = c.shared_ff == 0 ? 0 : SECOND ? columns : (c.shared_ff + held - 1) / held;
+  const int64_t most = ((int64_t)c.tokens * c.top / BM + c.experts) * columns + (int64_t)((c.tokens + BM - 1) / BM) * shared_columns;
+  if (most > 0x7fffffff) BT_REFUSE("expert_products: %lld tiles are too many", (long long)most);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)most), dim3(256), lds, s, c);
+  return bt_check_launch("expert_products");
+}
+
+template <typename T, int BM, int STAGES>
+static int launch_expert_form(hipStream_t s, const ExpertProductsCall& c) {
+  if (c.second) return launch_expert_products<T, BM, STAGES, true, false>(s, c);
+  return c.act < 2 ? launch_expert_products<T, BM, STAGES, false, true>(s, c) : launch_expert_products<T, BM, STAGES, false, false>(s, c);
+}
+
+BT_EXPORT int bt_expert_products_call(void* stream, const ExpertProductsCall* c) {
+  if (c->tokens <= 0) return BT_OK;
+  const int row_k = c->dtype == 0 ? 32 : 64, elems = c->dtype == 0 ? 4 : 8;
+  if (c->dtype != 0 && c->dtype != 1) BT_REFUSE("expert_products: element type %d is neither float nor bfloat16", c->dtype);
+  if (c->experts <= 0 || c->experts > GROUP_MAX_EXPERTS || c->identity < 0 || c->top <= 0 || c->ff <= 0 || c->shared_ff < 0 || c->act < 0 || c->act > 4)
+    BT_REFUSE("expert_products: %d experts (1..%d) of %d, %d a token, activation %d", c->experts, GROUP_MAX_EXPERTS, c->ff, c->top, c->act);
+  if (c->width % row_k || c->ff % row_k || c->shared_ff % row_k)
+    BT_REFUSE("expert_products: width %d and experts of %d and %d must be multiples of %d", c->width, c->ff, c->shared_ff, row_k);
+  const int64_t inner = (int64_t)c->experts * c->ff + c->shared_ff;
+  if (c->ld_w % elems || c->ldh % elems || c->ld_out % 4 || c->plane % 4 || c->ld_w < (c->second ? inner : c->width) || c->ldh < c->width || c->ld_out < c->width ||
+      c->pitch < c->tokens || c->tokens >= 1 << GROUP_PLACE_BITS)
+    BT_REFUSE("expert_products: rows too short or not of whole 16 bytes");
+  if (!c->rows || !c->counts || !c->h || !c->w || !c->weights || !c->hidden || (c->shared_ff && !c->shared_hidden) || (c->second && !c->out) ||
+      (((uintptr_t)c->h | (uintptr_t)c->w | (uintptr_t)c->hidden | (uintptr_t)c->shared_hidden | (uintptr_t)c->out) & 15))
+    BT_REFUSE("expert_products: missing operand, or one that is not aligned to 16 bytes");
+  hipStream_t s = (hipStream_t)stream;
+  if (c->dtype == 0) return launch_expert_form<float, 64, 3>(s, *c);
+  return (int64_t)c->tokens * c->top >= (int64_t)EXPERT_TALL_ROWS * c->experts ? launch_expert_form<bf16_t, 128, 2>(s, *c)
+                                                                              : launch_expert_form<bf16_t, 64, 3>(s, *c);
 }
 
 // hidden[t][e * ff + i] *= the token's weight of expert e, for `experts` experts side by side, from the router's logits of

@@ -209,6 +209,22 @@ class RouteCall(ctypes.Structure):
     _step_fields_ = {"tokens": "tokens"}
 
 
+class GroupExpertsCall(ctypes.Structure):
+    _fields_ = [("dtype", _c_int), ("tokens", _c_int), ("experts", _c_int), ("identity", _c_int), ("top", _c_int), ("width", _c_int),
+                ("weights", _c_ptr), ("rows", _c_ptr), ("pitch", _c_i64), ("counts", _c_ptr), ("h", _c_ptr), ("ldh", _c_i64),
+                ("out", _c_ptr), ("plane", _c_i64), ("ld_out", _c_i64)]
+    _step_fields_ = {"tokens": "tokens"}
+
+
+class ExpertProductsCall(ctypes.Structure):
+    _fields_ = [("dtype", _c_int), ("second", _c_int), ("tokens", _c_int), ("experts", _c_int), ("identity", _c_int), ("top", _c_int),
+                ("ff", _c_int), ("shared_ff", _c_int), ("width", _c_int), ("rows", _c_ptr), ("pitch", _c_i64), ("counts", _c_ptr),
+                ("h", _c_ptr), ("ldh", _c_i64), ("w", _c_ptr), ("ld_w", _c_i64), ("weights", _c_ptr), ("gate", _c_ptr),
+                ("hidden", _c_ptr), ("shared_hidden", _c_ptr), ("out", _c_ptr), ("plane", _c_i64), ("ld_out", _c_i64),
+                ("act", _c_int), ("limit", _c_float), ("alpha", _c_float)]
+    _step_fields_ = {"tokens": "tokens"}
+
+
 class WeighExpertsCall(ctypes.Structure):
     _fields_ = [("route", RouteCall), ("ff", _c_int), ("logits", _c_ptr), ("ld_logits", _c_i64), ("hidden", _c_ptr), ("ld_hidden", _c_i64)]
     _step_fields_ = {"route.tokens": "tokens"}
@@ -1442,6 +1458,46 @@ def gated_experts(gu, weights, gate, experts, ff, shared_ff, identity, hidden, h
                              act=act, limit=limit or 0.0, alpha=alpha,
                              hidden=hidden.data_ptr(), ld_hidden=hidden.stride(0), h=_ptr(h),
                              ldh=h.stride(0) if h is not None else 0, identity_out=_ptr(identity_out)))
+
+
+GROUPED_EXPERTS = True       # tests switch it off to compare
+
+
+def groups_experts(tokens, experts, top, ff, shared_ff, width, dtype):
+    """Whether a step's experts are run on the rows that use them (``grouped_experts``): from 65 tokens on (below, one
+    product that reads all matrices once is all there is to do), where a token uses at most half of the experts and at
+    most four, each of which leaves a plane for the norm to read, and the sizes are whole rows of a tile."""
+    row = 64 if dtype == torch.bfloat16 else 32
+    return GROUPED_EXPERTS and tokens > 64 and experts <= 64 and 2 * top <= experts and top <= 4 and \
+        width % row == 0 and ff % row == 0 and shared_ff % row == 0
+
+
+def grouped_experts(h, weights, gate, in_weight, down_weight, experts, ff, shared_ff, identity, top, step, out, limit=None, alpha=1.0,
+                    unit=None):
+    """out [top (+ 1 with ``shared_ff``), rows, width] float32: plane j holds the output of each row's j-th expert (in the order
+    of the experts) times its weight, an identity expert's, or zeros, the last plane the shared expert's times ``gate``;
+    operands as in ``gated_experts``, ``in_weight`` and ``down_weight`` the matrices of the products around it."""
+    tokens, width = h.shape
+    pitch = step.token_capacity
+    rows = step.buffer("experts.rows", experts + 1, pitch, "int32")           # (the last row: the counts)
+    counts = rows[experts]
+    hidden = step.buffer("experts.listed", tokens * top, ff, h.dtype)
+    shared = step.buffer("experts.shared", tokens, shared_ff, h.dtype) if shared_ff else None
+    if out.dtype != torch.float32 or out.stride(2) != 1 or h.stride(1) != 1 or out.shape[0] != top + (1 if shared_ff else 0):
+        raise KernelError(f"grouped_experts: float32 planes for {top} choices, got {tuple(out.shape)} {out.dtype}")
+    module, dtype = _module("experts"), DTYPE_CODES[h.dtype]
+    _launch(module, "bt_group_experts_call",
+            GroupExpertsCall(dtype=dtype, tokens=tokens, experts=experts, identity=identity, top=top, width=width,
+                             weights=weights.data_ptr(), rows=rows.data_ptr(), pitch=pitch, counts=counts.data_ptr(), h=h.data_ptr(),
+                             ldh=h.stride(0), out=out.data_ptr(), plane=out.stride(0), ld_out=out.stride(1)))
+    act = EXPERT_UNITS[unit] if unit is not None else (0 if limit is None else 1)
+    for second, matrix in ((0, in_weight), (1, down_weight)):
+        _launch(module, "bt_expert_products_call",
+                ExpertProductsCall(dtype=dtype, second=second, tokens=tokens, experts=experts, identity=identity, top=top, ff=ff,
+                                   shared_ff=shared_ff, width=width, rows=rows.data_ptr(), pitch=pitch, counts=counts.data_ptr(),
+                                   h=h.data_ptr(), ldh=h.stride(0), w=matrix.data_ptr(), ld_w=matrix.stride(0),
+                                   weights=weights.data_ptr(), gate=_ptr(gate), hidden=hidden.data_ptr(), shared_hidden=_ptr(shared),
+                                   out=out.data_ptr(), plane=out.stride(0), ld_out=out.stride(1), act=act, limit=limit or 0.0, alpha=alpha))
 
 
 # --- norms in parts, capped logits -------------------------------------------------------------

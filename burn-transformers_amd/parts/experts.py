@@ -26,15 +26,15 @@ expert's output is added as it is).
           an identity expert's output being h itself,
         + sigmoid(shared_mix . h) * shared(h)
 
-How a step computes it: ONE product with every expert's gate and up matrices laid one behind the
+How a step of up to 64 tokens computes it: ONE product with every expert's gate and up matrices laid one behind the
 other (the shared expert's last), a kernel that applies silu(gate) * up times the token's weight of
 that expert (zero where it was not chosen, the sigmoid gate for the shared expert), and ONE product
-with the down matrices laid side by side, which so sums the weighted outputs.  No token is moved
-and nothing depends on the host knowing the choice, so the step is a fixed list of kernels like
-every other; the price is that every expert multiplies every token.  In decode steps that costs
-little once tokens * top reaches the number of experts (all matrices are read anyway); a prompt does
-experts / top times the routed arithmetic, which a grouped product over tokens sorted by expert
-would save.
+with the down matrices laid side by side, which so sums the weighted outputs.  Every expert multiplies every token,
+which costs little while all matrices are read anyway.
+
+Steps of more tokens run every expert on the rows that use it (``kernels.library.grouped_experts``): the rows are
+listed on the GPU, gathered while they are brought in, and every choice's output lies in a plane of its own that the
+norm behind adds.  Nothing depends on the host knowing the choice either, so a step is a fixed list of kernels both ways.
 
 In small steps the router's logits come from the same product (``rides``: units without a gate whose activation the product
 has, a router that the products' type holds exactly, nothing else beside the experts): its rows lie before the up matrices,
@@ -150,6 +150,11 @@ class RoutedExperts(FeedForward):
         mix = step.buffer("experts.mix", tokens, 1, "float32") if self.shared_mix is not None else None
         K.route(h, self.router, self.correction, self.top, self.groups, self.keep, weights, self.shared_mix, mix,
                 score=self.score, group_rank=self.group_rank, normalize=self.normalize, bias=self.router_bias)
+        if K.groups_experts(tokens, self.experts, self.top, self.ff, self.shared_ff, self.width, step.dtype):
+            partials = step.partial_sums("experts.partials", self.top + (1 if self.shared_ff else 0), tokens, self.width)
+            K.grouped_experts(h, weights, mix, self.in_weight, self.down_weight, self.experts, self.ff, self.shared_ff, self.identity,
+                              self.top, step, partials, limit=self.limit, alpha=self.alpha, unit=None if self.gated else self.unit)
+            return Delta(partials, None)
         fused = step.buffer("experts.fused", tokens, self.fused_cols, step.dtype)
         K.gemm(h, self.in_weight, K.epilogue_store(fused), packed=self.in_packed)
         hidden = step.buffer("experts.hidden", tokens, self.hidden_cols, step.dtype)

@@ -1,0 +1,103 @@
+"""Experts run on the rows that use them, against every expert on every row in 64 bits."""
+
+import pytest
+import torch
+
+from burn_transformers_amd.kernels import library as K
+from burn_transformers_amd.parts import lookup
+from burn_transformers_amd.parts.base import ResidualStream
+
+from step_helpers import make_step
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DTYPES = {"float32": torch.float32, "bfloat16": torch.bfloat16}
+
+
+def unit_of(kind, g, u, limit):
+    if kind == "gated" and limit is not None:
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        return g * torch.sigmoid(1.5 * g) * (u + 1.0)
+    if kind == "gated":
+        return g * torch.sigmoid(g) * u
+    return {"gelu_erf": torch.nn.functional.gelu(u), "silu": u * torch.sigmoid(u), "squared_relu": u.clamp(min=0.0) ** 2}[kind]
+
+
+# rows around a tile's 64 and 128, experts that nobody chose and one that all chose (its list is all rows), identity
+# experts among a row's choices (`zero`: weights that are exactly zero although chosen), a shared expert of another
+# width with and without its gate, widths of one tile and of several that are not whole
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("tokens,width,experts,top,ff,shared_ff,identity,kind,limit,mix,skew", [
+    (65, 64, 8, 2, 64, 0, 0, "gated", None, False, "even"), (129, 128, 4, 2, 192, 128, 1, "gated", None, True, "even"),
+    (300, 192, 8, 1, 64, 64, 0, "squared_relu", None, False, "one"), (520, 64, 8, 3, 128, 192, 2, "gelu_erf", None, True, "even"),
+    (1000, 64, 16, 4, 64, 0, 0, "gated", 2.0, False, "one"), (257, 320, 5, 2, 320, 64, 0, "silu", None, False, "zero"),
+    (700, 64, 4, 2, 64, 0, 0, "gated", None, False, "one")])
+def test_experts_on_their_rows(dtype, tokens, width, experts, top, ff, shared_ff, identity, kind, limit, mix, skew):
+    gen = torch.Generator().manual_seed(tokens + width + experts)
+    dt, outputs = DTYPES[dtype], experts + identity
+    draw = lambda *shape: torch.randn(*shape, generator=gen).to(dt).double()
+    scale = width ** -0.5
+    tensors = {"router": torch.zeros(outputs, width)}
+    made = {}
+    for e in list(range(experts)) + (["shared"] if shared_ff else []):
+        inner = shared_ff if e == "shared" else ff
+        name = (lambda role: f"shared_{role}") if e == "shared" else (lambda role: f"{role}_{e}")
+        made[e] = [(draw(inner, width) * scale).to(dt).double(), (draw(inner, width) * scale).to(dt).double(), (draw(width, inner) * inner ** -0.5).to(dt).double()]
+        for role, tensor in zip(("gate", "up", "down"), made[e]):
+            if role != "gate" or kind == "gated":
+                tensors[name(role)] = tensor.to(dt)
+    if mix:
+        tensors["shared_mix"] = torch.zeros(1, width)
+    params = {"width": width, "experts": experts, "ff": ff, "identity": identity, "top": top, "shared_ff": shared_ff, "limit": limit,
+              "alpha": 1.5, "unit": kind}
+    part = lookup("feed_forward", "routed_experts")(params, {k: v.to(DEV) for k, v in tensors.items()})
+    h = draw(tokens, width)
+    # weights as the router leaves them: `top` of a row's outputs, the others zero
+    scores = torch.rand(tokens, outputs, generator=gen)
+    if skew == "one":                                                   # everybody chooses expert 1, nobody expert 2
+        scores[:, 1], scores[:, 2] = 2.0, -1.0
+    chosen = scores.topk(top, -1).indices
+    weights = torch.zeros(tokens, outputs).scatter_(1, chosen, torch.rand(tokens, top, generator=gen) + 0.1)
+    if skew == "zero":
+        weights[::7] = 0.0
+    gate = torch.rand(tokens, 1, generator=gen) if mix else None
+    want = torch.zeros(tokens, width, dtype=torch.float64)
+    for e in range(experts):
+        g, u, d = made[e]
+        want += weights[:, e:e + 1].double() * (unit_of(kind, h @ g.T, h @ u.T, limit) @ d.T)
+    want += weights[:, experts:].double().sum(1, keepdim=True) * h
+    if shared_ff:
+        g, u, d = made["shared"]
+        out = unit_of(kind, h @ g.T, h @ u.T, limit) @ d.T
+        want += out * (gate.double() if mix else 1.0)
+    step = make_step(dt, [tokens])
+    planes = torch.full((top + (1 if shared_ff else 0), tokens + 3, width), float("nan"), device=DEV)[:, :tokens]
+    assert K.groups_experts(tokens, experts, top, ff, shared_ff, width, dt) == (2 * top <= experts)
+    K.grouped_experts(h.to(dt).to(DEV), weights.to(DEV), None if gate is None else gate.to(DEV), part.in_weight, part.down_weight,
+                      experts, ff, shared_ff, identity, top, step, planes, limit=limit, alpha=1.5, unit=None if kind == "gated" else kind)
+    got = planes.sum(0).cpu().double()
+    error = float((got - want).abs().max() / want.abs().max())
+    # units rounded once to the products' type; sums of a few hundred 32-bit products
+    assert error < (3e-6 if dtype == "float32" else 8e-3), error
+
+
+def test_a_part_takes_them_in_steps_of_many_tokens():
+    """The part's two ways give the same sums, in steps on both sides of the rule."""
+    gen = torch.Generator().manual_seed(3)
+    width, experts, ff = 128, 8, 128
+    tensors = {"router": torch.randn(experts, width, generator=gen) * 0.1}
+    for e in range(experts):
+        for role, shape in (("gate", (ff, width)), ("up", (ff, width)), ("down", (width, ff))):
+            tensors[f"{role}_{e}"] = (torch.randn(shape, generator=gen) * 0.1).to(torch.bfloat16)
+    part = lookup("feed_forward", "routed_experts")({"width": width, "experts": experts, "ff": ff, "top": 2}, {k: v.to(DEV) for k, v in tensors.items()})
+    for tokens in (64, 65, 200):
+        h = torch.randn(tokens, width, generator=gen).to(torch.bfloat16).to(DEV)
+        sums = []
+        for way in (True, False):
+            K.GROUPED_EXPERTS = way
+            try:
+                delta = part.forward(h, make_step(torch.bfloat16, [tokens]), ResidualStream(torch.zeros(tokens, width, device=DEV)))
+                sums.append(delta.partials.sum(0).cpu().double())
+            finally:
+                K.GROUPED_EXPERTS = True
+        assert float((sums[0] - sums[1]).abs().max() / sums[1].abs().max()) < 1.2e-2
