@@ -588,14 +588,6 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
 // every wave's part of W S0 and R S0 meets in LDS.  The operands of the next KB_AHEAD - 1 blocks are on their way.
 #define KB_AHEAD 4
 
-// A barrier that waits for this wave's LDS traffic only: operands asked for blocks ahead stay on their way.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);                      // lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 template <int FORM, int TW>
 struct KbStage {
   floatx4 w[FORM == 0 ? TW : 1], r[TW], ku[TW], a[TW], u;

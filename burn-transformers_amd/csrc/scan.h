@@ -26,6 +26,14 @@ __device__ __forceinline__ float sum_of_16_lanes(float v) {
   return v;
 }
 
+// A barrier that waits for this wave's LDS traffic only: operands asked for blocks ahead stay on their way.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);                      // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus_f(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
 

@@ -487,6 +487,9 @@ struct HeadScanCall {
   int span;
   int max_count;
   float* carry;
+  // null, or room for what blocks of 16 tokens leave, aligned to 16 bytes: (tokens / 16 + n_seqs + 1) blocks of 32 groups * state +
+  // 288 heads floats; with it long sequences go in blocks on the matrix units
+  float* blocks;
 };
 
 // The state of a slot is laid out for this kernel's lanes: [heads][tiles of 4 channels][state][4], so
@@ -644,6 +647,251 @@ static void launch_head_scan_r(hipStream_t stream, const HeadScanCall& c) {
   hipLaunchKernelGGL((head_scan_kernel<R, 0>), grid, block, (size_t)chunk * per_token * sizeof(float), stream, c, chunk, 1, tiles);
 }
 
+// --- the same in blocks of sixteen tokens on the matrix units -----------------------------------
+//
+// With one decay a head a block of 16 tokens does to the state what a few products do.  With a_t the product of the
+// block's decays up to and with token t, b_s that of the decays behind token s and
+//     G = C B^T,   M[t][s] = G[t][s] g_(s+1) .. g_t dt_s   (s <= t):
+//     y = diag(a) C S0 + M x + D x,   S = a_16 S0 + B^T diag(b dt) x
+// B and C are the group's, so one kernel lays them out for the lanes once for all heads, with G behind every head's M, a and
+// b dt, and a second one walks the blocks in order with the state in registers (v_mfma_f32_16x16x4_f32: 32 bits throughout;
+// decays are only multiplied with each other).  Operand layouts and the K values' order as in linear_attention.hip: a
+// lane's four values of a 16 x 16 tile lie side by side, step i of a product takes K number 4 g + i in lane group g, and
+// results land where the next product reads them.
+#define HB_TOKENS 16
+#define HB_HEADS 8              // heads a work-group of the first kernel prepares
+// Steps whose longest sequence brings at least this many tokens go in blocks.  Measured (us, as whole sequences or spans / in
+// blocks; 32 heads of 64 x 128): 2 x 40 tokens 16.1 / 13.2, 16 x 40 48.7 / 36.1, 2 x 128 39 / 17, 2 x 1,024 225 / 58, 8 x 300 141 / 60.
+// Of the longest, 11 us go to the operands; a block then takes 0.7 us, 0.25 of them on the matrix units: a wave is alone on
+// its SIMD and pays every instruction around them, and the trip through LDS, itself.
+#define HB_MIN_TOKENS 40
+
+// Floats of a block: a group's C and B [tiles of 16 state elements][64 lanes][4] each, then every head's M [64][4], a [16], b dt [16].
+__host__ __device__ __forceinline__ int64_t hb_floats(const HeadScanCall& c) {
+  return (int64_t)c.groups * 2 * HB_TOKENS * c.state + (int64_t)c.heads * (HB_TOKENS * HB_TOKENS + 2 * HB_TOKENS);
+}
+__device__ __forceinline__ float* hb_place(const HeadScanCall& c, int seq, int block) {
+  return c.blocks + (int64_t)(c.seq_off[seq] / HB_TOKENS + seq + block) * hb_floats(c);
+}
+
+template <int DT>
+__global__ void __launch_bounds__(256) head_blocks_kernel(HeadScanCall c) {
+  constexpr int DIM = 16 * DT, PITCH = DIM + 4;
+  __shared__ __attribute__((aligned(16))) float B[HB_TOKENS][PITCH], C[HB_TOKENS][PITCH];
+  __shared__ __attribute__((aligned(16))) floatx4 parts[4][64];
+  __shared__ float steps[HB_HEADS][HB_TOKENS], decays[HB_HEADS][HB_TOKENS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
+  const int seq = blockIdx.z, first = c.seq_off[seq] + (int)blockIdx.x * HB_TOKENS;
+  const int count = min(HB_TOKENS, c.seq_off[seq + 1] - first);
+  if (count <= 0) return;                                                // (the whole work-group)
+  const int per_group = c.heads / c.groups, sets = (per_group + HB_HEADS - 1) / HB_HEADS;
+  const int group = blockIdx.y / sets, head0 = group * per_group + blockIdx.y % sets * HB_HEADS;
+  const int heads = min(HB_HEADS, (group + 1) * per_group - head0);
+  float* place = hb_place(c, seq, blockIdx.x);
+  // rows behind the sequence's end hold zeros and decay by one: they change nothing
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    const int i = (tid + 256 * j) / DIM, d = (tid + 256 * j) % DIM;
+    const int64_t at = (int64_t)(first + min(i, count - 1)) * c.ld + group * DIM + d;
+    const float b = c.B[at], q = c.C[at];
+    B[i][d] = i < count ? b : 0.f;
+    C[i][d] = i < count ? q : 0.f;
+  }
+  if (tid < HB_HEADS * HB_TOKENS) {
+    const int h = tid / HB_TOKENS, i = tid % HB_TOKENS, head = head0 + min(h, heads - 1);
+    const float step = softplus_f(c.dt_raw[(int64_t)(first + min(i, count - 1)) * c.ld_dt + head] + c.dt_bias[head]);
+    steps[h][i] = i < count ? step : 0.f;
+    decays[h][i] = i < count ? expf(-expf(c.A_log[head]) * step) : 1.f;
+  }
+  __syncthreads();
+  floatx4 sums = {0.f, 0.f, 0.f, 0.f};
+  floatx4* frag = reinterpret_cast<floatx4*>(place + (int64_t)group * 2 * HB_TOKENS * DIM);
+  for (int tile = wave; tile < DT; tile += 4) {
+    const floatx4 q = *reinterpret_cast<const floatx4*>(&C[n][16 * tile + 4 * g]), k = *reinterpret_cast<const floatx4*>(&B[n][16 * tile + 4 * g]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], k[i], sums, 0, 0, 0);
+    if (blockIdx.y % sets == 0) {
+      floatx4 u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) u[i] = B[4 * g + i][16 * tile + n];
+      frag[64 * tile + lane] = q;
+      frag[64 * (DT + tile) + lane] = u;
+    }
+  }
+  parts[wave][lane] = sums;                                              // lane holds G[4 g + i][n]
+  __syncthreads();
+  const int t = tid >> 4, s = tid & 15;
+  float product = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) product += reinterpret_cast<const float*>(&parts[w][16 * (t >> 2) + s])[t & 3];
+  for (int h = 0; h < heads; ++h) {
+    float decay = 1.f;                                                   // of the tokens behind s up to t
+#pragma unroll
+    for (int r = 1; r < HB_TOKENS; ++r) decay *= r > s && r <= t ? decays[h][r] : 1.f;
+    float* mine = place + (int64_t)c.groups * 2 * HB_TOKENS * DIM + (int64_t)(head0 + h) * (HB_TOKENS * HB_TOKENS + 2 * HB_TOKENS);
+    mine[(t + 16 * (s >> 2)) * 4 + (s & 3)] = s <= t ? product * decay * steps[h][s] : 0.f;
+    if (s == 0) mine[HB_TOKENS * HB_TOKENS + t] = decays[h][0] * decay;
+    if (t == HB_TOKENS - 1) mine[HB_TOKENS * HB_TOKENS + HB_TOKENS + s] = decay * steps[h][s];
+  }
+}
+
+// One work-group per 16 channels of a head and sequence; four waves share the state elements, every wave's part of
+// C S0 (and one step of M x) meets in LDS.  The operands of the next HB_AHEAD - 1 blocks are on their way.
+#define HB_AHEAD 4
+
+template <int TW>
+struct HbStage {
+  floatx4 c[TW], b[TW], a, strength;
+  float m, x[4], all;
+};
+
+template <int DT>
+__global__ void __launch_bounds__(256, 2) head_blocks_walk_kernel(HeadScanCall c) {
+  constexpr int TW = (DT + 3) / 4, DIM = 16 * DT;
+  __shared__ __attribute__((aligned(16))) floatx4 parts[2][4][64];
+  // the columns of a head and sequence, and the heads of a group, read the same operands: they are numbered onto one XCD
+  const int columns = c.vdim / 16, pair = blockIdx.x / (8 * columns) * 8 + blockIdx.x % 8;
+  if (pair >= c.heads * c.n_seqs) return;
+  const int column = blockIdx.x / 8 % columns, head = pair % c.heads, seq = pair / c.heads;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
+  const int first = c.seq_off[seq], count = c.seq_off[seq + 1] - first;
+  if (count <= 0) return;
+  const int blocks = (count + HB_TOKENS - 1) / HB_TOKENS, group = head / (c.heads / c.groups);
+  const int64_t stride = hb_floats(c) * 4;
+  const int vtiles = (c.vdim + 3) / 4, p = 16 * column + n;
+  float* slot = c.S + (int64_t)c.slots[seq] * c.state_stride + ((int64_t)head * vtiles + p / 4) * DIM * 4 + p % 4;
+  auto mine = [&](int j) { return DT % 4 == 0 || wave * TW + j < DT; };
+  floatx4 S[TW];
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[j][i] = mine(j) ? slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] : 0.f;
+  const float Dh = c.D[head];
+  // a block's operands: one address that all lanes share, and every lane's distances from it
+  uint32_t from_tile[TW], from_x[4], from_last[4];
+#pragma unroll
+  for (int j = 0; j < TW; ++j) from_tile[j] = (group * 2 * HB_TOKENS * DIM + 256 * min(wave * TW + j, DT - 1) + 4 * lane) * 4;
+  const uint32_t from_head = (c.groups * 2 * HB_TOKENS * DIM + head * (HB_TOKENS * HB_TOKENS + 2 * HB_TOKENS)) * 4;
+  const uint32_t from_m = from_head + (4 * lane + wave) * 4, from_a = from_head + (HB_TOKENS * HB_TOKENS + 4 * g) * 4;
+  const int left = count - (blocks - 1) * HB_TOKENS;                      // tokens of the last block
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    from_x[i] = (uint32_t)((4 * g + i) * c.ld + p) * 4;
+    from_last[i] = (uint32_t)(min(4 * g + i, left - 1) * c.ld + p) * 4;
+  }
+  const char* at = reinterpret_cast<const char*>(hb_place(c, seq, 0));
+  const char* x_at = reinterpret_cast<const char*>(c.x + (int64_t)first * c.ld + head * c.vdim);
+  int row = 4 * g + wave, fetched = 0;                                   // a wave finishes every fourth token
+  float* out = c.y + (first + (int64_t)min(row, count - 1)) * c.ld_y + head * c.vdim + p;
+  const int64_t out_step = HB_TOKENS * c.ld_y;
+  HbStage<TW> stages[HB_AHEAD];
+  auto load4 = [&](uint32_t from) { return *reinterpret_cast<const floatx4*>(at + from); };
+  auto fetch = [&](HbStage<TW>& st) {
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      st.c[j] = load4(from_tile[j]);
+      st.b[j] = load4(from_tile[j] + HB_TOKENS * DIM * 4);
+    }
+    st.a = load4(from_a);
+    st.strength = load4(from_a + HB_TOKENS * 4);
+    st.m = *reinterpret_cast<const float*>(at + from_m);
+    st.all = *reinterpret_cast<const float*>(at + from_head + (HB_TOKENS * HB_TOKENS + HB_TOKENS - 1) * 4);
+    const bool last = fetched >= blocks - 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) st.x[i] = *reinterpret_cast<const float*>(x_at + (last ? from_last[i] : from_x[i]));
+    // on to the next block; at the end the last one's operands are asked for again and not used
+    const bool more = ++fetched < blocks;
+    at += more ? stride : 0;
+    x_at += more ? HB_TOKENS * c.ld * 4 : 0;
+  };
+  // a block's outputs are added up from LDS while the next block's products run
+  float pending = 0.f;
+  auto finish = [&](int turn) {
+    const float* r = reinterpret_cast<const float*>(&parts[turn][0][lane]) + wave;
+    const float y = ((r[0] + r[256]) + (r[512] + r[768])) + pending;
+    if (row < count) *out = y;
+    row += HB_TOKENS;
+    out += out_step;
+  };
+  auto walk = [&](HbStage<TW>& st, int turn, int block) {
+    // (a sum a tile, taken in turn: an instruction that adds to the one before it waits for it)
+    floatx4 sums[TW];
+    float x[4], u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[i] = block * HB_TOKENS + 4 * g + i < count ? st.x[i] : 0.f;
+      u[i] = st.strength[i] * x[i];
+    }
+    const float own = (wave & 2) ? ((wave & 1) ? x[3] : x[2]) : ((wave & 1) ? x[1] : x[0]);
+#pragma unroll
+    for (int j = 0; j < TW; ++j) sums[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        if (mine(j)) sums[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.c[j][i], S[j][i], sums[j], 0, 0, 0);
+    const floatx4 within = __builtin_amdgcn_mfma_f32_16x16x4f32(st.m, own, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < TW; ++j) S[j] *= st.all;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        if (mine(j)) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.b[j][i], u[i], S[j], 0, 0, 0);
+    if (TW > 1) sums[0] += sums[TW - 1];
+    parts[turn][wave][lane] = sums[0] * st.a + within;
+    if (block > 0) finish(turn ^ 1);
+    lds_barrier();
+    pending = Dh * own;
+  };
+#pragma unroll
+  for (int i = 0; i < HB_AHEAD - 1; ++i) {
+    fetch(stages[i]);
+    __builtin_amdgcn_sched_barrier(0);                     // (in order: a stage is waited for by the loads behind it)
+  }
+  for (int block = 0; block < blocks; block += HB_AHEAD) {
+#pragma unroll
+    for (int i = 0; i < HB_AHEAD; ++i) {
+      if (block + i >= blocks) break;                      // (the same for all four waves)
+      fetch(stages[(i + HB_AHEAD - 1) % HB_AHEAD]);
+      walk(stages[i], i & 1, block + i);
+    }
+  }
+  finish((blocks - 1) & 1);
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+    if (mine(j))
+#pragma unroll
+      for (int i = 0; i < 4; ++i) slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] = S[j][i];
+}
+
+template <int DT>
+static void launch_head_blocks(hipStream_t stream, const HeadScanCall& c) {
+  const int sets = (c.heads / c.groups + HB_HEADS - 1) / HB_HEADS;
+  dim3 side((c.max_count + HB_TOKENS - 1) / HB_TOKENS, c.groups * sets, c.n_seqs), block(256);
+  dim3 walk((unsigned)((c.heads * c.n_seqs + 7) / 8 * 8 * (c.vdim / 16)));
+  hipLaunchKernelGGL((head_blocks_kernel<DT>), side, block, 0, stream, c);
+  hipLaunchKernelGGL((head_blocks_walk_kernel<DT>), walk, block, 0, stream, c);
+}
+
+// True if the call went in blocks: it brings the room, tiles of 16 and enough tokens.
+static bool head_blocks(hipStream_t stream, const HeadScanCall& c) {
+  if (!c.blocks || c.max_count < HB_MIN_TOKENS || c.state % 16 != 0 || c.state > 128 || c.vdim % 16 != 0 || c.n_seqs > 65535 ||
+      (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30 || c.groups > 4096 || hb_floats(c) > 1 << 28 || 64 * c.ld > 1 << 30)
+    return false;
+  switch (c.state / 16) {
+    case 1: launch_head_blocks<1>(stream, c); break;
+    case 2: launch_head_blocks<2>(stream, c); break;
+    case 3: launch_head_blocks<3>(stream, c); break;
+    case 4: launch_head_blocks<4>(stream, c); break;
+    case 5: launch_head_blocks<5>(stream, c); break;
+    case 6: launch_head_blocks<6>(stream, c); break;
+    case 7: launch_head_blocks<7>(stream, c); break;
+    default: launch_head_blocks<8>(stream, c); break;
+  }
+  return true;
+}
+
 BT_EXPORT int bt_head_scan_call(void* stream, const HeadScanCall* c) {
   if (c->tokens <= 0) return BT_OK;
   if (c->heads <= 0 || c->vdim <= 0 || c->state <= 0 || c->state > 256 || c->groups <= 0 || c->heads % c->groups != 0 || c->n_seqs <= 0)
@@ -654,7 +902,9 @@ BT_EXPORT int bt_head_scan_call(void* stream, const HeadScanCall* c) {
       c->state_stride < (int64_t)c->heads * c->state * ((c->vdim + 3) / 4 * 4))
     BT_REFUSE("head_scan: rows or state too short for %d heads of %d", c->heads, c->vdim);
   if ((int64_t)c->tokens * c->ld >= (int64_t)1 << 31) BT_REFUSE("head_scan: the rows of B and C are addressed with 32 bits");
+  if ((uintptr_t)c->blocks % 16 != 0) BT_REFUSE("head_scan: the room for blocks is not aligned to 16 bytes");
   hipStream_t s = (hipStream_t)stream;
+  if (head_blocks(s, *c)) return bt_check_launch("head_scan");
   const int per = (c->state + 15) / 16;
   if (per <= 1) launch_head_scan_r<1>(s, *c);
   else if (per <= 2) launch_head_scan_r<2>(s, *c);

@@ -173,7 +173,7 @@ class HeadScanCall(ctypes.Structure):
                 ("groups", _c_int), ("x", _c_ptr), ("B", _c_ptr), ("C", _c_ptr), ("ld", _c_i64), ("dt_raw", _c_ptr),
                 ("ld_dt", _c_i64), ("dt_bias", _c_ptr), ("A_log", _c_ptr), ("D", _c_ptr), ("y", _c_ptr),
                 ("ld_y", _c_i64), ("S", _c_ptr), ("state_stride", _c_i64), ("seq_off", _c_ptr), ("slots", _c_ptr),
-                ("span", _c_int), ("max_count", _c_int), ("carry", _c_ptr)]
+                ("span", _c_int), ("max_count", _c_int), ("carry", _c_ptr), ("blocks", _c_ptr)]
     _step_fields_ = {"tokens": "tokens", "max_count": "max_count"}
 
 
@@ -1342,10 +1342,23 @@ def selective_scan(x, z, dt, B, C, A_log, D, out, state, step, carry=None):
                               span=SCAN_SPAN if carry is not None else 0, max_count=step.max_count, carry=_ptr(carry)))
 
 
-def head_scan(x, B, C, dt_raw, dt_bias, A_log, D, y, state, step, heads, vdim, elements, groups, carry=None):
+SCAN_BLOCK = 16       # tokens of a block of the scans that go in blocks (csrc/linear_attention.hip, csrc/state_space.hip)
+
+
+def head_blocks(step, heads, vdim, elements, groups):
+    """Room for what the blocks of a step's long sequences leave to the kernel that walks them, for a step of any shape
+    of its class; None for steps that never go in blocks."""
+    if step.max_count <= 1 or step.token_capacity < 2 * SCAN_BLOCK or elements % 16 or elements > 128 or vdim % 16:
+        return None
+    floats = groups * 2 * SCAN_BLOCK * elements + heads * (SCAN_BLOCK * SCAN_BLOCK + 2 * SCAN_BLOCK)
+    return step.buffer("scan.head_blocks", step.token_capacity // SCAN_BLOCK + step.n_seqs + 1, floats, "float32")
+
+
+def head_scan(x, B, C, dt_raw, dt_bias, A_log, D, y, state, step, heads, vdim, elements, groups, carry=None, blocks=None):
     """The scan with one decay per head (see csrc/state_space.hip); x, B and C are column ranges of
     the same float32 rows; ``state`` [slots, >= heads * elements * vdim rounded up to 4] float32, in a
-    layout of the kernel's own."""
+    layout of the kernel's own.  ``blocks``: room from ``head_blocks``; with it long sequences go in blocks of tokens on the
+    matrix units."""
     if x.stride(0) != B.stride(0) or x.stride(0) != C.stride(0):
         raise KernelError("head_scan: x, B and C must be column ranges of the same rows")
     _launch(_module("state_space"), "bt_head_scan_call",
@@ -1354,7 +1367,8 @@ def head_scan(x, B, C, dt_raw, dt_bias, A_log, D, y, state, step, heads, vdim, e
                          ld_dt=dt_raw.stride(0), dt_bias=dt_bias.data_ptr(), A_log=A_log.data_ptr(), D=D.data_ptr(),
                          y=y.data_ptr(), ld_y=y.stride(0), S=state.data_ptr(), state_stride=state.stride(0),
                          seq_off=step.seq_off.data_ptr(), slots=step.slots.data_ptr(),
-                         span=SCAN_SPAN if carry is not None else 0, max_count=step.max_count, carry=_ptr(carry)))
+                         span=SCAN_SPAN if carry is not None else 0, max_count=step.max_count, carry=_ptr(carry),
+                         blocks=_ptr(blocks)))
 
 
 def gated_norm(y, z, weight, parts, eps, out):
@@ -1543,7 +1557,6 @@ def soft_cap(logits, cap):
 
 # --- linear attention with a matrix state -------------------------------------------------------
 
-SCAN_BLOCK = 16       # tokens of a block of the keyed scan (csrc/linear_attention.hip)
 
 
 def scan_blocks(step, heads, dim, vdim):

@@ -141,7 +141,8 @@ class HeadScan(_Recurrent):
         y = step.buffer("scan.y", tokens, inner, "float32")
         K.head_scan(xbc[:, :inner], xbc[:, inner:inner + bc], xbc[:, inner + bc:], fused[:, inner + self.channels:],
                     self.dt_bias, self.A_log, self.D, y, scan_state, step, self.heads, self.vdim, self.state, self.groups,
-                    carry=K.scan_carry(step, self.scan_state, self.heads))
+                    carry=K.scan_carry(step, self.scan_state, self.heads),
+                    blocks=K.head_blocks(step, self.heads, self.vdim, self.state, self.groups))
         gated = step.buffer("scan.gated", tokens, self.inner_cols, step.dtype)
         K.gated_norm(y, fused[:, :inner], self.norm_weight, self.norm_groups, self.eps, gated)
         stream.add_product(step, gated, self.out_weight, packed=self.out_packed)

@@ -1,4 +1,4 @@
-"""The keyed scan in blocks of sixteen tokens on the matrix units, against the recurrence token by token in 64 bits."""
+"""The keyed scan and the scan with one decay a head in blocks of sixteen tokens on the matrix units, against the recurrence token by token in 64 bits."""
 
 import pytest
 import torch
@@ -94,5 +94,49 @@ def test_blocks_of_tokens(form, heads, kv_heads, dim, vdim, lengths, strong):
             got = state_rows(held, heads, dim, vdim).cpu()
             errors[name].append(max(rel_err(got[slot], w) for slot, w in zip(slots, want_state)))
     # a sum of 128 products of 32-bit values and a few hundred decays multiplied one after the other: some 1e-6
+    assert max(errors["blocks"]) < 5e-6, errors
+    assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
+
+
+@pytest.mark.parametrize("heads,groups,vdim,state,lengths,strong", [
+    (4, 1, 64, 128, [33, 1, 16, 47], False), (12, 1, 16, 16, [100, 32, 5], True), (6, 3, 48, 80, [49, 2], False),
+    (9, 1, 32, 48, [400], True), (2, 2, 16, 32, [64, 63, 65], False), (20, 2, 16, 128, [333, 17], False)])
+def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
+    gen = torch.Generator().manual_seed(heads * 1000 + state + len(lengths))
+    inner, bc = heads * vdim, groups * state
+    columns = inner + 2 * bc + heads + 1                                # an odd pitch
+    A_log, bias, D = torch.log(torch.rand(heads, generator=gen) * 7.0 + 1.0), torch.randn(heads, generator=gen) - 2.0, torch.randn(heads, generator=gen)
+    slots = list(reversed(range(len(lengths))))
+    held = torch.zeros(len(lengths), heads * state * vdim + 7, device=DEV)
+    walked = held.clone()
+    want_state = [torch.zeros(heads, state, vdim, dtype=torch.float64) for _ in lengths]
+    errors = {"blocks": [], "walk": []}
+    for part, counts in enumerate([lengths, [n % 40 + 40 for n in lengths]]):
+        rows = torch.randn(sum(counts), columns, generator=gen)
+        if strong:
+            rows[:, inner + 2 * bc:] *= 20.0
+        r, on = rows.double(), rows.to(DEV)
+        spread = lambda v: v.view(-1, groups, state).repeat_interleave(heads // groups, 1)
+        x, B, C = r[:, :inner].view(-1, heads, vdim), spread(r[:, inner:inner + bc]), spread(r[:, inner + bc:inner + 2 * bc])
+        dt = torch.nn.functional.softplus(r[:, inner + 2 * bc:inner + 2 * bc + heads] + bias.double(), threshold=50.0)
+        decay = torch.exp(-torch.exp(A_log.double()) * dt)[..., None].expand(-1, heads, state)
+        step = make_step(torch.float32, counts, starts=[0 if part == 0 else n for n in lengths], slots=slots)
+        want, at = [], 0
+        for s, n in enumerate(counts):
+            here = slice(at, at + n)
+            o, want_state[s] = recurrence(want_state[s], C[here], B[here], dt[here][..., None] * x[here], decay[here], None)
+            want.append((o + D.double()[:, None] * x[here]).reshape(n, inner))
+            at += n
+        want = torch.cat(want)
+        for name, slot_rows, room in (("blocks", held, K.head_blocks(step, heads, vdim, state, groups)), ("walk", walked, None)):
+            y = torch.full((sum(counts), inner + 2), float("nan"), device=DEV)
+            if room is not None:
+                room.fill_(float("nan"))
+            K.head_scan(on[:, :inner], on[:, inner:inner + bc], on[:, inner + bc:inner + 2 * bc], on[:, inner + 2 * bc:], bias.to(DEV), A_log.to(DEV),
+                        D.to(DEV), y, slot_rows, step, heads, vdim, state, groups, blocks=room)
+            assert bool(torch.isnan(y[:, inner:]).all())
+            errors[name].append(rel_err(y[:, :inner].cpu(), want))
+            got = state_rows(slot_rows, heads, state, vdim).cpu()
+            errors[name].append(max(rel_err(got[slot], w) for slot, w in zip(slots, want_state)))
     assert max(errors["blocks"]) < 5e-6, errors
     assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
