@@ -77,13 +77,13 @@ static int simd_count() {
 
 // Into spans of how many tokens a step's long sequences are cut, 0 for not at all.  Spans double the
 // arithmetic, so they pay only while whole sequences leave the chip short of waves: `waves` (those that
-// walk whole sequences) must be at most `fill` to a SIMD, and there are as many spans as bring four
-// times that, none shorter than the call's `span`, which its room for the spans' states was sized
+// walk whole sequences) must be at most `fill` to a SIMD, and there are as many spans as bring `times`
+// that, none shorter than the call's `span`, which its room for the spans' states was sized
 // for.  Measured for 2 x 1,024 tokens (us, whole / cut): the head scan with one wave to a SIMD 309 / 205,
 // with two 327 / 380; the selective scan with half a wave to a SIMD 334 / 176, with one 369 / 311.
-static int span_tokens(int span, int max_count, const float* carry, int64_t waves, int fill) {
+static int span_tokens(int span, int max_count, const float* carry, int64_t waves, int fill, int times = 4) {
   if (span <= 0 || !carry || waves > (int64_t)fill * simd_count()) return 0;
-  const int64_t wanted = 4 * (int64_t)fill * simd_count() / waves;
+  const int64_t wanted = times * (int64_t)fill * simd_count() / waves;
   int tokens = (int)((max_count + wanted - 1) / wanted);
   if (tokens < span) tokens = span;
   return max_count >= MIN_SPANS * tokens ? tokens : 0;

@@ -390,6 +390,126 @@ __global__ void __launch_bounds__(64) selective_scan_kernel(SelectiveScanCall c,
       for (int col = c.channels + lane; col < c.out_cols; col += 64) out[(int64_t)t * c.ld_out + col] = from_float<T>(0.f);
 }
 
+// The same with a lane a channel, for steps of many tokens: all N state elements of a channel lie in one lane's registers, so
+// nothing crosses lanes, and a token's B and C, the same for all channels, come through scalar loads (the instructions take
+// them as they are).  What is left is the recurrence's own arithmetic: an exponential and seven operations a state element
+// and token, 48 of the 54 cycles that a wave takes for them on its SIMD.  dt, x and z of the next SL_AHEAD tokens are on
+// their way meanwhile.
+//   exp(v), v = dt A <= 0, to the accuracy of expf: t = round(v / ln 2), then 2^t (1 + (v - t ln 2)); the factor makes up for
+//   the rounding of t, which the hardware's exponential would otherwise carry into the decay.
+#define SL_AHEAD 4
+// Taken by steps whose longest sequence brings SL_MIN_TOKENS tokens, or a quarter of that where a wave for every 64 channels of
+// every sequence makes SL_MIN_WAVES; smaller steps have more waves with eight lanes a channel.  Measured (us, eight lanes / one; 2,048
+// channels of 16): 2 x 32 tokens 14.7 / 18.0, 4 x 48 21.0 / 23.6, 2 x 64 25.8 / 22.5, 16 x 20 25.9 / 13.9, 2 x 256 60.6 / 31.2, 8 x 300 208 / 80,
+// 2 x 1,024 181 / 73 (of which 46 are the recurrence, gone through twice, and 8 the carry).
+#define SL_MIN_TOKENS 64
+#define SL_MIN_WAVES 256
+
+__device__ __forceinline__ float decay_of(float v) {
+  const float t = v * 1.44269504088896f;
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, fmaf(-t, 0.693147180559945f, v), e);
+}
+
+template <typename T, int N, int PHASE>
+__global__ void __launch_bounds__(64) selective_lanes_kernel(SelectiveScanCall c) {
+  typedef const __attribute__((address_space(4))) float* Uniform;
+  const int lane = threadIdx.x, ch = blockIdx.x * 64 + lane, seq = blockIdx.y, part = blockIdx.z;
+  const bool live = ch < c.channels;
+  const int chs = live ? ch : c.channels - 1;        // idle lanes read a valid channel and write nothing
+  int first = c.seq_off[seq], last = c.seq_off[seq + 1];
+  const int64_t per_span = (int64_t)c.channels * c.state + c.channels;
+  float* mine = nullptr;                             // this span's block of the carry
+  if (PHASE) {
+    first += part * c.span;
+    if (first >= last) return;
+    last = min(first + c.span, last);
+    mine = c.carry + span_block(c.seq_off, seq, c.span, part) * per_span;
+  }
+  if (first >= last) return;
+  float* held = c.S + (int64_t)c.slots[seq] * c.state_stride + (int64_t)chs * N;
+  const float* start = PHASE == 3 ? mine - per_span + (int64_t)chs * N : held;
+  float A[N], S[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    A[n] = fmaxf(-expf(c.A_log[(int64_t)chs * N + n]), -1e8f);
+    S[n] = PHASE != 1 ? start[n] : 0.f;
+  }
+  const float Dc = c.D[chs];
+  T* out = static_cast<T*>(c.out) + (int64_t)first * c.ld_out + chs;
+  const float *dt_at = c.dt + (int64_t)first * c.ld_dt + chs, *x_at = c.x + (int64_t)first * c.ld_x + chs, *z_at = c.z + (int64_t)first * c.ld_z + chs;
+  const float *b_at = c.B + (int64_t)first * c.ld_bc, *c_at = c.C + (int64_t)first * c.ld_bc;
+  const int count = last - first;
+  float dts[SL_AHEAD], xs[SL_AHEAD], zs[SL_AHEAD], dt_sum = 0.f;
+  auto fetch = [&](int t, int u) {                   // (behind the end the last token again, which is not used)
+    const int64_t i = min(t, count - 1);
+    dts[u] = dt_at[i * c.ld_dt];
+    xs[u] = x_at[i * c.ld_x];
+    if (PHASE != 1) zs[u] = z_at[i * c.ld_z];
+  };
+  // a token's B and C are asked for while the token before is worked on (scalar registers: one wait a token, not two)
+  float b[N], q[N];
+  auto fetch_row = [&](int t, float* b_to, float* q_to) {
+    const int64_t i = (int64_t)min(t, count - 1) * c.ld_bc;
+    const Uniform from_b = (Uniform)(b_at + i), from_q = (Uniform)(c_at + i);
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      b_to[n] = from_b[n];
+      if (PHASE != 1) q_to[n] = from_q[n];
+    }
+  };
+  auto token = [&](int t, int u) {
+    const float dt = dts[u], xv = xs[u], z = PHASE != 1 ? zs[u] : 0.f;
+    float b_next[N], q_next[N];
+    fetch_row(t + 1, b_next, q_next);
+    fetch(t + SL_AHEAD, u);
+    __builtin_amdgcn_sched_barrier(0);
+    const float step = fminf(dt, 1e30f), dx = dt * xv;               // (an infinite step: the decay is zero, not undefined)
+    float acc = 0.f, acc_odd = 0.f;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      S[n] = fmaf(decay_of(step * A[n]), S[n], dx * b[n]);
+      if (PHASE != 1) {
+        if (n & 1) acc_odd = fmaf(S[n], q[n], acc_odd);
+        else acc = fmaf(S[n], q[n], acc);
+      }
+    }
+    if (PHASE == 1) dt_sum += dt;
+    else if (live) out[(int64_t)t * c.ld_out] = from_float<T>((acc + acc_odd + Dc * xv) * silu_f(z));
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      b[n] = b_next[n];
+      if (PHASE != 1) q[n] = q_next[n];
+    }
+  };
+  fetch_row(0, b, q);
+#pragma unroll
+  for (int u = 0; u < SL_AHEAD; ++u) fetch(u, u);
+  int t = 0;
+  for (; t + SL_AHEAD <= count; t += SL_AHEAD)
+#pragma unroll
+    for (int u = 0; u < SL_AHEAD; ++u) token(t + u, u);
+#pragma unroll
+  for (int u = 0; u < SL_AHEAD - 1; ++u)
+    if (t + u < count) token(t + u, u);
+  if (PHASE == 1) {
+    if (live) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) mine[(int64_t)ch * N + n] = S[n];
+      mine[(int64_t)c.channels * c.state + ch] = dt_sum;
+    }
+    return;
+  }
+  if (PHASE == 0 && live) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) held[n] = S[n];
+  }
+  // the columns behind the last channel, which the next product reads as zeros
+  if (blockIdx.x == 0)
+    for (int i = first; i < last; ++i)
+      for (int col = c.channels + lane; col < c.out_cols; col += 64) static_cast<T*>(c.out)[(int64_t)i * c.ld_out + col] = from_float<T>(0.f);
+}
+
 // C_k = exp(A * sum of dt of span k) * C_(k-1) + E_k along every sequence, in place; C_(-1), the state the
 // sequence came with, is kept in front of its spans, and the last C goes into the slot.
 __global__ void __launch_bounds__(256) selective_carry_kernel(SelectiveScanCall c) {
@@ -434,8 +554,32 @@ static void launch_selective_scan_r(hipStream_t stream, const SelectiveScanCall&
   hipLaunchKernelGGL((selective_scan_kernel<T, R>), grid, block, (size_t)chunk * per_token * sizeof(float), stream, c, chunk, 0);
 }
 
+template <typename T, int N>
+static void launch_selective_lanes(hipStream_t stream, const SelectiveScanCall& c) {
+  const int groups = (c.channels + 63) / 64;
+  const int span = span_tokens(c.span, c.max_count, c.carry, (int64_t)groups * c.n_seqs, 1, 2);
+  if (span > 0 && (c.max_count + span - 1) / span <= 65535) {
+    SelectiveScanCall cut = c;
+    cut.span = span;
+    dim3 grid(groups, c.n_seqs, (c.max_count + span - 1) / span);
+    hipLaunchKernelGGL((selective_lanes_kernel<T, N, 1>), grid, dim3(64), 0, stream, cut);
+    hipLaunchKernelGGL(selective_carry_kernel, dim3((c.channels * c.state + 255) / 256, c.n_seqs), dim3(256), 0, stream, cut);
+    hipLaunchKernelGGL((selective_lanes_kernel<T, N, 3>), grid, dim3(64), 0, stream, cut);
+    return;
+  }
+  hipLaunchKernelGGL((selective_lanes_kernel<T, N, 0>), dim3(groups, c.n_seqs), dim3(64), 0, stream, c);
+}
+
 template <typename T>
 static int launch_selective_scan(hipStream_t stream, const SelectiveScanCall& c) {
+  const bool many = c.max_count >= SL_MIN_TOKENS ||
+      (c.max_count >= SL_MIN_TOKENS / 4 && (int64_t)((c.channels + 63) / 64) * c.n_seqs >= SL_MIN_WAVES);
+  if (many && (c.state == 8 || c.state == 16 || c.state == 32)) {
+    if (c.state == 8) launch_selective_lanes<T, 8>(stream, c);
+    else if (c.state == 16) launch_selective_lanes<T, 16>(stream, c);
+    else launch_selective_lanes<T, 32>(stream, c);
+    return bt_check_launch("selective_scan");
+  }
   const int per = (c.state + 7) / 8;
   if (per <= 1) launch_selective_scan_r<T, 1>(stream, c);
   else if (per <= 2) launch_selective_scan_r<T, 2>(stream, c);

@@ -1316,21 +1316,26 @@ def dt_project(low, weight, bias, out, act="softplus"):
 SCAN_SPAN = 64        # tokens of a span of a long sequence (sequences of three spans or more are cut); 0: never cut
 
 
-def scan_carry(step, state_floats, extra_floats):
+def scan_carry(step, state_floats, extra_floats, span=None):
     """Room for the states of the spans a step's long sequences are cut into (csrc/state_space.hip,
     "Spans"): one block a span and one more a sequence; at most tokens / span + sequences spans exist
-    in a step of any shape of its class.  None for steps that are too short to be cut."""
-    if not SCAN_SPAN or step.token_capacity < 3 * SCAN_SPAN or step.max_count <= 1:
+    in a step of any shape of its class.  None for steps that are too short to be cut.  ``span``: tokens of a span
+    where that is not ``SCAN_SPAN``."""
+    span = SCAN_SPAN if span is None else span
+    if not SCAN_SPAN or step.token_capacity < 3 * span or step.max_count <= 1:
         return None
-    blocks = step.token_capacity // SCAN_SPAN + 2 * step.n_seqs + 2
+    blocks = step.token_capacity // span + 2 * step.n_seqs + 2
     return step.buffer("scan.carry", blocks, state_floats + extra_floats, "float32")
 
 
-def selective_scan(x, z, dt, B, C, A_log, D, out, state, step, carry=None):
+SELECTIVE_SPAN = 16   # ... and of the selective scan's with a channel a lane
+
+
+def selective_scan(x, z, dt, B, C, A_log, D, out, state, step, carry=None, span=None):
     """The selective scan with one state row per channel (see csrc/state_space.hip), gated by
     silu(z); ``state`` [slots, >= channels * state elements] float32 is read and left updated.
     ``carry``: room from ``scan_carry`` (channels * elements state floats, channels extra); with it
-    long sequences are scanned in spans side by side."""
+    long sequences are scanned in spans side by side, of at least ``span`` tokens (what the room was made for)."""
     channels, elements = A_log.shape
     _launch(_module("state_space"), "bt_selective_scan_call",
             SelectiveScanCall(out_dtype=DTYPE_CODES[out.dtype], tokens=x.shape[0], n_seqs=step.n_seqs, channels=channels,
@@ -1339,7 +1344,7 @@ def selective_scan(x, z, dt, B, C, A_log, D, out, state, step, carry=None):
                               ld_bc=B.stride(0), A_log=A_log.data_ptr(), D=D.data_ptr(), out=out.data_ptr(),
                               ld_out=out.stride(0), S=state.data_ptr(), state_stride=state.stride(0),
                               seq_off=step.seq_off.data_ptr(), slots=step.slots.data_ptr(),
-                              span=SCAN_SPAN if carry is not None else 0, max_count=step.max_count, carry=_ptr(carry)))
+                              span=(span or SCAN_SPAN) if carry is not None else 0, max_count=step.max_count, carry=_ptr(carry)))
 
 
 SCAN_BLOCK = 16       # tokens of a block of the scans that go in blocks (csrc/linear_attention.hip, csrc/state_space.hip)

@@ -94,7 +94,7 @@ class SelectiveScan(_Recurrent):
         gated = step.buffer("scan.gated", tokens, self.inner_cols, step.dtype)
         K.selective_scan(x, xz[:, inner:], dt, low[:, self.dt_rank:self.dt_rank + self.state],
                          low[:, self.dt_rank + self.state:], self.A_log, self.D, gated, scan_state, step,
-                         carry=K.scan_carry(step, self.scan_state, inner))
+                         carry=K.scan_carry(step, self.scan_state, inner, K.SELECTIVE_SPAN), span=K.SELECTIVE_SPAN)
         stream.add_product(step, gated, self.out_weight, packed=self.out_packed)
 
 

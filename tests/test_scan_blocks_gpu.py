@@ -1,4 +1,4 @@
-"""The keyed scan and the scan with one decay a head in blocks of sixteen tokens on the matrix units, against the recurrence token by token in 64 bits."""
+"""The selective scan with a channel a lane, the keyed scan and the scan with one decay a head in blocks of sixteen tokens on the matrix units, against the recurrence token by token in 64 bits."""
 
 import pytest
 import torch
@@ -140,3 +140,44 @@ def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
             errors[name].append(max(rel_err(got[slot], w) for slot, w in zip(slots, want_state)))
     assert max(errors["blocks"]) < 5e-6, errors
     assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
+
+
+# channels that do not fill a wave, all sizes of state that lanes take, steps on both sides of the rule, spans that end
+# within a sequence, a second portion from a state that is not zero; `strong`: steps so long that decays vanish
+@pytest.mark.parametrize("channels,state,lengths,spans,strong", [
+    (100, 16, [64, 1, 130], True, False), (64, 8, [65, 63], False, True), (200, 32, [300, 17, 64], True, False), (70, 16, [500], True, True),
+    (1100, 16, [20] * 16, True, False), (48, 16, [63, 5], True, False)])
+def test_channels_in_lanes(channels, state, lengths, spans, strong):
+    gen = torch.Generator().manual_seed(channels + state + len(lengths))
+    A_log, D = torch.log(torch.rand(channels, state, generator=gen) * 7.0 + 0.5), torch.randn(channels, generator=gen)
+    A = -torch.exp(A_log.double())
+    slots = list(reversed(range(len(lengths))))
+    held = torch.zeros(len(lengths), channels * state + 3, device=DEV)
+    want_state = [torch.zeros(channels, state, dtype=torch.float64) for _ in lengths]
+    for part, counts in enumerate([lengths, [n % 40 + 40 for n in lengths]]):
+        total = sum(counts)
+        rows = torch.randn(total, 3 * channels + 2 * state + 1, generator=gen)
+        x, z, raw, B, C = rows.split([channels, channels, channels, state, state + 1], 1)
+        dt = torch.nn.functional.softplus(raw * (20.0 if strong else 1.0) - 2.0)
+        if strong:
+            dt[5], x[5] = 1e30, 0.0                                     # an endless step that writes nothing leaves nothing behind
+        step = make_step(torch.float32, counts, starts=[0 if part == 0 else n for n in lengths], slots=slots)
+        want, at = torch.zeros(total, channels, dtype=torch.float64), 0
+        for s, n in enumerate(counts):
+            S = want_state[s]
+            for t in range(at, at + n):
+                S = torch.exp(dt[t].double()[:, None] * A) * S + (dt[t] * x[t]).double()[:, None] * B[t].double()
+                zt = z[t].double()
+                want[t] = ((S * C[t, :state].double()).sum(1) + D.double() * x[t].double()) * zt * torch.sigmoid(zt)
+            want_state[s], at = S, at + n
+        out = torch.full((total, channels + 6), float("nan"), device=DEV)
+        carry = K.scan_carry(step, channels * state, channels, K.SELECTIVE_SPAN) if spans else None
+        on = lambda v: v.contiguous().to(DEV)
+        bc = on(torch.cat([B, C], 1))
+        K.selective_scan(on(x), on(z), on(dt), bc[:, :state], bc[:, state:2 * state], A_log.to(DEV), D.to(DEV), out, held, step, carry=carry,
+                         span=K.SELECTIVE_SPAN)
+        assert bool((out[:, channels:] == 0).all())
+        # an exponential and a handful of roundings a token, of decays that sum to at most 1 / (1 - decay) tokens' worth
+        assert rel_err(out[:, :channels].cpu(), want) < 3e-6
+        for slot, w in zip(slots, want_state):
+            assert rel_err(held[slot, :channels * state].view(channels, state).cpu(), w) < 3e-6
