@@ -109,6 +109,78 @@ __global__ void __launch_bounds__(256) causal_conv_kernel(CausalConvCall c) {
   }
 }
 
+// The same for steps of many tokens: a thread takes a channel of CONV_RUN tokens one after the other, so that an input is read
+// once and not once a tap, the taps stay in registers and all of a run's inputs are on their way together; a run that
+// begins a sequence takes its window's front from the state, one that straddles two goes token by token.  Sums are taken in
+// the same order as above.  Measured with the state's kernel (us, a token a thread / in runs; channels of 4 taps): 2,048 tokens of 2,048
+// 28.4 / 12.4 (the bytes: 6.9), 2 x 256 of 2,048 9.3 / 5.9, 16 x 40 11.2 / 6.8, 3 x 100 of 1,536 6.6 / 7.4; runs of 16 17.2.
+#define CONV_RUN 8
+#define CONV_MIN_TOKENS 384
+
+template <typename T, int TAPS>
+__global__ void __launch_bounds__(256) causal_conv_run_kernel(CausalConvCall c) {
+  const int t0 = blockIdx.x * CONV_RUN, ch = blockIdx.y * blockDim.x + threadIdx.x;
+  const int count = min(CONV_RUN, c.tokens - t0);
+  T* cast = static_cast<T*>(c.cast);
+  if (ch >= c.channels) {
+    if (cast && ch < c.cast_cols)
+      for (int i = 0; i < count; ++i) cast[(int64_t)(t0 + i) * c.ld_cast + ch] = from_float<T>(0.f);
+    return;
+  }
+  float w[TAPS];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) w[j] = c.weight[(int64_t)ch * TAPS + j];
+  const float bias = c.bias ? c.bias[ch] : 0.f;
+  const float* in = c.in + (int64_t)t0 * c.ld_in + ch;
+  float* out = c.out + (int64_t)t0 * c.ld_out + ch;
+  // most runs are whole and lie in one sequence: no token of theirs asks where it stands
+  const int seq0 = c.tok_seq[t0];
+  if (count == CONV_RUN && seq0 == c.tok_seq[t0 + CONV_RUN - 1]) {
+    const int before = t0 - c.seq_off[seq0];                // tokens of the sequence in front of the run
+    const float* held = c.state + (int64_t)c.slots[seq0] * c.state_stride + ch;
+    float u[CONV_RUN + TAPS - 1];
+#pragma unroll
+    for (int i = 0; i < CONV_RUN + TAPS - 1; ++i) {
+      const int src = before + i - (TAPS - 1);
+      u[i] = *(i >= TAPS - 1 || src >= 0 ? in + (int64_t)(i - (TAPS - 1)) * c.ld_in : held + (int64_t)(TAPS - 1 + src) * c.channels);
+    }
+#pragma unroll
+    for (int i = 0; i < CONV_RUN; ++i) {
+      float sum = bias;
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) sum = fmaf(w[j], u[i + j], sum);
+      const float y = c.act == 0 ? silu_f(sum) : sum;
+      out[(int64_t)i * c.ld_out] = y;
+      if (cast) cast[(int64_t)(t0 + i) * c.ld_cast + ch] = from_float<T>(y);
+    }
+    return;
+  }
+  for (int i = 0; i < count; ++i) {
+    const int t = t0 + i, seq = c.tok_seq[t], local = t - c.seq_off[seq];
+    const float* held = c.state + (int64_t)c.slots[seq] * c.state_stride;
+    float sum = bias;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+      const int back = TAPS - 1 - j, src = local - back;
+      sum = fmaf(w[j], src >= 0 ? in[(int64_t)(i - back) * c.ld_in] : held[(int64_t)(TAPS - 1 + src) * c.channels + ch], sum);
+    }
+    const float y = c.act == 0 ? silu_f(sum) : sum;
+    out[(int64_t)i * c.ld_out] = y;
+    if (cast) cast[(int64_t)t * c.ld_cast + ch] = from_float<T>(y);
+  }
+}
+
+template <typename T>
+static bool launch_conv_run(hipStream_t stream, const CausalConvCall& c, int cols) {
+  dim3 grid((c.tokens + CONV_RUN - 1) / CONV_RUN, (cols + 255) / 256), block(256);
+  switch (c.taps) {
+    case 2: hipLaunchKernelGGL((causal_conv_run_kernel<T, 2>), grid, block, 0, stream, c); return true;
+    case 3: hipLaunchKernelGGL((causal_conv_run_kernel<T, 3>), grid, block, 0, stream, c); return true;
+    case 4: hipLaunchKernelGGL((causal_conv_run_kernel<T, 4>), grid, block, 0, stream, c); return true;
+  }
+  return false;
+}
+
 // After the convolution: the state becomes the last taps - 1 inputs of each sequence.
 __global__ void __launch_bounds__(256) conv_state_kernel(CausalConvCall c) {
   const int seq = blockIdx.x;
@@ -145,7 +217,10 @@ BT_EXPORT int bt_causal_conv_call(void* stream, const CausalConvCall* c) {
       hipLaunchKernelGGL((causal_conv_kernel<bf16_t, true>), grid, block, 0, (hipStream_t)stream, *c);
     return bt_check_launch("causal_conv");
   }
-  if (c->cast_dtype == 0)
+  const bool run = c->tokens >= CONV_MIN_TOKENS && (c->cast_dtype == 0 ? launch_conv_run<float>((hipStream_t)stream, *c, cols)
+                                                                      : launch_conv_run<bf16_t>((hipStream_t)stream, *c, cols));
+  if (run) {
+  } else if (c->cast_dtype == 0)
     hipLaunchKernelGGL((causal_conv_kernel<float, false>), grid, block, 0, (hipStream_t)stream, *c);
   else
     hipLaunchKernelGGL((causal_conv_kernel<bf16_t, false>), grid, block, 0, (hipStream_t)stream, *c);
