@@ -42,6 +42,7 @@ struct RouteCall {
   int group_rank;           // a group's score is the sum of its so many best (corrected) scores; 0 or 1: its best
   int normalize;            // 1: the chosen experts' scores over their sum; 0: the scores as they are
   const float* bias;        // [experts] or null: added to the logits
+  unsigned long long* used; // [tokens] or null: bit e of a token's word is set where its weight of expert e < 64 is not zero
 };
 
 // The best (value, index) of a wave; among equal values the lowest index.  Every lane gets it.
@@ -221,8 +222,102 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
   const float inverse = route_choice(c, early, score, choice);
   // the one store of a lane's experts: the chosen ones' scores over their sum, zero elsewhere
   float* weights = c.weights + (int64_t)t * c.experts;
-  for (int e = lane; e < c.experts; e += 64) weights[e] = choice[e] == INFINITY ? score[e] * inverse : 0.f;
+  for (int e = lane; e < c.experts; e += 64) {
+    const float w = choice[e] == INFINITY ? score[e] * inverse : 0.f;
+    weights[e] = w;
+    if (e < 64 && c.used) {
+      const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
+      if (lane == 0) c.used[t] = used;
+    }
+  }
   if (c.gate_w && lane == 0) c.gate[t] = 1.0f / (1.0f + expf(-gate_sum));
+}
+
+// The same for steps of many tokens: a work-group takes sixteen tokens, whose logits are a product of 16 rows by the router's
+// outputs on the matrix units (v_mfma_f32_16x16x4_f32: h widened, the router's 32 bits as they are), its sixteen waves a
+// sixteenth of the columns each, so that the router is read once for sixteen tokens and not once a token; then every
+// wave makes the choice of one of them.  Of an instruction's four K values step i takes column 4 g + i of a lane group's
+// four, which are one read.  A work-group's own chain (two trips to memory, the sums' meeting, the choice) is 8 us whatever
+// the step, so steps of fewer than ROUTE_ROWS_MIN tokens keep a work-group a token.  Measured in a step (us, a work-group a token /
+// sixteen): 1,809 tokens of 1,024 columns, 9 outputs and a gate 15.3 / 10.7, 2,447 of 8 outputs 11.0 / 8.8; alone, 1,024 tokens 6.7 /
+// 8.3, 2,048 10.0 / 8.6, 4,096 15.1 / 8.7.
+#define ROUTE_ROWS 16
+#define ROUTE_ROWS_TILES 2      // (most outputs: 32)
+#define ROUTE_ROWS_AHEAD 4      // chunks of 16 columns on their way
+
+template <typename T, int TILES>
+__global__ void __launch_bounds__(64 * ROUTE_ROWS) route_rows_kernel(RouteCall c) {
+  typedef __attribute__((__vector_size__(4 * sizeof(T)))) T T4;
+  __shared__ __attribute__((aligned(16))) floatx4 parts[ROUTE_ROWS][TILES][64];
+  __shared__ float score[ROUTE_ROWS][16 * TILES], choice[ROUTE_ROWS][16 * TILES];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
+  const int t0 = blockIdx.x * ROUTE_ROWS, outputs = c.experts + (c.gate_w ? 1 : 0);
+  const T* h = static_cast<const T*>(c.h) + (int64_t)min(t0 + n, c.tokens - 1) * c.ldh + 4 * g;
+  const float* rows[TILES];                          // an output beyond the last reads the last one's row and is dropped
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) {
+    const int e = min(16 * j + n, outputs - 1);
+    rows[j] = (e < c.experts ? c.W + (int64_t)e * c.width : c.gate_w) + 4 * g;
+  }
+  RouteEarly early;
+  early.load(c);
+  floatx4 sums[TILES];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) sums[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int chunks = c.width / 16;
+  for (int k0 = wave; k0 < chunks; k0 += ROUTE_ROWS * ROUTE_ROWS_AHEAD) {
+    T4 xs[ROUTE_ROWS_AHEAD];
+    floatx4 ws[ROUTE_ROWS_AHEAD][TILES];
+#pragma unroll
+    for (int u = 0; u < ROUTE_ROWS_AHEAD; ++u) {
+      const int col = 16 * min(k0 + ROUTE_ROWS * u, chunks - 1);
+      xs[u] = *reinterpret_cast<const T4*>(h + col);
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) ws[u][j] = *reinterpret_cast<const floatx4*>(rows[j] + col);
+    }
+#pragma unroll
+    for (int u = 0; u < ROUTE_ROWS_AHEAD; ++u) {
+      if (k0 + ROUTE_ROWS * u >= chunks) break;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) sums[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_float(xs[u][i]), ws[u][j][i], sums[j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) parts[wave][j][lane] = sums[j];        // lane holds tokens 4 g + i, output n
+  __syncthreads();
+  for (int k = tid; k < ROUTE_ROWS * 16 * TILES; k += 64 * ROUTE_ROWS) {
+    const int t = k / (16 * TILES), e = k % (16 * TILES), from = 16 * (t >> 2) + (e & 15);
+    float logit = 0.f;
+#pragma unroll
+    for (int w = 0; w < ROUTE_ROWS; ++w) logit += reinterpret_cast<const float*>(&parts[w][e >> 4][from])[t & 3];
+    score[t][e] = logit;
+  }
+  __syncthreads();
+  const int t = t0 + wave;
+  if (t >= c.tokens) return;
+  const float gate_sum = score[wave][c.gate_w ? c.experts : 0];
+  const float inverse = route_choice(c, early, score[wave], choice[wave]);
+  const float w = lane < c.experts && choice[wave][lane] == INFINITY ? score[wave][lane] * inverse : 0.f;
+  if (lane < c.experts) c.weights[(int64_t)t * c.experts + lane] = w;
+  const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
+  if (lane == 0 && c.used) c.used[t] = used;
+  if (lane == 0 && c.gate_w) c.gate[t] = 1.0f / (1.0f + expf(-gate_sum));
+}
+
+#define ROUTE_ROWS_MIN 1536
+
+template <typename T>
+static bool launch_route_rows(hipStream_t stream, const RouteCall& c) {
+  const int outputs = c.experts + (c.gate_w ? 1 : 0), tiles = (outputs + 15) / 16;
+  if (c.tokens < ROUTE_ROWS_MIN || tiles > ROUTE_ROWS_TILES || c.width % 16 != 0 || c.ldh % 4 != 0 || ((uintptr_t)c.h & (4 * sizeof(T) - 1)) ||
+      (((uintptr_t)c.W | (uintptr_t)c.gate_w) & 15))
+    return false;
+  dim3 grid((c.tokens + ROUTE_ROWS - 1) / ROUTE_ROWS), block(64 * ROUTE_ROWS);
+  if (tiles == 1) hipLaunchKernelGGL((route_rows_kernel<T, 1>), grid, block, 0, stream, c);
+  else hipLaunchKernelGGL((route_rows_kernel<T, 2>), grid, block, 0, stream, c);
+  return true;
 }
 
 static const char* route_refusal(const RouteCall* c) {
@@ -244,6 +339,8 @@ BT_EXPORT int bt_route_call(void* stream, const RouteCall* c) {
     BT_REFUSE("route: %d of %d experts a token, %d of %d groups, score %d: %s", c->top, c->experts, c->keep, c->groups, c->score, wrong);
   if (c->width <= 0) BT_REFUSE("route: width %d must be positive", c->width);
   if (!c->h || !c->W || !c->weights || (c->gate_w && !c->gate)) BT_REFUSE("route: missing operand");
+  if (c->dtype == 0 ? launch_route_rows<float>((hipStream_t)stream, *c) : launch_route_rows<bf16_t>((hipStream_t)stream, *c))
+    return bt_check_launch("route");
   // (measured at 2,048 tokens of width 2,048: 32 us with sixteen waves a token, 18 with four)
   dim3 grid(c->tokens), block(c->tokens <= 256 ? ROUTE_THREADS : 256);
   if (c->dtype == 0)
@@ -419,6 +516,7 @@ struct GroupExpertsCall {
   int top;
   int width;
   const float* weights;     // [tokens][experts + identity]
+  const unsigned long long* used;   // [tokens], as route leaves it
   int* rows;                // [experts][pitch]: the tokens that use an expert, in order
   int64_t pitch;
   int* counts;              // [experts]
@@ -438,13 +536,9 @@ __global__ void __launch_bounds__(1024) group_experts_kernel(GroupExpertsCall c)
     int base = 0;
     for (int t0 = 0; t0 < c.tokens; t0 += 1024) {
       const int t = t0 + threadIdx.x;
-      const float* w = c.weights + (int64_t)(t < c.tokens ? t : 0) * outputs;
-      bool mine = false;
-      int place = 0;
-      if (t < c.tokens) {
-        mine = w[e] != 0.f;
-        for (int i = 0; i < e; ++i) place += w[i] != 0.f ? 1 : 0;
-      }
+      const unsigned long long word = t < c.tokens ? c.used[t] : 0;
+      const bool mine = word >> e & 1;
+      const int place = __builtin_popcountll(word & ((1ull << e) - 1));
       const unsigned long long all = __builtin_amdgcn_ballot_w64(mine);
       if (lane == 0) found[wave] = __builtin_popcountll(all);
       __syncthreads();
@@ -462,9 +556,9 @@ __global__ void __launch_bounds__(1024) group_experts_kernel(GroupExpertsCall c)
   }
   const int t = ((int)blockIdx.x - c.experts) * 16 + wave;              // a wave a token
   if (t >= c.tokens) return;
-  const float* w = c.weights + (int64_t)t * outputs;
-  const int used = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < c.experts && w[lane < c.experts ? lane : 0] != 0.f));
+  const int used = __builtin_popcountll(c.used[t] & (~0ull >> (64 - c.experts)));
   if (used >= c.top) return;
+  const float* w = c.weights + (int64_t)t * outputs;
   float own = 0.f;
   for (int i = 0; i < c.identity; ++i) own += w[c.experts + i];
   const T* h = static_cast<const T*>(c.h) + (int64_t)t * c.ldh;
@@ -479,7 +573,7 @@ BT_EXPORT int bt_group_experts_call(void* stream, const GroupExpertsCall* c) {
   if (c->experts <= 0 || c->experts > GROUP_MAX_EXPERTS || c->identity < 0 || c->top <= 0 || c->top > 64 || c->width <= 0)
     BT_REFUSE("group_experts: %d experts (1..%d), %d identity experts, %d a token", c->experts, GROUP_MAX_EXPERTS, c->identity, c->top);
   if (c->tokens >= 1 << GROUP_PLACE_BITS) BT_REFUSE("group_experts: %d tokens are too many", c->tokens);
-  if (!c->weights || !c->rows || !c->counts || !c->h || !c->out || c->pitch < c->tokens || c->ldh < c->width || c->ld_out < c->width)
+  if (!c->weights || !c->used || !c->rows || !c->counts || !c->h || !c->out || c->pitch < c->tokens || c->ldh < c->width || c->ld_out < c->width)
     BT_REFUSE("group_experts: missing operand or rows too short");
   dim3 grid(c->experts + (c->tokens + 15) / 16), block(1024);
   if (c->dtype == 0)

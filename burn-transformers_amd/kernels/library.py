@@ -205,13 +205,13 @@ class RouteCall(ctypes.Structure):
     _fields_ = [("dtype", _c_int), ("tokens", _c_int), ("width", _c_int), ("experts", _c_int), ("top", _c_int),
                 ("groups", _c_int), ("keep", _c_int), ("h", _c_ptr), ("ldh", _c_i64), ("W", _c_ptr),
                 ("correction", _c_ptr), ("gate_w", _c_ptr), ("weights", _c_ptr), ("gate", _c_ptr), ("score", _c_int),
-                ("group_rank", _c_int), ("normalize", _c_int), ("bias", _c_ptr)]
+                ("group_rank", _c_int), ("normalize", _c_int), ("bias", _c_ptr), ("used", _c_ptr)]
     _step_fields_ = {"tokens": "tokens"}
 
 
 class GroupExpertsCall(ctypes.Structure):
     _fields_ = [("dtype", _c_int), ("tokens", _c_int), ("experts", _c_int), ("identity", _c_int), ("top", _c_int), ("width", _c_int),
-                ("weights", _c_ptr), ("rows", _c_ptr), ("pitch", _c_i64), ("counts", _c_ptr), ("h", _c_ptr), ("ldh", _c_i64),
+                ("weights", _c_ptr), ("used", _c_ptr), ("rows", _c_ptr), ("pitch", _c_i64), ("counts", _c_ptr), ("h", _c_ptr), ("ldh", _c_i64),
                 ("out", _c_ptr), ("plane", _c_i64), ("ld_out", _c_i64)]
     _step_fields_ = {"tokens": "tokens"}
 
@@ -1427,7 +1427,7 @@ def differential(rows, heads, vdim, pitch, weight, post, eps, out):
 # --- routed feed-forward ----------------------------------------------------------------------
 
 def route(h, router, correction, top, groups, keep, weights, gate_weight=None, gate=None, score="softmax",
-          group_rank=1, normalize=True, bias=None):
+          group_rank=1, normalize=True, bias=None, used=None):
     """Per row of ``h``: softmax of the float32 router's logits over all experts, the ``top`` experts
     with the largest score + ``correction`` among the best ``keep`` of ``groups`` equal groups (groups
     <= 1: among all), and into ``weights`` [rows, experts] the chosen experts' scores divided by their
@@ -1435,13 +1435,13 @@ def route(h, router, correction, top, groups, keep, weights, gate_weight=None, g
     ``score`` "sigmoid": each logit's sigmoid instead of the softmax; ``group_rank`` n: a group's score is the
     sum of its n best; ``normalize`` False: the chosen experts' scores as they are.  ``score`` "chosen": the choice is made
     by logit + ``correction``, the weights are the softmax over the chosen logits alone.  ``bias`` ([experts] float32):
-    added to the logits."""
+    added to the logits.  ``used`` (int64 [rows]): bit e of a row's word is set where its weight of expert e < 64 is not zero."""
     _launch(_module("experts"), "bt_route_call",
             RouteCall(dtype=DTYPE_CODES[h.dtype], tokens=h.shape[0], width=router.shape[1], experts=router.shape[0],
                       top=top, groups=groups, keep=keep, h=h.data_ptr(), ldh=h.stride(0), W=router.data_ptr(),
                       correction=_ptr(correction), gate_w=_ptr(gate_weight), weights=weights.data_ptr(), gate=_ptr(gate),
                       score={"softmax": 0, "sigmoid": 1, "chosen": 2}[score], group_rank=group_rank, normalize=1 if normalize else 0,
-                      bias=_ptr(bias)))
+                      bias=_ptr(bias), used=_ptr(used)))
 
 
 def weigh_experts(logits, bias, correction, top, groups, keep, hidden, experts, ff, score="softmax", group_rank=1, normalize=True):
@@ -1491,11 +1491,11 @@ def groups_experts(tokens, experts, top, ff, shared_ff, width, dtype):
         width % row == 0 and ff % row == 0 and shared_ff % row == 0
 
 
-def grouped_experts(h, weights, gate, in_weight, down_weight, experts, ff, shared_ff, identity, top, step, out, limit=None, alpha=1.0,
+def grouped_experts(h, weights, used, gate, in_weight, down_weight, experts, ff, shared_ff, identity, top, step, out, limit=None, alpha=1.0,
                     unit=None):
     """out [top (+ 1 with ``shared_ff``), rows, width] float32: plane j holds the output of each row's j-th expert (in the order
     of the experts) times its weight, an identity expert's, or zeros, the last plane the shared expert's times ``gate``;
-    operands as in ``gated_experts``, ``in_weight`` and ``down_weight`` the matrices of the products around it."""
+    ``used`` as ``route`` leaves it, operands as in ``gated_experts``, ``in_weight`` and ``down_weight`` the matrices of the products around it."""
     tokens, width = h.shape
     pitch = step.token_capacity
     rows = step.buffer("experts.rows", experts + 1, pitch, "int32")           # (the last row: the counts)
@@ -1507,7 +1507,7 @@ def grouped_experts(h, weights, gate, in_weight, down_weight, experts, ff, share
     module, dtype = _module("experts"), DTYPE_CODES[h.dtype]
     _launch(module, "bt_group_experts_call",
             GroupExpertsCall(dtype=dtype, tokens=tokens, experts=experts, identity=identity, top=top, width=width,
-                             weights=weights.data_ptr(), rows=rows.data_ptr(), pitch=pitch, counts=counts.data_ptr(), h=h.data_ptr(),
+                             weights=weights.data_ptr(), used=used.data_ptr(), rows=rows.data_ptr(), pitch=pitch, counts=counts.data_ptr(), h=h.data_ptr(),
                              ldh=h.stride(0), out=out.data_ptr(), plane=out.stride(0), ld_out=out.stride(1)))
     act = EXPERT_UNITS[unit] if unit is not None else (0 if limit is None else 1)
     for second, matrix in ((0, in_weight), (1, down_weight)):

@@ -148,11 +148,13 @@ class RoutedExperts(FeedForward):
             return Delta(partials, None)
         weights = step.buffer("experts.weights", tokens, self.outputs, "float32")
         mix = step.buffer("experts.mix", tokens, 1, "float32") if self.shared_mix is not None else None
+        grouped = K.groups_experts(tokens, self.experts, self.top, self.ff, self.shared_ff, self.width, step.dtype)
+        used = step.buffer("experts.used", tokens, 1, "int64") if grouped else None
         K.route(h, self.router, self.correction, self.top, self.groups, self.keep, weights, self.shared_mix, mix,
-                score=self.score, group_rank=self.group_rank, normalize=self.normalize, bias=self.router_bias)
-        if K.groups_experts(tokens, self.experts, self.top, self.ff, self.shared_ff, self.width, step.dtype):
+                score=self.score, group_rank=self.group_rank, normalize=self.normalize, bias=self.router_bias, used=used)
+        if grouped:
             partials = step.partial_sums("experts.partials", self.top + (1 if self.shared_ff else 0), tokens, self.width)
-            K.grouped_experts(h, weights, mix, self.in_weight, self.down_weight, self.experts, self.ff, self.shared_ff, self.identity,
+            K.grouped_experts(h, weights, used, mix, self.in_weight, self.down_weight, self.experts, self.ff, self.shared_ff, self.identity,
                               self.top, step, partials, limit=self.limit, alpha=self.alpha, unit=None if self.gated else self.unit)
             return Delta(partials, None)
         fused = step.buffer("experts.fused", tokens, self.fused_cols, step.dtype)

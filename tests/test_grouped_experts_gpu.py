@@ -73,7 +73,8 @@ def test_experts_on_their_rows(dtype, tokens, width, experts, top, ff, shared_ff
     step = make_step(dt, [tokens])
     planes = torch.full((top + (1 if shared_ff else 0), tokens + 3, width), float("nan"), device=DEV)[:, :tokens]
     assert K.groups_experts(tokens, experts, top, ff, shared_ff, width, dt) == (2 * top <= experts)
-    K.grouped_experts(h.to(dt).to(DEV), weights.to(DEV), None if gate is None else gate.to(DEV), part.in_weight, part.down_weight,
+    used = ((weights != 0).long() << torch.arange(outputs)).sum(1).to(DEV)
+    K.grouped_experts(h.to(dt).to(DEV), weights.to(DEV), used, None if gate is None else gate.to(DEV), part.in_weight, part.down_weight,
                       experts, ff, shared_ff, identity, top, step, planes, limit=limit, alpha=1.5, unit=None if kind == "gated" else kind)
     got = planes.sum(0).cpu().double()
     error = float((got - want).abs().max() / want.abs().max())
@@ -101,3 +102,35 @@ def test_a_part_takes_them_in_steps_of_many_tokens():
             finally:
                 K.GROUPED_EXPERTS = True
         assert float((sums[0] - sums[1]).abs().max() / sums[1].abs().max()) < 1.2e-2
+
+
+# sixteen tokens a work-group: tokens that are no multiple, outputs of one to four tiles, a gate beside them, groups, every
+# kind of score, corrections and biases, rows that lie apart; the choice itself is that of the kernel for few tokens
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("tokens,width,outputs,top,groups,keep,score,rank,normalize,extras", [
+    (128, 64, 8, 2, 1, 1, "softmax", 1, True, ""), (333, 1024, 9, 2, 3, 2, "softmax", 1, True, "correction gate"),
+    (150, 48, 16, 4, 4, 2, "sigmoid", 2, False, "gate"), (200, 80, 33, 3, 1, 1, "chosen", 1, True, "bias"), (129, 16, 64, 8, 8, 3, "softmax", 1, True, "correction bias")])
+def test_router_of_many_tokens(dtype, tokens, width, outputs, top, groups, keep, score, rank, normalize, extras):
+    gen = torch.Generator().manual_seed(tokens + outputs)
+    h = torch.randn(tokens, width + 8, generator=gen).to(DTYPES[dtype]).to(DEV)[:, :width]
+    router = (torch.randn(outputs, width, generator=gen) * width ** -0.5).to(DEV)
+    correction = (torch.randn(outputs, generator=gen) * 0.1).to(DEV) if "correction" in extras else None
+    bias = torch.randn(outputs, generator=gen).to(DEV) if "bias" in extras else None
+    mix = torch.randn(width, generator=gen).to(DEV) if "gate" in extras else None
+    many, few = [dict(weights=torch.full((tokens, outputs), float("nan"), device=DEV), gate=torch.full((tokens, 1), float("nan"), device=DEV),
+                      used=torch.zeros(tokens, dtype=torch.int64, device=DEV)) for _ in range(2)]
+    run = lambda rows, to, part: K.route(rows, router, correction, top, groups, keep, to["weights"][part], mix, to["gate"][part] if mix is not None else None,
+                                         score=score, group_rank=rank, normalize=normalize, bias=bias, used=to["used"][part])
+    run(h, many, slice(0, tokens))
+    for begin in range(0, tokens, 100):
+        part = slice(begin, min(begin + 100, tokens))
+        run(h[part], few, part)
+    assert torch.equal((many["weights"] != 0), (few["weights"] != 0))
+    # logits of size one from sums of `width` products in another order
+    assert float((many["weights"] - few["weights"]).abs().max()) < 4e-6
+    want = ((many["weights"] != 0).long() << torch.arange(outputs, device=DEV)).sum(1)
+    assert torch.equal(many["used"], want) and torch.equal(few["used"], want)
+    if mix is not None:
+        assert float((many["gate"] - few["gate"]).abs().max()) < 4e-6
+        exact = torch.sigmoid(h.double() @ mix.double())
+        assert float((many["gate"][:, 0].double() - exact).abs().max()) < 4e-6
