@@ -30,11 +30,17 @@ from .registry import register
 # 8,192 keys 47.7 / 29.6 / 23.0 / 19.3 / 23.6; eight sequences (200 pairs of sequence and head
 # already) lose with any cut, 73 / 80 / 85 us at 8,192 keys.  So: no more work-groups than
 # compute units, at least RUN_BYTES of keys and values per run, and no cut below SPLIT_BYTES.
+# Heads of more than 64 channels in bfloat16 are cut into eight runs at least where the pairs leave compute units for them (the
+# joining kernel asks for eight records at once): 8 heads of 128 on 2, eight sequences, us a call with 1 / 2 / 4 / 8 / 16 runs:
+# 300 keys 7.5 / 8.7 / 7.7 / 7.7 / 8.1, 600 10.8 / 11.7 / 8.9 / 8.6 / 9.6, 1,000 15.6 / 13.3 / 11.1 / 9.9 / 10.8, 2,000 25.4 /
+# 18.7 / 13.3 / 11.2 / 12.2; one sequence of 1,000 14.6 / 11.9 / 9.5 / 8.5 / 9.2; 16 heads on 4, eight of 1,000 15.6 / 13.6 / 11.5 /
+# 10.7 / 15.0.
 # (With the joining kernel that asks for eight runs' records at once, one sequence measures 7.1 us
 # in eight runs at 1,024 keys where one run takes 8.8; in the step that gained 0.2 % at batch 1,
 # the second kernel's place in the chain costing what its work-groups save: not taken.)
 SPLIT_BYTES = 384 << 10
 RUN_BYTES = 128 << 10
+JOINED_AT_ONCE = 8      # runs
 # A prompt step with few tiles of queries (a chunk of a prompt) cuts the keys of every tile into runs
 # of at least this many blocks of 64 keys for every 256 tokens of the step (prompt_runs).
 PROMPT_RUN_BLOCKS = 8
@@ -114,7 +120,8 @@ class CausalSelfAttention(Mixer):
         if pair_bytes <= SPLIT_BYTES:
             return 1
         pairs = step.n_seqs * self.kv_heads
-        return max(1, min(compute_units(device) // pairs, pair_bytes // RUN_BYTES, 64))
+        least = JOINED_AT_ONCE if step.dtype_is_bf16 and self.head_dim > 64 else 1
+        return max(1, min(compute_units(device) // pairs, max(pair_bytes // RUN_BYTES, least), 64))
 
     def prompt_runs(self, step, device, q_heads=None):
         """Into how many runs a prompt step's query tiles cut their keys: a chunk of a prompt behind

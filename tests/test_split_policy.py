@@ -112,6 +112,16 @@ def test_decode_runs_at_measured_sizes(monkeypatch):
     assert _runs(monkeypatch, 1, 8192, decode=False) == 1
 
 
+def test_decode_runs_of_wide_heads(monkeypatch):
+    """Heads of 128 in bfloat16: eight runs at least, as far as there are compute units."""
+    assert _runs(monkeypatch, 8, 1024, kv_heads=2, head_dim=128) == 8
+    assert _runs(monkeypatch, 8, 8192, kv_heads=2, head_dim=128) == 16
+    assert _runs(monkeypatch, 32, 1024, kv_heads=2, head_dim=128) == 4
+    assert _runs(monkeypatch, 200, 1024, kv_heads=2, head_dim=128) == 1
+    assert _runs(monkeypatch, 8, 1024, kv_heads=2, head_dim=128, window=512) == 1
+    assert _runs(monkeypatch, 8, 1024, kv_heads=2, head_dim=128, bf16=False) == 8      # (by the bytes of a run)
+
+
 def test_context_classes():
     from burn_transformers_amd.engine.step import StepPlan, context_limit
     assert [context_limit(n) for n in (1, 1024, 1025, 2048, 2049, 5000)] == [1024, 1024, 2048, 2048, 4096, 8192]
