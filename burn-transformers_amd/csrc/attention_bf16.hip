@@ -1105,6 +1105,11 @@ attention_prefill_wide_kernel(AttnArgs a) {
 // reduction overlaps the other's loads (57 -> 42 us).
 #define DECODE_WAVES 8
 
+template <int N>
+struct Shares {
+  static constexpr int value = N;
+};
+
 // KEEPS: some first positions stay visible beside a window or a chunk (a form of its own: the walk over two stretches of keys
 // and its test cost the other 0.3 us of 6.5).
 template <bool KEEPS>
@@ -1189,43 +1194,53 @@ attention_decode_kernel(AttnArgs a) {
   float total = l[0];
   total += __shfl_xor(total, 16, 64);
   total += __shfl_xor(total, 32, 64);
-  if (has_query) {
+  // Only the waves that had a tile leave a share (a short run keeps one or two busy): a share each of `group` rows is
+  // written, read and weighed again by every element of the output.  With every wave's share (us, 16 heads of 128 on one, eight
+  // sequences, in eight runs) 30 keys 11.6, 100 11.5, 1,000 12.5; so 8.0, 8.1, 10.3.  8 heads on 2: 1,000 keys 10.0 -> 9.7.
+  const int busy = tile_end - tile_begin, shares = busy <= 1 ? 1 : busy <= 2 ? 2 : busy <= 4 ? 4 : DECODE_WAVES;
+  if (has_query && wave < shares) {
     if (g == 0) {
       sm_m[wave * group + i16] = m[0];
       sm_l[wave * group + i16] = total;
     }
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sm_o[(wave * group + i16) * HD + dt * 16 + 4 * g + r] = o[0][dt][r];
+      *reinterpret_cast<floatx4*>(sm_o + (wave * group + i16) * HD + dt * 16 + 4 * g) = o[0][dt];
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < group * HD; e += DECODE_WAVES * 64) {
-    int j = e / HD, channel = e % HD;
-    float top = sm_m[j];
+  auto gather = [&](auto known) {
+    constexpr int SHARES = decltype(known)::value;
+    for (int e = threadIdx.x; e < group * HD; e += DECODE_WAVES * 64) {
+      int j = e / HD, channel = e % HD;
+      float top = sm_m[j];
 #pragma unroll
-    for (int w = 1; w < DECODE_WAVES; ++w) top = fmaxf(top, sm_m[w * group + j]);
-    float num = 0.f, den = 0.f;
-    if (top != -INFINITY) {
+      for (int w = 1; w < SHARES; ++w) top = fmaxf(top, sm_m[w * group + j]);
+      float num = 0.f, den = 0.f;
+      if (top != -INFINITY) {
 #pragma unroll
-      for (int w = 0; w < DECODE_WAVES; ++w) {
-        float f = exp2f(sm_m[w * group + j] - top);   // the maxima are kept in powers of two
-        num += sm_o[(w * group + j) * HD + channel] * f;
-        den += sm_l[w * group + j] * f;
+        for (int w = 0; w < SHARES; ++w) {
+          float f = exp2f(sm_m[w * group + j] - top);   // the maxima are kept in powers of two
+          num += sm_o[(w * group + j) * HD + channel] * f;
+          den += sm_l[w * group + j] * f;
+        }
+      }
+      if (splits == 1) {
+        den += top != -INFINITY ? bt_sink_term_pow2(a.sink, kv_head * group + j, top) : 0.f;
+        put1(a, tok, kv_head * group + j, channel, FORM == 2 ? num : den > 0.f ? num / den : 0.f);
+      } else {     // this run's share, for attention_join_kernel
+        float* mine = a.partial + (((int64_t)seq * a.q_heads + kv_head * group + j) * splits + split) * (HD + 2);
+        mine[channel] = num;
+        if (channel == 0) {
+          mine[HD] = top;
+          mine[HD + 1] = den;
+        }
       }
     }
-    if (splits == 1) {
-      den += top != -INFINITY ? bt_sink_term_pow2(a.sink, kv_head * group + j, top) : 0.f;
-      put1(a, tok, kv_head * group + j, channel, FORM == 2 ? num : den > 0.f ? num / den : 0.f);
-    } else {     // this run's share, for attention_join_kernel
-      float* mine = a.partial + (((int64_t)seq * a.q_heads + kv_head * group + j) * splits + split) * (HD + 2);
-      mine[channel] = num;
-      if (channel == 0) {
-        mine[HD] = top;
-        mine[HD + 1] = den;
-      }
-    }
-  }
+  };
+  if (shares == 1) gather(Shares<1>());
+  else if (shares == 2) gather(Shares<2>());
+  else if (shares == 4) gather(Shares<4>());
+  else gather(Shares<DECODE_WAVES>());
 }
 
 // Joins the runs of attention_decode_kernel (a row is a sequence's one token) or of
