@@ -69,9 +69,10 @@ struct RouteEarly {
 };
 
 // From a token's logits to its experts, by ONE wave: the experts dealt to its lanes, maxima and choices as wave
-// reductions.  `score` holds the logits and afterwards the scores, `choice` afterwards +inf where an expert was chosen
-// (both in LDS).  Returns the factor on the chosen experts' scores.
-__device__ __forceinline__ float route_choice(const RouteCall& c, const RouteEarly& early, float* score, float* choice) {
+// reductions.  `score` holds the logits and afterwards the scores, `choice` afterwards the token's weight of every expert,
+// zero where it was not chosen (both in LDS, written by the lane whose expert it is).  At most `top` experts are chosen whatever
+// the values: a lane remembers which of its experts are taken, no value stands for it (a correction or logit may be infinite).
+__device__ __forceinline__ void route_choice(const RouteCall& c, const RouteEarly& early, float* score, float* choice) {
   const int lane = threadIdx.x & 63;
   if (c.bias)                                       // a lane keeps to its own experts
     for (int e = lane, j = 0; e < c.experts; e += 64, ++j) score[e] += j < 4 ? early.bias[j < 4 ? j : 0] : c.bias[e];
@@ -136,22 +137,21 @@ __device__ __forceinline__ float route_choice(const RouteCall& c, const RouteEar
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   float sum = 0.f;
+  unsigned taken = 0;                              // bit j: the lane's expert lane + 64 j (ROUTE_MAX_EXPERTS: sixteen of them)
   for (int k = 0; k < c.top; ++k) {
     float value = -INFINITY;
     int index = 0x7fffffff;
-    for (int e = lane; e < c.experts; e += 64) {
+    for (int e = lane, j = 0; e < c.experts; e += 64, ++j) {
       const float v = choice[e];
-      if (v > value && v != INFINITY) { value = v; index = e; }     // (ascending e: the lowest index among equals; +inf: taken)
+      if (v > value && !(taken >> j & 1)) { value = v; index = e; }     // (ascending e: the lowest index among equals)
     }
     wave_best(value, index);
-    if (index == 0x7fffffff) break;                // (nothing left to choose: refused on the host)
-    if (lane == (index & 63)) choice[index] = INFINITY;            // taken: its owner marks it
+    if (index == 0x7fffffff) break;                // (nothing left above minus infinity, or what is left is not a number)
+    if (lane == (index & 63)) taken |= 1u << (index >> 6);
     sum += score[index];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  return c.normalize ? 1.0f / (sum + 1e-20f) : 1.0f;
+  const float inverse = c.normalize ? 1.0f / (sum + 1e-20f) : 1.0f;
+  for (int e = lane, j = 0; e < c.experts; e += 64, ++j) choice[e] = taken >> j & 1 ? score[e] * inverse : 0.f;
 }
 
 // One work-group of sixteen waves per token.  Logits: a wave takes whole outputs (two at a time, the
@@ -168,7 +168,7 @@ __device__ __forceinline__ float route_choice(const RouteCall& c, const RouteEar
 template <typename T>
 __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
   __shared__ float score[ROUTE_MAX_EXPERTS];      // logits, then softmax scores
-  __shared__ float choice[ROUTE_MAX_EXPERTS];     // scores with the correction; +inf once taken, -inf where shut out
+  __shared__ float choice[ROUTE_MAX_EXPERTS];     // scores with the correction, -inf where shut out; then the weights
   __shared__ float gate_sum;
   const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const T* h = static_cast<const T*>(c.h) + (int64_t)t * c.ldh;
@@ -219,11 +219,11 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
   }
   __syncthreads();
   if (wave != 0) return;
-  const float inverse = route_choice(c, early, score, choice);
+  route_choice(c, early, score, choice);
   // the one store of a lane's experts: the chosen ones' scores over their sum, zero elsewhere
   float* weights = c.weights + (int64_t)t * c.experts;
   for (int e = lane; e < c.experts; e += 64) {
-    const float w = choice[e] == INFINITY ? score[e] * inverse : 0.f;
+    const float w = choice[e];
     weights[e] = w;
     if (e < 64 && c.used) {
       const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
@@ -298,8 +298,8 @@ __global__ void __launch_bounds__(64 * ROUTE_ROWS) route_rows_kernel(RouteCall c
   const int t = t0 + wave;
   if (t >= c.tokens) return;
   const float gate_sum = score[wave][c.gate_w ? c.experts : 0];
-  const float inverse = route_choice(c, early, score[wave], choice[wave]);
-  const float w = lane < c.experts && choice[wave][lane] == INFINITY ? score[wave][lane] * inverse : 0.f;
+  route_choice(c, early, score[wave], choice[wave]);
+  const float w = lane < c.experts ? choice[wave][lane] : 0.f;
   if (lane < c.experts) c.weights[(int64_t)t * c.experts + lane] = w;
   const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
   if (lane == 0 && c.used) c.used[t] = used;
@@ -537,8 +537,8 @@ __global__ void __launch_bounds__(1024) group_experts_kernel(GroupExpertsCall c)
     for (int t0 = 0; t0 < c.tokens; t0 += 1024) {
       const int t = t0 + threadIdx.x;
       const unsigned long long word = t < c.tokens ? c.used[t] : 0;
-      const bool mine = word >> e & 1;
       const int place = __builtin_popcountll(word & ((1ull << e) - 1));
+      const bool mine = (word >> e & 1) && place < c.top;             // (there is room for `top` choices of a token)
       const unsigned long long all = __builtin_amdgcn_ballot_w64(mine);
       if (lane == 0) found[wave] = __builtin_popcountll(all);
       __syncthreads();
@@ -863,7 +863,6 @@ struct WeighExpertsCall {
 template <typename T>
 __global__ void __launch_bounds__(256) weigh_experts_kernel(WeighExpertsCall w) {
   __shared__ float score[ROUTE_MAX_EXPERTS], choice[ROUTE_MAX_EXPERTS];
-  __shared__ float factor;
   typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
   constexpr int PER = 16 / sizeof(T);
   const RouteCall& c = w.route;
@@ -881,11 +880,10 @@ __global__ void __launch_bounds__(256) weigh_experts_kernel(WeighExpertsCall w) 
     RouteEarly early;
     early.load(c);
     for (int e = lane; e < c.experts; e += 64) score[e] = logits[e];
-    const float inverse = route_choice(c, early, score, choice);
-    if (lane == 0) factor = inverse;
+    route_choice(c, early, score, choice);
   }
   __syncthreads();
-  auto weight = [&](int e) { return choice[e] == INFINITY ? score[e] * factor : 0.f; };
+  auto weight = [&](int e) { return choice[e]; };
   if (!whole) {
     for (int col = piece; col < columns; col += gridDim.y * blockDim.x) {
       const float f = weight(col / w.ff);

@@ -134,3 +134,90 @@ def test_router_of_many_tokens(dtype, tokens, width, outputs, top, groups, keep,
         assert float((many["gate"] - few["gate"]).abs().max()) < 4e-6
         exact = torch.sigmoid(h.double() @ mix.double())
         assert float((many["gate"][:, 0].double() - exact).abs().max()) < 4e-6
+
+
+def chosen_by(scores, corrected, top, groups, keep):
+    """[rows, outputs] of booleans: the ``top`` largest corrected scores (the lower index among equals) in the ``keep`` groups
+    with the largest best."""
+    rows, outputs = scores.shape
+    if groups > 1:
+        best = corrected.view(rows, groups, -1).amax(-1)
+        kept = best.sort(dim=-1, descending=True, stable=True).indices[:, :keep]
+        open_ = torch.zeros(rows, groups, dtype=torch.bool).scatter_(1, kept, True).repeat_interleave(outputs // groups, 1)
+        corrected = corrected.masked_fill(~open_, float("-inf"))
+    order = corrected.sort(dim=-1, descending=True, stable=True).indices[:, :top]
+    return torch.zeros(rows, outputs, dtype=torch.bool).scatter_(1, order, True)
+
+
+# a correction or a logit without end is one choice like any other and no sign of one that was made: never more than `top`
+# experts, however many there are of them, in every kernel that makes the choice
+@pytest.mark.parametrize("tokens", [3, 64, 200, 1537])
+@pytest.mark.parametrize("score,groups,keep,endless", [
+    ("softmax", 1, 1, [5]), ("softmax", 1, 1, [0, 2, 3, 7]), ("sigmoid", 4, 2, [5]), ("softmax", 4, 2, [1, 6]), ("chosen", 1, 1, [2, 4, 6])])
+def test_endless_corrections_are_choices_like_others(tokens, score, groups, keep, endless):
+    gen = torch.Generator().manual_seed(tokens + len(endless))
+    width, outputs, top = 64, 8, 2
+    h = torch.randn(tokens, width, generator=gen)
+    router = torch.randn(outputs, width, generator=gen) * width ** -0.5
+    extra = torch.randn(outputs, generator=gen) * 0.1
+    extra[endless] = float("inf")
+    logits = h.double() @ router.double().T
+    scores = {"softmax": logits.softmax(-1), "sigmoid": logits.sigmoid(), "chosen": logits}[score]
+    mask = chosen_by(scores, scores + extra.double(), top, groups, keep)
+    assert bool((mask.sum(1) == top).all())
+    weights, used = torch.full((tokens, outputs), -1.0, device=DEV), torch.zeros(tokens, dtype=torch.int64, device=DEV)
+    # (a "chosen" score weighs by the logits with their bias: of infinite ones nobody knows the softmax)
+    more = {"bias": extra.to(DEV)} if score == "chosen" else {}
+    K.route(h.to(DEV), router.to(DEV), None if more else extra.to(DEV), top, groups, keep, weights, score=score, used=used, **more)
+    got = weights.cpu()
+    assert torch.equal(got != 0, mask)                                  # (not a number is not zero)
+    assert torch.equal(used.cpu(), (mask.long() << torch.arange(outputs)).sum(1))
+    if score != "chosen":
+        want = torch.where(mask, scores, 0.0)
+        assert float((got.double() - want / want.sum(1, keepdim=True)).abs().max()) < 4e-6
+
+
+def test_a_part_with_an_endless_correction_on_both_sides_of_the_rule():
+    gen = torch.Generator().manual_seed(5)
+    width, experts, ff = 128, 8, 128
+    correction = torch.randn(experts, generator=gen) * 0.1
+    correction[3] = float("inf")
+    tensors = {"router": torch.randn(experts, width, generator=gen) * 0.1, "correction": correction}
+    for e in range(experts):
+        for role, shape in (("gate", (ff, width)), ("up", (ff, width)), ("down", (width, ff))):
+            tensors[f"{role}_{e}"] = torch.randn(shape, generator=gen) * 0.1
+    part = lookup("feed_forward", "routed_experts")({"width": width, "experts": experts, "ff": ff, "top": 2}, {k: v.to(DEV) for k, v in tensors.items()})
+    h = torch.randn(200, width, generator=gen)
+    scores = (h.double() @ tensors["router"].double().T).softmax(-1)
+    weights = torch.where(chosen_by(scores, scores + correction.double(), 2, 1, 1), scores, 0.0)
+    weights /= weights.sum(1, keepdim=True)
+    want = sum(weights[:, e:e + 1] * (unit_of("gated", h.double() @ tensors[f"gate_{e}"].double().T, h.double() @ tensors[f"up_{e}"].double().T, None)
+                                      @ tensors[f"down_{e}"].double().T) for e in range(experts))
+    for tokens in (1, 64, 65, 200):
+        delta = part.forward(h[:tokens].to(DEV), make_step(torch.float32, [tokens]), ResidualStream(torch.zeros(tokens, width, device=DEV)))
+        got = delta.partials.sum(0).cpu().double()
+        # sums of 128 products of 32-bit values, two of them one behind the other
+        assert float((got - want[:tokens]).abs().max() / want.abs().max()) < 5e-6
+
+
+def test_a_token_has_room_for_its_choices_only():
+    """Words that name more than ``top`` experts: the first ``top`` of them count, and no plane behind theirs is touched."""
+    gen = torch.Generator().manual_seed(6)
+    tokens, width, experts, ff, top = 130, 64, 8, 64, 2
+    matrices = [[torch.randn(ff, width, generator=gen) * 0.1, torch.randn(ff, width, generator=gen) * 0.1, torch.randn(width, ff, generator=gen) * 0.1] for _ in range(experts)]
+    tensors = {"router": torch.zeros(experts, width)}
+    for e, made in enumerate(matrices):
+        tensors.update({f"{role}_{e}": m for role, m in zip(("gate", "up", "down"), made)})
+    part = lookup("feed_forward", "routed_experts")({"width": width, "experts": experts, "ff": ff, "top": top}, {k: v.to(DEV) for k, v in tensors.items()})
+    h = torch.randn(tokens, width, generator=gen)
+    named = torch.rand(tokens, experts, generator=gen).topk(4, -1).indices
+    weights = torch.zeros(tokens, experts).scatter_(1, named, torch.rand(tokens, 4, generator=gen) + 0.1)
+    used = ((weights != 0).long() << torch.arange(experts)).sum(1)
+    first = (weights != 0) & ((weights != 0).cumsum(1) <= top)
+    planes = torch.full((top + 1, tokens, width), float("nan"), device=DEV)
+    step = make_step(torch.float32, [tokens])
+    K.grouped_experts(h.to(DEV), weights.to(DEV), used.to(DEV), None, part.in_weight, part.down_weight, experts, ff, 0, 0, top, step, planes[:top])
+    want = sum(torch.where(first, weights, 0.0)[:, e:e + 1].double() * (unit_of("gated", h.double() @ g.double().T, h.double() @ u.double().T, None) @ d.double().T)
+               for e, (g, u, d) in enumerate(matrices))
+    assert float((planes[:top].sum(0).cpu().double() - want).abs().max() / want.abs().max()) < 5e-6
+    assert bool(torch.isnan(planes[top]).all())
