@@ -136,8 +136,9 @@ def stream_product_splits(step, a, weight):
             K.deep_form_rows(rows, a.shape[1], a.stride(0), width, sliced=True) else 1
     if step.dtype_is_bf16:
         return split_count(rows, width, a.shape[1], compute_units(a.device), 32)
-    if rows > 64:
-        return K.float_split_count(rows, width, a.shape[1], compute_units(a.device)) if a.stride(0) % 4 == 0 else 1
+    if rows > 64:       # (the rule weighs the rows themselves: it is asked for the step's class, whose steps share one launch list)
+        most = step.token_capacity if rows == step.n_tokens else rows
+        return K.float_split_count(most, width, a.shape[1], compute_units(a.device)) if a.stride(0) % 4 == 0 else 1
     if a.shape[1] % 4 == 0 and a.stride(0) % 4 == 0:        # what the float32 MFMA kernels take
         return split_count(rows, width, a.shape[1], compute_units(a.device), 16)
     return 1

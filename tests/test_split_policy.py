@@ -173,3 +173,25 @@ def test_products_of_short_prompts_and_how_they_cut_k():
             for k in (64, 128, 768, 1024, 1600, 6400):
                 splits = deep_split_count(rows, columns, k)
                 assert 1 <= splits <= 4 and (splits == 1 or (k // 64) // splits >= 4)
+
+
+def test_float_products_are_cut_alike_in_all_steps_of_a_class(monkeypatch):
+    """One launch list serves all steps of a class, so the slices of a float32 product may not depend on which of them came first."""
+    from types import SimpleNamespace
+    import torch
+    from burn_transformers_amd.engine.step import token_capacity
+    from burn_transformers_amd.kernels.library import float_split_count
+    from burn_transformers_amd.parts import base
+    monkeypatch.setattr(base, "compute_units", lambda device: 256)
+
+    def cuts(rows, columns, k):
+        step = SimpleNamespace(dtype_is_bf16=False, n_tokens=rows, token_capacity=token_capacity(rows))
+        return base.stream_product_splits(step, torch.empty(rows, k, device="meta"), torch.empty(columns, k, device="meta"))
+
+    asked_exactly = 0
+    for columns, k in ((768, 768), (768, 3072), (1024, 1024), (1024, 2048), (1024, 4096), (1600, 1600), (1600, 6400), (2048, 2048)):
+        for most in range(128, 2305, 64):
+            found = {cuts(rows, columns, k) for rows in range(most - 63, most + 1)}
+            assert len(found) == 1, (columns, k, most, found)
+            asked_exactly += len({float_split_count(rows, columns, k) for rows in range(most - 63, most + 1)}) > 1
+    assert asked_exactly > 0                                            # the rule itself turns within classes
