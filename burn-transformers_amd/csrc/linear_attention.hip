@@ -506,16 +506,16 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
       col[t] = (v[0] + v[1]) + (v[2] + v[3]);
     }
 #pragma unroll
-    for (int t = 0; t < KB_TOKENS; ++t) col[t] *= strength[sub];
+    for (int t = 0; t < KB_TOKENS; ++t) col[t] = t >= sub ? col[t] * strength[sub] : 0.f;
 #pragma unroll
     for (int t = 0; t < KB_TOKENS; ++t)
       if ((lane >> 4) == (t & 3)) T[t][sub] = col[t];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {                                        // rows 4 i + g; behind the diagonal P is zero or col is
+    for (int i = 0; i < 4; ++i) {                                        // rows 4 i + g; P holds nothing behind the diagonal
       const int t = 4 * i + (lane >> 4);
       float m = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4 * i + 4; ++e) m = fmaf(e <= t ? P[t][e] : 0.f, col[e], m);
+      for (int e = 0; e < 4 * i + 4; ++e) m = e <= t ? fmaf(P[t][e], col[e], m) : m;
       M[t][sub] = m;
     }
   }
@@ -545,6 +545,15 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
   floatx4 tb, mb = *reinterpret_cast<const floatx4*>(&M[n][4 * g]);
   if (FORM == 0) tb = *reinterpret_cast<const floatx4*>(&T[n][4 * g]);
   floatx4* frag = reinterpret_cast<floatx4*>(place);
+  // T and M hold zeros for the tokens behind a row's own, and the products take them: a value there that is not finite
+  // would make this row's not a number.  Where a result is not finite it is summed again, over the row's own tokens only.
+  auto finite = [](floatx4 v) { return fabsf((v[0] + v[1]) + (v[2] + v[3])) < INFINITY; };
+  auto own = [](const float* row, int t, auto value) {
+    float sum = 0.f;
+#pragma unroll 1
+    for (int s = 0; s <= t; ++s) sum = fmaf(row[s], value(s), sum);
+    return sum;
+  };
   for (int tile = wave; tile < DT; tile += 4) {
     const int d = 16 * tile + n;
     floatx4 r = *reinterpret_cast<const floatx4*>(&Q[n][16 * tile + 4 * g]), u;
@@ -556,6 +565,13 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
         w = __builtin_amdgcn_mfma_f32_16x16x4f32(kd, tb[i], w, 0, 0, 0);
         r = __builtin_amdgcn_mfma_f32_16x16x4f32(kd, -mb[i], r, 0, 0, 0);
       }
+      if (__builtin_expect(!(finite(w) && finite(r)), 0))
+        for (int i = 0; i < 4; ++i) {
+          const int from = 16 * tile + 4 * g + i;
+          auto kd = [&](int s) { return K[s][from]; };
+          w[i] = own(T[n], n, kd);
+          r[i] = Q[n][from] - own(M[n], n, kd);
+        }
       frag[64 * tile + lane] = w;
     }
 #pragma unroll
@@ -577,6 +593,13 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
       if (FORM == 0) u = __builtin_amdgcn_mfma_f32_16x16x4f32(tb[i], v[i], u, 0, 0, 0);
       o = __builtin_amdgcn_mfma_f32_16x16x4f32(mb[i], v[i], o, 0, 0, 0);
     }
+    if (__builtin_expect(!(finite(o) && (FORM == 1 || finite(u))), 0))
+      for (int i = 0; i < 4; ++i) {
+        const int t = min(4 * g + i, count - 1);                         // (rows behind the sequence's end are not used)
+        auto value = [&](int s) { return v_rows[(int64_t)s * c.ld_v + 16 * tile + n]; };
+        if (FORM == 0) u[i] = own(T[t], t, value);
+        o[i] = own(M[t], t, value);
+      }
     frag[64 * (3 * DT + tile) + lane] = FORM == 0 ? u : v;
 #pragma unroll
     for (int i = 0; i < 4; ++i)

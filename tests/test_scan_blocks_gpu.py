@@ -98,6 +98,47 @@ def test_blocks_of_tokens(form, heads, kv_heads, dim, vdim, lengths, strong):
     assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
 
 
+# one token of one sequence whose operand is not finite, in the middle of a block and at its end: earlier tokens and other
+# sequences do not see it, later ones as in the walk (an endless step is a decay of nothing and stays finite)
+@pytest.mark.parametrize("form,where,value", [
+    (form, where, value) for form in ("head", "channel", "forget")
+    for where, value in (("v", "inf"), ("v", "nan"), ("k", "inf"), ("k", "nan"), ("q", "inf"), ("g", "nan"), ("g", "inf"), ("beta", "nan"))
+    if form != "forget" or where not in ("k", "beta")])                 # (the forget gate has no such operands)
+@pytest.mark.parametrize("token", [21, 31, 39])
+def test_a_token_that_is_not_finite_spoils_no_earlier_one(form, where, value, token):
+    gen = torch.Generator().manual_seed(7)
+    heads, dim, vdim, lengths = 2, 64, 32, [40, 50]
+    qk, inner = heads * dim, heads * vdim
+    decays = heads if form == "head" else heads * dim
+    total = sum(lengths)
+    A_log, bias, lower = torch.zeros(heads, device=DEV), torch.randn(decays, generator=gen).to(DEV), (torch.rand(decays, generator=gen) * 0.9).to(DEV)
+    rows = torch.randn(total, 2 * qk + inner + decays + heads, generator=gen)
+    at = {"q": 3, "k": qk + 3, "v": 2 * qk + 3, "g": 2 * qk + inner, "beta": 2 * qk + inner + decays}[where]
+    spoiled = rows.clone()
+    spoiled[token, at] = float(value)
+    step = make_step(torch.float32, lengths)
+    results = {}
+    for name, source, blocked in (("clean", rows, True), ("blocks", spoiled, True), ("walk", spoiled, False)):
+        on, state = source.to(DEV), torch.zeros(len(lengths), heads * dim * vdim, device=DEV)
+        y = torch.full((total, inner), -7.0, device=DEV)
+        extra = dict(g_bias=bias, lower=lower) if form == "forget" else \
+            dict(beta=on[:, -heads:], A_log=A_log, unit=False, q_scale=1.0, decay_per_head=form == "head", dt_bias=bias)
+        if form != "forget":
+            on[:, :2 * qk] *= dim ** -0.5
+        K.keyed_scan(on[:, :qk], None if form == "forget" else on[:, qk:2 * qk], on[:, 2 * qk:2 * qk + inner], on[:, 2 * qk + inner:2 * qk + inner + decays],
+                     y, state, step, heads, heads, dim, vdim, "forget" if form == "forget" else "delta",
+                     blocks=K.scan_blocks(step, heads, dim, vdim) if blocked else None, **extra)
+        results[name] = (y.cpu(), state.cpu())
+    (clean, _), (blocks, state), (walk, walked) = results["clean"], results["blocks"], results["walk"]
+    # (a block with such a token sums in another order: a few roundings of 32 bits)
+    assert rel_err(blocks[:token], clean[:token].double()) < 2e-6
+    assert torch.equal(blocks[lengths[0]:], clean[lengths[0]:])
+    assert torch.equal(torch.isfinite(blocks), torch.isfinite(walk)) and torch.equal(torch.isfinite(state), torch.isfinite(walked))
+    assert bool(torch.isfinite(blocks).all()) == (where == "g" and value == "inf")
+    kept = torch.isfinite(walk)
+    assert rel_err(blocks[kept], walk[kept].double()) < 1e-5
+
+
 @pytest.mark.parametrize("heads,groups,vdim,state,lengths,strong", [
     (4, 1, 64, 128, [33, 1, 16, 47], False), (12, 1, 16, 16, [100, 32, 5], True), (6, 3, 48, 80, [49, 2], False),
     (9, 1, 32, 48, [400], True), (2, 2, 16, 32, [64, 63, 65], False), (20, 2, 16, 128, [333, 17], False)])
