@@ -607,11 +607,24 @@ __global__ void __launch_bounds__(256) selective_carry_kernel(SelectiveScanCall 
   slot[index] = state;
 }
 
+// Spans of the scan with eight lanes a channel may be as short as the call's room allows where a sequence brings 64 tokens, and 128
+// for each wave that a SIMD has; elsewhere they have 64 at least: three launches and twice the arithmetic cost more than
+// they save.  Measured (us, spans of 64 / of 16 or more): states of 24 to 32, 2 x 64 tokens on 512 waves (half a wave to a SIMD) 31.8 /
+// 26.8, 2 x 128 62.1 / 38.0, 2 x 256 117 / 64, 128 tokens on 256 waves 57 / 28, on 1,024 67.6 / 61.4, but 64 tokens on 1,024 35.6 / 37.3, 3 x 56
+// on 768 29.0 / 32.0, 4 x 63 on 1,024 34.9 / 37.8; states of 16, 2 x 128 48 / 29, 64 tokens on 1,024 waves 27.8 / 28.3, 3 x 56 22.5 / 23.7.
+#define SS_LONG_SPAN 64
+
+static int shortest_span(const SelectiveScanCall& c, int64_t waves) {
+  const bool few = c.max_count >= SS_LONG_SPAN && (int64_t)c.max_count * simd_count() >= 2 * SS_LONG_SPAN * waves;
+  return few || c.span <= 0 || c.span >= SS_LONG_SPAN ? c.span : SS_LONG_SPAN;
+}
+
 template <typename T, int R>
 static void launch_selective_scan_r(hipStream_t stream, const SelectiveScanCall& c) {
   const int per_token = 2 * 8 * R + 24;
   dim3 block(64);
-  const int span = span_tokens(c.span, c.max_count, c.carry, (int64_t)((c.channels + 7) / 8) * c.n_seqs, 2);
+  const int64_t waves = (int64_t)((c.channels + 7) / 8) * c.n_seqs;
+  const int span = span_tokens(shortest_span(c, waves), c.max_count, c.carry, waves, 2);
   if (span > 0) {
     SelectiveScanCall cut = c;
     cut.span = span;

@@ -222,3 +222,26 @@ def test_channels_in_lanes(channels, state, lengths, spans, strong):
         assert rel_err(out[:, :channels].cpu(), want) < 3e-6
         for slot, w in zip(slots, want_state):
             assert rel_err(held[slot, :channels * state].view(channels, state).cpu(), w) < 3e-6
+
+
+# which sequences the scan with eight lanes a channel cuts into spans (only then does it write the room for them): 64 tokens and
+# 128 for each wave a SIMD has (four to each of 256 compute units), sequences of three spans of 64 whatever the waves
+@pytest.mark.parametrize("channels,state,counts,cut", [
+    (2048, 24, [64] * 2, True), (2048, 24, [63] * 2, False), (2048, 16, [56] * 3, False), (2048, 32, [48], False), (4096, 24, [64] * 2, False),
+    (4096, 24, [128] * 2, True), (2048, 64, [128] * 8, False), (2048, 24, [192] * 8, True), (2048, 24, [200] * 9, False)])
+def test_which_sequences_eight_lanes_cut(channels, state, counts, cut):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    total = sum(counts)
+    step = make_step(torch.float32, counts)
+    x, z, dt, bc = [torch.rand(total, n, device=DEV) for n in (channels, channels, channels, 2 * state)]
+    A_log, D = torch.zeros(channels, state, device=DEV), torch.zeros(channels, device=DEV)
+    held, out = torch.zeros(len(counts), channels * state, device=DEV), torch.empty(total, channels, device=DEV)
+    carry = K.scan_carry(step, channels * state, channels, K.SELECTIVE_SPAN)
+    if carry is None:
+        assert not cut
+        return
+    carry.fill_(float("nan"))
+    K.selective_scan(x, z, dt, bc[:, :state], bc[:, state:], A_log, D, out, held, step, carry=carry, span=K.SELECTIVE_SPAN)
+    assert bool(torch.isfinite(carry).any()) == cut
+    assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(held).all())
