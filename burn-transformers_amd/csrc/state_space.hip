@@ -476,8 +476,11 @@ __global__ void __launch_bounds__(64) selective_scan_kernel(SelectiveScanCall c,
 // Taken by steps whose longest sequence brings SL_MIN_TOKENS tokens, or a quarter of that where a wave for every 64 channels of
 // every sequence makes SL_MIN_WAVES; smaller steps have more waves with eight lanes a channel.  Measured (us, eight lanes / one; 2,048
 // channels of 16): 2 x 32 tokens 14.7 / 18.0, 4 x 48 21.0 / 23.6, 2 x 64 25.8 / 22.5, 16 x 20 25.9 / 13.9, 2 x 256 60.6 / 31.2, 8 x 300 208 / 80,
-// 2 x 1,024 181 / 73 (of which 46 are the recurrence, gone through twice, and 8 the carry).
+// 2 x 1,024 181 / 73 (of which 46 are the recurrence, gone through twice, and 8 the carry).  Channels of 8: 2 x 64 18.1 / 17.1, 2 x 1,024 124 / 51.
+// Of 32, whose tokens' B and C are more than a wave's scalar registers: 2 x 64 26.8 / 39.7, 2 x 160 44.8 / 46.0, 2 x 256 63.6 / 58.8, 2 x 1,024
+// 293 / 130, 16 x 20 40.2 / 26.8: from three times as many tokens on.
 #define SL_MIN_TOKENS 64
+#define SL_MIN_TOKENS_32 192
 #define SL_MIN_WAVES 256
 
 __device__ __forceinline__ float decay_of(float v) {
@@ -660,7 +663,7 @@ static void launch_selective_lanes(hipStream_t stream, const SelectiveScanCall& 
 
 template <typename T>
 static int launch_selective_scan(hipStream_t stream, const SelectiveScanCall& c) {
-  const bool many = c.max_count >= SL_MIN_TOKENS ||
+  const bool many = c.max_count >= (c.state == 32 ? SL_MIN_TOKENS_32 : SL_MIN_TOKENS) ||
       (c.max_count >= SL_MIN_TOKENS / 4 && (int64_t)((c.channels + 63) / 64) * c.n_seqs >= SL_MIN_WAVES);
   if (many && (c.state == 8 || c.state == 16 || c.state == 32)) {
     if (c.state == 8) launch_selective_lanes<T, 8>(stream, c);

@@ -187,7 +187,8 @@ def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
 # within a sequence, a second portion from a state that is not zero; `strong`: steps so long that decays vanish
 @pytest.mark.parametrize("channels,state,lengths,spans,strong", [
     (100, 16, [64, 1, 130], True, False), (64, 8, [65, 63], False, True), (200, 32, [300, 17, 64], True, False), (70, 16, [500], True, True),
-    (1100, 16, [20] * 16, True, False), (48, 16, [63, 5], True, False)])
+    (1100, 16, [20] * 16, True, False), (48, 16, [63, 5], True, False), (100, 32, [191, 64], True, False), (100, 32, [192, 2], True, True),
+    (100, 24, [64, 200], True, False)])
 def test_channels_in_lanes(channels, state, lengths, spans, strong):
     gen = torch.Generator().manual_seed(channels + state + len(lengths))
     A_log, D = torch.log(torch.rand(channels, state, generator=gen) * 7.0 + 0.5), torch.randn(channels, generator=gen)
