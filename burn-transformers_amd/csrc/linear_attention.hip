@@ -396,12 +396,14 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
   __shared__ __attribute__((aligned(16))) float K[KB_TOKENS][PITCH], Q[KB_TOKENS][PITCH], G[KB_TOKENS][PITCH];
   __shared__ __attribute__((aligned(16))) float A[KB_TOKENS][KB_TOKENS], P[KB_TOKENS][KB_TOKENS], T[KB_TOKENS][20], M[KB_TOKENS][20];
   __shared__ float strength[KB_TOKENS], one[KB_TOKENS];                  // beta, and a decay the whole head shares
-  const int seq = blockIdx.z, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int first = c.seq_off[seq] + (int)blockIdx.x * KB_TOKENS;
+  const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int part;
+  const int seq = piece_sequence(c.seq_off, c.n_seqs, KB_TOKENS, blockIdx.y, part);
+  const int first = c.seq_off[seq] + part * KB_TOKENS;
   const int count = min(KB_TOKENS, c.seq_off[seq + 1] - first);
   if (count <= 0) return;                                                // (the whole work-group)
   const int shared = FORM == 0 ? head / (c.heads / c.kv_heads) : head;
-  float* place = kb_place(c, seq, blockIdx.x, head);
+  float* place = kb_place(c, seq, part, head);
   const float rate = FORM == 0 ? -expf(c.A_log[head]) : 0.f;
   const bool per_head = FORM == 0 && c.decay_span == 1;
   if (FORM == 0 && tid < KB_TOKENS) {
@@ -732,7 +734,7 @@ __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall
 
 template <int DT>
 static void launch_keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
-  dim3 side((c.max_count + KB_TOKENS - 1) / KB_TOKENS, c.heads, c.n_seqs), block(256);
+  dim3 side(c.heads, c.tokens / KB_TOKENS + c.n_seqs), block(256);      // (the heads of a piece side by side: they share rows)
   dim3 walk((unsigned)((c.heads * c.n_seqs + 7) / 8 * 8 * (c.vdim / 16)));
   if (c.form == 0) {
     hipLaunchKernelGGL((keyed_blocks_kernel<0, DT>), side, block, 0, stream, c);
@@ -745,7 +747,9 @@ static void launch_keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
 
 // True if the call went in blocks: it brings the room, tiles of 16 and enough tokens.
 static bool keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
-  if (!c.blocks || c.max_count < KB_MIN_TOKENS || c.dim % 16 != 0 || c.dim > 128 || c.vdim % 16 != 0) return false;
+  if (!c.blocks || c.max_count < KB_MIN_TOKENS || c.dim % 16 != 0 || c.dim > 128 || c.vdim % 16 != 0 ||
+      c.tokens / KB_TOKENS + c.n_seqs > 65535 || (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30)
+    return false;
   switch (c.dim / 16) {
     case 1: launch_keyed_blocks<1>(stream, c); break;
     case 2: launch_keyed_blocks<2>(stream, c); break;

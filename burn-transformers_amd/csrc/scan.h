@@ -59,6 +59,26 @@ __device__ __forceinline__ int64_t span_block(const int* seq_off, int seq, int s
   return (int64_t)(seq_off[seq] / span + 2 * seq + 1 + part);
 }
 
+// Where pieces of `size` tokens are worked on side by side, piece k of sequence s is number seq_off[s] / size + s + k: all pieces of a
+// step have numbers below tokens / size + n_seqs, whatever its sequences bring (a grid of the longest sequence's pieces
+// for every sequence is mostly empty where a prompt comes beside single tokens: of 500 and 63 x 1 tokens with 8 heads 16,384
+// work-groups for 784, and the keyed scan took 256 us for 62).  A wave finds the sequence of a number, 64 sequences at a time; `part` is the piece (it may lie
+// behind the sequence's end).
+__device__ __forceinline__ int piece_sequence(const int* seq_off, int n_seqs, int size, int number, int& part) {
+  const int lane = threadIdx.x & 63;
+  int seq = 0, first = 0;
+  for (int s0 = 0; s0 < n_seqs; s0 += 64) {
+    const int s = s0 + lane, at = s < n_seqs ? seq_off[s] / size + s : 0x7fffffff;
+    const unsigned long long reached = __builtin_amdgcn_ballot_w64(at <= number);      // (the numbers grow with s)
+    if (reached == 0) break;
+    const int last = 63 - __builtin_clzll(reached);
+    seq = s0 + last;
+    first = __builtin_amdgcn_readlane(at, last);
+    if (last < 63) break;
+  }
+  part = number - first;
+  return seq;
+}
 
 // Sequences of at least this many spans are cut (fewer gain nothing over walking them).
 #define MIN_SPANS 3
@@ -88,4 +108,3 @@ static int span_tokens(int span, int max_count, const float* carry, int64_t wave
   if (tokens < span) tokens = span;
   return max_count >= MIN_SPANS * tokens ? tokens : 0;
 }
-

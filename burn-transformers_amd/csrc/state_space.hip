@@ -916,13 +916,14 @@ __global__ void __launch_bounds__(256) head_blocks_kernel(HeadScanCall c) {
   __shared__ __attribute__((aligned(16))) floatx4 parts[4][64];
   __shared__ float steps[HB_HEADS][HB_TOKENS], decays[HB_HEADS][HB_TOKENS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
-  const int seq = blockIdx.z, first = c.seq_off[seq] + (int)blockIdx.x * HB_TOKENS;
+  int part;
+  const int seq = piece_sequence(c.seq_off, c.n_seqs, HB_TOKENS, blockIdx.y, part), first = c.seq_off[seq] + part * HB_TOKENS;
   const int count = min(HB_TOKENS, c.seq_off[seq + 1] - first);
   if (count <= 0) return;                                                // (the whole work-group)
   const int per_group = c.heads / c.groups, sets = (per_group + HB_HEADS - 1) / HB_HEADS;
-  const int group = blockIdx.y / sets, head0 = group * per_group + blockIdx.y % sets * HB_HEADS;
+  const int group = blockIdx.x / sets, head0 = group * per_group + blockIdx.x % sets * HB_HEADS;
   const int heads = min(HB_HEADS, (group + 1) * per_group - head0);
-  float* place = hb_place(c, seq, blockIdx.x);
+  float* place = hb_place(c, seq, part);
   // rows behind the sequence's end hold zeros and decay by one: they change nothing
 #pragma unroll
   for (int j = 0; j < DT; ++j) {
@@ -945,7 +946,7 @@ __global__ void __launch_bounds__(256) head_blocks_kernel(HeadScanCall c) {
     const floatx4 q = *reinterpret_cast<const floatx4*>(&C[n][16 * tile + 4 * g]), k = *reinterpret_cast<const floatx4*>(&B[n][16 * tile + 4 * g]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], k[i], sums, 0, 0, 0);
-    if (blockIdx.y % sets == 0) {
+    if (blockIdx.x % sets == 0) {
       floatx4 u;
 #pragma unroll
       for (int i = 0; i < 4; ++i) u[i] = B[4 * g + i][16 * tile + n];
@@ -1103,7 +1104,7 @@ __global__ void __launch_bounds__(256, 2) head_blocks_walk_kernel(HeadScanCall c
 template <int DT>
 static void launch_head_blocks(hipStream_t stream, const HeadScanCall& c) {
   const int sets = (c.heads / c.groups + HB_HEADS - 1) / HB_HEADS;
-  dim3 side((c.max_count + HB_TOKENS - 1) / HB_TOKENS, c.groups * sets, c.n_seqs), block(256);
+  dim3 side(c.groups * sets, c.tokens / HB_TOKENS + c.n_seqs), block(256);
   dim3 walk((unsigned)((c.heads * c.n_seqs + 7) / 8 * 8 * (c.vdim / 16)));
   hipLaunchKernelGGL((head_blocks_kernel<DT>), side, block, 0, stream, c);
   hipLaunchKernelGGL((head_blocks_walk_kernel<DT>), walk, block, 0, stream, c);
@@ -1111,7 +1112,7 @@ static void launch_head_blocks(hipStream_t stream, const HeadScanCall& c) {
 
 // True if the call went in blocks: it brings the room, tiles of 16 and enough tokens.
 static bool head_blocks(hipStream_t stream, const HeadScanCall& c) {
-  if (!c.blocks || c.max_count < HB_MIN_TOKENS || c.state % 16 != 0 || c.state > 128 || c.vdim % 16 != 0 || c.n_seqs > 65535 ||
+  if (!c.blocks || c.max_count < HB_MIN_TOKENS || c.state % 16 != 0 || c.state > 128 || c.vdim % 16 != 0 || c.tokens / HB_TOKENS + c.n_seqs > 65535 ||
       (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30 || c.groups > 4096 || hb_floats(c) > 1 << 28 || 64 * c.ld > 1 << 30)
     return false;
   switch (c.state / 16) {

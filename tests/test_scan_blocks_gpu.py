@@ -37,7 +37,8 @@ def state_rows(state, heads, dim, vdim):
     ("head", 4, 2, 128, 128, [33, 1, 16, 47], False), ("head", 2, 2, 16, 16, [100, 32, 5], True),
     ("channel", 2, 1, 128, 32, [64, 17, 31], False), ("channel", 3, 3, 80, 48, [49, 2], True),
     ("forget", 2, 2, 128, 128, [130, 15, 1], False), ("forget", 3, 3, 48, 80, [35, 64], True),
-    ("channel", 1, 1, 64, 16, [400], False), ("forget", 1, 1, 32, 64, [333], True)])
+    ("channel", 1, 1, 64, 16, [400], False), ("forget", 1, 1, 32, 64, [333], True), ("head", 2, 2, 32, 32, [300] + [1] * 70 + [20], False),
+    ("forget", 2, 2, 32, 16, [1] * 64 + [300, 16, 1], False)])
 def test_blocks_of_tokens(form, heads, kv_heads, dim, vdim, lengths, strong):
     gen = torch.Generator().manual_seed(heads * 1000 + dim + len(lengths))
     qk, inner = kv_heads * dim, heads * vdim
@@ -141,7 +142,7 @@ def test_a_token_that_is_not_finite_spoils_no_earlier_one(form, where, value, to
 
 @pytest.mark.parametrize("heads,groups,vdim,state,lengths,strong", [
     (4, 1, 64, 128, [33, 1, 16, 47], False), (12, 1, 16, 16, [100, 32, 5], True), (6, 3, 48, 80, [49, 2], False),
-    (9, 1, 32, 48, [400], True), (2, 2, 16, 32, [64, 63, 65], False), (20, 2, 16, 128, [333, 17], False)])
+    (9, 1, 32, 48, [400], True), (2, 2, 16, 32, [64, 63, 65], False), (20, 2, 16, 128, [333, 17], False), (4, 1, 32, 32, [300] + [1] * 70 + [20], False)])
 def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
     gen = torch.Generator().manual_seed(heads * 1000 + state + len(lengths))
     inner, bc = heads * vdim, groups * state
