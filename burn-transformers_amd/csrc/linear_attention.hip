@@ -330,13 +330,20 @@ __global__ void __launch_bounds__(256) keyed_carry_kernel(KeyedScanCall c, int t
   slot[index] = state;
 }
 
+// Into spans of how many tokens the forget gate's long sequences are cut, 0 for not at all.
+static int keyed_span(const KeyedScanCall& c) {
+  const int tiles = (c.vdim + 3) / 4, groups = (tiles + KS_WAVES - 1) / KS_WAVES;
+  const int span = c.form == 1 ? span_tokens(c.span, c.max_count, c.carry, (int64_t)groups * KS_WAVES * c.heads * c.n_seqs, 1) : 0;
+  return span > 0 && (int64_t)c.n_seqs * ((c.max_count + span - 1) / span) <= 65535 ? span : 0;
+}
+
 template <int R>
 static void launch_keyed_scan(hipStream_t stream, const KeyedScanCall& c) {
   const int per_token = (c.form == 0 ? 3 : 2) * 16 * R + 8 * KS_WAVES + 1;      // planes, (v, beta) pairs, a decay
   const int tiles = (c.vdim + 3) / 4, groups = (tiles + KS_WAVES - 1) / KS_WAVES;
   dim3 block(KS_THREADS);
-  const int span = c.form == 1 ? span_tokens(c.span, c.max_count, c.carry, (int64_t)groups * KS_WAVES * c.heads * c.n_seqs, 1) : 0;
-  if (span > 0 && (int64_t)c.n_seqs * ((c.max_count + span - 1) / span) <= 65535) {
+  const int span = keyed_span(c);
+  if (span > 0) {
     KeyedScanCall cut = c;
     cut.span = span;
     const int chunk = span < KsRun<R>::MOST ? span : KsRun<R>::MOST;
@@ -732,6 +739,26 @@ __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall
 // 19.9 / 19.5, 13.8 / 13.0; 16 x 40 tokens 42.8 / 37.0, 56.3 / 39.3, 32.8 / 28.4; 4 x 48 tokens 22.9 / 19.6, 29.2 / 22.1, 20.0 / 15.0.
 #define KB_MIN_TOKENS 40
 
+// From there on the cheaper way is taken, by what was measured of both (us; a state of R tiles of 16 key channels): token by token a
+// launch and a token's chain for every token of the longest sequence, in spans the chain of one span twice and a step of the
+// carry for every span; in blocks two launches and a block's chain, and for every sequence that is short beside the longest one
+// the work-groups that bring its state in and out (they hold a compute unit's registers, two to a unit).  Measured (start
+// to end, token by token or in spans / in blocks): forget gate, 2 heads of 16 x 16, 4,000 tokens 36 / 90, 4 of 64 x 64 68 / 106, 8 of 128 x 128
+// 246 / 167; delta rule with one decay a head, 8 heads of 128 x 128, 40 tokens and 63 single ones 33 / 54, 100 and 63 46 / 55, 500 and 63
+// 192 / 61, 1,000 and 200 375 / 149; 16 heads, 64 and 31 36 / 55; 2 heads of 16 x 16, 40 tokens 11 / 15.
+static bool blocks_pay(const KeyedScanCall& c) {
+  const float r = c.dim / 16, longest = c.max_count;
+  const int span = keyed_span(c);
+  const float token = c.form == 1 ? 0.11f + 0.0275f * r : c.decay_span == 1 ? 0.17f + 0.026f * r : 0.165f + 0.043f * r;
+  const float start = c.form == 1 ? 3.5f : 3.f + 0.4f * r;
+  const float walk = span == 0 ? start + token * longest
+                               : 2.f + 2.f * token * span * span_crowding((int64_t)c.heads * (c.vdim / 4), c.tokens, span) +
+                                     (0.3f + 2e-5f * c.heads * c.dim * c.vdim) * (longest / span);
+  const float others = short_sequences(c.tokens, c.n_seqs, c.max_count) * (c.heads * (c.vdim / 16)) * (0.003f + 4e-5f * c.dim);
+  const float blocks = (c.form == 1 ? 8.f + 0.6f * r + (0.0195f + 0.0026f * r) * longest : 13.f + 0.5f * r + (0.028f + 0.0033f * r) * longest) + others;
+  return blocks < walk;
+}
+
 template <int DT>
 static void launch_keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
   dim3 side(c.heads, c.tokens / KB_TOKENS + c.n_seqs), block(256);      // (the heads of a piece side by side: they share rows)
@@ -748,7 +775,7 @@ static void launch_keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
 // True if the call went in blocks: it brings the room, tiles of 16 and enough tokens.
 static bool keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
   if (!c.blocks || c.max_count < KB_MIN_TOKENS || c.dim % 16 != 0 || c.dim > 128 || c.vdim % 16 != 0 ||
-      c.tokens / KB_TOKENS + c.n_seqs > 65535 || (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30)
+      c.tokens / KB_TOKENS + c.n_seqs > 65535 || (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30 || !blocks_pay(c))
     return false;
   switch (c.dim / 16) {
     case 1: launch_keyed_blocks<1>(stream, c); break;

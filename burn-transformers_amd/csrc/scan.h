@@ -108,3 +108,18 @@ static int span_tokens(int span, int max_count, const float* carry, int64_t wave
   if (tokens < span) tokens = span;
   return max_count >= MIN_SPANS * tokens ? tokens : 0;
 }
+
+// What a token of a span costs beside one of a wave alone on its SIMD, with `waves` walking a sequence: spans bring up to four
+// times `fill` to a SIMD, which then share it (measured: four take 1.6 to 2 times as long as one).
+static float span_crowding(int64_t waves, int tokens, int span) {
+  const float on_a_simd = (float)waves * tokens / span / simd_count();
+  return on_a_simd > 1.f ? 1.f + 0.2f * (on_a_simd - 1.f) : 1.f;
+}
+
+// How many sequences of a step it holds beyond those that would bring its tokens at the longest one's length: none where all are
+// alike, all but one where a prompt comes beside single tokens.
+static int64_t short_sequences(int tokens, int n_seqs, int max_count) {
+  const int64_t alike = ((int64_t)tokens + max_count - 1) / max_count;
+  return n_seqs > alike ? n_seqs - alike : 0;
+}
+

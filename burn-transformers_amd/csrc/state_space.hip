@@ -858,12 +858,17 @@ __global__ void __launch_bounds__(256) head_carry_kernel(HeadScanCall c, int til
   slot[index] = state;
 }
 
+// Into spans of how many tokens the step's long sequences are cut, 0 for not at all.
+static int head_span(const HeadScanCall& c) {
+  return span_tokens(c.span, c.max_count, c.carry, (int64_t)((c.vdim + 3) / 4) * c.heads * c.n_seqs, 1);
+}
+
 template <int R>
 static void launch_head_scan_r(hipStream_t stream, const HeadScanCall& c) {
   const int per_token = 2 * 16 * R + 16 * HS_WAVES;
   const int tiles = (c.vdim + 3) / 4, groups = (tiles + HS_WAVES - 1) / HS_WAVES;
   dim3 block(64 * HS_WAVES);
-  const int span = span_tokens(c.span, c.max_count, c.carry, (int64_t)tiles * c.heads * c.n_seqs, 1);
+  const int span = head_span(c);
   if (span > 0) {
     HeadScanCall cut = c;
     cut.span = span;
@@ -1110,10 +1115,24 @@ static void launch_head_blocks(hipStream_t stream, const HeadScanCall& c) {
   hipLaunchKernelGGL((head_blocks_walk_kernel<DT>), walk, block, 0, stream, c);
 }
 
+// Whether blocks are the cheaper way, by what was measured of both as for the keyed scan (linear_attention.hip; R tiles of 16
+// state elements).  Measured (us, token by token or in spans / in blocks): 8 heads of 64 x 16, 4,000 tokens 55 / 138, 1,000 25 / 42, 64 tokens 9 / 12;
+// 24 of 64 x 64, 4,000 tokens 174 / 125; 32 of 64 x 128, 64 tokens and 31 single ones 29 / 41, 300 and 20 95 / 36, 1,000 and 200 306 / 193.
+static bool blocks_pay(const HeadScanCall& c) {
+  const float r = c.state / 16, longest = c.max_count;
+  const int span = head_span(c);
+  const float token = 0.06f + 0.03f * r;
+  const float walk = span == 0 ? 3.5f + token * longest
+                               : 2.f + 2.f * token * span * span_crowding((int64_t)c.heads * (c.vdim / 4), c.tokens, span) +
+                                     (0.45f + 1.6e-5f * c.heads * c.state * c.vdim) * (longest / span);
+  const float others = short_sequences(c.tokens, c.n_seqs, c.max_count) * (c.heads * (c.vdim / 16)) * (0.003f + 4e-5f * c.state);
+  return 9.f + 0.2f * r + (0.0335f + 0.001f * r) * longest + others < walk;
+}
+
 // True if the call went in blocks: it brings the room, tiles of 16 and enough tokens.
 static bool head_blocks(hipStream_t stream, const HeadScanCall& c) {
   if (!c.blocks || c.max_count < HB_MIN_TOKENS || c.state % 16 != 0 || c.state > 128 || c.vdim % 16 != 0 || c.tokens / HB_TOKENS + c.n_seqs > 65535 ||
-      (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30 || c.groups > 4096 || hb_floats(c) > 1 << 28 || 64 * c.ld > 1 << 30)
+      (int64_t)c.heads * c.n_seqs * (c.vdim / 16) > 1 << 30 || c.groups > 4096 || hb_floats(c) > 1 << 28 || 64 * c.ld > 1 << 30 || !blocks_pay(c))
     return false;
   switch (c.state / 16) {
     case 1: launch_head_blocks<1>(stream, c); break;

@@ -247,3 +247,37 @@ def test_which_sequences_eight_lanes_cut(channels, state, counts, cut):
     K.selective_scan(x, z, dt, bc[:, :state], bc[:, state:], A_log, D, out, held, step, carry=carry, span=K.SELECTIVE_SPAN)
     assert bool(torch.isfinite(carry).any()) == cut
     assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(held).all())
+
+
+# which way a step goes (only blocks write their room): the longest sequence, how many are short beside it, sizes of heads and states;
+# `spans`: with room for spans
+@pytest.mark.parametrize("form,heads,dim,vdim,counts,spans,blocked", [
+    ("head", 8, 128, 128, [1024] * 2, False, True), ("head", 8, 128, 128, [39], False, False), ("channel", 8, 128, 128, [40], False, True),
+    ("head", 8, 128, 128, [40] + [1] * 63, False, False), ("head", 8, 128, 128, [500] + [1] * 63, False, True), ("head", 2, 16, 16, [40], False, False),
+    ("forget", 8, 128, 128, [100] * 16, True, True), ("forget", 2, 16, 16, [1000], True, False), ("forget", 2, 16, 16, [1000], False, True),
+    ("forget", 8, 128, 128, [4000], True, True), ("scan", 32, 128, 64, [1024] * 2, True, True), ("scan", 8, 16, 64, [1000], True, False),
+    ("scan", 32, 128, 64, [64] + [1] * 31, True, False), ("scan", 32, 128, 64, [300] + [1] * 20, True, True)])
+def test_which_steps_go_in_blocks(form, heads, dim, vdim, counts, spans, blocked):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are those of 256 compute units")
+    gen, total, inner = torch.Generator().manual_seed(9), sum(counts), heads * vdim
+    step = make_step(torch.float32, counts)
+    state, y = torch.zeros(len(counts), heads * dim * vdim, device=DEV), torch.empty(total, inner, device=DEV)
+    if form == "scan":
+        room, carry = K.head_blocks(step, heads, vdim, dim, 1), K.scan_carry(step, heads * dim * vdim, heads) if spans else None
+        on, zeros = torch.randn(total, inner + 2 * dim + heads, generator=gen).to(DEV), torch.zeros(heads, device=DEV)
+    else:
+        qk, decays = heads * dim, heads if form == "head" else heads * dim
+        room, carry = K.scan_blocks(step, heads, dim, vdim), K.scan_carry(step, heads * dim * vdim, heads * dim) if spans else None
+        on, zeros = torch.randn(total, 2 * qk + inner + decays + heads, generator=gen).to(DEV), torch.zeros(decays, device=DEV)
+    room.fill_(float("nan"))
+    if form == "scan":
+        K.head_scan(on[:, :inner], on[:, inner:inner + dim], on[:, inner + dim:inner + 2 * dim], on[:, inner + 2 * dim:], zeros, zeros, zeros, y, state,
+                    step, heads, vdim, dim, 1, carry=carry, blocks=room)
+    else:
+        extra = dict(g_bias=zeros, lower=zeros + 0.5) if form == "forget" else \
+            dict(beta=on[:, -heads:], A_log=zeros[:heads], unit=True, q_scale=dim ** -0.5, decay_per_head=form == "head", dt_bias=zeros)
+        K.keyed_scan(on[:, :qk], None if form == "forget" else on[:, qk:2 * qk], on[:, 2 * qk:2 * qk + inner], on[:, 2 * qk + inner:2 * qk + inner + decays],
+                     y, state, step, heads, heads, dim, vdim, "forget" if form == "forget" else "delta", carry=carry, blocks=room, **extra)
+    assert bool(torch.isfinite(room).any()) == blocked
+    assert bool(torch.isfinite(y).all()) and bool(torch.isfinite(state).all())
