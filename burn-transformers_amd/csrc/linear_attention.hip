@@ -405,10 +405,10 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
   __shared__ float strength[KB_TOKENS], one[KB_TOKENS];                  // beta, and a decay the whole head shares
   const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int part;
-  const int seq = piece_sequence(c.seq_off, c.n_seqs, KB_TOKENS, blockIdx.y, part);
+  const int seq = piece_sequence(c.seq_off, c.n_seqs, c.tokens, c.max_count, KB_TOKENS, blockIdx.y, part);
+  if (seq < 0) return;                                                   // (the whole work-group)
   const int first = c.seq_off[seq] + part * KB_TOKENS;
   const int count = min(KB_TOKENS, c.seq_off[seq + 1] - first);
-  if (count <= 0) return;                                                // (the whole work-group)
   const int shared = FORM == 0 ? head / (c.heads / c.kv_heads) : head;
   float* place = kb_place(c, seq, part, head);
   const float rate = FORM == 0 ? -expf(c.A_log[head]) : 0.f;

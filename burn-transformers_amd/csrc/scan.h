@@ -59,25 +59,37 @@ __device__ __forceinline__ int64_t span_block(const int* seq_off, int seq, int s
   return (int64_t)(seq_off[seq] / span + 2 * seq + 1 + part);
 }
 
-// Where pieces of `size` tokens are worked on side by side, piece k of sequence s is number seq_off[s] / size + s + k: all pieces of a
-// step have numbers below tokens / size + n_seqs, whatever its sequences bring (a grid of the longest sequence's pieces
-// for every sequence is mostly empty where a prompt comes beside single tokens: of 500 and 63 x 1 tokens with 8 heads 16,384
-// work-groups for 784, and the keyed scan took 256 us for 62).  A wave finds the sequence of a number, 64 sequences at a time; `part` is the piece (it may lie
-// behind the sequence's end).
-__device__ __forceinline__ int piece_sequence(const int* seq_off, int n_seqs, int size, int number, int& part) {
-  const int lane = threadIdx.x & 63;
-  int seq = 0, first = 0;
-  for (int s0 = 0; s0 < n_seqs; s0 += 64) {
-    const int s = s0 + lane, at = s < n_seqs ? seq_off[s] / size + s : 0x7fffffff;
-    const unsigned long long reached = __builtin_amdgcn_ballot_w64(at <= number);      // (the numbers grow with s)
-    if (reached == 0) break;
-    const int last = 63 - __builtin_clzll(reached);
-    seq = s0 + last;
-    first = __builtin_amdgcn_readlane(at, last);
-    if (last < 63) break;
+// Pieces of `size` tokens that are worked on side by side are numbered through the step, a sequence's behind those of the ones
+// before it: there are at most tokens / size + n_seqs of them, whatever its sequences bring (a grid of the longest
+// sequence's pieces for every sequence is mostly empty where a prompt comes beside single tokens: of 500 and 63 x 1 tokens with
+// 8 heads 16,384 work-groups for 784, and the keyed scan took 256 us for 62).  Where all sequences are alike the sequence of a
+// number is a quotient, elsewhere a wave finds it, 64 sequences at a time; `part` is the piece.  Numbers behind the last piece have no
+// sequence (-1): they come last, so that the others are dealt evenly to the compute units (empty ones among them cost the
+// selective scan a fifth).
+__device__ __forceinline__ int piece_sequence(const int* seq_off, int n_seqs, int tokens, int longest, int size, int number, int& part) {
+  if ((int64_t)n_seqs * longest == tokens) {
+    const int pieces = (longest + size - 1) / size, seq = number / pieces;
+    part = number - seq * pieces;
+    return seq < n_seqs ? seq : -1;
   }
-  part = number - first;
-  return seq;
+  const int lane = threadIdx.x & 63;
+  for (int s0 = 0; s0 < n_seqs; s0 += 64) {
+    const int s = s0 + lane, pieces = s < n_seqs ? (seq_off[s + 1] - seq_off[s] + size - 1) / size : 0;
+    int upto = pieces;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int before = __shfl_up(upto, o, 64);
+      upto += lane >= o ? before : 0;
+    }
+    const unsigned long long reached = __builtin_amdgcn_ballot_w64(upto > number);
+    if (reached != 0) {
+      const int first = __builtin_ctzll(reached);
+      part = number - (__builtin_amdgcn_readlane(upto, first) - __builtin_amdgcn_readlane(pieces, first));
+      return s0 + first;
+    }
+    number -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return -1;
 }
 
 // Sequences of at least this many spans are cut (fewer gain nothing over walking them).

@@ -492,9 +492,12 @@ __device__ __forceinline__ float decay_of(float v) {
 template <typename T, int N, int PHASE>
 __global__ void __launch_bounds__(64) selective_lanes_kernel(SelectiveScanCall c) {
   typedef const __attribute__((address_space(4))) float* Uniform;
-  const int lane = threadIdx.x, ch = blockIdx.x * 64 + lane, seq = blockIdx.y, part = blockIdx.z;
+  const int lane = threadIdx.x, ch = blockIdx.x * 64 + lane;
   const bool live = ch < c.channels;
   const int chs = live ? ch : c.channels - 1;        // idle lanes read a valid channel and write nothing
+  int part = 0;
+  const int seq = PHASE ? piece_sequence(c.seq_off, c.n_seqs, c.tokens, c.max_count, c.span, blockIdx.y, part) : blockIdx.y;
+  if (PHASE && seq < 0) return;
   int first = c.seq_off[seq], last = c.seq_off[seq + 1];
   const int64_t per_span = (int64_t)c.channels * c.state + c.channels;
   float* mine = nullptr;                             // this span's block of the carry
@@ -645,14 +648,26 @@ static void launch_selective_scan_r(hipStream_t stream, const SelectiveScanCall&
   hipLaunchKernelGGL((selective_scan_kernel<T, R>), grid, block, (size_t)chunk * per_token * sizeof(float), stream, c, chunk, 0);
 }
 
+// Waves of 64 channels that the step's tokens would make if all its sequences were as long as the longest: a prompt beside single
+// tokens is one long walk and is cut into spans, however many tokens come with it.
+static int64_t lane_waves(const SelectiveScanCall& c) {
+  return (int64_t)((c.channels + 63) / 64) * (((int64_t)c.tokens + c.max_count - 1) / c.max_count);
+}
+
+// Spans have the room's shortest length at least, and so many tokens that walking one twice (0.27 us a token with 16 states, twice that
+// with 32) takes no less than the carry, which goes through them in order (0.36 us each): measured (us) for one sequence of 4,000 tokens
+// of 128 channels 110 in spans of 16, 78 so, of 512 channels 125 and 85.  Measured beside single tokens (eight lanes a channel / one by the sequences' number /
+// so; 2,048 channels of 16): 1,000 and 32 345 / 497 / 60, 500 and 63 175 / 243 / 49, 64 and 31 25 / 34 / 23.
 template <typename T, int N>
 static void launch_selective_lanes(hipStream_t stream, const SelectiveScanCall& c) {
   const int groups = (c.channels + 63) / 64;
-  const int span = span_tokens(c.span, c.max_count, c.carry, (int64_t)groups * c.n_seqs, 1, 2);
-  if (span > 0 && (c.max_count + span - 1) / span <= 65535) {
+  int shortest = c.span;
+  while (shortest > 0 && 3 * (int64_t)shortest * shortest * (N > 16 ? N / 16 : 1) < 2 * (int64_t)c.max_count) ++shortest;
+  const int span = span_tokens(shortest, c.max_count, c.carry, lane_waves(c), 1, 2);
+  if (span > 0 && c.tokens / span + c.n_seqs <= 65535) {
     SelectiveScanCall cut = c;
     cut.span = span;
-    dim3 grid(groups, c.n_seqs, (c.max_count + span - 1) / span);
+    dim3 grid(groups, c.tokens / span + c.n_seqs);
     hipLaunchKernelGGL((selective_lanes_kernel<T, N, 1>), grid, dim3(64), 0, stream, cut);
     hipLaunchKernelGGL(selective_carry_kernel, dim3((c.channels * c.state + 255) / 256, c.n_seqs), dim3(256), 0, stream, cut);
     hipLaunchKernelGGL((selective_lanes_kernel<T, N, 3>), grid, dim3(64), 0, stream, cut);
@@ -663,8 +678,10 @@ static void launch_selective_lanes(hipStream_t stream, const SelectiveScanCall& 
 
 template <typename T>
 static int launch_selective_scan(hipStream_t stream, const SelectiveScanCall& c) {
-  const bool many = c.max_count >= (c.state == 32 ? SL_MIN_TOKENS_32 : SL_MIN_TOKENS) ||
-      (c.max_count >= SL_MIN_TOKENS / 4 && (int64_t)((c.channels + 63) / 64) * c.n_seqs >= SL_MIN_WAVES);
+  // (many short sequences beside the longest are waves of a few tokens: 64 tokens and 31 single ones 25 us with eight lanes, 30 with one)
+  const bool others = short_sequences(c.tokens, c.n_seqs, c.max_count) * ((c.channels + 63) / 64) > 512;
+  const bool many = c.max_count >= (c.state == 32 ? SL_MIN_TOKENS_32 : others ? 2 * SL_MIN_TOKENS : SL_MIN_TOKENS) ||
+      (c.max_count >= SL_MIN_TOKENS / 4 && lane_waves(c) >= SL_MIN_WAVES);
   if (many && (c.state == 8 || c.state == 16 || c.state == 32)) {
     if (c.state == 8) launch_selective_lanes<T, 8>(stream, c);
     else if (c.state == 16) launch_selective_lanes<T, 16>(stream, c);
@@ -922,9 +939,9 @@ __global__ void __launch_bounds__(256) head_blocks_kernel(HeadScanCall c) {
   __shared__ float steps[HB_HEADS][HB_TOKENS], decays[HB_HEADS][HB_TOKENS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, n = lane & 15;
   int part;
-  const int seq = piece_sequence(c.seq_off, c.n_seqs, HB_TOKENS, blockIdx.y, part), first = c.seq_off[seq] + part * HB_TOKENS;
-  const int count = min(HB_TOKENS, c.seq_off[seq + 1] - first);
-  if (count <= 0) return;                                                // (the whole work-group)
+  const int seq = piece_sequence(c.seq_off, c.n_seqs, c.tokens, c.max_count, HB_TOKENS, blockIdx.y, part);
+  if (seq < 0) return;                                                   // (the whole work-group)
+  const int first = c.seq_off[seq] + part * HB_TOKENS, count = min(HB_TOKENS, c.seq_off[seq + 1] - first);
   const int per_group = c.heads / c.groups, sets = (per_group + HB_HEADS - 1) / HB_HEADS;
   const int group = blockIdx.x / sets, head0 = group * per_group + blockIdx.x % sets * HB_HEADS;
   const int heads = min(HB_HEADS, (group + 1) * per_group - head0);

@@ -189,7 +189,8 @@ def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
 @pytest.mark.parametrize("channels,state,lengths,spans,strong", [
     (100, 16, [64, 1, 130], True, False), (64, 8, [65, 63], False, True), (200, 32, [300, 17, 64], True, False), (70, 16, [500], True, True),
     (1100, 16, [20] * 16, True, False), (48, 16, [63, 5], True, False), (100, 32, [191, 64], True, False), (100, 32, [192, 2], True, True),
-    (100, 24, [64, 200], True, False)])
+    (100, 24, [64, 200], True, False), (100, 16, [300] + [1] * 70 + [20], True, False), (70, 8, [1] * 64 + [200, 16, 1], True, False),
+    (130, 32, [1, 400, 1, 1], True, False)])
 def test_channels_in_lanes(channels, state, lengths, spans, strong):
     gen = torch.Generator().manual_seed(channels + state + len(lengths))
     A_log, D = torch.log(torch.rand(channels, state, generator=gen) * 7.0 + 0.5), torch.randn(channels, generator=gen)
@@ -247,6 +248,14 @@ def test_which_sequences_eight_lanes_cut(channels, state, counts, cut):
     K.selective_scan(x, z, dt, bc[:, :state], bc[:, state:], A_log, D, out, held, step, carry=carry, span=K.SELECTIVE_SPAN)
     assert bool(torch.isfinite(carry).any()) == cut
     assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(held).all())
+
+
+# a long sequence is cut into spans whatever stands beside it: single tokens are no waves that would fill the chip
+@pytest.mark.parametrize("channels,state,counts,cut", [
+    (2048, 16, [1000] + [1] * 32, True), (2048, 16, [300] * 8, True), (2048, 16, [1000] * 40, False), (2048, 32, [500] + [1] * 63, True),
+    (2048, 16, [64] + [1] * 31, False), (4096, 16, [40] + [1] * 63, False)])
+def test_which_sequences_lanes_cut(channels, state, counts, cut):
+    test_which_sequences_eight_lanes_cut(channels, state, counts, cut)
 
 
 # which way a step goes (only blocks write their room): the longest sequence, how many are short beside it, sizes of heads and states;
