@@ -111,11 +111,14 @@ __global__ void __launch_bounds__(256) causal_conv_kernel(CausalConvCall c) {
 
 // The same for steps of many tokens: a thread takes a channel of CONV_RUN tokens one after the other, so that an input is read
 // once and not once a tap, the taps stay in registers and all of a run's inputs are on their way together; a run that
-// begins a sequence takes its window's front from the state, one that straddles two goes token by token.  Sums are taken in
-// the same order as above.  Measured with the state's kernel (us, a token a thread / in runs; channels of 4 taps): 2,048 tokens of 2,048
-// 28.4 / 12.4 (the bytes: 6.9), 2 x 256 of 2,048 9.3 / 5.9, 16 x 40 11.2 / 6.8, 3 x 100 of 1,536 6.6 / 7.4; runs of 16 17.2.
+// begins a sequence takes its window's front from the state, one that straddles two reads the tables for every token.  Sums are
+// taken in the same order as above.  Measured with the state's kernel (us, a token a thread / in runs; channels of 4 taps): 2,048 tokens of 2,048
+// 28.4 / 12.4 (the bytes: 6.9), 2 x 256 of 2,048 9.3 / 5.9, 16 x 40 11.2 / 6.8, 3 x 100 of 1,536 6.6 / 7.4; runs of 16 17.2.  A run that
+// straddles has one trip to memory more, which few values do not hide: 500 and 63 x 1 tokens of 300 channels 6.7 / 7.6, of 2,048 11.3 / 9.2,
+// 100 x 16 of 300 7.9 / 7.6 (token after token within the run 9.4, 10.9, 8.0).
 #define CONV_RUN 8
 #define CONV_MIN_TOKENS 384
+#define CONV_MIN_VALUES 350000
 
 template <typename T, int TAPS>
 __global__ void __launch_bounds__(256) causal_conv_run_kernel(CausalConvCall c) {
@@ -155,18 +158,28 @@ __global__ void __launch_bounds__(256) causal_conv_run_kernel(CausalConvCall c) 
     }
     return;
   }
-  for (int i = 0; i < count; ++i) {
-    const int t = t0 + i, seq = c.tok_seq[t], local = t - c.seq_off[seq];
-    const float* held = c.state + (int64_t)c.slots[seq] * c.state_stride;
-    float sum = bias;
+  // (all tokens' table reads, then all their inputs on their way together; behind the step's end the last token again)
+  float u[CONV_RUN][TAPS];
+#pragma unroll
+  for (int i = 0; i < CONV_RUN; ++i) {
+    const int k = min(i, count - 1), seq = c.tok_seq[t0 + k], local = t0 + k - c.seq_off[seq];
+    const float* held = c.state + (int64_t)c.slots[seq] * c.state_stride + ch;
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) {
       const int back = TAPS - 1 - j, src = local - back;
-      sum = fmaf(w[j], src >= 0 ? in[(int64_t)(i - back) * c.ld_in] : held[(int64_t)(TAPS - 1 + src) * c.channels + ch], sum);
+      u[i][j] = *(src >= 0 ? in + (int64_t)(k - back) * c.ld_in : held + (int64_t)(TAPS - 1 + src) * c.channels);
     }
+  }
+#pragma unroll
+  for (int i = 0; i < CONV_RUN; ++i) {
+    float sum = bias;
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) sum = fmaf(w[j], u[i][j], sum);
     const float y = c.act == 0 ? silu_f(sum) : sum;
-    out[(int64_t)i * c.ld_out] = y;
-    if (cast) cast[(int64_t)t * c.ld_cast + ch] = from_float<T>(y);
+    if (i < count) {
+      out[(int64_t)i * c.ld_out] = y;
+      if (cast) cast[(int64_t)(t0 + i) * c.ld_cast + ch] = from_float<T>(y);
+    }
   }
 }
 
@@ -217,7 +230,7 @@ BT_EXPORT int bt_causal_conv_call(void* stream, const CausalConvCall* c) {
       hipLaunchKernelGGL((causal_conv_kernel<bf16_t, true>), grid, block, 0, (hipStream_t)stream, *c);
     return bt_check_launch("causal_conv");
   }
-  const bool run = c->tokens >= CONV_MIN_TOKENS && (c->cast_dtype == 0 ? launch_conv_run<float>((hipStream_t)stream, *c, cols)
+  const bool run = c->tokens >= CONV_MIN_TOKENS && (int64_t)c->tokens * c->channels >= CONV_MIN_VALUES && (c->cast_dtype == 0 ? launch_conv_run<float>((hipStream_t)stream, *c, cols)
                                                                       : launch_conv_run<bf16_t>((hipStream_t)stream, *c, cols));
   if (run) {
   } else if (c->cast_dtype == 0)
