@@ -7,6 +7,8 @@
 //   * selective scan (one state row per channel, one decay per state element), with the output gate
 //   * scan with one decay per head and a state of [state, head size] (state-space duality form)
 //   * gate, then RMS norm in equal parts
+#include <type_traits>
+
 #include "host.h"
 #include "scan.h"
 
@@ -524,11 +526,16 @@ __global__ void __launch_bounds__(64) selective_lanes_kernel(SelectiveScanCall c
   float* held = c.S + (int64_t)c.slots[seq] * c.state_stride + (int64_t)chs * N;
   const float* start = PHASE == 3 ? mine - per_span + (int64_t)chs * N : held;
   float A[N], S[N];
+  bool mild = true;
 #pragma unroll
   for (int n = 0; n < N; ++n) {
-    A[n] = fmaxf(-expf(c.A_log[(int64_t)chs * N + n]), -1e8f);
+    A[n] = -expf(c.A_log[(int64_t)chs * N + n]);
     S[n] = PHASE != 1 ? start[n] : 0.f;
+    mild = mild && A[n] >= -1e8f;
   }
+  // (a product of a step, at most 1e30, and a mild A is finite; beyond, where the exponential above would end in a difference of
+  // infinities, the whole wave takes expf)
+  const bool all_mild = __builtin_amdgcn_ballot_w64(!mild) == 0;
   const float Dc = c.D[chs];
   T* out = static_cast<T*>(c.out) + (int64_t)first * c.ld_out + chs;
   const float *dt_at = c.dt + (int64_t)first * c.ld_dt + chs, *x_at = c.x + (int64_t)first * c.ld_x + chs, *z_at = c.z + (int64_t)first * c.ld_z + chs;
@@ -552,7 +559,7 @@ __global__ void __launch_bounds__(64) selective_lanes_kernel(SelectiveScanCall c
       if (PHASE != 1) q_to[n] = from_q[n];
     }
   };
-  auto token = [&](int t, int u) {
+  auto token = [&](int t, int u, auto steep) __attribute__((always_inline)) {
     const float dt = dts[u], xv = xs[u], z = PHASE != 1 ? zs[u] : 0.f;
     float b_next[N], q_next[N];
     fetch_row(t + 1, b_next, q_next);
@@ -562,7 +569,7 @@ __global__ void __launch_bounds__(64) selective_lanes_kernel(SelectiveScanCall c
     float acc = 0.f, acc_odd = 0.f;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      S[n] = fmaf(decay_of(step * A[n]), S[n], dx * b[n]);
+      S[n] = fmaf(decltype(steep)::value ? expf(dt * A[n]) : decay_of(step * A[n]), S[n], dx * b[n]);
       if (PHASE != 1) {
         if (n & 1) acc_odd = fmaf(S[n], q[n], acc_odd);
         else acc = fmaf(S[n], q[n], acc);
@@ -579,13 +586,17 @@ __global__ void __launch_bounds__(64) selective_lanes_kernel(SelectiveScanCall c
   fetch_row(0, b, q);
 #pragma unroll
   for (int u = 0; u < SL_AHEAD; ++u) fetch(u, u);
-  int t = 0;
-  for (; t + SL_AHEAD <= count; t += SL_AHEAD)
+  auto walk = [&](auto steep) __attribute__((always_inline)) {
+    int t = 0;
+    for (; t + SL_AHEAD <= count; t += SL_AHEAD)
 #pragma unroll
-    for (int u = 0; u < SL_AHEAD; ++u) token(t + u, u);
+      for (int u = 0; u < SL_AHEAD; ++u) token(t + u, u, steep);
 #pragma unroll
-  for (int u = 0; u < SL_AHEAD - 1; ++u)
-    if (t + u < count) token(t + u, u);
+    for (int u = 0; u < SL_AHEAD - 1; ++u)
+      if (t + u < count) token(t + u, u, steep);
+  };
+  if (__builtin_expect(all_mild, 1)) walk(std::false_type());
+  else walk(std::true_type());
   if (PHASE == 1) {
     if (live) {
 #pragma unroll

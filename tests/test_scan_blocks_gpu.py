@@ -290,3 +290,32 @@ def test_which_steps_go_in_blocks(form, heads, dim, vdim, counts, spans, blocked
                      y, state, step, heads, heads, dim, vdim, "forget" if form == "forget" else "delta", carry=carry, blocks=room, **extra)
     assert bool(torch.isfinite(room).any()) == blocked
     assert bool(torch.isfinite(y).all()) and bool(torch.isfinite(state).all())
+
+
+def test_steep_decays_of_channels_in_lanes():
+    """A decay's exponent is the step times exp(A_log), however large that is: steps of nearly nothing, of nothing and without end."""
+    gen, channels, state, total = torch.Generator().manual_seed(10), 70, 16, 100
+    A_log = torch.rand(channels, state, generator=gen) * 2.0
+    A_log[::3] = torch.rand(A_log[::3].shape, generator=gen) * 3.0 + 18.0          # exp(A_log): 6.6e7 to 1.3e9
+    A_log[5] = 80.0
+    x, z, B, C = [torch.randn(total, n, generator=gen) for n in (channels, channels, state, state)]
+    dt = torch.exp(torch.rand(total, channels, generator=gen) * 4.0 - 21.0)          # 7.6e-10 to 4e-8
+    dt[40, ::2], dt[41], x[41], dt[60, 5] = 0.0, float("inf"), 0.0, 1e-30
+    x[40] = x[60] = 0.0
+    S, want = torch.zeros(channels, state, dtype=torch.float64), []
+    A = -torch.exp(A_log.double())
+    for t in range(total):
+        step = dt[t].double()[:, None]
+        S = torch.exp((step * A).clamp(min=-800.0)) * S + torch.where(x[t][:, None] == 0, 0.0, step * x[t].double()[:, None] * B[t].double())
+        zt = z[t].double()
+        want.append((S * C[t].double()).sum(1) * zt * torch.sigmoid(zt))
+    held, out = torch.zeros(1, channels * state, device=DEV), torch.empty(total, channels, device=DEV)
+    step = make_step(torch.float32, [total])
+    dt[41] = 1e38                                                       # (an infinite step times no input is not a number)
+    on = lambda v: v.contiguous().to(DEV)
+    bc = on(torch.cat([B, C], 1))
+    K.selective_scan(on(x), on(z), on(dt), bc[:, :state], bc[:, state:], on(A_log), torch.zeros(channels, device=DEV), out, held, step,
+                     carry=K.scan_carry(step, channels * state, channels, K.SELECTIVE_SPAN), span=K.SELECTIVE_SPAN)
+    # exponents of up to 50 are products rounded to 32 bits: 50 * 2^-24, a few tokens' worth
+    assert rel_err(out.cpu(), torch.stack(want)) < 1e-5
+    assert rel_err(held.view(channels, state).cpu(), S) < 1e-5
