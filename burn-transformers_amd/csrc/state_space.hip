@@ -1027,10 +1027,16 @@ struct HbStage {
   float m, x[4], all;
 };
 
+// M's zeros for the tokens behind a row's own are multiplied too, so an x there that is not finite makes the row not a number.  A
+// work-group that has met one (`seen` is not a number then) goes through its sequence again behind the walk, token by token from the state
+// that still lies in its slot.  (us for 2 x 1,024 tokens of 32 heads of 64 x 128 / 4,000 of 24 of 64 x 64: without 57.5 / 123.5, so 58.2 / 129;
+// summing again in the block that holds it, a test for every block, 60 to 62 / 130 to 138; a second walk over blocks in this
+// kernel 59 / 131, in a function of its own, for its scratch memory, 72 / 136.)
 template <int DT>
 __global__ void __launch_bounds__(256, 2) head_blocks_walk_kernel(HeadScanCall c) {
   constexpr int TW = (DT + 3) / 4, DIM = 16 * DT;
   __shared__ __attribute__((aligned(16))) floatx4 parts[2][4][64];
+  __shared__ int spoiled[4];
   // the columns of a head and sequence, and the heads of a group, read the same operands: they are numbered onto one XCD
   const int columns = c.vdim / 16, pair = blockIdx.x / (8 * columns) * 8 + blockIdx.x % 8;
   if (pair >= c.heads * c.n_seqs) return;
@@ -1049,6 +1055,7 @@ __global__ void __launch_bounds__(256, 2) head_blocks_walk_kernel(HeadScanCall c
 #pragma unroll
     for (int i = 0; i < 4; ++i) S[j][i] = mine(j) ? slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] : 0.f;
   const float Dh = c.D[head];
+  float seen = 0.f;
   // a block's operands: one address that all lanes share, and every lane's distances from it
   uint32_t from_tile[TW], from_x[4], from_last[4];
 #pragma unroll
@@ -1113,6 +1120,7 @@ __global__ void __launch_bounds__(256, 2) head_blocks_walk_kernel(HeadScanCall c
       for (int j = 0; j < TW; ++j)
         if (mine(j)) sums[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.c[j][i], S[j][i], sums[j], 0, 0, 0);
     const floatx4 within = __builtin_amdgcn_mfma_f32_16x16x4f32(st.m, own, floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    seen = fmaf(own, 0.f, seen);
 #pragma unroll
     for (int j = 0; j < TW; ++j) S[j] *= st.all;
 #pragma unroll
@@ -1140,6 +1148,35 @@ __global__ void __launch_bounds__(256, 2) head_blocks_walk_kernel(HeadScanCall c
     }
   }
   finish((blocks - 1) & 1);
+  const int found = __builtin_amdgcn_ballot_w64(!(seen == 0.f)) != 0;
+  if (lane == 0) spoiled[wave] = found;
+  __syncthreads();
+  if (__builtin_expect(spoiled[0] | spoiled[1] | spoiled[2] | spoiled[3], 0)) {
+    // sixteen lanes a channel, every sixteenth state element in each of them
+    const int channel = 16 * column + (tid >> 4), part = tid & 15;
+    float* held = c.S + (int64_t)c.slots[seq] * c.state_stride + ((int64_t)head * vtiles + channel / 4) * DIM * 4 + channel % 4;
+    float state[DT];
+#pragma unroll
+    for (int j = 0; j < DT; ++j) state[j] = held[(part + 16 * j) * 4];
+    const float rate = expf(c.A_log[head]);
+#pragma unroll 1
+    for (int t = first; t < first + count; ++t) {
+      const float step = softplus_f(c.dt_raw[(int64_t)t * c.ld_dt + head] + c.dt_bias[head]), decay = expf(-rate * step);
+      const float value = c.x[(int64_t)t * c.ld + head * c.vdim + channel];
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < DT; ++j) {
+        const int64_t at = (int64_t)t * c.ld + group * DIM + part + 16 * j;
+        state[j] = fmaf(decay, state[j], c.B[at] * (step * value));
+        sum = fmaf(state[j], c.C[at], sum);
+      }
+      sum = sum_of_16_lanes(sum);
+      if (part == 0) c.y[(int64_t)t * c.ld_y + head * c.vdim + channel] = fmaf(Dh, value, sum);
+    }
+#pragma unroll
+    for (int j = 0; j < DT; ++j) held[(part + 16 * j) * 4] = state[j];
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < TW; ++j)
     if (mine(j))

@@ -184,6 +184,39 @@ def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
     assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
 
 
+# the same for the scan with one decay a head
+@pytest.mark.parametrize("where,value", [("x", "inf"), ("x", "-inf"), ("x", "nan"), ("B", "inf"), ("B", "nan"), ("C", "inf"), ("dt", "nan"), ("dt", "inf")])
+@pytest.mark.parametrize("token", [0, 21, 31, 38, 39])
+def test_a_token_that_is_not_finite_spoils_no_earlier_one_of_a_head(where, value, token):
+    gen = torch.Generator().manual_seed(8)
+    heads, vdim, state, lengths = 2, 32, 64, [40, 50]
+    inner, total = heads * vdim, sum(lengths)
+    A_log, bias, D = torch.zeros(heads, device=DEV), torch.randn(heads, generator=gen).to(DEV), torch.randn(heads, generator=gen).to(DEV)
+    rows = torch.randn(total, inner + 2 * state + heads, generator=gen)
+    spoiled = rows.clone()
+    spoiled[token, {"x": 3, "B": inner + 3, "C": inner + state + 3, "dt": inner + 2 * state}[where]] = float(value)
+    step = make_step(torch.float32, lengths)
+    results = {}
+    for name, source, blocked in (("clean", rows, True), ("blocks", spoiled, True), ("walk", spoiled, False)):
+        on, held = source.to(DEV), torch.zeros(len(lengths), heads * state * vdim, device=DEV)
+        y = torch.full((total, inner), -7.0, device=DEV)
+        room = K.head_blocks(step, heads, vdim, state, 1) if blocked else None
+        if blocked:
+            room.fill_(float("nan"))
+        K.head_scan(on[:, :inner], on[:, inner:inner + state], on[:, inner + state:inner + 2 * state], on[:, inner + 2 * state:], bias, A_log, D, y, held, step,
+                    heads, vdim, state, 1, blocks=room)
+        assert not blocked or bool(torch.isfinite(room).any())          # (it did go in blocks)
+        results[name] = (y.cpu(), held.cpu())
+    (clean, _), (blocks, ended), (walk, walked) = results["clean"], results["blocks"], results["walk"]
+    # (a block with such a token sums in another order: a few roundings of 32 bits)
+    assert token == 0 or rel_err(blocks[:token], clean[:token].double()) < 2e-6
+    assert torch.equal(blocks[lengths[0]:], clean[lengths[0]:])
+    assert torch.equal(torch.isfinite(blocks), torch.isfinite(walk)) and torch.equal(torch.isfinite(ended), torch.isfinite(walked))
+    assert not bool(torch.isfinite(blocks).all())
+    kept = torch.isfinite(walk)
+    assert rel_err(blocks[kept], walk[kept].double()) < 1e-5
+
+
 # channels that do not fill a wave, all sizes of state that lanes take, steps on both sides of the rule, spans that end
 # within a sequence, a second portion from a state that is not zero; `strong`: steps so long that decays vanish
 @pytest.mark.parametrize("channels,state,lengths,spans,strong", [
