@@ -17,15 +17,17 @@ def rel_err(got, want):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+# tokens on both sides of the rule that chooses the kernel by the heads of all tokens
+@pytest.mark.parametrize("longest", [600, 2300])
 # heads and sizes on both sides of a wave's four heads and 128 channels, one odd size that the general kernel takes
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,rot,norm,neighbours,same", [
     (8, 2, 128, 128, 64, "head", False, False), (6, 3, 64, 32, 64, "whole", False, False), (2, 1, 128, 128, 128, None, False, False),
     (5, 5, 16, 48, 8, "head", True, False), (4, 4, 32, 32, 0, "whole", False, True), (1, 1, 6, 2, 2, "head", True, False),
     (3, 1, 10, 10, 6, "head", False, False)])
-def test_rotation_of_many_tokens(dtype, heads, kv_heads, dim, vdim, rot, norm, neighbours, same):
+def test_rotation_of_many_tokens(dtype, longest, heads, kv_heads, dim, vdim, rot, norm, neighbours, same):
     dt = DTYPES[dtype]
     hd = (max(dim, vdim) + 15) // 16 * 16
-    totals, counts = [600, 70, 131], [600, 66, 103]
+    totals, counts = [longest, 70, 131], [longest, 66, 103]
     case = PagedCase(totals, counts, kv_heads, hd, dt, DEV, seed=1)
     gen = torch.Generator().manual_seed(2)
     n = case.n_tokens
