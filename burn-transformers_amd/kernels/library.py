@@ -1491,6 +1491,26 @@ def groups_experts(tokens, experts, top, ff, shared_ff, width, dtype):
         width % row == 0 and ff % row == 0 and shared_ff % row == 0
 
 
+GROUPED_SAVED = 1.4e9        # operations, at least
+GROUPED_SAVED_A_PLANE = 0.75e9
+
+
+def grouped_experts_pay(tokens, experts, top, ff, shared_ff, width, matrices, dtype):
+    """Whether that is also the cheaper way, for steps of up to ``tokens`` tokens, the most of their class (one launch list serves a
+    class): two products with few tiles, each a chain as long as its K, and a plane for every choice cost more than one
+    product over all experts saves while that has little to do.  So bfloat16 steps of up to 1,024 tokens ask for as many
+    operations less, with ``matrices`` (two, or three with a gate) an expert, as measured (us, every expert on every row / on
+    their rows): 4 experts of 512 x 512, one a token, 130 tokens (0.6 GF at the class's most) 19.9 / 23.0, 260 (1.5) 23.1 / 22.7; 4 of
+    1,024 x 512, two a token, and a shared one, 130 (1.2) 24.4 / 27.3, 400 (2.8) 33.5 / 36.9, 773 (5.2) 42.4 / 39.1; 8 of 256 x 128, two a
+    token, 400 (0.5) 19.7 / 20.0, 1,200 30.3 / 27.3; 16 of 1,024 x 256, four a token, and a shared one 130 (3.6) 31.7 / 33.1, 200 (4.8) 38.4 /
+    33.8; 8 of 1,024 x 512, two a token, 65 (2.4) 26.0 / 25.7.  Where a token uses an eighth of the experts or less it pays from 65
+    tokens on (64 of 256 x 64, four a token, 25.5 / 23.4), as it does everywhere in float32 (8 of 64 x 64, two a token, 65 tokens 65 / 20)."""
+    if dtype != torch.bfloat16 or experts >= 8 * top or tokens > 1024:
+        return True
+    saved = 2.0 * matrices * tokens * width * ff * (experts - top)
+    return saved >= max(GROUPED_SAVED, GROUPED_SAVED_A_PLANE * (top + (1 if shared_ff else 0)))
+
+
 def grouped_experts(h, weights, used, gate, in_weight, down_weight, experts, ff, shared_ff, identity, top, step, out, limit=None, alpha=1.0,
                     unit=None):
     """out [top (+ 1 with ``shared_ff``), rows, width] float32: plane j holds the output of each row's j-th expert (in the order

@@ -32,7 +32,8 @@ that expert (zero where it was not chosen, the sigmoid gate for the shared exper
 with the down matrices laid side by side, which so sums the weighted outputs.  Every expert multiplies every token,
 which costs little while all matrices are read anyway.
 
-Steps of more tokens run every expert on the rows that use it (``kernels.library.grouped_experts``): the rows are
+Steps of more tokens run every expert on the rows that use it where that is the cheaper way (``kernels.library.grouped_experts``,
+``grouped_experts_pay``): the rows are
 listed on the GPU, gathered while they are brought in, and every choice's output lies in a plane of its own that the
 norm behind adds.  Nothing depends on the host knowing the choice either, so a step is a fixed list of kernels both ways.
 
@@ -148,7 +149,9 @@ class RoutedExperts(FeedForward):
             return Delta(partials, None)
         weights = step.buffer("experts.weights", tokens, self.outputs, "float32")
         mix = step.buffer("experts.mix", tokens, 1, "float32") if self.shared_mix is not None else None
-        grouped = K.groups_experts(tokens, self.experts, self.top, self.ff, self.shared_ff, self.width, step.dtype)
+        most = step.token_capacity if tokens == step.n_tokens else tokens
+        grouped = K.groups_experts(tokens, self.experts, self.top, self.ff, self.shared_ff, self.width, step.dtype) and \
+            K.grouped_experts_pay(most, self.experts, self.top, self.ff, self.shared_ff, self.width, 3 if self.gated else 2, step.dtype)
         used = step.buffer("experts.used", tokens, 1, "int64") if grouped else None
         K.route(h, self.router, self.correction, self.top, self.groups, self.keep, weights, self.shared_mix, mix,
                 score=self.score, group_rank=self.group_rank, normalize=self.normalize, bias=self.router_bias, used=used)

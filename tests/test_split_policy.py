@@ -195,3 +195,49 @@ def test_float_products_are_cut_alike_in_all_steps_of_a_class(monkeypatch):
             assert len(found) == 1, (columns, k, most, found)
             asked_exactly += len({float_split_count(rows, columns, k) for rows in range(most - 63, most + 1)}) > 1
     assert asked_exactly > 0                                            # the rule itself turns within classes
+
+
+def test_which_experts_run_on_their_rows():
+    """Few operations less are no reason to; whatever is decided holds for all steps of a class, whose launch list is one."""
+    import torch
+    from types import SimpleNamespace
+    from burn_transformers_amd.engine.step import token_capacity
+    from burn_transformers_amd.kernels import library as K
+    from burn_transformers_amd.parts.experts import RoutedExperts
+
+    def way(tokens, experts, top, ff, shared_ff, width, dtype=torch.bfloat16, unit="gated"):
+        """True: on their rows, by the calls that the part makes."""
+        made = []
+        part = RoutedExperts.__new__(RoutedExperts)
+        part.__dict__.update(rides=False, experts=experts, identity=0, outputs=experts, top=top, ff=ff, shared_ff=shared_ff, width=width, gated=unit == "gated", unit=unit,
+                             shared_mix=None, router=None, correction=None, groups=1, keep=1, score="softmax", group_rank=1, normalize=True, router_bias=None,
+                             in_weight=None, down_weight=None, limit=None, alpha=1.0, in_packed=None, down_packed=None, fused_cols=8, hidden_cols=8)
+        buffer = lambda key, *sizes: torch.empty(1, device="meta")
+        step = SimpleNamespace(n_tokens=tokens, token_capacity=token_capacity(tokens), dtype=dtype, dtype_is_bf16=dtype == torch.bfloat16, buffer=buffer, partial_sums=buffer)
+        taken = {}
+
+        class Chosen(Exception):
+            pass
+
+        def route(*args, used=None, **more):
+            taken["way"] = used is not None
+            raise Chosen
+        held, K.route = K.route, route
+        try:
+            part.forward(torch.empty(tokens, width, dtype=dtype, device="meta"), step, None)
+        except Chosen:
+            pass
+        finally:
+            K.route = held
+        return taken["way"]
+
+    assert not way(64, 8, 2, 1024, 0, 1024) and way(65, 8, 2, 1024, 0, 1024) and way(65, 8, 2, 512, 0, 1024)
+    assert not way(200, 4, 1, 512, 0, 512) and way(300, 4, 1, 512, 0, 512)
+    assert not way(200, 4, 2, 512, 512, 1024) and way(773, 4, 2, 512, 512, 1024)
+    assert not way(400, 8, 2, 128, 0, 256) and way(1100, 8, 2, 128, 0, 256)
+    assert not way(100, 16, 4, 256, 256, 1024) and way(200, 16, 4, 256, 256, 1024)
+    assert way(65, 64, 4, 64, 0, 256) and way(65, 8, 2, 64, 0, 64, torch.float32) and not way(64, 8, 2, 64, 0, 64, torch.float32)
+    for sizes in ((4, 1, 512, 0, 512), (4, 2, 512, 512, 1024), (8, 2, 128, 0, 256), (16, 4, 256, 256, 1024), (8, 2, 512, 0, 1024)):
+        for unit in ("gated", "silu"):
+            for most in range(128, 1217, 64):
+                assert len({way(rows, *sizes, unit=unit) for rows in range(most - 63, most + 1)}) == 1
