@@ -862,7 +862,7 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
   if (dtype == 0) {
     const float *a = (const float*)A, *w = (const float*)W;
     const bool deep_ok = K % (TILE_ROW_BYTES / 4) == 0 && (int64_t)M * lda * 4 < ((int64_t)1 << 32) && (int64_t)N * K * 4 < ((int64_t)1 << 32);
-    if (variant == 2 || variant == 3) BT_REFUSE("gemm_tile: float products have the general form only, not variant %d", variant);
+    if (variant == 2 || variant == 3) BT_REFUSE("gemm_tile: of the variants 1 to 3 float products have the general form only, not variant %d", variant);
     if (variant >= 4 && !deep_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 32 and operands below 4 GiB", K);
     if (variant == 0 && deep_ok) {
       const int64_t small = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits, tall = (int64_t)((M + 127) / 128) * ((N + 63) / 64) * splits;
