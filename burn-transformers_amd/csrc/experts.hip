@@ -505,8 +505,8 @@ BT_EXPORT int bt_gated_experts_call(void* stream, const GatedExpertsCall* c) {
 // of 128; 8 experts of the width, two a token): width 1,024 with gates, 128 tokens 37 / 33 / 42, 512 61 / 40 / 48, 1,024 97 / 58 / 57, 2,048
 // 157 / 91 / 88, 4,096 289 / 154 / 142; width 2,048 without gates and a shared expert, 200 tokens 98 / 51 / 69, 773 250 / 102 / 101, 2,048
 // 378 / 221 / 192.  One work-group to a unit with more stages loses (128 rows in four: 106 us at 2,048 tokens).  Float: width
-// 1,024 with gates, 128 tokens 104 / 92 / 150, 2,048 908 / 310 / 353.  From 65 tokens on the rows win or draw (65 tokens of 1,024
-// without gates: 36.6 / 37.2).  What bounds them is what a compute unit pulls, as in the plain products' deep forms: 0.5 to 0.6 PFLOP/s.
+// 1,024 with gates, 128 tokens 104 / 92 / 150, 2,048 908 / 310 / 353.  65 tokens of 1,024 without gates draw (36.6 / 37.2);
+// where the experts have less to do every expert on every row is the cheaper way, and the caller takes it.  What bounds them is what a compute unit pulls, as in the plain products' deep forms: 0.5 to 0.6 PFLOP/s.
 #define EXPERT_TALL_ROWS 192
 
 struct GroupExpertsCall {

@@ -734,7 +734,7 @@ __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall
       for (int i = 0; i < 4; ++i) slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] = S[j][i];
 }
 
-// Steps whose longest sequence brings at least this many tokens go in blocks.  Below, two launches cost what walking
+// Steps whose longest sequence brings at least this many tokens may go in blocks (blocks_pay).  Below, two launches cost what walking
 // does (us, token by token / in blocks; one decay a head, one a key channel, forget gate): 2 x 32 tokens 16.0 / 17.2,
 // 19.9 / 19.5, 13.8 / 13.0; 16 x 40 tokens 42.8 / 37.0, 56.3 / 39.3, 32.8 / 28.4; 4 x 48 tokens 22.9 / 19.6, 29.2 / 22.1, 20.0 / 15.0.
 #define KB_MIN_TOKENS 40

@@ -941,7 +941,7 @@ static void launch_head_scan_r(hipStream_t stream, const HeadScanCall& c) {
 // results land where the next product reads them.
 #define HB_TOKENS 16
 #define HB_HEADS 8              // heads a work-group of the first kernel prepares
-// Steps whose longest sequence brings at least this many tokens go in blocks.  Measured (us, as whole sequences or spans / in
+// Steps whose longest sequence brings at least this many tokens may go in blocks (blocks_pay).  Measured (us, as whole sequences or spans / in
 // blocks; 32 heads of 64 x 128): 2 x 40 tokens 16.1 / 13.2, 16 x 40 48.7 / 36.1, 2 x 128 39 / 17, 2 x 1,024 225 / 58, 8 x 300 141 / 60.
 // Of the longest, 11 us go to the operands; a block then takes 0.7 us, 0.25 of them on the matrix units: a wave is alone on
 // its SIMD and pays every instruction around them, and the trip through LDS, itself.
