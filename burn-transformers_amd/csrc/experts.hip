@@ -72,7 +72,8 @@ struct RouteEarly {
 // reductions.  `score` holds the logits and afterwards the scores, `choice` afterwards the token's weight of every expert,
 // zero where it was not chosen (both in LDS, written by the lane whose expert it is).  At most `top` experts are chosen whatever
 // the values: a lane remembers which of its experts are taken, no value stands for it (a correction or logit may be infinite).
-__device__ __forceinline__ void route_choice(const RouteCall& c, const RouteEarly& early, float* score, float* choice) {
+// Returns the weight of the lane's first expert.
+__device__ __forceinline__ float route_choice(const RouteCall& c, const RouteEarly& early, float* score, float* choice) {
   const int lane = threadIdx.x & 63;
   if (c.bias)                                       // a lane keeps to its own experts
     for (int e = lane, j = 0; e < c.experts; e += 64, ++j) score[e] += j < 4 ? early.bias[j < 4 ? j : 0] : c.bias[e];
@@ -137,6 +138,22 @@ __device__ __forceinline__ void route_choice(const RouteCall& c, const RouteEarl
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   float sum = 0.f;
+  if (c.experts <= 64) {                           // (an expert a lane: nothing is read again while they are chosen)
+    const float own = lane < c.experts ? score[lane] : 0.f, corrected = lane < c.experts ? choice[lane] : -INFINITY;
+    bool taken = false;
+    for (int k = 0; k < c.top; ++k) {
+      const bool left = corrected > -INFINITY && !taken;
+      float value = left ? corrected : -INFINITY;
+      int index = left ? lane : 0x7fffffff;
+      wave_best(value, index);
+      if (index == 0x7fffffff) break;              // (nothing left above minus infinity, or what is left is not a number)
+      if (lane == index) taken = true;
+      sum += score[index];
+    }
+    const float weight = taken ? own * (c.normalize ? 1.0f / (sum + 1e-20f) : 1.0f) : 0.f;
+    if (lane < c.experts) choice[lane] = weight;
+    return weight;
+  }
   unsigned taken = 0;                              // bit j: the lane's expert lane + 64 j (ROUTE_MAX_EXPERTS: sixteen of them)
   for (int k = 0; k < c.top; ++k) {
     float value = -INFINITY;
@@ -146,12 +163,13 @@ __device__ __forceinline__ void route_choice(const RouteCall& c, const RouteEarl
       if (v > value && !(taken >> j & 1)) { value = v; index = e; }     // (ascending e: the lowest index among equals)
     }
     wave_best(value, index);
-    if (index == 0x7fffffff) break;                // (nothing left above minus infinity, or what is left is not a number)
+    if (index == 0x7fffffff) break;
     if (lane == (index & 63)) taken |= 1u << (index >> 6);
     sum += score[index];
   }
   const float inverse = c.normalize ? 1.0f / (sum + 1e-20f) : 1.0f;
   for (int e = lane, j = 0; e < c.experts; e += 64, ++j) choice[e] = taken >> j & 1 ? score[e] * inverse : 0.f;
+  return choice[lane];
 }
 
 // One work-group of sixteen waves per token.  Logits: a wave takes whole outputs (two at a time, the
@@ -219,11 +237,11 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
   }
   __syncthreads();
   if (wave != 0) return;
-  route_choice(c, early, score, choice);
+  const float first = route_choice(c, early, score, choice);
   // the one store of a lane's experts: the chosen ones' scores over their sum, zero elsewhere
   float* weights = c.weights + (int64_t)t * c.experts;
   for (int e = lane; e < c.experts; e += 64) {
-    const float w = choice[e];
+    const float w = e < 64 ? first : choice[e];
     weights[e] = w;
     if (e < 64 && c.used) {
       const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
@@ -298,20 +316,22 @@ __global__ void __launch_bounds__(64 * ROUTE_ROWS) route_rows_kernel(RouteCall c
   const int t = t0 + wave;
   if (t >= c.tokens) return;
   const float gate_sum = score[wave][c.gate_w ? c.experts : 0];
-  route_choice(c, early, score[wave], choice[wave]);
-  const float w = lane < c.experts ? choice[wave][lane] : 0.f;
+  const float w = route_choice(c, early, score[wave], choice[wave]);    // (zero behind the experts, of which there are at most 64)
   if (lane < c.experts) c.weights[(int64_t)t * c.experts + lane] = w;
   const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
   if (lane == 0 && c.used) c.used[t] = used;
   if (lane == 0 && c.gate_w) c.gate[t] = 1.0f / (1.0f + expf(-gate_sum));
 }
 
+// (Few outputs of wide rows from 1,792 tokens on: 8 of 4,096 float columns 1,536 tokens 13.7 / 16.6, 1,800 16.3 / 16.9; of 4,096 bfloat16 ones 14.8 /
+// 16.5 and 17.9 / 16.9, of 1,024 7.9 / 8.1 and 9.4 / 8.2.)
 #define ROUTE_ROWS_MIN 1536
+#define ROUTE_ROWS_MIN_FEW 1792
 
 template <typename T>
 static bool launch_route_rows(hipStream_t stream, const RouteCall& c) {
   const int outputs = c.experts + (c.gate_w ? 1 : 0), tiles = (outputs + 15) / 16;
-  if (c.tokens < ROUTE_ROWS_MIN || tiles > ROUTE_ROWS_TILES || c.width % 16 != 0 || c.ldh % 4 != 0 || ((uintptr_t)c.h & (4 * sizeof(T) - 1)) ||
+  if (c.tokens < (outputs <= 8 && c.width >= 1024 ? ROUTE_ROWS_MIN_FEW : ROUTE_ROWS_MIN) || tiles > ROUTE_ROWS_TILES || c.width % 16 != 0 || c.ldh % 4 != 0 || ((uintptr_t)c.h & (4 * sizeof(T) - 1)) ||
       (((uintptr_t)c.W | (uintptr_t)c.gate_w) & 15))
     return false;
   dim3 grid((c.tokens + ROUTE_ROWS - 1) / ROUTE_ROWS), block(64 * ROUTE_ROWS);
