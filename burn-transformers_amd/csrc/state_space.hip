@@ -986,12 +986,15 @@ __global__ void __launch_bounds__(256) head_blocks_kernel(HeadScanCall c) {
     decays[h][i] = i < count ? expf(-expf(c.A_log[head]) * step) : 1.f;
   }
   __syncthreads();
-  floatx4 sums = {0.f, 0.f, 0.f, 0.f};
+  // (four sums side by side, added in pairs: one chain of a wave's 32 products rounds a third more than the walk's sums do)
+  floatx4 sums[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sums[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   floatx4* frag = reinterpret_cast<floatx4*>(place + (int64_t)group * 2 * HB_TOKENS * DIM);
   for (int tile = wave; tile < DT; tile += 4) {
     const floatx4 q = *reinterpret_cast<const floatx4*>(&C[n][16 * tile + 4 * g]), k = *reinterpret_cast<const floatx4*>(&B[n][16 * tile + 4 * g]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sums = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], k[i], sums, 0, 0, 0);
+    for (int i = 0; i < 4; ++i) sums[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], k[i], sums[i], 0, 0, 0);
     if (blockIdx.x % sets == 0) {
       floatx4 u;
 #pragma unroll
@@ -1000,12 +1003,11 @@ __global__ void __launch_bounds__(256) head_blocks_kernel(HeadScanCall c) {
       frag[64 * (DT + tile) + lane] = u;
     }
   }
-  parts[wave][lane] = sums;                                              // lane holds G[4 g + i][n]
+  parts[wave][lane] = (sums[0] + sums[1]) + (sums[2] + sums[3]);         // lane holds G[4 g + i][n]
   __syncthreads();
   const int t = tid >> 4, s = tid & 15;
-  float product = 0.f;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) product += reinterpret_cast<const float*>(&parts[w][16 * (t >> 2) + s])[t & 3];
+  auto part_of = [&](int w) { return reinterpret_cast<const float*>(&parts[w][16 * (t >> 2) + s])[t & 3]; };
+  const float product = (part_of(0) + part_of(1)) + (part_of(2) + part_of(3));
   for (int h = 0; h < heads; ++h) {
     float decay = 1.f;                                                   // of the tokens behind s up to t
 #pragma unroll

@@ -184,6 +184,30 @@ def test_heads_in_blocks_of_tokens(heads, groups, vdim, state, lengths, strong):
     assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
 
 
+# read-outs of heads in blocks against 64 bits, in the 2-norm: as exact as token by token (their roundings differ by some hundredths; one
+# chain of 32 products a wave for the blocks' C B^T was a third further off)
+@pytest.mark.parametrize("state", [64, 128])
+@pytest.mark.parametrize("shift", [-2.0, 0.5])
+def test_heads_in_blocks_are_as_exact(state, shift):
+    gen, heads, vdim, total = torch.Generator().manual_seed(11), 8, 64, 500
+    inner = heads * vdim
+    rows = torch.randn(total, inner + 2 * state + heads, generator=gen)
+    A_log, bias, D = torch.log(torch.rand(heads, generator=gen) * 15.0 + 1.0), torch.randn(heads, generator=gen) * 0.5 + shift, torch.ones(heads)
+    r, on, step = rows.double(), rows.to(DEV), make_step(torch.float32, [total])
+    x, B, C = r[:, :inner].view(-1, heads, vdim), r[:, None, inner:inner + state], r[:, None, inner + state:inner + 2 * state]
+    dt = torch.nn.functional.softplus(r[:, inner + 2 * state:] + bias.double(), threshold=50.0)
+    decay = torch.exp(-torch.exp(A_log.double()) * dt)[..., None].expand(-1, heads, state)
+    want, _ = recurrence(torch.zeros(heads, state, vdim, dtype=torch.float64), C.expand(-1, heads, -1), B.expand(-1, heads, -1), dt[..., None] * x, decay, None)
+    want = (want + x).reshape(total, inner)
+    errors = []
+    for room in (K.head_blocks(step, heads, vdim, state, 1), None):
+        y, held = torch.empty(total, inner, device=DEV), torch.zeros(1, heads * state * vdim, device=DEV)
+        K.head_scan(on[:, :inner], on[:, inner:inner + state], on[:, inner + state:inner + 2 * state], on[:, inner + 2 * state:], bias.to(DEV), A_log.to(DEV),
+                    D.to(DEV), y, held, step, heads, vdim, state, 1, blocks=room)
+        errors.append(float((y.double().cpu() - want).norm() / want.norm()))
+    assert errors[0] < 1.15 * errors[1], errors
+
+
 # the same for the scan with one decay a head
 @pytest.mark.parametrize("where,value", [("x", "inf"), ("x", "-inf"), ("x", "nan"), ("B", "inf"), ("B", "nan"), ("C", "inf"), ("dt", "nan"), ("dt", "inf")])
 @pytest.mark.parametrize("token", [0, 21, 31, 38, 39])
