@@ -121,6 +121,10 @@ __global__ void __launch_bounds__(256) causal_conv_kernel(CausalConvCall c) {
 #define CONV_RUN 8
 #define CONV_MIN_TOKENS 384
 #define CONV_MIN_VALUES 350000
+// ... and where several sequences may straddle runs, of which few taps gain less (300 and 100 x 1 tokens: of 1,024 channels 2 taps 5.6 / 6.4, 3 6.1 /
+// 6.8, 4 6.8 / 7.3, of 2,048 2 taps 6.9 / 7.3, 4 9.6 / 8.8; 120 x 5 of 900 2 taps 6.2 / 6.9, 4 8.6 / 8.2).
+#define CONV_MIN_VALUES_MANY 500000
+#define CONV_MIN_VALUES_MANY_FEW_TAPS 1000000
 
 template <typename T, int TAPS>
 __global__ void __launch_bounds__(256) causal_conv_run_kernel(CausalConvCall c) {
@@ -232,8 +236,9 @@ BT_EXPORT int bt_causal_conv_call(void* stream, const CausalConvCall* c) {
       hipLaunchKernelGGL((causal_conv_kernel<bf16_t, true>), grid, block, 0, (hipStream_t)stream, *c);
     return bt_check_launch("causal_conv");
   }
-  const bool run = c->tokens >= CONV_MIN_TOKENS && (int64_t)c->tokens * c->channels >= CONV_MIN_VALUES && (c->cast_dtype == 0 ? launch_conv_run<float>((hipStream_t)stream, *c, cols)
-                                                                      : launch_conv_run<bf16_t>((hipStream_t)stream, *c, cols));
+  const int least = c->n_seqs == 1 ? CONV_MIN_VALUES : c->taps >= 4 ? CONV_MIN_VALUES_MANY : CONV_MIN_VALUES_MANY_FEW_TAPS;
+  const bool run = c->tokens >= CONV_MIN_TOKENS && (int64_t)c->tokens * c->channels >= least &&
+                   (c->cast_dtype == 0 ? launch_conv_run<float>((hipStream_t)stream, *c, cols) : launch_conv_run<bf16_t>((hipStream_t)stream, *c, cols));
   if (run) {
   } else if (c->cast_dtype == 0)
     hipLaunchKernelGGL((causal_conv_kernel<float, false>), grid, block, 0, (hipStream_t)stream, *c);

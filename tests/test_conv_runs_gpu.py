@@ -16,7 +16,8 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("taps", [2, 3, 4, 5])
 @pytest.mark.parametrize("lengths,channels,act,dtype", [([384], 40, "silu", None), ([3, 1, 2, 400, 9, 17], 300, "none", "bfloat16"),
                                                         ([64] * 7, 257, "silu", "float32"), ([390], 900, "silu", None), ([3, 1, 2, 400, 9, 17], 1000, "none", "bfloat16"),
-                                                        ([1] * 20 + [380] + [5] * 9, 900, "silu", "float32")])
+                                                        ([1] * 20 + [380] + [5] * 9, 900, "silu", "float32"),
+                                                        ([3, 1, 2, 400, 9, 17], 2400, "none", "bfloat16"), ([1] * 20 + [380] + [5] * 9, 2300, "silu", "float32")])
 def test_runs_of_tokens(taps, lengths, channels, act, dtype):
     gen = torch.Generator().manual_seed(taps * 100 + channels)
     weight, bias = torch.randn(channels, taps, generator=gen), torch.randn(channels, generator=gen)
