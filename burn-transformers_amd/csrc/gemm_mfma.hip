@@ -1,6 +1,6 @@
 // Matrix products on the MFMA units of gfx950, C[M,N] = A[M,K] . W[N,K]^T with 32-bit
 // accumulation, in bfloat16 and in float (the float instructions multiply and add in full
-// 32-bit: no reduced-precision mode exists in them).  Both operands are K-contiguous, which is
+// 32-bit: no reduced-precision mode exists in them; products made of parts keep all 24 bits of both operands).  Both operands are K-contiguous, which is
 // what an MFMA lane wants: consecutive K values in one 16-byte load.
 //
 //   gemm_tile    128 x 128 x 64 tiles for many rows (prefill).  Four waves, each a quarter of the
@@ -9,7 +9,8 @@
 //                flight during the multiplication, tiles numbered so that each XCD's L2 sees
 //                neighbours.  (The kernel is a template over the tile and the prefetch depth;
 //                larger tiles and deeper prefetch were measured and lost to this one: they
-//                leave room for one work-group per compute unit only.)
+//                leave room for one work-group per compute unit only.)  Float products of many tiles are
+//                made of the products of three bfloat16 parts of each operand (gemm_tile_parts_kernel).
 //   gemm_skinny  up to 64 rows (decode).  The product is bound by streaming W once from HBM:
 //                a work-group owns 16 columns, its eight waves split K, every lane keeps several
 //                16-byte loads of W in flight, v_mfma_f32_16x16x32_bf16 does the arithmetic and
@@ -547,6 +548,208 @@ gemm_tile_deep_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict_
   }
 }
 
+// Float products of many rows on the bfloat16 matrix instructions, sixteen times the rate of the float ones.
+// A float is the sum of three bfloat16 values (8 + 8 + 8 bits: the nearest to it, the upper bits of what that leaves, the
+// rest) and a product of two floats the sum of nine products of such parts, each exact in 32 bits.  The six
+// largest are added up in 32 bits, the smallest first; the three left out are below 2^-24 of the product.  A sum is rounded
+// 6 K / 16 times where the float instructions round it K / 2 times and more: against 64 bits the error is 0.67 of theirs at
+// K = 32, 0.85 at K = 768, 0.88 at K = 3072.
+// A tile goes from memory to registers (two tiles of K = 32 on their way), is cut there into its parts, every value once for
+// the whole work-group, and lies in LDS as three planes of bfloat16 in three stages: the tile that is multiplied, the
+// next one, whose first operands are read behind the multiplications of the second half of this one, and the one being cut.
+// One barrier a tile; eight waves, two to a SIMD, so that one's cutting fills the other's matrix instructions.
+// A value beyond the largest bfloat16, an infinity or a NaN makes parts whose products are not the floats' (infinity times
+// a part that is zero): they all leave a sum that is not finite, and sums that are not finite are made again from the floats.
+// Values below 2^-110 lose bits that fall below the smallest bfloat16, 2^-133.
+// What bounds it: 1.05 us for a tile of 128 x 128 x 32 where the matrix instructions take 0.64; 0.73 without the loads from memory and
+// the cutting, the same with four tiles on their way in place of two: a compute unit's requests (256 lines a tile), not their
+// latency.  Measured (us, float instructions / 128 x 64 / 128 x 128): 400 x 3072 x 768 33 / 23 / 30; 2298 x 768 x 768
+// 35 / 24 / 31; 2298 x 2304 x 768 85 / 68 / 66; 2298 x 3072 x 768 105 / 90 / 71; 2298 x 768 x 3072 in two slices 108 / 84 / 66;
+// 4096 x 1600 x 6400 800 / 653 / 493 (170 TFLOP/s).  Not taken: four waves (every wave's cutting shows: 554 for the last), 64 x 64
+// tiles (19.0 where the float instructions take 18.8: a unit alone waits for its lines either way), matrix instructions
+// and cutting interleaved one by one by hand (the same).
+struct FloatParts {
+  int part[3];
+};
+__device__ __forceinline__ FloatParts float_parts(float x0, float x1) {      // of two floats, a pair to a word
+  typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+  FloatParts p;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const bf16x2 near = {(bf16_t)x0, (bf16_t)x1};
+    const int i0 = __builtin_bit_cast(int, x0), i1 = __builtin_bit_cast(int, x1);
+    p.part[i] = i == 0 ? __builtin_bit_cast(int, near) : (int)__builtin_amdgcn_perm(i1, i0, 0x07060302);
+    x0 -= __builtin_bit_cast(float, i == 0 ? p.part[i] << 16 : i0 & (int)0xffff0000);
+    x1 -= __builtin_bit_cast(float, (i == 0 ? p.part[i] : i1) & (int)0xffff0000);
+  }
+  return p;
+}
+
+template <int BM, int BN, int WM, int WN>
+__global__ void __launch_bounds__(WM * WN * 64)
+gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ W, int M, int N,
+                       int K, Epilogue epi, int tiles_m, int tiles_n, int group_m) {
+  constexpr int ROWS = BM + BN, THREADS = WM * WN * 64;
+  constexpr int PLANE_BYTES = ROWS * 64, STAGE_BYTES = 3 * PLANE_BYTES;       // a row: 32 values of K in bfloat16
+  constexpr int STEP = THREADS / 8, LOADS = ROWS / STEP;                      // eight lanes a row's 128 bytes
+  constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
+  constexpr int SETS = 2;                         // tiles on their way from memory
+  static_assert(ROWS % STEP == 0 && BM % STEP == 0 && TM >= 1 && TN >= 1, "whole loads and whole blocks for every wave");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];         // [3][3 planes][ROWS][64 bytes]
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave % WM, wn = wave / WM;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
+  // (an XCD's run of tiles is a block of group_m by as many columns, about square: it pulls the fewest rows of A and W)
+  const int per_group = group_m * tiles_n, first = tile / per_group * group_m, rest = tile % per_group;
+  const int rows_m = group_m < tiles_m - first ? group_m : tiles_m - first;
+  const int m_base = (first + rest % rows_m) * BM, n_base = rest / rows_m * BN;
+  const int split = blockIdx.z, splits = gridDim.z;
+  const int k_tiles = K / 32;
+  const int kt_begin = (int)((int64_t)k_tiles * split / splits);
+  const int count = (int)((int64_t)k_tiles * (split + 1) / splits) - kt_begin;
+
+  const int row = tid >> 3, quad = tid & 7;
+  unsigned off[LOADS];
+  int put[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    const int stage_row = row + STEP * j;
+    const bool from_w = STEP * j >= BM;
+    int at = from_w ? n_base + stage_row - BM : m_base + stage_row;
+    const int limit = from_w ? N : M;
+    at = at < limit ? at : limit - 1;
+    off[j] = (unsigned)(((int64_t)at * (from_w ? (int64_t)K : lda) + quad * 4) * 4);
+    put[j] = stage_row * 64 + (((quad >> 1) ^ ((stage_row >> 2) & 3)) << 4) + (quad & 1) * 8;
+  }
+  const unsigned char* a_bytes = reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * TILE_ROW_BYTES;
+  const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * TILE_ROW_BYTES;
+  floatx4 held[SETS][LOADS];
+  int fetched = 0;
+  auto fetch = [&](floatx4* set, int j) {
+    set[j] = *reinterpret_cast<const floatx4*>((STEP * j >= BM ? w_bytes : a_bytes) + off[j]);
+  };
+  auto advance = [&] {         // (no branch: behind the last tile comes the last again)
+    const int64_t step = ++fetched < count ? TILE_ROW_BYTES : 0;
+    a_bytes += step;
+    w_bytes += step;
+  };
+  auto cut = [&](const floatx4* set, int j, int stage) {
+    unsigned char* base = lds + stage * STAGE_BYTES + put[j];
+    const FloatParts lo = float_parts(set[j][0], set[j][1]), hi = float_parts(set[j][2], set[j][3]);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<int2*>(base + p * PLANE_BYTES) = make_int2(lo.part[p], hi.part[p]);
+  };
+  int w_rd[2], a_rd[2];        // (blocks of 32 rows lie 2,048 bytes apart, the swizzle repeats every sixteen rows)
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int chunk = ((2 * kk + g) ^ ((l32 >> 2) & 3)) << 4;
+    a_rd[kk] = (wm * (BM / WM) + l32) * 64 + chunk;
+    w_rd[kk] = (BM + wn * (BN / WN) + l32) * 64 + chunk;
+  }
+  int4v op[2][3][TM + TN];     // of a half of a tile (sixteen values of K): the planes of the wave's blocks of A, then of W
+  constexpr int READS = 3 * (TM + TN);
+  auto read = [&](int stage, int kk, int r) {
+    const int p = r / (TM + TN), b = r % (TM + TN);
+    const unsigned char* base = lds + stage * STAGE_BYTES + p * PLANE_BYTES;
+    op[kk][p][b] = *reinterpret_cast<const int4v*>(base + (b < TM ? a_rd[kk] + b * 2048 : w_rd[kk] + (b - TM) * 2048));
+  };
+  floatx16 acc[TN][TM];
+#pragma unroll
+  for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0.f;
+  auto meet = [&] {            // this wave's planes are written; its loads from memory stay on their way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // one tile: twelve products of parts (six to a half), beside each a share of the reads of the half after it, of the
+  // cutting of the tile after the next and of the loads of the one SETS behind that
+  int now = 0, next = 1, free = 2;              // stages
+  auto turn = [&](floatx4* set) {
+    constexpr int OF_W[6] = {0, 2, 1, 0, 1, 0}, OF_A[6] = {2, 0, 1, 1, 0, 0};      // the smallest products first
+#pragma unroll
+    for (int c = 0; c < 12; ++c) {
+      const int kk = c / 6, p = c % 6;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+        for (int bm = 0; bm < TM; ++bm)
+          Mma<bf16_t>::block32(acc[bn][bm], op[kk][OF_W[p]][TM + bn], op[kk][OF_A[p]][bm]);
+#pragma unroll
+      for (int r = 0; r < READS; ++r)
+        if (r * 6 / READS == p) read(kk == 0 ? now : next, kk ^ 1, r);
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j)
+        if (j * 12 / LOADS == c) {
+          cut(set, j, free);
+          fetch(set, j);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    advance();
+    meet();
+    const int was = now;
+    now = next, next = free, free = was;
+  };
+  if (count > 0) {
+#pragma unroll
+    for (int t = 0; t < SETS + 2; ++t) {
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) {
+        if (t >= SETS) cut(held[t - SETS], j, t - SETS);
+        fetch(held[t % SETS], j);
+      }
+      advance();
+    }
+    meet();
+#pragma unroll
+    for (int r = 0; r < READS; ++r) read(0, 0, r);
+    int left = count;
+    for (; left >= SETS; left -= SETS)
+#pragma unroll
+      for (int t = 0; t < SETS; ++t) turn(held[(t + 2) % SETS]);
+#pragma unroll
+    for (int t = 0; t < SETS - 1; ++t)
+      if (t < left) turn(held[(t + 2) % SETS]);
+  }
+
+  const float* a_part = A + (int64_t)kt_begin * 32;
+  const float* w_part = W + (int64_t)kt_begin * 32;
+#pragma unroll
+  for (int bm = 0; bm < TM; ++bm) {
+    const int m = m_base + wm * (BM / WM) + bm * 32 + l32;
+#pragma unroll
+    for (int bn = 0; bn < TN; ++bn) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
+        const int n0 = n_base + wn * (BN / WN) + bn * 32 + q * 8 + g * 4;
+        if (m >= M) continue;
+        bool finite = true;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) finite = finite && fabsf(v[i]) < INFINITY;
+        if (!finite) {
+          for (int i = 0; i < 4; ++i) {
+            const float* a = a_part + (int64_t)m * lda;
+            const float* w = w_part + (int64_t)(n0 + i < N ? n0 + i : N - 1) * K;
+            float sum = 0.f;
+#pragma nounroll
+            for (int k = 0; k < count * 32; ++k) sum = fmaf(a[k], w[k], sum);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = c == i ? sum : v[c];
+          }
+        }
+        epilogue4<float>(epi, N, m, n0, v, split);
+      }
+    }
+  }
+}
+
 // Memory latency on this GPU is about a microsecond and one compute unit alone pulls only a few
 // per cent of the HBM bandwidth, while a decode step is hundreds of short kernels.  So the
 // skinny kernel (a) wants at least as many work-groups as there are compute units, which is
@@ -825,9 +1028,27 @@ static int launch_deep_form(hipStream_t s, const T* a, int64_t lda, const T* w, 
   return bt_check_launch("gemm_tile");
 }
 
-// variants 4 .. 7: the deep forms (64 x 64 with 8 or 4 stages, 128 x 64 with 6 or 3)
-template <typename T>
-static int launch_deep(hipStream_t s, int variant, const T* a, int64_t lda, const T* w, int M, int N, int K,
+template <int BM, int BN, int WM, int WN>
+static int launch_parts_form(hipStream_t s, const float* a, int64_t lda, const float* w, int M, int N, int K,
+                             const Epilogue& epi, int splits) {
+  auto kernel = gemm_tile_parts_kernel<BM, BN, WM, WN>;
+  const size_t lds = (size_t)3 * 3 * (BM + BN) * 64;
+  static bool raised = false;
+  if (!raised) {
+    hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (err != hipSuccess) BT_REFUSE("gemm_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));
+    raised = true;
+  }
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int group_m = (int)(sqrtf((float)tiles_m * tiles_n * splits / 8 * BN / BM) + 0.5f);
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n, 1, splits), dim3(WM * WN * 64), lds, s, a, lda, w, M, N, K, epi, tiles_m,
+                     tiles_n, group_m < 1 ? 1 : group_m);
+  return bt_check_launch("gemm_tile");
+}
+
+// variants 4 .. 7: the deep forms (64 x 64 with 8 or 4 stages, 128 x 64 with 6 or 3); for float products the last two are
+// the forms on parts (128 x 64, 128 x 128)
+static int launch_deep(hipStream_t s, int variant, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K,
                        const Epilogue& epi, int splits) {
   switch (variant) {
     case 4: return launch_deep_form<64, 64, 8>(s, a, lda, w, M, N, K, epi, splits);
@@ -837,19 +1058,28 @@ static int launch_deep(hipStream_t s, int variant, const T* a, int64_t lda, cons
   }
   BT_REFUSE("gemm_tile: unknown form %d", variant);
 }
+static int launch_deep(hipStream_t s, int variant, const float* a, int64_t lda, const float* w, int M, int N, int K,
+                       const Epilogue& epi, int splits) {
+  switch (variant) {
+    case 4: return launch_deep_form<64, 64, 8>(s, a, lda, w, M, N, K, epi, splits);
+    case 5: return launch_deep_form<64, 64, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 6: return launch_parts_form<128, 64, 4, 2>(s, a, lda, w, M, N, K, epi, splits);
+    case 7: return launch_parts_form<128, 128, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
+  }
+  BT_REFUSE("gemm_tile: unknown form %d", variant);
+}
 
 // dtype: 0 float, 1 bfloat16 (the codes of every entry point that takes both).
 // variant: 0 = the fastest form the operands allow; 1 = template, 2 = lean, 3 = direct to LDS,
 // 4 .. 7 = direct to LDS with smaller tiles and more stages (asked for by tests, by measurements
 // and, for steps of some tens to some hundreds of rows, by the caller; a form that cannot take
 // the operands is refused; float has the template and the forms 4 .. 7).
-// Float products take the deep forms wherever K is a multiple of 32: the template's tile of 128 x 128 takes a compute unit
-// 2.4 us for 32 values of K (0.44 GFLOP/us of the 0.61 its matrix units have) and leaves most units idle where there
-// are few tiles; 64 x 64 in four stages takes 0.65, 128 x 64 in three 1.2 (1.85 times as long for twice the work), two
-// work-groups to a unit.  A unit's share comes in whole tiles, so the busiest unit decides: 64 x 64 unless 1.85 times the
-// rounds of the taller tiles are fewer.  Measured (us, template / 64 x 64 / 128 x 64): 65 x 768 x 3072 230 / 63 / 114;
-// 400 x 3072 x 768 63 / 33 / 34; 800 x 4096 x 1024 88 / 81 / 75; 2298 x 768 x 3072 226 / 115 / 117; 2298 x 2304 x 768 113 / 92 / 86;
-// 2298 x 1600 x 6400 468 / 460 / 427; 4096 x 3072 x 768 170 / 178 / 170; 4096 x 1600 x 6400 876 / 793 / 847.
+// Float products take the tiles of 64 x 64 or the forms on parts wherever K is a multiple of 32 (the template's tile of 128 x 128
+// takes a compute unit 2.4 us for 32 values of K and leaves most units idle where there are few tiles).  While the tiles of
+// 64 x 64 have a unit each, they win: 0.65 us for 32 values of K where a tile of 128 x 64 on parts takes 0.73 (65 x 768 x 3072 62
+// against 72; 1000 x 768 x 768 18.8 against 21.9).  Beyond, a unit's share comes in whole tiles of the forms on parts, one to a unit
+// at a time, and the busiest unit decides: 128 x 128 takes 1.27 to 1.58 times as long as 128 x 64 for twice the work (figures
+// with the kernel).
 BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, const void* W, int M, int N, int K,
                            const Epilogue* epi, int splits, int variant) {
   if (M <= 0) return BT_OK;
@@ -865,8 +1095,9 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
     if (variant == 2 || variant == 3) BT_REFUSE("gemm_tile: of the variants 1 to 3 float products have the general form only, not variant %d", variant);
     if (variant >= 4 && !deep_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 32 and operands below 4 GiB", K);
     if (variant == 0 && deep_ok) {
-      const int64_t small = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits, tall = (int64_t)((M + 127) / 128) * ((N + 63) / 64) * splits;
-      variant = 20 * ((small + 255) / 256) <= 37 * ((tall + 255) / 256) ? 5 : 7;
+      const int64_t rows = (M + 127) / 128 * (int64_t)splits;
+      const int64_t rounds = (rows * ((N + 63) / 64) + 255) / 256, wide_rounds = (rows * ((N + 127) / 128) + 255) / 256;
+      variant = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits <= 256 ? 5 : 2 * rounds <= 3 * wide_rounds ? 6 : 7;
     }
     if (variant >= 4) return launch_deep(s, variant, a, lda, w, M, N, K, *epi, splits);
     launch_tile<float, 128, 128, 2, 2, 1>(s, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits);

@@ -965,18 +965,22 @@ def deep_split_count(rows, columns, k, units=256):
 
 
 def float_split_count(rows, columns, k, units=256):
-    """The same for float32 products of more than 64 rows, whose tiles of 64 x 64 (1) or 128 x 64 (1.85) take a
-    compute unit 0.65 us for 32 values of K: as many slices, at most four, each at least four tiles of K long, as leave the
-    busiest unit the least to do, the slices the norm reads in addition counted at 4.5 TB/s; none for a gain below a
-    tenth.  Measured (us, slices 1 / 2 / 4): 65 x 768 x 3072 63 / 34 / 19; 400 x 768 x 3072 64 / 35 / 34; 800 x 768 x 3072 63 /
-    60 / 48; 1200 x 768 x 3072 65 / 62 / 62; 65 x 768 x 768 18.9 / 11.5 / 7.8."""
+    """The same for float32 products of more than 64 rows: as many slices, at most four, each at least four tiles of K
+    long, as leave the busiest unit the least to do, the slices the norm reads in addition counted at 4.5 TB/s; none for a
+    gain below a tenth, and none where the tiles of 64 x 64 have most units busy already.  For 32 values of K a tile of 64 x 64
+    takes a unit 0.65 us while there is at most one to a unit; beyond that tiles of 128 x 64 take 0.8 us and of 128 x 128 1.22
+    (``bt_gemm_tile`` chooses).  Measured (us, slices 1 / 2 / 4): 65 x 768 x 3072 62 / 34 / 19; 400 x 768 x 3072 64 / 35 / 34;
+    2298 x 768 x 3072 79 / 66 / -; 65 x 768 x 768 18.9 / 11.5 / 7.8."""
     if rows <= 64 or k % 32:
+        return 1
+    tiles = lambda m, n: (rows + m - 1) // m * ((columns + n - 1) // n)
+    if 3 * units < 4 * tiles(64, 64) <= 4 * units:
         return 1
 
     def cost(splits):
-        tiles = lambda m: (rows + m - 1) // m * ((columns + 63) // 64) * splits
-        rounds = min((tiles(64) + units - 1) // units, 1.85 * ((tiles(128) + units - 1) // units))
-        return rounds / splits * (k // 32) * 0.65 + (splits - 1) * rows * columns * 8 / 4.5e6
+        rounds = lambda m, n: (tiles(m, n) * splits + units - 1) // units
+        step = 0.65 if rounds(64, 64) == 1 else min(0.8 * rounds(128, 64), 1.22 * rounds(128, 128))
+        return (k // 32) / splits * step + (splits - 1) * rows * columns * 8 / 4.5e6
     best = min((s for s in range(1, 5) if s == 1 or (k // 32) // s >= 4), key=cost)
     return best if cost(best) < 0.9 * cost(1) else 1
 
