@@ -19,6 +19,7 @@ typedef __bf16 bf16_t;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
 void bt_set_error(const char* fmt, ...);

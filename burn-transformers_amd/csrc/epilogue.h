@@ -306,3 +306,145 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int N, int m, int n
     }
   }
 }
+
+// The epilogue of a whole wave's TM x TN blocks of 32 x 32 (lane holds D[i][j]: i = 8 (r / 4) + 4 g + r % 4 the column, j = lane
+// % 32 the row): through LDS, so that memory sees whole rows' 16-byte pieces instead of 32 rows' 8 bytes with every
+// instruction, and with all that a step needs from memory asked for together.  One call of epilogue4 after the other took 5 us
+// (stored rows) to 12 us (the residual stream, whose old values every call waited for) of a product of 128 x 128 tiles.
+// `scratch`: TILE_SCRATCH bytes of this wave's own; every wave has passed a barrier behind its last read of it.
+template <int TM, int TN>
+constexpr int tile_scratch_bytes() { return TM * 32 * (TN * 32 * 4 + 16); }
+
+template <typename T, int TM, int TN>
+__device__ __forceinline__ void epilogue_tile(const Epilogue& e, int M, int N, int m0, int n0, floatx16 (&acc)[TN][TM], int split,
+                                              unsigned char* scratch) {
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+  constexpr int COLUMNS = TN * 32, ROWS = TM * 32;
+  const bool f32 = sizeof(T) == 4 || e.mode == EPI_F32 || e.mode == EPI_RESIDUAL;
+  const int piece = f32 ? 4 : 8;                       // values in 16 bytes
+  // key/value columns: the wave's columns are all queries, or all keys or all values of one head
+  const int kv_column = n0 - e.n_q, kv_last = kv_column + COLUMNS - 1;
+  const bool scatter = e.mode == EPI_QKV && kv_column >= 0 && kv_last < 2 * e.n_kv && kv_column / e.kv.head_dim == kv_last / e.kv.head_dim &&
+                       kv_column / e.n_kv == kv_last / e.n_kv && (e.kv.head_dim & 7) == 0 && (((uintptr_t)e.kv.keys | (uintptr_t)e.kv.values) & 15) == 0;
+  const bool values = scatter && kv_column >= e.n_kv, keys = scatter && !values;
+  const bool whole = (e.mode != EPI_QKV || n0 + COLUMNS <= e.n_q || scatter) && e.out_rows == 0 && N % piece == 0 && e.ldo % piece == 0 &&
+                     e.split_stride % piece == 0 && (((uintptr_t)e.out | (uintptr_t)e.bias) & 15) == 0;
+  auto spread = [&](auto element) {                    // the wave's rows into LDS
+    typedef decltype(element) E;
+    constexpr int PITCH = COLUMNS * (int)sizeof(E) + 16;
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm)
+#pragma unroll
+      for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
+          store4<E>(reinterpret_cast<E*>(scratch + (bm * 32 + l32) * PITCH) + bn * 32 + q * 8 + g * 4, v, 4, true);
+        }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (a wave's accesses of LDS are served in order)
+  };
+  if (!whole) {                                        // (the same for the whole wave)
+    spread(0.f);
+#pragma nounroll
+    for (int i = lane; i < ROWS * COLUMNS / 4; i += 64) {
+      const int r = i / (COLUMNS / 4), c = i % (COLUMNS / 4) * 4;
+      const floatx4 row = *reinterpret_cast<const floatx4*>(scratch + r * (COLUMNS * 4 + 16) + c * 4);
+      const float v[4] = {row[0], row[1], row[2], row[3]};
+      if (m0 + r < M) epilogue4<T>(e, N, m0 + r, n0 + c, v, split);
+    }
+    return;
+  }
+  if (e.bias != nullptr && split == 0) {
+    floatx4 b[TN][4];
+#pragma unroll
+    for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + bn * 32 + q * 8 + g * 4;
+        b[bn][q] = *reinterpret_cast<const floatx4*>(e.bias + (n < N ? n : 0));
+      }
+#pragma unroll
+    for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+      for (int bm = 0; bm < TM; ++bm)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[bn][bm][r] += b[bn][r >> 2][r & 3];
+  }
+  if (e.mode == EPI_ACT) {
+#pragma unroll
+    for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+      for (int bm = 0; bm < TM; ++bm)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[bn][bm][r] = activate<T>(acc[bn][bm][r], e.act);
+  }
+  if (values) {          // four positions lie interleaved: every lane stores its own row's channels, 8 bytes of a line for four rows
+    const int c = kv_column - e.n_kv, head = c / e.kv.head_dim;
+    int seq[TM], pos[TM];
+    T* plane[TM];
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm) {
+      const int m = m0 + bm * 32 + l32 < M ? m0 + bm * 32 + l32 : M - 1;
+      seq[bm] = e.tok_seq[m];
+      pos[bm] = e.tok_pos[m];
+    }
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm)
+      plane[bm] = static_cast<T*>(e.kv.values) + kv_block_base(e.kv, seq[bm], pos[bm], head) + value_offset(e.kv.head_dim, pos[bm], c % e.kv.head_dim + 4 * g);
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm) {
+      if (m0 + bm * 32 + l32 >= M) continue;
+#pragma unroll
+      for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) plane[bm][4 * (bn * 32 + 8 * (r >> 2) + (r & 3))] = from_float<T>(acc[bn][bm][r]);
+    }
+    return;
+  }
+  auto exchange = [&](auto element) {
+    typedef decltype(element) E;
+    constexpr int PIECE = 16 / (int)sizeof(E), LANES = COLUMNS / PIECE, TURNS = ROWS * LANES / 64;   // lanes a row, pieces a lane
+    constexpr int PITCH = COLUMNS * (int)sizeof(E) + 16;
+    const int n = n0 + lane % LANES * PIECE;
+    E* row[TURNS];
+    floatx4 old[TURNS];
+    int seq[TURNS], pos[TURNS];
+    if (keys) {
+#pragma unroll
+      for (int t = 0; t < TURNS; ++t) {
+        int m = m0 + (64 / LANES) * t + lane / LANES;
+        m = m < M ? m : M - 1;
+        seq[t] = e.tok_seq[m];
+        pos[t] = e.tok_pos[m];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TURNS; ++t) {
+      int m = m0 + (64 / LANES) * t + lane / LANES;
+      m = m < M ? m : M - 1;
+      if (keys) {
+        const int c = n - e.n_q;
+        row[t] = static_cast<E*>(e.kv.keys) + kv_block_base(e.kv, seq[t], pos[t], c / e.kv.head_dim) + key_offset(e.kv.head_dim, pos[t], c % e.kv.head_dim);
+      } else {
+        row[t] = static_cast<E*>(e.out) + (e.mode == EPI_F32 ? (int64_t)split * e.split_stride : 0) + (int64_t)m * e.ldo + (n < N ? n : 0);
+      }
+      if constexpr (sizeof(E) == 4)
+        if (e.mode == EPI_RESIDUAL) old[t] = *reinterpret_cast<const floatx4*>(row[t]);
+    }
+    spread(element);
+#pragma unroll
+    for (int t = 0; t < TURNS; ++t) {
+      const int r = (64 / LANES) * t + lane / LANES;
+      int4v v = *reinterpret_cast<const int4v*>(scratch + r * PITCH + lane % LANES * 16);
+      if constexpr (sizeof(E) == 4)
+        if (e.mode == EPI_RESIDUAL) v = __builtin_bit_cast(int4v, __builtin_bit_cast(floatx4, v) + old[t]);
+      if (m0 + r < M && n < N) *reinterpret_cast<int4v*>(row[t]) = v;
+    }
+  };
+  if constexpr (sizeof(T) == 4) {
+    exchange(0.f);
+  } else {
+    if (f32) exchange(0.f);
+    else exchange((bf16_t)0.f);
+  }
+}

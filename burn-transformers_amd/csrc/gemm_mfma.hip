@@ -3,14 +3,11 @@
 // 32-bit: no reduced-precision mode exists in them; products made of parts keep all 24 bits of both operands).  Both operands are K-contiguous, which is
 // what an MFMA lane wants: consecutive K values in one 16-byte load.
 //
-//   gemm_tile    128 x 128 x 64 tiles for many rows (prefill).  Four waves, each a quarter of the
-//                tile as 2 x 2 blocks of v_mfma_f32_32x32x16_bf16; operands staged through LDS
-//                with an XOR swizzle of the 16-byte chunks, the next tile's global loads in
-//                flight during the multiplication, tiles numbered so that each XCD's L2 sees
-//                neighbours.  (The kernel is a template over the tile and the prefetch depth;
-//                larger tiles and deeper prefetch were measured and lost to this one: they
-//                leave room for one work-group per compute unit only.)  Float products of many tiles are
-//                made of the products of three bfloat16 parts of each operand (gemm_tile_parts_kernel).
+//   gemm_tile    tiles of 64 x 64 to 128 x 256 for many rows (prefill): gemm_tile_pipe_kernel, whose
+//                operands go straight into LDS and whose loop is tile.h's; gemm_tile_kernel for any K
+//                and operands of 4 GiB and more, through registers.  Tiles are numbered so that each XCD's L2
+//                sees neighbours.  Float products of many tiles are made of the products of three
+//                bfloat16 parts of each operand (gemm_tile_parts_kernel).
 //   gemm_skinny  up to 64 rows (decode).  The product is bound by streaming W once from HBM:
 //                a work-group owns 16 columns, its eight waves split K, every lane keeps several
 //                16-byte loads of W in flight, v_mfma_f32_16x16x32_bf16 does the arithmetic and
@@ -20,8 +17,7 @@
 // The weights are the MFMA "A" operand (rows = output columns n), the activations the "B"
 // operand (columns = rows m), so a lane ends up with four consecutive n of one m.
 //
-// The tile kernel's general form and the skinny kernel are templates over the element type; the
-// two leaner forms of the tile kernel are bfloat16 only.
+// All are templates over the element type but the one on parts.
 
 #include "host.h"
 #include "tile.h"
@@ -174,378 +170,49 @@ gemm_tile_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, 
   }
 }
 
-// The same 128 x 128 x 64 tiling for K a multiple of 64 and operands below 4 GiB, written so that
-// the loop over K holds almost nothing but loads, LDS traffic and MFMAs.  Counters
-// (SQ_INSTS_VALU against SQ_INSTS_VALU_MFMA_MOPS) showed five ordinary vector instructions per
-// MFMA in the template above, nearly all of them address arithmetic.  Here every address is a
-// uniform base that a scalar add advances, plus a per-lane offset computed once: global loads
-// take a 32-bit lane offset, LDS accesses one lane offset plus an immediate (rows 32 apart share
-// their swizzle and lie 4096 bytes apart; the two stages are 32 KiB apart).
-#define FAST_STAGE_BYTES (256 * TILE_ROW_BYTES)
-#define FAST_W_BYTES (128 * TILE_ROW_BYTES)
-
-__global__ void __launch_bounds__(256)
-gemm_tile_fast_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int N,
-                      int K, Epilogue epi, int tiles_m, int tiles_n) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * FAST_STAGE_BYTES];
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int l32 = lane & 31, g = lane >> 5;
+// Tiles of BM x BN on TilePipe (tile.h).  K a multiple of 64 (float: 32), operands below 4 GiB.
+// What bounds it is LDS: a tile of 128 x 128 x 64 moves 32 KiB into it and 64 (four waves) or 96 KiB (eight) out of it, at 128
+// bytes a cycle 750 or 1,000 cycles beside 512 of the matrix instructions; a tile of 128 x 256 1,400 beside 1,024.  Behind that 4.5
+// to 5 us whatever K is: launch, first loads, last stores.  Measured (us; in brackets the forms this one replaced, whose loop copied
+// its accumulators and whose epilogue waited for memory sixteen times, and the vendor's library; bias included): 300 x 3072 x 1024
+// 7.1 (10.4, 9.4); 566 x 1024 x 1024 into the residual stream 7.8 (11.8, 9.4); 566 x 4096 x 1024 12.8 (17.6, 13.7); 566 x
+// 1024 x 4096 16.8 (29.6, 18.1); 1295 x 1024 x 1024 10.4 (23.6, 11.2); 1295 x 4096 x 1024 20.1 (25.9, 21.1); 2048 x 1600 x 1600 20.5
+// (32.4, 22.0); 2048 x 1600 x 6400 59 (75, 60); 2048 x 4800 x 1600 45.6 (59, 38); 4096 x 4096 x 4096 138 (179, 93).
+template <typename T, int BM, int BN, int WM, int WN, int STAGES>
+__global__ void __launch_bounds__(WM * WN * 64, 2)
+gemm_tile_pipe_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
+                      int K, Epilogue epi, int tiles_m, int tiles_n, int group_m) {
+  typedef TilePipe<T, BM, BN, WM, WN, STAGES> Pipe;
+  constexpr int ROW_K = 8 * Mma<T>::ELEMS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // [STAGES][BM + BN][128 bytes]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
-  const int m_base = (tile % tiles_m) * 128, n_base = (tile / tiles_m) * 128;
-  const int split = blockIdx.z, splits = gridDim.z;
-  const int k_tiles = K / TILE_K;
-  const int kt_begin = (int)((int64_t)k_tiles * split / splits);
-  const int count = (int)((int64_t)k_tiles * (split + 1) / splits) - kt_begin;
-
-  const int c = tid & 7, r0 = tid >> 3;
-  unsigned a_off[4], w_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int m = m_base + r0 + 32 * i, n = n_base + r0 + 32 * i;
-    m = m < M ? m : M - 1;
-    n = n < N ? n : N - 1;
-    a_off[i] = (unsigned)(((int64_t)m * lda + c * 8) * 2);
-    w_off[i] = (unsigned)(((int64_t)n * K + c * 8) * 2);
-  }
-  const unsigned char* a_k = reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * (TILE_K * 2);
-  const unsigned char* w_k = reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * (TILE_K * 2);
-  const int st_off = swizzled(r0, c);
-  int w_rd[4], a_rd[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    w_rd[kk] = FAST_W_BYTES + swizzled(wn * 64 + l32, 2 * kk + g);
-    a_rd[kk] = swizzled(wm * 64 + l32, 2 * kk + g);
-  }
-
-  int4v ra[4], rw[4];
-  auto load_tile = [&]() {     // the tile a_k, w_k point at; then advance them
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ra[i] = *reinterpret_cast<const int4v*>(a_k + a_off[i]);
-      rw[i] = *reinterpret_cast<const int4v*>(w_k + w_off[i]);
-    }
-    a_k += TILE_K * 2;
-    w_k += TILE_K * 2;
-  };
-  auto store_tile = [&](int stage_bytes) {
-    unsigned char* base = lds + stage_bytes + st_off;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<int4v*>(base + i * 4096) = ra[i];
-      *reinterpret_cast<int4v*>(base + FAST_W_BYTES + i * 4096) = rw[i];
-    }
-  };
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-    for (int bm = 0; bm < 2; ++bm)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0.f;
-
-  if (count > 0) {
-    load_tile();
-    store_tile(0);
-  }
-  __syncthreads();
-  // one loop body, no exit in its middle: the accumulators then stay where the MFMAs want them
-  // (with the loop unrolled by two and left from its middle, the compiler copied all of them
-  // between register files in every iteration)
-  int stage_bytes = 0;
-  for (int i = 0; i < count; ++i) {
-    const bool more = i + 1 < count;
-    if (more) load_tile();
-    const unsigned char* base = lds + stage_bytes;
-    bf16x8 wop[4][2], aop[4][2];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        wop[kk][b] = *reinterpret_cast<const bf16x8*>(base + w_rd[kk] + b * 4096);
-        aop[kk][b] = *reinterpret_cast<const bf16x8*>(base + a_rd[kk] + b * 4096);
-      }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-        for (int bm = 0; bm < 2; ++bm)
-          acc[bn][bm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wop[kk][bn], aop[kk][bm], acc[bn][bm], 0, 0, 0);
-    stage_bytes ^= FAST_STAGE_BYTES;
-    if (more) store_tile(stage_bytes);
-    __syncthreads();
-  }
-
-  // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m)
-#pragma unroll
-  for (int bm = 0; bm < 2; ++bm) {
-    const int m = m_base + wm * 64 + bm * 32 + l32;
-#pragma unroll
-    for (int bn = 0; bn < 2; ++bn) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
-        int n0 = n_base + wn * 64 + bn * 32 + q * 8 + g * 4;
-        if (m < M) epilogue4<bf16_t>(epi, N, m, n0, v, split);
-      }
-    }
-  }
-}
-
-// The third form of the same tiling moves the operands from memory straight into LDS
-// (global_load_lds_dwordx4: every lane names 16 bytes in memory, the wave's 64 pieces land in one
-// contiguous KiB of LDS), which frees the staging registers and, more to the point, lets
-// DMA_STAGES - 1 tiles be in flight while one is multiplied: the products above are bound by
-// memory latency (one tile in flight per work-group, two work-groups per compute unit), not by
-// MFMA or LDS throughput.  The compiler's own bookkeeping would wait for ALL such loads before any
-// LDS read, so the waits are written by hand (s_waitcnt vmcnt(n) with n = loads of the tiles that
-// may still be in flight) and the work-group meets at a bare s_barrier:
-//     wait for my loads of tile i | barrier | start the loads of tile i + STAGES - 1 into the
-//     stage tile i - 1 was read from | read tile i from LDS | multiply
-// The swizzle is applied on the memory side: lane l of the load that fills rows 8 s .. 8 s + 7
-// writes physical chunk l % 8 of row 8 s + l / 8, so it fetches the logical chunk that belongs
-// there.  K must be a multiple of 64, operands below 4 GiB.
-#define DMA_STAGES 4
-#define DMA_LOADS 8   // global_load_lds instructions per wave and tile
-
-__global__ void __launch_bounds__(256)
-gemm_tile_dma_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int N,
-                     int K, Epilogue epi, int tiles_m, int tiles_n) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // [DMA_STAGES][256 rows][128 bytes]
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int l32 = lane & 31, g = lane >> 5;
-  const int tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
-  const int m_base = (tile % tiles_m) * 128, n_base = (tile / tiles_m) * 128;
-  const int split = blockIdx.z, splits = gridDim.z;
-  const int k_tiles = K / TILE_K;
-  const int kt_begin = (int)((int64_t)k_tiles * split / splits);
-  const int count = (int)((int64_t)k_tiles * (split + 1) / splits) - kt_begin;
-
-  // waves 0 and 1 fetch A's 128 rows, waves 2 and 3 W's: load j of a wave fills stage rows
-  // 64 * wave + 8 j .. + 7 (rows 128 .. 255 of a stage are W's)
-  const bool fetch_w = wave >= 2;
-  const unsigned char* src = reinterpret_cast<const unsigned char*>(fetch_w ? W : A) +
-                             (int64_t)kt_begin * (TILE_K * 2);
-  unsigned off[DMA_LOADS];
-#pragma unroll
-  for (int j = 0; j < DMA_LOADS; ++j) {
-    int stage_row = 64 * wave + 8 * j + (lane >> 3);
-    int chunk = (lane & 7) ^ ((stage_row >> 1) & 7);
-    int row = (stage_row & 127) + (fetch_w ? n_base : m_base);
-    int limit = fetch_w ? N : M;
-    row = row < limit ? row : limit - 1;
-    off[j] = (unsigned)(((int64_t)row * (fetch_w ? (int64_t)K : lda) + chunk * 8) * 2);
-  }
-  auto issue = [&](int stage) {   // the tile `src` points at, into `stage`; then advance
-#pragma unroll
-    for (int j = 0; j < DMA_LOADS; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(src + off[j]),
-          (__attribute__((address_space(3))) void*)(lds + stage * FAST_STAGE_BYTES + (64 * wave + 8 * j) * TILE_ROW_BYTES),
-          16, 0, 0);
-    src += TILE_K * 2;
-  };
-  int w_rd[4], a_rd[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    w_rd[kk] = FAST_W_BYTES + swizzled(wn * 64 + l32, 2 * kk + g);
-    a_rd[kk] = swizzled(wm * 64 + l32, 2 * kk + g);
-  }
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-    for (int bm = 0; bm < 2; ++bm)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0.f;
-
-#pragma unroll
-  for (int t = 0; t < DMA_STAGES - 1; ++t)
-    if (t < count) issue(t);
-  int stage = 0, next_stage = DMA_STAGES - 1;
-  for (int i = 0; i < count; ++i) {
-    // tiles i + 1 .. i + STAGES - 2 (those that exist) may still be in flight
-    int newer = count - 1 - i;
-    if (newer >= DMA_STAGES - 2) wait_vmcnt<DMA_LOADS * (DMA_STAGES - 2)>();
-    else if (newer == 1) wait_vmcnt<DMA_LOADS>();
-    else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (i + DMA_STAGES - 1 < count) issue(next_stage);
-    const unsigned char* base = lds + stage * FAST_STAGE_BYTES;
-    bf16x8 wop[4][2], aop[4][2];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        wop[kk][b] = *reinterpret_cast<const bf16x8*>(base + w_rd[kk] + b * 4096);
-        aop[kk][b] = *reinterpret_cast<const bf16x8*>(base + a_rd[kk] + b * 4096);
-      }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-        for (int bm = 0; bm < 2; ++bm)
-          acc[bn][bm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wop[kk][bn], aop[kk][bm], acc[bn][bm], 0, 0, 0);
-    stage = stage + 1 == DMA_STAGES ? 0 : stage + 1;
-    next_stage = next_stage + 1 == DMA_STAGES ? 0 : next_stage + 1;
-  }
-
-  // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m)
-#pragma unroll
-  for (int bm = 0; bm < 2; ++bm) {
-    const int m = m_base + wm * 64 + bm * 32 + l32;
-#pragma unroll
-    for (int bn = 0; bn < 2; ++bn) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
-        int n0 = n_base + wn * 64 + bn * 32 + q * 8 + g * 4;
-        if (m < M) epilogue4<bf16_t>(epi, N, m, n0, v, split);
-      }
-    }
-  }
-}
-
-// The direct-to-LDS form again, for products of some tens to some hundreds of rows (short prompts,
-// chunks of prompts): a template over the tile (BM x BN, 64 or 128 each, four waves as 2 x 2) and
-// the number of stages.  Such a product has too few tiles of 128 x 128 to fill the chip, and with
-// smaller tiles a work-group has less arithmetic per byte it pulls, so that its time is the 25 (or
-// 100) trips to memory of its loop over K unless several of them are in flight at once.  Same layout
-// of a stage as above (A's rows, then W's, 128 bytes each, the swizzle applied on the memory side),
-// same waits written by hand.  K a multiple of 64, operands below 4 GiB.
-// Measured at 128 rows (us; the vendor's library beside it): tiles of 64 x 64 in four stages 4800 x
-// 1600 12.0 (17.3), 6400 x 1600 13.6 (18.2), and with K cut into four slices of pending partial sums
-// 1600 x 1600 5.9 (11.2), 1600 x 6400 12.1 (18.4); at 256 rows tiles of 128 x 64 take 17.4 (20.0) and
-// 20.0 (21.4), two slices of 64 x 64 7.4 (11.7) and 19.2 (23.9); sliced products win up to 512 rows
-// (9.5 and 30.7 against 12.1 and 32.4), the others lose to the library from 512 rows on.  Four stages
-// (64 KiB, two work-groups to a compute unit) do as well as eight or better.
-// What bounds these forms is what the compute units pull, not what they multiply: a work-group
-// gets a tile of 64 x 64 (16 KiB) about every 0.4 us, one of 128 x 64 every 0.6 us and one of 128 x
-// 128 every 0.85 us, whatever the number of stages; with the matrix instructions and the LDS reads
-// taken out the times stay.  Measured and not taken, all at 128 rows and within 10 % of the above:
-// a ring of register sets in place of the direct loads (slower), waves that do nothing but issue the
-// loads (2, 4 or 8 loads a wave and tile: the same times), all rows of the step against 32 columns
-// with the weights in a ring of their own, 8 or 16 tiles deep, filled by a wave of its own (the
-// same), each work-group starting its walk over K at another tile (the same).  All work-groups
-// together pull at 6 to 12 TB/s through the L2s, more the more of them share a compute unit; a
-// kernel that only reads as much without a loop does 27 TB/s from the L2 and 6.6 from memory.
-// For prompts of thousands of rows a tile of 256 x 256 on eight waves (twice the multiplications
-// per byte pulled) was measured too, in two forms.  With K in steps of 64 its two stages of 64 KiB
-// are all that the LDS holds, so one tile is in flight at a time and its latency is not hidden:
-// 2048 x 4800 x 1600 took 86 us where the lean form takes 70 and the vendor's library 39.  With K in
-// steps of 32 and four stages of 32 KiB (rows two to a 128-byte line, swizzled free of bank
-// conflicts) three tiles are in flight, but a wave's load then asks for sixteen half cache lines
-// where it asked for eight whole ones, and a compute unit pulls half the bytes: 88 us.  What a
-// compute unit pulls is a number of cache lines a microsecond (about 300), not of bytes.
-template <typename T, int BM, int BN, int STAGES>
-__global__ void __launch_bounds__(256)
-gemm_tile_deep_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
-                      int K, Epilogue epi, int tiles_m, int tiles_n) {
-  constexpr int ELEMS = Mma<T>::ELEMS, ROW_K = 8 * ELEMS;       // K values in 16 bytes and in a stage's row
-  constexpr int ROWS = BM + BN;                   // rows of a stage
-  constexpr int STAGE_BYTES = ROWS * TILE_ROW_BYTES;
-  constexpr int LOADS = ROWS / 32;                // global_load_lds instructions per wave and tile (8 rows each)
-  constexpr int TM = BM / 64, TN = BN / 64;       // 32-wide MFMA blocks of a wave's (BM / 2) x (BN / 2)
-  static_assert((BM == 64 || BM == 128) && (BN == 64 || BN == 128) && STAGES >= 3 && LOADS * (STAGES - 2) < 64,
-                "tiles of 64 or 128, and no more loads in flight than the wave's counter holds");
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // [STAGES][ROWS][128 bytes]
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int l32 = lane & 31, g = lane >> 5;
-  const int tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
-  const int m_base = (tile % tiles_m) * BM, n_base = (tile / tiles_m) * BN;
+  // (an XCD's run of tiles is a block of group_m by as many columns, about square: it pulls the fewest rows of A and W)
+  const int per_group = group_m * tiles_n, first = tile / per_group * group_m, rest = tile % per_group;
+  const int rows_m = group_m < tiles_m - first ? group_m : tiles_m - first;
+  const int m_base = (first + rest % rows_m) * BM, n_base = rest / rows_m * BN;
   const int split = blockIdx.z, splits = gridDim.z;
   const int k_tiles = K / ROW_K;
   const int kt_begin = (int)((int64_t)k_tiles * split / splits);
   const int count = (int)((int64_t)k_tiles * (split + 1) / splits) - kt_begin;
-
-  // load j of wave w fills stage rows 8 (LOADS w + j) .. + 7: A's rows below BM, W's from there on
-  const unsigned char* a_bytes = reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * TILE_ROW_BYTES;
-  const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * TILE_ROW_BYTES;
-  unsigned off[LOADS];
-  bool from_w[LOADS];
+  floatx16 acc[Pipe::TN][Pipe::TM];
 #pragma unroll
-  for (int j = 0; j < LOADS; ++j) {
-    int first_row = __builtin_amdgcn_readfirstlane(8 * (LOADS * wave + j));
-    from_w[j] = first_row >= BM;                  // (the same for the whole wave: eight rows never straddle BM)
-    int stage_row = first_row + (lane >> 3);
-    int chunk = (lane & 7) ^ ((stage_row >> 1) & 7);
-    int row = from_w[j] ? n_base + stage_row - BM : m_base + stage_row;
-    int limit = from_w[j] ? N : M;
-    row = row < limit ? row : limit - 1;
-    off[j] = (unsigned)(((int64_t)row * (from_w[j] ? (int64_t)K : lda) + chunk * ELEMS) * sizeof(T));
-  }
-  auto issue = [&](int stage) {   // the tile a_bytes / w_bytes point at, into `stage`; then advance
+  for (int bn = 0; bn < Pipe::TN; ++bn)
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)((from_w[j] ? w_bytes : a_bytes) + off[j]),
-          (__attribute__((address_space(3))) void*)(lds + stage * STAGE_BYTES + 8 * (LOADS * wave + j) * TILE_ROW_BYTES),
-          16, 0, 0);
-    a_bytes += TILE_ROW_BYTES;
-    w_bytes += TILE_ROW_BYTES;
-  };
-  int w_rd[4], a_rd[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    w_rd[kk] = BM * TILE_ROW_BYTES + swizzled(wn * (BN / 2) + l32, 2 * kk + g);
-    a_rd[kk] = swizzled(wm * (BM / 2) + l32, 2 * kk + g);
-  }
-  floatx16 acc[TN][TM];
-#pragma unroll
-  for (int bn = 0; bn < TN; ++bn)
-#pragma unroll
-    for (int bm = 0; bm < TM; ++bm)
+    for (int bm = 0; bm < Pipe::TM; ++bm)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0.f;
-
-#pragma unroll
-  for (int t = 0; t < STAGES - 1; ++t)
-    if (t < count) issue(t);
-  int stage = 0, next_stage = STAGES - 1;
-  for (int i = 0; i < count; ++i) {
-    // tiles i + 1 .. i + STAGES - 2 (those that exist) may still be in flight
-    wait_for_all_but<STAGES - 2, LOADS>(count - 1 - i);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (i + STAGES - 1 < count) issue(next_stage);
-    const unsigned char* base = lds + stage * STAGE_BYTES;
-    int4v wop[4][TN], aop[4][TM];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-#pragma unroll
-      for (int b = 0; b < TN; ++b) wop[kk][b] = *reinterpret_cast<const int4v*>(base + w_rd[kk] + b * 4096);
-#pragma unroll
-      for (int b = 0; b < TM; ++b) aop[kk][b] = *reinterpret_cast<const int4v*>(base + a_rd[kk] + b * 4096);
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int bn = 0; bn < TN; ++bn)
-#pragma unroll
-        for (int bm = 0; bm < TM; ++bm) Mma<T>::block32(acc[bn][bm], wop[kk][bn], aop[kk][bm]);
-    stage = stage + 1 == STAGES ? 0 : stage + 1;
-    next_stage = next_stage + 1 == STAGES ? 0 : next_stage + 1;
-  }
-
-  // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m)
-#pragma unroll
-  for (int bm = 0; bm < TM; ++bm) {
-    const int m = m_base + wm * (BM / 2) + bm * 32 + l32;
-#pragma unroll
-    for (int bn = 0; bn < TN; ++bn) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
-        int n0 = n_base + wn * (BN / 2) + bn * 32 + q * 8 + g * 4;
-        if (m < M) epilogue4<T>(epi, N, m, n0, v, split);
-      }
-    }
-  }
+  Pipe::template multiply<unsigned>(
+      lds, reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * TILE_ROW_BYTES,
+      reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * TILE_ROW_BYTES, count,
+      [&](int stage_row, bool from_w) {
+        const int row = from_w ? n_base + stage_row - BM : m_base + stage_row, limit = from_w ? N : M;
+        return (int64_t)(row < limit ? row : limit - 1) * (from_w ? (int64_t)K : lda) * (int64_t)sizeof(T);
+      },
+      acc);
+  __syncthreads();
+  epilogue_tile<T, Pipe::TM, Pipe::TN>(epi, M, N, m_base + wave % WM * (BM / WM), n_base + wave / WM * (BN / WN), acc, split,
+                                       lds + wave * tile_scratch_bytes<Pipe::TM, Pipe::TN>());
 }
 
 // Float products of many rows on the bfloat16 matrix instructions, sixteen times the rate of the float ones.
@@ -721,33 +388,29 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
   const float* a_part = A + (int64_t)kt_begin * 32;
   const float* w_part = W + (int64_t)kt_begin * 32;
 #pragma unroll
-  for (int bm = 0; bm < TM; ++bm) {
-    const int m = m_base + wm * (BM / WM) + bm * 32 + l32;
+  for (int bn = 0; bn < TN; ++bn)
 #pragma unroll
-    for (int bn = 0; bn < TN; ++bn) {
+    for (int bm = 0; bm < TM; ++bm) {
+      bool finite = true;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float v[4] = {acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
-        const int n0 = n_base + wn * (BN / WN) + bn * 32 + q * 8 + g * 4;
-        if (m >= M) continue;
-        bool finite = true;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) finite = finite && fabsf(v[i]) < INFINITY;
-        if (!finite) {
-          for (int i = 0; i < 4; ++i) {
-            const float* a = a_part + (int64_t)m * lda;
-            const float* w = w_part + (int64_t)(n0 + i < N ? n0 + i : N - 1) * K;
-            float sum = 0.f;
+      for (int r = 0; r < 16; ++r) finite = finite && fabsf(acc[bn][bm][r]) < INFINITY;
+      if (finite) continue;
+      const int m = m_base + wm * (BM / WM) + bm * 32 + l32;
+      const float* a = a_part + (int64_t)(m < M ? m : M - 1) * lda;
 #pragma nounroll
-            for (int k = 0; k < count * 32; ++k) sum = fmaf(a[k], w[k], sum);
+      for (int i = 0; i < 16; ++i) {
+        const int n = n_base + wn * (BN / WN) + bn * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
+        const float* w = w_part + (int64_t)(n < N ? n : N - 1) * K;
+        float sum = 0.f;
+#pragma nounroll
+        for (int k = 0; k < count * 32; ++k) sum = fmaf(a[k], w[k], sum);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = c == i ? sum : v[c];
-          }
-        }
-        epilogue4<float>(epi, N, m, n0, v, split);
+        for (int r = 0; r < 16; ++r) acc[bn][bm][r] = r == i ? sum : acc[bn][bm][r];
       }
     }
-  }
+  __syncthreads();
+  epilogue_tile<float, TM, TN>(epi, M, N, m_base + wm * (BM / WM), n_base + wn * (BN / WN), acc, split,
+                               lds + wave * tile_scratch_bytes<TM, TN>());
 }
 
 // Memory latency on this GPU is about a microsecond and one compute unit alone pulls only a few
@@ -1012,19 +675,27 @@ static void launch_tile(hipStream_t stream, const T* A, int64_t lda, const T* W,
                      K, epi, tiles_m, tiles_n);
 }
 
-template <int BM, int BN, int STAGES, typename T>
-static int launch_deep_form(hipStream_t s, const T* a, int64_t lda, const T* w, int M, int N, int K,
-                            const Epilogue& epi, int splits) {
-  auto kernel = gemm_tile_deep_kernel<T, BM, BN, STAGES>;
-  const size_t lds = (size_t)STAGES * (BM + BN) * TILE_ROW_BYTES;
+// Rows of tiles that make a run of tiles of one XCD about square.
+static int tile_group(int tiles_m, int tiles_n, int splits, int bm, int bn) {
+  const int rows = (int)(sqrtf((float)tiles_m * tiles_n * splits / 8 * bn / bm) + 0.5f);
+  return rows < 1 ? 1 : rows;
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES, typename T>
+static int launch_pipe(hipStream_t s, const T* a, int64_t lda, const T* w, int M, int N, int K, const Epilogue& epi, int splits) {
+  typedef TilePipe<T, BM, BN, WM, WN, STAGES> Pipe;
+  auto kernel = gemm_tile_pipe_kernel<T, BM, BN, WM, WN, STAGES>;
+  const size_t stages = (size_t)STAGES * Pipe::STAGE_BYTES, scratch = (size_t)WM * WN * tile_scratch_bytes<Pipe::TM, Pipe::TN>();
+  const size_t lds = stages > scratch ? stages : scratch;
   static bool raised = false;
   if (!raised) {
     hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (err != hipSuccess) BT_REFUSE("gemm_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));
     raised = true;
   }
-  int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n, 1, splits), dim3(256), lds, s, a, lda, w, M, N, K, epi, tiles_m, tiles_n);
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n, 1, splits), dim3(WM * WN * 64), lds, s, a, lda, w, M, N, K, epi, tiles_m,
+                     tiles_n, tile_group(tiles_m, tiles_n, splits, BM, BN));
   return bt_check_launch("gemm_tile");
 }
 
@@ -1040,40 +711,57 @@ static int launch_parts_form(hipStream_t s, const float* a, int64_t lda, const f
     raised = true;
   }
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int group_m = (int)(sqrtf((float)tiles_m * tiles_n * splits / 8 * BN / BM) + 0.5f);
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n, 1, splits), dim3(WM * WN * 64), lds, s, a, lda, w, M, N, K, epi, tiles_m,
-                     tiles_n, group_m < 1 ? 1 : group_m);
+                     tiles_n, tile_group(tiles_m, tiles_n, splits, BM, BN));
   return bt_check_launch("gemm_tile");
 }
 
-// variants 4 .. 7: the deep forms (64 x 64 with 8 or 4 stages, 128 x 64 with 6 or 3); for float products the last two are
-// the forms on parts (128 x 64, 128 x 128)
-static int launch_deep(hipStream_t s, int variant, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K,
+// The forms of the tile kernel for whole tiles of K.
+static int launch_form(hipStream_t s, int variant, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K,
                        const Epilogue& epi, int splits) {
   switch (variant) {
-    case 4: return launch_deep_form<64, 64, 8>(s, a, lda, w, M, N, K, epi, splits);
-    case 5: return launch_deep_form<64, 64, 4>(s, a, lda, w, M, N, K, epi, splits);
-    case 6: return launch_deep_form<128, 64, 6>(s, a, lda, w, M, N, K, epi, splits);
-    case 7: return launch_deep_form<128, 64, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 2: return launch_pipe<128, 128, 2, 2, 2>(s, a, lda, w, M, N, K, epi, splits);
+    case 3: return launch_pipe<128, 128, 2, 4, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 4: return launch_pipe<64, 64, 2, 2, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 5: return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 6: return launch_pipe<64, 128, 1, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 7: return launch_pipe<128, 256, 2, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
   }
   BT_REFUSE("gemm_tile: unknown form %d", variant);
 }
-static int launch_deep(hipStream_t s, int variant, const float* a, int64_t lda, const float* w, int M, int N, int K,
+static int launch_form(hipStream_t s, int variant, const float* a, int64_t lda, const float* w, int M, int N, int K,
                        const Epilogue& epi, int splits) {
   switch (variant) {
-    case 4: return launch_deep_form<64, 64, 8>(s, a, lda, w, M, N, K, epi, splits);
-    case 5: return launch_deep_form<64, 64, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 4: return launch_pipe<64, 64, 2, 2, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 5: return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
     case 6: return launch_parts_form<128, 64, 4, 2>(s, a, lda, w, M, N, K, epi, splits);
     case 7: return launch_parts_form<128, 128, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
   }
   BT_REFUSE("gemm_tile: unknown form %d", variant);
 }
 
+// Which form a bfloat16 product takes: the one whose busiest compute unit is done first.  A unit with n tiles needs, for every 64
+// values of K, 0.17 us a tile of 64 x 64 (0.2 from three on, when three work-groups of three stages share its LDS: up to two have four
+// stages), 0.28 / 0.62 / 0.33 n for one / two / more tiles of 64 x 128, 0.5 for 128 x 128 on eight waves (one work-group a unit),
+// 0.8 / 0.52 n for one / more on four waves (two work-groups), 0.9 for 128 x 256 (one); around that the fixed times below.  Within 15 % of what
+// 300 to 4,096 rows, 1,024 to 6,400 columns and K of 1,024 to 6,400 measured (figures with the kernel).
+static int tile_form(int M, int N, int K, int splits) {
+  const float turns = (float)(K / TILE_K) / splits;
+  auto share = [&](int bm, int bn) { return (float)(((int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * splits + 255) / 256); };
+  const float small = share(64, 64), tall = share(64, 128), square = share(128, 128), wide = share(128, 256);
+  const float cost[5] = {4.6f + turns * (small <= 2 ? 0.17f : 0.2f) * small, 5.f + turns * (tall <= 1 ? 0.28f : tall <= 2 ? 0.62f : 0.33f * tall),
+                         2.5f + square * (2.8f + 0.5f * turns), 5.5f + turns * (square <= 1 ? 0.8f : 0.52f * square),
+                         3.f + wide * (3.5f + 0.9f * turns)};
+  const int form[5] = {small <= 2 ? 5 : 4, 6, 3, 2, 7};
+  int best = 0;
+  for (int i = 1; i < 5; ++i)
+    if (cost[i] < cost[best]) best = i;
+  return form[best];
+}
+
 // dtype: 0 float, 1 bfloat16 (the codes of every entry point that takes both).
-// variant: 0 = the fastest form the operands allow; 1 = template, 2 = lean, 3 = direct to LDS,
-// 4 .. 7 = direct to LDS with smaller tiles and more stages (asked for by tests, by measurements
-// and, for steps of some tens to some hundreds of rows, by the caller; a form that cannot take
-// the operands is refused; float has the template and the forms 4 .. 7).
+// variant: 0 = the fastest form the operands allow; 1 = the general form; 2 .. 7 = launch_form's (asked for by tests and
+// measurements; a form that cannot take the operands is refused; float has the general form and 4 .. 7).
 // Float products take the tiles of 64 x 64 or the forms on parts wherever K is a multiple of 32 (the template's tile of 128 x 128
 // takes a compute unit 2.4 us for 32 values of K and leaves most units idle where there are few tiles).  While the tiles of
 // 64 x 64 have a unit each, they win: 0.65 us for 32 values of K where a tile of 128 x 64 on parts takes 0.73 (65 x 768 x 3072 62
@@ -1091,46 +779,28 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
   hipStream_t s = (hipStream_t)stream;
   if (dtype == 0) {
     const float *a = (const float*)A, *w = (const float*)W;
-    const bool deep_ok = K % (TILE_ROW_BYTES / 4) == 0 && (int64_t)M * lda * 4 < ((int64_t)1 << 32) && (int64_t)N * K * 4 < ((int64_t)1 << 32);
+    const bool whole_ok = K % (TILE_ROW_BYTES / 4) == 0 && (int64_t)M * lda * 4 < ((int64_t)1 << 32) && (int64_t)N * K * 4 < ((int64_t)1 << 32);
     if (variant == 2 || variant == 3) BT_REFUSE("gemm_tile: of the variants 1 to 3 float products have the general form only, not variant %d", variant);
-    if (variant >= 4 && !deep_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 32 and operands below 4 GiB", K);
-    if (variant == 0 && deep_ok) {
+    if (variant >= 4 && !whole_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 32 and operands below 4 GiB", K);
+    if (variant == 0 && whole_ok) {
       const int64_t rows = (M + 127) / 128 * (int64_t)splits;
       const int64_t rounds = (rows * ((N + 63) / 64) + 255) / 256, wide_rounds = (rows * ((N + 127) / 128) + 255) / 256;
       variant = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits <= 256 ? 5 : 2 * rounds <= 3 * wide_rounds ? 6 : 7;
     }
-    if (variant >= 4) return launch_deep(s, variant, a, lda, w, M, N, K, *epi, splits);
+    if (variant >= 4) return launch_form(s, variant, a, lda, w, M, N, K, *epi, splits);
     launch_tile<float, 128, 128, 2, 2, 1>(s, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits);
     return bt_check_launch("gemm_tile");
   }
   const bf16_t* a = (const bf16_t*)A;
   const bf16_t* w = (const bf16_t*)W;
   const int64_t four_gib = (int64_t)1 << 32;
-  const bool lean_ok = K % TILE_K == 0 && (int64_t)M * lda * 2 < four_gib && (int64_t)N * K * 2 < four_gib;
-  // Direct to LDS keeps three tiles in flight but leaves room for one work-group per compute
-  // unit; it wins when there is at most one tile per compute unit anyway, the lean form (two
-  // work-groups per unit) when there are more.
-  if (variant == 0) variant = !lean_ok ? 1 : ((int64_t)((M + 127) / 128) * ((N + 127) / 128) * splits <= 256 ? 3 : 2);
-  if (variant != 1 && !lean_ok)
-    BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 64 and operands below 4 GiB", K);
-  if (variant >= 4) return launch_deep(s, variant, a, lda, w, M, N, K, *epi, splits);
-  int tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
-  dim3 grid(tiles_m * tiles_n, 1, splits);
-  if (variant == 3) {
-    size_t lds = (size_t)DMA_STAGES * FAST_STAGE_BYTES;
-    static bool raised = false;
-    if (!raised) {
-      hipError_t err = hipFuncSetAttribute((const void*)gemm_tile_dma_kernel,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (err != hipSuccess) BT_REFUSE("gemm_tile: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));
-      raised = true;
-    }
-    hipLaunchKernelGGL(gemm_tile_dma_kernel, grid, dim3(256), lds, s, a, lda, w, M, N, K, *epi, tiles_m, tiles_n);
-  } else if (variant == 2) {
-    hipLaunchKernelGGL(gemm_tile_fast_kernel, grid, dim3(256), 0, s, a, lda, w, M, N, K, *epi, tiles_m, tiles_n);
-  } else {
-    launch_tile<bf16_t, 128, 128, 2, 2, 1>(s, a, lda, w, M, N, K, *epi, splits);
+  const bool whole_ok = K % TILE_K == 0 && (int64_t)M * lda * 2 < four_gib && (int64_t)N * K * 2 < four_gib;
+  if (variant == 0) variant = whole_ok ? tile_form(M, N, K, splits) : 1;
+  if (variant != 1) {
+    if (!whole_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 64 and operands below 4 GiB", K);
+    return launch_form(s, variant, a, lda, w, M, N, K, *epi, splits);
   }
+  launch_tile<bf16_t, 128, 128, 2, 2, 1>(s, a, lda, w, M, N, K, *epi, splits);
   return bt_check_launch("gemm_tile");
 }
 

@@ -6,8 +6,6 @@
 
 #define TILE_ROW_BYTES 128
 
-typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
-
 // What a lane's 16-byte operand read is to the matrix cores.  bfloat16: eight K values, one
 // instruction of depth 32 (16-wide blocks; the lane's K group is lane / 16) or 16 (32-wide
 // blocks; lane / 32).  float: four K values, taken by four instructions of depth 4 (or 2), the
@@ -75,3 +73,101 @@ __device__ __forceinline__ void wait_for_all_but(int newer) {
     else wait_for_all_but<NEWER - 1, LOADS>(newer);
   }
 }
+
+// A tile's product over K: operands go from memory straight into LDS (128-byte rows, BM of A, then BN of W, swizzled on the
+// memory side) and from there into the matrix units, on WM x WN waves, each with TM x TN blocks of 32 x 32.
+//   stages   STAGES tiles of 128 bytes of K lie in LDS or are on their way; one barrier a tile
+//   operands a quarter's are read while the quarter two before it is multiplied; those of the next tile's first half behind
+//            the barrier, beside the second half of this one, so that the barrier and the reads' latency show nowhere
+//   the loop is one straight line: behind the last tile the last one is asked for again, so that the waits are constants.  (A
+//            test inside made the compiler copy all accumulators once or twice a tile, 64 to 128 moves beside 16 matrix
+//            instructions, and the time of a tile was taken for what a compute unit can pull; a unit pulls 150 GB/s.)
+template <typename T, int BM, int BN, int WM, int WN, int STAGES>
+struct TilePipe {
+  static constexpr int WAVES = WM * WN, ROWS = BM + BN, STAGE_BYTES = ROWS * TILE_ROW_BYTES;
+  static constexpr int STEP = 8 * WAVES, LOADS = ROWS / STEP;      // a wave's load instruction: eight rows
+  static constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
+  static_assert(BM % STEP == 0 && BN % STEP == 0 && TM >= 1 && TN >= 1 && STAGES >= 2 && (STAGES - 1) * LOADS < 64,
+                "whole loads, whole blocks, and no more loads in flight than the wave's counter holds");
+
+  // acc += the product of `count` tiles; row_bytes(stage_row, from_w): what that row's first byte lies behind `a` or `w`.
+  // On return every wave's loads have landed and nobody reads the stages any more once all have passed the next barrier.
+  template <typename Offset, typename RowBytes>
+  static __device__ __forceinline__ void multiply(unsigned char* lds, const unsigned char* a, const unsigned char* w, int count,
+                                                  RowBytes row_bytes, floatx16 (&acc)[TN][TM]) {
+    if (count <= 0) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave % WM, wn = wave / WM, l32 = lane & 31, g = lane >> 5;
+    Offset off[LOADS];
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const int stage_row = STEP * j + 8 * wave + (lane >> 3);
+      off[j] = (Offset)(row_bytes(stage_row, STEP * j >= BM) + (((lane & 7) ^ ((stage_row >> 1) & 7)) << 4));
+    }
+    int issued = 0;
+    auto issue = [&](int stage) {
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((STEP * j >= BM ? w : a) + off[j]),
+                                         (__attribute__((address_space(3))) void*)(lds + stage * STAGE_BYTES + (STEP * j + 8 * wave) * TILE_ROW_BYTES),
+                                         16, 0, 0);
+      const int step = ++issued < count ? TILE_ROW_BYTES : 0;
+      a += step;
+      w += step;
+    };
+    int w_rd[4], a_rd[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      w_rd[kk] = BM * TILE_ROW_BYTES + swizzled(wn * (BN / WN) + l32, 2 * kk + g);
+      a_rd[kk] = swizzled(wm * (BM / WM) + l32, 2 * kk + g);
+    }
+    int4v op[4][TM + TN];
+    auto read = [&](int stage, int kk) {
+      const unsigned char* base = lds + stage * STAGE_BYTES;
+#pragma unroll
+      for (int b = 0; b < TM; ++b) op[kk][b] = *reinterpret_cast<const int4v*>(base + a_rd[kk] + b * 4096);
+#pragma unroll
+      for (int b = 0; b < TN; ++b) op[kk][TM + b] = *reinterpret_cast<const int4v*>(base + w_rd[kk] + b * 4096);
+    };
+    auto quarter = [&](int kk) {
+#pragma unroll
+      for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+        for (int bm = 0; bm < TM; ++bm) Mma<T>::block32(acc[bn][bm], op[kk][TM + bn], op[kk][bm]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto turn = [&](int stage, int next, bool more) {
+      read(stage, 2);
+      quarter(0);
+      read(stage, 3);
+      quarter(1);
+      if (more) {       // this wave's loads of the next tile have landed and its reads of this one are done: so have everyone's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue(stage);
+        __builtin_amdgcn_sched_barrier(0);
+        read(next, 0);
+      }
+      quarter(2);
+      if (more) read(next, 1);
+      quarter(3);
+    };
+#pragma unroll
+    for (int t = 0; t < STAGES; ++t) issue(t);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    read(0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    int stage = 0, next = 1;
+    for (int i = 1; i < count; ++i) {
+      turn(stage, next, true);
+      stage = next;
+      next = next + 1 == STAGES ? 0 : next + 1;
+    }
+    turn(stage, next, false);
+    wait_vmcnt<0>();
+  }
+};

@@ -625,9 +625,8 @@ def library_products():
     """The module that runs prompt-sized bfloat16 products through hipBLASLt, or None.
 
     The reference leaves its matrix products to its backend's library (src/attention.rs:481-513
-    and the feed-forward call ``linear``); here the vendor's library takes the products of steps
-    with more than 256 rows (512 for those that add to the residual stream: ``deep_form_rows``),
-    where it is about 1.6 times as fast as the tile kernel of this package at GPT-2 XL sizes, and
+    and the feed-forward call ``linear``); here the vendor's library takes the large products (``own_tiles`` says which;
+    1.2 to 1.5 times as fast as the tile kernel of this package at 2,048 rows of GPT-2 XL's wide matrices), and
     the hand-written kernels keep everything else.  The library is
     opened from the copy that came with torch's HIP runtime and checked once against the tile
     kernel; if it cannot be opened, or disagrees, the tile kernel does those products too, and
@@ -848,7 +847,7 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
     library where it is usable and has the epilogue; float32 operands that are not multiples of
     four wide go to the plain kernel), or one of "plain", "tile", "skinny", "library" to force one.
     variant picks one of the tile kernel's forms (0: the fastest the operands allow, 1: any K,
-    2: lean, 3: direct to LDS) or, for the skinny kernel, the output columns a work-group owns
+    2 to 7: others, see ``bt_gemm_tile``) or, for the skinny kernel, the output columns a work-group owns
     (8, 12, ... 32; 0: chosen for balance).  ``a`` may be a :class:`Normalized`.
     packed: a :class:`PackedWeight` of ``w`` (or directly (``pack_columns(w, columns)``, columns)), read in
     place of ``w`` where the skinny kernel runs and the copy fits the step.
@@ -883,16 +882,8 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
             impl = "skinny"
         elif dtype == FLOAT32:
             impl = "tile"
-        elif deep_form_rows(m, k, a.stride(0), n, sliced=splits > 1, scatters=epilogue.mode == EPI_QKV):
-            # short prompts and chunks: the tile kernel's deep forms (see ``deep_form_rows``)
+        elif own_tiles(m, n, k, a.stride(0), sliced=splits > 1, scatters=epilogue.mode == EPI_QKV):
             impl = "tile"
-            if variant == 0:
-                # tiles of 64 x 64 in four stages, two work-groups to a compute unit.  (Tiles of 128 x
-                # 64 in three stages beyond 128 rows were the choice once: alone they measure the same
-                # at 256 rows, 19.9 against 19.5 us for 4800 x 1600, and lose at 129 to 192 rows, where
-                # the small tiles still have a compute unit each, 18.9 against 12.9 us; a prompt of 160
-                # tokens through 12 layers 1.08 -> 0.97 ms, of 256 tokens 1.20 -> 1.17 ms.)
-                variant = 5
         else:
             impl = "library" if splits == 1 and _library_takes(epilogue) and library_products() \
                 and _library_has_algorithm(a.stride(0), m, n, k, epilogue) else "tile"
@@ -920,25 +911,40 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
         _launch(_module("gemm_mfma"), "bt_gemm_skinny_call", call)
 
 
-DEEP_FORM_ROWS = 256          # most rows of a bfloat16 product that the tile kernel's deep forms take ...
+DEEP_FORM_ROWS = 256          # most rows of a bfloat16 product that the tile kernel takes whatever its other sizes ...
 DEEP_FORM_SLICED_ROWS = 512   # ... and of one that leaves partial sums of slices of K pending ...
 DEEP_FORM_SCATTER_ROWS = 384  # ... and of one that scatters keys and values into the cache
+OWN_TILES = 256               # beyond: most tiles of 128 x 128 of a product that the tile kernel takes ...
+OWN_SCATTER_TILES = 288       # ... and of one that scatters keys and values; its fewest tiles of 64 x 64 ...
+OWN_LEAST_TILES = 128
+OWN_SHORT_K = 512             # ... and its shortest K
+OWN_LONG_K, OWN_LONG_ROWS = 2048, 768     # from this K on: up to so many rows
 
 
 def deep_form_rows(m, k, lda, n, sliced=False, scatters=False):
-    """Whether a bfloat16 product of ``m`` rows is one for the tile kernel's deep forms (tiles of
-    64 x 64 or 128 x 64 brought straight into LDS, several of them on their way at once): 65 to
-    256 rows, where it has too few tiles of 128 x 128 to fill the chip and the vendor's library
-    takes 16 to 24 us whatever the shape (measured at widths 1,600 and 6,400: these forms take a
-    quarter to a third less); where the product may leave slices of K pending (``sliced``: the two
-    products that add to the residual stream) up to 512 rows, and up to 45 % less.  Beyond, the
-    library wins.  The fused projection of a mixer (``scatters``) stays up to 384 rows: the
-    library's product cannot scatter keys and values into the cache, and the copy behind it costs
-    5 us (4800 x 1600 at 320 and 384 rows: 19.5 and 19.7 us here, 18.7 and 18.9 + 5.1 there; at 512
-    rows 28.4 against 20.8 + 5.0).  The forms read K in tiles of 64 and address their operands with
-    32 bits."""
+    """Whether a bfloat16 product of ``m`` rows is the tile kernel's by its rows alone: up to 256, up to 512 where the product
+    may leave slices of K pending (``sliced``: the two products that add to the residual stream), up to 384 for the fused
+    projection of a mixer (``scatters``).  The kernel reads K in tiles of 64 and addresses its operands with 32 bits."""
     limit = DEEP_FORM_SLICED_ROWS if sliced else DEEP_FORM_SCATTER_ROWS if scatters else DEEP_FORM_ROWS
     return 64 < m <= limit and k % 64 == 0 and m * lda * 2 < (1 << 32) and n * k * 2 < (1 << 32)
+
+
+def own_tiles(m, n, k, lda, sliced=False, scatters=False):
+    """Whether a bfloat16 product of more than 64 rows is the tile kernel's; the others are the vendor's library's.  By its rows
+    alone (``deep_form_rows``), or while a tile of 128 x 128 of it finds a compute unit of its own: measured inside steps (us, tile
+    kernel / library) 566 x 4096 x 1024 17.0 / 17.4, 1295 x 1024 x 1024 13.0 / 14.9, 1959 x 1024 x 1024 13.7 / 15.1, alone 2048 x 1600 x
+    1600 20.5 / 22.0; beyond it, alone, 2048 x 4096 x 1024 23.3 / 21.7, 2048 x 6400 x 1600 54 / 36.  The fused projection of a mixer
+    (``scatters``) a little beyond: the library cannot scatter keys and values, and the copy behind its product costs 6 to
+    8 us (1295 x 3072 x 1024 22.4 / 16.6 + 6.8, 1959 rows 32.5 / 20.0 + 8.2).  Where K is long and rows are many, or tiles few, the library
+    cuts K where this product does not (566 x 1024 x 4096 16.8 / 18.1, 1295 rows 24.4 / 22.2; 2048 x 128 x 2048 13.8 / 11.5).  A K below 512 (not measured) and
+    columns that are no multiple of eight (not stored in whole rows) are the library's."""
+    if deep_form_rows(m, k, lda, n, sliced, scatters):
+        return True
+    if m <= 64 or k % 64 or n % 8 or k < OWN_SHORT_K or m * lda * 2 >= (1 << 32) or n * k * 2 >= (1 << 32):
+        return False
+    if k >= OWN_LONG_K and m > OWN_LONG_ROWS or ((m + 63) // 64) * ((n + 63) // 64) < OWN_LEAST_TILES:
+        return False
+    return ((m + 127) // 128) * ((n + 127) // 128) <= (OWN_SCATTER_TILES if scatters else OWN_TILES)
 
 
 def deep_split_count(rows, columns, k, units=256):
@@ -988,7 +994,7 @@ def float_split_count(rows, columns, k, units=256):
 def prompt_products_in_library(m, n, k, lda, scatters=False):
     """Whether a bfloat16 product of a step of ``m`` rows goes to the vendor's library (which cannot
     scatter keys and values into the cache: the caller then copies them)."""
-    return m > 64 and not deep_form_rows(m, k, lda, n, scatters=scatters) and library_products() is not None
+    return m > 64 and not own_tiles(m, n, k, lda, scatters=scatters) and library_products() is not None
 
 
 def _library_has_algorithm(lda, m, n, k, epilogue):
@@ -1229,7 +1235,7 @@ def activation_needs_a_pass(a, w, activation):
     there without one, and ``activate`` follows (2,048 rows of 4096 x 1024: 24 + 8 us where the tile kernel with
     the activation in its epilogue takes 43)."""
     if a.dtype != torch.bfloat16 or isinstance(a, (Chunked, Normalized)) or not 64 < a.shape[0] <= 65535 or \
-            deep_form_rows(a.shape[0], a.shape[1], a.stride(0), w.shape[0]):
+            own_tiles(a.shape[0], w.shape[0], a.shape[1], a.stride(0)):
         return False
     return activation == "squared_relu" and library_products() is not None
 
