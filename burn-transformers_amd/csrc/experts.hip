@@ -22,6 +22,8 @@
 #include "host.h"
 #include "tile.h"
 
+#include <type_traits>
+
 #define ROUTE_THREADS 1024
 #define ROUTE_MAX_EXPERTS 1024
 
@@ -515,8 +517,7 @@ BT_EXPORT int bt_gated_experts_call(void* stream, const GatedExpertsCall* c) {
 // a plane of its own; the norm behind adds the planes as it adds any partial sums.  The expert that every token uses is
 // one more group whose list is all tokens.  Which expert and rows a work-group takes follows from the counts, which are
 // on the GPU: the grid is the most tiles there can be, and work-groups beyond the counted ones leave at once.
-// Of K the tiles hold 128-byte rows as the plain products' deep forms do (tile.h); 128 columns and BM rows of a tile on four
-// waves.  Where units have a gate, the two 32-wide blocks of a wave's columns are 32 gate rows and the up rows beside them.
+// The tiles are TilePipe's (tile.h): 128 columns and BM rows on four waves.  Where units have a gate, the two 32-wide blocks of a wave's columns are 32 gate rows and the up rows beside them.
 #define GROUP_PLACE_BITS 24        // a list's entry: the token, and behind it which of the token's choices the expert is
 #define GROUP_MAX_EXPERTS 64       // (a lane an expert)
 
@@ -526,7 +527,10 @@ BT_EXPORT int bt_gated_experts_call(void* stream, const GatedExpertsCall* c) {
 // 157 / 91 / 88, 4,096 289 / 154 / 142; width 2,048 without gates and a shared expert, 200 tokens 98 / 51 / 69, 773 250 / 102 / 101, 2,048
 // 378 / 221 / 192.  One work-group to a unit with more stages loses (128 rows in four: 106 us at 2,048 tokens).  Float: width
 // 1,024 with gates, 128 tokens 104 / 92 / 150, 2,048 908 / 310 / 353.  65 tokens of 1,024 without gates draw (36.6 / 37.2);
-// where the experts have less to do every expert on every row is the cheaper way, and the caller takes it.  What bounds them is what a compute unit pulls, as in the plain products' deep forms: 0.5 to 0.6 PFLOP/s.
+// where the experts have less to do every expert on every row is the cheaper way, and the caller takes it.  Those figures are of a loop that waited for
+// its operands behind every barrier and stored rows 8 bytes at a time; with TilePipe and the shared expert's tiles dealt over the XCDs, at 1,809 tokens of
+// width 1,024 with a shared expert of 2,048: units 53.7 -> 48.3 us, outputs 43.0 -> 34.4; 2,048 tokens without one 43.9 -> 40.8 and 24.7 -> 22.1.
+// What bounds them: two rounds of tiles of sixteen turns each, 5 us of launch, first loads and last stores beside 17 us of LDS traffic.
 #define EXPERT_TALL_ROWS 192
 
 struct GroupExpertsCall {
@@ -643,18 +647,24 @@ __device__ __forceinline__ bool group_tile(const ExpertProductsCall& c, int colu
     const int r = __shfl_up(rows_to, o, 64), t = __shfl_up(tiles_to, o, 64);
     if (lane >= o) { rows_to += r; tiles_to += t; }
   }
-  const int routed = __builtin_amdgcn_readlane(tiles_to, 63) * columns;
-  const int all = routed + (c.tokens + BM - 1) / BM * shared_columns;
+  const int routed = __builtin_amdgcn_readlane(tiles_to, 63) * columns, to_all = (c.tokens + BM - 1) / BM * shared_columns;
+  const int all = routed + to_all;
   if ((int)blockIdx.x >= all) return false;
-  const int id = xcd_contiguous(blockIdx.x, all);
-  if (id >= routed) {
+  // Every XCD takes its run of the shared expert's tiles first and of the others behind: in the second product they have their own K,
+  // and numbered in one line some XCDs had the long ones alone (43 us where the others were done after 28).
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  auto start = [&](int n) { return xcd * (n >> 3) + (xcd < (n & 7) ? xcd : n & 7); };
+  const int own = (to_all >> 3) + (xcd < (to_all & 7) ? 1 : 0);
+  if (local < own) {
+    const int id = start(to_all) + local;
     tile.expert = -1;
-    tile.first = (id - routed) / shared_columns * BM;
-    tile.column = (id - routed) % shared_columns;
+    tile.first = id / shared_columns * BM;
+    tile.column = id % shared_columns;
     tile.count = c.tokens;
     tile.slot = 0;
     return true;
   }
+  const int id = start(all) - start(to_all) + local - own;
   const int row_tile = id / columns;
   tile.column = id % columns;
   tile.expert = __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles_to > row_tile));
@@ -665,10 +675,9 @@ __device__ __forceinline__ bool group_tile(const ExpertProductsCall& c, int colu
 }
 
 template <typename T, int BM, int STAGES, bool SECOND, bool GATED>
-__global__ void __launch_bounds__(256) expert_products_kernel(ExpertProductsCall c) {
+__global__ void __launch_bounds__(256, 2) expert_products_kernel(ExpertProductsCall c) {
   constexpr int ELEMS = Mma<T>::ELEMS, ROW_K = 8 * ELEMS, BN = 128;
-  constexpr int STAGE_BYTES = (BM + BN) * TILE_ROW_BYTES;
-  constexpr int LOADS = (BM + BN) / 32;
+  typedef TilePipe<T, BM, BN, 2, 2, STAGES> Pipe;
   constexpr int TM = BM / 64;
   constexpr int HELD = !SECOND && GATED ? 64 : 128;                     // output columns of a tile
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // [STAGES][BM + BN][128 bytes]
@@ -694,39 +703,6 @@ __global__ void __launch_bounds__(256) expert_products_kernel(ExpertProductsCall
     w = static_cast<const T*>(c.w) + (int64_t)(shared ? c.experts : tile.expert) * c.ff * (GATED ? 2 : 1) * c.ld_w;
   }
   const int64_t ld_a = SECOND ? ff : c.ldh;
-  const unsigned char* a_bytes = reinterpret_cast<const unsigned char*>(a);
-  const unsigned char* w_bytes = reinterpret_cast<const unsigned char*>(w);
-  const int count = (SECOND ? ff : c.width) / ROW_K;
-  int64_t off[LOADS];
-  bool from_w[LOADS];
-#pragma unroll
-  for (int j = 0; j < LOADS; ++j) {
-    const int first_row = __builtin_amdgcn_readfirstlane(8 * (LOADS * wave + j));
-    from_w[j] = first_row >= BM;                  // (eight rows never straddle BM)
-    const int stage_row = first_row + (lane >> 3), chunk = (lane & 7) ^ ((stage_row >> 1) & 7);
-    int64_t row;
-    if (from_w[j]) {
-      const int r = stage_row - BM;
-      int n = !SECOND && GATED ? n_base + (r >> 6) * 32 + (r & 31) : n_base + r;
-      n = n < n_end ? n : n_end - 1;
-      row = (!SECOND && GATED && (r & 32) ? ff : 0) + n;
-    } else {
-      int m = tile.first + stage_row;
-      m = m < tile.count ? m : tile.count - 1;
-      row = SECOND ? m : token(m);
-    }
-    off[j] = (row * (from_w[j] ? c.ld_w : ld_a) + chunk * ELEMS) * (int64_t)sizeof(T);
-  }
-  auto issue = [&](int stage) {
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)((from_w[j] ? w_bytes : a_bytes) + off[j]),
-          (__attribute__((address_space(3))) void*)(lds + stage * STAGE_BYTES + 8 * (LOADS * wave + j) * TILE_ROW_BYTES),
-          16, 0, 0);
-    a_bytes += TILE_ROW_BYTES;
-    w_bytes += TILE_ROW_BYTES;
-  };
   // the rows' tokens and weights are asked for before the operands
   int held[TM];
   float weight[TM];
@@ -741,12 +717,6 @@ __global__ void __launch_bounds__(256) expert_products_kernel(ExpertProductsCall
       else if (c.gate) weight[bm] = c.gate[t];
     }
   }
-  int w_rd[4], a_rd[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) {
-    w_rd[kk] = BM * TILE_ROW_BYTES + swizzled(wn * 64 + l32, 2 * kk + g);
-    a_rd[kk] = swizzled(wm * (BM / 2) + l32, 2 * kk + g);
-  }
   floatx16 acc[2][TM];
 #pragma unroll
   for (int bn = 0; bn < 2; ++bn)
@@ -754,77 +724,74 @@ __global__ void __launch_bounds__(256) expert_products_kernel(ExpertProductsCall
     for (int bm = 0; bm < TM; ++bm)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0.f;
-#pragma unroll
-  for (int t = 0; t < STAGES - 1; ++t)
-    if (t < count) issue(t);
-  int stage = 0, next_stage = STAGES - 1;
-  for (int i = 0; i < count; ++i) {
-    wait_for_all_but<STAGES - 2, LOADS>(count - 1 - i);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (i + STAGES - 1 < count) issue(next_stage);
-    const unsigned char* base = lds + stage * STAGE_BYTES;
-    int4v wop[4][2], aop[4][TM];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-#pragma unroll
-      for (int b = 0; b < 2; ++b) wop[kk][b] = *reinterpret_cast<const int4v*>(base + w_rd[kk] + b * 4096);
-#pragma unroll
-      for (int b = 0; b < TM; ++b) aop[kk][b] = *reinterpret_cast<const int4v*>(base + a_rd[kk] + b * 4096);
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
-#pragma unroll
-        for (int bm = 0; bm < TM; ++bm) Mma<T>::block32(acc[bn][bm], wop[kk][bn], aop[kk][bm]);
-    stage = stage + 1 == STAGES ? 0 : stage + 1;
-    next_stage = next_stage + 1 == STAGES ? 0 : next_stage + 1;
-  }
+  Pipe::template multiply<int64_t>(
+      lds, reinterpret_cast<const unsigned char*>(a), reinterpret_cast<const unsigned char*>(w), (SECOND ? ff : c.width) / ROW_K,
+      [&](int stage_row, bool from_w) {
+        if (!from_w) {
+          const int m = tile.first + stage_row < tile.count ? tile.first + stage_row : tile.count - 1;
+          return (SECOND ? m : token(m)) * ld_a * (int64_t)sizeof(T);
+        }
+        const int r = stage_row - BM;
+        int n = !SECOND && GATED ? n_base + (r >> 6) * 32 + (r & 31) : n_base + r;
+        n = n < n_end ? n : n_end - 1;
+        return ((!SECOND && GATED && (r & 32) ? ff : 0) + n) * c.ld_w * (int64_t)sizeof(T);
+      },
+      acc);
+  __syncthreads();
 
-  // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m)
+  // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m); its rows go through LDS, so that memory
+  // sees 16-byte pieces of whole rows
+  typedef typename std::conditional<SECOND, float, T>::type Out;
+  constexpr int COLUMNS = HELD / 2, PIECE = 16 / (int)sizeof(Out), LANES = COLUMNS / PIECE, PITCH = COLUMNS * (int)sizeof(Out) + 16;
+  unsigned char* scratch = lds + wave * (BM / 2 * PITCH);
   GatedExpertsCall unit;
   unit.act = c.act;
   unit.limit = c.limit;
   unit.alpha = c.alpha;
 #pragma unroll
-  for (int bm = 0; bm < TM; ++bm) {
-    if (held[bm] < 0) continue;
-    const int m = tile.first + wm * (BM / 2) + bm * 32 + l32;
-    if (SECOND) {
-      const int t = held[bm] & ((1 << GROUP_PLACE_BITS) - 1), place = shared ? c.top : held[bm] >> GROUP_PLACE_BITS;
-      float* out = c.out + place * c.plane + (int64_t)t * c.ld_out;
+  for (int bm = 0; bm < TM; ++bm)
 #pragma unroll
-      for (int bn = 0; bn < 2; ++bn)
+    for (int bn = 0; bn < COLUMNS / 32; ++bn)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n_base + wn * 64 + bn * 32 + q * 8 + g * 4;
-          if (n < n_end) *reinterpret_cast<floatx4*>(out + n) = floatx4{acc[bn][bm][4 * q], acc[bn][bm][4 * q + 1], acc[bn][bm][4 * q + 2], acc[bn][bm][4 * q + 3]};
+      for (int q = 0; q < 4; ++q) {
+        typedef __attribute__((__vector_size__(4 * sizeof(Out)))) Out Out4;
+        Out4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (SECOND) v[i] = acc[bn][bm][4 * q + i];
+          else v[i] = from_float<T>(weight[bm] * (GATED ? gated_unit(unit, acc[0][bm][4 * q + i], acc[1][bm][4 * q + i])
+                                                        : plain_unit(unit, acc[bn][bm][4 * q + i])));
         }
-    } else {
-      T* out = shared ? static_cast<T*>(c.shared_hidden) + (int64_t)m * ff : static_cast<T*>(c.hidden) + (int64_t)(tile.slot + m) * ff;
+        *reinterpret_cast<Out4*>(scratch + (bm * 32 + l32) * PITCH + (bn * 32 + q * 8 + g * 4) * (int)sizeof(Out)) = v;
+      }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (a wave's accesses of LDS are served in order)
+  const int n = n_base + wn * COLUMNS + lane % LANES * PIECE;
+  constexpr int TURNS = BM / 2 * LANES / 64;
+  int row[TURNS];
 #pragma unroll
-      for (int bn = 0; bn < (GATED ? 1 : 2); ++bn)
+  for (int t = 0; t < TURNS; ++t) {
+    const int m = tile.first + wm * (BM / 2) + (64 / LANES) * t + lane / LANES;
+    row[t] = m < tile.count ? (SECOND ? entry(m) : m) : -1;
+  }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n_base + (GATED ? wn * 32 : wn * 64 + bn * 32) + q * 8 + g * 4;
-          if (n >= n_end) continue;
-          typedef __attribute__((__vector_size__(4 * sizeof(T)))) T T4;
-          T4 v;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            v[i] = from_float<T>(weight[bm] * (GATED ? gated_unit(unit, acc[0][bm][4 * q + i], acc[1][bm][4 * q + i])
-                                                     : plain_unit(unit, acc[bn][bm][4 * q + i])));
-          *reinterpret_cast<T4*>(out + n) = v;
-        }
-    }
+  for (int t = 0; t < TURNS; ++t) {
+    const int4v v = *reinterpret_cast<const int4v*>(scratch + ((64 / LANES) * t + lane / LANES) * PITCH + lane % LANES * 16);
+    if (row[t] < 0 || n >= n_end) continue;
+    Out* out;
+    if constexpr (SECOND)
+      out = c.out + (shared ? c.top : row[t] >> GROUP_PLACE_BITS) * c.plane + (int64_t)(row[t] & ((1 << GROUP_PLACE_BITS) - 1)) * c.ld_out;
+    else
+      out = shared ? static_cast<T*>(c.shared_hidden) + (int64_t)row[t] * ff : static_cast<T*>(c.hidden) + (int64_t)(tile.slot + row[t]) * ff;
+    *reinterpret_cast<int4v*>(out + n) = v;
   }
 }
 
 template <typename T, int BM, int STAGES, bool SECOND, bool GATED>
 static int launch_expert_products(hipStream_t s, const ExpertProductsCall& c) {
   auto kernel = expert_products_kernel<T, BM, STAGES, SECOND, GATED>;
-  const size_t lds = (size_t)STAGES * (BM + 128) * TILE_ROW_BYTES;
+  // (a wave leaves BM / 2 rows of its half of the columns there in the end, 16 bytes between them)
+  const size_t stages = (size_t)STAGES * (BM + 128) * TILE_ROW_BYTES, rows = (size_t)2 * BM * ((SECOND ? 256 : 64 * sizeof(T)) + 16);
+  const size_t lds = stages > rows ? stages : rows;
   static bool raised = false;
   if (!raised) {
     hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
