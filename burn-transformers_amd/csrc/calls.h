@@ -10,6 +10,7 @@
 
 #include "attention.h"
 #include "epilogue.h"
+#include "route.h"
 
 // Rows of the float32 residual stream that the skinny product normalises itself.
 struct NormOperand {
@@ -69,6 +70,11 @@ struct GemmCall {
   const void* W;
   Epilogue epi;
   NormOperand norm;
+};
+
+struct WeighedGemmCall {
+  GemmCall gemm;
+  WeighedRows rows;
 };
 
 struct AttentionCall {
