@@ -795,12 +795,22 @@ static int launch_parts_form(hipStream_t s, const float* a, int64_t lda, const f
 // The forms of the tile kernel for whole tiles of K.
 static int launch_form(hipStream_t s, int variant, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N, int K,
                        const Epilogue& epi, int splits) {
+  // A long K with one tile to a unit at most: the LDS is its own, and more tiles on their way hide more of the weights' way from
+  // memory (cold weights, us: 200 x 1600 x 6400 28.1 -> 24.8; a shorter K pays for the longer start: 290 x 2048 x 1024 6.6 -> 7.3,
+  // and prompts of 220 tokens at width 1,024, whose K is 2,048 at most, 1,009 -> 1,017).
+  auto alone = [&](int bm, int bn) {
+    return K / TILE_K / splits >= 48 && (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * splits <= 256;
+  };
   switch (variant) {
     case 2: return launch_pipe<128, 128, 2, 2, 2>(s, a, lda, w, M, N, K, epi, splits);
     case 3: return launch_pipe<128, 128, 2, 4, 4>(s, a, lda, w, M, N, K, epi, splits);
     case 4: return launch_pipe<64, 64, 2, 2, 3>(s, a, lda, w, M, N, K, epi, splits);
-    case 5: return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
-    case 6: return launch_pipe<64, 128, 1, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 5:
+      if (alone(64, 64)) return launch_pipe<64, 64, 2, 2, 8>(s, a, lda, w, M, N, K, epi, splits);
+      return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 6:
+      if (alone(64, 128)) return launch_pipe<64, 128, 1, 4, 6>(s, a, lda, w, M, N, K, epi, splits);
+      return launch_pipe<64, 128, 1, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
     case 7: return launch_pipe<128, 256, 2, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
   }
   BT_REFUSE("gemm_tile: unknown form %d", variant);

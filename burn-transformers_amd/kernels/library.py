@@ -891,7 +891,8 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
             impl = "skinny"
         elif dtype == FLOAT32:
             impl = "tile"
-        elif own_tiles(m, n, k, a.stride(0), sliced=splits > 1, scatters=epilogue.mode == EPI_QKV):
+        elif own_tiles(m, n, k, a.stride(0), sliced=splits > 1, scatters=epilogue.mode == EPI_QKV,
+                       residual=epilogue.mode == EPI_RESIDUAL):
             impl = "tile"
         else:
             impl = "library" if splits == 1 and _library_takes(epilogue) and library_products() \
@@ -923,11 +924,12 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
 DEEP_FORM_ROWS = 256          # most rows of a bfloat16 product that the tile kernel takes whatever its other sizes ...
 DEEP_FORM_SLICED_ROWS = 512   # ... and of one that leaves partial sums of slices of K pending ...
 DEEP_FORM_SCATTER_ROWS = 384  # ... and of one that scatters keys and values into the cache
-OWN_TILES = 256               # beyond: most tiles of 128 x 128 of a product that the tile kernel takes ...
-OWN_SCATTER_TILES = 288       # ... and of one that scatters keys and values; its fewest tiles of 64 x 64 ...
-OWN_LEAST_TILES = 128
-OWN_SHORT_K = 512             # ... and its shortest K
-OWN_LONG_K, OWN_LONG_ROWS = 2048, 768     # from this K on: up to so many rows
+OWN_TILES = 256               # beyond: most tiles of 64 x 128 of a product that the tile kernel takes ...
+OWN_LONG_K, OWN_LONG_TILES = 2048, 128    # ... from this K on, and ...
+OWN_SCATTER_TILES = 512       # ... of one that scatters keys and values; most tiles of 128 x 128 of one that ...
+OWN_RESIDUAL_TILES = 256      # ... adds to the residual stream; the fewest tiles of 64 x 64 and the shortest K
+OWN_LEAST_TILES, OWN_SHORT_K = 128, 512
+
 
 
 def deep_form_rows(m, k, lda, n, sliced=False, scatters=False):
@@ -938,22 +940,28 @@ def deep_form_rows(m, k, lda, n, sliced=False, scatters=False):
     return 64 < m <= limit and k % 64 == 0 and m * lda * 2 < (1 << 32) and n * k * 2 < (1 << 32)
 
 
-def own_tiles(m, n, k, lda, sliced=False, scatters=False):
+def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False):
     """Whether a bfloat16 product of more than 64 rows is the tile kernel's; the others are the vendor's library's.  By its rows
-    alone (``deep_form_rows``), or while a tile of 128 x 128 of it finds a compute unit of its own: measured inside steps (us, tile
-    kernel / library) 566 x 4096 x 1024 17.0 / 17.4, 1295 x 1024 x 1024 13.0 / 14.9, 1959 x 1024 x 1024 13.7 / 15.1, alone 2048 x 1600 x
-    1600 20.5 / 22.0; beyond it, alone, 2048 x 4096 x 1024 23.3 / 21.7, 2048 x 6400 x 1600 54 / 36.  The fused projection of a mixer
-    (``scatters``) a little beyond: the library cannot scatter keys and values, and the copy behind its product costs 6 to
-    8 us (1295 x 3072 x 1024 22.4 / 16.6 + 6.8, 1959 rows 32.5 / 20.0 + 8.2).  Where K is long and rows are many, or tiles few, the library
-    cuts K where this product does not (566 x 1024 x 4096 16.8 / 18.1, 1295 rows 24.4 / 22.2; 2048 x 128 x 2048 13.8 / 11.5).  A K below 512 (not measured) and
-    columns that are no multiple of eight (not stored in whole rows) are the library's."""
+    alone (``deep_form_rows``), or while a tile of 64 x 128 of it finds a compute unit of its own: measured (us, tile kernel /
+    library) at K = 1,024 610 x 3072 9.4 / 10.4, 1024 x 2048 9.3 / 10.6, 1500 x 1024 9.1 / 9.9, with more tiles 610 x 4096 12.5 / 12.0, 768 x
+    3072 12.3 / 12.0, 1500 x 2048 12.8 / 11.7; K = 1,600 450 x 4096 12.3 / 13.9, 610 x 4096 15.9 / 15.1.  With a
+    longer K the library cuts K where this product does not: half as many tiles (K = 2,048 with cold weights: 610 x 2048 16.4 / 15.0, 768 x 2048 17.4 / 14.9; K = 4,096: 450 x 2048 15.9 / 18.0, 610 x
+    2048 29.2 / 23.4), and for the same reason not too few (2048 x 128 x 2048 13.8 / 11.5).  What adds to the residual stream
+    (``residual``) while a tile of 128 x 128 finds a unit of its own, since the library reads and writes the stream in a
+    slower way (1295 x 1024 x 1024 10.4 / 11.2, 2048 x 1600 x 1600 20.5 / 22.0).  The fused projection of a mixer (``scatters``) up to two tiles of 64 x
+    128 a unit: the library cannot scatter keys and values, and the copy behind its product costs 6 to 8 us (1295 x 3072 x 1024
+    22.4 / 16.6 + 6.8 inside a step, 1959 rows 32.5 / 20.0 + 8.2).  A K below 512 (not measured) and columns that are no multiple of
+    eight (not stored in whole rows) are the library's."""
     if deep_form_rows(m, k, lda, n, sliced, scatters):
         return True
     if m <= 64 or k % 64 or n % 8 or k < OWN_SHORT_K or m * lda * 2 >= (1 << 32) or n * k * 2 >= (1 << 32):
         return False
-    if k >= OWN_LONG_K and m > OWN_LONG_ROWS or ((m + 63) // 64) * ((n + 63) // 64) < OWN_LEAST_TILES:
+    tiles = lambda rows, columns: ((m + rows - 1) // rows) * ((n + columns - 1) // columns)
+    if tiles(64, 64) < OWN_LEAST_TILES:
         return False
-    return ((m + 127) // 128) * ((n + 127) // 128) <= (OWN_SCATTER_TILES if scatters else OWN_TILES)
+    if k >= OWN_LONG_K:
+        return tiles(64, 128) <= OWN_LONG_TILES
+    return tiles(64, 128) <= (OWN_SCATTER_TILES if scatters else OWN_TILES) or (residual and tiles(128, 128) <= OWN_RESIDUAL_TILES)
 
 
 def deep_split_count(rows, columns, k, units=256):

@@ -77,8 +77,9 @@ def test_scattered_keys_and_values(dtype, heads, kv_heads, hd):
 
 
 def test_which_products_are_the_tile_kernels():
-    assert K.own_tiles(566, 4096, 1024, 1024) and K.own_tiles(2048, 1600, 1600, 1600)
-    assert not K.own_tiles(2048, 4096, 1024, 1024) and not K.own_tiles(1295, 1024, 4096, 4096) and K.own_tiles(566, 1024, 4096, 4096)
+    assert K.own_tiles(610, 3072, 1024, 1024) and K.own_tiles(1024, 2048, 1024, 1024) and K.own_tiles(450, 2048, 4096, 4096)
+    assert not K.own_tiles(610, 4096, 1024, 1024) and not K.own_tiles(610, 2048, 4096, 4096)
+    assert K.own_tiles(2048, 1600, 1600, 1600, residual=True) and not K.own_tiles(2048, 1600, 1600, 1600)
     assert K.own_tiles(1295, 3072, 1024, 1024, scatters=True) and not K.own_tiles(2048, 3072, 1024, 1024, scatters=True)
     assert not K.own_tiles(2048, 128, 1024, 1024)            # too few tiles
     assert not K.own_tiles(64, 1024, 1024, 1024) and not K.own_tiles(566, 1024, 1000, 1000) and not K.own_tiles(300, 517, 1600, 1600)
