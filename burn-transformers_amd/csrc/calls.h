@@ -10,7 +10,6 @@
 
 #include "attention.h"
 #include "epilogue.h"
-#include "route.h"
 
 // Rows of the float32 residual stream that the skinny product normalises itself.
 struct NormOperand {
@@ -70,11 +69,6 @@ struct GemmCall {
   const void* W;
   Epilogue epi;
   NormOperand norm;
-};
-
-struct WeighedGemmCall {
-  GemmCall gemm;
-  WeighedRows rows;
 };
 
 struct AttentionCall {

@@ -24,8 +24,6 @@
 #include "epilogue.h"
 #include "calls.h"
 
-#include <type_traits>
-
 #define TILE_K 64            // bfloat16 values in a 128-byte row of an LDS tile
 
 // BM x BN tiles of 128-byte rows (64 bfloat16 or 32 float K values), WM x WN waves, each wave
@@ -434,22 +432,13 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
 // statistics are computed while the weights are on their way.
 __device__ float bt_norm_zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
-//
-// QPL == SKINNY_WEIGHED (bfloat16, up to 16 rows, up to 64 experts): the rows are the units of a step's experts, not yet weighed.
-// Eight more waves of every work-group make the tokens' choices, one each, while the first eight stream the weights; an expert's
-// sums are weighed when a wave goes on to the next one's chunks (whole chunks of an expert: ff a multiple of 32), where a
-// kernel before the product weighed the rows and rounded them to bfloat16 once more.
-#define SKINNY_WEIGHED -1
 template <typename T, int MT, int NT, int U, int WAVES, int QPL = 0, bool CHUNKED = false, int KIND = EPILOGUE_COMMON>
-__global__ void __launch_bounds__(WAVES * (QPL == SKINNY_WEIGHED ? 128 : 64))
+__global__ void __launch_bounds__(WAVES * 64)
 gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
-                   int K, Epilogue epi, int tile_columns,
-                   typename std::conditional<QPL == SKINNY_WEIGHED, WeighedRows, NormOperand>::type norm, int packed, int a_rows) {
+                   int K, Epilogue epi, int tile_columns, NormOperand norm, int packed, int a_rows) {
   constexpr int ELEMS = Mma<T>::ELEMS;      // K values in a lane's 16-byte load
   constexpr int CHUNK = 4 * ELEMS;          // K values the wave's four K groups cover together
-  constexpr bool NORM = QPL > 0, WEIGHED = QPL == SKINNY_WEIGHED;
-  static_assert(!WEIGHED || (MT == 1 && sizeof(T) == 2 && !CHUNKED && 2 * WAVES >= WEIGHED_MAX_ROWS), "weighed rows are row-major bfloat16, two to a wave at most");
-  __shared__ float factors[WEIGHED ? WEIGHED_MAX_ROWS : 1][WEIGHED ? WEIGHED_MAX_EXPERTS : 1], scores[WEIGHED ? WAVES : 1][WEIGHED ? WEIGHED_MAX_EXPERTS : 1];
+  constexpr bool NORM = QPL > 0;
   static_assert(!NORM || (MT == 1 && sizeof(T) == 2), "the fused norm is for bfloat16 and up to 16 rows");
   extern __shared__ __attribute__((aligned(16))) unsigned char normed[];   // NORM: [16][K * 2 + 16] bytes
   const int normed_pitch = K * 2 + 16;      // the 16 bytes spread the rows over the LDS banks
@@ -466,27 +455,6 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
   const int n_base = blockIdx.x * tile_columns;
   const int n_end = n_base + tile_columns < N ? n_base + tile_columns : N;   // one past this work-group's last column
   const int split = blockIdx.y, splits = gridDim.y;
-  if constexpr (WEIGHED)
-    if (wave >= WAVES) {                   // the second half of the waves: a token's choice each
-      RouteEarly early;
-      early.load(norm.route);
-      const int first = wave - WAVES;
-      float logit[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {        // (rows and experts that do not exist read a logit that does)
-        const int r = first + j * WAVES < M ? first + j * WAVES : M - 1;
-        logit[j] = norm.logits[(int64_t)r * norm.ld_logits + (lane < norm.route.experts ? lane : 0)];
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        if (first + j * WAVES < M) {
-          scores[first][lane] = logit[j];
-          route_choice(norm.route, early, scores[first], factors[first + j * WAVES]);
-        }
-      __syncthreads();                     // the choices are made
-      __syncthreads();                     // (the others' sums)
-      return;
-    }
   // packed: W is not [N][K] but, for each work-group's `tile_columns` columns, the chunks of K one
   // after the other, [group][chunk][tile_columns][CHUNK], K and the last group padded with zeros:
   // a wave's load of a chunk is then one contiguous run of bytes and a work-group reads one
@@ -516,11 +484,8 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
   // a bit mask) and multiplied.  Nothing that depends on a lane or on loaded data stands between
   // the loads, so the compiler has no reason to wait for one before it issues the next.
   // Rows beyond M repeat row M - 1; their results are dropped by the epilogue.
-  const int all_chunks = (K + CHUNK - 1) / CHUNK, per_wave = (all_chunks + splits * WAVES - 1) / (splits * WAVES);
-  // (WEIGHED: a wave's chunks lie behind one another, of one expert or two: its sums are weighed once or twice, and late)
-  const int stride = WEIGHED ? 1 : splits * WAVES;
-  const int begin = WEIGHED ? (split * WAVES + wave) * per_wave : split * WAVES + wave;
-  const int chunks = WEIGHED ? (begin + per_wave < all_chunks ? begin + per_wave : all_chunks) : all_chunks;
+  const int chunks = (K + CHUNK - 1) / CHUNK;
+  const int stride = splits * WAVES;
   floatx4 acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -550,46 +515,10 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
       }
     }
   };
-  // WEIGHED: the sums of one expert's chunks, weighed when the next one's begin (a lane's sums are all of row i16); the first to
-  // be weighed wait for the choices
-  floatx4 weighed[WEIGHED ? NT : 1];
-  int expert = 0, expert_end = 0;          // the sums' expert, and one past its last chunk
-  bool chosen = false;
-  auto begin_expert = [&](int chunk) {
-    if constexpr (WEIGHED) {
-      const int of_one = norm.ff / CHUNK;
-      expert = chunk / of_one < norm.route.experts ? chunk / of_one : norm.route.experts;
-      expert_end = expert < norm.route.experts ? (expert + 1) * of_one : all_chunks;
-    }
-  };
-  auto weigh = [&] {
-    if constexpr (WEIGHED) {
-      if (!chosen) __syncthreads();
-      chosen = true;
-      const float f = expert < norm.route.experts ? factors[i16 < M ? i16 : M - 1][expert] : 1.f;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          weighed[nt][r] += f != 0.f ? f * acc[0][nt][r] : 0.f;
-          acc[0][nt][r] = 0.f;
-        }
-    }
-  };
-  if constexpr (WEIGHED) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) weighed[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    begin_expert(begin);
-  }
   auto multiply = [&](int c0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       int keep = (c0 + u * stride) * CHUNK + g * ELEMS < K ? -1 : 0;
-      if constexpr (WEIGHED)
-        if (c0 + u * stride >= expert_end && c0 + u * stride < chunks) {
-          weigh();
-          begin_expert(c0 + u * stride);
-        }
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         int4v w = wv[u][nt] & keep;
@@ -609,7 +538,7 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
       av[u][0] = *reinterpret_cast<const int4v*>(normed + row * normed_pitch + kc * 2);
     }
   };
-  int c0 = begin;
+  int c0 = split * WAVES + wave;
   if constexpr (NORM) {
     const int quads = K >> 2;
     const float4* g4 = reinterpret_cast<const float4*>(norm.gamma);
@@ -688,11 +617,6 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
     issue(c0);
     if constexpr (NORM) operands_from_lds(c0);
     multiply(c0);
-  }
-  if constexpr (WEIGHED) {
-    weigh();
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[0][nt] = weighed[nt];
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -966,23 +890,13 @@ static int launch_skinny_norm(hipStream_t s, const NormOperand& norm, const bf16
   return BT_OK;
 }
 
-static void launch_skinny_weighed(hipStream_t s, const WeighedRows& rows, const bf16_t* a, int64_t lda, const bf16_t* w, int M, int N,
-                                  int K, const Epilogue& epi, int splits, int columns, int packed) {
-  dim3 grid((N + columns - 1) / columns, splits), block(1024);
-  if (columns <= 16)
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, 1, 1, 8, 8, SKINNY_WEIGHED>), grid, block, 0, s, a, lda, w, M, N, K, epi, columns, rows, packed, 0);
-  else
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, 1, 2, 8, 8, SKINNY_WEIGHED>), grid, block, 0, s, a, lda, w, M, N, K, epi, columns, rows, packed, 0);
-}
-
 // norm: null, or the activations are the normalised rows it describes (then A and lda are ignored)
-// weighed: null, or the rows of A are to be weighed first (see the kernel).
 // a_rows: 0, or A is chunk-major with that many rows (activation_offset in common.h; lda is not used).
 // packed_columns: 0, or W is the packed form of the matrix for that many columns per work-group (see
 // the kernel), which then is the number of columns a work-group takes.
-static int skinny(void* stream, int dtype, const void* A, int64_t lda, const void* W, int M, int N, int K,
-                  const Epilogue* epi, int splits, int variant, const NormOperand* norm, int packed_columns,
-                  int a_rows, const WeighedRows* weighed) {
+BT_EXPORT int bt_gemm_skinny(void* stream, int dtype, const void* A, int64_t lda, const void* W, int M, int N, int K,
+                             const Epilogue* epi, int splits, int variant, const NormOperand* norm, int packed_columns,
+                             int a_rows) {
   if (M <= 0) return BT_OK;
   if (M > 64) BT_REFUSE("gemm_skinny: %d rows, at most 64", M);
   if (dtype != 0 && dtype != 1) BT_REFUSE("gemm_skinny: element type %d is neither float nor bfloat16", dtype);
@@ -1033,9 +947,7 @@ static int skinny(void* stream, int dtype, const void* A, int64_t lda, const voi
       if (best < 0 || cost < best) { best = cost; columns = c; }
     }
   }
-  if (weighed != nullptr) {
-    launch_skinny_weighed((hipStream_t)stream, *weighed, (const bf16_t*)A, lda, (const bf16_t*)W, M, N, K, *epi, splits, columns, packed);
-  } else if (norm != nullptr) {
+  if (norm != nullptr) {
     rc = launch_skinny_norm((hipStream_t)stream, *norm, (const bf16_t*)W, M, N, K, *epi, splits, columns, packed);
     if (rc) return rc;
   } else if (dtype == 0) {
@@ -1052,19 +964,7 @@ BT_EXPORT int bt_gemm_tile_call(void* stream, const GemmCall* c) {
     BT_REFUSE("gemm_tile: no rows to normalise, no chunk-major rows and no packed weights");
   return bt_gemm_tile(stream, c->dtype, c->A, c->lda, c->W, c->M, c->N, c->K, &c->epi, c->splits, c->variant);
 }
-BT_EXPORT int bt_gemm_weighed_call(void* stream, const WeighedGemmCall* w) {
-  const GemmCall* c = &w->gemm;
-  const RouteCall* route = &w->rows.route;
-  if (c->M <= 0) return BT_OK;
-  if (const char* wrong = route_refusal(route)) BT_REFUSE("gemm_weighed: %d of %d experts a token: %s", route->top, route->experts, wrong);
-  if (c->dtype != 1 || c->M > WEIGHED_MAX_ROWS || route->experts > WEIGHED_MAX_EXPERTS || c->has_norm || c->a_rows || c->epi.mode != EPI_F32)
-    BT_REFUSE("gemm_weighed: up to %d plain rows of bfloat16 and %d experts, into partial sums (got %d rows, %d experts)", WEIGHED_MAX_ROWS,
-              WEIGHED_MAX_EXPERTS, c->M, route->experts);
-  if (w->rows.ff <= 0 || w->rows.ff % 32 != 0 || (int64_t)route->experts * w->rows.ff > c->K || !w->rows.logits || w->rows.ld_logits < route->experts || !c->A)
-    BT_REFUSE("gemm_weighed: rows of %d columns do not hold %d experts of %d (a multiple of 32)", c->K, route->experts, w->rows.ff);
-  return skinny(stream, c->dtype, c->A, c->lda, c->W, c->M, c->N, c->K, &c->epi, c->splits, c->variant, nullptr, c->packed_columns, 0, &w->rows);
-}
 BT_EXPORT int bt_gemm_skinny_call(void* stream, const GemmCall* c) {
-  return skinny(stream, c->dtype, c->A, c->lda, c->W, c->M, c->N, c->K, &c->epi, c->splits, c->variant,
-                        c->has_norm ? &c->norm : nullptr, c->packed_columns, c->a_rows, nullptr);
+  return bt_gemm_skinny(stream, c->dtype, c->A, c->lda, c->W, c->M, c->N, c->K, &c->epi, c->splits, c->variant,
+                        c->has_norm ? &c->norm : nullptr, c->packed_columns, c->a_rows);
 }

@@ -225,15 +225,6 @@ class ExpertProductsCall(ctypes.Structure):
     _step_fields_ = {"tokens": "tokens"}
 
 
-class WeighedRows(ctypes.Structure):
-    _fields_ = [("route", RouteCall), ("ff", _c_int), ("logits", _c_ptr), ("ld_logits", _c_i64)]
-
-
-class WeighedGemmCall(ctypes.Structure):
-    _fields_ = [("gemm", GemmCall), ("rows", WeighedRows)]
-    _step_fields_ = {"gemm.M": "tokens", "rows.route.tokens": "tokens"}
-
-
 class WeighExpertsCall(ctypes.Structure):
     _fields_ = [("route", RouteCall), ("ff", _c_int), ("logits", _c_ptr), ("ld_logits", _c_i64), ("hidden", _c_ptr), ("ld_hidden", _c_i64)]
     _step_fields_ = {"route.tokens": "tokens"}
@@ -1471,46 +1462,17 @@ def route(h, router, correction, top, groups, keep, weights, gate_weight=None, g
                       bias=_ptr(bias), used=_ptr(used)))
 
 
-def _router_choice(hidden, bias, correction, experts, top, groups, keep, score, group_rank, normalize):
-    return RouteCall(dtype=DTYPE_CODES[hidden.dtype], tokens=hidden.shape[0], experts=experts, top=top, groups=groups, keep=keep,
-                     correction=_ptr(correction), score={"softmax": 0, "sigmoid": 1, "chosen": 2}[score], group_rank=group_rank,
-                     normalize=1 if normalize else 0, bias=_ptr(bias))
-
-
 def weigh_experts(logits, bias, correction, top, groups, keep, hidden, experts, ff, score="softmax", group_rank=1, normalize=True):
     """hidden[t, e * ff + i] *= the weight of expert e for token t, the choice made as in ``route`` from the float32 router
     ``logits`` [rows, >= experts]; columns of ``hidden`` behind the experts stay."""
     if logits.dtype != torch.float32 or logits.stride(1) != 1 or hidden.stride(1) != 1:
         raise KernelError(f"weigh_experts: float32 logits and plain rows, got {logits.dtype}")
+    call = RouteCall(dtype=DTYPE_CODES[hidden.dtype], tokens=hidden.shape[0], experts=experts, top=top, groups=groups, keep=keep,
+                     correction=_ptr(correction), score={"softmax": 0, "sigmoid": 1, "chosen": 2}[score], group_rank=group_rank,
+                     normalize=1 if normalize else 0, bias=_ptr(bias))
     _launch(_module("experts"), "bt_weigh_experts_call",
-            WeighExpertsCall(route=_router_choice(hidden, bias, correction, experts, top, groups, keep, score, group_rank, normalize), ff=ff,
-                             logits=logits.data_ptr(), ld_logits=logits.stride(0), hidden=hidden.data_ptr(), ld_hidden=hidden.stride(0)))
-
-
-WEIGHED_MAX_ROWS, WEIGHED_MAX_EXPERTS = 16, 64
-
-
-def weighs_in_product(hidden, experts, ff):
-    """Whether ``gemm_weighed`` takes these rows: bfloat16, up to 16 of them, up to 64 experts whose width is a multiple of 32."""
-    return hidden.dtype == torch.bfloat16 and hidden.shape[0] <= WEIGHED_MAX_ROWS and experts <= WEIGHED_MAX_EXPERTS and ff % 32 == 0
-
-
-def gemm_weighed(logits, bias, correction, top, groups, keep, hidden, experts, ff, w, epilogue, splits=1, packed=None, score="softmax",
-                 group_rank=1, normalize=True):
-    """``weigh_experts`` and the product of its rows in one kernel: every work-group of the skinny product makes the choice itself
-    and weighs the experts' sums in 32-bit (``hidden`` stays as it is, nothing is rounded once more).  ``epilogue``: 32-bit partial sums."""
-    m, k = hidden.shape
-    if logits.dtype != torch.float32 or logits.stride(1) != 1 or hidden.stride(1) != 1 or logits.shape[0] < m:
-        raise KernelError(f"gemm_weighed: float32 logits and plain rows, got {logits.dtype}")
-    if w.shape[1] != k or not w.is_contiguous() or w.dtype != hidden.dtype or not weighs_in_product(hidden, experts, ff):
-        raise KernelError(f"gemm_weighed: rows [{m},{k}] {hidden.dtype} of {experts} experts of {ff} and weights {tuple(w.shape)} {w.dtype} do not fit")
-    packed = packed.for_step(m, splits) if packed is not None else None
-    weights, columns = (packed[0].data_ptr(), packed[1]) if packed is not None else (w.data_ptr(), 0)
-    _launch(_module("gemm_mfma"), "bt_gemm_weighed_call",
-            WeighedGemmCall(gemm=GemmCall(dtype=BFLOAT16, M=m, N=w.shape[0], K=k, splits=splits, packed_columns=columns, A=hidden.data_ptr(),
-                                          lda=hidden.stride(0), W=weights, epi=epilogue),
-                            rows=WeighedRows(route=_router_choice(hidden, bias, correction, experts, top, groups, keep, score, group_rank, normalize),
-                                             ff=ff, logits=logits.data_ptr(), ld_logits=logits.stride(0))))
+            WeighExpertsCall(route=call, ff=ff, logits=logits.data_ptr(), ld_logits=logits.stride(0), hidden=hidden.data_ptr(),
+                             ld_hidden=hidden.stride(0)))
 
 
 EXPERT_UNITS = {"gated_silu": 0, "gated_clamped": 1, "gelu_erf": 2, "silu": 3, "squared_relu": 4}

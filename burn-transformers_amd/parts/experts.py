@@ -141,15 +141,11 @@ class RoutedExperts(FeedForward):
             logits = step.buffer("experts.logits", tokens, self.logit_cols, "float32")
             hidden = step.buffer("experts.hidden", tokens, self.hidden_cols, step.dtype)
             K.gemm(h, self.first_weight, K.epilogue_f32_act(logits, self.logit_cols, hidden, self.unit), packed=self.first_packed)
-            choice = (logits, self.router_bias, self.correction, self.top, self.groups, self.keep, hidden, self.experts, self.ff)
-            how = {"score": self.score, "group_rank": self.group_rank, "normalize": self.normalize}
+            K.weigh_experts(logits, self.router_bias, self.correction, self.top, self.groups, self.keep, hidden, self.experts, self.ff,
+                            score=self.score, group_rank=self.group_rank, normalize=self.normalize)
             splits = stream_product_splits(step, hidden, self.down_weight)
             partials = step.partial_sums("experts.partials", splits, tokens, self.width)
-            if K.weighs_in_product(hidden, self.experts, self.ff):
-                K.gemm_weighed(*choice, self.down_weight, K.epilogue_f32(partials), splits=splits, packed=self.down_packed, **how)
-            else:
-                K.weigh_experts(*choice, **how)
-                K.gemm(hidden, self.down_weight, K.epilogue_f32(partials), splits=splits, packed=self.down_packed)
+            K.gemm(hidden, self.down_weight, K.epilogue_f32(partials), splits=splits, packed=self.down_packed)
             return Delta(partials, None)
         weights = step.buffer("experts.weights", tokens, self.outputs, "float32")
         mix = step.buffer("experts.mix", tokens, 1, "float32") if self.shared_mix is not None else None
