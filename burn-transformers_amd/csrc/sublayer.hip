@@ -103,8 +103,9 @@ __global__ void __launch_bounds__(256) output_norm_kernel(OutputNormCall c) {
 // of a thread (partial sums, bias, the stream, the scale) is issued before the first is used, so a
 // row costs one round trip to memory.  A decode step has few rows: one row's latency is its time.
 // A thread's columns are KMAX / 4 quads of neighbours, a load for each (QUADS), or lie 256 apart where the rows are no whole
-// quads.  What bounds it is the chain of a row: its loads, two sums over the work-group, its stores.  8 rows of 2,048 with two
-// partial sums and the next norm 5.4 -> 4.85 us with quads, 773 rows 8.7 -> 8.1.
+// quads.  What bounds it is the chain of a row: its loads, two sums over the work-group, its stores.  With two partial sums and
+// the next norm, one column a load / quads (us, in a HIP graph): 8 rows of 2,048 4.44 / 3.75, of 1,024 3.54 / 3.18; 773 of 2,048
+// 7.86 / 7.35; 1,809 of 1,024 with four partial sums 9.28 / 8.89.
 template <int KMAX, bool QUADS>
 struct RowColumns {
   __device__ __forceinline__ static int column(int k) {
@@ -137,12 +138,39 @@ struct RowColumns {
         if (column(k) < width) row[column(k)] = from_float<O>(v[k]);
     }
   }
+  // The thread's columns that lie 256 apart, of values that are zero beyond the row: what a sum over the row adds up, so that it
+  // is the same number whichever way the row was read.  `row`: LDS for 256 * KMAX values; a barrier stands between its users.
+  // (8 rows of 2,048, columns 256 apart read one by one / quads through LDS / quads added up as they lie: 4.44 / 3.75 / 3.73 us.)
+  __device__ __forceinline__ static void apart(const float (&v)[KMAX], float* row, float (&w)[KMAX]) {
+    if constexpr (QUADS) {
+#pragma unroll
+      for (int k = 0; k < KMAX; k += 4) *reinterpret_cast<floatx4*>(row + column(k)) = floatx4{v[k], v[k + 1], v[k + 2], v[k + 3]};
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < KMAX; ++k) w[k] = row[threadIdx.x + 256 * k];
+    } else {
+#pragma unroll
+      for (int k = 0; k < KMAX; ++k) w[k] = v[k];
+    }
+  }
+  // block_sum of what `apart` left (whose barrier stands in place of the one before the sum's own)
+  __device__ __forceinline__ static float sum(float partial, float* scratch) {
+    if constexpr (!QUADS) return block_sum(partial, scratch);
+    partial = wave_sum(partial);
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = partial;
+    __syncthreads();
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) total += scratch[i];
+    return total;
+  }
 };
 
 template <typename T, int KMAX, bool QUADS>
 __global__ void __launch_bounds__(256) output_norm_small_kernel(OutputNormCall c) {
   typedef RowColumns<KMAX, QUADS> Columns;
   __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float row_buf[QUADS ? 256 * KMAX : 4];
   const int t = blockIdx.x;
   float* xr = c.x + (int64_t)t * c.width;
   // Every load of a thread is issued before the first is used and none stands behind a branch of its
@@ -185,18 +213,23 @@ __global__ void __launch_bounds__(256) output_norm_small_kernel(OutputNormCall c
 #pragma unroll
   for (int k = 0; k < KMAX; ++k)
     if (!in_row[k]) v[k] = xv[k] = g[k] = b[k] = 0.f;
-  float partial = 0.f;
+  float w[KMAX], partial = 0.f;
+  Columns::apart(v, row_buf, w);
   if (c.kind == 0) {          // a layer norm: the mean first, then the squared distances from it
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) partial += v[k];
-    const float mean = block_sum(partial, scratch) / (float)c.width;
+    for (int k = 0; k < KMAX; ++k) partial += w[k];
+    const float mean = Columns::sum(partial, scratch) / (float)c.width;
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) v[k] = in_row[k] ? v[k] - mean : 0.f;
+    for (int k = 0; k < KMAX; ++k) {
+      v[k] = in_row[k] ? v[k] - mean : 0.f;
+      w[k] = (int)threadIdx.x + 256 * k < c.width ? w[k] - mean : 0.f;
+    }
     partial = 0.f;
+    __syncthreads();
   }
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) partial += v[k] * v[k];
-  const float scale = c.mult / sqrtf(block_sum(partial, scratch) / (float)c.width + c.eps);
+  for (int k = 0; k < KMAX; ++k) partial += w[k] * w[k];
+  const float scale = c.mult / sqrtf(Columns::sum(partial, scratch) / (float)c.width + c.eps);
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) v[k] = in_row[k] ? v[k] * scale * g[k] + b[k] + xv[k] : 0.f;
   Columns::store(xr, c.width, v);
@@ -207,19 +240,21 @@ __global__ void __launch_bounds__(256) output_norm_small_kernel(OutputNormCall c
   }
   if (c.next_out) {           // the norm that reads the new row next, from the registers that hold it
     float next_mean = 0.f;
+    Columns::apart(v, row_buf, w);
     if (c.next_kind == 0) {
       float sum = 0.f;
 #pragma unroll
-      for (int k = 0; k < KMAX; ++k) sum += v[k];
-      next_mean = block_sum(sum, scratch) / (float)c.width;
+      for (int k = 0; k < KMAX; ++k) sum += w[k];
+      next_mean = Columns::sum(sum, scratch) / (float)c.width;
+      __syncthreads();
     }
     float squares = 0.f;
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) {
-      const float d = in_row[k] ? v[k] - next_mean : 0.f;
+      const float d = (int)threadIdx.x + 256 * k < c.width ? w[k] - next_mean : 0.f;
       squares += d * d;
     }
-    const float next_rstd = 1.0f / sqrtf(block_sum(squares, scratch) / (float)c.width + c.next_eps);
+    const float next_rstd = 1.0f / sqrtf(Columns::sum(squares, scratch) / (float)c.width + c.next_eps);
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) v[k] = (v[k] - next_mean) * next_rstd * g2[k] + (c.next_beta ? b2[k] : 0.f);
     if (c.next_dtype == 0) Columns::store(static_cast<float*>(c.next_out) + (int64_t)t * c.next_ld, c.width, v);
