@@ -1,6 +1,6 @@
 // Matrix products on the MFMA units of gfx950, C[M,N] = A[M,K] . W[N,K]^T with 32-bit
 // accumulation, in bfloat16 and in float (the float instructions multiply and add in full
-// 32-bit: no reduced-precision mode exists in them; products made of parts keep all 24 bits of both operands).  Both operands are K-contiguous, which is
+// 32-bit: no reduced-precision mode exists in them; products made of parts: see gemm_tile_parts_kernel).  Both operands are K-contiguous, which is
 // what an MFMA lane wants: consecutive K values in one 16-byte load.
 //
 //   gemm_tile    tiles of 64 x 64 to 128 x 256 for many rows (prefill): gemm_tile_pipe_kernel, whose
@@ -216,11 +216,13 @@ gemm_tile_pipe_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict_
 }
 
 // Float products of many rows on the bfloat16 matrix instructions, sixteen times the rate of the float ones.
-// A float is the sum of three bfloat16 values (8 + 8 + 8 bits: the nearest to it, the upper bits of what that leaves, the
-// rest) and a product of two floats the sum of nine products of such parts, each exact in 32 bits.  The six
-// largest are added up in 32 bits, the smallest first; the three left out are below 2^-24 of the product.  A sum is rounded
-// 6 K / 16 times where the float instructions round it K / 2 times and more: against 64 bits the error is 0.67 of theirs at
-// K = 32, 0.85 at K = 768, 0.88 at K = 3072.
+// A float is the sum of three bfloat16 values (the nearest to it, the nearest to what that leaves, the rest, which has at most
+// seven bits) and a product of two floats the sum of nine products of such parts, each exact in 32 bits.  The six
+// largest are added up in 32 bits, the smallest first.  The three left out come to less than 2^-24 of the product, as much as rounding
+// it to 32 bits may cost: over all mantissas the second part is at most 2^-8.005 of a float and the third 2^-17.002 (with the
+// second part cut off instead of rounded 2^-16.01, and twice as much left out), 2^-27.5 (root of the mean square) over drawn ones, of either sign.
+// Beside that a sum is rounded 6 K / 16 times where the float instructions, which do not round products, round it K / 2 times and more:
+// against 64 bits the error of normal values is 0.67 of theirs at K = 32, 0.85 at K = 768, 0.88 at K = 3072.
 // A tile goes from memory to registers (two tiles of K = 32 on their way), is cut there into its parts, every value once for
 // the whole work-group, and lies in LDS as three planes of bfloat16 in three stages: the tile that is multiplied, the
 // next one, whose first operands are read behind the multiplications of the second half of this one, and the one being cut.
@@ -244,10 +246,9 @@ __device__ __forceinline__ FloatParts float_parts(float x0, float x1) {      // 
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const bf16x2 near = {(bf16_t)x0, (bf16_t)x1};
-    const int i0 = __builtin_bit_cast(int, x0), i1 = __builtin_bit_cast(int, x1);
-    p.part[i] = i == 0 ? __builtin_bit_cast(int, near) : (int)__builtin_amdgcn_perm(i1, i0, 0x07060302);
-    x0 -= __builtin_bit_cast(float, i == 0 ? p.part[i] << 16 : i0 & (int)0xffff0000);
-    x1 -= __builtin_bit_cast(float, (i == 0 ? p.part[i] : i1) & (int)0xffff0000);
+    p.part[i] = __builtin_bit_cast(int, near);
+    x0 -= __builtin_bit_cast(float, p.part[i] << 16);
+    x1 -= __builtin_bit_cast(float, p.part[i] & (int)0xffff0000);
   }
   return p;
 }
