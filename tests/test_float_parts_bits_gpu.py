@@ -31,3 +31,62 @@ def test_products_keep_what_a_rounding_would(variant):
     # sixteen products, each short of less than 2^-24 of itself; the sums stay below one: a tenth of that for their roundings
     bound = 16 * x.double()[:, None] * w.double()[None, :] * 2.0 ** -24 * 1.1
     assert float(((product(a, b, variant) - want).abs() / bound).max()) < 1.0
+
+
+@pytest.mark.parametrize("variant", [6, 7])
+@pytest.mark.parametrize("m,n,k,splits", [(130, 140, 96, 1), (300, 260, 800, 3)])
+def test_tiles_that_are_not_finite_are_the_float_instructions(variant, m, n, k, splits):
+    """Where a sum of a tile is not finite the whole tile has the float instructions' numbers, and the other tiles keep theirs."""
+    gen = torch.Generator().manual_seed(m + k)
+    a, w = torch.randn(m, k, generator=gen), torch.randn(n, k, generator=gen)
+    plain, floats = product(a, w, variant, splits), product(a, w, 5, splits)
+    for value in (float("nan"), float("inf"), torch.finfo(torch.float32).max):
+        held = a.clone()
+        held[m - 1, k - 1], held[m - 1, 0] = value, value          # the last block of rows; of slices, the first and the last
+        got, want = product(held, w, variant, splits), product(held, w, 5, splits)
+        last = (m - 1) // 128 * 128
+        assert torch.equal(got[:last], plain[:last])
+        assert torch.equal(torch.isnan(got[last:]), torch.isnan(want[last:]))
+        if splits == 1:
+            assert torch.equal(torch.nan_to_num(got[last:]), torch.nan_to_num(want[last:]))
+        else:                # (slices without such a value keep their sums)
+            fine = slice(last, m - 1)
+            assert float((got[fine] - want[fine]).abs().max() / floats.abs().max()) < 1e-5
+        assert torch.equal(got[m - 1], want[m - 1]) or torch.isnan(want[m - 1]).any()
+
+
+@pytest.mark.parametrize("variant", [6, 7])
+def test_values_that_are_not_finite_cost_no_more_than_the_tile_twice(variant):
+    """A row that is not finite must not hold up every other of the step: the float instructions are below three times the parts' time."""
+    a, w = torch.randn(1200, 768, device=DEV), torch.randn(2304, 768, device=DEV)
+    out = torch.empty(1, 1200, 2304, device=DEV)
+
+    def best(rows):
+        times = []
+        for _ in range(6):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(5):
+                K.gemm(rows, w, K.epilogue_f32(out), impl="tile", variant=variant)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+    spoilt = a.clone()
+    spoilt[7::128] = float("nan")
+    # measured 2 to 3 times; every sum made again by itself, one after the other, took 12 to 100 times
+    assert best(spoilt) < 6 * best(a)
+
+
+@pytest.mark.parametrize("variant", [6, 7])
+@pytest.mark.parametrize("a_exponent,w_exponent", [(-100, 60), (-109, 100), (-118, 100), (-128, 110), (-140, 120), (-70, -58)])
+def test_very_small_values(variant, a_exponent, w_exponent):
+    """Beside the roundings of any product, a value loses what falls below the smallest bfloat16: 2^-134 at most."""
+    gen = torch.Generator().manual_seed(-a_exponent)
+    scaled = lambda rows, exponent: (torch.randn(rows, 64, generator=gen, dtype=torch.float64) * 2.0 ** exponent).float()
+    a, w = scaled(130, a_exponent), scaled(140, w_exponent)
+    want, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    lost = 2.0 ** -134 * (w.double().abs().sum(1)[None, :] + a.double().abs().sum(1)[:, None])
+    # 24 roundings of a sum of 64 products, each at most 2^-24 of their sizes, what is left out, and sums below the smallest normal float
+    bound = 25 * 2.0 ** -24 * size + lost + 64 * 2.0 ** -149
+    assert float(((product(a, w, variant) - want).abs() / bound).max()) < 1.0
