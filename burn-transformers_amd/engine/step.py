@@ -24,7 +24,7 @@ def token_capacity(tokens):
     """The class of a step by its tokens: steps of up to 64 tokens are their own class; beyond, the
     classes are 65 .. 128, 129 .. 192 and so on.  Every step of a class lays its tables out for the
     class's most tokens and reserves its workspaces for them, and every choice of kernels that the
-    parts make by a step's rows is the same for a whole class (they turn at 64, 128 and 256 rows or weigh the class's most), so
+    parts make by a step's rows is the same for a whole class (they turn at multiples of 64 rows or weigh the class's most), so
     that one launch list serves the class: only the counts in its calls differ from step to step."""
     return tokens if tokens <= BLOCK else (tokens + BLOCK - 1) // BLOCK * BLOCK
 

@@ -917,10 +917,9 @@ DEEP_FORM_SLICED_ROWS = 512   # ... and of one that leaves partial sums of slice
 DEEP_FORM_SCATTER_ROWS = 384  # ... and of one that scatters keys and values into the cache
 OWN_TILES = 256               # beyond: most tiles of 64 x 128 of a product that the tile kernel takes ...
 OWN_LONG_K, OWN_LONG_TILES = 2048, 128    # ... from this K on, and ...
-OWN_SCATTER_TILES = 512       # ... of one that scatters keys and values; most tiles of 128 x 128 of one that ...
-OWN_RESIDUAL_TILES = 256      # ... adds to the residual stream; the fewest tiles of 64 x 64 and the shortest K
+OWN_SCATTER_TILES = 512       # ... of one that scatters keys and values, whatever its K; most tiles of 128 x 128 of one ...
+OWN_RESIDUAL_TILES = 256      # ... with a shorter K that adds to the residual stream; the fewest tiles of 64 x 64 and the shortest K
 OWN_LEAST_TILES, OWN_SHORT_K = 128, 512
-
 
 
 def deep_form_rows(m, k, lda, n, sliced=False, scatters=False):
@@ -936,13 +935,20 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False):
     alone (``deep_form_rows``), or while a tile of 64 x 128 of it finds a compute unit of its own: measured (us, tile kernel /
     library) at K = 1,024 610 x 3072 9.4 / 10.4, 1024 x 2048 9.3 / 10.6, 1500 x 1024 9.1 / 9.9, with more tiles 610 x 4096 12.5 / 12.0, 768 x
     3072 12.3 / 12.0, 1500 x 2048 12.8 / 11.7; K = 1,600 450 x 4096 12.3 / 13.9, 610 x 4096 15.9 / 15.1.  With a
-    longer K the library cuts K where this product does not: half as many tiles (K = 2,048 with cold weights: 610 x 2048 16.4 / 15.0, 768 x 2048 17.4 / 14.9; K = 4,096: 450 x 2048 15.9 / 18.0, 610 x
-    2048 29.2 / 23.4), and for the same reason not too few (2048 x 128 x 2048 13.8 / 11.5).  What adds to the residual stream
-    (``residual``) while a tile of 128 x 128 finds a unit of its own, since the library reads and writes the stream in a
-    slower way (1295 x 1024 x 1024 10.4 / 11.2, 2048 x 1600 x 1600 20.5 / 22.0).  The fused projection of a mixer (``scatters``) up to two tiles of 64 x
-    128 a unit: the library cannot scatter keys and values, and the copy behind its product costs 6 to 8 us (1295 x 3072 x 1024
-    22.4 / 16.6 + 6.8 inside a step, 1959 rows 32.5 / 20.0 + 8.2).  A K below 512 (not measured) and columns that are no multiple of
-    eight (not stored in whole rows) are the library's."""
+    K of 2,048 and more the library cuts K where this product does not: half as many tiles (K = 2,048 with cold weights: 610 x 2048 16.4 / 15.0, 768 x 2048 17.4 / 14.9; K = 4,096: 450 x 2048 15.9 / 18.0, 610 x
+    2048 29.2 / 23.4), and for the same reason not too few (2048 x 128 x 2048 13.8 / 11.5).
+    What adds to the residual stream (``residual``) with a shorter K while a tile of 128 x 128 finds a unit of its own, since the library reads
+    and writes the stream in a slower way: called behind one another 1295 x 1024 x 1024 10.8 / 11.0, 1295 x 1600 x 1600 18.2 / 16.0, 1600 rows 19.0 /
+    17.6, 2048 rows 20.1 / 20.9, 2048 x 2048 x 1984 25.1 / 23.2, but two microseconds better inside a step: prompts of GPT-2 xl of 1,296 to 1,600
+    tokens 8,650 / 8,660, 9,214 / 9,166 and 9,286 / 9,293, of 1,800 9,705 / 9,753, of 2,048 10,427 / 10,559.  From K = 2,048 on it has no more tiles than
+    others (1295 x 2048 x 2048 21.8 / 19.6, 2,048 rows 25.7 / 23.8).
+    The fused projection of a mixer (``scatters``) up to two tiles of 64 x 128 a unit whatever K: the library cannot scatter keys and values, and the
+    copy behind its product costs 6 to 8 us (1295 x 3072 x 1024 16.3 / 23.2, 768 x 4800 x 1600 21.7 / 28.3, 640 x 6144 x 2048 25.9 / 30.5, 768 x 5120 x
+    3072 36.7 / 38.8, 640 x 6144 x 4096 48.5 / 47.3; beyond it 1024 x 4800 x 1600 31.0 / 29.8, 768 x 6144 x 2048 36.2 / 32.8).  Those are heads of 64
+    and 128; of 80 and 48, whose keys and values the kernel stores call by call, 768 x 4800 x 1600 takes 24.8 / 28.2, 640 x 3840 x 1280
+    19.6 / 18.9, 1024 x 3840 x 1280 21.5 / 21.9, 768 x 4608 x 1536 24.6 / 25.1.  A K below 512 (not measured) and columns that are no multiple of
+    eight (not stored in whole rows) are the library's.  Rows count in whole tiles of 64 and 128 only: steps of one class (``engine.step.token_capacity``)
+    choose alike."""
     if deep_form_rows(m, k, lda, n, sliced, scatters):
         return True
     if m <= 64 or k % 64 or n % 8 or k < OWN_SHORT_K or m * lda * 2 >= (1 << 32) or n * k * 2 >= (1 << 32):
@@ -950,7 +956,7 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False):
     tiles = lambda rows, columns: ((m + rows - 1) // rows) * ((n + columns - 1) // columns)
     if tiles(64, 64) < OWN_LEAST_TILES:
         return False
-    if k >= OWN_LONG_K:
+    if k >= OWN_LONG_K and not scatters:
         return tiles(64, 128) <= OWN_LONG_TILES
     return tiles(64, 128) <= (OWN_SCATTER_TILES if scatters else OWN_TILES) or (residual and tiles(128, 128) <= OWN_RESIDUAL_TILES)
 

@@ -130,7 +130,7 @@ def stream_product_splits(step, a, weight):
     """Into how many slices of K a product that feeds the residual stream is cut (see
     ``ResidualStream.add_product``)."""
     rows, width = a.shape[0], weight.shape[0]
-    if step.dtype_is_bf16 and rows > 64:       # a short prompt or chunk: the tile kernel's deep forms
+    if step.dtype_is_bf16 and rows > 64:       # a short prompt or chunk: the tile kernel's, whose slices may stay pending
         return K.deep_split_count(rows, width, a.shape[1], compute_units(a.device)) \
             if not isinstance(a, K.Chunked) and a.stride(1) == 1 and \
             K.deep_form_rows(rows, a.shape[1], a.stride(0), width, sliced=True) else 1

@@ -175,6 +175,25 @@ def test_products_of_short_prompts_and_how_they_cut_k():
                 assert 1 <= splits <= 4 and (splits == 1 or (k // 64) // splits >= 4)
 
 
+def test_which_products_leave_the_library_whatever_their_k():
+    """A fused projection that scatters keys and values keeps its line where K is long, what adds to the stream does not."""
+    from burn_transformers_amd.kernels.library import own_tiles
+    for k in (1024, 1984, 2048, 4096):
+        assert own_tiles(640, 6144, k, k, scatters=True) and not own_tiles(768, 6144, k, k, scatters=True)     # 480 and 576 tiles of 64 x 128
+    assert own_tiles(2048, 2048, 1984, 1984, residual=True) and not own_tiles(2048, 2048, 2048, 2048, residual=True)
+    assert own_tiles(512, 2048, 2048, 2048) and not own_tiles(513, 2048, 2048, 2048)
+
+
+def test_products_leave_the_library_alike_in_all_steps_of_a_class():
+    """One launch list serves all steps of a class: whose product it is may not depend on which of them came first."""
+    from burn_transformers_amd.engine.step import token_capacity
+    from burn_transformers_amd.kernels.library import own_tiles
+    for n, k in ((768, 768), (1600, 1600), (3072, 1024), (4800, 1600), (6144, 2048), (1024, 4096)):
+        for options in ({}, {"sliced": True}, {"scatters": True}, {"residual": True}):
+            for rows in range(65, 1700):
+                assert own_tiles(rows, n, k, k, **options) == own_tiles(token_capacity(rows), n, k, k, **options)
+
+
 def test_float_products_are_cut_alike_in_all_steps_of_a_class(monkeypatch):
     """One launch list serves all steps of a class, so the slices of a float32 product may not depend on which of them came first."""
     from types import SimpleNamespace
