@@ -149,7 +149,7 @@ def test_whether_a_graph_pays_is_decided_by_the_median_of_the_measured_steps():
 
 def test_products_of_short_prompts_and_how_they_cut_k():
     """``deep_form_rows`` / ``deep_split_count``: 65 to 256 rows with K a multiple of 64 go to the
-    tile kernel's deep forms, up to 512 where slices of K may stay pending and up to 384 where keys and
+    tile kernel, up to 512 where slices of K may stay pending and up to 384 where keys and
     values are scattered into the cache (the vendor's library would need a copy behind it); a residual-writing one
     cuts K so that every work-group has a compute unit, or at most two share one, into at most four
     slices of at least four tiles of K."""

@@ -18,9 +18,10 @@ def operands(m, n, k, dtype, seed):
     return a, w, bias, a.double() @ w.double().t()
 
 
-# one to five tiles of K (forms have two to four stages); rows and columns on both sides of whole tiles; columns that are no
+# one to seven tiles of K (forms have two to four stages) and so many that 64 x 64 takes eight and 64 x 128 six, whole and in slices; rows and columns on both sides of whole tiles; columns that are no
 # multiple of eight or four, which leave the epilogue's whole rows for single values
-@pytest.mark.parametrize("m,n,tiles", [(65, 64, 1), (128, 256, 2), (130, 136, 3), (257, 260, 4), (300, 129, 5), (70, 514, 7)])
+@pytest.mark.parametrize("m,n,tiles", [(65, 64, 1), (128, 256, 2), (130, 136, 3), (257, 260, 4), (300, 129, 5), (70, 514, 7),
+                                       (70, 130, 49), (130, 200, 150)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_epilogues_of_every_form(dtype, m, n, tiles):
     k = tiles * (64 if dtype == torch.bfloat16 else 32)
@@ -53,9 +54,8 @@ def test_epilogues_of_every_form(dtype, m, n, tiles):
 # heads whose columns fill a wave's blocks (64, 128), that leave them (48, 80); sequences that start anywhere in a tile
 @pytest.mark.parametrize("heads,kv_heads,hd", [(4, 4, 64), (3, 1, 128), (4, 2, 32), (5, 5, 48), (2, 2, 80)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_scattered_keys_and_values(dtype, heads, kv_heads, hd):
+def test_scattered_keys_and_values(dtype, heads, kv_heads, hd, k=128):
     totals, counts = [70, 3, 129, 64, 200], [69, 3, 1, 64, 130]
-    k = 128
     n_q, n_kv, m = heads * hd, kv_heads * hd, sum(counts)
     a, w, bias, want = operands(m, n_q + 2 * n_kv, k, dtype, hd)
     want = want + bias.double()
@@ -74,6 +74,12 @@ def test_scattered_keys_and_values(dtype, heads, kv_heads, hd):
                 assert torch.equal(after[at:at + total - count], before[at:at + total - count]), form      # older positions stay
                 assert float((after[at + total - count:at + total] - want[row:row + count, first:first + n_kv]).abs().max() / scale) < bound, form
             row, at = row + count, at + total
+
+
+def test_scattered_keys_and_values_behind_a_long_k():
+    """The forms of eight and six stages."""
+    test_scattered_keys_and_values(torch.bfloat16, 4, 4, 64, k=49 * 64)
+    test_scattered_keys_and_values(torch.bfloat16, 5, 5, 48, k=49 * 64)
 
 
 def test_which_products_are_the_tile_kernels():
