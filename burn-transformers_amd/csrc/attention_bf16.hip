@@ -734,7 +734,6 @@ __global__ void __launch_bounds__(SPLIT_THREADS)
 attention_prefill_split_kernel(AttnArgs a) {
   static_assert(2 * PREFILL_WAVES * 64 == 512 && SPLIT_PRODUCERS * 64 == 256,
                 "two 16-byte pieces of a block's keys and two of its values per bringing thread");
-  typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
   extern __shared__ __attribute__((aligned(16))) unsigned char split_lds[];   // [2 turns][2 blocks][SHARED_STAGE]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);

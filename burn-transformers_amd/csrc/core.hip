@@ -629,7 +629,6 @@ kv_store_bf16_kernel(const bf16_t* __restrict__ k_rows, const bf16_t* __restrict
   const int hd = kv.head_dim, width = kv.kv_heads * hd;
   bf16_t* keys = static_cast<bf16_t*>(kv.keys);
   bf16_t* values = static_cast<bf16_t*>(kv.values);
-  typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
   const int pieces = width >> 3;
   for (int q = threadIdx.x; q < n * pieces; q += 256) {
     int i = q / pieces, c = (q - i * pieces) * 8;

@@ -311,7 +311,7 @@ __device__ __forceinline__ void epilogue4(const Epilogue& e, int N, int m, int n
 // % 32 the row): through LDS, so that memory sees whole rows' 16-byte pieces instead of 32 rows' 8 bytes with every
 // instruction, and with all that a step needs from memory asked for together.  One call of epilogue4 after the other took 5 us
 // (stored rows) to 12 us (the residual stream, whose old values every call waited for) of a product of 128 x 128 tiles.
-// `scratch`: TILE_SCRATCH bytes of this wave's own; every wave has passed a barrier behind its last read of it.
+// `scratch`: tile_scratch_bytes<TM, TN>() of this wave's own; every wave has passed a barrier behind its last read of it.
 template <int TM, int TN>
 constexpr int tile_scratch_bytes() { return TM * 32 * (TN * 32 * 4 + 16); }
 

@@ -455,7 +455,6 @@ __global__ void __launch_bounds__(256) gated_experts_kernel(GatedExpertsCall c) 
 // The same for units without a gate whose columns can be taken 16 bytes at a time: no piece lies in two experts.
 template <typename T>
 __global__ void __launch_bounds__(256) plain_experts_kernel(GatedExpertsCall c) {
-  typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
   constexpr int PER = 16 / sizeof(T);
   const int t = blockIdx.x, routed = c.experts * c.ff / PER, pieces = c.hidden_cols / PER;
   const int4v* up = reinterpret_cast<const int4v*>(static_cast<const T*>(c.gu) + (int64_t)t * c.ld_gu);
@@ -850,7 +849,6 @@ struct WeighExpertsCall {
 template <typename T>
 __global__ void __launch_bounds__(256) weigh_experts_kernel(WeighExpertsCall w) {
   __shared__ float score[ROUTE_MAX_EXPERTS], choice[ROUTE_MAX_EXPERTS];
-  typedef __attribute__((__vector_size__(4 * sizeof(int)))) int int4v;
   constexpr int PER = 16 / sizeof(T);
   const RouteCall& c = w.route;
   const int t = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;

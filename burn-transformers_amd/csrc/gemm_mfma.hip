@@ -27,10 +27,9 @@
 #define TILE_K 64            // bfloat16 values in a 128-byte row of an LDS tile
 
 // BM x BN tiles of 128-byte rows (64 bfloat16 or 32 float K values), WM x WN waves, each wave
-// (BM / WM) x (BN / WN) as 32-wide MFMA blocks; LDS holds two stages.  PF register sets hold tiles on their way
-// from memory to LDS: with one, the loads of tile i + 1 fly while tile i is multiplied; with
-// two, tile i + 1 waits in registers and the loads of tile i + 2 fly.
-template <typename T, int BM, int BN, int WM, int WN, int PF>
+// (BM / WM) x (BN / WN) as 32-wide MFMA blocks; LDS holds two stages, registers the tile
+// on its way from memory to LDS: the loads of tile i + 1 fly while tile i is multiplied.
+template <typename T, int BM, int BN, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64)
 gemm_tile_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
                  int K, Epilogue epi, int tiles_m, int tiles_n) {
@@ -58,8 +57,8 @@ gemm_tile_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, 
   // the registers of the larger tiles.
   const int c = tid & 7, r0 = tid >> 3;
   constexpr int A_CHUNKS = BM / ROW_STEP;
-  int4v regs[PF][PER_THREAD];
-  auto load_tile = [&](int set, int kt) {
+  int4v regs[PER_THREAD];
+  auto load_tile = [&](int kt) {
     // a chunk beyond K (a multiple of the chunk) reads the row's last chunk and is cleared when stored
     int k = kt * ROW_K + c * ELEMS;
     int kc = k < K ? k : K - ELEMS;
@@ -74,15 +73,15 @@ gemm_tile_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, 
         int n = n_base + row - BM;
         src = W + (int64_t)(n < N ? n : N - 1) * K;
       }
-      regs[set][i] = *reinterpret_cast<const int4v*>(src + kc);
+      regs[i] = *reinterpret_cast<const int4v*>(src + kc);
     }
   };
-  auto store_tile = [&](int set, int kt, int stage) {
+  auto store_tile = [&](int kt, int stage) {
     int keep = kt * ROW_K + c * ELEMS < K ? -1 : 0;
     unsigned char* base = lds + stage * (ROWS * TILE_ROW_BYTES);
 #pragma unroll
     for (int i = 0; i < PER_THREAD; ++i)
-      *reinterpret_cast<int4v*>(base + swizzled(r0 + ROW_STEP * i, c)) = regs[set][i] & keep;
+      *reinterpret_cast<int4v*>(base + swizzled(r0 + ROW_STEP * i, c)) = regs[i] & keep;
   };
 
   floatx16 acc[TN][TM];
@@ -119,39 +118,17 @@ gemm_tile_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, 
   };
 
   const int count = kt_end - kt_begin;
-  if (PF == 1) {
-    // tile i is multiplied from stage i % 2 while the loads of tile i + 1 fly into the registers
-    if (count > 0) {
-      load_tile(0, kt_begin);
-      store_tile(0, kt_begin, 0);
-    }
+  // tile i is multiplied from stage i % 2 while the loads of tile i + 1 fly into the registers
+  if (count > 0) {
+    load_tile(kt_begin);
+    store_tile(kt_begin, 0);
+  }
+  __syncthreads();
+  for (int i = 0; i < count; ++i) {
+    if (i + 1 < count) load_tile(kt_begin + i + 1);
+    multiply(i & 1);
+    if (i + 1 < count) store_tile(kt_begin + i + 1, (i + 1) & 1);
     __syncthreads();
-    for (int i = 0; i < count; ++i) {
-      if (i + 1 < count) load_tile(0, kt_begin + i + 1);
-      multiply(i & 1);
-      if (i + 1 < count) store_tile(0, kt_begin + i + 1, (i + 1) & 1);
-      __syncthreads();
-    }
-  } else {
-    // tile i is multiplied from stage i % 2 while tile i + 1 sits in register set (i + 1) % 2 and
-    // the loads of tile i + 2 fly into the other set
-    if (count > 0) {
-      load_tile(0, kt_begin);
-      if (count > 1) load_tile(PF - 1, kt_begin + 1);
-      store_tile(0, kt_begin, 0);
-    }
-    __syncthreads();
-    for (int i = 0; i < count; i += 2) {
-      if (i + 2 < count) load_tile(0, kt_begin + i + 2);
-      multiply(0);
-      if (i + 1 < count) store_tile(PF - 1, kt_begin + i + 1, 1);
-      __syncthreads();
-      if (i + 1 >= count) break;
-      if (i + 3 < count) load_tile(PF - 1, kt_begin + i + 3);
-      multiply(1);
-      if (i + 2 < count) store_tile(0, kt_begin + i + 2, 0);
-      __syncthreads();
-    }
   }
 
   // lane holds D[i][j]: i = 8 * (r / 4) + 4 * g + r % 4 (column n), j = lane % 32 (row m)
@@ -680,12 +657,12 @@ static int check_operands(const char* who, int elems, const void* A, int64_t lda
   return BT_OK;
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int PF>
+template <typename T, int BM, int BN, int WM, int WN>
 static void launch_tile(hipStream_t stream, const T* A, int64_t lda, const T* W, int M, int N, int K,
                         const Epilogue& epi, int splits) {
   int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   size_t lds = (size_t)2 * (BM + BN) * TILE_ROW_BYTES;
-  auto kernel = gemm_tile_kernel<T, BM, BN, WM, WN, PF>;
+  auto kernel = gemm_tile_kernel<T, BM, BN, WM, WN>;
   if (lds > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n, 1, splits), dim3(WM * WN * 64), lds, stream, A, lda, W, M, N,
@@ -759,7 +736,7 @@ static int launch_form(hipStream_t s, int variant, const bf16_t* a, int64_t lda,
 static int launch_form(hipStream_t s, int variant, const float* a, int64_t lda, const float* w, int M, int N, int K,
                        const Epilogue& epi, int splits) {
   switch (variant) {
-    case 4: return launch_pipe<64, 64, 2, 2, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 4:                // (three stages are for units that share their LDS: no rule wants them here)
     case 5: return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
     case 6: return launch_parts_form<128, 64, 4, 2>(s, a, lda, w, M, N, K, epi, splits);
     case 7: return launch_parts_form<128, 128, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
@@ -788,7 +765,7 @@ static int tile_form(int M, int N, int K, int splits) {
 
 // dtype: 0 float, 1 bfloat16 (the codes of every entry point that takes both).
 // variant: 0 = the fastest form the operands allow; 1 = the general form; 2 .. 7 = launch_form's (asked for by tests and
-// measurements; a form that cannot take the operands is refused; float has the general form and 4 .. 7).
+// measurements; a form that cannot take the operands is refused; float has the general form, 5 (4 is the same), 6 and 7).
 // Float products take the tiles of 64 x 64 or the forms on parts wherever K is a multiple of 32 (the template's tile of 128 x 128
 // takes a compute unit 2.4 us for 32 values of K and leaves most units idle where there are few tiles).  While the tiles of
 // 64 x 64 have a unit each, they win: 0.65 us for 32 values of K where a tile of 128 x 64 on parts takes 0.73 (65 x 768 x 3072 62
@@ -815,7 +792,7 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
       variant = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits <= 256 ? 5 : 2 * rounds <= 3 * wide_rounds ? 6 : 7;
     }
     if (variant >= 4) return launch_form(s, variant, a, lda, w, M, N, K, *epi, splits);
-    launch_tile<float, 128, 128, 2, 2, 1>(s, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits);
+    launch_tile<float, 128, 128, 2, 2>(s, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits);
     return bt_check_launch("gemm_tile");
   }
   const bf16_t* a = (const bf16_t*)A;
@@ -827,7 +804,7 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
     if (!whole_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 64 and operands below 4 GiB", K);
     return launch_form(s, variant, a, lda, w, M, N, K, *epi, splits);
   }
-  launch_tile<bf16_t, 128, 128, 2, 2, 1>(s, a, lda, w, M, N, K, *epi, splits);
+  launch_tile<bf16_t, 128, 128, 2, 2>(s, a, lda, w, M, N, K, *epi, splits);
   return bt_check_launch("gemm_tile");
 }
 

@@ -63,17 +63,6 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int NEWER, int LOADS>
-__device__ __forceinline__ void wait_for_all_but(int newer) {
-  // waits until at most `newer` tiles' loads (LOADS instructions each) of this wave are in flight
-  if constexpr (NEWER == 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (newer >= NEWER) wait_vmcnt<NEWER * LOADS>();
-    else wait_for_all_but<NEWER - 1, LOADS>(newer);
-  }
-}
-
 // A tile's product over K: operands go from memory straight into LDS (128-byte rows, BM of A, then BN of W, swizzled on the
 // memory side) and from there into the matrix units, on WM x WN waves, each with TM x TN blocks of 32 x 32.
 //   stages   STAGES tiles of 128 bytes of K lie in LDS or are on their way; one barrier a tile
