@@ -883,7 +883,7 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
         elif dtype == FLOAT32:
             impl = "tile"
         elif own_tiles(m, n, k, a.stride(0), sliced=splits > 1, scatters=epilogue.mode == EPI_QKV,
-                       residual=epilogue.mode == EPI_RESIDUAL):
+                       residual=epilogue.mode == EPI_RESIDUAL, gelu=epilogue.mode == EPI_ACT and _library_takes(epilogue)):
             impl = "tile"
         else:
             impl = "library" if splits == 1 and _library_takes(epilogue) and library_products() \
@@ -915,7 +915,7 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
 DEEP_FORM_ROWS = 256          # most rows of a bfloat16 product that the tile kernel takes whatever its other sizes ...
 DEEP_FORM_SLICED_ROWS = 512   # ... and of one that leaves partial sums of slices of K pending ...
 DEEP_FORM_SCATTER_ROWS = 384  # ... and of one that scatters keys and values into the cache
-OWN_TILES = 256               # beyond: most tiles of 64 x 128 of a product that the tile kernel takes ...
+OWN_TILES = 256               # beyond: most tiles of 64 x 128 of a product that the tile kernel takes (with a GELU, of 64 x 64) ...
 OWN_LONG_K, OWN_LONG_TILES = 2048, 128    # ... from this K on, and ...
 OWN_SCATTER_TILES = 512       # ... of one that scatters keys and values, whatever its K; most tiles of 128 x 128 of one ...
 OWN_RESIDUAL_TILES = 256      # ... with a shorter K that adds to the residual stream; the fewest tiles of 64 x 64 and the shortest K
@@ -930,7 +930,7 @@ def deep_form_rows(m, k, lda, n, sliced=False, scatters=False):
     return 64 < m <= limit and k % 64 == 0 and m * lda * 2 < (1 << 32) and n * k * 2 < (1 << 32)
 
 
-def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False):
+def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=False):
     """Whether a bfloat16 product of more than 64 rows is the tile kernel's; the others are the vendor's library's.  By its rows
     alone (``deep_form_rows``), or while a tile of 64 x 128 of it finds a compute unit of its own: measured (us, tile kernel /
     library) at K = 1,024 610 x 3072 9.4 / 10.4, 1024 x 2048 9.3 / 10.6, 1500 x 1024 9.1 / 9.9, with more tiles 610 x 4096 12.5 / 12.0, 768 x
@@ -946,7 +946,10 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False):
     copy behind its product costs 6 to 8 us (1295 x 3072 x 1024 16.3 / 23.2, 768 x 4800 x 1600 21.7 / 28.3, 640 x 6144 x 2048 25.9 / 30.5, 768 x 5120 x
     3072 36.7 / 38.8, 640 x 6144 x 4096 48.5 / 47.3; beyond it 1024 x 4800 x 1600 31.0 / 29.8, 768 x 6144 x 2048 36.2 / 32.8).  Those are heads of 64
     and 128; of 80 and 48, whose keys and values the kernel stores call by call, 768 x 4800 x 1600 takes 24.8 / 28.2, 640 x 3840 x 1280
-    19.6 / 18.9, 1024 x 3840 x 1280 21.5 / 21.9, 768 x 4608 x 1536 24.6 / 25.1.  A K below 512 (not measured) and columns that are no multiple of
+    19.6 / 18.9, 1024 x 3840 x 1280 21.5 / 21.9, 768 x 4608 x 1536 24.6 / 25.1.
+    With the GELU that the library has too (``gelu``) while a tile of 64 x 64 finds a unit of its own: a lane's 32 values of a tile of 64 x 128, of which
+    every one is some forty instructions, show (300 x 3072 x 768 8.1 / 8.3, 640 x 1600 x 1600 10.5 / 12.2; beyond it 400 x 3072 x 768 11.6 / 10.0, 300 x 4096 x
+    1024 12.7 / 10.7, 1600 x 1024 x 1024 12.9 / 11.1; prompts of 400 tokens of GPT-2 small 713 / 702, of medium 1,633 / 1,610).  A K below 512 (not measured) and columns that are no multiple of
     eight (not stored in whole rows) are the library's.  Rows count in whole tiles of 64 and 128 only: steps of one class (``engine.step.token_capacity``)
     choose alike."""
     if deep_form_rows(m, k, lda, n, sliced, scatters):
@@ -954,7 +957,7 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False):
     if m <= 64 or k % 64 or n % 8 or k < OWN_SHORT_K or m * lda * 2 >= (1 << 32) or n * k * 2 >= (1 << 32):
         return False
     tiles = lambda rows, columns: ((m + rows - 1) // rows) * ((n + columns - 1) // columns)
-    if tiles(64, 64) < OWN_LEAST_TILES:
+    if tiles(64, 64) < OWN_LEAST_TILES or (gelu and tiles(64, 64) > OWN_TILES):
         return False
     if k >= OWN_LONG_K and not scatters:
         return tiles(64, 128) <= OWN_LONG_TILES

@@ -182,6 +182,9 @@ def test_which_products_leave_the_library_whatever_their_k():
         assert own_tiles(640, 6144, k, k, scatters=True) and not own_tiles(768, 6144, k, k, scatters=True)     # 480 and 576 tiles of 64 x 128
     assert own_tiles(2048, 2048, 1984, 1984, residual=True) and not own_tiles(2048, 2048, 2048, 2048, residual=True)
     assert own_tiles(512, 2048, 2048, 2048) and not own_tiles(513, 2048, 2048, 2048)
+    # the activation that the library has too: while tiles of 64 x 64 have a unit each, or by the rows alone
+    assert own_tiles(300, 3072, 768, 768, gelu=True) and own_tiles(400, 3072, 768, 768) and not own_tiles(400, 3072, 768, 768, gelu=True)
+    assert own_tiles(256, 6400, 1600, 1600, gelu=True) and not own_tiles(257, 6400, 1600, 1600, gelu=True)
 
 
 def test_products_leave_the_library_alike_in_all_steps_of_a_class():
@@ -189,7 +192,7 @@ def test_products_leave_the_library_alike_in_all_steps_of_a_class():
     from burn_transformers_amd.engine.step import token_capacity
     from burn_transformers_amd.kernels.library import own_tiles
     for n, k in ((768, 768), (1600, 1600), (3072, 1024), (4800, 1600), (6144, 2048), (1024, 4096)):
-        for options in ({}, {"sliced": True}, {"scatters": True}, {"residual": True}):
+        for options in ({}, {"sliced": True}, {"scatters": True}, {"residual": True}, {"gelu": True}):
             for rows in range(65, 1700):
                 assert own_tiles(rows, n, k, k, **options) == own_tiles(token_capacity(rows), n, k, k, **options)
 
