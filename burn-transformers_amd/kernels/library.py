@@ -970,13 +970,13 @@ def deep_split_count(rows, columns, k, units=256):
     of 64 x 64 of one slice) a compute unit of its own, or, where even two slices are too many for
     that, as many as leave at most two work-groups to a unit; at most four (the norm behind the
     product reads them all), each at least four tiles of K long.  Measured at width 1,600 on 256
-    units (us for 1600 x 1600 and 1600 x 6400, slices 2 / 3 / 4): 128 rows 7.1 / 6.3 / 5.9 and 18.9 /
-    14.5 / 12.1; 192 rows 7.3 / 6.5 / 7.2 and 18.8 / 14.7 / 18.8; 256 rows 7.4 / 7.9 / 7.5 and 19.2 /
-    22.4 / 18.8; 384 rows 9.3 / 8.4 / 10.9 and 29.3 / 23.1 / 26.5; 512 rows 9.5 / 12.1 / 12.1 and 30.7 /
-    32.2 / 31.0 (the vendor's library: 11.1 to 12.2 and 18.3 to 32.4).  Measured and not taken: tiles
+    units with weights from memory (us for 1600 x 1600 and 1600 x 6400, slices 1 / 2 / 3 / 4; the vendor's library): 128 rows 8.9 / 6.9 /
+    6.3 / 6.1 (11.1) and 33.0 / 19.7 / 14.8 / 12.6 (18.1); 192 rows 8.9 / 7.0 / 6.5 / 7.8 (11.3) and 32.6 / 19.7 / 15.1 / 17.9 (23.6); 256
+    rows 9.0 / 7.2 / 8.5 / 8.1 (11.5) and 32.5 / 19.9 / 21.4 / 18.1 (23.6); 384 rows 9.3 / 9.7 / 9.0 / 9.8 (11.9) and 32.2 / 28.0 / 21.7 /
+    22.0 (31.5); 512 rows 9.6 / 10.2 / 11.4 / 11.0 (12.2) and 32.5 / 28.7 / 26.5 / 22.4 (31.2).  Measured and not taken, on the loop before this one: tiles
     of 128 x 128 in four slices for 1600 x 6400 at 512 rows (25.2 us alone against 30.3, but 29.5 in
     the step, where the norm behind it also reads four slices instead of two), and slices beyond 512
-    rows (640 rows: 10.1 and 30.7 against the library's 12.2 and 32.7, which the norm's second
+    rows (640 rows, two slices: 10.7 and 29.6 against the library's 12.3 and 31.7, which the norm's second
     reading of two slices takes back)."""
     if not deep_form_rows(rows, k, k, columns, sliced=True):
         return 1
