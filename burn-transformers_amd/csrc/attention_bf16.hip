@@ -276,8 +276,7 @@ __device__ __forceinline__ void attend_tile(const TileOperands& tile, int kb, in
 #pragma unroll
     for (int nq = 0; nq < NQ; ++nq) {
       float top = own[nq];
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      top = across<32>(across<16>(top, LaneMax()), LaneMax());
       float alpha;
       const float delta = raise_maximum(m[nq], top, alpha);
       l[nq] *= alpha;
@@ -445,8 +444,7 @@ attention_prefill_kernel(AttnArgs a) {
 #pragma unroll
   for (int nq = 0; nq < PREFILL_NQ; ++nq) {
     float total = l[nq];
-    total += __shfl_xor(total, 16, 64);
-    total += __shfl_xor(total, 32, 64);
+    total = across<32>(across<16>(total, LaneSum()), LaneSum());
     total += bt_sink_term_pow2(a.sink, head, m[nq]);
     float inv = FORM == 2 ? 1.0f : total > 0.f ? 1.0f / total : 0.f;
     if (qpos[nq] < 0) continue;
@@ -552,8 +550,7 @@ __device__ __forceinline__ void attend_block(const Operands& blk, int kb, int va
 #pragma unroll
     for (int nq = 0; nq < NQ; ++nq) {
       float top = own[nq];
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      top = across<32>(across<16>(top, LaneMax()), LaneMax());
       float alpha;
       const float delta = raise_maximum(m[nq], top, alpha);
 #pragma unroll
@@ -1191,8 +1188,7 @@ attention_decode_kernel(AttnArgs a) {
     attend(current, walk.at(place));
   }
   float total = l[0];
-  total += __shfl_xor(total, 16, 64);
-  total += __shfl_xor(total, 32, 64);
+  total = across<32>(across<16>(total, LaneSum()), LaneSum());
   // Only the waves that had a tile leave a share (a short run keeps one or two busy): a share each of `group` rows is
   // written, read and weighed again by every element of the output.  With every wave's share (us, 16 heads of 128 on one, eight
   // sequences, in eight runs) 30 keys 11.6, 100 11.5, 1,000 12.5; so 8.0, 8.1, 10.3.  8 heads on 2: 1,000 keys 10.0 -> 9.7.

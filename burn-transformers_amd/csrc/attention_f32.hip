@@ -198,8 +198,7 @@ attention_f32_mfma_kernel(AttnArgs a) {
       float top = -INFINITY;
 #pragma unroll
       for (int t = 0; t < 4; ++t) top = fmaxf(top, fmaxf(fmaxf(s[t][0], s[t][1]), fmaxf(s[t][2], s[t][3])));
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      top = across<32>(across<16>(top, LaneMax()), LaneMax());
       const float new_max = fmaxf(run_max, top * c2);          // in powers of two
       // nothing seen so far, this block included: everything stays at its start
       const float rescale = new_max == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(run_max - new_max);   // 2^-inf = 0 at the first block seen
@@ -232,8 +231,7 @@ attention_f32_mfma_kernel(AttnArgs a) {
     }
   }
   float total = run_sum;
-  total += __shfl_xor(total, 16, 64);
-  total += __shfl_xor(total, 32, 64);
+  total = across<32>(across<16>(total, LaneSum()), LaneSum());
   total += bt_sink_term_pow2(a.sink, head, run_max);        // (the maximum is the same in a query's four lanes)
   if (exists) {
     const int64_t tok = off + q0 + mine;

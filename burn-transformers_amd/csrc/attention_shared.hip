@@ -174,8 +174,7 @@ attention_shared_kernel(AttnArgs a, int tiles_max) {
       float top = -INFINITY;
 #pragma unroll
       for (int t = 0; t < 4; ++t) top = fmaxf(top, fmaxf(fmaxf(x[t][0], x[t][1]), fmaxf(x[t][2], x[t][3])));
-      top = fmaxf(top, __shfl_xor(top, 16, 64));
-      top = fmaxf(top, __shfl_xor(top, 32, 64));
+      top = across<32>(across<16>(top, LaneMax()), LaneMax());
       const float next = fmaxf(m, top * c);
       const float alpha = next == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - next);      // (2^-inf = 0 before the first key seen)
       const float use = next == -INFINITY ? 0.f : next;
@@ -228,8 +227,7 @@ attention_shared_kernel(AttnArgs a, int tiles_max) {
     }
   }
   if (weighs) {
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = across<32>(across<16>(l, LaneSum()), LaneSum());
     if (g == 0) {
       s_sum[sq][sh][i16] = l;
       if (sh == 0) s_max[sq][i16] = m;

@@ -89,36 +89,101 @@ __host__ __device__ __forceinline__ int64_t activation_offset(int rows, int64_t 
   return rows > 0 ? ((int64_t)(column / CHUNK) * rows + row) * CHUNK + column % CHUNK : (int64_t)row * pitch + column;
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// Reductions over a wave without LDS: v_permlane32_swap and v_permlane16_swap bring the lanes 32 and 16 apart together, rotations
+// inside rows of sixteen those 8 and 4 apart, quad permutations the last two.  Six steps of one or two vector instructions, where a
+// shuffle through LDS (__shfl_xor) has every step wait some 50 ns for its lane: a decode step's kernels have one to four reductions
+// in a row on their critical path.  (Decode steps, us: GPT-2 small, one sequence, 337 -> 319, xl, eight sequences, 2,068 -> 2,019.)  The pairs and their order are those of a butterfly from 32 down to 1, so the sums are the same
+// bit for bit.  (The rotations by 8 and 4 meet lane ^ 8 and lane ^ 4 only because the values are alike by then in the lanes
+// further apart.)
+template <int APART>      // 32 or 16: in every lane the values of its pair, the one of the lower lanes first
+__device__ __forceinline__ void lane_pair(int v, int& low, int& high) {
+  static_assert(APART == 32 || APART == 16, "lanes of the two halves, or of neighbouring rows of sixteen");
+  if constexpr (APART == 32) {
+    const auto both = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    low = both[0];
+    high = both[1];
+  } else {
+    const auto both = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    low = both[0];
+    high = both[1];
+  }
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+template <int CONTROL>
+__device__ __forceinline__ int lane_moved(int v) { return __builtin_amdgcn_update_dpp(0, v, CONTROL, 0xf, 0xf, true); }
+template <int CONTROL>
+__device__ __forceinline__ float lane_moved(float v) {
+  return __builtin_bit_cast(float, lane_moved<CONTROL>(__builtin_bit_cast(int, v)));
 }
+struct LaneSum {
+  __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct LaneMax {
+  __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+template <int APART, typename F>
+__device__ __forceinline__ float across(float v, F f) {       // with the lane 32 or 16 away
+  int low, high;
+  lane_pair<APART>(__builtin_bit_cast(int, v), low, high);
+  return f(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
+}
+template <typename F>
+__device__ __forceinline__ float row_reduce(float v, F f) {   // over the sixteen lanes of a row
+  v = f(v, lane_moved<0x128>(v));                             // row_ror:8
+  v = f(v, lane_moved<0x124>(v));                             // row_ror:4
+  v = f(v, lane_moved<0x4e>(v));                              // quad_perm:[2,3,0,1]
+  return f(v, lane_moved<0xb1>(v));                           // quad_perm:[1,0,3,2]
+}
+// The value of lane ^ 2^STEP, steps taken from the highest down (see above for steps 3 and 2).
+template <int STEP>
+__device__ __forceinline__ int lane_other(int v) {
+  if constexpr (STEP >= 4) {
+    int low, high;
+    lane_pair<1 << STEP>(v, low, high);
+    return threadIdx.x & (1 << STEP) ? low : high;
+  } else {
+    return lane_moved<STEP == 3 ? 0x128 : STEP == 2 ? 0x124 : STEP == 1 ? 0x4e : 0xb1>(v);
+  }
+}
+// The best (value, index) of a wave; among equal values the lowest index.  Every lane gets it.
+template <int STEP = 5>
+__device__ __forceinline__ void wave_best(float& value, int& index) {
+  const float other = __builtin_bit_cast(float, lane_other<STEP>(__builtin_bit_cast(int, value)));
+  const int other_index = lane_other<STEP>(index);
+  if (other > value || (other == value && other_index < index)) { value = other; index = other_index; }
+  if constexpr (STEP > 0) wave_best<STEP - 1>(value, index);
+}
+__device__ __forceinline__ float wave_sum(float v) { return row_reduce(across<16>(across<32>(v, LaneSum()), LaneSum()), LaneSum()); }
+__device__ __forceinline__ float wave_max(float v) { return row_reduce(across<16>(across<32>(v, LaneMax()), LaneMax()), LaneMax()); }
 
-// Block-wide reductions for blocks of up to 1024 threads; `scratch` holds 32 floats of LDS.
-// Every thread gets the result.  Safe to call repeatedly with the same scratch.
-__device__ __forceinline__ float block_sum(float v, float* scratch) {
-  v = wave_sum(v);
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, waves = (blockDim.x + 63) >> 6;
+// Block-wide reductions for blocks of up to 1024 threads; `scratch` holds 32 floats of LDS, on 16 bytes.
+// Every thread gets the result.  Safe to call repeatedly with the same scratch.  THREADS: the block's size where it is a
+// constant (the waves' shares are then read together and not in a loop that waits for each); 0 otherwise.
+template <int THREADS, typename F>
+__device__ __forceinline__ float block_join(float v, float* scratch, float start, F f) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  float total = 0.f;
-  for (int w = 0; w < waves; ++w) total += scratch[w];
+  float total = start;
+  if constexpr (THREADS > 0) {
+    constexpr int WAVES = THREADS / 64;
+    static_assert(THREADS % 256 == 0, "whole quads of waves");
+    floatx4 part[WAVES / 4];
+#pragma unroll
+    for (int q = 0; q < WAVES / 4; ++q) part[q] = reinterpret_cast<const floatx4*>(scratch)[q];
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) total = f(total, part[w >> 2][w & 3]);
+  } else {
+    const int waves = (blockDim.x + 63) >> 6;
+    for (int w = 0; w < waves; ++w) total = f(total, scratch[w]);
+  }
   return total;
 }
+template <int THREADS = 0>
+__device__ __forceinline__ float block_sum(float v, float* scratch) {
+  return block_join<THREADS>(wave_sum(v), scratch, 0.f, LaneSum());
+}
+template <int THREADS = 0>
 __device__ __forceinline__ float block_max(float v, float* scratch) {
-  v = wave_max(v);
-  int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, waves = (blockDim.x + 63) >> 6;
-  __syncthreads();
-  if (lane == 0) scratch[wave] = v;
-  __syncthreads();
-  float top = scratch[0];
-  for (int w = 1; w < waves; ++w) top = fmaxf(top, scratch[w]);
-  return top;
+  return block_join<THREADS>(wave_max(v), scratch, NAN, LaneMax());
 }

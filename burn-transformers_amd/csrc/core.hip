@@ -124,7 +124,7 @@ add_norm_vec_kernel(float* __restrict__ x, const float* __restrict__ delta, int6
                     const float* __restrict__ bias, const float* __restrict__ gamma,
                     const float* __restrict__ beta, float eps, int kind, T* __restrict__ out,
                     const int* __restrict__ rows, int width, int write_back, int out_rows) {
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   const int r = blockIdx.x;
   const int t = rows ? rows[r] : r;
   const int quads = width >> 2;
@@ -163,7 +163,7 @@ add_norm_vec_kernel(float* __restrict__ x, const float* __restrict__ delta, int6
     }
   }
   if (out == nullptr) return;
-  float total = block_sum(partial, scratch);
+  float total = block_sum<256>(partial, scratch);
   float mean = 0.f, rstd;
   if (kind == 0) {
     mean = total / (float)width;
@@ -175,7 +175,7 @@ add_norm_vec_kernel(float* __restrict__ x, const float* __restrict__ delta, int6
         sq += a0 * a0 + a1 * a1 + a2 * a2 + a3 * a3;
       }
     }
-    float var = block_sum(sq, scratch) / (float)width;
+    float var = block_sum<256>(sq, scratch) / (float)width;
     rstd = 1.0f / sqrtf(var + eps);
   } else {
     rstd = 1.0f / sqrtf(total / (float)width + eps);
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(256)
 attention_plain_kernel(AttnArgs a) {
   __shared__ float qs[PLAIN_MAX_HEAD];
   __shared__ float ps[PLAIN_CHUNK];
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   int t = blockIdx.x, head = blockIdx.y;
   int hd = a.kv.head_dim;
   int group = a.q_heads / a.kv.kv_heads;
@@ -507,7 +507,7 @@ attention_plain_kernel(AttnArgs a) {
       ps[i] = s;
       local_max = fmaxf(local_max, s);
     }
-    float chunk_max = block_max(local_max, scratch);
+    float chunk_max = block_max<256>(local_max, scratch);
     float new_max = a.form == 2 ? 0.f : fmaxf(run_max, chunk_max);
     float rescale = (run_max == -INFINITY) ? 0.f : expf(run_max - new_max);
     float local_sum = 0.f;
@@ -517,7 +517,7 @@ attention_plain_kernel(AttnArgs a) {
       ps[i] = p;
       local_sum += p;
     }
-    float chunk_sum = block_sum(local_sum, scratch);
+    float chunk_sum = block_sum<256>(local_sum, scratch);
     run_sum = run_sum * rescale + chunk_sum;
     run_max = new_max;
     __syncthreads();
@@ -739,7 +739,7 @@ struct SamplePartial {
 __global__ void __launch_bounds__(SAMPLE_THREADS)
 sample_chunks_kernel(const float* __restrict__ logits, int64_t ld, int vocab, int chunk_len, float divisor,
                      SamplePartial* __restrict__ partials) {
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   __shared__ int best_index[SAMPLE_THREADS / 64];
   __shared__ float best_value[SAMPLE_THREADS / 64];
   const int row = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x;
@@ -757,11 +757,7 @@ sample_chunks_kernel(const float* __restrict__ logits, int64_t ld, int vocab, in
 #pragma unroll
   for (int i = 0; i < SAMPLE_PER_THREAD; ++i)
     if (v[i] > top) { top = v[i]; arg = lo + tid + i * SAMPLE_THREADS; }
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(top, o, 64);
-    int oa = __shfl_xor(arg, o, 64);
-    if (ov > top || (ov == top && oa < arg)) { top = ov; arg = oa; }
-  }
+  wave_best(top, arg);
   if ((tid & 63) == 0) { best_value[tid >> 6] = top; best_index[tid >> 6] = arg; }
   __syncthreads();
   top = best_value[0]; arg = best_index[0];
@@ -772,7 +768,7 @@ sample_chunks_kernel(const float* __restrict__ logits, int64_t ld, int vocab, in
 #pragma unroll
     for (int i = 0; i < SAMPLE_PER_THREAD; ++i) mine += expf(v[i] - top);   // exp(-inf) = 0 beyond the chunk
   }
-  float total = block_sum(mine, scratch);
+  float total = block_sum<SAMPLE_THREADS>(mine, scratch);
   if (tid == 0) partials[row * gridDim.x + chunk] = SamplePartial{top, total, arg, 0};
 }
 
@@ -1064,11 +1060,7 @@ select_processed_kernel(ProcessArgs a) {
 #pragma unroll
   for (int i = 0; i < PER; ++i)
     if (z[i] > top) { top = z[i]; arg = tid + i * SELECT_THREADS; }   // rising indices: `>` keeps the lowest
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(top, o, 64);
-    int oa = __shfl_xor(arg, o, 64);
-    if (ov > top || (ov == top && oa < arg)) { top = ov; arg = oa; }
-  }
+  wave_best(top, arg);
   __syncthreads();
   if (lane == 0) { wave_f[wave] = top; wave_i[wave] = arg; }
   __syncthreads();

@@ -47,16 +47,6 @@ struct RouteCall {
   unsigned long long* used; // [tokens] or null: bit e of a token's word is set where its weight of expert e < 64 is not zero
 };
 
-// The best (value, index) of a wave; among equal values the lowest index.  Every lane gets it.
-__device__ __forceinline__ void wave_best(float& value, int& index) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float other = __shfl_xor(value, o, 64);
-    const int other_index = __shfl_xor(index, o, 64);
-    if (other > value || (other == value && other_index < index)) { value = other; index = other_index; }
-  }
-}
-
 // Corrections and biases of a lane's first four experts.
 struct RouteEarly {
   float correction[4], bias[4];

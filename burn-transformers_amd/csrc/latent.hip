@@ -38,7 +38,7 @@ struct LatentNormCall {
 
 template <typename T>
 __global__ void __launch_bounds__(256) latent_norm_kernel(LatentNormCall c) {
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   const int t = blockIdx.x;
   const bool query = blockIdx.y == 0;
   const int n = query ? c.q_rank : c.kv_rank;
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) latent_norm_kernel(LatentNormCall c) {
   const float* gamma = query ? c.q_gamma : c.kv_gamma;
   float partial = 0.f;
   for (int col = threadIdx.x; col < n; col += blockDim.x) partial += row[col] * row[col];
-  const float rstd = 1.0f / sqrtf(block_sum(partial, scratch) / (float)n + c.eps);
+  const float rstd = 1.0f / sqrtf(block_sum<256>(partial, scratch) / (float)n + c.eps);
   if (query) {
     T* out = static_cast<T*>(c.q_out) + (int64_t)t * c.ld_q;
     for (int col = threadIdx.x; col < c.q_cols; col += blockDim.x)

@@ -1274,7 +1274,7 @@ struct GatedNormCall {
 template <typename T>
 __global__ void __launch_bounds__(256) gated_norm_kernel(GatedNormCall c) {
   extern __shared__ float row_buf[];
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   const int t = blockIdx.x, part = blockIdx.y;
   const int n = c.channels / c.parts, base = part * n;
   float partial = 0.f;
@@ -1283,7 +1283,7 @@ __global__ void __launch_bounds__(256) gated_norm_kernel(GatedNormCall c) {
     row_buf[i] = v;
     partial += v * v;
   }
-  const float rstd = 1.0f / sqrtf(block_sum(partial, scratch) / (float)n + c.eps);
+  const float rstd = 1.0f / sqrtf(block_sum<256>(partial, scratch) / (float)n + c.eps);
   T* out = static_cast<T*>(c.out) + (int64_t)t * c.ld_out;
   for (int i = threadIdx.x; i < n; i += blockDim.x) out[base + i] = from_float<T>(row_buf[i] * rstd * c.weight[base + i]);
   if (part == 0)

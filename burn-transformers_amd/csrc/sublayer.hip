@@ -48,7 +48,7 @@ __device__ __forceinline__ float next_norm(const OutputNormCall& c, float v, flo
 template <typename T>
 __global__ void __launch_bounds__(256) output_norm_kernel(OutputNormCall c) {
   extern __shared__ float row_buf[];
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   const int t = blockIdx.x;
   float* xr = c.x + (int64_t)t * c.width;
   float partial = 0.f;
@@ -63,13 +63,13 @@ __global__ void __launch_bounds__(256) output_norm_kernel(OutputNormCall c) {
     row_buf[col] = v;
     partial += v;
   }
-  const float mean = c.kind == 0 ? block_sum(partial, scratch) / (float)c.width : 0.f;
+  const float mean = c.kind == 0 ? block_sum<256>(partial, scratch) / (float)c.width : 0.f;
   partial = 0.f;
   for (int col = threadIdx.x; col < c.width; col += blockDim.x) {
     const float d = row_buf[col] - mean;
     partial += d * d;
   }
-  const float total = block_sum(partial, scratch);
+  const float total = block_sum<256>(partial, scratch);
   const float scale = c.mult / sqrtf(total / (float)c.width + c.eps);
   T* cast = static_cast<T*>(c.cast);
   for (int col = threadIdx.x; col < c.width; col += blockDim.x) {
@@ -87,10 +87,10 @@ __global__ void __launch_bounds__(256) output_norm_kernel(OutputNormCall c) {
     float sum = 0.f;
     if (c.next_kind == 0)
       for (int col = threadIdx.x; col < c.width; col += blockDim.x) sum += row_buf[col];
-    const float next_mean = c.next_kind == 0 ? block_sum(sum, scratch) / (float)c.width : 0.f;
+    const float next_mean = c.next_kind == 0 ? block_sum<256>(sum, scratch) / (float)c.width : 0.f;
     sum = 0.f;
     for (int col = threadIdx.x; col < c.width; col += blockDim.x) sum += (row_buf[col] - next_mean) * (row_buf[col] - next_mean);
-    const float next_rstd = 1.0f / sqrtf(block_sum(sum, scratch) / (float)c.width + c.next_eps);
+    const float next_rstd = 1.0f / sqrtf(block_sum<256>(sum, scratch) / (float)c.width + c.next_eps);
     for (int col = threadIdx.x; col < c.width; col += blockDim.x) {
       const float y = next_norm(c, row_buf[col], next_mean, next_rstd, col);
       if (c.next_dtype == 0) static_cast<float*>(c.next_out)[(int64_t)t * c.next_ld + col] = y;
@@ -155,7 +155,7 @@ struct RowColumns {
   }
   // block_sum of what `apart` left (whose barrier stands in place of the one before the sum's own)
   __device__ __forceinline__ static float sum(float partial, float* scratch) {
-    if constexpr (!QUADS) return block_sum(partial, scratch);
+    if constexpr (!QUADS) return block_sum<256>(partial, scratch);
     partial = wave_sum(partial);
     if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = partial;
     __syncthreads();
@@ -169,7 +169,7 @@ struct RowColumns {
 template <typename T, int KMAX, bool QUADS>
 __global__ void __launch_bounds__(256) output_norm_small_kernel(OutputNormCall c) {
   typedef RowColumns<KMAX, QUADS> Columns;
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[32];
   __shared__ __attribute__((aligned(16))) float row_buf[QUADS ? 256 * KMAX : 4];
   const int t = blockIdx.x;
   float* xr = c.x + (int64_t)t * c.width;
@@ -350,30 +350,34 @@ struct PolyNormCall {
   int64_t ldo;
 };
 
-// Three block-wide sums with one meeting of the waves (blocks of up to 1024 threads).
+// Three sums over a work-group of 256 threads with one meeting of the waves; `scratch` holds 12 floats of LDS, on 16 bytes.
 __device__ __forceinline__ void block_sum3(float& a, float& b, float& d, float* scratch) {
   a = wave_sum(a);
   b = wave_sum(b);
   d = wave_sum(d);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, waves = (blockDim.x + 63) >> 6;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (lane == 0) {
     scratch[wave * 3] = a;
     scratch[wave * 3 + 1] = b;
     scratch[wave * 3 + 2] = d;
   }
   __syncthreads();
+  floatx4 part[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) part[q] = reinterpret_cast<const floatx4*>(scratch)[q];
   a = b = d = 0.f;
-  for (int w = 0; w < waves; ++w) {
-    a += scratch[w * 3];
-    b += scratch[w * 3 + 1];
-    d += scratch[w * 3 + 2];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    a += part[(w * 3) >> 2][(w * 3) & 3];
+    b += part[(w * 3 + 1) >> 2][(w * 3 + 1) & 3];
+    d += part[(w * 3 + 2) >> 2][(w * 3 + 2) & 3];
   }
 }
 
 template <typename T>
 __global__ void __launch_bounds__(256) poly_norm_kernel(PolyNormCall c) {
   extern __shared__ float row_buf[];
-  __shared__ float scratch[48];
+  __shared__ __attribute__((aligned(16))) float scratch[12];
   const int t = blockIdx.x;
   const float* zr = c.z + (int64_t)t * c.ldz;
   float s2 = 0.f, s4 = 0.f, s6 = 0.f;
