@@ -17,8 +17,8 @@ enum EpilogueMode {
   EPI_TURN = 6,      // out[m][n] = acc, of every turn.pitch columns the turn.dim from turn.at on rotated in neighbouring pairs
                      //   by the row's position (element type T; the skinny kernel only)
 };
-// What the skinny kernel is built for: the common modes, or one of the two that are forms of the kernel of their own.
-enum EpilogueKind { EPILOGUE_COMMON = 0, EPILOGUE_TWO = 1, EPILOGUE_TURN = 2 };
+// What the skinny kernel is built for: the common modes, or one of the three that are forms of the kernel of their own.
+enum EpilogueKind { EPILOGUE_COMMON = 0, EPILOGUE_TWO = 1, EPILOGUE_TURN = 2, EPILOGUE_QKV = 3 };
 
 enum Activation {
   ACT_GELU_TANH = 0,
@@ -98,134 +98,137 @@ __device__ __forceinline__ void store4<bf16_t>(bf16_t* dst, const float* v, int 
   }
 }
 
-// What an epilogue needs from memory besides the accumulators, fetched at the START of a kernel
-// so that no load is left on the critical path after the last multiply: the bias (plus the old
-// value of the residual stream in EPI_RESIDUAL) and, for the key/value scatter, where the row's
-// token lives in the paged cache.
-struct EpiloguePrefetch {
-  float add[4];      // EPI_TURN: the amplitudes of the two pairs, then their frequencies (0: not turned)
-  int64_t kv_base;   // start of the (block, head) plane of the token; valid for key/value columns
-  int pos;
+// What the skinny kernel's epilogue adds to the sums of neighbouring columns: the bias, and in EPI_RESIDUAL the old values of the
+// residual stream.
+template <int KIND, int VALUES>
+__device__ __forceinline__ void epilogue_addends(const Epilogue& e, int M, int n_end, int m, int n0, int split, float (&add)[VALUES]) {
+#pragma unroll
+  for (int i = 0; i < VALUES; ++i) add[i] = 0.f;
+  if (KIND == EPILOGUE_TURN) return;
+  int n[VALUES];                            // (values beyond the rows or columns are dropped)
+#pragma unroll
+  for (int i = 0; i < VALUES; ++i) n[i] = n0 + i < n_end ? n0 + i : n_end - 1;
+  if (e.bias != nullptr && split == 0) {
+#pragma unroll
+    for (int i = 0; i < VALUES; ++i) add[i] = e.bias[n[i]];
+  }
+  if (KIND == EPILOGUE_COMMON && e.mode == EPI_RESIDUAL) {
+    const float* x = static_cast<const float*>(e.out) + (int64_t)(m < M ? m : M - 1) * e.ldo;
+#pragma unroll
+    for (int i = 0; i < VALUES; ++i) add[i] += x[n[i]];
+  }
+}
+
+// What the skinny kernel's epilogue looks up, by a wave that multiplies nothing: loads that depend on each other would wait for
+// all the weights before them in a wave that streams (they return in order), which put a second round trip to memory behind
+// every product.  Of up to 16 * MT rows (and 16 * NT columns).
+template <int KIND, int MT, int NT>
+struct EpilogueTables {       // (the other kinds need none)
+  __device__ __forceinline__ void fill(const Epilogue&, int, int) {}
+};
+template <int MT, int NT>
+struct EpilogueTables<EPILOGUE_QKV, MT, NT> {
+  int64_t plane[16 * MT];     // where the block of the row's token starts in the cache, and the token's position
+  int pos[16 * MT];
+  __device__ __forceinline__ void fill(const Epilogue& e, int M, int) {
+    const int m = threadIdx.x & 63;
+    if (m < M) {
+      const int p = e.tok_pos[m], seq = e.tok_seq[m];
+      pos[m] = p;
+      plane[m] = kv_plane(e.kv, e.kv.blocks[(int64_t)seq * e.kv.max_blocks + p / BT_KV_BLOCK], 0);
+    }
+  }
+};
+template <int MT, int NT>
+struct EpilogueTables<EPILOGUE_TURN, MT, NT> {
+  float2 turn[16 * MT][8 * NT];      // amplitude times cosine and sine of a row's pair of columns
+  __device__ __forceinline__ void fill(const Epilogue& e, int M, int n_base) {
+    for (int at = threadIdx.x & 63; at < M * 8 * NT; at += 64) {
+      const int m = at / (8 * NT), pair = at % (8 * NT);
+      const int j = (n_base + 2 * pair) % e.turn.pitch - e.turn.at;
+      const bool turned = j >= 0 && j < e.turn.dim;
+      float sn = 0.f, cs = 1.f;
+      const float f = turned ? e.turn.inv_freq[j >> 1] : 0.f;
+      if (f != 0.f) sincosf((float)e.tok_pos[m] * f, &sn, &cs);
+      turn[m][pair] = make_float2(cs, sn);
+    }
+  }
 };
 
-// A valid address for the loads of an epilogue mode that is not in use: the prefetch below has
-// no branches, so every load in it is always issued (and its result discarded where unused).
-__device__ int bt_dummy_words[4] = {0, 0, 0, 0};
-
-__device__ __forceinline__ EpiloguePrefetch epilogue_prefetch(const Epilogue& e, int M, int N, int m, int n0,
-                                                              int split) {
-  // Branch-free on purpose: with no control flow the compiler issues these loads among the
-  // caller's own and waits for none of them before it has to.
-  EpiloguePrefetch p;
-  const int mm = m < M ? m : M - 1;
-  const bool with_bias = e.bias != nullptr && split == 0;
-  const bool residual = e.mode == EPI_RESIDUAL;
-  const bool scatter = e.mode == EPI_QKV;
-  const float* dummy = reinterpret_cast<const float*>(bt_dummy_words);
-  const float* bias = with_bias ? e.bias : dummy;
-  const float* x = residual ? static_cast<const float*>(e.out) + (int64_t)mm * e.ldo : dummy;
-  const int* tok_seq = scatter ? e.tok_seq : bt_dummy_words;
-  const int* tok_pos = scatter ? e.tok_pos : bt_dummy_words;
-  int seq = tok_seq[scatter ? mm : 0];
-  int pos = tok_pos[scatter ? mm : 0];
+// Stores of neighbours: together where all are inside and the place is aligned.
+template <typename T, int VALUES>
+__device__ __forceinline__ void store_values(T* dst, const float (&v)[VALUES], int count) {
+  typedef __attribute__((__vector_size__(VALUES * sizeof(T)))) T Ts;
+  if (VALUES > 1 && count >= VALUES && ((uintptr_t)dst & (VALUES * sizeof(T) - 1)) == 0) {
+    Ts all;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int nn = n0 + i < N ? n0 + i : N - 1;
-    float b = bias[with_bias ? nn : 0];
-    float xv = x[residual ? nn : 0];
-    p.add[i] = (with_bias ? b : 0.f) + (residual ? xv : 0.f);
-  }
-  // key/value columns: where the token's position lives in the paged cache
-  int c = n0 - e.n_q;
-  if (c >= e.n_kv) c -= e.n_kv;
-  const bool kv_column = scatter && n0 >= e.n_q && n0 < N;
-  const int head = kv_column ? c / e.kv.head_dim : 0;
-  const int* blocks = kv_column ? e.kv.blocks : bt_dummy_words;
-  int block = blocks[kv_column ? (int64_t)seq * e.kv.max_blocks + pos / BT_KV_BLOCK : 0];
-  p.kv_base = kv_plane(e.kv, block, head);
-  p.pos = pos;
-  return p;
-}
-
-// The same for EPI_TURN: the row's position and the frequencies of the two pairs.
-__device__ __forceinline__ EpiloguePrefetch epilogue_prefetch_turn(const Epilogue& e, int M, int m, int n0) {
-  EpiloguePrefetch p = {};
-  p.pos = e.tok_pos[m < M ? m : M - 1];
-  const int j = n0 % e.turn.pitch - e.turn.at;       // (even: the pairs of four columns are 0, 1 and 2, 3)
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const bool turned = j + 2 * i >= 0 && j + 2 * i < e.turn.dim;
-    const float f = e.turn.inv_freq[turned ? (j + 2 * i) >> 1 : 0];
-    p.add[i] = turned ? e.turn.amplitude : 1.f;
-    p.add[2 + i] = turned ? f : 0.f;
-  }
-  return p;
-}
-
-// The epilogue with everything but the accumulators already in registers.  KIND: EPI_F32_ACT and EPI_TURN are forms of
-// the kernel of their own, so that the others carry none of them.
-template <typename T, int KIND = EPILOGUE_COMMON>
-__device__ __forceinline__ void epilogue4_prefetched(const Epilogue& e, int N, int m, int n0, const float* acc,
-                                                     int split, const EpiloguePrefetch& p) {
-  int count = N - n0 < 4 ? N - n0 : 4;
-  if (count <= 0) return;
-  float v[4];
-  bool aligned = (e.ldo & 3) == 0;
-  if constexpr (KIND == EPILOGUE_TURN) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float sn = 0.f, cs = 1.f;
-      if (p.add[2 + i] != 0.f) sincosf((float)p.pos * p.add[2 + i], &sn, &cs);
-      v[2 * i] = p.add[i] * (acc[2 * i] * cs - acc[2 * i + 1] * sn);
-      v[2 * i + 1] = p.add[i] * (acc[2 * i + 1] * cs + acc[2 * i] * sn);
-    }
-    store4<T>(static_cast<T*>(e.out) + (int64_t)m * e.ldo + n0, v, count, aligned);
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = acc[i] + p.add[i];
-  if constexpr (KIND == EPILOGUE_TWO) {
-    if (n0 < e.n_q) {
-      store4<float>(static_cast<float*>(e.out) + (int64_t)m * e.ldo + n0, v, count, aligned);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = activate<T>(v[i], e.act);
-      const int c = n0 - e.n_q;
-      if (e.out_rows == 0) store4<T>(static_cast<T*>(e.out2) + (int64_t)m * e.ldo2 + c, v, count, (e.ldo2 & 3) == 0);
-      else store4<T>(static_cast<T*>(e.out2) + activation_offset<T>(e.out_rows, e.ldo2, m, c), v, count, true);
-    }
-    return;
-  }
-  if (e.mode == EPI_STORE) {
-    if (e.out_rows == 0) store4<T>(static_cast<T*>(e.out) + (int64_t)m * e.ldo + n0, v, count, aligned);     // (one branch for all threads)
-    else store4<T>(static_cast<T*>(e.out) + activation_offset<T>(e.out_rows, e.ldo, m, n0), v, count, true);
-  } else if (e.mode == EPI_ACT) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = activate<T>(v[i], e.act);
-    if (e.out_rows == 0) store4<T>(static_cast<T*>(e.out) + (int64_t)m * e.ldo + n0, v, count, aligned);     // (one branch for all threads)
-    else store4<T>(static_cast<T*>(e.out) + activation_offset<T>(e.out_rows, e.ldo, m, n0), v, count, true);
-  } else if (e.mode == EPI_F32) {
-    store4<float>(static_cast<float*>(e.out) + (int64_t)split * e.split_stride + (int64_t)m * e.ldo + n0,
-                  v, count, aligned);
-  } else if (e.mode == EPI_RESIDUAL) {
-    store4<float>(static_cast<float*>(e.out) + (int64_t)m * e.ldo + n0, v, count, aligned);
+    for (int i = 0; i < VALUES; ++i) all[i] = from_float<T>(v[i]);
+    *reinterpret_cast<Ts*>(dst) = all;
   } else {
-    if (n0 < e.n_q) {
-      store4<T>(static_cast<T*>(e.out) + (int64_t)m * e.ldo + n0, v, count, aligned);
-    } else {
-      int c = n0 - e.n_q;
-      bool is_value = c >= e.n_kv;
-      if (is_value) c -= e.n_kv;
-      int channel = c % e.kv.head_dim;
-      if (!is_value) {
-        store4<T>(static_cast<T*>(e.kv.keys) + p.kv_base + key_offset(e.kv.head_dim, p.pos, channel), v, count, true);
-      } else {
-        T* dst = static_cast<T*>(e.kv.values) + p.kv_base + value_offset(e.kv.head_dim, p.pos, channel);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)     // consecutive channels of one position lie four elements apart
+    for (int i = 0; i < VALUES; ++i)
+      if (i < count) dst[i] = from_float<T>(v[i]);
+  }
+}
+
+// The skinny kernel's epilogue for VALUES neighbouring columns of a row, inside four: v are the sums with what is added to them,
+// column is n0 inside the work-group.  One value a lane with up to sixteen rows: a wave that takes four of each lane has most of
+// its lanes idle then, and the longer chain behind the last barrier showed in every product (0.3 us, with a GELU 0.7, of 2.7 and 3.7).
+template <typename T, int KIND, int VALUES, typename Tables>
+__device__ __forceinline__ void epilogue_values(const Epilogue& e, int N, int m, int n0, int column, float (&v)[VALUES], int split,
+                                                const Tables& tables) {
+  const int count = N - n0;
+  if constexpr (KIND == EPILOGUE_TURN) {    // (pairs of columns are one lane's or two neighbours'; N is whole pairs)
+    float y[VALUES];
+#pragma unroll
+    for (int i = 0; i < VALUES; ++i) {
+      const float other = VALUES == 1 ? lane_moved<0xb1>(v[i]) : v[VALUES == 1 ? i : i ^ 1];
+      const int j = (n0 + i) % e.turn.pitch - e.turn.at;
+      const float2 t = tables.turn[m][(column + i) >> 1];
+      const float amplitude = j >= 0 && j < e.turn.dim ? e.turn.amplitude : 1.f;
+      const bool odd = (column + i) & 1;
+      y[i] = amplitude * fmaf(odd ? other : v[i], odd ? t.y : t.x, odd ? v[i] * t.x : -(other * t.y));
+    }
+    if (count > 0) store_values<T, VALUES>(static_cast<T*>(e.out) + (int64_t)m * e.ldo + n0, y, count);
+    return;
+  }
+  if (count <= 0) return;
+  if constexpr (KIND == EPILOGUE_TWO) {
+    if (n0 < e.n_q) {                       // (n_q is a multiple of four)
+      store_values<float, VALUES>(static_cast<float*>(e.out) + (int64_t)m * e.ldo + n0, v, count);
+    } else {
+#pragma unroll
+      for (int i = 0; i < VALUES; ++i) v[i] = activate<T>(v[i], e.act);
+      store_values<T, VALUES>(static_cast<T*>(e.out2) + activation_offset<T>(e.out_rows, e.ldo2, m, n0 - e.n_q), v, count);
+    }
+  } else if constexpr (KIND == EPILOGUE_QKV) {
+    if (n0 < e.n_q) {
+      store_values<T, VALUES>(static_cast<T*>(e.out) + (int64_t)m * e.ldo + n0, v, count);
+    } else {                                // (queries, keys, values and heads are multiples of sixteen columns)
+      int c = n0 - e.n_q;
+      const bool is_value = c >= e.n_kv;
+      if (is_value) c -= e.n_kv;
+      const int head = c / e.kv.head_dim, channel = c % e.kv.head_dim;
+      const int64_t base = tables.plane[m] + (int64_t)head * e.kv.head_stride;
+      const int pos = tables.pos[m];
+      if (!is_value) {
+        store_values<T, VALUES>(static_cast<T*>(e.kv.keys) + base + key_offset(e.kv.head_dim, pos, channel), v, count);
+      } else {
+        T* dst = static_cast<T*>(e.kv.values) + base + value_offset(e.kv.head_dim, pos, channel);
+#pragma unroll
+        for (int i = 0; i < VALUES; ++i)    // consecutive channels of one position lie four elements apart
           if (i < count) dst[4 * i] = from_float<T>(v[i]);
       }
     }
+  } else if (e.mode == EPI_STORE || e.mode == EPI_ACT) {
+    if (e.mode == EPI_ACT) {
+#pragma unroll
+      for (int i = 0; i < VALUES; ++i) v[i] = activate<T>(v[i], e.act);
+    }
+    store_values<T, VALUES>(static_cast<T*>(e.out) + activation_offset<T>(e.out_rows, e.ldo, m, n0), v, count);
+  } else {                                  // EPI_F32, EPI_RESIDUAL (whose products are not split)
+    store_values<float, VALUES>(static_cast<float*>(e.out) + (e.mode == EPI_F32 ? (int64_t)split * e.split_stride : 0) + (int64_t)m * e.ldo + n0, v,
+                                count);
   }
 }
 

@@ -407,12 +407,22 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
                                lds + wave * tile_scratch_bytes<TM, TN>());
 }
 
-// Memory latency on this GPU is about a microsecond and one compute unit alone pulls only a few
-// per cent of the HBM bandwidth, while a decode step is hundreds of short kernels.  So the
-// skinny kernel (a) wants at least as many work-groups as there are compute units, which is
-// what splitting K is for when there are few output columns, and (b) has ONE round trip to
-// memory on its critical path: everything the epilogue needs (bias, old residual, cache
-// addresses) is fetched together with the first batch of weights, without a branch in between.
+// What bounds it at a decode step's sizes, from clocks inside the kernel (768 x 768, one row, us): from one kernel's last wave to the
+// next one's first 1.45, its waves' start 0.2, addresses and loads 0.35, memory 0.35, the waves' meeting and the epilogue 0.4 (with
+// a GELU 0.8).  So beside enough work-groups (splitting K is for products of few columns) what counts is the chain of
+// instructions of one work-group, and the loads that its compute unit takes, 16 cycles each whatever they bring:
+//   addresses are a scalar base and a 32-bit offset a lane, from numbers that the host has worked out (SkinnyOperands); a batch's loads
+//   have scalar branches between them and nothing else; K's partial chunk is outside the batches;
+//   up to eight rows (four) two (four) chunks of the activations come with one load, and two of the weights where a work-group has
+//   eight columns (AP, WP below: 768 x 3072, one row 4.8 -> 4.3; 1600 x 1600, eight rows 4.3 -> 4.1);
+//   what depends on a table of the step is looked up by a wave that streams nothing (EpilogueTables): in a streaming wave it stood
+//   behind all the weights, a second trip to memory in every product;
+//   the epilogue takes one value a lane (VALUES below: 3072 x 768 with a GELU 3.7 -> 3.4).
+// In all, against a kernel with none of these (weights from memory, in a HIP graph, us): one row 768 x 768 3.1 -> 2.7, 768 x 3072 5.2 ->
+// 4.3, 3072 x 768 with a norm and a GELU 5.1 -> 4.2; eight rows 4800 x 1600 6.0 -> 5.4, 6400 x 1600 with a GELU 6.9 -> 6.1, 1600 x 6400
+// in five slices 6.4 -> 6.1, 18432 x 2048 16.5 -> 15.5; 64 rows 1600 x 6400 in five 11.4 -> 10.1.  Tried: loads without branches
+// (chunks that do not exist read again: 5.2 -> 5.5 for 768 x 3072), lanes without a row or column masked out of the loads (no
+// gain: a load costs its 16 cycles), the bias ahead of the weights (2.7 -> 2.9).
 // MT row blocks of 16 (activations) by NT column blocks of 16 (weights) per work-group.  With
 // more than 16 rows the activations a work-group reads (all rows, its whole K range) outweigh its
 // weights, and they are read once per work-group: two column blocks halve that traffic.
@@ -426,118 +436,164 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
 // statistics are computed while the weights are on their way.
 __device__ float bt_norm_zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
-template <typename T, int MT, int NT, int U, int WAVES, int QPL = 0, bool CHUNKED = false, int KIND = EPILOGUE_COMMON>
-__global__ void __launch_bounds__(WAVES * 64)
-gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
-                   int K, Epilogue epi, int tile_columns, NormOperand norm, int packed, int a_rows) {
+// Eight waves that stream, and one beside them that looks up the tables of the epilogues that have any.
+constexpr int skinny_threads(int waves, int kind) { return (waves + (kind == EPILOGUE_QKV || kind == EPILOGUE_TURN)) * 64; }
+// Waves a SIMD has room for: two work-groups a compute unit where the registers allow it without spilling (at eight rows the forms of
+// two column blocks do too: 123 registers).
+constexpr int skinny_occupancy(int mt, int nt, int qpl) { return mt == 1 && nt == 1 && qpl == 0 ? 4 : 2; }
+
+// Of a load that holds `16 / ROWS` chunks of ROWS rows in every sixteen lanes, the operand of chunk `sub`: its rows in the first ROWS lanes.
+template <int ROWS>
+__device__ __forceinline__ int4v lanes_down(int4v v, int sub) {      // (sub: a constant where this is used)
+  if (ROWS == 16 || sub == 0) return v;
+  int4v r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)        // row_ror:16 - sub * ROWS: lane j takes what lane j + sub * ROWS holds
+    r[i] = ROWS == 8 ? lane_moved<0x128>(v[i]) : sub == 1 ? lane_moved<0x12c>(v[i]) : sub == 2 ? lane_moved<0x128>(v[i]) : lane_moved<0x124>(v[i]);
+  return r;
+}
+
+// The skinny kernel's operands as its addresses need them, in one line of the arguments (64 bytes).
+// tile_columns: how many of its 16 * NT output columns a work-group really owns (a multiple of
+// four).  Fewer than all of them is for balance: 300 work-groups of 16 columns leave 44 of 256
+// compute units with twice the bytes of the others, 400 of 12 columns leave every unit at most
+// 24 columns.  The lanes of the columns left out repeat the last real one and store nothing.
+// W is [N][K], or packed: for each work-group's `tile_columns` columns the chunks of K one
+// after the other, [group][chunk][tile_columns][64 bytes], K and the last group padded with zeros:
+// a wave's load of a chunk is then one contiguous run of bytes and a work-group reads one
+// contiguous block front to back.  A is row-major or chunk-major (activation_offset in common.h): the
+// 64 lanes of an operand load then read one contiguous KiB.
+struct SkinnyOperands {
+  const void* W;
+  const void* A;
+  int64_t w_group;                 // bytes from a work-group's first column to the next one's
+  int w_step, a_step;              // bytes from a chunk of 64 bytes of K to the next
+  unsigned w_pitch, a_pitch;       // bytes from a column to the next, from a row to the next
+  int whole, rest;                 // whole chunks of K, values behind them
+  int M, N, tile_columns, splits;
+};
+template <typename T>
+static SkinnyOperands skinny_operands(const void* A, int64_t lda, const void* W, int M, int N, int K, int splits, int columns, int packed,
+                                      int a_rows) {
+  constexpr int CHUNK = 64 / (int)sizeof(T);
+  SkinnyOperands o;
+  o.W = W;
+  o.A = A;
+  o.whole = K / CHUNK;
+  o.rest = K % CHUNK;
+  o.w_step = packed ? columns * 64 : 64;
+  o.w_pitch = packed ? 64u : (unsigned)(K * sizeof(T));
+  o.w_group = packed ? (int64_t)((K + CHUNK - 1) / CHUNK) * o.w_step : (int64_t)columns * K * (int64_t)sizeof(T);
+  o.a_step = a_rows > 0 ? a_rows * 64 : 64;
+  o.a_pitch = a_rows > 0 ? 64u : (unsigned)(lda * (int64_t)sizeof(T));
+  o.M = M;
+  o.N = N;
+  o.tile_columns = columns;
+  o.splits = splits;
+  return o;
+}
+
+template <typename T, int MT, int NT, int U, int WAVES, int QPL, int KIND, int AP, int WP>
+__global__ void __launch_bounds__(skinny_threads(WAVES, KIND), skinny_occupancy(MT, NT, QPL))
+gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   constexpr int ELEMS = Mma<T>::ELEMS;      // K values in a lane's 16-byte load
-  constexpr int CHUNK = 4 * ELEMS;          // K values the wave's four K groups cover together
-  constexpr bool NORM = QPL > 0;
+  constexpr bool NORM = QPL > 0, TABLES = KIND == EPILOGUE_QKV || KIND == EPILOGUE_TURN;
   static_assert(!NORM || (MT == 1 && sizeof(T) == 2), "the fused norm is for bfloat16 and up to 16 rows");
   extern __shared__ __attribute__((aligned(16))) unsigned char normed[];   // NORM: [16][K * 2 + 16] bytes
-  const int normed_pitch = K * 2 + 16;      // the 16 bytes spread the rows over the LDS banks
-  // tile_columns: how many of its 16 * NT output columns a work-group really owns (a multiple of
-  // four).  Fewer than all of them is for balance: 300 work-groups of 16 columns leave 44 of 256
-  // compute units with twice the bytes of the others, 400 of 12 columns leave every unit at most
-  // 24 columns.  The lanes of the columns left out repeat the last real one and store nothing.
-  __shared__ __attribute__((aligned(16))) float red[WAVES][MT * NT][64][4];
-  static_assert(MT * NT <= WAVES, "one wave finishes each block of the work-group's output");
+  const int M = o.M, whole = o.whole, rest = o.rest, splits = o.splits;
+  const int K = whole * (4 * ELEMS) + rest, normed_pitch = K * 2 + 16;      // the 16 bytes spread the rows over the LDS banks
+  __shared__ __attribute__((aligned(16))) float red[WAVES][MT * NT][4][80];
+  __shared__ EpilogueTables<KIND, MT, NT> tables;
   // the wave's number is the same in all its lanes: saying so keeps every test on it a scalar
   // branch, which costs no wait for loads in flight (a divergent one does)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int n_base = blockIdx.x * o.tile_columns;
+  const int n_end = n_base + o.tile_columns < o.N ? n_base + o.tile_columns : o.N;   // one past this work-group's last column
+  if (TABLES && wave == WAVES) {            // the wave that looks up what the epilogue needs: nothing here waits for weights
+    tables.fill(epi, M, n_base);
+    if constexpr (NORM) __syncthreads();
+    __syncthreads();
+    return;
+  }
   const int i16 = lane & 15, g = lane >> 4;
-  const int n_base = blockIdx.x * tile_columns;
-  const int n_end = n_base + tile_columns < N ? n_base + tile_columns : N;   // one past this work-group's last column
-  const int split = blockIdx.y, splits = gridDim.y;
-  // packed: W is not [N][K] but, for each work-group's `tile_columns` columns, the chunks of K one
-  // after the other, [group][chunk][tile_columns][CHUNK], K and the last group padded with zeros:
-  // a wave's load of a chunk is then one contiguous run of bytes and a work-group reads one
-  // contiguous block front to back.
-  const int w_chunk_pitch = packed ? tile_columns * CHUNK : CHUNK;     // elements from one chunk to the next
-  const T* w_row[NT];
+  const int split = blockIdx.y;
+  // Addresses are a uniform base and a lane's offset of 32 bits, which one addition moves from chunk to chunk.
+  const char* w_base = static_cast<const char*>(o.W) + (int64_t)blockIdx.x * o.w_group;
+  const char* a_base = static_cast<const char*>(o.A);
+  const int c_first = split * WAVES + wave, stride = splits * WAVES;
+  const unsigned w_jump = stride * o.w_step, a_jump = stride * o.a_step;
+  // AP chunks of the activations to a load where the rows are few enough, WP of the weights: sixteen lanes hold 16 / AP rows of
+  // the wave's chunk u, then of u + 1, ..., and a rotation in the row of lanes brings the later ones down.  (Lanes whose chunk
+  // does not exist read the last whole one; what they hold is not multiplied.)
+  constexpr int A_ROWS = 16 / AP, W_COLS = 16 / WP;
+  static_assert(U % AP == 0 && U % WP == 0 && (MT == 1 || AP == 1) && (NT == 1 || WP == 1), "whole loads of one block");
+  unsigned w_off[NT], a_off[MT], w_most = 0, a_most = 0;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
-    int n = n_base + nt * 16 + i16;
-    n = n < n_end ? n : n_end - 1;
-    w_row[nt] = packed ? W + ((int64_t)blockIdx.x * ((K + CHUNK - 1) / CHUNK) * tile_columns + (n - n_base)) * CHUNK
-                       : W + (int64_t)n * K;
+    const int n = WP > 1 ? i16 % W_COLS : nt * 16 + i16, last = n_end - n_base - 1;
+    const unsigned column = (unsigned)(n < last ? n : last) * o.w_pitch + g * 16;
+    w_off[nt] = column + (c_first + i16 / W_COLS * (WP > 1 ? stride : 0)) * o.w_step;
+    if (WP > 1) w_most = column + (whole - 1) * o.w_step;
   }
-  // CHUNKED: the activations are chunk-major (activation_offset in common.h) with a_rows rows: the
-  // 64 lanes of an operand load then read one contiguous KiB.  (A form of the kernel of its own, so
-  // that the row-major form keeps its loads free of anything computed per lane between them.)
-  const int a_chunk_pitch = CHUNKED ? a_rows * CHUNK : CHUNK;      // elements from one chunk of a row to its next
-  const T* a_row[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    int m = mt * 16 + i16;
-    a_row[mt] = CHUNKED ? A + (int64_t)(m < M ? m : M - 1) * CHUNK : A + (int64_t)(m < M ? m : M - 1) * lda;
+  for (int mt = 0; mt < MT; ++mt) {         // (rows beyond M repeat the last; the epilogue drops them)
+    const int m = AP > 1 ? i16 % A_ROWS : mt * 16 + i16;
+    const unsigned row = (unsigned)(m < M ? m : M - 1) * o.a_pitch + g * 16;
+    a_off[mt] = row + (c_first + i16 / A_ROWS * (AP > 1 ? stride : 0)) * o.a_step;
+    if (AP > 1) a_most = row + (whole - 1) * o.a_step;
   }
-  // A batch is two phases.  First every load of the batch is issued: a chunk beyond K is
-  // skipped by a scalar branch, a group beyond K (a multiple of the group) inside the last chunk
-  // reads the row's last group instead.  Only then are the weights of such a group cleared (with
-  // a bit mask) and multiplied.  Nothing that depends on a lane or on loaded data stands between
-  // the loads, so the compiler has no reason to wait for one before it issues the next.
-  // Rows beyond M repeat row M - 1; their results are dropped by the epilogue.
-  const int chunks = (K + CHUNK - 1) / CHUNK;
-  const int stride = splits * WAVES;
+  auto from = [](const char* base, unsigned off) { return *reinterpret_cast<const int4v*>(base + off); };
   floatx4 acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-  int4v wv[U][NT], av[U][MT];
+  // A batch: all its loads, then what waits for them.  (A place whose chunk does not exist is neither loaded nor multiplied.)
+  int4v wv[U / WP][NT], av[U / AP][MT];
   auto issue = [&](int c0) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int cc = c0 + u * stride;
+    for (int u = 0; u < U; ++u)
+      if ((u % WP == 0 || (!NORM && u % AP == 0)) && c0 + u * stride < whole) {
+        if (u % WP == 0) {
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) wv[u][nt] = int4v{0, 0, 0, 0};
+          for (int nt = 0; nt < NT; ++nt) {
+            const unsigned off = w_off[nt] + u * w_jump;
+            wv[u / WP][nt] = from(w_base, WP > 1 && off > w_most ? w_most : off);
+          }
+        }
+        if (!NORM && u % AP == 0) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) av[u][mt] = int4v{0, 0, 0, 0};
-      if (cc < chunks) {
-        int k = cc * CHUNK + g * ELEMS;
-        int kc = k < K ? k : K - ELEMS;
-        int wc = packed ? cc * w_chunk_pitch + g * ELEMS : kc;      // (the packed chunks are whole: zeros beyond K)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) wv[u][nt] = *reinterpret_cast<const int4v*>(w_row[nt] + wc);
-        if constexpr (!NORM) {
-          // (kc is a multiple of ELEMS inside one chunk: chunk kc / CHUNK, offset kc % CHUNK)
-          int ac = CHUNKED ? (kc / CHUNK) * a_chunk_pitch + kc % CHUNK : kc;
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) av[u][mt] = *reinterpret_cast<const int4v*>(a_row[mt] + ac);
+          for (int mt = 0; mt < MT; ++mt) {
+            const unsigned off = a_off[mt] + u * a_jump;
+            av[u / AP][mt] = from(a_base, AP > 1 && off > a_most ? a_most : off);
+          }
         }
       }
-    }
   };
   auto multiply = [&](int c0) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int keep = (c0 + u * stride) * CHUNK + g * ELEMS < K ? -1 : 0;
+    for (int u = 0; u < U; ++u)
+      if (c0 + u * stride < whole) {
+        int4v a[MT];
+        if constexpr (NORM) {               // the operand from LDS
+          a[0] = *reinterpret_cast<const int4v*>(normed + (i16 < M ? i16 : M - 1) * normed_pitch + (c0 + u * stride) * 64 + g * 16);
+        } else {
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        int4v w = wv[u][nt] & keep;
+          for (int mt = 0; mt < MT; ++mt) a[mt] = lanes_down<A_ROWS>(av[u / AP][mt], u % AP);
+        }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) Mma<T>::block16(acc[mt][nt], w, av[u][mt]);
+        for (int nt = 0; nt < NT; ++nt) {
+          const int4v w = lanes_down<W_COLS>(wv[u / WP][nt], u % WP);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) Mma<T>::block16(acc[mt][nt], w, a[mt]);
+        }
       }
-    }
   };
-  // NORM: the operand of every chunk of the batch from LDS (a chunk beyond K reads the row's last
-  // group, as the loads from memory do; its weights are cleared)
-  auto operands_from_lds = [&](int c0) {
-    const int row = i16 < M ? i16 : M - 1;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      int k = (c0 + u * stride) * CHUNK + g * ELEMS;
-      int kc = k < K ? k : K - ELEMS;
-      av[u][0] = *reinterpret_cast<const int4v*>(normed + row * normed_pitch + kc * 2);
-    }
-  };
-  int c0 = split * WAVES + wave;
+  int c0 = c_first;
   if constexpr (NORM) {
     const int quads = K >> 2;
     const float4* g4 = reinterpret_cast<const float4*>(norm.gamma);
-    const float4* b4 = reinterpret_cast<const float4*>(norm.beta);
-    const float4* z4 = reinterpret_cast<const float4*>(bt_norm_zeros);
+    const float4* b4 = reinterpret_cast<const float4*>(norm.beta ? norm.beta : bt_norm_zeros);
     float4 xv[QPL], gv[QPL], bv[QPL];
     auto load_row = [&](int r) {
       const float4* xr = reinterpret_cast<const float4*>(norm.x + (int64_t)r * norm.ldx);
@@ -547,7 +603,7 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
         int cc = c < quads ? c : 0;          // lanes beyond the row read its start; the result is never used
         xv[q] = xr[cc];
         gv[q] = g4[cc];
-        bv[q] = norm.beta ? b4[cc] : z4[0];
+        bv[q] = b4[norm.beta ? cc : 0];
       }
     };
     auto normalise_row = [&](int r) {
@@ -590,41 +646,67 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
       normalise_row(wave + WAVES);
     }
     __syncthreads();
-    operands_from_lds(c0);
   } else {
     issue(c0);
   }
-  // wave w < MT * NT finishes row block w / NT of column block w % NT: lane holds D[i][j],
-  // i = 4 * (lane / 16) + r (column n), j = lane % 16 (row m); what its epilogue needs is
-  // fetched now, behind the first batch
-  const int blocks = MT * NT;
-  const int mine = wave < blocks ? wave : 0;
-  const int out_m = (mine / NT) * 16 + i16, out_n0 = n_base + (mine % NT) * 16 + g * 4;
-  EpiloguePrefetch pre = {};
-  if constexpr (KIND == EPILOGUE_TURN) {
-    if (wave < blocks) pre = epilogue_prefetch_turn(epi, M, out_m, out_n0);
-  } else {
-    if (wave < blocks) pre = epilogue_prefetch(epi, M, n_end, out_m, out_n0, split);
-  }
-  multiply(c0);
-  for (c0 += stride * U; c0 < chunks; c0 += stride * U) {
-    issue(c0);
-    if constexpr (NORM) operands_from_lds(c0);
+  // A thread finishes one output value, or VALUES neighbours of a row: what is added to them is fetched now, behind the first batch,
+  // so that no load is left on the critical path after the last multiply.
+  constexpr int COLUMNS = 16 * NT, THREADS = 64 * WAVES, VALUES = (16 * MT * COLUMNS + THREADS - 1) / THREADS;
+  static_assert(VALUES == 1 || VALUES == 2 || VALUES == 4, "neighbours inside four columns");
+  const int out_m = tid * VALUES / COLUMNS, column = tid * VALUES % COLUMNS;
+  float add[VALUES];
+  epilogue_addends<KIND>(epi, M, n_end, out_m, n_base + column, split, add);
+  for (;;) {
     multiply(c0);
+    c0 += U * stride;
+    if (c0 >= whole) break;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) w_off[nt] += U * w_jump;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) a_off[mt] += U * a_jump;
+    issue(c0);
   }
+  // K's partial chunk, for the wave whose turn it is (widths that are no multiple of 64 bytes: one more trip to memory for them):
+  // a group beyond K reads the last one inside, its weights are cleared
+  if (rest != 0 && wave == whole % WAVES && split == whole / WAVES % splits) {
+    const int keep = g * ELEMS < rest ? -1 : 0, inside = (rest / ELEMS - 1 - g) * 16 & ~keep;
+    const int4v zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = nt * 16 + i16, last = n_end - n_base - 1;
+      const int4v w = from(w_base, (unsigned)(n < last ? n : last) * o.w_pitch + whole * o.w_step + g * 16 + inside);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int m = mt * 16 + i16 < M ? mt * 16 + i16 : M - 1;
+        const int4v a = NORM ? *reinterpret_cast<const int4v*>(normed + m * normed_pitch + whole * 64 + g * 16 + inside)
+                             : from(a_base, (unsigned)m * o.a_pitch + whole * o.a_step + g * 16 + inside);
+        Mma<T>::block16(acc[mt][nt], keep ? w : zero, a);
+      }
+    }
+  }
+  // lane holds D[i][j]: i = 4 g + r the column, j = i16 the row.  (The groups lie 80 floats apart: neighbouring columns of four
+  // rows are then in 64 different banks.)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-      *reinterpret_cast<floatx4*>(&red[wave][mt * NT + nt][lane][0]) = acc[mt][nt];
+      *reinterpret_cast<floatx4*>(&red[wave][mt * NT + nt][g][i16 * 4]) = acc[mt][nt];
   __syncthreads();
-  if (wave < blocks) {
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+  if (out_m < M) {                          // (whole quads of lanes: the turned pairs are together)
+    const float* part = &red[0][out_m / 16 * NT + column / 16][column % 16 / 4][out_m % 16 * 4 + column % 4];
+    typedef __attribute__((__vector_size__(VALUES * sizeof(float)))) float floats;
+    float v[VALUES];
+    floats share[WAVES];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w)
+    for (int w = 0; w < WAVES; ++w) share[w] = *reinterpret_cast<const floats*>(part + w * (MT * NT * 320));
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] += red[w][wave][lane][r];
-    if (out_m < M) epilogue4_prefetched<T, KIND>(epi, n_end, out_m, out_n0, v, split, pre);   // nothing beyond n_end
+    for (int i = 0; i < VALUES; ++i) {
+      v[i] = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v[i] += share[w][i];
+      v[i] += add[i];
+    }
+    epilogue_values<T, KIND>(epi, n_end, out_m, n_base + column, column, v, split, tables);
   }
 }
 
@@ -811,73 +893,75 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
 template <typename T>
 static void launch_skinny(hipStream_t s, const T* a, int64_t lda, const T* w, int M, int N, int K, const Epilogue& epi,
                           int splits, int columns, int packed, int a_rows) {
-  dim3 grid((N + columns - 1) / columns, splits), block(512);
+  dim3 grid((N + columns - 1) / columns, splits);
   const NormOperand none = {};
-  const bool two = epi.mode == EPI_F32_ACT, turn = epi.mode == EPI_TURN;
-#define LAUNCH_SKINNY(MT, NT, U)                                                                                   \
-  do {                                                                                                             \
-    if (turn)                                                                                                      \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, false, EPILOGUE_TURN>), grid, block, 0, s, a, lda, w, M, N, K, \
-                         epi, columns, none, packed, 0);                                                           \
-    else if (two && a_rows > 0)                                                                                         \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, true, EPILOGUE_TWO>), grid, block, 0, s, a, lda, w, M, N, K, \
-                         epi, columns, none, packed, a_rows);                                                      \
-    else if (two)                                                                                                  \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, false, EPILOGUE_TWO>), grid, block, 0, s, a, lda, w, M, N, K, \
-                         epi, columns, none, packed, 0);                                                           \
-    else if (a_rows > 0)                                                                                           \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, true>), grid, block, 0, s, a, lda, w, M, N, K, epi, \
-                         columns, none, packed, a_rows);                                                           \
-    else                                                                                                           \
-      hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8>), grid, block, 0, s, a, lda, w, M, N, K, epi, columns, \
-                         none, packed, 0);                                                                         \
+  const SkinnyOperands o = skinny_operands<T>(a, lda, w, M, N, K, splits, columns, packed, a_rows);
+#define LAUNCH_SKINNY_FORM(MT, NT, U, KIND, AP, WP) \
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, KIND, AP, WP>), grid, dim3(skinny_threads(8, KIND)), 0, s, o, epi, none)
+#define LAUNCH_SKINNY(MT, NT, U, AP, WP)                                                          \
+  do {                                                                                            \
+    if (epi.mode == EPI_TURN) LAUNCH_SKINNY_FORM(MT, NT, U, EPILOGUE_TURN, AP, WP);               \
+    else if (epi.mode == EPI_QKV) LAUNCH_SKINNY_FORM(MT, NT, U, EPILOGUE_QKV, AP, WP);            \
+    else if (epi.mode == EPI_F32_ACT) LAUNCH_SKINNY_FORM(MT, NT, U, EPILOGUE_TWO, AP, WP);        \
+    else LAUNCH_SKINNY_FORM(MT, NT, U, EPILOGUE_COMMON, AP, WP);                                  \
   } while (0)
+  // eight loads in flight where a wave has more than four chunks of K to go through (measured at
+  // 17 and 32 rows: 6.4 -> 6.1 us and 6.6 -> 6.4 us for 4800 x 1600; with four chunks or fewer
+  // the longer batch only adds loads that are skipped, 4.2 -> 4.4 us for 1600 x 1600 in two slices)
+  constexpr int chunk = 4 * Mma<T>::ELEMS;
+  const int per_wave = (((K + chunk - 1) / chunk + splits - 1) / splits + 7) / 8;
   if (M <= 16) {
-    if (columns <= 16) LAUNCH_SKINNY(1, 1, 8); else LAUNCH_SKINNY(1, 2, 8);
-  } else if (M <= 32) {
-    // eight loads in flight where a wave has more than four chunks of K to go through (measured at
-    // 17 and 32 rows: 6.4 -> 6.1 us and 6.6 -> 6.4 us for 4800 x 1600; with four chunks or fewer
-    // the longer batch only adds loads that are skipped, 4.2 -> 4.4 us for 1600 x 1600 in two slices)
-    constexpr int chunk = 4 * Mma<T>::ELEMS;
-    const int per_wave = (((K + chunk - 1) / chunk + splits - 1) / splits + 7) / 8;
-    if (per_wave > 4) {
-      if (columns <= 16) LAUNCH_SKINNY(2, 1, 8); else LAUNCH_SKINNY(2, 2, 8);
+    if (per_wave <= 4) {
+      if (columns <= 16) LAUNCH_SKINNY(1, 1, 4, 1, 1); else LAUNCH_SKINNY(1, 2, 4, 1, 1);
+    } else if (M <= 4) {
+      if (columns == 8) LAUNCH_SKINNY(1, 1, 8, 4, 2); else if (columns <= 16) LAUNCH_SKINNY(1, 1, 8, 4, 1); else LAUNCH_SKINNY(1, 2, 8, 4, 1);
+    } else if (M <= 8) {
+      if (columns == 8) LAUNCH_SKINNY(1, 1, 8, 2, 2); else if (columns <= 16) LAUNCH_SKINNY(1, 1, 8, 2, 1); else LAUNCH_SKINNY(1, 2, 8, 2, 1);
     } else {
-      if (columns <= 16) LAUNCH_SKINNY(2, 1, 4); else LAUNCH_SKINNY(2, 2, 4);
+      if (columns <= 16) LAUNCH_SKINNY(1, 1, 8, 1, 1); else LAUNCH_SKINNY(1, 2, 8, 1, 1);
+    }
+  } else if (M <= 32) {
+    if (per_wave > 4) {
+      if (columns <= 16) LAUNCH_SKINNY(2, 1, 8, 1, 1); else LAUNCH_SKINNY(2, 2, 8, 1, 1);
+    } else {
+      if (columns <= 16) LAUNCH_SKINNY(2, 1, 4, 1, 1); else LAUNCH_SKINNY(2, 2, 4, 1, 1);
     }
   } else {
-    if (columns <= 16) LAUNCH_SKINNY(4, 1, 2); else LAUNCH_SKINNY(4, 2, 2);
+    if (columns <= 16) LAUNCH_SKINNY(4, 1, 2, 1, 1); else LAUNCH_SKINNY(4, 2, 2, 1, 1);
   }
 #undef LAUNCH_SKINNY
+#undef LAUNCH_SKINNY_FORM
 }
 
 // The product of the normalised rows of a float32 residual stream (see NormOperand): bfloat16
 // weights, up to 16 rows, K up to 2048 and a multiple of 8.
 static int launch_skinny_norm(hipStream_t s, const NormOperand& norm, const bf16_t* w, int M, int N, int K,
                               const Epilogue& epi, int splits, int columns, int packed) {
-  dim3 grid((N + columns - 1) / columns, splits), block(512);
+  dim3 grid((N + columns - 1) / columns, splits);
   size_t lds = (size_t)16 * (K * 2 + 16);
-#define LAUNCH_NORM(NT, QPL)                                                                                   \
+  const SkinnyOperands o = skinny_operands<bf16_t>(nullptr, K, w, M, N, K, splits, columns, packed, 0);
+#define LAUNCH_NORM(NT, QPL, WP)                                                                               \
   do {                                                                                                         \
-    if (epi.mode == EPI_F32_ACT) LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_TWO);                                      \
-    else if (epi.mode == EPI_TURN) LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_TURN);                                   \
-    else LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_COMMON);                                                           \
+    if (epi.mode == EPI_F32_ACT) LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_TWO, WP);    \
+    else if (epi.mode == EPI_TURN) LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_TURN, WP);    \
+    else if (epi.mode == EPI_QKV) LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_QKV, WP);    \
+    else LAUNCH_NORM_FORM(NT, QPL, EPILOGUE_COMMON, WP);    \
   } while (0)
-#define LAUNCH_NORM_FORM(NT, QPL, KIND)                                                                        \
+#define LAUNCH_NORM_FORM(NT, QPL, KIND, WP)                                                                        \
   do {                                                                                                         \
-    auto kernel = gemm_skinny_kernel<bf16_t, 1, NT, 8, 8, QPL, false, KIND>;                                                \
+    auto kernel = gemm_skinny_kernel<bf16_t, 1, NT, 8, 8, QPL, KIND, 1, WP>;                                                       \
     static size_t granted = 0;    /* statically allocated LDS comes on top: ask for room beyond the default */ \
     if (lds > granted) {                                                                                       \
       hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
       if (err != hipSuccess) BT_REFUSE("gemm_skinny: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));   \
       granted = lds;                                                                                           \
     }                                                                                                          \
-    hipLaunchKernelGGL(kernel, grid, block, lds, s, (const bf16_t*)nullptr, (int64_t)0, w, M, N, K, epi, columns, norm, packed, 0); \
+    hipLaunchKernelGGL(kernel, grid, dim3(skinny_threads(8, KIND)), lds, s, o, epi, norm);                                     \
   } while (0)
   if (K <= 1024) {
-    if (columns <= 16) LAUNCH_NORM(1, 4); else LAUNCH_NORM(2, 4);
+    if (columns == 8) LAUNCH_NORM(1, 4, 2); else if (columns <= 16) LAUNCH_NORM(1, 4, 1); else LAUNCH_NORM(2, 4, 1);
   } else {
-    if (columns <= 16) LAUNCH_NORM(1, 8); else LAUNCH_NORM(2, 8);
+    if (columns == 8) LAUNCH_NORM(1, 8, 2); else if (columns <= 16) LAUNCH_NORM(1, 8, 1); else LAUNCH_NORM(2, 8, 1);
   }
 #undef LAUNCH_NORM
 #undef LAUNCH_NORM_FORM
@@ -940,6 +1024,14 @@ BT_EXPORT int bt_gemm_skinny(void* stream, int dtype, const void* A, int64_t lda
       int64_t cost = ((groups + compute_units - 1) / compute_units) * (per * (c + M) + 160);
       if (best < 0 || cost < best) { best = cost; columns = c; }
     }
+  }
+  // (the kernel's offsets have 32 bits)
+  const int64_t size = 16 / elems, a_bytes = a_rows != 0 ? (int64_t)a_rows * K * size : ((int64_t)(M - 1) * lda + K) * size;
+  const int64_t w_bytes = (int64_t)columns * (K + 4 * elems) * size;
+  if (a_bytes >= (int64_t)1 << 31 || w_bytes >= (int64_t)1 << 31) {
+    if (packed || a_rows != 0 || norm != nullptr || epi->mode == EPI_F32_ACT || epi->mode == EPI_TURN)
+      BT_REFUSE("gemm_skinny: rows of pitch %lld and K %d reach beyond 2 GiB", (long long)lda, K);
+    return bt_gemm_tile(stream, dtype, A, lda, W, M, N, K, epi, splits, 1);
   }
   if (norm != nullptr) {
     rc = launch_skinny_norm((hipStream_t)stream, *norm, (const bf16_t*)W, M, N, K, *epi, splits, columns, packed);
