@@ -68,6 +68,11 @@ __device__ __forceinline__ float bt_sink_term_pow2(const float* sink, int head, 
   return sink ? exp2f(sink[head] * 1.4426950408889634f - top) : 0.f;
 }
 
+// The same from the sink's logit, for kernels that have asked for it when they started.
+__device__ __forceinline__ float bt_sink_of_pow2(const float* sink, float logit, float top) {
+  return sink ? exp2f(logit * 1.4426950408889634f - top) : 0.f;
+}
+
 __device__ __forceinline__ float bt_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 // The gate's factor on channel `channel` of head `head` of token `tok`.
@@ -77,6 +82,13 @@ __device__ __forceinline__ float bt_output_gate(const AttnArgs& a, int64_t tok, 
   const int column = a.gate_span == 1 ? head * a.gate_dim + (none ? 0 : channel) : head;
   const float factor = bt_sigmoid(a.gate[tok * a.ld_gate + column]);
   return none ? 1.f : factor;
+}
+
+// The logit of that factor alone, 0 without a gate: kernels of one token a sequence ask for it when they start.
+__device__ __forceinline__ float bt_output_logit(const AttnArgs& a, int64_t tok, int head, int channel) {
+  if (!a.gate) return 0.f;
+  const int column = a.gate_span == 1 ? head * a.gate_dim + (channel >= a.gate_dim ? 0 : channel) : head;
+  return a.gate[tok * a.ld_gate + column];
 }
 
 // What forms and output stages need of their arguments; nullptr, or what is wrong.

@@ -165,10 +165,10 @@ __device__ __forceinline__ void put4(const AttnArgs& a, int64_t tok, int head, i
   bf16x4 packed = {(bf16_t)w[0], (bf16_t)w[1], (bf16_t)w[2], (bf16_t)w[3]};
   *reinterpret_cast<bf16x4*>(static_cast<bf16_t*>(a.out) + place) = packed;
 }
-// One channel, row-major or chunk-major.
-__device__ __forceinline__ void put1(const AttnArgs& a, int tok, int head, int channel, float v) {
+// One channel, row-major or chunk-major.  `gate`: its logit (bt_output_logit), asked for long before.
+__device__ __forceinline__ void put1(const AttnArgs& a, int tok, int head, int channel, float v, float gate) {
   if constexpr (STAGED) {
-    v *= bt_output_gate(a, tok, head, channel);
+    if (a.gate && !(a.gate_span == 1 && channel >= a.gate_dim)) v *= bt_sigmoid(gate);
     if (a.out_f32) {
       static_cast<float*>(a.out)[(int64_t)tok * a.ldo + head * HD + channel] = v;
       return;
@@ -1123,9 +1123,9 @@ attention_decode_kernel(AttnArgs a) {
   float* sm_l = sm + DECODE_WAVES * group;            // [DECODE_WAVES][group]
   float* sm_o = sm + 2 * DECODE_WAVES * group;        // [DECODE_WAVES][group][HD]
   // One token per sequence, in the order of the sequences: token `seq` belongs to sequence `seq`.
-  // The query, the position and (without a window) the blocks of this wave's first two tiles do
-  // not depend on each other, so their loads fly together; the keys and values then need one
-  // more trip to memory, not two.
+  // The query, the position and the sequence's blocks do not depend on each other, so their loads fly together; the keys
+  // and values then need one more trip to memory, not two.  Without a window or runs the first two tiles' blocks are known
+  // at once and come through the scalar cache (0.3 us sooner); otherwise, and for later tiles, a lane holds an entry of the table.
   const int tok = seq;
   const bf16_t* Q = static_cast<const bf16_t*>(a.q);
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -1140,6 +1140,15 @@ attention_decode_kernel(AttnArgs a) {
     int entry0 = (32 * wave) / BT_KV_BLOCK, entry1 = (32 * wave + stride) / BT_KV_BLOCK;
     early_block0 = block_row[entry0 < last_entry ? entry0 : last_entry];
     early_block1 = block_row[entry1 < last_entry ? entry1 : last_entry];
+  }
+  int held_blocks = 0;
+  if (!early || last_entry >= 2 * stride / BT_KV_BLOCK) held_blocks = block_row[lane < last_entry ? lane : last_entry];
+  // what a thread's first element of the output needs beside the sums
+  float first_gate = 0.f, first_sink = 0.f;
+  if (splits == 1 && ((STAGED && a.gate) || a.sink) && (int)threadIdx.x < group * HD) {
+    const int j = kv_head * group + threadIdx.x / HD;
+    if (STAGED) first_gate = bt_output_logit(a, tok, j, threadIdx.x % HD);
+    if (a.sink) first_sink = a.sink[j];
   }
   const int pos = a.seq_start[seq];
   bf16x8 q[1][NKS];
@@ -1164,9 +1173,10 @@ attention_decode_kernel(AttnArgs a) {
   const int tile_end = tile_begin + per_split < tiles ? tile_begin + per_split : tiles;
   const int first = 32 * (tile_begin + wave), end = 32 * tile_end;      // (places of the walk)
   const int kin = first & (BT_KV_BLOCK - 1);                            // (the same every turn: a stride is four blocks)
-  // plane of the tile at kb: from the blocks fetched early where they apply, else from the table
-  auto plane_of = [&](int kb, int j) {
-    int block = (early && j < 2) ? (j == 0 ? early_block0 : early_block1) : block_row[kb / BT_KV_BLOCK];
+  auto plane_of = [&](int kb, int j) {       // (contexts beyond 64 blocks look the later ones up)
+    const int entry = kb / BT_KV_BLOCK;
+    const int block = early && j < 2 ? (j == 0 ? early_block0 : early_block1)
+                      : entry < 64   ? __builtin_amdgcn_readlane(held_blocks, entry) : block_row[entry];
     return kv_plane(a.kv, block, kv_head);
   };
   const Scoring sc = scoring_of(a, head);
@@ -1220,8 +1230,10 @@ attention_decode_kernel(AttnArgs a) {
         }
       }
       if (splits == 1) {
-        den += top != -INFINITY ? bt_sink_term_pow2(a.sink, kv_head * group + j, top) : 0.f;
-        put1(a, tok, kv_head * group + j, channel, FORM == 2 ? num : den > 0.f ? num / den : 0.f);
+        const bool again = e >= DECODE_WAVES * 64;
+        den += top != -INFINITY ? bt_sink_of_pow2(a.sink, again && a.sink ? a.sink[kv_head * group + j] : first_sink, top) : 0.f;
+        put1(a, tok, kv_head * group + j, channel, FORM == 2 ? num : den > 0.f ? num / den : 0.f,
+             STAGED && again ? bt_output_logit(a, tok, kv_head * group + j, channel) : first_gate);
       } else {     // this run's share, for attention_join_kernel
         float* mine = a.partial + (((int64_t)seq * a.q_heads + kv_head * group + j) * splits + split) * (HD + 2);
         mine[channel] = num;
@@ -1251,9 +1263,13 @@ attention_join_kernel(AttnArgs a, int n_rows) {
   if (pair >= n_rows * a.q_heads) return;      // (a whole wave; there is no barrier)
   const int row = pair / a.q_heads, head = pair % a.q_heads;
   const float* runs = a.partial + (int64_t)pair * a.splits * (HD + 2);
-  float top = -INFINITY, den = 0.f, num[NCH];
+  float top = -INFINITY, den = 0.f, num[NCH], gate[NCH];
+  const float sink = a.sink ? a.sink[head] : 0.f;
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) num[c] = 0.f;
+  for (int c = 0; c < NCH; ++c) {
+    num[c] = 0.f;
+    gate[c] = STAGED ? bt_output_logit(a, row, head, lane + 64 * c < HD ? lane + 64 * c : 0) : 0.f;
+  }
   for (int s0 = 0; s0 < a.splits; s0 += 8) {
     float m[8], l[8], o[8][NCH];
 #pragma unroll
@@ -1285,11 +1301,11 @@ attention_join_kernel(AttnArgs a, int n_rows) {
     }
     top = new_top;
   }
-  if (top != -INFINITY) den += bt_sink_term_pow2(a.sink, head, top);
+  if (top != -INFINITY) den += bt_sink_of_pow2(a.sink, sink, top);
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     const int channel = lane + 64 * c;
-    if (channel < HD) put1(a, row, head, channel, FORM == 2 ? num[c] : den > 0.f ? num[c] / den : 0.f);
+    if (channel < HD) put1(a, row, head, channel, FORM == 2 ? num[c] : den > 0.f ? num[c] / den : 0.f, gate[c]);
   }
 }
 

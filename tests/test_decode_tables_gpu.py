@@ -1,0 +1,55 @@
+"""Decode attention over block tables around 64 entries (a lane of a wave holds one entry each; later ones are looked up): with and
+without a window, in one run and in several, with more query heads than fill a work-group once and a gate and a sink."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from burn_transformers_amd.kernels import library as K  # noqa: E402
+from kernel_helpers import PagedCase  # noqa: E402
+from test_kernels_gpu import DEV, rel_err  # noqa: E402
+
+
+@pytest.mark.parametrize("window", [0, 300])
+@pytest.mark.parametrize("runs", [1, 3])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("totals", [[1, 513, 30], [4095, 4096, 4097, 4161], [5000, 12, 8190]])
+def test_tables_around_a_wave(totals, hd, runs, window):
+    dt = torch.bfloat16
+    case = PagedCase(totals, [1] * len(totals), 2, hd, dt, DEV, seed=hd + len(totals))
+    gen = torch.Generator().manual_seed(hd)
+    q = (torch.randn(len(totals), 8 * hd, generator=gen) * 0.5).to(dt).to(DEV)
+    out = torch.full((len(totals), 8 * hd), float("nan"), dtype=dt, device=DEV)
+    partial = torch.full((len(totals) * 8 * runs, hd + 2), float("nan"), device=DEV) if runs > 1 else None
+    args = K.attention_args(q, out, case.view(), case.tok_seq, case.tok_pos, case.seq_off, case.seq_start,
+                            8, len(totals), 1, 0.3, window, partial)
+    K.attention(args, dt, decode=True)
+    # probabilities and stored rows in bfloat16: 2^-9 each, relative to the largest value of a row of weights of one
+    assert rel_err(out, case.reference(q, 8, 0.3, window)) < 1.2e-2
+
+
+@pytest.mark.parametrize("runs", [1, 3])
+@pytest.mark.parametrize("heads,kv", [(4, 4), (16, 1)])           # one head a work-group, more elements than threads
+@pytest.mark.parametrize("span", [0, 1])
+def test_gates_and_sinks_asked_for_early(runs, heads, kv, span):
+    dt, hd, totals = torch.bfloat16, 128, [700, 65, 1]
+    case = PagedCase(totals, [1] * 3, kv, hd, dt, DEV, seed=heads)
+    gen = torch.Generator().manual_seed(heads + span)
+    q = (torch.randn(3, heads * hd, generator=gen) * 0.5).to(dt).to(DEV)
+    sink = torch.randn(heads, generator=gen).to(DEV)
+    gate = torch.randn(3, heads * (hd - 16 if span else 1), generator=gen).to(DEV)
+    partial = torch.full((3 * heads * runs, hd + 2), float("nan"), device=DEV) if runs > 1 else None
+
+    def attend(**more):
+        out = torch.full((3, heads * hd), float("nan"), dtype=torch.float32 if "gate" in more else dt, device=DEV)
+        args = K.attention_args(q, out, case.view(), case.tok_seq, case.tok_pos, case.seq_off, case.seq_start, heads, 3, 1, 0.3, 0, partial,
+                                sink=sink, **more)
+        K.attention(args, dt, decode=True)
+        return out.cpu().double().view(3, heads, hd)
+    plain = attend()
+    factor = torch.sigmoid(gate.cpu().double()).view(3, heads, -1)
+    if span:
+        factor = torch.cat([factor, torch.ones(3, heads, 16, dtype=torch.float64)], -1)
+    gated = attend(gate=gate, gate_dim=hd - 16 if span else 0)
+    assert bool(((gated - plain * factor).abs() <= 2.0 ** -8 * plain.abs() + 1e-6).all())       # the rounding of the row without a gate
