@@ -51,6 +51,11 @@ __device__ __forceinline__ float output_gate(const AttnArgs& a, int64_t tok, int
   return STAGED ? bt_output_gate(a, tok, head, channel) : 1.f;
 }
 
+// The factor from its logit (bt_output_logit), asked for long before.
+__device__ __forceinline__ float gate_factor(const AttnArgs& a, int channel, float logit) {
+  return STAGED && a.gate && !(a.gate_span == 1 && channel >= a.gate_dim) ? bt_sigmoid(logit) : 1.f;
+}
+
 #define F32M_QUERIES 64
 
 template <int HD>
@@ -253,30 +258,46 @@ attention_f32_mfma_kernel(AttnArgs a) {
 // One token per sequence (a decode step): the tiled kernel above would give each work-group a
 // single query and leave three of its four waves only the staging.  Here a work-group still
 // takes one (sequence, head), but its four waves take the blocks of 64 keys in turn and read them
-// straight from the cache: scores with lane = key (a lane reads its own key's row, the query comes
-// from LDS as a broadcast), the block's softmax statistics as wave reductions, values with lane =
-// channel (four keys per 16-byte read, as the cache lays them out; the probabilities come back
-// from LDS as broadcasts).  The four waves' running results meet in LDS at the end.
+// straight from the cache.  A load of keys is four whole rows, sixteen lanes each: a lane multiplies the four channels it has
+// (or twice four) by the query's, which it keeps, and the sixteen lanes of a row add up without LDS; lane 16 g + i then keeps the
+// score of key 4 i + g.  (With a row a lane every load touched 64 rows, 16 bytes of each, 64 KiB of them at a time through an
+// L1 of 32.)  The block's softmax statistics are wave reductions; values come with lane = channel (four keys per 16-byte
+// read, as the cache lays them out; the probabilities come back from LDS as broadcasts) and are asked for together with the keys
+// where the registers allow.  The four waves' running results meet in LDS at the end.  12 heads of 64, four sequences of up to 1,000
+// tokens in four runs, us with the kernel that joins them: 12.8 with a row a lane and a value after the other, 10.3 so.
 template <int CPT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 attention_f32_decode_kernel(AttnArgs a) {
   constexpr int MAX_HD = 64 * CPT;
-  __shared__ __attribute__((aligned(16))) float qs[MAX_HD];
   __shared__ __attribute__((aligned(16))) float ps[4][BT_KV_BLOCK];
   __shared__ float part_max[4], part_sum[4];
   __shared__ __attribute__((aligned(16))) float part_acc[4][MAX_HD];
   const int hd = a.kv.head_dim;
   const int seq = blockIdx.x, head = blockIdx.y, kv_head = head / (a.q_heads / a.kv.kv_heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int* block_row = a.kv.blocks + (int64_t)seq * a.kv.max_blocks;
+  const int held_blocks = block_row[lane < a.kv.max_blocks ? lane : a.kv.max_blocks - 1];     // (one trip with the position)
   const int pos = a.seq_start[seq];                     // the query's position: token `seq` of the step
   const float* q = static_cast<const float*>(a.q) + (int64_t)seq * a.ldq + head * hd;
-  if (tid < hd) qs[tid] = q[tid];
-  __syncthreads();
+  const int splits = a.splits > 1 ? a.splits : 1, split = blockIdx.z;
+  int channels[CPT];                                    // the first of the lane's four channels of a key (beyond the head: 0)
+  bool real[CPT];
+  float4 qv[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; ++j) {
+    real[j] = 4 * (l16 + 16 * j) < hd;
+    channels[j] = real[j] ? 4 * (l16 + 16 * j) : 0;
+    qv[j] = *reinterpret_cast<const float4*>(q + channels[j]);
+  }
+  float gate[CPT];
+#pragma unroll
+  for (int j = 0; j < CPT; ++j) gate[j] = STAGED && splits == 1 ? bt_output_logit(a, seq, head, lane + 64 * j) : 0.f;
+  const float sink = a.sink && splits == 1 ? a.sink[head] : 0.f;
   const int lo = bt_first_seen(pos, a.window, a.chunk);
   const KeyWalk walk = bt_key_walk(lo / BT_KV_BLOCK, (a.keep + BT_KV_BLOCK - 1) / BT_KV_BLOCK, 1);      // (in blocks)
   const SeenKeys sees = bt_seen_keys(pos, lo, a.keep);
   int first_place = 0, last_place = walk.places(pos / BT_KV_BLOCK);
-  const int splits = a.splits > 1 ? a.splits : 1, split = blockIdx.z;
   if (splits > 1) {       // this work-group's run of the blocks (it may be empty)
     const int per_split = (last_place + splits) / splits;
     first_place += split * per_split;
@@ -285,31 +306,41 @@ attention_f32_decode_kernel(AttnArgs a) {
   const float* keys = static_cast<const float*>(a.kv.keys);
   const float* values = static_cast<const float*>(a.kv.values);
   const float bias = FORM == 2 && a.score_bias ? a.score_bias[head] : 0.f;
-  float run_max = FIRST_MAXIMUM, run_sum = 0.f, acc[CPT];
+  float run_max = FIRST_MAXIMUM, run_sum = 0.f;
+  floatx4 four[CPT];         // of a channel, of every fourth key: chains a quarter as long
 #pragma unroll
-  for (int j = 0; j < CPT; ++j) acc[j] = 0.f;
+  for (int j = 0; j < CPT; ++j) four[j] = floatx4{0.f, 0.f, 0.f, 0.f};
   for (int place = first_place + wave; place <= last_place; place += 4) {
     const int block = walk.at(place);
-    int physical = a.kv.blocks[(int64_t)seq * a.kv.max_blocks + block];
-    int64_t base = kv_plane(a.kv, physical, kv_head);
-    // this lane's key: row `lane` of the block
-    const float4* krow = reinterpret_cast<const float4*>(keys + base + (int64_t)lane * hd);
-    const int quads = hd >> 2;
-    float4 kreg[16 * CPT];                     // the whole row in flight at once: one trip to memory, not sixteen
+    const int physical = block < 64 ? __builtin_amdgcn_readlane(held_blocks, block) : block_row[block];
+    const int64_t base = kv_plane(a.kv, physical, kv_head);
+    const float *kblock = keys + base, *vblock = values + base;
+    float4 kreg[CPT][16], vreg[BT_KV_BLOCK / 4];
 #pragma unroll
-    for (int c4 = 0; c4 < 16 * CPT; ++c4) kreg[c4] = krow[c4 < quads ? c4 : 0];
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) kreg[j][i] = *reinterpret_cast<const float4*>(kblock + (4 * i + g) * hd + channels[j]);
+    auto fetch_values = [&](int j) {        // the 64 values of channel lane + 64 j
+      const int cc = lane + 64 * j < hd ? lane + 64 * j : 0;
+#pragma unroll
+      for (int k4 = 0; k4 < BT_KV_BLOCK / 4; ++k4) vreg[k4] = *reinterpret_cast<const float4*>(vblock + (k4 * hd + cc) * 4);
+    };
+    if (CPT == 1) fetch_values(0);
     float s = 0.f;
 #pragma unroll
-    for (int c4 = 0; c4 < 16 * CPT; ++c4) {
-      if (c4 < quads) {
-        float4 q4 = *reinterpret_cast<const float4*>(qs + c4 * 4);
-        s = fmaf(q4.x, kreg[c4].x, s);
-        s = fmaf(q4.y, kreg[c4].y, s);
-        s = fmaf(q4.z, kreg[c4].z, s);
-        s = fmaf(q4.w, kreg[c4].w, s);
+    for (int i = 0; i < 16; ++i) {
+      float dot = 0.f;
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) {
+        const float4 k4 = kreg[j][i];
+        const float four = fmaf(qv[j].w, k4.w, fmaf(qv[j].z, k4.z, fmaf(qv[j].y, k4.y, qv[j].x * k4.x)));
+        dot += real[j] ? four : 0.f;
       }
+      dot = row_reduce(dot, LaneSum());
+      s = l16 == i ? dot : s;
     }
-    const bool seen = sees(block * BT_KV_BLOCK + lane);
+    const int in_block = 4 * l16 + g;
+    const bool seen = sees(block * BT_KV_BLOCK + in_block);
     float p, rescale = 1.f;
     if constexpr (FORM == 2) {
       p = seen ? bt_sigmoid(fmaf(s, a.scale, bias)) : 0.f;
@@ -322,28 +353,23 @@ attention_f32_decode_kernel(AttnArgs a) {
       run_sum = fmaf(run_sum, rescale, wave_sum(p));
       run_max = new_max;
     }
-    ps[wave][lane] = p;                                             // read back below by this wave only
+    ps[wave][in_block] = p;                                         // read back below by this wave only
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) acc[j] *= rescale;
+    for (int j = 0; j < CPT; ++j) four[j] *= rescale;
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-      const int channel = lane + 64 * j;
-      const int cc = channel < hd ? channel : 0;
-      float4 vreg[BT_KV_BLOCK / 4];            // the channel's 64 values in flight at once
-#pragma unroll
-      for (int k4 = 0; k4 < BT_KV_BLOCK / 4; ++k4)
-        vreg[k4] = *reinterpret_cast<const float4*>(values + base + (int64_t)(k4 * hd + cc) * 4);
+      if (CPT > 1) fetch_values(j);
 #pragma unroll
       for (int k4 = 0; k4 < BT_KV_BLOCK / 4; ++k4) {
         float4 p4 = *reinterpret_cast<const float4*>(&ps[wave][k4 * 4]);
         // a position that holds no token yet may hold anything (0 * NaN is NaN): not multiplied
-        acc[j] = p4.x != 0.f ? fmaf(p4.x, vreg[k4].x, acc[j]) : acc[j];
-        acc[j] = p4.y != 0.f ? fmaf(p4.y, vreg[k4].y, acc[j]) : acc[j];
-        acc[j] = p4.z != 0.f ? fmaf(p4.z, vreg[k4].z, acc[j]) : acc[j];
-        acc[j] = p4.w != 0.f ? fmaf(p4.w, vreg[k4].w, acc[j]) : acc[j];
+        four[j][0] = p4.x != 0.f ? fmaf(p4.x, vreg[k4].x, four[j][0]) : four[j][0];
+        four[j][1] = p4.y != 0.f ? fmaf(p4.y, vreg[k4].y, four[j][1]) : four[j][1];
+        four[j][2] = p4.z != 0.f ? fmaf(p4.z, vreg[k4].z, four[j][2]) : four[j][2];
+        four[j][3] = p4.w != 0.f ? fmaf(p4.w, vreg[k4].w, four[j][3]) : four[j][3];
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");          // the probabilities are overwritten next turn
@@ -355,7 +381,7 @@ attention_f32_decode_kernel(AttnArgs a) {
   }
 #pragma unroll
   for (int j = 0; j < CPT; ++j)
-    if (lane + 64 * j < hd) part_acc[wave][lane + 64 * j] = acc[j];
+    if (lane + 64 * j < hd) part_acc[wave][lane + 64 * j] = (four[j][0] + four[j][1]) + (four[j][2] + four[j][3]);
   __syncthreads();
   if (wave == 0) {
     float top = fmaxf(fmaxf(part_max[0], part_max[1]), fmaxf(part_max[2], part_max[3]));
@@ -373,8 +399,8 @@ attention_f32_decode_kernel(AttnArgs a) {
         den = fmaf(part_sum[w], f, den);
       }
       if (splits == 1) {
-        den += bt_sink_term(a.sink, head, top);
-        out[channel] = (FORM == 2 ? num : den > 0.f ? num / den : 0.f) * output_gate(a, seq, head, channel);
+        den += a.sink ? expf(sink - top) : 0.f;
+        out[channel] = (FORM == 2 ? num : den > 0.f ? num / den : 0.f) * gate_factor(a, channel, gate[j]);
       } else {                                                      // this run's share, for attention_f32_join_kernel
         mine[channel] = num;
         if (channel == 0) {
@@ -386,25 +412,50 @@ attention_f32_decode_kernel(AttnArgs a) {
   }
 }
 
-// Joins the runs of attention_f32_decode_kernel: a work-group of one wave per (sequence, head).
+// Joins the runs of attention_f32_decode_kernel: a work-group of one wave per (sequence, head).  The records of eight runs are asked for
+// together.
 __global__ void __launch_bounds__(64)
 attention_f32_join_kernel(AttnArgs a) {
-  const int hd = a.kv.head_dim;
+  const int hd = a.kv.head_dim, pitch = hd + 2;
   const int seq = blockIdx.x / a.q_heads, head = blockIdx.x % a.q_heads;
-  const float* runs = a.partial + ((int64_t)seq * a.q_heads + head) * a.splits * (hd + 2);
-  float top = -INFINITY;
-  for (int s = 0; s < a.splits; ++s) top = fmaxf(top, runs[s * (hd + 2) + hd]);
+  const float* runs = a.partial + ((int64_t)seq * a.q_heads + head) * a.splits * pitch;
+  const float sink = a.sink ? a.sink[head] : 0.f;
   float* out = static_cast<float*>(a.out) + (int64_t)seq * a.ldo + head * hd;
   for (int channel = threadIdx.x; channel < hd; channel += 64) {
-    float num = 0.f, den = 0.f;
-    for (int s = 0; s < a.splits; ++s) {                            // an empty run: maximum -inf, weight 0
-      float run_top = runs[s * (hd + 2) + hd];
-      float f = run_top == -INFINITY ? 0.f : expf(run_top - top);
-      num = fmaf(runs[s * (hd + 2) + channel], f, num);
-      den = fmaf(runs[s * (hd + 2) + hd + 1], f, den);
+    const float gate = STAGED ? bt_output_logit(a, seq, head, channel) : 0.f;
+    float m[8], l[8], o[8], top = -INFINITY;
+    auto ask = [&](int s0, bool all) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float* record = runs + (int64_t)(s0 + j < a.splits ? s0 + j : s0) * pitch;
+        m[j] = record[hd];
+        if (all) l[j] = record[hd + 1];
+        if (all) o[j] = record[channel];
+      }
+    };
+    for (int s0 = a.splits > 8 ? 8 : 0; s0 < a.splits; s0 += 8) {       // (the first eight last: they stay in registers if they are all)
+      ask(s0, a.splits <= 8);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) top = fmaxf(top, m[j]);
     }
-    den += bt_sink_term(a.sink, head, top);
-    out[channel] = (FORM == 2 ? num : den > 0.f ? num / den : 0.f) * output_gate(a, seq, head, channel);
+    if (a.splits > 8) {
+      ask(0, true);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) top = fmaxf(top, m[j]);
+    }
+    float num = 0.f, den = 0.f;
+    for (int s0 = 0; s0 < a.splits; s0 += 8) {
+      if (s0 > 0) ask(s0, true);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (s0 + j < a.splits) {                                    // an empty run: maximum -inf, weight 0
+          const float f = m[j] == -INFINITY ? 0.f : expf(m[j] - top);
+          num = fmaf(o[j], f, num);
+          den = fmaf(l[j], f, den);
+        }
+    }
+    den += a.sink ? expf(sink - top) : 0.f;
+    out[channel] = (FORM == 2 ? num : den > 0.f ? num / den : 0.f) * gate_factor(a, channel, gate);
   }
 }
 
