@@ -1101,11 +1101,6 @@ attention_prefill_wide_kernel(AttnArgs a) {
 // reduction overlaps the other's loads (57 -> 42 us).
 #define DECODE_WAVES 8
 
-template <int N>
-struct Shares {
-  static constexpr int value = N;
-};
-
 // KEEPS: some first positions stay visible beside a window or a chunk (a form of its own: the walk over two stretches of keys
 // and its test cost the other 0.3 us of 6.5).
 template <bool KEEPS>
@@ -1244,10 +1239,10 @@ attention_decode_kernel(AttnArgs a) {
       }
     }
   };
-  if (shares == 1) gather(Shares<1>());
-  else if (shares == 2) gather(Shares<2>());
-  else if (shares == 4) gather(Shares<4>());
-  else gather(Shares<DECODE_WAVES>());
+  if (shares == 1) gather(Constant<1>());
+  else if (shares == 2) gather(Constant<2>());
+  else if (shares == 4) gather(Constant<4>());
+  else gather(Constant<DECODE_WAVES>());
 }
 
 // Joins the runs of attention_decode_kernel (a row is a sequence's one token) or of

@@ -31,6 +31,12 @@ int bt_check_launch(const char* what);
     return BT_REFUSED;            \
   } while (0)
 
+// A number as a type: what a choice made once hands to the code that is compiled for it.
+template <int N>
+struct Constant {
+  static constexpr int value = N;
+};
+
 __device__ __forceinline__ float to_float(float v) { return v; }
 __device__ __forceinline__ float to_float(bf16_t v) { return (float)v; }
 

@@ -60,17 +60,24 @@ struct Epilogue {
 // (0.5 (1 + tanh u) = 1 / (1 + exp(-2u))) evaluated with the hardware exponential: its error
 // (a few ulp of float32) is far below the rounding of the bfloat16 result, and it is a handful of
 // instructions instead of some forty for each of the millions of elements a prefill produces.
-template <typename T>
-__device__ __forceinline__ float activate(float x, int act) {
-  if (act == ACT_GELU_TANH) {
+template <typename T, int ACT>
+__device__ __forceinline__ float activate_as(float x) {
+  if constexpr (ACT == ACT_GELU_TANH) {
     // 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3)))
     float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
     if (sizeof(T) == 2) return x / (1.0f + __expf(-2.0f * inner));
     return 0.5f * x * (1.0f + tanhf(inner));
+  } else if constexpr (ACT == ACT_SQUARED_RELU) {
+    return x > 0.f ? x * x : 0.f;
+  } else {
+    // x (1 + erf(x / sqrt 2)) / 2
+    return 0.5f * x * (1.0f + erff(x * 0.7071067811865476f));
   }
-  if (act == ACT_SQUARED_RELU) return x > 0.f ? x * x : 0.f;
-  // x (1 + erf(x / sqrt 2)) / 2
-  return 0.5f * x * (1.0f + erff(x * 0.7071067811865476f));
+}
+template <typename T>
+__device__ __forceinline__ float activate(float x, int act) {
+  return act == ACT_GELU_TANH ? activate_as<T, ACT_GELU_TANH>(x) : act == ACT_SQUARED_RELU ? activate_as<T, ACT_SQUARED_RELU>(x)
+                                                                                            : activate_as<T, ACT_GELU_ERF>(x);
 }
 
 template <typename T>
@@ -374,12 +381,19 @@ __device__ __forceinline__ void epilogue_tile(const Epilogue& e, int M, int N, i
         for (int r = 0; r < 16; ++r) acc[bn][bm][r] += b[bn][r >> 2][r & 3];
   }
   if (e.mode == EPI_ACT) {
+    // (one choice for all values: with the choice at every value the code of every activation lay between each two of them, 64 KiB
+    // for 128 x 256, and fetching it took 2.6 to 5 us of a work-group's epilogue)
+    auto all = [&](auto act) {
 #pragma unroll
-    for (int bn = 0; bn < TN; ++bn)
+      for (int bn = 0; bn < TN; ++bn)
 #pragma unroll
-      for (int bm = 0; bm < TM; ++bm)
+        for (int bm = 0; bm < TM; ++bm)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[bn][bm][r] = activate<T>(acc[bn][bm][r], e.act);
+          for (int r = 0; r < 16; ++r) acc[bn][bm][r] = activate_as<T, decltype(act)::value>(acc[bn][bm][r]);
+    };
+    if (e.act == ACT_GELU_TANH) all(Constant<ACT_GELU_TANH>());
+    else if (e.act == ACT_SQUARED_RELU) all(Constant<ACT_SQUARED_RELU>());
+    else all(Constant<ACT_GELU_ERF>());
   }
   if (values) {          // four positions lie interleaved: every lane stores its own row's channels, 8 bytes of a line for four rows
     const int c = kv_column - e.n_kv, head = c / e.kv.head_dim;

@@ -387,18 +387,26 @@ struct GatedExpertsCall {
   float alpha;
 };
 
-__device__ __forceinline__ float plain_unit(const GatedExpertsCall& c, float u) {
-  if (c.act == 4) return u > 0.f ? u * u : 0.f;
-  return c.act == 2 ? 0.5f * u * (1.0f + erff(u * 0.70710678118654752f)) : u / (1.0f + expf(-u));
+template <int ACT>
+__device__ __forceinline__ float plain_unit_as(float u) {
+  if constexpr (ACT == 4) return u > 0.f ? u * u : 0.f;
+  else if constexpr (ACT == 2) return 0.5f * u * (1.0f + erff(u * 0.70710678118654752f));
+  else return u / (1.0f + expf(-u));
 }
-
-__device__ __forceinline__ float gated_unit(const GatedExpertsCall& c, float g, float u) {
-  if (c.act == 1) {
-    g = fminf(g, c.limit);
-    u = fminf(fmaxf(u, -c.limit), c.limit);
-    return g / (1.0f + expf(-c.alpha * g)) * (u + 1.0f);
+template <int ACT>
+__device__ __forceinline__ float gated_unit_as(float limit, float alpha, float g, float u) {
+  if constexpr (ACT == 1) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
   }
   return g / (1.0f + expf(-g)) * u;
+}
+__device__ __forceinline__ float plain_unit(const GatedExpertsCall& c, float u) {
+  return c.act == 4 ? plain_unit_as<4>(u) : c.act == 2 ? plain_unit_as<2>(u) : plain_unit_as<3>(u);
+}
+__device__ __forceinline__ float gated_unit(const GatedExpertsCall& c, float g, float u) {
+  return c.act == 1 ? gated_unit_as<1>(c.limit, c.alpha, g, u) : gated_unit_as<0>(c.limit, c.alpha, g, u);
 }
 
 template <typename T>
@@ -733,26 +741,36 @@ __global__ void __launch_bounds__(256, 2) expert_products_kernel(ExpertProductsC
   typedef typename std::conditional<SECOND, float, T>::type Out;
   constexpr int COLUMNS = HELD / 2, PIECE = 16 / (int)sizeof(Out), LANES = COLUMNS / PIECE, PITCH = COLUMNS * (int)sizeof(Out) + 16;
   unsigned char* scratch = lds + wave * (BM / 2 * PITCH);
-  GatedExpertsCall unit;
-  unit.act = c.act;
-  unit.limit = c.limit;
-  unit.alpha = c.alpha;
+  auto units = [&](auto act) {
+    constexpr int ACT = decltype(act)::value;
 #pragma unroll
-  for (int bm = 0; bm < TM; ++bm)
+    for (int bm = 0; bm < TM; ++bm)
 #pragma unroll
-    for (int bn = 0; bn < COLUMNS / 32; ++bn)
+      for (int bn = 0; bn < COLUMNS / 32; ++bn)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        typedef __attribute__((__vector_size__(4 * sizeof(Out)))) Out Out4;
-        Out4 v;
+        for (int q = 0; q < 4; ++q) {
+          typedef __attribute__((__vector_size__(4 * sizeof(Out)))) Out Out4;
+          Out4 v;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (SECOND) v[i] = acc[bn][bm][4 * q + i];
-          else v[i] = from_float<T>(weight[bm] * (GATED ? gated_unit(unit, acc[0][bm][4 * q + i], acc[1][bm][4 * q + i])
-                                                        : plain_unit(unit, acc[bn][bm][4 * q + i])));
+          for (int i = 0; i < 4; ++i) {
+            if constexpr (SECOND) v[i] = acc[bn][bm][4 * q + i];
+            else if constexpr (GATED) v[i] = from_float<T>(weight[bm] * gated_unit_as<ACT>(c.limit, c.alpha, acc[0][bm][4 * q + i], acc[1][bm][4 * q + i]));
+            else v[i] = from_float<T>(weight[bm] * plain_unit_as<ACT>(acc[bn][bm][4 * q + i]));
+          }
+          *reinterpret_cast<Out4*>(scratch + (bm * 32 + l32) * PITCH + (bn * 32 + q * 8 + g * 4) * (int)sizeof(Out)) = v;
         }
-        *reinterpret_cast<Out4*>(scratch + (bm * 32 + l32) * PITCH + (bn * 32 + q * 8 + g * 4) * (int)sizeof(Out)) = v;
-      }
+  };
+  // (one choice for all values: with the choice at every value all units' code lay between each two of them)
+  if constexpr (SECOND) {
+    units(Constant<0>());
+  } else if constexpr (GATED) {
+    if (c.act == 1) units(Constant<1>());
+    else units(Constant<0>());
+  } else {
+    if (c.act == 4) units(Constant<4>());
+    else if (c.act == 2) units(Constant<2>());
+    else units(Constant<3>());
+  }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (a wave's accesses of LDS are served in order)
   const int n = n_base + wn * COLUMNS + lane % LANES * PIECE;
   constexpr int TURNS = BM / 2 * LANES / 64;
