@@ -914,7 +914,16 @@ static void launch_skinny(hipStream_t s, const T* a, int64_t lda, const T* w, in
     if (per_wave <= 4) {
       if (columns <= 16) LAUNCH_SKINNY(1, 1, 4, 1, 1); else LAUNCH_SKINNY(1, 2, 4, 1, 1);
     } else if (M <= 4) {
-      if (columns == 8) LAUNCH_SKINNY(1, 1, 8, 4, 2); else if (columns <= 16) LAUNCH_SKINNY(1, 1, 8, 4, 1); else LAUNCH_SKINNY(1, 2, 8, 4, 1);
+      // (up to twelve chunks a wave in one batch: 768 x 3072, one row 4.26 -> 4.04 us; four rows 1024 x 9216 in four slices 6.1 -> 5.7)
+      if (columns <= 16 && per_wave > 8 && per_wave <= 12) {
+        if (columns == 8) LAUNCH_SKINNY(1, 1, 12, 4, 2); else LAUNCH_SKINNY(1, 1, 12, 4, 1);
+      } else if (columns == 8) {
+        LAUNCH_SKINNY(1, 1, 8, 4, 2);
+      } else if (columns <= 16) {
+        LAUNCH_SKINNY(1, 1, 8, 4, 1);
+      } else {
+        LAUNCH_SKINNY(1, 2, 8, 4, 1);
+      }
     } else if (M <= 8) {
       if (columns == 8) LAUNCH_SKINNY(1, 1, 8, 2, 2); else if (columns <= 16) LAUNCH_SKINNY(1, 1, 8, 2, 1); else LAUNCH_SKINNY(1, 2, 8, 2, 1);
     } else {
