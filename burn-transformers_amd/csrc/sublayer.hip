@@ -105,7 +105,8 @@ __global__ void __launch_bounds__(256) output_norm_kernel(OutputNormCall c) {
 // A thread's columns are KMAX / 4 quads of neighbours, a load for each (QUADS), or lie 256 apart where the rows are no whole
 // quads.  What bounds it is the chain of a row: its loads, two sums over the work-group, its stores.  With two partial sums and
 // the next norm, one column a load / quads (us, in a HIP graph): 8 rows of 2,048 4.44 / 3.75, of 1,024 3.54 / 3.18; 773 of 2,048
-// 7.86 / 7.35; 1,809 of 1,024 with four partial sums 9.28 / 8.89.
+// 7.86 / 7.35; 1,809 of 1,024 with four partial sums 9.28 / 8.89.  Since then shorter sums over a wave (8 rows of 2,048 3.42) and only what is
+// there read, the call's fields asked for together (3.24).
 template <int KMAX, bool QUADS>
 struct RowColumns {
   __device__ __forceinline__ static int column(int k) {
@@ -173,46 +174,56 @@ __global__ void __launch_bounds__(256) output_norm_small_kernel(OutputNormCall c
   __shared__ __attribute__((aligned(16))) float row_buf[QUADS ? 256 * KMAX : 4];
   const int t = blockIdx.x;
   float* xr = c.x + (int64_t)t * c.width;
-  // Every load of a thread is issued before the first is used and none stands behind a branch of its
-  // own (columns beyond the row and partial sums beyond the last are read from a valid place and
-  // dropped): loads behind branches, or in a loop of unknown length, are waited for one by one, and
-  // a row then costs as many round trips to memory as it has of them (measured: 14 us for 16 of them).
-  float v[KMAX], xv[KMAX], g[KMAX], b[KMAX], g2[KMAX], b2[KMAX];
+  // Every load of a thread is issued before the first is used and none waits for another (columns beyond the row are read from a
+  // valid place and dropped).  What is not there is not read: a wave's load of sixteen bytes a lane takes a compute unit 16
+  // cycles whatever it brings.  Those behind a branch (the same for every thread) stand first, the sum's own then, and last, in any case, what is
+  // used behind the sum: so the wait for the sum's operands counts what is behind them and lets it come meanwhile.
+  float v[KMAX], xv[KMAX], g[KMAX], b[KMAX], g2[KMAX], b2[KMAX], part[4][KMAX];
   bool in_row[KMAX];
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) in_row[k] = Columns::column(k) < c.width;
-  Columns::load(c.next_out ? c.next_gamma : c.gamma, c.width, g2);
-  Columns::load(c.next_out && c.next_beta ? c.next_beta : c.gamma, c.width, b2);
-  Columns::load(c.gamma, c.width, g);
-  Columns::load(c.beta ? c.beta : c.gamma, c.width, b);          // (read in any case, used only where there is one)
+  for (int k = 0; k < KMAX; ++k) {
+    in_row[k] = Columns::column(k) < c.width;
+    v[k] = b[k] = b2[k] = g2[k] = part[2][k] = part[3][k] = 0.f;
+  }
+  // (the call's fields together at the start: the ones a branch asks for would be waited for in it)
+  asm volatile("" ::"s"(c.bias), "s"(c.beta), "s"(c.gamma), "s"(c.cast), "s"(c.next_out), "s"(c.next_gamma), "s"(c.next_beta), "s"(c.delta),
+               "s"(c.delta_stride), "s"(c.ldd), "s"(c.kind), "s"(c.next_kind));
+  const float* row = c.n_delta ? c.delta + (int64_t)t * c.ldd : xr;
+  if (c.beta) Columns::load(c.beta, c.width, b);
+  if (c.next_out) {
+    Columns::load(c.next_gamma, c.width, g2);
+    if (c.next_beta) Columns::load(c.next_beta, c.width, b2);
+  }
+  if (c.n_delta && c.bias) Columns::load(c.bias, c.width, v);
+  if (c.n_delta > 2) {
+    Columns::load(row + 2 * c.delta_stride, c.width, part[2]);
+    Columns::load(row + (c.n_delta > 3 ? 3 : 2) * c.delta_stride, c.width, part[3]);
+  }
+  Columns::load(row, c.width, part[0]);
+  Columns::load(row + (c.n_delta > 1 ? c.delta_stride : 0), c.width, part[1]);
   Columns::load(xr, c.width, xv);
-  Columns::load(c.bias ? c.bias : c.gamma, c.width, v);
+  Columns::load(c.gamma, c.width, g);
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     b[k] = c.beta ? c.mult * b[k] : 0.f;
-    v[k] = c.bias ? v[k] : 0.f;
+    v[k] += part[0][k];
+    v[k] += c.n_delta > 1 ? part[1][k] : 0.f;
+    v[k] += part[2][k];
+    v[k] += c.n_delta > 3 ? part[3][k] : 0.f;
   }
-  if (c.n_delta == 0) {
+  for (int s0 = 4; s0 < c.n_delta; s0 += 4) {              // four partial sums at a time, all their loads together
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) { v[k] = xv[k]; xv[k] = 0.f; }
-  } else {
-    const float* row = c.delta + (int64_t)t * c.ldd;
-    for (int s0 = 0; s0 < c.n_delta; s0 += 4) {            // four partial sums at a time, all their loads together
-      float part[4][KMAX];
+    for (int u = 0; u < 4; ++u) Columns::load(row + (s0 + u < c.n_delta ? s0 + u : c.n_delta - 1) * c.delta_stride, c.width, part[u]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) Columns::load(row + (s0 + u < c.n_delta ? s0 + u : c.n_delta - 1) * c.delta_stride, c.width, part[u]);
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int k = 0; k < KMAX; ++k) v[k] += s0 + u < c.n_delta ? part[u][k] : 0.f;
-    }
-    if (!c.accumulate)
-#pragma unroll
-      for (int k = 0; k < KMAX; ++k) xv[k] = 0.f;
+      for (int k = 0; k < KMAX; ++k) v[k] += s0 + u < c.n_delta ? part[u][k] : 0.f;
   }
+  if (!c.accumulate)
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k)
-    if (!in_row[k]) v[k] = xv[k] = g[k] = b[k] = 0.f;
+    for (int k = 0; k < KMAX; ++k) xv[k] = 0.f;
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) v[k] = in_row[k] ? v[k] : 0.f;
   float w[KMAX], partial = 0.f;
   Columns::apart(v, row_buf, w);
   if (c.kind == 0) {          // a layer norm: the mean first, then the squared distances from it
