@@ -52,13 +52,122 @@ struct RouteEarly {
   float correction[4], bias[4];
   __device__ __forceinline__ void load(const RouteCall& c) {
     const int lane = threadIdx.x & 63;
+    correction[0] = c.correction && lane < c.experts ? c.correction[lane] : 0.f;
+    bias[0] = c.bias && lane < c.experts ? c.bias[lane] : 0.f;
+    if (c.experts <= 64) return;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 1; j < 4; ++j) {
       correction[j] = c.correction && lane + 64 * j < c.experts ? c.correction[lane + 64 * j] : 0.f;
       bias[j] = c.bias && lane + 64 * j < c.experts ? c.bias[lane + 64 * j] : 0.f;
     }
   }
 };
+
+// The groups that stay open, of lane g group g: the best `keep` by their scores.  `choice` holds the corrected scores in LDS.
+__device__ __forceinline__ bool route_group_open(const RouteCall& c, const float* choice) {
+  const int lane = threadIdx.x & 63;
+  // a group's score is its best corrected score; the best `keep` groups stay open, the experts of
+  // the others are shut out (minus infinity, since corrected scores may be negative).  Lane g
+  // holds group g (at most 64 groups).
+  const int per = c.experts / c.groups;
+  float group_score = -INFINITY;
+  if (lane < c.groups) {
+    if (c.group_rank <= 1) {
+      for (int i = 0; i < per; ++i) group_score = fmaxf(group_score, choice[lane * per + i]);
+    } else {
+      // the sum of the group's `group_rank` best: best after best, each below the one before it or
+      // an equal one at a higher index
+      float last = INFINITY;
+      int last_index = -1;
+      group_score = 0.f;
+      for (int r = 0; r < c.group_rank && r < per; ++r) {
+        float best = -INFINITY;
+        int best_index = -1;
+        for (int i = 0; i < per; ++i) {
+          const float v = choice[lane * per + i];
+          const bool left = v < last || (v == last && i > last_index);
+          if (left && (best_index < 0 || v > best)) { best = v; best_index = i; }
+        }
+        group_score += best;
+        last = best;
+        last_index = best_index;
+      }
+    }
+  }
+  bool open = false;
+  for (int kept = 0; kept < c.keep; ++kept) {
+    float value = (lane < c.groups && !open) ? group_score : -INFINITY;
+    int index = (lane < c.groups && !open) ? lane : 0x7fffffff;
+    // (a group whose score is minus infinity itself still ranks before no group at all)
+    unsigned long long candidates = __builtin_amdgcn_ballot_w64(lane < c.groups && !open);
+    wave_best(value, index);
+    if (index == 0x7fffffff) index = __builtin_ctzll(candidates);
+    if (lane == index) open = true;
+  }
+  return open;
+}
+
+// From a token's logits to its experts, by ONE wave, for at most 64 experts: an expert a lane, `logit` its lane's.  What this takes is a chain of
+// reductions and of trips to LDS behind a product that is itself 2 us, so values stay in lanes: an expert's rank is the number of
+// lanes that go before it (their values read lane by lane, independent of each other), where choosing the best, `top` times over, is as many
+// reductions one after the other; these stay where the experts are many beside the chosen.
+// Measured (us, by reductions with everything in LDS / so): a decode step's weigh_experts of 4 and 8 tokens, 2 of 8 experts, 3.54 / 2.91.
+// `choice`: LDS of the wave, used by groups.  Returns the token's weight of the lane's expert, zero where it was not chosen or there is none.
+__device__ __forceinline__ float route_lanes(const RouteCall& c, const RouteEarly& early, float logit, float* choice) {
+  const int lane = threadIdx.x & 63;
+  const bool mine = lane < c.experts;
+  const float z = c.bias ? logit + early.bias[0] : logit;
+  float s;
+  if (c.score == 1) {
+    s = 1.0f / (1.0f + expf(-z));
+  } else {
+    const float top_logit = wave_max(mine ? fmaxf(-INFINITY, z) : -INFINITY);
+    s = expf(z - top_logit);
+    if (c.score == 0) s /= wave_sum(mine ? s : 0.f);
+  }
+  const float own = mine ? s : 0.f;
+  float corrected = mine ? (c.score == 2 ? z : s) + early.correction[0] : -INFINITY;
+  if (c.groups > 1) {
+    if (mine) choice[lane] = corrected;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const unsigned long long open = __builtin_amdgcn_ballot_w64(route_group_open(c, choice));
+    if (mine && !(open >> (lane / (c.experts / c.groups)) & 1)) corrected = -INFINITY;
+  }
+  const bool can = corrected > -INFINITY;          // (not minus infinity and a number: the others are never chosen)
+  const float value = can ? corrected : -INFINITY;
+  float sum = 0.f;
+  bool taken = false;
+  auto score_of = [&](int expert) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, own), expert)); };
+  if (c.experts <= 16 * c.top) {
+    int rank = 0;
+    for (int j0 = 0; j0 < c.experts; j0 += 8)
+#pragma unroll
+      for (int j = j0; j < j0 + 8; ++j) {          // (lanes behind the experts hold minus infinity, which goes before nothing)
+        const float other = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, value), j));
+        rank += other > value || (other == value && j < lane) ? 1 : 0;
+      }
+    taken = can && rank < c.top;
+    for (int k = 0; k < c.top; ++k) {
+      const unsigned long long at = __builtin_amdgcn_ballot_w64(can && rank == k);
+      if (at == 0) break;
+      sum += score_of(__builtin_ctzll(at));
+    }
+  } else {
+    for (int k = 0; k < c.top; ++k) {
+      const bool left = can && !taken;
+      float best = left ? value : -INFINITY;
+      int index = left ? lane : 0x7fffffff;
+      wave_best(best, index);
+      index = __builtin_amdgcn_readfirstlane(index);
+      if (index == 0x7fffffff) break;              // (nothing left)
+      if (lane == index) taken = true;
+      sum += score_of(index);
+    }
+  }
+  return taken ? own * (c.normalize ? 1.0f / (sum + 1e-20f) : 1.0f) : 0.f;
+}
 
 // From a token's logits to its experts, by ONE wave: the experts dealt to its lanes, maxima and choices as wave
 // reductions.  `score` holds the logits and afterwards the scores, `choice` afterwards the token's weight of every expert,
@@ -85,44 +194,8 @@ __device__ __forceinline__ float route_choice(const RouteCall& c, const RouteEar
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (c.groups > 1) {
-    // a group's score is its best corrected score; the best `keep` groups stay open, the experts of
-    // the others are shut out (minus infinity, since corrected scores may be negative).  Lane g
-    // holds group g (at most 64 groups).
     const int per = c.experts / c.groups;
-    float group_score = -INFINITY;
-    if (lane < c.groups) {
-      if (c.group_rank <= 1) {
-        for (int i = 0; i < per; ++i) group_score = fmaxf(group_score, choice[lane * per + i]);
-      } else {
-        // the sum of the group's `group_rank` best: best after best, each below the one before it or
-        // an equal one at a higher index
-        float last = INFINITY;
-        int last_index = -1;
-        group_score = 0.f;
-        for (int r = 0; r < c.group_rank && r < per; ++r) {
-          float best = -INFINITY;
-          int best_index = -1;
-          for (int i = 0; i < per; ++i) {
-            const float v = choice[lane * per + i];
-            const bool left = v < last || (v == last && i > last_index);
-            if (left && (best_index < 0 || v > best)) { best = v; best_index = i; }
-          }
-          group_score += best;
-          last = best;
-          last_index = best_index;
-        }
-      }
-    }
-    bool open = false;
-    for (int kept = 0; kept < c.keep; ++kept) {
-      float value = (lane < c.groups && !open) ? group_score : -INFINITY;
-      int index = (lane < c.groups && !open) ? lane : 0x7fffffff;
-      // (a group whose score is minus infinity itself still ranks before no group at all)
-      unsigned long long candidates = __builtin_amdgcn_ballot_w64(lane < c.groups && !open);
-      wave_best(value, index);
-      if (index == 0x7fffffff) index = __builtin_ctzll(candidates);
-      if (lane == index) open = true;
-    }
+    const bool open = route_group_open(c, choice);
     if (lane < c.groups && !open)
       for (int i = 0; i < per; ++i) choice[lane * per + i] = -INFINITY;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -130,22 +203,6 @@ __device__ __forceinline__ float route_choice(const RouteCall& c, const RouteEar
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   float sum = 0.f;
-  if (c.experts <= 64) {                           // (an expert a lane: nothing is read again while they are chosen)
-    const float own = lane < c.experts ? score[lane] : 0.f, corrected = lane < c.experts ? choice[lane] : -INFINITY;
-    bool taken = false;
-    for (int k = 0; k < c.top; ++k) {
-      const bool left = corrected > -INFINITY && !taken;
-      float value = left ? corrected : -INFINITY;
-      int index = left ? lane : 0x7fffffff;
-      wave_best(value, index);
-      if (index == 0x7fffffff) break;              // (nothing left above minus infinity, or what is left is not a number)
-      if (lane == index) taken = true;
-      sum += score[index];
-    }
-    const float weight = taken ? own * (c.normalize ? 1.0f / (sum + 1e-20f) : 1.0f) : 0.f;
-    if (lane < c.experts) choice[lane] = weight;
-    return weight;
-  }
   unsigned taken = 0;                              // bit j: the lane's expert lane + 64 j (ROUTE_MAX_EXPERTS: sixteen of them)
   for (int k = 0; k < c.top; ++k) {
     float value = -INFINITY;
@@ -229,7 +286,7 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
   }
   __syncthreads();
   if (wave != 0) return;
-  const float first = route_choice(c, early, score, choice);
+  const float first = c.experts <= 64 ? route_lanes(c, early, lane < c.experts ? score[lane] : 0.f, choice) : route_choice(c, early, score, choice);
   // the one store of a lane's experts: the chosen ones' scores over their sum, zero elsewhere
   float* weights = c.weights + (int64_t)t * c.experts;
   for (int e = lane; e < c.experts; e += 64) {
@@ -308,7 +365,7 @@ __global__ void __launch_bounds__(64 * ROUTE_ROWS) route_rows_kernel(RouteCall c
   const int t = t0 + wave;
   if (t >= c.tokens) return;
   const float gate_sum = score[wave][c.gate_w ? c.experts : 0];
-  const float w = route_choice(c, early, score[wave], choice[wave]);    // (zero behind the experts, of which there are at most 64)
+  const float w = route_lanes(c, early, lane < c.experts ? score[wave][lane] : 0.f, choice[wave]);
   if (lane < c.experts) c.weights[(int64_t)t * c.experts + lane] = w;
   const unsigned long long used = __builtin_amdgcn_ballot_w64(w != 0.f);
   if (lane == 0 && c.used) c.used[t] = used;
@@ -868,30 +925,44 @@ __global__ void __launch_bounds__(256) weigh_experts_kernel(WeighExpertsCall w) 
   int piece = blockIdx.y * blockDim.x + threadIdx.x;
   int4v held = {0, 0, 0, 0};
   if (whole && piece < pieces) held = *reinterpret_cast<const int4v*>(hidden + (int64_t)piece * PER);      // on its way during the choice
-  if (wave == 0) {
-    const float* logits = w.logits + (int64_t)t * w.ld_logits;
-    RouteEarly early;
-    early.load(c);
-    for (int e = lane; e < c.experts; e += 64) score[e] = logits[e];
-    route_choice(c, early, score, choice);
+  int expert = min(piece, pieces - 1) * PER / w.ff;   // (the division, too)
+  const float* logits = w.logits + (int64_t)t * w.ld_logits;
+  RouteEarly early;
+  early.load(c);
+  const float* weights = choice;
+  if (c.experts <= 64) {                           // (every wave for itself: none waits for another)
+    float* own = choice + 64 * wave;
+    const float weight = route_lanes(c, early, lane < c.experts ? logits[lane] : 0.f, own);
+    if (lane < c.experts) own[lane] = weight;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    weights = own;
+  } else {
+    if (wave == 0) {
+      for (int e = lane; e < c.experts; e += 64) score[e] = logits[e];
+      route_choice(c, early, score, choice);
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  auto weight = [&](int e) { return choice[e]; };
   if (!whole) {
     for (int col = piece; col < columns; col += gridDim.y * blockDim.x) {
-      const float f = weight(col / w.ff);
+      const float f = weights[col / w.ff];
       hidden[col] = from_float<T>(f != 0.f ? f * to_float(hidden[col]) : 0.f);
     }
     return;
   }
   for (; piece < pieces; piece += gridDim.y * blockDim.x) {
-    const float f = weight(piece * PER / w.ff);
+    const float f = weights[expert];
     T* values = reinterpret_cast<T*>(&held);
 #pragma unroll
     for (int i = 0; i < PER; ++i) values[i] = from_float<T>(f != 0.f ? f * to_float(values[i]) : 0.f);
     *reinterpret_cast<int4v*>(hidden + (int64_t)piece * PER) = held;
     const int next = piece + gridDim.y * blockDim.x;
-    if (next < pieces) held = *reinterpret_cast<const int4v*>(hidden + (int64_t)next * PER);
+    if (next < pieces) {
+      held = *reinterpret_cast<const int4v*>(hidden + (int64_t)next * PER);
+      expert = next * PER / w.ff;
+    }
   }
 }
 
