@@ -304,10 +304,11 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
 // outputs on the matrix units (v_mfma_f32_16x16x4_f32: h widened, the router's 32 bits as they are), its sixteen waves a
 // sixteenth of the columns each, so that the router is read once for sixteen tokens and not once a token; then every
 // wave makes the choice of one of them.  Of an instruction's four K values step i takes column 4 g + i of a lane group's
-// four, which are one read.  A work-group's own chain (two trips to memory, the sums' meeting, the choice) is 8 us whatever
-// the step, so steps of fewer than ROUTE_ROWS_MIN tokens keep a work-group a token.  Measured in a step (us, a work-group a token /
-// sixteen): 1,809 tokens of 1,024 columns, 9 outputs and a gate 15.3 / 10.7, 2,447 of 8 outputs 11.0 / 8.8; alone, 1,024 tokens 6.7 /
-// 8.3, 2,048 10.0 / 8.6, 4,096 15.1 / 8.7.
+// four, which are one read.  A work-group's own chain (two trips to memory, the sums' meeting, the choice) is 5 to
+// 7 us for 512 and 1,024 columns whatever the step, so steps of fewer than ROUTE_ROWS_MIN tokens keep a work-group a token.  Measured (us, a
+// work-group a token / sixteen; outputs of columns): 9 of 1,024 1,000 tokens 5.5 / 6.6, 1,200 6.5 / 6.6, 1,400 7.2 / 6.6, 1,530 7.4 / 6.6; 17 of 1,024 1,000
+// 7.8 / 8.7, 1,200 9.1 / 8.7, 1,530 10.4 / 8.7; 8 of 512 1,000 4.6 / 4.8, 1,200 4.9 / 4.8, 1,530 5.5 / 4.8; 32 of 2,048 600 15.3 / 15.3, 1,530 25.9 / 15.4.  In a step of
+// 1,809 tokens 9 outputs of 1,024 and a gate take 8.5.
 #define ROUTE_ROWS 16
 #define ROUTE_ROWS_TILES 2      // (most outputs: 32)
 #define ROUTE_ROWS_AHEAD 4      // chunks of 16 columns on their way
@@ -372,9 +373,9 @@ __global__ void __launch_bounds__(64 * ROUTE_ROWS) route_rows_kernel(RouteCall c
   if (lane == 0 && c.gate_w) c.gate[t] = 1.0f / (1.0f + expf(-gate_sum));
 }
 
-// (Few outputs of wide rows from 1,792 tokens on: 8 of 4,096 float columns 1,536 tokens 13.7 / 16.6, 1,800 16.3 / 16.9; of 4,096 bfloat16 ones 14.8 /
-// 16.5 and 17.9 / 16.9, of 1,024 7.9 / 8.1 and 9.4 / 8.2.)
-#define ROUTE_ROWS_MIN 1536
+// (Few outputs of wide rows from 1,792 tokens on: 8 of 1,024 bfloat16 columns 1,530 tokens 5.5 / 6.2, 1,780 6.0 / 6.2; of 4,096 1,530 13.8 / 14.7, 1,780 15.6 /
+// 14.8; of 4,096 float ones 13.3 / 14.9 and 14.5 / 14.8.)
+#define ROUTE_ROWS_MIN 1280
 #define ROUTE_ROWS_MIN_FEW 1792
 
 template <typename T>
