@@ -160,17 +160,21 @@ __global__ void __launch_bounds__(HR_WAVES * 64) head_rotary_kernel(HeadRotaryCa
 // barrier.  Taken for rows of whole pairs up to 128 channels.  Measured against the kernel above (us, above / this; 8 heads on 2 of 128, 64
 // channels turned, bfloat16, a norm a head): 512 tokens 5.3 / 4.9, 768 6.9 / 5.2, 1,024 8.2 / 5.4, 2,048 13.9 / 7.7.  What is left is the
 // sines (the angles reduced in 32 bits) and the values' stores of two bytes: bytes alone would take 3.4 us at 1,809 tokens.
-// Taken where there is enough to share, by the heads of all tokens: with one norm over all heads, which the kernel above works out once a
-// head, from 128 tokens on, elsewhere from 768.  Measured (us, the kernel above / this; queries on keys of channels, heads of all tokens in brackets): with that norm 8 on
-// 2 of 128 128 tokens (1,536) 3.6 / 4.8, 256 4.1 / 4.9, 512 (6,144) 5.6 / 5.0, 6 on 2 of 128 512 (5,120) 5.0 / 5.4, 768 6.4 / 5.9, 4 on 1 of 64 768 (4,608) 4.8 / 4.3, 2 on 1 of
-// 128 1,024 (4,096) 4.4 / 4.8, 1,536 (6,144) 5.5 / 5.0, 12 on 12 of 64 128 (4,608) 4.2 / 5.0, 192 (6,912) 5.2 / 5.2, 256 6.3 / 5.4; with a norm a head 2 on 1 of 128 1,280
+// Taken where there is enough to share: with one norm over all heads, which the kernel above works out once a head, from 128 tokens on
+// for rows of 1,024 query channels, and elsewhere, as without such a norm from 768 tokens on, by the heads of all tokens.  The two kernels add a norm's
+// squares in different orders (columns 64 apart, pairs 128 apart), so the lines with norms also say which sums a step has: they stay where they are even
+// where the kernel above is now the faster one.  Measured (us, the kernel above / this; queries on keys of channels, heads of all tokens in brackets): one norm over all
+// heads, 8 on 2 of 128 128 tokens 3.6 / 4.8, 256 4.1 / 4.9, 512 (6,144) 5.6 / 5.0, 6 on 2 of 128 512 (5,120) 5.0 / 5.4, 768 6.4 / 5.9, 4 on 1 of 64 768 (4,608) 4.8 / 4.3, 2 on 1 of
+// 128 1,024 (4,096) 4.4 / 4.8, 1,536 (6,144) 5.5 / 5.0, 12 on 12 of 64 128 (4,608) 4.2 / 5.0, 192 (6,912) 5.2 / 5.2, 256 6.3 / 5.4; a norm a head, 2 on 1 of 128 1,280
 // (5,120) 4.8 / 4.8, 1,536 (6,144) 5.3 / 4.8, 3 on 1 1,280 (6,400) 6.1 / 5.1, 4 on 4 of 32 512 (6,144) 4.5 / 4.9, 768 5.7 / 5.1; without a norm 2 on 1 of 64 768 (3,072) 3.4 / 3.6, 1,024
 // (4,096) 3.7 / 3.7, 1,280 4.2 / 3.9, 1 on 1 of 64 768 (2,304) 3.3 / 3.3, 4 on 1 of 128 768 (4,608) 4.7 / 3.6.
 #define HRR_UNITS 4
 #define HRR_MIN_TOKENS 768
 #define HRR_MIN_TOKENS_WHOLE 128
+#define HRR_WHOLE_COLUMNS 1024
 #define HRR_MIN_HEADS 4096
-#define HRR_MIN_HEADS_NORM 6144
+#define HRR_MIN_HEADS_WHOLE 6144
+#define HRR_MIN_HEADS_NORM 7680
 
 template <typename T>
 __global__ void __launch_bounds__(256) head_rotary_rows_kernel(HeadRotaryCall c) {
@@ -297,7 +301,7 @@ BT_EXPORT int bt_head_rotary_call(void* stream, const HeadRotaryCall* c) {
   const uintptr_t pair = (c->dtype == 0 ? 8 : 4) - 1;      // of two elements of the outputs
   const bool norms = c->q_gamma || c->k_gamma, whole = norms && c->norm_span == 1;
   const bool many = c->tokens >= (whole ? HRR_MIN_TOKENS_WHOLE : HRR_MIN_TOKENS) &&
-                    (int64_t)c->tokens * units >= (norms ? HRR_MIN_HEADS_NORM : HRR_MIN_HEADS);
+                    ((whole && (int64_t)c->heads * c->dim >= HRR_WHOLE_COLUMNS) || (int64_t)c->tokens * units >= (whole ? HRR_MIN_HEADS_WHOLE : norms ? HRR_MIN_HEADS_NORM : HRR_MIN_HEADS));
   const bool rows = many && c->maps == 1 && hd <= 128 && hd % 2 == 0 && c->dim % 2 == 0 && c->vdim % 2 == 0 && c->ld % 2 == 0 &&
                     c->ld_q % 2 == 0 && c->kv.block_stride % 2 == 0 && c->kv.head_stride % 2 == 0 && (c->pairing == 1 || c->rot_dims % 4 == 0) && ((uintptr_t)c->in & 7) == 0 &&
                     (((uintptr_t)c->q_out | (uintptr_t)c->kv.keys | (uintptr_t)c->kv.values) & pair) == 0;
