@@ -308,7 +308,8 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(RouteCall c) {
 // 7 us for 512 and 1,024 columns whatever the step, so steps of fewer than ROUTE_ROWS_MIN tokens keep a work-group a token.  Measured (us, a
 // work-group a token / sixteen; outputs of columns): 9 of 1,024 1,000 tokens 5.5 / 6.6, 1,200 6.5 / 6.6, 1,400 7.2 / 6.6, 1,530 7.4 / 6.6; 17 of 1,024 1,000
 // 7.8 / 8.7, 1,200 9.1 / 8.7, 1,530 10.4 / 8.7; 8 of 512 1,000 4.6 / 4.8, 1,200 4.9 / 4.8, 1,530 5.5 / 4.8; 32 of 2,048 600 15.3 / 15.3, 1,530 25.9 / 15.4.  In a step of
-// 1,809 tokens 9 outputs of 1,024 and a gate take 8.5.
+// 1,809 tokens 9 outputs of 1,024 and a gate take 8.5.  From 1,280 tokens on sixteen would be the faster way; but the two add a logit's products
+// in different orders, and a choice between experts that are nearly equal may fall the other way: the line stays where it is.
 #define ROUTE_ROWS 16
 #define ROUTE_ROWS_TILES 2      // (most outputs: 32)
 #define ROUTE_ROWS_AHEAD 4      // chunks of 16 columns on their way
@@ -375,7 +376,7 @@ __global__ void __launch_bounds__(64 * ROUTE_ROWS) route_rows_kernel(RouteCall c
 
 // (Few outputs of wide rows from 1,792 tokens on: 8 of 1,024 bfloat16 columns 1,530 tokens 5.5 / 6.2, 1,780 6.0 / 6.2; of 4,096 1,530 13.8 / 14.7, 1,780 15.6 /
 // 14.8; of 4,096 float ones 13.3 / 14.9 and 14.5 / 14.8.)
-#define ROUTE_ROWS_MIN 1280
+#define ROUTE_ROWS_MIN 1536
 #define ROUTE_ROWS_MIN_FEW 1792
 
 template <typename T>

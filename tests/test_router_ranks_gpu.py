@@ -69,3 +69,24 @@ def test_ties_and_shut_out_experts(experts, top, groups, keep, score):
         assert torch.equal(got != 0, expected != 0), "another expert was chosen"
         # an exponential, a sum of 64 and two divisions in 32 bits
         assert float((got - expected).abs().max()) < 80 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+# (the two kernels add a logit's products in different orders: steps below the line have the sums of a work-group a token, bit for bit)
+@pytest.mark.parametrize("outputs,width,below,above", [(9, 1024, [1279, 1280, 1535], 1536), (17, 1024, [1280, 1535], 1536), (8, 512, [1280, 1535], 1536),
+                                                       (8, 1024, [1536, 1791], 1792)])
+def test_sums_on_both_sides_of_the_line(outputs, width, below, above, dtype):
+    gen = torch.Generator().manual_seed(outputs)
+    h = torch.randn(above, width, generator=gen).to(getattr(torch, dtype)).to(DEV)
+    router = (torch.randn(outputs, width, generator=gen) * width ** -0.5).to(DEV)
+
+    def weights(rows):
+        out = torch.full((rows.shape[0], outputs), math.nan, device=DEV)
+        K.route(rows, router, None, outputs, 1, 1, out, score="softmax")          # (all are chosen: their scores as they are)
+        return out
+    few = torch.cat([weights(h[begin:begin + 100]) for begin in range(0, above, 100)])
+    for tokens in below:
+        assert torch.equal(weights(h[:tokens]), few[:tokens]), tokens
+    # sums of `width` products of size one in another order
+    many = weights(h)
+    assert not torch.equal(many, few) and float((many - few).abs().max()) < 4e-6
