@@ -438,8 +438,8 @@ __device__ float bt_norm_zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
 // Eight waves that stream, and one beside them that looks up the tables of the epilogues that have any.
 constexpr int skinny_threads(int waves, int kind) { return (waves + (kind == EPILOGUE_QKV || kind == EPILOGUE_TURN)) * 64; }
-// Waves a SIMD has room for: two work-groups a compute unit where the registers allow it without spilling (at eight rows the forms of
-// two column blocks do too: 123 registers).
+// Waves a SIMD must have room for: two work-groups of eight waves a compute unit for forms of one block.  (Those of two blocks take 97 to 119
+// registers and so have room too.)
 constexpr int skinny_occupancy(int mt, int nt, int qpl) { return mt == 1 && nt == 1 && qpl == 0 ? 4 : 2; }
 
 // Of a load that holds `16 / ROWS` chunks of ROWS rows in every sixteen lanes, the operand of chunk `sub`: its rows in the first ROWS lanes.
@@ -554,17 +554,22 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if ((u % WP == 0 || (!NORM && u % AP == 0)) && c0 + u * stride < whole) {
+        // (a place's lanes add their offsets here and not before the batch's first load, which kept them all in registers at once: the forms of
+        // eight chunks and two blocks took 138, so that one work-group of theirs shared a compute unit with no other.  18432 x 2048, nine rows
+        // 18.7 us, so 16.5.  Not volatile: behind an assembly statement that may do anything loads no longer go through the scalar cache.)
+        unsigned w_to = u * w_jump, a_to = u * a_jump;
+        asm("" : "+s"(w_to), "+s"(a_to));
         if (u % WP == 0) {
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) {
-            const unsigned off = w_off[nt] + u * w_jump;
+            const unsigned off = w_off[nt] + w_to;
             wv[u / WP][nt] = from(w_base, WP > 1 && off > w_most ? w_most : off);
           }
         }
         if (!NORM && u % AP == 0) {
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
-            const unsigned off = a_off[mt] + u * a_jump;
+            const unsigned off = a_off[mt] + a_to;
             av[u / AP][mt] = from(a_base, AP > 1 && off > a_most ? a_most : off);
           }
         }
