@@ -126,13 +126,44 @@ __device__ __forceinline__ void epilogue_addends(const Epilogue& e, int M, int n
   }
 }
 
-// What the skinny kernel's epilogue looks up, by a wave that multiplies nothing: loads that depend on each other would wait for
-// all the weights before them in a wave that streams (they return in order), which put a second round trip to memory behind
-// every product.  Of up to 16 * MT rows (and 16 * NT columns).
-template <int KIND, int MT, int NT>
-struct EpilogueTables {       // (the other kinds need none)
-  __device__ __forceinline__ void fill(const Epilogue&, int, int) {}
+// What the skinny kernel's epilogue looks up in the step's tables, of up to 16 * MT rows (and 16 * NT columns).  As vector loads of
+// the waves that stream, the lookups, which depend on each other, would wait for all the weights before them (loads return in order): a second
+// round trip to memory behind every product.  For forms of one column block a ninth wave, which multiplies nothing, does it meanwhile (`fill`; of
+// turned columns up to sixteen rows, more sines than that take one wave too long).  Nine waves put three on one SIMD, which leaves them 168
+// registers each, and room for two work-groups a compute unit only up to 96.  The forms of two column blocks have neither, so there every streaming
+// wave takes a share: places of tokens through the scalar cache (TokenPlaces), sines of its own values (TurnedPairs).  Measured (us, a ninth wave in all
+// forms / so): 4800 x 1600 into the cache, one row with a norm 7.9 / 6.3, 24 rows 12.5 / 8.1; 9216 x 3072, eight rows 16.0 / 14.5; turned 10240 x 1536, 24 rows 20.9 /
+// 13.3, 2560 x 768, 64 rows 7.5 / 6.3.  The streaming waves' share in all forms: 2304 x 768 with a norm 3.8 -> 4.0, 1280 x 384 turned 2.7 -> 3.4.
+// A share of the rows' places:
+template <int ROWS, int WAVES>
+struct TokenPlaces {
+  static constexpr int SHARE = ROWS / WAVES;
+  int pos[SHARE], seq[SHARE], block[SHARE];
+  __device__ __forceinline__ void ask(const Epilogue& e, int M, int wave) {
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) {       // (rows beyond M repeat the last)
+      const int m = wave + WAVES * i < M ? wave + WAVES * i : M - 1;
+      pos[i] = e.tok_pos[m];
+      seq[i] = e.tok_seq[m];
+    }
+  }
+  __device__ __forceinline__ void look(const Epilogue& e) {
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) block[i] = e.kv.blocks[(int64_t)seq[i] * e.kv.max_blocks + pos[i] / BT_KV_BLOCK];
+  }
+  template <typename Tables>
+  __device__ __forceinline__ void put(const Epilogue& e, int wave, Tables& tables) const {
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+      for (int i = 0; i < SHARE; ++i) {
+        tables.plane[wave + WAVES * i] = kv_plane(e.kv, block[i], 0);
+        tables.pos[wave + WAVES * i] = pos[i];
+      }
+    }
+  }
 };
+template <int KIND, int MT, int NT>
+struct EpilogueTables {};     // (the other kinds need none)
 template <int MT, int NT>
 struct EpilogueTables<EPILOGUE_QKV, MT, NT> {
   int64_t plane[16 * MT];     // where the block of the row's token starts in the cache, and the token's position
@@ -148,7 +179,7 @@ struct EpilogueTables<EPILOGUE_QKV, MT, NT> {
 };
 template <int MT, int NT>
 struct EpilogueTables<EPILOGUE_TURN, MT, NT> {
-  float2 turn[16 * MT][8 * NT];      // amplitude times cosine and sine of a row's pair of columns
+  float2 turn[16 * MT][8 * NT];      // cosine and sine of a row's pair of columns
   __device__ __forceinline__ void fill(const Epilogue& e, int M, int n_base) {
     for (int at = threadIdx.x & 63; at < M * 8 * NT; at += 64) {
       const int m = at / (8 * NT), pair = at % (8 * NT);
@@ -158,6 +189,32 @@ struct EpilogueTables<EPILOGUE_TURN, MT, NT> {
       const float f = turned ? e.turn.inv_freq[j >> 1] : 0.f;
       if (f != 0.f) sincosf((float)e.tok_pos[m] * f, &sn, &cs);
       turn[m][pair] = make_float2(cs, sn);
+    }
+  }
+};
+// The sines of a thread's own values: asked for behind the first batch of weights, worked out behind the products.
+template <int VALUES>
+struct TurnedPairs {
+  static constexpr int PAIRS = (VALUES + 1) / 2;
+  int pos;
+  float f[PAIRS];
+  float2 turn[PAIRS];
+  __device__ __forceinline__ void ask(const Epilogue& e, int M, int m, int n0) {
+    pos = e.tok_pos[m < M ? m : M - 1];
+    const int j = n0 % e.turn.pitch - e.turn.at;       // (of an odd column the pair is the even one's)
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      const bool turned = j + 2 * p >= 0 && j + 2 * p < e.turn.dim;
+      const float there = e.turn.inv_freq[turned ? (j + 2 * p) >> 1 : 0];
+      f[p] = turned ? there : 0.f;
+    }
+  }
+  __device__ __forceinline__ void work() {
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      float sn = 0.f, cs = 1.f;
+      if (f[p] != 0.f) sincosf((float)pos * f[p], &sn, &cs);
+      turn[p] = make_float2(cs, sn);
     }
   }
 };
@@ -181,9 +238,10 @@ __device__ __forceinline__ void store_values(T* dst, const float (&v)[VALUES], i
 // The skinny kernel's epilogue for VALUES neighbouring columns of a row, inside four: v are the sums with what is added to them,
 // column is n0 inside the work-group.  One value a lane with up to sixteen rows: a wave that takes four of each lane has most of
 // its lanes idle then, and the longer chain behind the last barrier showed in every product (0.3 us, with a GELU 0.7, of 2.7 and 3.7).
+// tables: EpilogueTables; turn: what the values' pairs turn by.
 template <typename T, int KIND, int VALUES, typename Tables>
 __device__ __forceinline__ void epilogue_values(const Epilogue& e, int N, int m, int n0, int column, float (&v)[VALUES], int split,
-                                                const Tables& tables) {
+                                                const Tables& tables, const float2* turn) {
   const int count = N - n0;
   if constexpr (KIND == EPILOGUE_TURN) {    // (pairs of columns are one lane's or two neighbours'; N is whole pairs)
     float y[VALUES];
@@ -191,7 +249,7 @@ __device__ __forceinline__ void epilogue_values(const Epilogue& e, int N, int m,
     for (int i = 0; i < VALUES; ++i) {
       const float other = VALUES == 1 ? lane_moved<0xb1>(v[i]) : v[VALUES == 1 ? i : i ^ 1];
       const int j = (n0 + i) % e.turn.pitch - e.turn.at;
-      const float2 t = tables.turn[m][(column + i) >> 1];
+      const float2 t = turn[i >> 1];
       const float amplitude = j >= 0 && j < e.turn.dim ? e.turn.amplitude : 1.f;
       const bool odd = (column + i) & 1;
       y[i] = amplitude * fmaf(odd ? other : v[i], odd ? t.y : t.x, odd ? v[i] * t.x : -(other * t.y));

@@ -415,8 +415,8 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
 //   have scalar branches between them and nothing else; K's partial chunk is outside the batches;
 //   up to eight rows (four) two (four) chunks of the activations come with one load, and two of the weights where a work-group has
 //   eight columns (AP, WP below: 768 x 3072, one row 4.8 -> 4.3; 1600 x 1600, eight rows 4.3 -> 4.1);
-//   what depends on a table of the step is looked up by a wave that streams nothing (EpilogueTables): in a streaming wave it stood
-//   behind all the weights, a second trip to memory in every product;
+//   what depends on a table of the step is looked up by a wave that streams nothing or through the scalar cache (EpilogueTables): as a
+//   streaming wave's vector loads it stood behind all the weights, a second trip to memory in every product;
 //   the epilogue takes one value a lane (VALUES below: 3072 x 768 with a GELU 3.7 -> 3.4).
 // In all, against a kernel with none of these (weights from memory, in a HIP graph, us): one row 768 x 768 3.1 -> 2.7, 768 x 3072 5.2 ->
 // 4.3, 3072 x 768 with a norm and a GELU 5.1 -> 4.2; eight rows 4800 x 1600 6.0 -> 5.4, 6400 x 1600 with a GELU 6.9 -> 6.1, 1600 x 6400
@@ -436,8 +436,9 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
 // statistics are computed while the weights are on their way.
 __device__ float bt_norm_zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
-// Eight waves that stream, and one beside them that looks up the tables of the epilogues that have any.
-constexpr int skinny_threads(int waves, int kind) { return (waves + (kind == EPILOGUE_QKV || kind == EPILOGUE_TURN)) * 64; }
+// Eight waves that stream, and in some forms a ninth beside them (EpilogueTables).
+constexpr bool skinny_ninth(int kind, int mt, int nt) { return nt == 1 && (kind == EPILOGUE_QKV || (kind == EPILOGUE_TURN && mt == 1)); }
+constexpr int skinny_threads(int waves, int kind, int mt, int nt) { return (waves + skinny_ninth(kind, mt, nt)) * 64; }
 // Waves a SIMD must have room for: two work-groups of eight waves a compute unit for forms of one block.  (Those of two blocks take 97 to 119
 // registers and so have room too.)
 constexpr int skinny_occupancy(int mt, int nt, int qpl) { return mt == 1 && nt == 1 && qpl == 0 ? 4 : 2; }
@@ -494,26 +495,29 @@ static SkinnyOperands skinny_operands(const void* A, int64_t lda, const void* W,
 }
 
 template <typename T, int MT, int NT, int U, int WAVES, int QPL, int KIND, int AP, int WP>
-__global__ void __launch_bounds__(skinny_threads(WAVES, KIND), skinny_occupancy(MT, NT, QPL))
+__global__ void __launch_bounds__(skinny_threads(WAVES, KIND, MT, NT), skinny_occupancy(MT, NT, QPL))
 gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   constexpr int ELEMS = Mma<T>::ELEMS;      // K values in a lane's 16-byte load
-  constexpr bool NORM = QPL > 0, TABLES = KIND == EPILOGUE_QKV || KIND == EPILOGUE_TURN;
+  constexpr bool NORM = QPL > 0, NINTH = skinny_ninth(KIND, MT, NT), OWN_SINES = KIND == EPILOGUE_TURN && !NINTH,
+                 OWN_PLACES = KIND == EPILOGUE_QKV && !NINTH;
   static_assert(!NORM || (MT == 1 && sizeof(T) == 2), "the fused norm is for bfloat16 and up to 16 rows");
   extern __shared__ __attribute__((aligned(16))) unsigned char normed[];   // NORM: [16][K * 2 + 16] bytes
   const int M = o.M, whole = o.whole, rest = o.rest, splits = o.splits;
   const int K = whole * (4 * ELEMS) + rest, normed_pitch = K * 2 + 16;      // the 16 bytes spread the rows over the LDS banks
   __shared__ __attribute__((aligned(16))) float red[WAVES][MT * NT][4][80];
-  __shared__ EpilogueTables<KIND, MT, NT> tables;
+  __shared__ EpilogueTables<OWN_SINES ? (int)EPILOGUE_COMMON : KIND, MT, NT> tables;
   // the wave's number is the same in all its lanes: saying so keeps every test on it a scalar
   // branch, which costs no wait for loads in flight (a divergent one does)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int n_base = blockIdx.x * o.tile_columns;
   const int n_end = n_base + o.tile_columns < o.N ? n_base + o.tile_columns : o.N;   // one past this work-group's last column
-  if (TABLES && wave == WAVES) {            // the wave that looks up what the epilogue needs: nothing here waits for weights
-    tables.fill(epi, M, n_base);
-    if constexpr (NORM) __syncthreads();
-    __syncthreads();
-    return;
+  if constexpr (NINTH) {
+    if (wave == WAVES) {                    // nothing here waits for weights
+      tables.fill(epi, M, n_base);
+      if constexpr (NORM) __syncthreads();
+      __syncthreads();
+      return;
+    }
   }
   const int i16 = lane & 15, g = lane >> 4;
   const int split = blockIdx.y;
@@ -595,6 +599,19 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
       }
   };
   int c0 = c_first;
+  // (With batches of two chunks the lookups' two trips are spread over the kernel: right behind the first batch, which is soon there,
+  // 33 rows of 4800 x 1600 took 9.7 us, so 9.5.  With more chunks they are over before the weights come; one row with a norm 6.5 spread, so 6.3.)
+  TokenPlaces<16 * MT, WAVES> places;       // OWN_PLACES only
+  constexpr bool SPREAD = MT == 4;
+  auto look_up = [&]() {
+    if constexpr (OWN_PLACES) {
+      places.ask(epi, M, wave);
+      if constexpr (!SPREAD) {
+        places.look(epi);
+        places.put(epi, wave, tables);
+      }
+    }
+  };
   if constexpr (NORM) {
     const int quads = K >> 2;
     const float4* g4 = reinterpret_cast<const float4*>(norm.gamma);
@@ -645,6 +662,7 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
     };
     if (wave < M) load_row(wave);            // (the wave's number is scalar: no lane-dependent branch)
     issue(c0);                               // the weights of the first batch, behind the row
+    look_up();
     if (wave < M) normalise_row(wave);
     if (wave + WAVES < M) {
       load_row(wave + WAVES);
@@ -653,6 +671,7 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
     __syncthreads();
   } else {
     issue(c0);
+    look_up();
   }
   // A thread finishes one output value, or VALUES neighbours of a row: what is added to them is fetched now, behind the first batch,
   // so that no load is left on the critical path after the last multiply.
@@ -661,6 +680,9 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   const int out_m = tid * VALUES / COLUMNS, column = tid * VALUES % COLUMNS;
   float add[VALUES];
   epilogue_addends<KIND>(epi, M, n_end, out_m, n_base + column, split, add);
+  TurnedPairs<VALUES> pairs;                // EPILOGUE_TURN only
+  if constexpr (OWN_SINES) pairs.ask(epi, M, out_m, n_base + column);
+  if constexpr (OWN_PLACES && SPREAD) places.look(epi);
   for (;;) {
     multiply(c0);
     c0 += U * stride;
@@ -689,6 +711,8 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
       }
     }
   }
+  if constexpr (OWN_PLACES && SPREAD) places.put(epi, wave, tables);
+  if constexpr (OWN_SINES) pairs.work();
   // lane holds D[i][j]: i = 4 g + r the column, j = i16 the row.  (The groups lie 80 floats apart: neighbouring columns of four
   // rows are then in 64 different banks.)
 #pragma unroll
@@ -711,7 +735,11 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
       for (int w = 0; w < WAVES; ++w) v[i] += share[w][i];
       v[i] += add[i];
     }
-    epilogue_values<T, KIND>(epi, n_end, out_m, n_base + column, column, v, split, tables);
+    if constexpr (NINTH && KIND == EPILOGUE_TURN) {
+#pragma unroll
+      for (int p = 0; p < pairs.PAIRS; ++p) pairs.turn[p] = tables.turn[out_m][(column >> 1) + p];
+    }
+    epilogue_values<T, KIND>(epi, n_end, out_m, n_base + column, column, v, split, tables, pairs.turn);
   }
 }
 
@@ -902,7 +930,7 @@ static void launch_skinny(hipStream_t s, const T* a, int64_t lda, const T* w, in
   const NormOperand none = {};
   const SkinnyOperands o = skinny_operands<T>(a, lda, w, M, N, K, splits, columns, packed, a_rows);
 #define LAUNCH_SKINNY_FORM(MT, NT, U, KIND, AP, WP) \
-  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, KIND, AP, WP>), grid, dim3(skinny_threads(8, KIND)), 0, s, o, epi, none)
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, KIND, AP, WP>), grid, dim3(skinny_threads(8, KIND, MT, NT)), 0, s, o, epi, none)
 #define LAUNCH_SKINNY(MT, NT, U, AP, WP)                                                          \
   do {                                                                                            \
     if (epi.mode == EPI_TURN) LAUNCH_SKINNY_FORM(MT, NT, U, EPILOGUE_TURN, AP, WP);               \
@@ -970,7 +998,7 @@ static int launch_skinny_norm(hipStream_t s, const NormOperand& norm, const bf16
       if (err != hipSuccess) BT_REFUSE("gemm_skinny: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));   \
       granted = lds;                                                                                           \
     }                                                                                                          \
-    hipLaunchKernelGGL(kernel, grid, dim3(skinny_threads(8, KIND)), lds, s, o, epi, norm);                                     \
+    hipLaunchKernelGGL(kernel, grid, dim3(skinny_threads(8, KIND, 1, NT)), lds, s, o, epi, norm);                                     \
   } while (0)
   if (K <= 1024) {
     if (columns == 8) LAUNCH_NORM(1, 4, 2); else if (columns <= 16) LAUNCH_NORM(1, 4, 1); else LAUNCH_NORM(2, 4, 1);

@@ -59,3 +59,9 @@ def test_two_work_groups_of_the_skinny_product_share_a_compute_unit():
     forms = [f for f in skinny_forms() if f[4] == 0 and not (f[0] * f[1] == 4 and f[2] == 8) and f[6][".max_flat_workgroup_size"] == 512]
     assert len(forms) > 20
     assert not [f for f in forms if f[6][".vgpr_count"] + f[6].get(".agpr_count", 0) > 128]
+
+
+def test_no_form_of_the_skinny_product_spills():
+    forms = list(skinny_forms())
+    assert len(forms) > 100
+    assert not [f for f in forms if f[6][".vgpr_spill_count"] or f[6][".private_segment_fixed_size"]]
