@@ -265,6 +265,10 @@ attention_f32_mfma_kernel(AttnArgs a) {
 // read, as the cache lays them out; the probabilities come back from LDS as broadcasts) and are asked for together with the keys
 // where the registers allow.  The four waves' running results meet in LDS at the end.  12 heads of 64, four sequences of up to 1,000
 // tokens in four runs, us with the kernel that joins them: 12.8 with a row a lane and a value after the other, 10.3 so.
+// Loads take a uniform base and a lane's offset of 32 bits: with an address of 64 bits a load the 32 of a head's keys alone took 64 registers,
+// and heads of more than 64 channels spilled 71 of them at two work-groups a compute unit.  Measured (us, addresses a load / so): 16 heads of 128, eight
+// sequences of 1,000 tokens 72.5 / 33.4 (in four runs with their join 50.6 / 32.6), 32 heads of 128 on 8, four sequences in four runs 35.3 / 18.9, 20 of 80,
+// eight in four 59.9 / 29.4; 12 of 64, four in four 11.7 / 10.8, 32 in one 38.6 / 38.7.
 template <int CPT>
 __global__ void __launch_bounds__(256, 2)
 attention_f32_decode_kernel(AttnArgs a) {
@@ -281,14 +285,15 @@ attention_f32_decode_kernel(AttnArgs a) {
   const int pos = a.seq_start[seq];                     // the query's position: token `seq` of the step
   const float* q = static_cast<const float*>(a.q) + (int64_t)seq * a.ldq + head * hd;
   const int splits = a.splits > 1 ? a.splits : 1, split = blockIdx.z;
-  int channels[CPT];                                    // the first of the lane's four channels of a key (beyond the head: 0)
+  unsigned key_off[CPT];                                // bytes to the lane's four channels of its row of a load (beyond the head: its first)
   bool real[CPT];
   float4 qv[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
     real[j] = 4 * (l16 + 16 * j) < hd;
-    channels[j] = real[j] ? 4 * (l16 + 16 * j) : 0;
-    qv[j] = *reinterpret_cast<const float4*>(q + channels[j]);
+    const int channel = real[j] ? 4 * (l16 + 16 * j) : 0;
+    key_off[j] = 4 * (g * hd + channel);
+    qv[j] = *reinterpret_cast<const float4*>(q + channel);
   }
   float gate[CPT];
 #pragma unroll
@@ -314,16 +319,16 @@ attention_f32_decode_kernel(AttnArgs a) {
     const int block = walk.at(place);
     const int physical = block < 64 ? __builtin_amdgcn_readlane(held_blocks, block) : block_row[block];
     const int64_t base = kv_plane(a.kv, physical, kv_head);
-    const float *kblock = keys + base, *vblock = values + base;
+    const char *kblock = reinterpret_cast<const char*>(keys + base), *vblock = reinterpret_cast<const char*>(values + base);
     float4 kreg[CPT][16], vreg[BT_KV_BLOCK / 4];
 #pragma unroll
     for (int i = 0; i < 16; ++i)
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) kreg[j][i] = *reinterpret_cast<const float4*>(kblock + (4 * i + g) * hd + channels[j]);
+      for (int j = 0; j < CPT; ++j) kreg[j][i] = *reinterpret_cast<const float4*>(kblock + i * (16 * hd) + key_off[j]);
     auto fetch_values = [&](int j) {        // the 64 values of channel lane + 64 j
-      const int cc = lane + 64 * j < hd ? lane + 64 * j : 0;
+      const unsigned off = lane + 64 * j < hd ? 16 * (lane + 64 * j) : 0;
 #pragma unroll
-      for (int k4 = 0; k4 < BT_KV_BLOCK / 4; ++k4) vreg[k4] = *reinterpret_cast<const float4*>(vblock + (k4 * hd + cc) * 4);
+      for (int k4 = 0; k4 < BT_KV_BLOCK / 4; ++k4) vreg[k4] = *reinterpret_cast<const float4*>(vblock + k4 * (16 * hd) + off);
     };
     if (CPT == 1) fetch_values(0);
     float s = 0.f;
@@ -424,28 +429,25 @@ attention_f32_join_kernel(AttnArgs a) {
   for (int channel = threadIdx.x; channel < hd; channel += 64) {
     const float gate = STAGED ? bt_output_logit(a, seq, head, channel) : 0.f;
     float m[8], l[8], o[8], top = -INFINITY;
-    auto ask = [&](int s0, bool all) {
+    auto ask = [&](int s0) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float* record = runs + (int64_t)(s0 + j < a.splits ? s0 + j : s0) * pitch;
         m[j] = record[hd];
-        if (all) l[j] = record[hd + 1];
-        if (all) o[j] = record[channel];
+        l[j] = record[hd + 1];
+        o[j] = record[channel];
       }
     };
-    for (int s0 = a.splits > 8 ? 8 : 0; s0 < a.splits; s0 += 8) {       // (the first eight last: they stay in registers if they are all)
-      ask(s0, a.splits <= 8);
+    for (int s0 = 8; s0 < a.splits; s0 += 8) {        // (the first eight last, and whole: they stay in registers)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) top = fmaxf(top, m[j]);
+      for (int j = 0; j < 8; ++j) top = fmaxf(top, runs[(int64_t)(s0 + j < a.splits ? s0 + j : s0) * pitch + hd]);
     }
-    if (a.splits > 8) {
-      ask(0, true);
+    ask(0);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) top = fmaxf(top, m[j]);
-    }
+    for (int j = 0; j < 8; ++j) top = fmaxf(top, m[j]);
     float num = 0.f, den = 0.f;
     for (int s0 = 0; s0 < a.splits; s0 += 8) {
-      if (s0 > 0) ask(s0, true);
+      if (s0 > 0) ask(s0);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         if (s0 + j < a.splits) {                                    // an empty run: maximum -inf, weight 0

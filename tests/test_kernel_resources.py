@@ -65,3 +65,12 @@ def test_no_form_of_the_skinny_product_spills():
     forms = list(skinny_forms())
     assert len(forms) > 100
     assert not [f for f in forms if f[6][".vgpr_spill_count"] or f[6][".private_segment_fixed_size"]]
+
+
+@pytest.mark.parametrize("module", ["attention_f32", "attention_f32_softmax", "attention_f32_capped", "attention_f32_sigmoid"])
+def test_float32_decode_attention_keeps_its_keys_in_registers(module):
+    kernels = [k for k in kernels_of(module) if re.search(r"attention_f32_(decode|join)_kernel", k[".name"])]
+    assert len(kernels) == 3                          # heads of up to 64 and of up to 128, and the join of runs
+    assert not [k for k in kernels if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
+    # two work-groups of four waves a compute unit: a wave has half of the 512 registers a lane
+    assert not [k for k in kernels if k[".vgpr_count"] + k.get(".agpr_count", 0) > 256]
