@@ -504,7 +504,10 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char normed[];   // NORM: [16][K * 2 + 16] bytes
   const int M = o.M, whole = o.whole, rest = o.rest, splits = o.splits;
   const int K = whole * (4 * ELEMS) + rest, normed_pitch = K * 2 + 16;      // the 16 bytes spread the rows over the LDS banks
-  __shared__ __attribute__((aligned(16))) float red[WAVES][MT * NT][4][80];
+  // (72 floats for eight blocks: 80 KiB and the tables would keep a second work-group out.  Into the cache, us at 80 / 72:
+  // 33 rows of 9216 x 3072 30.2 / 28.2, 64 rows 40.5 / 38.0, 64 rows of 18432 x 2048 43.4 / 39.3)
+  constexpr int GROUP_PITCH = MT * NT > 4 ? 72 : 80;
+  __shared__ __attribute__((aligned(16))) float red[WAVES][MT * NT][4][GROUP_PITCH];
   __shared__ EpilogueTables<OWN_SINES ? (int)EPILOGUE_COMMON : KIND, MT, NT> tables;
   // the wave's number is the same in all its lanes: saying so keeps every test on it a scalar
   // branch, which costs no wait for loads in flight (a divergent one does)
@@ -713,8 +716,8 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   }
   if constexpr (OWN_PLACES && SPREAD) places.put(epi, wave, tables);
   if constexpr (OWN_SINES) pairs.work();
-  // lane holds D[i][j]: i = 4 g + r the column, j = i16 the row.  (The groups lie 80 floats apart: neighbouring columns of four
-  // rows are then in 64 different banks.)
+  // lane holds D[i][j]: i = 4 g + r the column, j = i16 the row.  (The groups lie 80 floats apart, or 72 where a lane reads four: what
+  // sixteen lanes' quads, or 64 lanes' values of a block, are read from is then in 64 different banks.)
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -727,7 +730,7 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
     float v[VALUES];
     floats share[WAVES];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) share[w] = *reinterpret_cast<const floats*>(part + w * (MT * NT * 320));
+    for (int w = 0; w < WAVES; ++w) share[w] = *reinterpret_cast<const floats*>(part + w * (MT * NT * 4 * GROUP_PITCH));
 #pragma unroll
     for (int i = 0; i < VALUES; ++i) {
       v[i] = 0.f;

@@ -61,6 +61,13 @@ def test_two_work_groups_of_the_skinny_product_share_a_compute_unit():
     assert not [f for f in forms if f[6][".vgpr_count"] + f[6].get(".agpr_count", 0) > 128]
 
 
+def test_lds_leaves_room_for_two_work_groups_of_the_skinny_product():
+    # (without a norm, whose rows are LDS of the launch)
+    forms = [f for f in skinny_forms() if f[4] == 0]
+    assert len(forms) > 100
+    assert not [f for f in forms if f[6][".group_segment_fixed_size"] > 160 * 1024 // 2]
+
+
 def test_no_form_of_the_skinny_product_spills():
     forms = list(skinny_forms())
     assert len(forms) > 100
