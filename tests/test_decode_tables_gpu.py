@@ -9,6 +9,7 @@ pytestmark = pytest.mark.gpu
 from burn_transformers_amd.kernels import library as K  # noqa: E402
 from kernel_helpers import PagedCase  # noqa: E402
 from test_kernels_gpu import DEV, rel_err  # noqa: E402
+from test_rotutar_kernels_gpu import sink_reference  # noqa: E402
 
 
 @pytest.mark.parametrize("window", [0, 300])
@@ -30,27 +31,36 @@ def test_tables_around_a_wave(totals, hd, dtype, runs, window):
     assert rel_err(out, case.reference(q, 8, 0.3, window)) < (1.2e-2 if dtype == "bfloat16" else 40 * 2.0 ** -24)
 
 
-@pytest.mark.parametrize("runs", [1, 3])
-@pytest.mark.parametrize("heads,kv", [(4, 4), (16, 1)])           # one head a work-group, more elements than threads
+# one head a work-group, more elements than threads; runs: whole, and around the eight records that a join reads together
+@pytest.mark.parametrize("runs", [1, 3, 11])
+@pytest.mark.parametrize("heads,kv", [(4, 4), (16, 1)])
 @pytest.mark.parametrize("span", [0, 1])
-def test_gates_and_sinks_asked_for_early(runs, heads, kv, span):
-    dt, hd, totals = torch.bfloat16, 128, [700, 65, 1]
+@pytest.mark.parametrize("hd,dtype", [(128, "bfloat16"), (128, "float32"), (64, "float32")])
+def test_gates_and_sinks_asked_for_early(runs, heads, kv, span, hd, dtype):
+    dt, totals = getattr(torch, dtype), [700, 65, 1]
     case = PagedCase(totals, [1] * 3, kv, hd, dt, DEV, seed=heads)
     gen = torch.Generator().manual_seed(heads + span)
     q = (torch.randn(3, heads * hd, generator=gen) * 0.5).to(dt).to(DEV)
-    sink = torch.randn(heads, generator=gen).to(DEV)
+    sink = torch.randn(heads, generator=gen) + torch.arange(heads) % 2 * 6           # (up to the size of all keys together)
     gate = torch.randn(3, heads * (hd - 16 if span else 1), generator=gen).to(DEV)
     partial = torch.full((3 * heads * runs, hd + 2), float("nan"), device=DEV) if runs > 1 else None
 
     def attend(**more):
         out = torch.full((3, heads * hd), float("nan"), dtype=torch.float32 if "gate" in more else dt, device=DEV)
         args = K.attention_args(q, out, case.view(), case.tok_seq, case.tok_pos, case.seq_off, case.seq_start, heads, 3, 1, 0.3, 0, partial,
-                                sink=sink, **more)
+                                sink=sink.to(DEV), **more)
         K.attention(args, dt, decode=True)
         return out.cpu().double().view(3, heads, hd)
     plain = attend()
+    # (the bounds of the test above, of every sequence's and head's row: a short context's rows are its values' size)
+    exact = sink_reference(case, q, heads, 0.3, 0, sink).view(3, heads, hd)
+    row_error = (plain - exact).norm(dim=-1) / exact.norm(dim=-1)
+    assert float(row_error.max()) < (1.2e-2 if dtype == "bfloat16" else 40 * 2.0 ** -24)
+    other = sink_reference(case, q, heads, 0.3, 0, sink.roll(1)).view(3, heads, hd)
+    assert bool(((other - exact).norm(dim=-1) / exact.norm(dim=-1)).gt(0.1).sum(1).ge(heads // 4).all()), "another head's sink would not show"
     factor = torch.sigmoid(gate.cpu().double()).view(3, heads, -1)
     if span:
         factor = torch.cat([factor, torch.ones(3, heads, 16, dtype=torch.float64)], -1)
     gated = attend(gate=gate, gate_dim=hd - 16 if span else 0)
-    assert bool(((gated - plain * factor).abs() <= 2.0 ** -8 * plain.abs() + 1e-6).all())       # the rounding of the row without a gate
+    last = 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -20        # the rounding of the row without a gate, or the sigmoid's
+    assert bool(((gated - plain * factor).abs() <= last * plain.abs() + 1e-6).all())
