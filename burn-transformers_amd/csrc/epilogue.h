@@ -130,9 +130,9 @@ __device__ __forceinline__ void epilogue_addends(const Epilogue& e, int M, int n
 // the waves that stream, the lookups, which depend on each other, would wait for all the weights before them (loads return in order): a second
 // round trip to memory behind every product.  For forms of one column block a ninth wave, which multiplies nothing, does it meanwhile (`fill`; of
 // turned columns up to sixteen rows, more sines than that take one wave too long).  Nine waves put three on one SIMD, which leaves them 168
-// registers each, and room for two work-groups a compute unit only up to 96.  The forms of two column blocks have neither, so there every streaming
-// wave takes a share: places of tokens through the scalar cache (TokenPlaces), sines of its own values (TurnedPairs).  Measured (us, a ninth wave in all
-// forms / so): 4800 x 1600 into the cache, one row with a norm 7.9 / 6.3, 24 rows 12.5 / 8.1; 9216 x 3072, eight rows 16.0 / 14.5; turned 10240 x 1536, 24 rows 20.9 /
+// registers each, and room for two work-groups a compute unit only up to 96.  The forms of two column blocks have neither, nor that of two row blocks and
+// eight chunks the latter, so there every streaming wave takes a share: places of tokens through the scalar cache (TokenPlaces), sines of its own values (TurnedPairs).  Measured (us, a ninth wave in all
+// forms / so): 4800 x 1600 into the cache, one row with a norm 7.9 / 6.3, 24 rows 12.5 / 8.1; 9216 x 3072, eight rows 16.0 / 14.5, 24 rows in 16 columns 29.3 / 26.9; turned 10240 x 1536, 24 rows 20.9 /
 // 13.3, 2560 x 768, 64 rows 7.5 / 6.3.  The streaming waves' share in all forms: 2304 x 768 with a norm 3.8 -> 4.0, 1280 x 384 turned 2.7 -> 3.4.
 // A share of the rows' places:
 template <int ROWS, int WAVES>

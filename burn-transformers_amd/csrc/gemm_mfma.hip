@@ -437,8 +437,10 @@ gemm_tile_parts_kernel(const float* __restrict__ A, int64_t lda, const float* __
 __device__ float bt_norm_zeros[4] = {0.f, 0.f, 0.f, 0.f};
 
 // Eight waves that stream, and in some forms a ninth beside them (EpilogueTables).
-constexpr bool skinny_ninth(int kind, int mt, int nt) { return nt == 1 && (kind == EPILOGUE_QKV || (kind == EPILOGUE_TURN && mt == 1)); }
-constexpr int skinny_threads(int waves, int kind, int mt, int nt) { return (waves + skinny_ninth(kind, mt, nt)) * 64; }
+constexpr bool skinny_ninth(int kind, int mt, int nt, int u) {
+  return nt == 1 && ((kind == EPILOGUE_QKV && mt * u < 16) || (kind == EPILOGUE_TURN && mt == 1));
+}
+constexpr int skinny_threads(int waves, int kind, int mt, int nt, int u) { return (waves + skinny_ninth(kind, mt, nt, u)) * 64; }
 // Waves a SIMD must have room for: two work-groups of eight waves a compute unit for forms of one block.  (Those of two blocks take 97 to 119
 // registers and so have room too.)
 constexpr int skinny_occupancy(int mt, int nt, int qpl) { return mt == 1 && nt == 1 && qpl == 0 ? 4 : 2; }
@@ -495,10 +497,10 @@ static SkinnyOperands skinny_operands(const void* A, int64_t lda, const void* W,
 }
 
 template <typename T, int MT, int NT, int U, int WAVES, int QPL, int KIND, int AP, int WP>
-__global__ void __launch_bounds__(skinny_threads(WAVES, KIND, MT, NT), skinny_occupancy(MT, NT, QPL))
+__global__ void __launch_bounds__(skinny_threads(WAVES, KIND, MT, NT, U), skinny_occupancy(MT, NT, QPL))
 gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   constexpr int ELEMS = Mma<T>::ELEMS;      // K values in a lane's 16-byte load
-  constexpr bool NORM = QPL > 0, NINTH = skinny_ninth(KIND, MT, NT), OWN_SINES = KIND == EPILOGUE_TURN && !NINTH,
+  constexpr bool NORM = QPL > 0, NINTH = skinny_ninth(KIND, MT, NT, U), OWN_SINES = KIND == EPILOGUE_TURN && !NINTH,
                  OWN_PLACES = KIND == EPILOGUE_QKV && !NINTH;
   static_assert(!NORM || (MT == 1 && sizeof(T) == 2), "the fused norm is for bfloat16 and up to 16 rows");
   extern __shared__ __attribute__((aligned(16))) unsigned char normed[];   // NORM: [16][K * 2 + 16] bytes
@@ -933,7 +935,7 @@ static void launch_skinny(hipStream_t s, const T* a, int64_t lda, const T* w, in
   const NormOperand none = {};
   const SkinnyOperands o = skinny_operands<T>(a, lda, w, M, N, K, splits, columns, packed, a_rows);
 #define LAUNCH_SKINNY_FORM(MT, NT, U, KIND, AP, WP) \
-  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, KIND, AP, WP>), grid, dim3(skinny_threads(8, KIND, MT, NT)), 0, s, o, epi, none)
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, MT, NT, U, 8, 0, KIND, AP, WP>), grid, dim3(skinny_threads(8, KIND, MT, NT, U)), 0, s, o, epi, none)
 #define LAUNCH_SKINNY(MT, NT, U, AP, WP)                                                          \
   do {                                                                                            \
     if (epi.mode == EPI_TURN) LAUNCH_SKINNY_FORM(MT, NT, U, EPILOGUE_TURN, AP, WP);               \
@@ -1001,7 +1003,7 @@ static int launch_skinny_norm(hipStream_t s, const NormOperand& norm, const bf16
       if (err != hipSuccess) BT_REFUSE("gemm_skinny: cannot get %zu bytes of LDS: %s", lds, hipGetErrorString(err));   \
       granted = lds;                                                                                           \
     }                                                                                                          \
-    hipLaunchKernelGGL(kernel, grid, dim3(skinny_threads(8, KIND, 1, NT)), lds, s, o, epi, norm);                                     \
+    hipLaunchKernelGGL(kernel, grid, dim3(skinny_threads(8, KIND, 1, NT, 8)), lds, s, o, epi, norm);                                     \
   } while (0)
   if (K <= 1024) {
     if (columns == 8) LAUNCH_NORM(1, 4, 2); else if (columns <= 16) LAUNCH_NORM(1, 4, 1); else LAUNCH_NORM(2, 4, 1);

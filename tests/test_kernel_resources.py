@@ -61,6 +61,13 @@ def test_two_work_groups_of_the_skinny_product_share_a_compute_unit():
     assert not [f for f in forms if f[6][".vgpr_count"] + f[6].get(".agpr_count", 0) > 128]
 
 
+def test_a_ninth_wave_keeps_no_second_work_group_out():
+    # nine waves are three on one SIMD, and two work-groups of nine five: 512 / 5 registers each, in eights
+    forms = [f for f in skinny_forms() if f[4] == 0 and f[6][".max_flat_workgroup_size"] == 576]
+    assert len(forms) > 20
+    assert not [f for f in forms if f[6][".vgpr_count"] + f[6].get(".agpr_count", 0) > 96]
+
+
 def test_lds_leaves_room_for_two_work_groups_of_the_skinny_product():
     # (without a norm, whose rows are LDS of the launch)
     forms = [f for f in skinny_forms() if f[4] == 0]
