@@ -613,7 +613,7 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
       places.ask(epi, M, wave);
       if constexpr (!SPREAD) {
         places.look(epi);
-        places.put(epi, wave, tables);
+        places.put(wave, tables);
       }
     }
   };
@@ -716,7 +716,7 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
       }
     }
   }
-  if constexpr (OWN_PLACES && SPREAD) places.put(epi, wave, tables);
+  if constexpr (OWN_PLACES && SPREAD) places.put(wave, tables);
   if constexpr (OWN_SINES) pairs.work();
   // lane holds D[i][j]: i = 4 g + r the column, j = i16 the row.  (The groups lie 80 floats apart, or 72 where a lane reads four: what
   // sixteen lanes' quads, or 64 lanes' values of a block, are read from is then in 64 different banks.)
