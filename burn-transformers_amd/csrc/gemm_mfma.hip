@@ -471,13 +471,13 @@ struct SkinnyOperands {
   const void* A;
   int64_t w_group;                 // bytes from a work-group's first column to the next one's
   int w_step, a_step;              // bytes from a chunk of 64 bytes of K to the next
-  unsigned w_pitch, a_pitch;       // bytes from a column to the next, from a row to the next
+  unsigned w_pitch, a_pitch;       // bytes from a column to the next, from a row to the next (of the form for far operands: sixteens of bytes)
   int whole, rest;                 // whole chunks of K, values behind them
   int M, N, tile_columns, splits;
 };
 template <typename T>
 static SkinnyOperands skinny_operands(const void* A, int64_t lda, const void* W, int M, int N, int K, int splits, int columns, int packed,
-                                      int a_rows) {
+                                      int a_rows, bool far = false) {
   constexpr int CHUNK = 64 / (int)sizeof(T);
   SkinnyOperands o;
   o.W = W;
@@ -485,10 +485,10 @@ static SkinnyOperands skinny_operands(const void* A, int64_t lda, const void* W,
   o.whole = K / CHUNK;
   o.rest = K % CHUNK;
   o.w_step = packed ? columns * 64 : 64;
-  o.w_pitch = packed ? 64u : (unsigned)(K * sizeof(T));
+  o.w_pitch = (unsigned)((packed ? 64 : K * sizeof(T)) / (far ? 16 : 1));
   o.w_group = packed ? (int64_t)((K + CHUNK - 1) / CHUNK) * o.w_step : (int64_t)columns * K * (int64_t)sizeof(T);
   o.a_step = a_rows > 0 ? a_rows * 64 : 64;
-  o.a_pitch = a_rows > 0 ? 64u : (unsigned)(lda * (int64_t)sizeof(T));
+  o.a_pitch = (unsigned)((a_rows > 0 ? 64 : lda * (int64_t)sizeof(T)) / (far ? 16 : 1));
   o.M = M;
   o.N = N;
   o.tile_columns = columns;
@@ -496,7 +496,8 @@ static SkinnyOperands skinny_operands(const void* A, int64_t lda, const void* W,
   return o;
 }
 
-template <typename T, int MT, int NT, int U, int WAVES, int QPL, int KIND, int AP, int WP>
+// FAR: with offsets of 64 bits, for rows or columns that lie or reach 2 GiB apart (launch_skinny_far).
+template <typename T, int MT, int NT, int U, int WAVES, int QPL, int KIND, int AP, int WP, int FAR = 0>
 __global__ void __launch_bounds__(skinny_threads(WAVES, KIND, MT, NT, U), skinny_occupancy(MT, NT, QPL))
 gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   constexpr int ELEMS = Mma<T>::ELEMS;      // K values in a lane's 16-byte load
@@ -527,31 +528,33 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   const int i16 = lane & 15, g = lane >> 4;
   const int split = blockIdx.y;
   // Addresses are a uniform base and a lane's offset of 32 bits, which one addition moves from chunk to chunk.
+  typedef typename std::conditional<FAR != 0, uint64_t, unsigned>::type Offset;
+  constexpr Offset PITCHES = FAR ? 16 : 1;
   const char* w_base = static_cast<const char*>(o.W) + (int64_t)blockIdx.x * o.w_group;
   const char* a_base = static_cast<const char*>(o.A);
   const int c_first = split * WAVES + wave, stride = splits * WAVES;
-  const unsigned w_jump = stride * o.w_step, a_jump = stride * o.a_step;
+  const Offset w_jump = (Offset)stride * o.w_step, a_jump = (Offset)stride * o.a_step;
   // AP chunks of the activations to a load where the rows are few enough, WP of the weights: sixteen lanes hold 16 / AP rows of
   // the wave's chunk u, then of u + 1, ..., and a rotation in the row of lanes brings the later ones down.  (Lanes whose chunk
   // does not exist read the last whole one; what they hold is not multiplied.)
   constexpr int A_ROWS = 16 / AP, W_COLS = 16 / WP;
   static_assert(U % AP == 0 && U % WP == 0 && (MT == 1 || AP == 1) && (NT == 1 || WP == 1), "whole loads of one block");
-  unsigned w_off[NT], a_off[MT], w_most = 0, a_most = 0;
+  Offset w_off[NT], a_off[MT], w_most = 0, a_most = 0;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int n = WP > 1 ? i16 % W_COLS : nt * 16 + i16, last = n_end - n_base - 1;
-    const unsigned column = (unsigned)(n < last ? n : last) * o.w_pitch + g * 16;
-    w_off[nt] = column + (c_first + i16 / W_COLS * (WP > 1 ? stride : 0)) * o.w_step;
-    if (WP > 1) w_most = column + (whole - 1) * o.w_step;
+    const Offset column = (Offset)(n < last ? n : last) * o.w_pitch * PITCHES + g * 16;
+    w_off[nt] = column + (Offset)(c_first + i16 / W_COLS * (WP > 1 ? stride : 0)) * o.w_step;
+    if (WP > 1) w_most = column + (Offset)(whole - 1) * o.w_step;
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {         // (rows beyond M repeat the last; the epilogue drops them)
     const int m = AP > 1 ? i16 % A_ROWS : mt * 16 + i16;
-    const unsigned row = (unsigned)(m < M ? m : M - 1) * o.a_pitch + g * 16;
-    a_off[mt] = row + (c_first + i16 / A_ROWS * (AP > 1 ? stride : 0)) * o.a_step;
-    if (AP > 1) a_most = row + (whole - 1) * o.a_step;
+    const Offset row = (Offset)(m < M ? m : M - 1) * o.a_pitch * PITCHES + g * 16;
+    a_off[mt] = row + (Offset)(c_first + i16 / A_ROWS * (AP > 1 ? stride : 0)) * o.a_step;
+    if (AP > 1) a_most = row + (Offset)(whole - 1) * o.a_step;
   }
-  auto from = [](const char* base, unsigned off) { return *reinterpret_cast<const int4v*>(base + off); };
+  auto from = [](const char* base, Offset off) { return *reinterpret_cast<const int4v*>(base + off); };
   floatx4 acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -566,19 +569,19 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
         // (a place's lanes add their offsets here and not before the batch's first load, which kept them all in registers at once: the forms of
         // eight chunks and two blocks took 138, so that one work-group of theirs shared a compute unit with no other.  18432 x 2048, nine rows
         // 18.7 us, so 16.5.  Not volatile: behind an assembly statement that may do anything loads no longer go through the scalar cache.)
-        unsigned w_to = u * w_jump, a_to = u * a_jump;
+        Offset w_to = u * w_jump, a_to = u * a_jump;
         asm("" : "+s"(w_to), "+s"(a_to));
         if (u % WP == 0) {
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) {
-            const unsigned off = w_off[nt] + w_to;
+            const Offset off = w_off[nt] + w_to;
             wv[u / WP][nt] = from(w_base, WP > 1 && off > w_most ? w_most : off);
           }
         }
         if (!NORM && u % AP == 0) {
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
-            const unsigned off = a_off[mt] + a_to;
+            const Offset off = a_off[mt] + a_to;
             av[u / AP][mt] = from(a_base, AP > 1 && off > a_most ? a_most : off);
           }
         }
@@ -706,12 +709,12 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const int n = nt * 16 + i16, last = n_end - n_base - 1;
-      const int4v w = from(w_base, (unsigned)(n < last ? n : last) * o.w_pitch + whole * o.w_step + g * 16 + inside);
+      const int4v w = from(w_base, (Offset)(n < last ? n : last) * o.w_pitch * PITCHES + (Offset)whole * o.w_step + g * 16 + inside);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         const int m = mt * 16 + i16 < M ? mt * 16 + i16 : M - 1;
         const int4v a = NORM ? *reinterpret_cast<const int4v*>(normed + m * normed_pitch + whole * 64 + g * 16 + inside)
-                             : from(a_base, (unsigned)m * o.a_pitch + whole * o.a_step + g * 16 + inside);
+                             : from(a_base, (Offset)m * o.a_pitch * PITCHES + (Offset)whole * o.a_step + g * 16 + inside);
         Mma<T>::block16(acc[mt][nt], keep ? w : zero, a);
       }
     }
@@ -980,6 +983,23 @@ static void launch_skinny(hipStream_t s, const T* a, int64_t lda, const T* w, in
 #undef LAUNCH_SKINNY_FORM
 }
 
+// The same products (and the same sums) where an offset inside the rows or a work-group's columns needs more than 31 bits, in one form:
+// a view of rows 2 GiB apart, or K of many millions.  Nobody's step has such a product, so its time was not looked at.
+template <typename T>
+static void launch_skinny_far(hipStream_t s, const T* a, int64_t lda, const T* w, int M, int N, int K, const Epilogue& epi, int splits,
+                              int columns, int packed, int a_rows) {
+  dim3 grid((N + columns - 1) / columns, splits);
+  const NormOperand none = {};
+  const SkinnyOperands o = skinny_operands<T>(a, lda, w, M, N, K, splits, columns, packed, a_rows, true);
+#define LAUNCH_FAR(KIND) \
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, 4, 2, 2, 8, 0, KIND, 1, 1, 1>), grid, dim3(skinny_threads(8, KIND, 4, 2, 2)), 0, s, o, epi, none)
+  if (epi.mode == EPI_TURN) LAUNCH_FAR(EPILOGUE_TURN);
+  else if (epi.mode == EPI_QKV) LAUNCH_FAR(EPILOGUE_QKV);
+  else if (epi.mode == EPI_F32_ACT) LAUNCH_FAR(EPILOGUE_TWO);
+  else LAUNCH_FAR(EPILOGUE_COMMON);
+#undef LAUNCH_FAR
+}
+
 // The product of the normalised rows of a float32 residual stream (see NormOperand): bfloat16
 // weights, up to 16 rows, K up to 2048 and a multiple of 8.
 static int launch_skinny_norm(hipStream_t s, const NormOperand& norm, const bf16_t* w, int M, int N, int K,
@@ -1072,17 +1092,17 @@ BT_EXPORT int bt_gemm_skinny(void* stream, int dtype, const void* A, int64_t lda
       if (best < 0 || cost < best) { best = cost; columns = c; }
     }
   }
-  // (the kernel's offsets have 32 bits)
-  const int64_t size = 16 / elems, a_bytes = a_rows != 0 ? (int64_t)a_rows * K * size : ((int64_t)(M - 1) * lda + K) * size;
+  // where 32 bits of offset do (rows to normalise are read without)
+  const int64_t size = 16 / elems, a_bytes = a_rows != 0 ? (int64_t)a_rows * K * size : norm != nullptr ? 0 : ((int64_t)(M - 1) * lda + K) * size;
   const int64_t w_bytes = (int64_t)columns * (K + 4 * elems) * size;
-  if (a_bytes >= (int64_t)1 << 31 || w_bytes >= (int64_t)1 << 31) {
-    if (packed || a_rows != 0 || norm != nullptr || epi->mode == EPI_F32_ACT || epi->mode == EPI_TURN)
-      BT_REFUSE("gemm_skinny: rows of pitch %lld and K %d reach beyond 2 GiB", (long long)lda, K);
-    return bt_gemm_tile(stream, dtype, A, lda, W, M, N, K, epi, splits, 1);
-  }
+  const bool far = a_bytes >= (int64_t)1 << 31 || w_bytes >= (int64_t)1 << 31;
   if (norm != nullptr) {
     rc = launch_skinny_norm((hipStream_t)stream, *norm, (const bf16_t*)W, M, N, K, *epi, splits, columns, packed);
     if (rc) return rc;
+  } else if (far && dtype == 0) {
+    launch_skinny_far<float>((hipStream_t)stream, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits, columns, packed, a_rows);
+  } else if (far) {
+    launch_skinny_far<bf16_t>((hipStream_t)stream, (const bf16_t*)A, lda, (const bf16_t*)W, M, N, K, *epi, splits, columns, packed, a_rows);
   } else if (dtype == 0) {
     launch_skinny<float>((hipStream_t)stream, (const float*)A, lda, (const float*)W, M, N, K, *epi, splits, columns, packed, a_rows);
   } else {

@@ -45,12 +45,14 @@ def notes_of(elf):
     return kernels
 
 
-def skinny_forms():
-    """(rows' blocks, column blocks, chunks a batch, waves, quads of a norm, epilogue's kind, metadata) of the skinny product's forms."""
+def skinny_forms(far=0):
+    """(rows' blocks, column blocks, chunks a batch, waves, quads of a norm, epilogue's kind, metadata) of the skinny product's forms (``far``: of
+    those with offsets of 64 bits)."""
     for kernel in kernels_of("gemm_mfma"):
         form = re.search(r"gemm_skinny_kernelI(?:f|DF16b)((?:Li\d+E)+)E", kernel[".name"])
-        if form:
-            yield tuple(int(n) for n in re.findall(r"Li(\d+)E", form.group(1))[:6]) + (kernel,)
+        numbers = [int(n) for n in re.findall(r"Li(\d+)E", form.group(1))] if form else []
+        if numbers and numbers[8] == far:
+            yield (*numbers[:6], kernel)
 
 
 def test_two_work_groups_of_the_skinny_product_share_a_compute_unit():
@@ -78,6 +80,7 @@ def test_lds_leaves_room_for_two_work_groups_of_the_skinny_product():
 def test_no_form_of_the_skinny_product_spills():
     forms = list(skinny_forms())
     assert len(forms) > 100
+    forms += skinny_forms(far=1)
     assert not [f for f in forms if f[6][".vgpr_spill_count"] or f[6][".private_segment_fixed_size"]]
 
 
