@@ -1,7 +1,7 @@
-// What a matrix product does with its accumulators.  Every GEMM kernel hands groups of four
-// consecutive output columns of one row to `epilogue4`, which adds the bias and then either
-// stores, applies the activation, writes 32-bit partial sums, or scatters a fused
-// query/key/value projection into the query buffer and the paged cache.
+// What a matrix product does with its accumulators: it adds the bias and then either stores, applies the
+// activation, writes 32-bit partial sums, or scatters a fused query/key/value projection into the query
+// buffer and the paged cache.  The skinny kernel hands 1, 2 or 4 neighbouring columns of a row to `epilogue_values`,
+// the plain and small tile kernels four to `epilogue4`, those whose tiles leave through LDS a whole tile to `epilogue_tile`.
 #pragma once
 
 #include "common.h"

@@ -901,8 +901,8 @@ BT_EXPORT int bt_expert_products_call(void* stream, const ExpertProductsCall* c)
 }
 
 // hidden[t][e * ff + i] *= the token's weight of expert e, for `experts` experts side by side, from the router's logits of
-// the token; columns behind them (an expert every token uses) stay.  A work-group makes the token's whole choice (its
-// first wave, a few reductions over the experts) and multiplies its share of the columns.
+// the token; columns behind them (an expert every token uses) stay.  A work-group makes the token's whole choice (of up to
+// 64 experts every wave for itself, by ranks in lanes; of more its first wave, a few reductions over the experts) and multiplies its share of the columns.
 struct WeighExpertsCall {
   RouteCall route;          // dtype: element type of `hidden`; tokens, experts, top, groups, keep, correction, score, group_rank,
                             // normalize, bias; nothing else is looked at
