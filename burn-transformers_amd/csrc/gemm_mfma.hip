@@ -507,9 +507,10 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char normed[];   // NORM: [16][K * 2 + 16] bytes
   const int M = o.M, whole = o.whole, rest = o.rest, splits = o.splits;
   const int K = whole * (4 * ELEMS) + rest, normed_pitch = K * 2 + 16;      // the 16 bytes spread the rows over the LDS banks
-  // (72 floats for eight blocks: 80 KiB and the tables would keep a second work-group out.  Into the cache, us at 80 / 72:
-  // 33 rows of 9216 x 3072 30.2 / 28.2, 64 rows 40.5 / 38.0, 64 rows of 18432 x 2048 43.4 / 39.3)
-  constexpr int GROUP_PITCH = MT * NT > 4 ? 72 : 80;
+  // (72 floats for eight blocks with tables: 80 KiB and the tables would keep a second work-group out.  Into the cache, us at 80 / 72:
+  // 33 rows of 9216 x 3072 30.2 / 28.2, 64 rows 40.5 / 38.0, 64 rows of 18432 x 2048 43.4 / 39.3.  Without tables 80 KiB are half of a unit's
+  // LDS and 80 floats the faster way: 64 rows of 6400 x 1600 with a GELU 11.2 / 11.3, 1600 x 6400 in five slices 10.4 / 10.5)
+  constexpr int GROUP_PITCH = MT * NT > 4 && OWN_PLACES ? 72 : 80;
   __shared__ __attribute__((aligned(16))) float red[WAVES][MT * NT][4][GROUP_PITCH];
   __shared__ EpilogueTables<OWN_SINES ? (int)EPILOGUE_COMMON : KIND, MT, NT> tables;
   // the wave's number is the same in all its lanes: saying so keeps every test on it a scalar
@@ -568,9 +569,10 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
       if ((u % WP == 0 || (!NORM && u % AP == 0)) && c0 + u * stride < whole) {
         // (a place's lanes add their offsets here and not before the batch's first load, which kept them all in registers at once: the forms of
         // eight chunks and two blocks took 138, so that one work-group of theirs shared a compute unit with no other.  18432 x 2048, nine rows
-        // 18.7 us, so 16.5.  Not volatile: behind an assembly statement that may do anything loads no longer go through the scalar cache.)
+        // 18.7 us, so 16.5.  Batches of two chunks have the registers, and the additions between their loads only cost: 64 rows of 50257 x 1600
+        // 61.8 us, so 60.4.  Not volatile: behind an assembly statement that may do anything loads no longer go through the scalar cache.)
         Offset w_to = u * w_jump, a_to = u * a_jump;
-        asm("" : "+s"(w_to), "+s"(a_to));
+        if constexpr (U > 2) asm("" : "+s"(w_to), "+s"(a_to));
         if (u % WP == 0) {
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) {
