@@ -947,9 +947,12 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=F
     3072 36.7 / 38.8, 640 x 6144 x 4096 48.5 / 47.3; beyond it 1024 x 4800 x 1600 31.0 / 29.8, 768 x 6144 x 2048 36.2 / 32.8).  Those are heads of 64
     and 128; of 80 and 48, whose keys and values the kernel stores call by call, 768 x 4800 x 1600 takes 24.8 / 28.2, 640 x 3840 x 1280
     19.6 / 18.9, 1024 x 3840 x 1280 21.5 / 21.9, 768 x 4608 x 1536 24.6 / 25.1.
-    With the GELU that the library has too (``gelu``) while a tile of 64 x 64 finds a unit of its own: a lane's 32 values of a tile of 64 x 128, of which
-    every one is some forty instructions, show (300 x 3072 x 768 8.1 / 8.3, 640 x 1600 x 1600 10.5 / 12.2; beyond it 400 x 3072 x 768 11.6 / 10.0, 300 x 4096 x
-    1024 12.7 / 10.7, 1600 x 1024 x 1024 12.9 / 11.1; prompts of 400 tokens of GPT-2 small 713 / 702, of medium 1,633 / 1,610).  A K below 512 (not measured) and columns that are no multiple of
+    With the GELU that the library has too (``gelu``) while a tile of 64 x 64 finds a unit of its own (weights from memory: 300 x 3072 x 768 6.9 / 8.3, 640 x 1600 x
+    1600 9.3 / 12.0, 1024 x 1024 x 1024 7.4 / 9.4).  That line was drawn when every value of a lane went through the code of all activations; with one choice
+    for a tile the tile kernel is the faster way beyond it too, while a tile of 64 x 128 finds a unit (400 x 3072 x 768 8.8 / 9.8, 640 rows 9.3 / 9.8, 300 x 4096 x 1024
+    12.0 / 13.6, 512 rows 12.3 / 13.9, 300 x 6400 x 1600 16.8 / 19.0, 1600 x 1024 x 1024 10.2 / 11.0) and no longer with more tiles than that (768 x 3072 x 768 12.3 / 11.1, 610 x 4096 x 1024 15.4 / 15.0,
+    384 x 6400 x 1600 21.6 / 20.9, 1295 x 4096 x 1024 26.4 / 24.0).  The line stays all the same: the two add a product up in different orders, and steps of these
+    rows keep the results that they have.  A K below 512 (not measured) and columns that are no multiple of
     eight (not stored in whole rows) are the library's.  Rows count in whole tiles of 64 and 128 only: steps of one class (``engine.step.token_capacity``)
     choose alike."""
     if deep_form_rows(m, k, lda, n, sliced, scatters):
