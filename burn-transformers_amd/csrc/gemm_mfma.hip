@@ -570,9 +570,10 @@ gemm_skinny_kernel(SkinnyOperands o, Epilogue epi, NormOperand norm) {
         // (a place's lanes add their offsets here and not before the batch's first load, which kept them all in registers at once: the forms of
         // eight chunks and two blocks took 138, so that one work-group of theirs shared a compute unit with no other.  18432 x 2048, nine rows
         // 18.7 us, so 16.5.  Batches of two chunks have the registers, and the additions between their loads only cost: 64 rows of 50257 x 1600
-        // 61.8 us, so 60.4.  Not volatile: behind an assembly statement that may do anything loads no longer go through the scalar cache.)
+        // 61.8 us, so 60.4; nor do the plain epilogues' forms with several chunks a load need it: eight rows of 18432 x 2048 19.5, so 19.0, while into the
+        // cache one row of 9216 x 3072 takes 13.5 with it and 15.7 without.  Not volatile: behind an assembly statement that may do anything loads no longer go through the scalar cache.)
         Offset w_to = u * w_jump, a_to = u * a_jump;
-        if constexpr (U > 2) asm("" : "+s"(w_to), "+s"(a_to));
+        if constexpr (U > 2 && (AP == 1 || KIND != EPILOGUE_COMMON)) asm("" : "+s"(w_to), "+s"(a_to));
         if (u % WP == 0) {
 #pragma unroll
           for (int nt = 0; nt < NT; ++nt) {
