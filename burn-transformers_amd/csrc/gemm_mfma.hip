@@ -3,11 +3,11 @@
 // 32-bit: no reduced-precision mode exists in them; products made of parts: see gemm_tile_parts_kernel).  Both operands are K-contiguous, which is
 // what an MFMA lane wants: consecutive K values in one 16-byte load.
 //
-//   gemm_tile    tiles of 64 x 64 to 128 x 256 for many rows (prefill): gemm_tile_pipe_kernel, whose
-//                operands go straight into LDS and whose loop is tile.h's; gemm_tile_kernel for any K
-//                and operands of 4 GiB and more, through registers.  Tiles are numbered so that each XCD's L2
-//                sees neighbours.  Float products of many tiles are made of the products of three
-//                bfloat16 parts of each operand (gemm_tile_parts_kernel).
+//   gemm_tile    tiles for many rows (prefill): of 64 x 96 to 256 x 160 (gemm_tile_blocks_kernel) and of 64 x 64
+//                (gemm_tile_pipe_kernel), whose operands go straight into LDS and whose loops are tile.h's;
+//                gemm_tile_kernel for any K and operands of 4 GiB and more, through registers.  Tiles are
+//                numbered so that each XCD's L2 sees neighbours.  Float products of many tiles are made of
+//                the products of three bfloat16 parts of each operand (gemm_tile_parts_kernel).
 //   gemm_skinny  up to 64 rows (decode).  The product is bound by streaming W once from HBM:
 //                a work-group owns 16 columns, its eight waves split K, every lane keeps several
 //                16-byte loads of W in flight, v_mfma_f32_16x16x32_bf16 does the arithmetic and
@@ -147,14 +147,11 @@ gemm_tile_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, 
   }
 }
 
-// Tiles of BM x BN on TilePipe (tile.h).  K a multiple of 64 (float: 32), operands below 4 GiB.
-// What bounds it is LDS: a tile of 128 x 128 x 64 moves 32 KiB into it and 64 (four waves) or 96 KiB (eight) out of it, at 128
-// bytes a cycle 750 or 1,000 cycles beside 512 of the matrix instructions; a tile of 128 x 256 1,400 beside 1,024.  Behind that 4.5
-// to 5 us whatever K is: launch, first loads, last stores.  Measured (us; in brackets the forms this one replaced, whose loop copied
-// its accumulators and whose epilogue waited for memory sixteen times, and the vendor's library; bias included): 300 x 3072 x 1024
-// 7.1 (10.4, 9.4); 566 x 1024 x 1024 into the residual stream 7.8 (11.8, 9.4); 566 x 4096 x 1024 12.8 (17.6, 13.7); 566 x
-// 1024 x 4096 16.8 (29.6, 18.1); 1295 x 1024 x 1024 10.4 (23.6, 11.2); 1295 x 4096 x 1024 20.1 (25.9, 21.1); 2048 x 1600 x 1600 20.5
-// (32.4, 22.0); 2048 x 1600 x 6400 59 (75, 60); 2048 x 4800 x 1600 45.6 (59, 38); 4096 x 4096 x 4096 138 (179, 93).
+// Tiles of 64 x 64 on TilePipe (tile.h).  K a multiple of 64 (float: 32), operands below 4 GiB.  Few rows, where a tile's start and end are
+// most of it: on four waves half a microsecond less than on the eight of BlockPipe (bias included, us: 300 x 3072 x 1024 7.1, the vendor's
+// library 9.4; 566 x 1024 x 1024 into the residual stream 7.7 / 9.3; 566 x 1024 x 4096 17.4 / 18.2).  Larger tiles were 128 x 128 and 128 x 256 of
+// blocks of 32 x 32 on this loop, whose waves wait for the reads that they have just asked for: 2048 x 4800 x 1600 50 us, BlockPipe 34; 1295 x 4096 x 1024
+// 23 / 20; 1600 x 1600 x 6400 53 / 46.
 template <typename T, int BM, int BN, int WM, int WN, int STAGES>
 __global__ void __launch_bounds__(WM * WN * 64, 2)
 gemm_tile_pipe_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
@@ -190,6 +187,48 @@ gemm_tile_pipe_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict_
   __syncthreads();
   epilogue_tile<T, Pipe::TM, Pipe::TN>(epi, M, N, m_base + wave % WM * (BM / WM), n_base + wave / WM * (BN / WN), acc, split,
                                        lds + wave * tile_scratch_bytes<Pipe::TM, Pipe::TN>());
+}
+
+// Tiles of BM x BN on BlockPipe (tile.h), which take a compute unit whole.  A tile is as large as leaves most units one: what bounds
+// it is what a unit can pull, 32 KiB under way at a time, so 256 x 160 x 64 takes 0.8 us where the matrix instructions alone need 0.72 and 128 x 128
+// x 64 0.45 where they need 0.31; around that 5 to 11 us of first loads (2), last stores (1 to 4) and launch, the epilogue
+// straight out of registers.  Measured with operands from memory (us, in brackets TilePipe's best form and the vendor's library):
+// 2048 x 4800 x 1600 with keys and values into the cache 34 (50, 47); 1295 x 3072 x 1024 likewise 16.6 (20, 24.7); 1959 x 1024 x 4096 into
+// the residual stream 27 (28, 30); 1295 x 4096 x 1024 with a GELU 20.3 (23, 23.8); 4096 x 1600 x 6400 87 (99, 95).
+// Tried: tiles of 256 x 208 and 256 x 256 (2048 x 6400 x 1600 42 us without an epilogue, the library 37, with one 164 registers spilled); a ninth wave that
+// asks for lines some turns ahead (55.8 -> 55.7 at 2048 x 1600 x 6400: requests bound it); W packed by tiles (2 to 8 % faster, a third copy of the weights).
+template <typename T, int BM, int BN, int WM, int WN, int SA, int SW>
+__global__ void __launch_bounds__(WM * WN * 64, 2)
+gemm_tile_blocks_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int M, int N,
+                        int K, Epilogue epi, int tiles_m, int tiles_n, int group_m) {
+  typedef BlockPipe<T, BM, BN, WM, WN, SA, SW> Pipe;
+  constexpr int ROW_K = 8 * Mma<T>::ELEMS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // SA stages of A's rows, SW of W's
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
+  const int per_group = group_m * tiles_n, first = tile / per_group * group_m, rest = tile % per_group;
+  const int rows_m = group_m < tiles_m - first ? group_m : tiles_m - first;
+  const int m_base = (first + rest % rows_m) * BM, n_base = rest / rows_m * BN;
+  const int split = blockIdx.z, splits = gridDim.z;
+  const int k_tiles = K / ROW_K;
+  const int kt_begin = (int)((int64_t)k_tiles * split / splits);
+  const int count = (int)((int64_t)k_tiles * (split + 1) / splits) - kt_begin;
+  floatx4 acc[Pipe::TN][Pipe::TM];
+#pragma unroll
+  for (int bn = 0; bn < Pipe::TN; ++bn)
+#pragma unroll
+    for (int bm = 0; bm < Pipe::TM; ++bm) acc[bn][bm] = floatx4{0.f, 0.f, 0.f, 0.f};
+  Pipe::template multiply<unsigned>(
+      lds, reinterpret_cast<const unsigned char*>(A) + (int64_t)kt_begin * TILE_ROW_BYTES,
+      reinterpret_cast<const unsigned char*>(W) + (int64_t)kt_begin * TILE_ROW_BYTES, count,
+      [&](int tile_row, bool from_w) {
+        const int row = (from_w ? n_base : m_base) + tile_row, limit = from_w ? N : M;
+        return (int64_t)(row < limit ? row : limit - 1) * (from_w ? (int64_t)K : lda) * (int64_t)sizeof(T);
+      },
+      acc);
+  __syncthreads();
+  epilogue_blocks<T, Pipe::TM, Pipe::TN>(epi, M, N, m_base + wave % WM * (BM / WM), n_base + wave / WM * (BN / WN), acc, split,
+                                         lds + wave * block_scratch_bytes<Pipe::TM, Pipe::TN>());
 }
 
 // Float products of many rows on the bfloat16 matrix instructions, sixteen times the rate of the float ones.
@@ -819,6 +858,23 @@ static int launch_pipe(hipStream_t s, const T* a, int64_t lda, const T* w, int M
   return bt_check_launch("gemm_tile");
 }
 
+template <int BM, int BN, int WM, int WN, int SA, int SW, typename T>
+static int launch_blocks(hipStream_t s, const T* a, int64_t lda, const T* w, int M, int N, int K, const Epilogue& epi, int splits) {
+  typedef BlockPipe<T, BM, BN, WM, WN, SA, SW> Pipe;
+  auto kernel = gemm_tile_blocks_kernel<T, BM, BN, WM, WN, SA, SW>;
+  static_assert(WM * WN * block_scratch_bytes<Pipe::TM, Pipe::TN>() <= Pipe::BYTES, "the epilogue's rows fit into the stages");
+  static bool raised = false;
+  if (!raised) {
+    hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Pipe::BYTES);
+    if (err != hipSuccess) BT_REFUSE("gemm_tile: cannot get %d bytes of LDS: %s", Pipe::BYTES, hipGetErrorString(err));
+    raised = true;
+  }
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n, 1, splits), dim3(WM * WN * 64), Pipe::BYTES, s, a, lda, w, M, N, K, epi, tiles_m,
+                     tiles_n, tile_group(tiles_m, tiles_n, splits, BM, BN));
+  return bt_check_launch("gemm_tile");
+}
+
 template <int BM, int BN, int WM, int WN>
 static int launch_parts_form(hipStream_t s, const float* a, int64_t lda, const float* w, int M, int N, int K,
                              const Epilogue& epi, int splits) {
@@ -842,20 +898,23 @@ static int launch_form(hipStream_t s, int variant, const bf16_t* a, int64_t lda,
   // A long K with one tile to a unit at most: the LDS is its own, and more tiles on their way hide more of the weights' way from
   // memory (cold weights, us: 200 x 1600 x 6400 28.1 -> 24.8; a shorter K pays for the longer start: 290 x 2048 x 1024 6.6 -> 7.3,
   // and prompts of 220 tokens at width 1,024, whose K is 2,048 at most, 1,009 -> 1,017).
-  auto alone = [&](int bm, int bn) {
-    return K / TILE_K / splits >= 48 && (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * splits <= 256;
-  };
+  const bool alone = K / TILE_K / splits >= 48 && (int64_t)((M + 63) / 64) * ((N + 63) / 64) * splits <= 256;
   switch (variant) {
-    case 2: return launch_pipe<128, 128, 2, 2, 2>(s, a, lda, w, M, N, K, epi, splits);
-    case 3: return launch_pipe<128, 128, 2, 4, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 2: return launch_blocks<128, 128, 4, 2, 4, 6>(s, a, lda, w, M, N, K, epi, splits);
+    case 3: return launch_blocks<256, 160, 4, 2, 3, 3>(s, a, lda, w, M, N, K, epi, splits);
     case 4: return launch_pipe<64, 64, 2, 2, 3>(s, a, lda, w, M, N, K, epi, splits);
     case 5:
-      if (alone(64, 64)) return launch_pipe<64, 64, 2, 2, 8>(s, a, lda, w, M, N, K, epi, splits);
+      if (alone) return launch_pipe<64, 64, 2, 2, 8>(s, a, lda, w, M, N, K, epi, splits);
       return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
-    case 6:
-      if (alone(64, 128)) return launch_pipe<64, 128, 1, 4, 6>(s, a, lda, w, M, N, K, epi, splits);
-      return launch_pipe<64, 128, 1, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
-    case 7: return launch_pipe<128, 256, 2, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 6: return launch_blocks<64, 128, 2, 4, 8, 5>(s, a, lda, w, M, N, K, epi, splits);
+    case 7: return launch_blocks<128, 256, 2, 4, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
+    case 8: return launch_blocks<64, 96, 4, 2, 8, 6>(s, a, lda, w, M, N, K, epi, splits);
+    case 9: return launch_blocks<128, 64, 4, 2, 5, 8>(s, a, lda, w, M, N, K, epi, splits);
+    case 10: return launch_blocks<128, 96, 4, 2, 5, 6>(s, a, lda, w, M, N, K, epi, splits);
+    case 11: return launch_blocks<128, 160, 4, 2, 4, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 12: return launch_blocks<128, 192, 2, 4, 4, 4>(s, a, lda, w, M, N, K, epi, splits);
+    case 13: return launch_blocks<256, 96, 4, 2, 3, 5>(s, a, lda, w, M, N, K, epi, splits);
+    case 14: return launch_blocks<256, 128, 4, 2, 3, 4>(s, a, lda, w, M, N, K, epi, splits);
   }
   BT_REFUSE("gemm_tile: unknown form %d", variant);
 }
@@ -870,28 +929,10 @@ static int launch_form(hipStream_t s, int variant, const float* a, int64_t lda, 
   BT_REFUSE("gemm_tile: unknown form %d", variant);
 }
 
-// Which form a bfloat16 product takes: the one whose busiest compute unit is done first.  A unit with n tiles needs, for every 64
-// values of K, 0.17 us a tile of 64 x 64 (0.2 from three on, when three work-groups of three stages share its LDS: up to two have four
-// stages), 0.28 / 0.62 / 0.33 n for one / two / more tiles of 64 x 128, 0.5 for 128 x 128 on eight waves (one work-group a unit),
-// 0.8 / 0.52 n for one / more on four waves (two work-groups), 0.9 for 128 x 256 (one); around that the fixed times below.  Within 15 % of what
-// 300 to 4,096 rows, 1,024 to 6,400 columns and K of 1,024 to 6,400 measured (figures with the kernel).
-static int tile_form(int M, int N, int K, int splits) {
-  const float turns = (float)(K / TILE_K) / splits;
-  auto share = [&](int bm, int bn) { return (float)(((int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * splits + 255) / 256); };
-  const float small = share(64, 64), tall = share(64, 128), square = share(128, 128), wide = share(128, 256);
-  const float cost[5] = {4.6f + turns * (small <= 2 ? 0.17f : 0.2f) * small, 5.f + turns * (tall <= 1 ? 0.28f : tall <= 2 ? 0.62f : 0.33f * tall),
-                         2.5f + square * (2.8f + 0.5f * turns), 5.5f + turns * (square <= 1 ? 0.8f : 0.52f * square),
-                         3.f + wide * (3.5f + 0.9f * turns)};
-  const int form[5] = {small <= 2 ? 5 : 4, 6, 3, 2, 7};
-  int best = 0;
-  for (int i = 1; i < 5; ++i)
-    if (cost[i] < cost[best]) best = i;
-  return form[best];
-}
-
 // dtype: 0 float, 1 bfloat16 (the codes of every entry point that takes both).
-// variant: 0 = the fastest form the operands allow; 1 = the general form; 2 .. 7 = launch_form's (asked for by tests and
-// measurements; a form that cannot take the operands is refused; float has the general form, 5 (4 is the same), 6 and 7).
+// variant: 1 = the general form; 2 .. 14 = launch_form's (a form that cannot take the operands is refused; float has the general form, 5 (4 is
+// the same), 6 and 7); 0 = of float products the fastest form the operands allow, of bfloat16 ones the tiles of 64 x 64 where they can be
+// taken (which form is the fastest is the caller's to say: kernels/library.py, tile_form).
 // Float products take the tiles of 64 x 64 or the forms on parts wherever K is a multiple of 32 (the template's tile of 128 x 128
 // takes a compute unit 2.4 us for 32 values of K and leaves most units idle where there are few tiles).  While the tiles of
 // 64 x 64 have a unit each, they win: 0.65 us for 32 values of K where a tile of 128 x 64 on parts takes 0.73 (65 x 768 x 3072 62
@@ -925,7 +966,7 @@ BT_EXPORT int bt_gemm_tile(void* stream, int dtype, const void* A, int64_t lda, 
   const bf16_t* w = (const bf16_t*)W;
   const int64_t four_gib = (int64_t)1 << 32;
   const bool whole_ok = K % TILE_K == 0 && (int64_t)M * lda * 2 < four_gib && (int64_t)N * K * 2 < four_gib;
-  if (variant == 0) variant = whole_ok ? tile_form(M, N, K, splits) : 1;
+  if (variant == 0) variant = whole_ok ? 5 : 1;
   if (variant != 1) {
     if (!whole_ok) BT_REFUSE("gemm_tile: this form needs K %d to be a multiple of 64 and operands below 4 GiB", K);
     return launch_form(s, variant, a, lda, w, M, N, K, *epi, splits);

@@ -160,3 +160,121 @@ struct TilePipe {
     wait_vmcnt<0>();
   }
 };
+
+// The same product on blocks of 16 x 16, for tiles that take a compute unit's LDS and registers whole: WM x WN waves, each TM x TN blocks,
+// SA tiles of A's rows and SW tiles of W's in LDS or on their way (W, which comes from memory, may be asked for further ahead than A,
+// which the kernel before left in the caches).  Differences from TilePipe, each measured at 2048 x 4800 x 1600 on 256 x 160 and 2048 x 6400 x
+// 1600 on 256 x 256 (weights from memory):
+//   reads     of the next half tile stand one before each of the first matrix instructions of this half, behind a wait that the
+//             compiler knows: with reads in front of them it waited for those as well (lgkmcnt(0)), a trip to LDS every half
+//   loads     of the tile after the last one in LDS stand between the matrix instructions of the half behind the barrier: eight
+//             waves that ask for all theirs at once wait for the address unit (33.7 -> 32.3 us)
+//   stages    two of A and three of W in 160 KiB where three of both do not fit (46.9 -> 42.2 us)
+// What a compute unit has asked for and not got is 32 KiB at most, however many stages there are: 150 GB/s out of L2, 95 from the
+// memory-side cache and 65 from memory, so a tile wants 2 * BM * BN / (BM + BN) operations a byte and one round of tiles over the
+// chip (figures of the forms with the kernels).
+template <typename T, int BM, int BN, int WM, int WN, int SA, int SW>
+struct BlockPipe {
+  static constexpr int WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
+  static constexpr int A_GROUPS = BM / 8, W_GROUPS = BN / 8;               // a wave's load instruction: eight rows
+  static constexpr int A_LOADS = A_GROUPS / WAVES, W_LEAST = W_GROUPS / WAVES, W_LOADS = (W_GROUPS + WAVES - 1) / WAVES;
+  static constexpr int LOADS = A_LOADS + W_LOADS;
+  static constexpr int A_STAGE = BM * TILE_ROW_BYTES, W_STAGE = BN * TILE_ROW_BYTES, BYTES = SA * A_STAGE + SW * W_STAGE;
+  static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0 && A_GROUPS % WAVES == 0 && SA >= 2 && SW >= 2 && BYTES <= 160 * 1024,
+                "whole blocks, whole loads of A, and what LDS holds");
+  // Loads that may still be on their way when the tile behind the barrier has landed: those behind its A (issued with W of the
+  // same turn, then whole turns) and behind its W.  (Waves with one load of W less than others wait for as many fewer.)
+  static constexpr int A_BEHIND = (SA - 2) * (A_LOADS + W_LEAST) + W_LEAST, W_BEHIND = (SW - 2) * (A_LOADS + W_LEAST);
+  static constexpr int BEHIND = A_BEHIND < W_BEHIND ? A_BEHIND : W_BEHIND;
+  static_assert((SA > SW ? SA : SW) * LOADS < 64, "no more loads in flight than the wave's counter holds");
+
+  // acc += the product of `count` tiles; row_bytes(row of the tile, of W): what that row's first byte lies behind `a` or `w`.
+  // On return every wave's loads have landed and nobody reads the stages any more once all have passed the next barrier.
+  template <typename Offset, typename RowBytes>
+  static __device__ __forceinline__ void multiply(unsigned char* lds, const unsigned char* a, const unsigned char* w, int count,
+                                                  RowBytes row_bytes, floatx4 (&acc)[TN][TM]) {
+    if (count <= 0) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave % WM, wn = wave / WM, i16 = lane & 15, g = lane >> 4;
+    Offset off[LOADS];
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const bool from_w = j >= A_LOADS;
+      const int row = 8 * ((from_w ? j - A_LOADS : j) * WAVES + wave) + (lane >> 3);
+      off[j] = (Offset)(row_bytes(row, from_w) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+    }
+    auto load = [&](int j, int a_stage, int w_stage) {
+      const bool from_w = j >= A_LOADS;
+      const int group = (from_w ? j - A_LOADS : j) * WAVES + wave;
+      if (!from_w || (j - A_LOADS + 1) * WAVES <= W_GROUPS || group < W_GROUPS)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)((from_w ? w : a) + off[j]),
+                                         (__attribute__((address_space(3))) void*)(lds + (from_w ? SA * A_STAGE + w_stage * W_STAGE : a_stage * A_STAGE) +
+                                                                                   group * (8 * TILE_ROW_BYTES)),
+                                         16, 0, 0);
+    };
+    int a_issued = 0, w_issued = 0;        // (behind the last tile the last one is asked for again)
+    auto a_next = [&]() { a += ++a_issued < count ? TILE_ROW_BYTES : 0; };
+    auto w_next = [&]() { w += ++w_issued < count ? TILE_ROW_BYTES : 0; };
+    int a_rd[2], w_rd[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      a_rd[half] = swizzled(wm * (BM / WM) + i16, 4 * half + g);
+      w_rd[half] = SA * A_STAGE + swizzled(wn * (BN / WN) + i16, 4 * half + g);
+    }
+    int4v op[2][TM + TN];
+    auto read = [&](int r, int half, int a_stage, int w_stage) {
+      op[half][r] = *reinterpret_cast<const int4v*>(lds + (r < TM ? a_stage * A_STAGE + a_rd[half] + r * (16 * TILE_ROW_BYTES)
+                                                                 : w_stage * W_STAGE + w_rd[half] + (r - TM) * (16 * TILE_ROW_BYTES)));
+    };
+    // Multiplies half a tile, reads the other half of the tile in the stages, or of the next tile, and asks for a tile.
+    auto multiply_half = [&](int half, bool reads, bool loads, int a_read, int w_read, int a_free, int w_free) {
+      constexpr int BLOCKS = TM * TN;
+      __builtin_amdgcn_s_waitcnt(0xc07f);                    // lgkmcnt(0): this half's operands, asked for half a tile ago
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < BLOCKS; ++x) {
+#pragma unroll
+        for (int r = 0; r < TM + TN; ++r)
+          if (reads && r * BLOCKS / (2 * (TM + TN)) == x) read(r, half ^ 1, a_read, w_read);
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j)
+          if (loads && (2 * j + 1) * BLOCKS / (2 * LOADS) == x) load(j, a_free, w_free);
+        __builtin_amdgcn_sched_barrier(0);
+        Mma<T>::block16(acc[x / TM][x % TM], op[half][TM + x / TM], op[half][x % TM]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < (SA > SW ? SA : SW); ++t) {
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j)
+        if (j < A_LOADS ? t < SA : t < SW) load(j, t, t);
+      if (t < SA) a_next();
+      if (t < SW) w_next();
+    }
+    wait_vmcnt<(SA - 1) * A_LOADS + (SW - 1) * W_LEAST>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < TM + TN; ++r) read(r, 0, 0, 0);
+    multiply_half(0, true, false, 0, 0, 0, 0);
+    int a_stage = 0, a_then = 1, w_stage = 0, w_then = 1;
+    for (int i = 1; i < count; ++i) {
+      // this wave's loads of the next tile have landed and its reads of this one are done: behind the barrier so have everyone's
+      __builtin_amdgcn_s_waitcnt((BEHIND & 15) | (BEHIND >> 4) << 14 | 0x70);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      multiply_half(1, true, true, a_then, w_then, a_stage, w_stage);
+      a_next();
+      w_next();
+      a_stage = a_then;
+      a_then = a_then + 1 == SA ? 0 : a_then + 1;
+      w_stage = w_then;
+      w_then = w_then + 1 == SW ? 0 : w_then + 1;
+      multiply_half(0, true, false, a_stage, w_stage, 0, 0);
+    }
+    multiply_half(1, false, false, 0, 0, 0, 0);
+    wait_vmcnt<0>();
+  }
+};

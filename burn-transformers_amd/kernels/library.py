@@ -6,6 +6,7 @@ that a kernel does not take raises :class:`KernelError` with the kernel's own me
 """
 
 import ctypes
+import functools
 import os
 import sys
 import threading
@@ -625,8 +626,7 @@ def library_products():
     """The module that runs prompt-sized bfloat16 products through hipBLASLt, or None.
 
     The reference leaves its matrix products to its backend's library (src/attention.rs:481-513
-    and the feed-forward call ``linear``); here the vendor's library takes the large products (``own_tiles`` says which;
-    1.2 to 1.5 times as fast as the tile kernel of this package at 2,048 rows of GPT-2 XL's wide matrices), and
+    and the feed-forward call ``linear``); here the vendor's library takes large products (``tile_kernel_takes`` says which), and
     the hand-written kernels keep everything else.  The library is
     opened from the copy that came with torch's HIP runtime and checked once against the tile
     kernel; if it cannot be opened, or disagrees, the tile kernel does those products too, and
@@ -847,7 +847,7 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
     library where it is usable and has the epilogue; float32 operands that are not multiples of
     four wide go to the plain kernel), or one of "plain", "tile", "skinny", "library" to force one.
     variant picks one of the tile kernel's forms (0: the fastest the operands allow, 1: any K,
-    2 to 7: others, see ``bt_gemm_tile``) or, for the skinny kernel, the output columns a work-group owns
+    2 to 14: others, see ``TILE_FORMS`` and ``bt_gemm_tile``) or, for the skinny kernel, the output columns a work-group owns
     (8, 12, ... 32; 0: chosen for balance).  ``a`` may be a :class:`Normalized`.
     packed: a :class:`PackedWeight` of ``w`` (or directly (``pack_columns(w, columns)``, columns)), read in
     place of ``w`` where the skinny kernel runs and the copy fits the step.
@@ -882,8 +882,8 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
             impl = "skinny"
         elif dtype == FLOAT32:
             impl = "tile"
-        elif own_tiles(m, n, k, a.stride(0), sliced=splits > 1, scatters=epilogue.mode == EPI_QKV,
-                       residual=epilogue.mode == EPI_RESIDUAL, gelu=epilogue.mode == EPI_ACT and _library_takes(epilogue)):
+        elif tile_kernel_takes(m, n, k, a.stride(0), sliced=splits > 1, scatters=epilogue.mode == EPI_QKV,
+                               residual=epilogue.mode == EPI_RESIDUAL, gelu=epilogue.mode == EPI_ACT and _library_takes(epilogue)):
             impl = "tile"
         else:
             impl = "library" if splits == 1 and _library_takes(epilogue) and library_products() \
@@ -904,6 +904,8 @@ def gemm(a, w, epilogue, splits=1, impl="auto", variant=0, packed=None):
             raise KernelError("gemm: the library product does not split K")
         _launch(lib, "bt_gemm_library_call", call)
     elif impl == "tile":
+        if variant == 0 and dtype == BFLOAT16 and _tile_operands(m, n, k, a.stride(0)):
+            call.variant = tile_form(-(-m // 64), n, k, splits)[1]
         _launch(_module("gemm_mfma"), "bt_gemm_tile_call", call)
     else:
         call.a_rows = a_rows
@@ -967,6 +969,59 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=F
     return tiles(64, 128) <= (OWN_SCATTER_TILES if scatters else OWN_TILES) or (residual and tiles(128, 128) <= OWN_RESIDUAL_TILES)
 
 
+def _tile_operands(m, n, k, lda):
+    """Whether the tile kernel's forms take the operands: K in tiles of 64, addresses of 32 bits."""
+    return k % 64 == 0 and m * lda * 2 < (1 << 32) and n * k * 2 < (1 << 32)
+
+
+# Forms of the bfloat16 tile kernel on blocks of 16 x 16 (``bt_gemm_tile``'s variants), of which a compute unit has one tile at a time: a
+# tile's rows and columns, us of a product by itself and for every 64 values of K, and what is added to both where every unit has a
+# tile.  Fitted to graphs of 24 products whose operands and results come from memory or the memory-side cache, 128 to 4,096 rows, 768 to 8,192 columns, K of
+# 768 to 6,400 with every epilogue of prompts (299 products; 5 to 8 % off on average).
+TILE_FORMS = {2: (128, 128, 5.6, 0.385, 0.65, 0.19), 3: (256, 160, 8.4, 0.71, 2.1, 0.3), 7: (128, 256, 7.1, 0.64, 0.0, 0.36),
+              8: (64, 96, 4.65, 0.24, 0.25, 0.085), 9: (128, 64, 4.6, 0.27, 0.45, 0.09), 10: (128, 96, 5.3, 0.33, 0.5, 0.125),
+              11: (128, 160, 6.1, 0.475, 0.75, 0.18), 12: (128, 192, 6.7, 0.515, 0.75, 0.235), 13: (256, 96, 6.8, 0.53, 0.95, 0.21),
+              14: (256, 128, 7.4, 0.61, 1.05, 0.275)}
+
+
+@functools.lru_cache(maxsize=4096)
+def tile_form(rows64, n, k, splits=1, units=256):
+    """(us, variant) of the form whose busiest compute unit is done first, for a product of ``rows64`` times 64 rows (steps of one
+    class choose alike): a form of ``TILE_FORMS``, or tiles of 64 x 64 on four waves, of which up to three share a unit.  Over the 299 products
+    the fastest forms take 6,223 us, those chosen 6,270.  (Large tiles that need every unit are counted 2 us longer: in such a graph they are not, but inside
+    steps 2048 x 4096 x 1024 took 3 to 5 us less on 208 tiles than on 256 and 1959 x 3072 x 1024 2.6 less on 192.)"""
+    turns, share = k / 64 / splits, -(-rows64 * -(-n // 64) * splits // units)
+    costs = [(4.9 + turns * (0.175, 0.42, 0.24 * share)[min(share, 3) - 1] + (0.8 if k >= 3072 else 0.0), 5 if share <= 2 else 4)]
+    for variant, (rows, columns, start, turn, full_start, full_turn) in TILE_FORMS.items():
+        tiles = -(-rows64 * 64 // rows) * -(-n // columns) * splits
+        rounds, filled = -(-tiles // units), min(1.0, tiles / units)
+        us = start + turn * turns + filled * (full_start + full_turn * turns) + (2.0 if filled > 0.94 and rows * columns >= 24576 else 0.0)
+        costs.append((us if rounds == 1 else 1.05 * rounds * us, variant))
+    return min(costs)
+
+
+def tile_kernel_takes(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=False):
+    """Whether a bfloat16 product of more than 64 rows is the tile kernel's: by ``own_tiles``, or where ``tile_form`` says that it is the
+    faster way.  The library's time is taken as a start, its operations at 1.05 PFLOP/s, its K and its results, keys and values copied behind it (8 %
+    off on average, 29 % at most: it jumps as its tiles fill the chip well or not); beside the plain library a twenty-fifth is left for that.
+    Measured (us, tile kernel / library) 2048 x 4800 x 1600 with keys and values scattered 34 / 47, 2048 x 3072 x 1024 19 / 25, 1295 x 3072 x 1024 16.6 /
+    24.7; into the residual stream 1959 x 1600 x 6400 53 / 58, 1959 x 1024 x 4096 27 / 30; the library's 2048 x 6400 x 1600 with a GELU 58 / 44, 1600 x 4096 x
+    1024 22.6 / 22.6, 4096 x 4096 x 1024 48 / 36.  Over the 299 products of ``TILE_FORMS`` the faster of the two ways takes 5,953 us, this choice
+    6,150, ``own_tiles`` alone 6,349."""
+    if own_tiles(m, n, k, lda, sliced, scatters, residual, gelu):
+        return True
+    if m <= 64 or n % 8 or k < OWN_SHORT_K or not _tile_operands(m, n, k, lda):
+        return False
+    results = 1e-6 * m64(m) * n
+    library = 5.9 + 1.9e-9 * m64(m) * n * k + 0.11 * k / 64 + 0.06 * results + (4.5 + 0.5 * results if scatters else 0.16 * results if residual else 0.0)
+    return tile_form(m64(m) // 64, n, k)[0] < (library if scatters else 0.96 * library)
+
+
+def m64(rows):
+    """Rows in whole 64s."""
+    return -(-rows // 64) * 64
+
+
 def deep_split_count(rows, columns, k, units=256):
     """Into how many slices of pending partial sums a residual-writing bfloat16 product of 65 to
     ``DEEP_FORM_SLICED_ROWS`` rows cuts its K range: as many as still give every work-group (a tile
@@ -1014,7 +1069,7 @@ def float_split_count(rows, columns, k, units=256):
 def prompt_products_in_library(m, n, k, lda, scatters=False):
     """Whether a bfloat16 product of a step of ``m`` rows goes to the vendor's library (which cannot
     scatter keys and values into the cache: the caller then copies them)."""
-    return m > 64 and not own_tiles(m, n, k, lda, scatters=scatters) and library_products() is not None
+    return m > 64 and not tile_kernel_takes(m, n, k, lda, scatters=scatters) and library_products() is not None
 
 
 def _library_has_algorithm(lda, m, n, k, epilogue):
@@ -1255,7 +1310,7 @@ def activation_needs_a_pass(a, w, activation):
     there without one, and ``activate`` follows (2,048 rows of 4096 x 1024: 24 + 8 us where the tile kernel with
     the activation in its epilogue takes 43)."""
     if a.dtype != torch.bfloat16 or isinstance(a, (Chunked, Normalized)) or not 64 < a.shape[0] <= 65535 or \
-            own_tiles(a.shape[0], w.shape[0], a.shape[1], a.stride(0)):
+            tile_kernel_takes(a.shape[0], w.shape[0], a.shape[1], a.stride(0)):
         return False
     return activation == "squared_relu" and library_products() is not None
 
