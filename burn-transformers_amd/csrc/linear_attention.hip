@@ -385,8 +385,7 @@ static void launch_keyed_scan(hipStream_t stream, const KeyedScanCall& c) {
 // lanes.  Measured, token by token / in blocks (us; 8 heads of 128 x 128, 2 x 1,024 tokens): delta rule with one decay
 // a head 386 / 78, one a key channel 522 / 82, forget gate (there in spans) 139 / 57; 2 x 128 tokens 52 / 24, 69 / 26,
 // 45 / 18.  The operands take 25 us (18 without T) of the long ones; the walk takes 0.87 us a block (0.63), of which the
-// matrix units are busy for 0.32 (0.21): a wave is alone on its SIMD, and the chain from S0 through LDS and back into S
-// is what is left.
+// matrix units are busy for 0.32 (0.21).  Since then (see KB_AHEAD) the walk takes 0.66 us a block (0.45), and 2 x 1,024 tokens 65 us (46).
 #define KB_TOKENS 16
 
 // Floats of one block and head: W, R and ku [tiles of 16 channels][64 lanes][4], T v [tiles of 16 values][64][4], a_B [dim].
@@ -618,38 +617,196 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
 
 // One work-group per 16 value channels of a head and sequence: four waves share the key channels (TW tiles of 16 each),
 // every wave's part of W S0 and R S0 meets in LDS.  The operands of the next KB_AHEAD - 1 blocks are on their way.
+// What bounds a block is one wave's chain on each SIMD: 24 matrix instructions (16 without W) of 32 cycles, the exchange, and the address unit,
+// which four waves' loads take 450 cycles (so: no load of what another wave has, a decay a lane and not four of which a quad's lanes all have
+// the same; a load behind each matrix instruction, the exchange while R S0 runs).  How far ahead they are asked for makes no difference (2, 4
+// and 6 blocks alike).  The loop takes whole turns of KB_AHEAD and the rest stands behind it: with a way out between two blocks the
+// compiler's waits in front of a turn are those of every way into it, and all loads are waited for.  Measured (us, 8 heads of 128 x 128, 2 x
+// 1,024 tokens, the walk alone): delta rule 56.9 -> 42.1, forget gate 40 -> 28.7.
 #define KB_AHEAD 4
+
+template <int N>
+struct Number {
+  static constexpr int value = N;
+};
+
+// f(Number<0>()) .. f(Number<N - 1>()): steps whose numbers choose code.
+template <int N, int FROM = 0, typename F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (FROM < N) {
+    f(Number<FROM>());
+    each<N, FROM + 1>(f);
+  }
+}
 
 template <int FORM, int TW>
 struct KbStage {
-  floatx4 w[FORM == 0 ? TW : 1], r[TW], ku[TW], a[TW], u;
-  float o;
+  floatx4 w[FORM == 0 ? TW : 1], r[TW], ku[TW];
+  float a[TW], o;
+  typename std::conditional<FORM == 0, float, floatx4>::type u;   // of T v the wave's quarter, or all of v
 };
 
-template <int FORM, int DT>
+// Spans of blocks (the forget gate).  A walk of few columns leaves compute units idle and the others with one wave to a SIMD, whose
+// chain from block to block is what the time is.  Its step is linear in S, so long sequences are cut into spans of c.span
+// tokens ("Spans" in scan.h): keyed_spans_kernel leaves the state behind every span but a sequence's last, the first one's from the
+// slot's state and the others' from zero, and their products of decays; the walk then takes every span side by side, from
+// the state that those add up to.  A span from zero is one product a block (u is v), without barriers.
+// Measured with the blocks' operands (us, whole sequences / in spans; 8 heads of 128 x 128): 2 x 1,024 tokens 45.5 / 45.1, 2,048 67.8 / 43.6,
+// 1,000 37.6 / 30.5, 640 28.2 / 26.4; 16 heads, 2,000 tokens 75.9 / 65.4; 8 heads of 64 x 64, 2,048 42.8 / 25.7.
+__device__ __forceinline__ int64_t kb_span_floats(const KeyedScanCall& c) { return (int64_t)c.heads * c.dim * c.vdim + (int64_t)c.heads * c.dim; }
+
+// The operands of a wave's TW tiles of key channels of a block that the state's update takes.
+template <int TW>
+struct KbUpdate {
+  floatx4 ku[TW], u;
+  float a[TW];
+};
+
+// Four channels' rows of S times their decays, of which a quad's four lanes hold one each.
+__device__ __forceinline__ void decay(floatx4& s, float a) {
+  s[0] *= dpp_move<0x00>(a);
+  s[1] *= dpp_move<0x55>(a);
+  s[2] *= dpp_move<0xAA>(a);
+  s[3] *= dpp_move<0xFF>(a);
+}
+
+template <int DT>
+__global__ void __launch_bounds__(256, 2) keyed_spans_kernel(KeyedScanCall c) {
+  constexpr int TW = (DT + 3) / 4, DIM = 16 * DT;
+  const int columns = c.vdim / 16, pair = blockIdx.x / (8 * columns) * 8 + blockIdx.x % 8;
+  const int column = blockIdx.x / 8 % columns, head = pair % c.heads;
+  int part;
+  const int seq = piece_sequence(c.seq_off, c.n_seqs, c.tokens, c.max_count, c.span, pair / c.heads, part);
+  if (seq < 0 || (part + 1) * c.span >= c.seq_off[seq + 1] - c.seq_off[seq]) return;   // nothing stands behind a sequence's last span
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
+  const int blocks = c.span / KB_TOKENS, vtiles = c.vdim / 4, p = 16 * column + n;
+  const int64_t stride = (int64_t)c.heads * kb_floats(DIM, c.vdim) * 4, of_head = ((int64_t)head * vtiles + p / 4) * DIM * 4 + p % 4;
+  const char* at = reinterpret_cast<const char*>(kb_place(c, seq, part * blocks, head));
+  float* const end = c.carry + span_block(c.seq_off, seq, c.span, part) * kb_span_floats(c);
+  uint32_t from_tile[TW], from_decay[TW];
+#pragma unroll
+  for (int j = 0; j < TW; ++j) {
+    const int tile = min(wave * TW + j, DT - 1);
+    from_tile[j] = (KB_TOKENS * 2 * DIM + 256 * tile + 4 * lane) * 4;
+    from_decay[j] = (KB_TOKENS * (3 * DIM + c.vdim) + 16 * tile + 4 * g + (n & 3)) * 4;
+  }
+  uint32_t from_u = (KB_TOKENS * 3 * DIM + 256 * column + 4 * lane) * 4;
+  KbUpdate<TW> stages[KB_AHEAD];
+  int fetched = 0;
+  auto load = [&](uint32_t& from) {                        // (as in the walk)
+    asm volatile("" : "+v"(from));
+    return (const __attribute__((address_space(1))) char*)at + from;
+  };
+  auto fetch = [&](KbUpdate<TW>& st) {
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      st.ku[j] = *reinterpret_cast<const __attribute__((address_space(1))) floatx4*>(load(from_tile[j]));
+      st.a[j] = *reinterpret_cast<const __attribute__((address_space(1))) float*>(load(from_decay[j]));
+    }
+    st.u = *reinterpret_cast<const __attribute__((address_space(1))) floatx4*>(load(from_u));
+    at += ++fetched < blocks ? stride : 0;                 // (at the end the last block's again, not used)
+  };
+  auto mine = [&](int j) { return DT % 4 == 0 || wave * TW + j < DT; };
+  floatx4 S[TW];
+  float P[TW];                                             // of channel 4 g + n % 4
+#pragma unroll
+  for (int i = 0; i < KB_AHEAD - 1; ++i) {
+    fetch(stages[i]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto row = [&](int j, int i) { return of_head + (int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4; };
+#pragma unroll
+  for (int j = 0; j < TW; ++j) {
+    P[j] = 1.f;
+    S[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (part == 0) {                                         // the slot's state, kept for the walk (whose last span writes the slot)
+    const float* slot = c.S + (int64_t)c.slots[seq] * c.state_stride;
+    float* const kept = end - kb_span_floats(c);
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+      if (mine(j))
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[j][i] = slot[row(j, i)];
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+      if (mine(j))
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kept[row(j, i)] = S[j][i];
+  }
+  landed(S);
+  auto step = [&](const KbUpdate<TW>& st) {
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      decay(S[j], st.a[j]);
+      P[j] *= st.a[j];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        if (mine(j)) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.ku[j][i], st.u[i], S[j], 0, 0, 0);
+  };
+  int block = 0;
+  for (; block + KB_AHEAD <= blocks; block += KB_AHEAD) {
+#pragma unroll
+    for (int i = 0; i < KB_AHEAD; ++i) {
+      fetch(stages[(i + KB_AHEAD - 1) % KB_AHEAD]);
+      __builtin_amdgcn_sched_barrier(0);
+      step(stages[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < KB_AHEAD - 1; ++i)
+    if (block + i < blocks) step(stages[i]);
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+    if (mine(j))
+#pragma unroll
+      for (int i = 0; i < 4; ++i) end[row(j, i)] = S[j][i];
+  if (column == 0 && n < 4) {
+#pragma unroll
+    for (int j = 0; j < TW; ++j)
+      if (mine(j)) end[(int64_t)c.heads * DIM * c.vdim + head * DIM + 16 * (wave * TW + j) + 4 * g + n] = P[j];
+  }
+}
+
+// SPANS: c.span tokens of a sequence a work-group, behind keyed_spans_kernel; otherwise whole sequences.
+template <int FORM, int DT, bool SPANS>
 __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall c) {
   constexpr int TW = (DT + 3) / 4, DIM = 16 * DT;
   __shared__ __attribute__((aligned(16))) floatx4 parts[2][2][4][64];   // [turn][W S0, R S0][wave][lane]
   // the columns of a head and sequence read the same operands: they are numbered onto one XCD (work-groups are dealt to
   // eight of them in turn), which reads them from memory once
   const int columns = c.vdim / 16, pair = blockIdx.x / (8 * columns) * 8 + blockIdx.x % 8;
-  if (pair >= c.heads * c.n_seqs) return;
-  const int column = blockIdx.x / 8 % columns, head = pair % c.heads, seq = pair / c.heads;
+  const int column = blockIdx.x / 8 % columns, head = pair % c.heads;
+  int seq = pair / c.heads, part = 0;
+  if constexpr (SPANS) seq = piece_sequence(c.seq_off, c.n_seqs, c.tokens, c.max_count, c.span, seq, part);
+  else if (seq >= c.n_seqs) return;
+  if (SPANS && seq < 0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, n = lane & 15;
-  const int first = c.seq_off[seq], count = c.seq_off[seq + 1] - first;
+  int first = c.seq_off[seq], count = c.seq_off[seq + 1] - first;
   if (count <= 0) return;
+  const bool cut = SPANS && count > c.span, last = !cut || (part + 1) * c.span >= count;
+  if constexpr (SPANS) {
+    first += part * c.span;
+    count = last ? count - part * c.span : c.span;
+  }
   const int blocks = (count + KB_TOKENS - 1) / KB_TOKENS;
   const int64_t stride = (int64_t)c.heads * kb_floats(DIM, c.vdim);
-  const float* place = kb_place(c, seq, 0, head);
+  const float* place = kb_place(c, seq, SPANS ? part * (c.span / KB_TOKENS) : 0, head);
   const int vtiles = (c.vdim + 3) / 4, p = 16 * column + n;
-  float* slot = c.S + (int64_t)c.slots[seq] * c.state_stride + ((int64_t)head * vtiles + p / 4) * DIM * 4 + p % 4;
+  const int64_t of_head = ((int64_t)head * vtiles + p / 4) * DIM * 4 + p % 4;
+  float* slot = c.S + (int64_t)c.slots[seq] * c.state_stride + of_head;
   // tiles of key channels are dealt in turn; a wave has all its TW tiles unless DT is no multiple of four
   auto mine = [&](int j) { return DT % 4 == 0 || wave * TW + j < DT; };
   floatx4 S[TW];
+  auto read = [&](const float* from, floatx4 (&to)[TW], int apart) {
 #pragma unroll
-  for (int j = 0; j < TW; ++j)
+    for (int j = 0; j < TW; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) S[j][i] = mine(j) ? slot[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * 4] : 0.f;
+      for (int i = 0; i < 4; ++i) to[j][i] = mine(j) ? from[(int64_t)(16 * (wave * TW + j) + 4 * g + i) * apart] : 0.f;
+  };
   KbStage<FORM, TW> stages[KB_AHEAD];
   // a block's operands: one address that all lanes share, and every lane's distances from it
   uint32_t from_tile[TW], from_decay[TW];
@@ -657,76 +814,163 @@ __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall
   for (int j = 0; j < TW; ++j) {
     const int tile = min(wave * TW + j, DT - 1);
     from_tile[j] = (256 * tile + 4 * lane) * 4;
-    from_decay[j] = (KB_TOKENS * (3 * DIM + c.vdim) + 16 * tile + 4 * g) * 4;
+    from_decay[j] = (KB_TOKENS * (3 * DIM + c.vdim) + 16 * tile + 4 * g + (n & 3)) * 4;
   }
-  const uint32_t from_u = (KB_TOKENS * 3 * DIM + 256 * column + 4 * lane) * 4;
+  uint32_t from_u = (KB_TOKENS * 3 * DIM + 256 * column + 4 * lane + (FORM == 0 ? wave : 0)) * 4;
+  uint32_t from_o = (uint32_t)((4 * g + wave) * c.ld_out + n) * 4;
+  const uint32_t from_last = (uint32_t)(min(4 * g + wave, count - (blocks - 1) * KB_TOKENS - 1) * c.ld_out + n) * 4;
   const char* at = reinterpret_cast<const char*>(place);
-  int row = 4 * g + wave, ahead = row, fetched = 0;        // a wave finishes every fourth token's read-out
-  float* out = c.out + (first + (int64_t)min(row, count - 1)) * c.ld_out + head * c.vdim + p;
-  const float* out_ahead = out;
+  float* const outs = c.out + (int64_t)first * c.ld_out + head * c.vdim + 16 * column;
+  const char* out_at = reinterpret_cast<const char*>(outs);
+  int row = 4 * g + wave, fetched = 0;                     // a wave finishes every fourth token's read-out
+  float* out = outs + (int64_t)min(row, count - 1) * c.ld_out + n;
   const int64_t out_step = KB_TOKENS * c.ld_out;
-  auto load4 = [&](uint32_t from) { return *reinterpret_cast<const floatx4*>(at + from); };
-  auto fetch = [&](KbStage<FORM, TW>& st) {
-#pragma unroll
-    for (int j = 0; j < TW; ++j) {
-      if (FORM == 0) st.w[j] = load4(from_tile[j]);
-      st.r[j] = load4(from_tile[j] + KB_TOKENS * DIM * 4);
-      st.ku[j] = load4(from_tile[j] + 2 * KB_TOKENS * DIM * 4);
-      st.a[j] = load4(from_decay[j]);
-    }
-    st.u = load4(from_u);
-    st.o = *out_ahead;
-    // on to the next block; at the end the last one's operands are asked for again and not used
-    at += ++fetched < blocks ? stride * 4 : 0;
-    ahead += KB_TOKENS;
-    out_ahead += ahead < count ? out_step : 0;
+  // (a distance is taken as a new number each time: widened once for all it would be added to the address in 64 bits at every load)
+  auto load4 = [&](uint32_t& from, int further) {
+    const char* base = at + further;
+    asm volatile("" : "+v"(from), "+s"(base));
+    return *reinterpret_cast<const __attribute__((address_space(1))) floatx4*>((const __attribute__((address_space(1))) char*)base + from);
   };
-  auto walk = [&](KbStage<FORM, TW>& st, int turn) {
-    floatx4 ws = {0.f, 0.f, 0.f, 0.f}, rs = ws;
-    if (FORM == 0) {
-#pragma unroll
-      for (int j = 0; j < TW; ++j)
-        if (mine(j))
-#pragma unroll
-          for (int i = 0; i < 4; ++i) ws = __builtin_amdgcn_mfma_f32_16x16x4f32(st.w[j][i], S[j][i], ws, 0, 0, 0);
+  auto load1 = [&](const char* base, uint32_t& from) {
+    asm volatile("" : "+v"(from));
+    return *reinterpret_cast<const float*>(base + from);
+  };
+  constexpr int LOADS = (FORM == 0 ? 4 : 3) * TW + 2;
+  auto fetch = [&](KbStage<FORM, TW>& st, auto number) {   // one of a block's LOADS, in order
+    constexpr int load = decltype(number)::value, j = load % TW, kind = load / TW + (FORM == 0 ? 0 : 1);
+    if constexpr (load >= LOADS) {
+      return;
+    } else if constexpr (load == LOADS - 1) {
+      if (fetched >= blocks - 1) from_o = from_last;
+      st.o = load1(out_at, from_o);
+      // on to the next block; at the end the last one's operands are asked for again and not used
+      const bool more = ++fetched < blocks;
+      at += more ? stride * 4 : 0;
+      out_at += more ? out_step * 4 : 0;
+    } else if constexpr (load == LOADS - 2) {
+      if constexpr (FORM == 0) st.u = load1(at, from_u);
+      else st.u = load4(from_u, 0);
+    } else if constexpr (kind == 0) {
+      st.w[j] = load4(from_tile[j], 0);
+    } else if constexpr (kind == 1) {
+      st.r[j] = load4(from_tile[j], KB_TOKENS * DIM * 4);
+    } else if constexpr (kind == 2) {
+      st.ku[j] = load4(from_tile[j], 2 * KB_TOKENS * DIM * 4);
+    } else {
+      st.a[j] = load1(at, from_decay[j]);
     }
-#pragma unroll
-    for (int j = 0; j < TW; ++j)
-      if (mine(j))
-#pragma unroll
-        for (int i = 0; i < 4; ++i) rs = __builtin_amdgcn_mfma_f32_16x16x4f32(st.r[j][i], S[j][i], rs, 0, 0, 0);
-    if (FORM == 0) parts[turn][0][wave][lane] = ws;
-    parts[turn][1][wave][lane] = rs;
-#pragma unroll
-    for (int j = 0; j < TW; ++j) S[j] *= st.a[j];
-    lds_barrier();
-    floatx4 u = st.u;
-    if (FORM == 0)
-      u -= (parts[turn][0][0][lane] + parts[turn][0][1][lane]) + (parts[turn][0][2][lane] + parts[turn][0][3][lane]);
-#pragma unroll
-    for (int j = 0; j < TW; ++j)
-      if (mine(j))
-#pragma unroll
-        for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.ku[j][i], u[i], S[j], 0, 0, 0);
-    const float* r = reinterpret_cast<const float*>(&parts[turn][1][0][lane]) + wave;
-    const float o = st.o + ((r[0] + r[256]) + (r[512] + r[768]));
+  };
+  // A block's read-out is added up from LDS behind the next block's barrier.
+  float pending = 0.f;
+  auto finish = [&](const float (&r)[4]) {
+    const float o = pending + ((r[0] + r[1]) + (r[2] + r[3]));
     if (row < count) *out = o;
     row += KB_TOKENS;
     out += out_step;
   };
+  auto read_outs = [&](int turn, float (&r)[4]) {
+    const float* at = reinterpret_cast<const float*>(&parts[turn][1][0][lane]) + wave;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = at[256 * i];
+  };
+  auto walk = [&](KbStage<FORM, TW>& st, int turn, bool behind, auto asks, KbStage<FORM, TW>& next) {
+    floatx4 ws[TW], rs[TW];
+#pragma unroll
+    for (int j = 0; j < TW; ++j) ws[j] = rs[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (FORM == 0) {                             // a quarter of T v is in every wave's part
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ws[0][i] = i == wave ? -st.u : 0.f;
+    }
+    // The products with S0, a load of the next block's operands behind each: one of 16 bytes a lane takes the address unit, which the
+    // four waves share, 16 cycles, and a wave that asks for all its ten at once waits for them.
+    auto ask = [&](auto number) {
+      if constexpr (decltype(asks)::value) fetch(next, number);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](floatx4 (&sum)[TW], const floatx4* op, auto number) {
+      constexpr int j = decltype(number)::value % TW, i = decltype(number)::value / TW;
+      if (mine(j)) sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[j][i], S[j][i], sum[j], 0, 0, 0);
+    };
+    constexpr int FIRST = FORM == 0 ? 4 * TW : 0;          // loads behind W's steps
+    if constexpr (FORM == 0) {
+      each<4 * TW>([&](auto x) { step(ws, st.w, x); ask(x); });
+      if (TW > 1) ws[0] += ws[TW - 1];
+      parts[turn][0][wave][lane] = ws[0];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    each<2 * TW>([&](auto x) { step(rs, st.r, x); ask(Number<FIRST + decltype(x)::value>()); });
+    lds_barrier();
+    floatx4 others[4];
+    float r[4];
+    if (FORM == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) others[i] = parts[turn][0][i][lane];
+    }
+    read_outs(turn ^ 1, r);
+    __builtin_amdgcn_sched_barrier(0);
+    each<2 * TW>([&](auto x) { step(rs, st.r, Number<2 * TW + decltype(x)::value>()); ask(Number<FIRST + 2 * TW + decltype(x)::value>()); });
+    ask(Number<FIRST + 4 * TW>());
+    static_assert(FIRST + 4 * TW + 1 >= LOADS, "every load has its place");
+    floatx4 u;
+    if constexpr (FORM == 0) u = -((others[0] + others[1]) + (others[2] + others[3]));
+    else u = st.u;
+#pragma unroll
+    for (int j = 0; j < TW; ++j) decay(S[j], st.a[j]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        if (mine(j)) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.ku[j][i], u[i], S[j], 0, 0, 0);
+    if (behind) finish(r);
+    if (TW > 1) rs[0] += rs[TW - 1];
+    parts[turn][1][wave][lane] = rs[0];
+    pending = st.o;
+  };
 #pragma unroll
   for (int i = 0; i < KB_AHEAD - 1; ++i) {
-    fetch(stages[i]);
+    each<LOADS>([&](auto load) { fetch(stages[i], load); });
     __builtin_amdgcn_sched_barrier(0);                     // (in order: a stage is waited for by the loads behind it)
   }
-  for (int block = 0; block < blocks; block += KB_AHEAD) {
+  if (!cut) {
+    read(slot, S, 4);
+  } else {                                                 // C(-1), or C(0) carried on: C(k) = P(k) C(k - 1) + E(k)
+    const int64_t span = kb_span_floats(c), products = (int64_t)c.heads * DIM * c.vdim + head * DIM;
+    const float* held = c.carry + span_block(c.seq_off, seq, c.span, part == 0 ? -1 : 0) * span;
+    read(held + of_head, S, 4);
+    if (part > 1) {
+      floatx4 E[TW], P[TW], E_next[TW], P_next[TW];
+      held += span;
+      read(held + of_head, E, 4);
+      read(held + products, P, 1);
+      for (int k = 1; k < part; ++k) {
+        if (k + 1 < part) held += span;                    // (the last one's again, not used)
+        read(held + of_head, E_next, 4);
+        read(held + products, P_next, 1);
 #pragma unroll
-    for (int i = 0; i < KB_AHEAD; ++i) {
-      if (block + i >= blocks) break;                      // (the same for all four waves)
-      fetch(stages[(i + KB_AHEAD - 1) % KB_AHEAD]);
-      walk(stages[i], i & 1);
+        for (int j = 0; j < TW; ++j) {
+          S[j] = P[j] * S[j] + E[j];
+          E[j] = E_next[j];
+          P[j] = P_next[j];
+        }
+      }
     }
   }
+  landed(S);
+  int block = 0;
+  for (; block + KB_AHEAD <= blocks; block += KB_AHEAD) {  // (whole turns: see KB_AHEAD)
+#pragma unroll
+    for (int i = 0; i < KB_AHEAD; ++i) {
+      walk(stages[i], i & 1, block + i > 0, Number<1>(), stages[(i + KB_AHEAD - 1) % KB_AHEAD]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < KB_AHEAD - 1; ++i)
+    if (block + i < blocks) walk(stages[i], i & 1, block + i > 0, Number<0>(), stages[i]);  // (the same for all four waves)
+  lds_barrier();
+  float r[4];
+  read_outs((blocks - 1) & 1, r);
+  finish(r);
+  if (!last) return;
 #pragma unroll
   for (int j = 0; j < TW; ++j)
     if (mine(j))
@@ -745,7 +989,8 @@ __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall
 // the work-groups that bring its state in and out (they hold a compute unit's registers, two to a unit).  Measured (start
 // to end, token by token or in spans / in blocks): forget gate, 2 heads of 16 x 16, 4,000 tokens 36 / 90, 4 of 64 x 64 68 / 106, 8 of 128 x 128
 // 246 / 167; delta rule with one decay a head, 8 heads of 128 x 128, 40 tokens and 63 single ones 33 / 54, 100 and 63 46 / 55, 500 and 63
-// 192 / 61, 1,000 and 200 375 / 149; 16 heads, 64 and 31 36 / 55; 2 heads of 16 x 16, 40 tokens 11 / 15.
+// 192 / 61, 1,000 and 200 375 / 149; 16 heads, 64 and 31 36 / 55; 2 heads of 16 x 16, 40 tokens 11 / 15.  With the walk as it is
+// now the forget gate in blocks, 4 heads of 64 x 64, 1,000 tokens 33 / 25; 2 of 16 x 16, 4,000 35 / 82.
 static bool blocks_pay(const KeyedScanCall& c) {
   const float r = c.dim / 16, longest = c.max_count;
   const int span = keyed_span(c);
@@ -755,20 +1000,43 @@ static bool blocks_pay(const KeyedScanCall& c) {
                                : 2.f + 2.f * token * span * span_crowding((int64_t)c.heads * (c.vdim / 4), c.tokens, span) +
                                      (0.3f + 2e-5f * c.heads * c.dim * c.vdim) * (longest / span);
   const float others = short_sequences(c.tokens, c.n_seqs, c.max_count) * (c.heads * (c.vdim / 16)) * (0.003f + 4e-5f * c.dim);
-  const float blocks = (c.form == 1 ? 8.f + 0.6f * r + (0.0195f + 0.0026f * r) * longest : 13.f + 0.5f * r + (0.028f + 0.0033f * r) * longest) + others;
+  const float blocks = (c.form == 1 ? 8.f + 0.6f * r + (0.0165f + 0.0011f * r) * longest : 13.f + 0.5f * r + (0.028f + 0.0033f * r) * longest) + others;
   return blocks < walk;
+}
+
+// Into spans of how many tokens the walk over blocks cuts the forget gate's sequences, 0 for not at all: as many as give every compute
+// unit the two work-groups it holds, where that makes at least three of the longest sequence.  Below 640 tokens the second kernel costs
+// what it gains (us, whole / in spans, 8 heads of 128 x 128: 2 x 512 31.9 / 33.2, 2 x 300 22.6 / 26.4, 256 19.1 / 18.5).
+#define KB_UNITS 256
+#define KB_SPAN_MIN 640
+static int keyed_block_span(const KeyedScanCall& c) {
+  if (c.form != 1 || c.span <= 0 || !c.carry) return 0;
+  const int64_t per_token = (int64_t)c.heads * (c.vdim / 16);
+  if (per_token * c.n_seqs >= 2 * KB_UNITS) return 0;
+  int64_t tokens = (c.tokens * per_token + 2 * KB_UNITS - 1) / (2 * KB_UNITS);
+  if (tokens < c.span) tokens = c.span;
+  tokens = (tokens + KB_TOKENS - 1) / KB_TOKENS * KB_TOKENS;
+  return c.max_count >= KB_SPAN_MIN && c.max_count >= 3 * tokens ? (int)tokens : 0;
 }
 
 template <int DT>
 static void launch_keyed_blocks(hipStream_t stream, const KeyedScanCall& c) {
   dim3 side(c.heads, c.tokens / KB_TOKENS + c.n_seqs), block(256);      // (the heads of a piece side by side: they share rows)
-  dim3 walk((unsigned)((c.heads * c.n_seqs + 7) / 8 * 8 * (c.vdim / 16)));
+  auto walks = [&](int64_t pieces) { return dim3((unsigned)((c.heads * pieces + 7) / 8 * 8 * (c.vdim / 16))); };
   if (c.form == 0) {
     hipLaunchKernelGGL((keyed_blocks_kernel<0, DT>), side, block, 0, stream, c);
-    hipLaunchKernelGGL((keyed_blocks_walk_kernel<0, DT>), walk, block, 0, stream, c);
+    hipLaunchKernelGGL((keyed_blocks_walk_kernel<0, DT, false>), walks(c.n_seqs), block, 0, stream, c);
+    return;
+  }
+  hipLaunchKernelGGL((keyed_blocks_kernel<1, DT>), side, block, 0, stream, c);
+  if (const int span = keyed_block_span(c)) {
+    KeyedScanCall cut = c;
+    cut.span = span;
+    const dim3 grid = walks(c.tokens / span + c.n_seqs);
+    hipLaunchKernelGGL(keyed_spans_kernel<DT>, grid, block, 0, stream, cut);
+    hipLaunchKernelGGL((keyed_blocks_walk_kernel<1, DT, true>), grid, block, 0, stream, cut);
   } else {
-    hipLaunchKernelGGL((keyed_blocks_kernel<1, DT>), side, block, 0, stream, c);
-    hipLaunchKernelGGL((keyed_blocks_walk_kernel<1, DT>), walk, block, 0, stream, c);
+    hipLaunchKernelGGL((keyed_blocks_walk_kernel<1, DT, false>), walks(c.n_seqs), block, 0, stream, c);
   }
 }
 

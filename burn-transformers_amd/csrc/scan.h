@@ -34,6 +34,14 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Waits for values that a loop with loads on their way starts from: asked for behind those, they would be waited for, and the loads
+// with them, in every turn (the compiler's wait is the same for all).
+template <int N>
+__device__ __forceinline__ void landed(floatx4 (&values)[N]) {
+#pragma unroll
+  for (int j = 0; j < N; ++j) asm volatile("" : "+v"(values[j]));
+}
+
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus_f(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
 

@@ -99,6 +99,39 @@ def test_blocks_of_tokens(form, heads, kv_heads, dim, vdim, lengths, strong):
     assert max(errors["blocks"]) < 3.0 * max(errors["walk"]), errors
 
 
+# the forget gate with room for spans: spans of 64 tokens and of more, two and many of a sequence, a last one of one token and whole,
+# sequences too short to be cut beside them, key channels that are no multiple of the waves' tiles
+@pytest.mark.parametrize("heads,dim,vdim,lengths,strong", [
+    (2, 128, 128, [705, 15, 1, 640], False), (3, 48, 80, [640, 127, 193], True), (1, 64, 16, [700, 64], False), (4, 80, 32, [1, 833, 1, 1], True),
+    (8, 128, 128, [1100, 90, 1030], False)])
+def test_blocks_of_tokens_in_spans(heads, dim, vdim, lengths, strong):
+    gen = torch.Generator().manual_seed(heads * 1000 + dim + len(lengths))
+    qk, inner, total = heads * dim, heads * vdim, sum(lengths)
+    rows = torch.randn(total, 2 * qk + inner + 3, generator=gen)
+    rows[:, qk:2 * qk] *= 20.0 if strong else 1.0
+    bias, lower = torch.randn(qk, generator=gen), torch.rand(qk, generator=gen) * (0.0 if strong else 0.9)
+    slots = list(reversed(range(len(lengths))))
+    state = torch.randn(len(lengths), qk * vdim, generator=gen)
+    step, on, held = make_step(torch.float32, lengths, starts=[5] * len(lengths), slots=slots), rows.to(DEV), state.to(DEV)
+    blocks, carry = K.scan_blocks(step, heads, dim, vdim), K.scan_carry(step, qk * vdim, qk)
+    blocks.fill_(float("nan"))
+    carry.fill_(float("nan"))
+    y = torch.full((total, inner + 2), float("nan"), device=DEV)
+    K.keyed_scan(on[:, :qk], None, on[:, 2 * qk:2 * qk + inner], on[:, qk:2 * qk], y, held, step, heads, heads, dim, vdim, "forget",
+                 g_bias=bias.to(DEV), lower=lower.to(DEV), carry=carry, blocks=blocks)
+    assert bool(torch.isnan(y[:, inner:]).all()) and bool(torch.isfinite(carry).any())          # (cut indeed)
+    r, q = rows.double(), rows[:, :qk].double()
+    decay = (lower.double() + (1.0 - lower.double()) * torch.sigmoid(r[:, qk:2 * qk] + bias.double())).view(-1, heads, dim)
+    q, v, at, want, got = (q * torch.sigmoid(q)).view(-1, heads, dim), r[:, 2 * qk:2 * qk + inner].view(-1, heads, vdim), 0, [], state_rows(held, heads, dim, vdim).cpu()
+    for slot, n in zip(slots, lengths):
+        here = slice(at, at + n)
+        o, behind = recurrence(state_rows(state, heads, dim, vdim)[slot].double(), q[here], 1.0 - decay[here], v[here], decay[here], None)
+        want.append(o.reshape(n, inner))
+        assert rel_err(got[slot], behind) < 5e-6                # (as in whole sequences: the spans' products are a few more of some hundred)
+        at += n
+    assert rel_err(y[:, :inner].cpu(), torch.cat(want)) < 5e-6
+
+
 # one token of one sequence whose operand is not finite, in the middle of a block and at its end: earlier tokens and other
 # sequences do not see it, later ones as in the walk (an endless step is a decay of nothing and stays finite)
 @pytest.mark.parametrize("form,where,value", [
