@@ -512,122 +512,130 @@ __global__ void __launch_bounds__(256) group_norm_kernel(GroupNormCall c) {
       cast[(int64_t)t * c.ld_cast + col] = from_float<T>(0.f);
 }
 
-// The same for rows of up to 256 * KMAX columns: a thread's columns live in registers, and every load of a
-// thread (partial sums of both terms, biases, the gate, the stream, the scale) is issued before the first is
-// used and none stands behind a branch of its own, so a row costs one round trip to memory (a decode step has
-// few rows: one row's latency is its time).  The parts' sums of squares meet in LDS, a wave a part.
-template <typename T, int KMAX>
+// The same for rows of up to 256 * KMAX columns: a thread's columns live in registers (RowColumns), every load of a thread (partial
+// sums of both terms, biases, the gate, the stream, the scale) is issued before the first is used, and what is not there is not read, so
+// a row costs one round trip to memory (a decode step has few rows: one row's latency is its time).  The parts' sums of squares meet in
+// LDS, a wave a part, in one order however the row was read.  What bounds it with many rows is memory: a row's 14 bytes a column take
+// 6 us of 2,048 rows of 1,024 at the copy's rate.  Measured (us, 2 parts, one partial sum; a column a load and absent operands' places read too / quads):
+// 2,048 rows of 1,024 8.3 / 6.5, of 2,048 13.9 / 11.2; 512 of 1,024 4.5 / 3.7; 8 of 2,048 with two 4.9 / 3.8, one of 1,024 3.5 / 2.9.
+template <typename T, int KMAX, bool QUADS>
 __global__ void __launch_bounds__(256) group_norm_small_kernel(GroupNormCall c) {
-  extern __shared__ float row_buf[];          // [width], then [groups] reciprocal roots
+  typedef RowColumns<KMAX, QUADS> Columns;
+  extern __shared__ __attribute__((aligned(16))) float row_buf[];       // [width], then [groups] reciprocal roots
   float* rstd = row_buf + c.width;
   const int t = blockIdx.x;
   const bool from_stream = c.n_delta == 0;
   const int source = from_stream && c.rows ? c.rows[t] : t;
   float* xr = c.x + (int64_t)source * c.width;
-  float v[KMAX], w[KMAX], xv[KMAX], g[KMAX], gt[KMAX];
-  int cc[KMAX];
+  float v[KMAX], w[KMAX], xv[KMAX], g[KMAX], gt[KMAX], part[4][KMAX], part2[4][KMAX];
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) {
-    const int col = threadIdx.x + 256 * k;
-    cc[k] = col < c.width ? col : 0;
-  }
-  const float* bias = c.bias ? c.bias : c.gamma;           // (read in any case, used only where there is one)
-  const float* bias2 = c.bias2 ? c.bias2 : c.gamma;
-  const float* gate = c.gate ? c.gate + (int64_t)t * c.ld_gate : c.gamma;
+  for (int k = 0; k < KMAX; ++k) v[k] = w[k] = gt[k] = part[0][k] = part[1][k] = part[2][k] = part[3][k] = 0.f;
+  // (the call's fields together at the start: the ones a branch asks for would be waited for in it)
+  asm volatile("" ::"s"(c.bias), "s"(c.bias2), "s"(c.gate), "s"(c.ld_gate), "s"(c.gamma), "s"(c.cast), "s"(c.delta), "s"(c.delta_stride),
+               "s"(c.ldd), "s"(c.n_delta2));
+  const float* row = from_stream ? xr : c.delta + (int64_t)t * c.ldd;
+  const float* row2 = c.delta2 + (int64_t)t * c.ldd2;
+  // one to four of a term's partial sums, from the s0-th on; those that are not there count nothing
+  auto ask = [&](const float* first, int64_t stride, int s0, int n, float (&to)[4][KMAX]) {
+    Columns::load(first + s0 * stride, c.width, to[0]);
+    if (s0 + 1 < n) Columns::load(first + (s0 + 1) * stride, c.width, to[1]);
+    if (s0 + 2 < n) Columns::load(first + (s0 + 2) * stride, c.width, to[2]);
+    if (s0 + 3 < n) Columns::load(first + (s0 + 3) * stride, c.width, to[3]);
+  };
+  auto add = [&](float (&sum)[KMAX], const float (&from)[4][KMAX], int s0, int n) {
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) {
-    g[k] = c.gamma[cc[k]];
-    xv[k] = xr[cc[k]];
-    v[k] = bias[cc[k]];
-    w[k] = bias2[cc[k]];
-    gt[k] = gate[cc[k]];
-  }
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) {
-    v[k] = c.bias ? v[k] : 0.f;
-    w[k] = c.bias2 ? w[k] : 0.f;
+      for (int k = 0; k < KMAX; ++k) sum[k] += s0 + u < n ? from[u][k] : 0.f;
+  };
+  if (c.gate) Columns::load(c.gate + (int64_t)t * c.ld_gate, c.width, gt);
+  if (!from_stream && c.bias) Columns::load(c.bias, c.width, v);
+  if (c.n_delta2 > 0) {
+    if (c.bias2) Columns::load(c.bias2, c.width, w);
+    ask(row2, c.delta2_stride, 0, c.n_delta2, part2);
   }
+  if (!from_stream) ask(row, c.delta_stride, 0, c.n_delta, part);
+  Columns::load(xr, c.width, xv);
+  Columns::load(c.gamma, c.width, g);
   if (from_stream) {
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) v[k] = xv[k];
   } else {
-    const float* row = c.delta + (int64_t)t * c.ldd;
-    for (int s0 = 0; s0 < c.n_delta; s0 += 4) {            // four partial sums at a time, all their loads together
-      float part[4][KMAX];
+    add(v, part, 0, c.n_delta);
+    for (int s0 = 4; s0 < c.n_delta; s0 += 4) {
+      ask(row, c.delta_stride, s0, c.n_delta, part);
+      add(v, part, s0, c.n_delta);
+    }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int sc = s0 + u < c.n_delta ? s0 + u : c.n_delta - 1;
-#pragma unroll
-        for (int k = 0; k < KMAX; ++k) part[u][k] = row[sc * c.delta_stride + cc[k]];
+    for (int k = 0; k < KMAX; ++k) v[k] *= c.scale;
+    if (c.n_delta2 > 0) {
+      add(w, part2, 0, c.n_delta2);
+      for (int s0 = 4; s0 < c.n_delta2; s0 += 4) {
+        ask(row2, c.delta2_stride, s0, c.n_delta2, part2);
+        add(w, part2, s0, c.n_delta2);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int k = 0; k < KMAX; ++k) v[k] += s0 + u < c.n_delta ? part[u][k] : 0.f;
+      for (int k = 0; k < KMAX; ++k) v[k] = fmaf(c.scale2, w[k], v[k]);
     }
-    const float* row2 = c.delta2 + (int64_t)t * c.ldd2;
-    for (int s0 = 0; s0 < c.n_delta2; s0 += 4) {
-      float part[4][KMAX];
+    if (c.gate) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int sc = s0 + u < c.n_delta2 ? s0 + u : c.n_delta2 - 1;
-#pragma unroll
-        for (int k = 0; k < KMAX; ++k) part[u][k] = row2[sc * c.delta2_stride + cc[k]];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int k = 0; k < KMAX; ++k) w[k] += s0 + u < c.n_delta2 ? part[u][k] : 0.f;
-    }
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-      v[k] *= c.scale;
-      if (c.n_delta2 > 0) v[k] = fmaf(c.scale2, w[k], v[k]);
-      if (c.gate) v[k] *= 1.0f / (1.0f + expf(-gt[k]));
+      for (int k = 0; k < KMAX; ++k) v[k] *= 1.0f / (1.0f + expf(-gt[k]));
     }
   }
+  Columns::store(row_buf, c.width, v);
+  const int per = c.width / c.groups;
+  int mine[KMAX];                             // which part a column (of quads: the quad's columns) lies in
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k) {
-    const int col = threadIdx.x + 256 * k;
-    if (col < c.width) row_buf[col] = v[k];
-  }
+  for (int k = 0; k < KMAX; ++k) mine[k] = QUADS && k % 4 ? mine[k & ~3] : Columns::column(k) < c.width ? Columns::column(k) / per : 0;
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-  const int per = c.width / c.groups;
-  for (int part = wave; part < c.groups; part += waves) {
+  for (int p = wave; p < c.groups; p += waves) {
+    const float* from = row_buf + p * per;
     float squares = 0.f;
-    for (int i = lane; i < per; i += 64) squares = fmaf(row_buf[part * per + i], row_buf[part * per + i], squares);
+    for (int i = lane; i < per; i += 512) {   // (eight reads at a time, added up one after the other)
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = i + 64 * u < per ? from[i + 64 * u] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) squares = fmaf(x[u], x[u], squares);
+    }
     squares = wave_sum(squares);
-    if (lane == 0) rstd[part] = 1.0f / sqrtf(squares / (float)per + c.eps);
+    if (lane == 0) rstd[p] = 1.0f / sqrtf(squares / (float)per + c.eps);
   }
   __syncthreads();
-  T* cast = static_cast<T*>(c.cast);
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
-    const int col = threadIdx.x + 256 * k;
-    if (col < c.width) {
-      float y = v[k] * rstd[col / per] * g[k];
-      if (!from_stream) {
-        y *= c.mult;
-        if (c.accumulate) y += xv[k];
-        xr[col] = y;
-      }
-      if (cast) cast[(int64_t)t * c.ld_cast + col] = from_float<T>(y);
+    v[k] = v[k] * rstd[mine[k]] * g[k];
+    if (!from_stream) {
+      v[k] *= c.mult;
+      if (c.accumulate) v[k] += xv[k];
     }
   }
-  if (cast)
-    for (int col = c.width + threadIdx.x; col < c.cast_cols; col += blockDim.x)
-      cast[(int64_t)t * c.ld_cast + col] = from_float<T>(0.f);
+  if (!from_stream) Columns::store(xr, c.width, v);
+  if (T* cast = static_cast<T*>(c.cast)) {
+    cast += (int64_t)t * c.ld_cast;
+    Columns::store(cast, c.width, v);
+    for (int col = c.width + threadIdx.x; col < c.cast_cols; col += blockDim.x) cast[col] = from_float<T>(0.f);
+  }
 }
 
 template <typename T>
 static void launch_group_norm(hipStream_t stream, const GroupNormCall& c) {
   const size_t lds = (size_t)(c.width + c.groups) * sizeof(float);
   dim3 grid(c.tokens), block(256);
-  if (c.width <= 1024)
-    hipLaunchKernelGGL((group_norm_small_kernel<T, 4>), grid, block, lds, stream, c);
+  const uintptr_t floats = (uintptr_t)c.x | (uintptr_t)c.delta | (uintptr_t)c.bias | (uintptr_t)c.delta2 | (uintptr_t)c.bias2 | (uintptr_t)c.gate |
+                           (uintptr_t)c.gamma;
+  const bool quads = c.width / c.groups % 4 == 0 && (floats & 15) == 0 && c.ldd % 4 == 0 && c.delta_stride % 4 == 0 && c.ldd2 % 4 == 0 &&
+                     c.delta2_stride % 4 == 0 && c.ld_gate % 4 == 0 &&
+                     (!c.cast || (c.ld_cast % 4 == 0 && ((uintptr_t)c.cast & (4 * sizeof(T) - 1)) == 0));
+  if (c.width <= 1024 && quads)
+    hipLaunchKernelGGL((group_norm_small_kernel<T, 4, true>), grid, block, lds, stream, c);
+  else if (c.width <= 1024)
+    hipLaunchKernelGGL((group_norm_small_kernel<T, 4, false>), grid, block, lds, stream, c);
+  else if (c.width <= 2048 && quads)
+    hipLaunchKernelGGL((group_norm_small_kernel<T, 8, true>), grid, block, lds, stream, c);
   else if (c.width <= 2048)
-    hipLaunchKernelGGL((group_norm_small_kernel<T, 8>), grid, block, lds, stream, c);
+    hipLaunchKernelGGL((group_norm_small_kernel<T, 8, false>), grid, block, lds, stream, c);
   else
     hipLaunchKernelGGL(group_norm_kernel<T>, grid, block, lds, stream, c);
 }

@@ -193,6 +193,34 @@ def test_norm_in_parts_of_a_sublayers_output(dtype, width, groups, two, gated):
     assert rel_err(out[:, :width], picked) < (4e-6 if dtype == "float32" else 5e-3)
 
 
+# rows read four columns at a time and one by one (a pitch that is no multiple of four): the same numbers; one to six partial sums of each
+# term, rows of one and two turns of columns and ragged ones
+@pytest.mark.parametrize("width,groups,n1,n2,gated,biased", [
+    (1024, 2, 1, 0, False, False), (1024, 4, 2, 1, False, True), (1020, 3, 3, 2, True, False), (2048, 2, 4, 0, True, True),
+    (1032, 2, 5, 6, False, True), (16, 4, 6, 1, True, True), (2040, 1, 1, 5, False, False)])
+def test_norm_in_parts_reads_rows_either_way(width, groups, n1, n2, gated, biased):
+    gen = torch.Generator().manual_seed(width + n1)
+    tokens, on = 9, lambda *shape: torch.randn(*shape, generator=gen).to(DEV)
+    x, d1, d2 = on(tokens, width), on(n1, tokens, width), on(max(n2, 1), tokens, width)
+    bias, bias2, gate, gamma = on(width), on(width), on(tokens, width), on(width)
+    v = 0.7 * (d1.double().sum(0) + (bias.double() if biased else 0.0))
+    if n2:
+        v = v + 1.3 * (d2.double().sum(0) + (bias2.double() if biased else 0.0))
+    v = v * torch.sigmoid(gate.double()) if gated else v
+    want = x.double().cpu() + 0.5 * plain.group_norm(v.cpu(), gamma.double().cpu(), groups, 1e-4)
+    results = []
+    for extra in (0, 4, 1):
+        apart = torch.full((n1, tokens, width + extra), float("nan"), device=DEV)
+        apart[:, :, :width] = d1
+        xs, cast = x.clone(), torch.full((tokens, width + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+        K.group_norm_output(xs, gamma, groups, 1e-4, apart[:, :, :width], bias if biased else None, 0.7, d2 if n2 else None,
+                            bias2 if biased and n2 else None, 1.3, gate=gate if gated else None, mult=0.5, cast=cast)
+        results.append((xs, cast))
+    assert rel_err(results[0][0], want) < 2e-6 and float(results[0][1][:, width:].abs().max()) == 0.0
+    for xs, cast in results[1:]:
+        assert torch.equal(xs, results[0][0]) and torch.equal(cast, results[0][1])
+
+
 def test_capped_logits():
     gen = torch.Generator().manual_seed(0)
     logits = torch.randn(5, 3001, generator=gen) * 40.0
