@@ -31,6 +31,26 @@ def test_poly_norm(out_dtype):
     assert float(out[:, 45:].float().abs().max()) == 0.0
 
 
+# whole quads of columns and ragged rows beside a pitch that allows no quads: the same numbers
+@pytest.mark.parametrize("columns", [4, 1020, 1024, 1028, 4096, 4100, 8192, 8196])
+def test_poly_norm_reads_rows_either_way(columns):
+    gen = torch.Generator().manual_seed(columns)
+    z, coefficients = torch.randn(5, columns, generator=gen), torch.randn(4, generator=gen)
+    want, results = plain.poly_norm(z.double(), coefficients.double(), 1e-5), []
+    for extra in (0, 8, 3):
+        padded = torch.full((5, columns + extra), float("nan"), device=DEVICE)
+        padded[:, :columns] = z.to(DEVICE)
+        for dtype in (torch.float32, torch.bfloat16):
+            out = torch.full((5, columns + 4), float("nan"), dtype=dtype, device=DEVICE)
+            K.poly_norm(padded, columns, coefficients.to(DEVICE), 1e-5, out)
+            results.append(out)
+    # a sum of squares of up to 8,196 values in 256 parts of up to 33: some 2^-24 each, and a few operations behind it
+    assert float((results[0][:, :columns].cpu().double() - want).abs().max() / want.abs().max()) < 3e-6
+    assert float(results[0][:, columns:].abs().max()) == 0.0
+    for i in range(2, 6):
+        assert torch.equal(results[i], results[i % 2])
+
+
 def test_output_norm_adds_the_scaled_norm_of_partial_sums():
     x, parts, bias, gamma = rand(5, 37, seed=2), rand(3, 5, 37, seed=3), rand(37, seed=4), rand(37, seed=5)
     xd = x.to(DEVICE)
