@@ -625,20 +625,6 @@ __global__ void __launch_bounds__(256, 4) keyed_blocks_kernel(KeyedScanCall c) {
 // 1,024 tokens, the walk alone): delta rule 56.9 -> 42.1, forget gate 40 -> 28.7.
 #define KB_AHEAD 4
 
-template <int N>
-struct Number {
-  static constexpr int value = N;
-};
-
-// f(Number<0>()) .. f(Number<N - 1>()): steps whose numbers choose code.
-template <int N, int FROM = 0, typename F>
-__device__ __forceinline__ void each(F&& f) {
-  if constexpr (FROM < N) {
-    f(Number<FROM>());
-    each<N, FROM + 1>(f);
-  }
-}
-
 template <int FORM, int TW>
 struct KbStage {
   floatx4 w[FORM == 0 ? TW : 1], r[TW], ku[TW];

@@ -42,6 +42,20 @@ __device__ __forceinline__ void landed(floatx4 (&values)[N]) {
   for (int j = 0; j < N; ++j) asm volatile("" : "+v"(values[j]));
 }
 
+template <int N>
+struct Number {
+  static constexpr int value = N;
+};
+
+// f(Number<0>()) .. f(Number<N - 1>()): steps whose numbers choose code.
+template <int N, int FROM = 0, typename F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (FROM < N) {
+    f(Number<FROM>());
+    each<N, FROM + 1>(f);
+  }
+}
+
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus_f(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
 
