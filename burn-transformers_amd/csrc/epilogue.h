@@ -535,8 +535,8 @@ __device__ __forceinline__ void epilogue_tile(const Epilogue& e, int M, int N, i
 // of registers.  Of 16-bit results the rows of sixteen lanes swap halves of two neighbouring blocks, so that a lane stores 16 bytes and a
 // row 64; of 32-bit ones a lane has 16 bytes and a row 64 already.  Every block of sixteen columns is queries, keys or values of one
 // head.  Values, of which four positions lie interleaved, go through LDS, where a lane takes four such positions of a channel, whatever row
-// they start at; what the wave does not have all four of is stored one by one.  (One by one for all whose quad does not start at a
-// multiple of four rows: 1295 x 3072 x 1024 in two sequences 23.6 us, aligned 15.6.)
+// they start at; where the wave's rows do not have all four behind one another (tokens may come in any order) each is stored by itself.  (One
+// by one for all whose quad does not start at a multiple of four rows: 1295 x 3072 x 1024 in two sequences 23.6 us, aligned 15.6.)
 // `scratch`: block_scratch_bytes<TM, TN>() of this wave's own.
 template <int TM, int TN>
 constexpr int block_scratch_bytes() { return 16 * (TN * 64 + 16) > TM * 16 * (8 + 32) ? 16 * (TN * 64 + 16) : TM * 16 * (8 + 32); }
@@ -676,15 +676,24 @@ __device__ __forceinline__ void epilogue_blocks(const Epilogue& e, int M, int N,
     // so 32.7.)
     const int hd = e.kv.head_dim;
     int64_t key_row[TM], value_row[TM];
-    uint64_t leads = 0;                                // rows whose position and the three behind it lie interleaved, all of them this wave's
+    uint64_t leads = 0, follows = 0;                   // rows whose position and the three behind it lie interleaved, all of them this wave's
+    auto before = [&](const int (&of)[TM], int bm) {   // of the row before (of the wave's first row: not used)
+      const int here = lane_moved<0x121>(of[bm]), last = lane_moved<0x121>(of[bm > 0 ? bm - 1 : 0]);     // (row_ror:1)
+      return i16 == 0 ? last : here;
+    };
 #pragma unroll
     for (int bm = 0; bm < TM; ++bm) {
-      const int m = m0 + bm * 16 + i16, third = m + 3 < M ? m + 3 : M - 1;
+      const bool here = m0 + bm * 16 + i16 < M;
+      const int seq_before = before(seq, bm), pos_before = before(pos, bm);      // (by all lanes: one that is switched off passes nothing on)
+      leads |= (__ballot(here && pos[bm] % 4 == 0) & 0xffff) << (16 * bm);
+      follows |= (__ballot(here && seq[bm] == seq_before && pos[bm] == pos_before + 1) & 0xffff) << (16 * bm);
+    }
+    leads &= follows >> 1 & follows >> 2 & follows >> 3;
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm) {
       const int64_t plane = (int64_t)e.kv.blocks[(int64_t)seq[bm] * e.kv.max_blocks + pos[bm] / BT_KV_BLOCK] * e.kv.block_stride;
       key_row[bm] = plane + key_offset(hd, pos[bm], 0);
       value_row[bm] = plane + value_offset(hd, pos[bm], 0);
-      const bool lead = pos[bm] % 4 == 0 && m + 3 < M && bm * 16 + i16 + 3 < TM * 16 && e.tok_seq[third] == seq[bm];
-      leads |= (__ballot(lead) & 0xffff) << (16 * bm);
     }
     const uint64_t together = leads | leads << 1 | leads << 2 | leads << 3;
     int64_t* const value_rows = reinterpret_cast<int64_t*>(scratch);

@@ -4,7 +4,9 @@ values scattered (quads of positions together, quads that start inside one, rows
 import pytest
 import torch
 
+from burn_transformers_amd.kernels import library as K
 import test_tile_forms_gpu as forms
+from kernel_helpers import PagedCase
 
 pytestmark = pytest.mark.gpu
 BLOCK_FORMS = (2, 3) + tuple(range(6, 15))
@@ -24,3 +26,29 @@ def test_epilogues(m, n, tiles):
 @pytest.mark.parametrize("heads,kv_heads,hd", [(4, 4, 64), (3, 1, 128), (4, 2, 32), (5, 5, 48), (2, 2, 80), (3, 3, 16)])
 def test_scattered(heads, kv_heads, hd):
     forms.test_scattered_keys_and_values(torch.bfloat16, heads, kv_heads, hd)
+
+
+# tokens of a step in any order: two of every four positions swapped, every fourth position first, two sequences' tokens between each other, drawn
+@pytest.mark.parametrize("order", ["swapped", "strided", "between", "drawn"])
+def test_scattered_in_any_order(order, heads=3, hd=48, k=128):
+    totals = counts = [64, 64, 130, 7]
+    width, m = heads * hd, sum(counts)
+    if order == "swapped":
+        rows = [r ^ 3 if r % 4 in (1, 2) else r for r in range(m - m % 4)] + list(range(m - m % 4, m))
+    elif order == "strided":
+        rows = [r for first in range(4) for r in range(first, m, 4)]
+    elif order == "between":          # a0 b1 b2 a3, b0 a1 a2 b3, ...
+        rows = [r + 64 * (r % 4 in (1, 2)) for r in range(64)] + [r + 64 * (r % 4 in (0, 3)) for r in range(64)] + list(range(128, m))
+    else:
+        rows = torch.randperm(m, generator=torch.Generator().manual_seed(3)).tolist()
+    assert sorted(rows) == list(range(m))
+    a, w, bias, want = forms.operands(m, 3 * width, k, torch.bfloat16, 5)
+    want = want + bias.double()
+    for form in BLOCK_FORMS:
+        case = PagedCase(totals, counts, heads, hd, torch.bfloat16, forms.DEV, seed=2)
+        q = torch.full((m, width), float("nan"), dtype=torch.bfloat16, device=forms.DEV)
+        K.gemm(a.to(forms.DEV), w.to(forms.DEV), K.epilogue_qkv(q, width, width, case.view(), case.tok_seq[rows].contiguous(), case.tok_pos[rows].contiguous(),
+                                                                bias.to(forms.DEV)), impl="tile", variant=form)
+        for got, first in ((case.read_back()[0], width), (case.read_back()[1], 2 * width)):
+            error = (got[rows].double().cpu() - want[:, first:first + width]).abs().max() / want.abs().max()
+            assert float(error) < 2.0 ** -8, (form, order, first)
