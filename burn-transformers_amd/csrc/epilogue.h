@@ -533,7 +533,7 @@ __device__ __forceinline__ void epilogue_tile(const Epilogue& e, int M, int N, i
 
 // The epilogue of a wave's TM x TN blocks of 16 x 16 (lane holds D[i][j]: i = 4 g + r the column, j = lane % 16 the row), straight out
 // of registers.  Of 16-bit results the rows of sixteen lanes swap halves of two neighbouring blocks, so that a lane stores 16 bytes and a
-// row 64; of 32-bit ones a lane has 16 bytes and a row 64 already.  Every block of sixteen columns is queries, keys or values of one
+// row 64; of 32-bit ones a lane has 16 bytes and a row 64 already (the residual stream's, which is read as well, goes through LDS).  Every block of sixteen columns is queries, keys or values of one
 // head.  Values, of which four positions lie interleaved, go through LDS, where a lane takes four such positions of a channel, whatever row
 // they start at; where the wave's rows do not have all four behind one another (tokens may come in any order) each is stored by itself.  (One
 // by one for all whose quad does not start at a multiple of four rows: 1295 x 3072 x 1024 in two sequences 23.6 us, aligned 15.6.)
@@ -601,34 +601,54 @@ __device__ __forceinline__ void epilogue_blocks(const Epilogue& e, int M, int N,
         for (int bm = 0; bm < TM; ++bm) acc[bn][bm] += b[bn];
     }
     if (f32) {
-      float* row[TM];
-      floatx4 old[2][TN];
-      const bool residual = e.mode == EPI_RESIDUAL;
-      auto ask = [&](int bm) {
+      float* const first = static_cast<float*>(e.out) + (e.mode == EPI_F32 ? (int64_t)split * e.split_stride : 0) + (n0 < N ? n0 : 0);
+      if (e.mode == EPI_RESIDUAL) {
+        // Through LDS, sixteen rows at a time, so that neighbouring lanes ask for neighbouring pieces of the stream's rows.  Asked for by the
+        // lanes that hold the sums, the pieces of neighbouring lanes are of sixteen rows, and the address unit, which takes sixteen lanes at a time,
+        // had 64 requests of every load (us, so / through LDS: 2048 x 1600 x 1600 in tiles of 128 x 128 24.4 / 22.7, 1959 x 1600 x 6400 55.5 / 54.2, 3072 x 1600 x
+        // 1600 in 128 x 160 27.2 / 25.7, 2048 x 1024 x 1024 in 128 x 64 12.9 / 12.1).  Stores, which nothing waits for, gain nothing by it, nor did 128 bytes of a
+        // row with every instruction (two neighbouring blocks' halves swapped) or the stream asked for before the bias.
+        constexpr int PITCH = COLUMNS * 4 + 16;
+        floatx4 old[2][TN];
+        auto at = [&](int t, int& r) {                 // the column of a lane's t-th piece of sixteen rows; its row in r
+          const int i = lane + 64 * t;
+          r = i / (4 * TN);
+          return 4 * (i - r * (4 * TN));
+        };
+        auto ask = [&](int bm) {
 #pragma unroll
-        for (int bn = 0; bn < TN; ++bn) {
-          const int c = bn * 16 + g * 4;
-          old[bm & 1][bn] = *reinterpret_cast<const floatx4*>(row[bm] + (n0 + c < N ? c : 0));
-        }
-      };
+          for (int t = 0; t < TN; ++t) {
+            int r;
+            const int c = at(t, r), m = m0 + bm * 16 + r;
+            old[bm & 1][t] = *reinterpret_cast<const floatx4*>(first + (int64_t)(m < M ? m : M - 1) * e.ldo + (n0 + c < N ? c : 0));
+          }
+        };
+        ask(0);
 #pragma unroll
-      for (int bm = 0; bm < TM; ++bm) {
-        const int m = m0 + bm * 16 + i16 < M ? m0 + bm * 16 + i16 : M - 1;
-        row[bm] = static_cast<float*>(e.out) + (e.mode == EPI_F32 ? (int64_t)split * e.split_stride : 0) + (int64_t)m * e.ldo + (n0 < N ? n0 : 0);
-      }
-      if (residual) ask(0);
-#pragma unroll
-      for (int bm = 0; bm < TM; ++bm) {
-        if (residual) {
+        for (int bm = 0; bm < TM; ++bm) {
           if (bm + 1 < TM) ask(bm + 1);
 #pragma unroll
-          for (int bn = 0; bn < TN; ++bn) acc[bn][bm] += old[bm & 1][bn];
+          for (int bn = 0; bn < TN; ++bn) *reinterpret_cast<floatx4*>(scratch + i16 * PITCH + (bn * 16 + g * 4) * 4) = acc[bn][bm];
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's accesses of LDS are served in order)
+#pragma unroll
+          for (int t = 0; t < TN; ++t) {
+            int r;
+            const int c = at(t, r), m = m0 + bm * 16 + r;
+            const floatx4 sum = *reinterpret_cast<const floatx4*>(scratch + r * PITCH + c * 4) + old[bm & 1][t];
+            if (m < M && n0 + c < N) *reinterpret_cast<floatx4*>(first + (int64_t)m * e.ldo + c) = sum;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
-        if (m0 + bm * 16 + i16 >= M) continue;
+        return;
+      }
+#pragma unroll
+      for (int bm = 0; bm < TM; ++bm) {
+        const int m = m0 + bm * 16 + i16;
+        if (m >= M) continue;
 #pragma unroll
         for (int bn = 0; bn < TN; ++bn) {
           const int c = bn * 16 + g * 4;
-          if (n0 + c < N) *reinterpret_cast<floatx4*>(row[bm] + c) = acc[bn][bm];
+          if (n0 + c < N) *reinterpret_cast<floatx4*>(first + (int64_t)m * e.ldo + c) = acc[bn][bm];
         }
       }
       return;

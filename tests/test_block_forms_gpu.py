@@ -28,6 +28,20 @@ def test_scattered(heads, kv_heads, hd):
     forms.test_scattered_keys_and_values(torch.bfloat16, heads, kv_heads, hd)
 
 
+# the residual stream, sixteen rows at a time: rows and columns that end inside a wave's, beside what is not the product's
+@pytest.mark.parametrize("m,n,pitch", [(65, 68, 72), (127, 160, 160), (257, 100, 104), (300, 332, 332), (130, 516, 520)])
+def test_residual_stream_between_others(m, n, pitch, k=192):
+    a, w, bias, want = forms.operands(m, n, k, torch.bfloat16, m)
+    x = torch.randn(m, n, generator=torch.Generator().manual_seed(n))
+    for form in BLOCK_FORMS:
+        room = torch.full((m + 2, pitch), float("nan"), device=forms.DEV)
+        room[:m, :n] = x.to(forms.DEV)
+        K.gemm(a.to(forms.DEV), w.to(forms.DEV), K.epilogue_residual(room[:m, :n], bias.to(forms.DEV)), impl="tile", variant=form)
+        exact = x.double() + want + bias.double()
+        assert float((room[:m, :n].double().cpu() - exact).abs().max() / exact.abs().max()) < 1e-5, form      # (32-bit sums of 192 products and three more)
+        assert torch.isnan(room[m:]).all() and torch.isnan(room[:, n:]).all(), form
+
+
 # tokens of a step in any order: two of every four positions swapped, every fourth position first, two sequences' tokens between each other, drawn
 @pytest.mark.parametrize("order", ["swapped", "strided", "between", "drawn"])
 def test_scattered_in_any_order(order, heads=3, hd=48, k=128):
