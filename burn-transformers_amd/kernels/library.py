@@ -989,14 +989,28 @@ def tile_form(rows64, n, k, splits=1, units=256):
     """(us, variant) of the form whose busiest compute unit is done first, for a product of ``rows64`` times 64 rows (steps of one
     class choose alike): a form of ``TILE_FORMS``, or tiles of 64 x 64 on four waves, of which up to three share a unit.  Over the 299 products
     the fastest forms take 6,223 us, those chosen 6,270.  (Large tiles that need every unit are counted 2 us longer: in such a graph they are not, but inside
-    steps 2048 x 4096 x 1024 took 3 to 5 us less on 208 tiles than on 256 and 1959 x 3072 x 1024 2.6 less on 192.)"""
+    steps 2048 x 4096 x 1024 took 3 to 5 us less on 208 tiles than on 256 and 1959 x 3072 x 1024 2.6 less on 192.)
+    Below twelve tiles of K, where those figures do not reach, starts and ends decide: small tiles start sooner than was fitted, their share of a
+    unit brings its results as well as its K, and a unit's second large tile needs no start of a kernel.  330 products of 65 to 4,096 rows, 64 to
+    8,192 columns and K of 64 to 704 take 2,721 us so, on the fastest forms 2,704, by the figures above 2,857 (us, by those / so: 125 x 2176 x 64 6.4 / 5.2,
+    910 x 192 x 64 6.2 / 5.0, 3482 x 4288 x 256 33.9 / 26.6, 2172 x 5568 x 576 53 / 31)."""
     turns, share = k / 64 / splits, -(-rows64 * -(-n // 64) * splits // units)
-    costs = [(4.9 + turns * (0.175, 0.42, 0.24 * share)[min(share, 3) - 1] + (0.8 if k >= 3072 else 0.0), 5 if share <= 2 else 4)]
+    short = turns < 12
+    if short:
+        small = (2.9 + 0.24 * turns, 4.8 + 0.47 * turns, 1.4 + share * (1.2 + 0.22 * turns))[min(share, 3) - 1]
+    else:
+        small = 4.9 + turns * (0.175, 0.42, 0.24 * share)[min(share, 3) - 1] + (0.8 if k >= 3072 else 0.0)
+    costs = [(small, 5 if share == 1 or (share == 2 and not short) else 4)]
     for variant, (rows, columns, start, turn, full_start, full_turn) in TILE_FORMS.items():
         tiles = -(-rows64 * 64 // rows) * -(-n // columns) * splits
         rounds, filled = -(-tiles // units), min(1.0, tiles / units)
-        us = start + turn * turns + filled * (full_start + full_turn * turns) + (2.0 if filled > 0.94 and rows * columns >= 24576 else 0.0)
-        costs.append((us if rounds == 1 else 1.05 * rounds * us, variant))
+        us = start + turn * turns + filled * (full_start + full_turn * turns)
+        if short:
+            us += (rounds - 1) * (us - 2.5)
+        else:
+            us += 2.0 if filled > 0.94 and rows * columns >= 24576 else 0.0
+            us *= 1.0 if rounds == 1 else 1.05 * rounds
+        costs.append((us, variant))
     return min(costs)
 
 

@@ -197,6 +197,25 @@ def test_products_leave_the_library_alike_in_all_steps_of_a_class():
                 assert own_tiles(rows, n, k, k, **options) == own_tiles(token_capacity(rows), n, k, k, **options)
 
 
+def test_forms_of_the_tile_kernel():
+    """Every form chosen is one that the kernel has; of products with few tiles of K the measured ones take the fastest form or one within a twentieth of it."""
+    import re
+    from burn_transformers_amd.kernels import library as K
+    from burn_transformers_amd.kernels.build import CSRC_DIR
+    with open(f"{CSRC_DIR}/gemm_mfma.hip") as source:
+        forms = source.read().split("static int launch_form(hipStream_t s, int variant, const bf16_t* a", 1)[1].split("unknown form", 1)[0]
+    known = {int(number) for number in re.findall(r"case (\d+):", forms)}
+    assert set(K.TILE_FORMS) | {4, 5} <= known
+    for rows64 in (2, 5, 9, 17, 32, 64):
+        for n in (64, 768, 1600, 4800, 8192, 50304):
+            for k in (64, 320, 768, 1600, 6400):
+                for splits in (1, 2, 4):
+                    assert K.tile_form(rows64, n, k, splits)[1] in set(K.TILE_FORMS) | {4, 5}
+    for rows, n, k, fast in ((125, 2176, 64, (4, 5)), (1584, 128, 64, (4, 5)), (910, 192, 64, (4, 5)), (66, 384, 192, (4, 5)), (112, 1344, 64, (4, 5)),
+                             (2172, 5568, 576, (7, 12, 14)), (2926, 7424, 704, (7, 14)), (1982, 7168, 576, (7, 14)), (3945, 832, 576, (2,)), (1148, 3584, 704, (2,))):
+        assert K.tile_form(-(-rows // 64), n, k)[1] in fast, (rows, n, k)
+
+
 def test_float_products_are_cut_alike_in_all_steps_of_a_class(monkeypatch):
     """One launch list serves all steps of a class, so the slices of a float32 product may not depend on which of them came first."""
     from types import SimpleNamespace
