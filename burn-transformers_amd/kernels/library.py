@@ -1014,21 +1014,30 @@ def tile_form(rows64, n, k, splits=1, units=256):
     return min(costs)
 
 
+MODEL_LONG_K, MODEL_COLUMNS = 6400, 12288      # the longest K and most columns whose way was measured
+LIBRARY_K_STEP, LIBRARY_STEP_FROM = 128, 1152  # what the library takes of K at a time, and from which K on that beats tiles of 64 x 64
+
+
 def tile_kernel_takes(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=False):
     """Whether a bfloat16 product of more than 64 rows is the tile kernel's: by ``own_tiles``, or where ``tile_form`` says that it is the
     faster way.  The library's time is taken as a start, its operations at 1.05 PFLOP/s, its K and its results, keys and values copied behind it (8 %
     off on average, 29 % at most: it jumps as its tiles fill the chip well or not); beside the plain library a twenty-fifth is left for that.
-    Measured (us, tile kernel / library) 2048 x 4800 x 1600 with keys and values scattered 34 / 47, 2048 x 3072 x 1024 19 / 25, 1295 x 3072 x 1024 16.6 /
-    24.7; into the residual stream 1959 x 1600 x 6400 53 / 58, 1959 x 1024 x 4096 27 / 30; the library's 2048 x 6400 x 1600 with a GELU 58 / 44, 1600 x 4096 x
-    1024 22.6 / 22.6, 4096 x 4096 x 1024 48 / 36.  Over the 299 products of ``TILE_FORMS`` the faster of the two ways takes 5,953 us, this choice
-    6,150, ``own_tiles`` alone 6,349."""
+    Measured with weights from memory over 628 products that ``own_tiles`` leaves to the library, of 65 to 4,096 rows, 64 to 12,160 columns and K of 512 to
+    8,192, each with its own epilogue: the library takes 15,278 us, the faster of the two ways 13,992, this choice 14,700; of the 243 that it takes from
+    the library two are slower by more than 3 % (356 x 8064 x 3200 with a GELU 33.7 / 31.6, 481 x 12096 x 4160 into the stream 60.7 / 58.7).  Of 4,097 to 16,384 rows 15 of 110 change, at 0.57 to 0.81 of the library's time.
+    Two bounds keep out what was slower.  Tiles of 64 x 64 with a long K that is a multiple of 128 stay behind the library, which reads K in such steps
+    and splits it (448 x 1024 x 2048 13.4 / 12.7, 440 x 832 x 1280 11.1 / 9.9, 18 of 28 by 3 to 12 %; K = 1,024 600 x 512 7.8 / 11.3, K = 1,856 1536 x 256 12.7 / 17.4).
+    Longer K and more columns than the model was held against go by ``own_tiles`` (3072 x 2048 x 8192 101 / 94)."""
     if own_tiles(m, n, k, lda, sliced, scatters, residual, gelu):
         return True
-    if m <= 64 or n % 8 or k < OWN_SHORT_K or not _tile_operands(m, n, k, lda):
+    if m <= 64 or n % 8 or not OWN_SHORT_K <= k <= MODEL_LONG_K or n > MODEL_COLUMNS or not _tile_operands(m, n, k, lda):
+        return False
+    us, variant = tile_form(m64(m) // 64, n, k)
+    if variant in (4, 5) and k >= LIBRARY_STEP_FROM and k % LIBRARY_K_STEP == 0 and not scatters:
         return False
     results = 1e-6 * m64(m) * n
     library = 5.9 + 1.9e-9 * m64(m) * n * k + 0.11 * k / 64 + 0.06 * results + (4.5 + 0.5 * results if scatters else 0.16 * results if residual else 0.0)
-    return tile_form(m64(m) // 64, n, k)[0] < (library if scatters else 0.96 * library)
+    return us < (library if scatters else 0.96 * library)
 
 
 def m64(rows):

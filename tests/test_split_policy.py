@@ -187,14 +187,36 @@ def test_which_products_leave_the_library_whatever_their_k():
     assert own_tiles(256, 6400, 1600, 1600, gelu=True) and not own_tiles(257, 6400, 1600, 1600, gelu=True)
 
 
+def test_which_products_the_tile_kernel_takes():
+    """``tile_kernel_takes``: ``own_tiles``' products and those whose form is the faster way, as measured beside the library; inside what was measured only."""
+    from burn_transformers_amd.kernels.library import own_tiles, tile_kernel_takes as takes
+    # faster on tiles by a tenth and more, left to the library by own_tiles
+    for m, n, k, options in ((400, 3072, 768, {"gelu": True}), (448, 1024, 1024, {"residual": True}), (600, 512, 1024, {}), (1536, 256, 1856, {"residual": True}),
+                             (768, 6144, 2048, {"scatters": True}), (2048, 4800, 1600, {"scatters": True}), (632, 3072, 576, {"gelu": True}), (6118, 1600, 6400, {})):
+        assert takes(m, n, k, k, **options) and not own_tiles(m, n, k, k, **options), (m, n, k)
+    # long K in steps of 128 on tiles of 64 x 64, and products that large tiles do not fill well
+    for m, n, k, options in ((448, 1024, 2048, {}), (440, 832, 1280, {}), (1318, 192, 1152, {"gelu": True}), (752, 512, 1792, {"residual": True}),
+                             (555, 768, 2560, {}), (2048, 128, 2048, {}), (2048, 6400, 1600, {"gelu": True}), (4096, 4096, 1024, {})):
+        assert not takes(m, n, k, k, **options), (m, n, k)
+    # beyond what the model was held against
+    for m in (65, 300, 513, 1024, 2048, 4096):
+        for n, k in ((2048, 6464), (2048, 8192), (1024, 16384), (12352, 1024), (50304, 1600), (32000, 1024)):
+            for options in ({}, {"scatters": True}, {"residual": True}, {"gelu": True}):
+                assert takes(m, n, k, k, **options) == own_tiles(m, n, k, k, **options), (m, n, k, options)
+    assert not takes(64, 1024, 1024, 1024) and not takes(566, 1024, 1000, 1000) and not takes(1300, 1604, 1600, 1600)
+
+
 def test_products_leave_the_library_alike_in_all_steps_of_a_class():
-    """One launch list serves all steps of a class: whose product it is may not depend on which of them came first."""
+    """One launch list serves all steps of a class: whose product it is, and on which form, may not depend on which of them came first."""
     from burn_transformers_amd.engine.step import token_capacity
-    from burn_transformers_amd.kernels.library import own_tiles
+    from burn_transformers_amd.kernels.library import own_tiles, tile_form, tile_kernel_takes
     for n, k in ((768, 768), (1600, 1600), (3072, 1024), (4800, 1600), (6144, 2048), (1024, 4096)):
         for options in ({}, {"sliced": True}, {"scatters": True}, {"residual": True}, {"gelu": True}):
             for rows in range(65, 1700):
-                assert own_tiles(rows, n, k, k, **options) == own_tiles(token_capacity(rows), n, k, k, **options)
+                capacity = token_capacity(rows)
+                assert own_tiles(rows, n, k, k, **options) == own_tiles(capacity, n, k, k, **options)
+                assert tile_kernel_takes(rows, n, k, k, **options) == tile_kernel_takes(capacity, n, k, k, **options)
+                assert tile_form(-(-rows // 64), n, k) == tile_form(-(-capacity // 64), n, k)
 
 
 def test_forms_of_the_tile_kernel():
