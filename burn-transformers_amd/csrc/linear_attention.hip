@@ -992,9 +992,12 @@ static bool blocks_pay(const KeyedScanCall& c) {
 
 // Into spans of how many tokens the walk over blocks cuts the forget gate's sequences, 0 for not at all: as many as give every compute
 // unit the two work-groups it holds, where that makes at least three of the longest sequence.  Below 640 tokens the second kernel costs
-// what it gains (us, whole / in spans, 8 heads of 128 x 128: 2 x 512 31.9 / 33.2, 2 x 300 22.6 / 26.4, 256 19.1 / 18.5).
+// what it gains, below 832 where several sequences give half the units and more a work-group (us, whole / in spans, 8 heads of 128 x 128: 256
+// tokens 19.1 / 18.5, 640 27.8 / 26.0, 1,000 37.6 / 30.5; 2 x 300 22.6 / 26.4, 2 x 512 31.9 / 33.2, 2 x 640 33.5 / 34.9, 2 x 768 36.7 / 37.3, 2 x 896 40.7 /
+// 40.0, 2 x 1,536 59.5 / 53.4; 4 heads 4 x 640 33.2 / 35.4, 4 x 1,024 44.0 / 43.0; 16 heads 640 32.6 / 32.7, 1,000 43.0 / 39.9; 12 heads 2 x 800 40.5 / 40.3).
 #define KB_UNITS 256
 #define KB_SPAN_MIN 640
+#define KB_SPAN_MIN_OF_MANY 832
 static int keyed_block_span(const KeyedScanCall& c) {
   if (c.form != 1 || c.span <= 0 || !c.carry) return 0;
   const int64_t per_token = (int64_t)c.heads * (c.vdim / 16);
@@ -1002,7 +1005,8 @@ static int keyed_block_span(const KeyedScanCall& c) {
   int64_t tokens = (c.tokens * per_token + 2 * KB_UNITS - 1) / (2 * KB_UNITS);
   if (tokens < c.span) tokens = c.span;
   tokens = (tokens + KB_TOKENS - 1) / KB_TOKENS * KB_TOKENS;
-  return c.max_count >= KB_SPAN_MIN && c.max_count >= 3 * tokens ? (int)tokens : 0;
+  const int least = c.n_seqs > 1 && 2 * per_token * c.n_seqs >= KB_UNITS ? KB_SPAN_MIN_OF_MANY : KB_SPAN_MIN;
+  return c.max_count >= least && c.max_count >= 3 * tokens ? (int)tokens : 0;
 }
 
 template <int DT>

@@ -132,6 +132,23 @@ def test_blocks_of_tokens_in_spans(heads, dim, vdim, lengths, strong):
     assert rel_err(y[:, :inner].cpu(), torch.cat(want)) < 5e-6
 
 
+# which steps are cut: one sequence from 640 tokens on, several that fill half the compute units from 832 on
+@pytest.mark.parametrize("heads,dim,vdim,lengths,cut", [
+    (8, 128, 128, [640], True), (8, 128, 128, [639], False), (8, 128, 128, [640, 640], False), (8, 128, 128, [831, 640], False), (8, 128, 128, [832, 640], True),
+    (4, 128, 128, [640] * 4, False), (4, 128, 128, [640, 640], True), (16, 128, 128, [640], True)])
+def test_which_steps_are_cut_into_spans(heads, dim, vdim, lengths, cut):
+    qk, total = heads * dim, sum(lengths)
+    step = make_step(torch.float32, lengths)
+    rows, y = torch.randn(total, 2 * qk + heads * vdim, device=DEV), torch.empty(total, heads * vdim, device=DEV)
+    blocks, carry = K.scan_blocks(step, heads, dim, vdim), K.scan_carry(step, qk * vdim, qk)
+    blocks.fill_(float("nan"))
+    carry.fill_(float("nan"))
+    K.keyed_scan(rows[:, :qk], None, rows[:, 2 * qk:], rows[:, qk:2 * qk], y, torch.zeros(len(lengths), qk * vdim, device=DEV), step, heads, heads, dim, vdim,
+                 "forget", g_bias=torch.zeros(qk, device=DEV), lower=torch.rand(qk, device=DEV), carry=carry, blocks=blocks)
+    assert bool(torch.isfinite(blocks).any())                                                   # (in blocks, not token by token)
+    assert bool(torch.isfinite(carry).any()) == cut
+
+
 # one token of one sequence whose operand is not finite, in the middle of a block and at its end: earlier tokens and other
 # sequences do not see it, later ones as in the walk (an endless step is a decay of nothing and stays finite)
 @pytest.mark.parametrize("form,where,value", [
