@@ -1015,7 +1015,7 @@ def tile_form(rows64, n, k, splits=1, units=256):
 
 
 MODEL_LONG_K, MODEL_COLUMNS = 6400, 12288      # the longest K and most columns whose way was measured
-LIBRARY_K_STEP, LIBRARY_STEP_FROM = 128, 1152  # what the library takes of K at a time, and from which K on that beats tiles of 64 x 64
+LIBRARY_K_STEP, LIBRARY_STEP_FROM, LIBRARY_LEAST_COLUMNS = 128, 1152, 128      # what the library takes of K at a time; from which K and columns on that beats tiles of 64 x 64
 
 
 def tile_kernel_takes(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=False):
@@ -1026,14 +1026,15 @@ def tile_kernel_takes(m, n, k, lda, sliced=False, scatters=False, residual=False
     8,192, each with its own epilogue: the library takes 15,278 us, the faster of the two ways 13,992, this choice 14,700; of the 243 that it takes from
     the library two are slower by more than 3 % (356 x 8064 x 3200 with a GELU 33.7 / 31.6, 481 x 12096 x 4160 into the stream 60.7 / 58.7).  Of 4,097 to 16,384 rows 15 of 110 change, at 0.57 to 0.81 of the library's time.
     Two bounds keep out what was slower.  Tiles of 64 x 64 with a long K that is a multiple of 128 stay behind the library, which reads K in such steps
-    and splits it (448 x 1024 x 2048 13.4 / 12.7, 440 x 832 x 1280 11.1 / 9.9, 18 of 28 by 3 to 12 %; K = 1,024 600 x 512 7.8 / 11.3, K = 1,856 1536 x 256 12.7 / 17.4).
+    and splits it (448 x 1024 x 2048 13.4 / 12.7, 440 x 832 x 1280 11.1 / 9.9, 18 of 28 by 3 to 12 %; K = 1,024 600 x 512 7.8 / 11.3, K = 1,856 1536 x 256 12.7 /
+    17.4), unless there are too few columns for it (3497 x 128 x 1536 with a GELU 10.9 / 16.2).
     Longer K and more columns than the model was held against go by ``own_tiles`` (3072 x 2048 x 8192 101 / 94)."""
     if own_tiles(m, n, k, lda, sliced, scatters, residual, gelu):
         return True
     if m <= 64 or n % 8 or not OWN_SHORT_K <= k <= MODEL_LONG_K or n > MODEL_COLUMNS or not _tile_operands(m, n, k, lda):
         return False
     us, variant = tile_form(m64(m) // 64, n, k)
-    if variant in (4, 5) and k >= LIBRARY_STEP_FROM and k % LIBRARY_K_STEP == 0 and not scatters:
+    if variant in (4, 5) and k >= LIBRARY_STEP_FROM and k % LIBRARY_K_STEP == 0 and n > LIBRARY_LEAST_COLUMNS and not scatters:
         return False
     results = 1e-6 * m64(m) * n
     library = 5.9 + 1.9e-9 * m64(m) * n * k + 0.11 * k / 64 + 0.06 * results + (4.5 + 0.5 * results if scatters else 0.16 * results if residual else 0.0)

@@ -192,7 +192,7 @@ def test_which_products_the_tile_kernel_takes():
     from burn_transformers_amd.kernels.library import own_tiles, tile_kernel_takes as takes
     # faster on tiles by a tenth and more, left to the library by own_tiles
     for m, n, k, options in ((400, 3072, 768, {"gelu": True}), (448, 1024, 1024, {"residual": True}), (600, 512, 1024, {}), (1536, 256, 1856, {"residual": True}),
-                             (768, 6144, 2048, {"scatters": True}), (2048, 4800, 1600, {"scatters": True}), (632, 3072, 576, {"gelu": True}), (6118, 1600, 6400, {})):
+                             (768, 6144, 2048, {"scatters": True}), (2048, 4800, 1600, {"scatters": True}), (632, 3072, 576, {"gelu": True}), (3497, 128, 1536, {"gelu": True}), (6118, 1600, 6400, {})):
         assert takes(m, n, k, k, **options) and not own_tiles(m, n, k, k, **options), (m, n, k)
     # long K in steps of 128 on tiles of 64 x 64, and products that large tiles do not fill well
     for m, n, k, options in ((448, 1024, 2048, {}), (440, 832, 1280, {}), (1318, 192, 1152, {"gelu": True}), (752, 512, 1792, {"residual": True}),
