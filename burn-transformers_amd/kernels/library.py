@@ -987,9 +987,12 @@ TILE_FORMS = {2: (128, 128, 5.6, 0.385, 0.65, 0.19), 3: (256, 160, 8.4, 0.71, 2.
 @functools.lru_cache(maxsize=4096)
 def tile_form(rows64, n, k, splits=1, units=256):
     """(us, variant) of the form whose busiest compute unit is done first, for a product of ``rows64`` times 64 rows (steps of one
-    class choose alike): a form of ``TILE_FORMS``, or tiles of 64 x 64 on four waves, of which up to three share a unit.  Over the 299 products
-    the fastest forms take 6,223 us, those chosen 6,270.  (Large tiles that need every unit are counted 2 us longer: in such a graph they are not, but inside
-    steps 2048 x 4096 x 1024 took 3 to 5 us less on 208 tiles than on 256 and 1959 x 3072 x 1024 2.6 less on 192.)
+    class choose alike): a form of ``TILE_FORMS``, or tiles of 64 x 64 on four waves, of which up to three share a unit.  Over 446 products of
+    72 to 4,096 rows with K of 768 to 8,192 the fastest forms take 12,053 us, those chosen 12,098.
+    Large tiles that need every unit are counted 2 us longer.  In graphs of one product they are not (12,082 us without), inside steps they are, here
+    and beside the library (us, with / without the 2): GPT-2 medium's prompts in chunks, 1959 x 3072 x 1024 on 192 tiles or on 256, 7,108 / 7,172, of 2,048 tokens
+    3,017 / 3,075; Salopel's of 2,048, 2048 x 4096 x 1024 in the library or on 256 tiles, 2,033 / 2,062; Rotutar's 2,843 / 2,863.  The other way Loselix's of 2,000 tokens
+    1,784 / 1,695 (5,120 columns on 256 tiles).  Prompts of 33 sizes in seven families took 0.9997 to 1.0015 of their time with it on three machines.
     Below twelve tiles of K, where those figures do not reach, starts and ends decide: small tiles start sooner than was fitted, their share of a
     unit brings its results as well as its K, and a unit's second large tile needs no start of a kernel.  330 products of 65 to 4,096 rows, 64 to
     8,192 columns and K of 64 to 704 take 2,721 us so, on the fastest forms 2,704, by the figures above 2,857 (us, by those / so: 125 x 2176 x 64 6.4 / 5.2,

@@ -196,7 +196,7 @@ def test_which_products_the_tile_kernel_takes():
         assert takes(m, n, k, k, **options) and not own_tiles(m, n, k, k, **options), (m, n, k)
     # long K in steps of 128 on tiles of 64 x 64, and products that large tiles do not fill well
     for m, n, k, options in ((448, 1024, 2048, {}), (440, 832, 1280, {}), (1318, 192, 1152, {"gelu": True}), (752, 512, 1792, {"residual": True}),
-                             (555, 768, 2560, {}), (2048, 128, 2048, {}), (2048, 6400, 1600, {"gelu": True}), (4096, 4096, 1024, {})):
+                             (555, 768, 2560, {}), (2048, 128, 2048, {}), (2048, 6400, 1600, {"gelu": True}), (1959, 4096, 1024, {"gelu": True}), (2048, 4096, 1024, {}), (4096, 4096, 1024, {})):
         assert not takes(m, n, k, k, **options), (m, n, k)
     # beyond what the model was held against
     for m in (65, 300, 513, 1024, 2048, 4096):
