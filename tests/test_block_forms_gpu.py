@@ -17,7 +17,7 @@ def block_forms(monkeypatch):
     monkeypatch.setitem(forms.FORMS, torch.bfloat16, BLOCK_FORMS)
 
 
-# (two to eight stages; tiles of 64 to 256 rows and 64 to 256 columns)
+# (three to eight stages; tiles of 64 to 256 rows and 64 to 256 columns)
 @pytest.mark.parametrize("m,n,tiles", [(65, 64, 1), (128, 256, 2), (130, 136, 3), (257, 264, 4), (300, 129, 5), (70, 514, 7), (258, 104, 9), (513, 328, 24)])
 def test_epilogues(m, n, tiles):
     forms.test_epilogues_of_every_form(torch.bfloat16, m, n, tiles)
@@ -26,6 +26,30 @@ def test_epilogues(m, n, tiles):
 @pytest.mark.parametrize("heads,kv_heads,hd", [(4, 4, 64), (3, 1, 128), (4, 2, 32), (5, 5, 48), (2, 2, 80), (3, 3, 16)])
 def test_scattered(heads, kv_heads, hd):
     forms.test_scattered_keys_and_values(torch.bfloat16, heads, kv_heads, hd)
+
+
+# every activation; no bias, a bias and an output that are not aligned to 16 bytes, rows apart by no whole 16 bytes: whole rows or single values, the same numbers
+@pytest.mark.parametrize("m,n", [(130, 328), (257, 104)])
+@pytest.mark.parametrize("activation", ["gelu_tanh", "gelu_erf", "squared_relu", None])
+def test_activations_and_places(m, n, activation, k=192):
+    a, w, bias, want = forms.operands(m, n, k, torch.bfloat16, n)
+    function = {"gelu_tanh": lambda x: torch.nn.functional.gelu(x, approximate="tanh"), "gelu_erf": torch.nn.functional.gelu,
+                "squared_relu": lambda x: torch.relu(x) ** 2, None: lambda x: x}[activation]
+    for form in BLOCK_FORMS:
+        shifted = torch.empty(n + 1, device=forms.DEV)[1:]
+        shifted.copy_(bias)
+        got = {}
+        for given in (None, bias.to(forms.DEV), shifted):
+            exact = function(want + (bias.double() if given is not None else 0.0))
+            for first, pitch in ((0, n), (1, n), (0, n + 3), (4, n + 8)):
+                room = torch.full((first + m * pitch + 8,), float("nan"), dtype=torch.bfloat16, device=forms.DEV)
+                out = room[first:first + m * pitch].view(m, pitch)[:, :n]
+                K.gemm(a.to(forms.DEV), w.to(forms.DEV), K.epilogue_store(out, given) if activation is None else K.epilogue_act(out, activation, given), impl="tile",
+                       variant=form)
+                # (the output's rounding)
+                assert float((out.double().cpu() - exact).abs().max() / exact.abs().max()) < 2.0 ** -8, (form, first, pitch)
+                assert int(torch.isnan(room).sum()) == room.numel() - m * n, (form, first, pitch)
+                assert torch.equal(out, got.setdefault(given is None, out.clone())), (form, first, pitch)
 
 
 # the residual stream, sixteen rows at a time: rows and columns that end inside a wave's, beside what is not the product's

@@ -119,7 +119,8 @@ def test_blocks_of_tokens_in_spans(heads, dim, vdim, lengths, strong):
     y = torch.full((total, inner + 2), float("nan"), device=DEV)
     K.keyed_scan(on[:, :qk], None, on[:, 2 * qk:2 * qk + inner], on[:, qk:2 * qk], y, held, step, heads, heads, dim, vdim, "forget",
                  g_bias=bias.to(DEV), lower=lower.to(DEV), carry=carry, blocks=blocks)
-    assert bool(torch.isnan(y[:, inner:]).all()) and bool(torch.isfinite(carry).any())          # (cut indeed)
+    assert bool(torch.isnan(y[:, inner:]).all())
+    assert bool(torch.isfinite(carry).any()) and bool(torch.isfinite(blocks).any())             # (cut indeed, and in blocks)
     r, q = rows.double(), rows[:, :qk].double()
     decay = (lower.double() + (1.0 - lower.double()) * torch.sigmoid(r[:, qk:2 * qk] + bias.double())).view(-1, heads, dim)
     q, v, at, want, got = (q * torch.sigmoid(q)).view(-1, heads, dim), r[:, 2 * qk:2 * qk + inner].view(-1, heads, vdim), 0, [], state_rows(held, heads, dim, vdim).cpu()
@@ -188,6 +189,36 @@ def test_a_token_that_is_not_finite_spoils_no_earlier_one(form, where, value, to
     assert bool(torch.isfinite(blocks).all()) == (where == "g" and value == "inf")
     kept = torch.isfinite(walk)
     assert rel_err(blocks[kept], walk[kept].double()) < 1e-5
+
+
+# the same where the sequence is cut into spans: a token of the first span, of one between, at a span's end and of the last; the walk token by token is whole
+@pytest.mark.parametrize("where,value", [("v", "inf"), ("v", "-inf"), ("v", "nan"), ("q", "inf"), ("q", "nan"), ("g", "nan"), ("g", "inf"), ("g", "-inf")])
+@pytest.mark.parametrize("token", [5, 250, 255, 699])
+def test_a_token_that_is_not_finite_in_a_cut_sequence(where, value, token):
+    gen = torch.Generator().manual_seed(9)
+    heads, dim, vdim, lengths = 4, 128, 64, [700, 650]
+    qk, inner, total = heads * dim, heads * vdim, sum(lengths)
+    bias, lower = torch.randn(qk, generator=gen).to(DEV), (torch.rand(qk, generator=gen) * 0.9).to(DEV)
+    rows = torch.randn(total, 2 * qk + inner, generator=gen)
+    spoiled = rows.clone()
+    spoiled[token, {"q": 3, "g": qk + 3, "v": 2 * qk + 3}[where]] = float(value)
+    step, results = make_step(torch.float32, lengths), {}
+    for name, source, blocked in (("clean", rows, True), ("spans", spoiled, True), ("walk", spoiled, False)):
+        on, state = source.to(DEV), torch.zeros(len(lengths), qk * vdim, device=DEV)
+        y = torch.full((total, inner), -7.0, device=DEV)
+        blocks, carry = (K.scan_blocks(step, heads, dim, vdim).fill_(float("nan")), K.scan_carry(step, qk * vdim, qk).fill_(float("nan"))) if blocked else (None, None)
+        K.keyed_scan(on[:, :qk], None, on[:, 2 * qk:], on[:, qk:2 * qk], y, state, step, heads, heads, dim, vdim, "forget", g_bias=bias, lower=lower, carry=carry,
+                     blocks=blocks)
+        assert not blocked or (bool(torch.isfinite(blocks).any()) and bool(torch.isfinite(carry).any()))
+        results[name] = (y.cpu(), state.cpu())
+    (clean, _), (spans, state), (walk, walked) = results["clean"], results["spans"], results["walk"]
+    # (a block with such a token sums in another order: a few roundings of 32 bits)
+    assert rel_err(spans[:token], clean[:token].double()) < 2e-6
+    assert torch.equal(spans[lengths[0]:], clean[lengths[0]:])
+    assert torch.equal(torch.isfinite(spans), torch.isfinite(walk)) and torch.equal(torch.isfinite(state), torch.isfinite(walked))
+    assert bool(torch.isfinite(spans).all()) == (where == "g" and value != "nan")
+    kept = torch.isfinite(walk)
+    assert rel_err(spans[kept], walk[kept].double()) < 1e-5
 
 
 @pytest.mark.parametrize("heads,groups,vdim,state,lengths,strong", [

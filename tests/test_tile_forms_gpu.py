@@ -18,8 +18,8 @@ def operands(m, n, k, dtype, seed):
     return a, w, bias, a.double() @ w.double().t()
 
 
-# one to seven tiles of K (forms have two to four stages) and so many that 64 x 64 takes eight and 64 x 128 six, whole and in slices; rows and columns on both sides of whole tiles; columns that are no
-# multiple of eight or four, which leave the epilogue's whole rows for single values
+# one to seven tiles of K (forms have three to eight stages) and so many that 64 x 64 takes eight, whole and in slices; rows and columns on both sides of whole tiles;
+# columns that are no multiple of eight or four, which leave the epilogue's whole rows for single values
 @pytest.mark.parametrize("m,n,tiles", [(65, 64, 1), (128, 256, 2), (130, 136, 3), (257, 260, 4), (300, 129, 5), (70, 514, 7),
                                        (70, 130, 49), (130, 200, 150)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -77,7 +77,7 @@ def test_scattered_keys_and_values(dtype, heads, kv_heads, hd, k=128):
 
 
 def test_scattered_keys_and_values_behind_a_long_k():
-    """The forms of eight and six stages."""
+    """The form of 64 x 64 with eight stages among all."""
     test_scattered_keys_and_values(torch.bfloat16, 4, 4, 64, k=49 * 64)
     test_scattered_keys_and_values(torch.bfloat16, 5, 5, 48, k=49 * 64)
 
