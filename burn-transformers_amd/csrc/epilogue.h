@@ -553,10 +553,11 @@ __device__ __forceinline__ void epilogue_blocks(const Epilogue& e, int M, int N,
                                                 unsigned char* scratch) {
   const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
   constexpr int COLUMNS = TN * 16;
-  const bool f32 = sizeof(T) == 4 || e.mode == EPI_F32 || e.mode == EPI_RESIDUAL;
+  static_assert(sizeof(T) == 2, "float products have no forms on these blocks");
+  const bool f32 = e.mode == EPI_F32 || e.mode == EPI_RESIDUAL;
   const int piece = f32 ? 4 : 8;                       // values in 16 bytes
   const bool scatters = e.mode == EPI_QKV && n0 + COLUMNS > e.n_q;
-  const bool whole = sizeof(T) == 2 && e.out_rows == 0 && N % piece == 0 && e.ldo % piece == 0 && e.split_stride % piece == 0 &&
+  const bool whole = e.out_rows == 0 && N % piece == 0 && e.ldo % piece == 0 && e.split_stride % piece == 0 &&
                      (((uintptr_t)e.out | (uintptr_t)e.bias) & 15) == 0 &&
                      (!scatters || (e.kv.head_dim % 16 == 0 && e.n_q % 16 == 0 && (((uintptr_t)e.kv.keys | (uintptr_t)e.kv.values) & 15) == 0));
   if (!whole) {                                        // (the same for the whole wave)
@@ -577,212 +578,210 @@ __device__ __forceinline__ void epilogue_blocks(const Epilogue& e, int M, int N,
     }
     return;
   }
-  if constexpr (sizeof(T) == 2) {
-    // what has to come from memory is asked for first: places of the rows' tokens, the bias, the first rows of the residual stream
-    int pos[TM], seq[TM];
-    if (scatters) {
+  // what has to come from memory is asked for first: places of the rows' tokens, the bias, the first rows of the residual stream
+  int pos[TM], seq[TM];
+  if (scatters) {
 #pragma unroll
-      for (int bm = 0; bm < TM; ++bm) {
-        const int m = m0 + bm * 16 + i16 < M ? m0 + bm * 16 + i16 : M - 1;
-        pos[bm] = e.tok_pos[m];
-        seq[bm] = e.tok_seq[m];
-      }
+    for (int bm = 0; bm < TM; ++bm) {
+      const int m = m0 + bm * 16 + i16 < M ? m0 + bm * 16 + i16 : M - 1;
+      pos[bm] = e.tok_pos[m];
+      seq[bm] = e.tok_seq[m];
     }
-    if (e.bias != nullptr && split == 0) {
-      floatx4 b[TN];
+  }
+  if (e.bias != nullptr && split == 0) {
+    floatx4 b[TN];
 #pragma unroll
-      for (int bn = 0; bn < TN; ++bn) {
-        const int n = n0 + bn * 16 + g * 4;
-        b[bn] = *reinterpret_cast<const floatx4*>(e.bias + (n < N ? n : 0));
-      }
-#pragma unroll
-      for (int bn = 0; bn < TN; ++bn)
-#pragma unroll
-        for (int bm = 0; bm < TM; ++bm) acc[bn][bm] += b[bn];
+    for (int bn = 0; bn < TN; ++bn) {
+      const int n = n0 + bn * 16 + g * 4;
+      b[bn] = *reinterpret_cast<const floatx4*>(e.bias + (n < N ? n : 0));
     }
-    if (f32) {
-      float* const first = static_cast<float*>(e.out) + (e.mode == EPI_F32 ? (int64_t)split * e.split_stride : 0) + (n0 < N ? n0 : 0);
-      if (e.mode == EPI_RESIDUAL) {
-        // Through LDS, sixteen rows at a time, so that neighbouring lanes ask for neighbouring pieces of the stream's rows.  Asked for by the
-        // lanes that hold the sums, the pieces of neighbouring lanes are of sixteen rows, and the address unit, which takes sixteen lanes at a time,
-        // had 64 requests of every load (us, so / through LDS: 2048 x 1600 x 1600 in tiles of 128 x 128 24.4 / 22.7, 1959 x 1600 x 6400 55.5 / 54.2, 3072 x 1600 x
-        // 1600 in 128 x 160 27.2 / 25.7, 2048 x 1024 x 1024 in 128 x 64 12.9 / 12.1).  Stores, which nothing waits for, gain nothing by it, nor did 128 bytes of a
-        // row with every instruction (two neighbouring blocks' halves swapped) or the stream asked for before the bias.
-        constexpr int PITCH = COLUMNS * 4 + 16;
-        floatx4 old[2][TN];
-        auto at = [&](int t, int& r) {                 // the column of a lane's t-th piece of sixteen rows; its row in r
-          const int i = lane + 64 * t;
-          r = i / (4 * TN);
-          return 4 * (i - r * (4 * TN));
-        };
-        auto ask = [&](int bm) {
 #pragma unroll
-          for (int t = 0; t < TN; ++t) {
-            int r;
-            const int c = at(t, r), m = m0 + bm * 16 + r;
-            old[bm & 1][t] = *reinterpret_cast<const floatx4*>(first + (int64_t)(m < M ? m : M - 1) * e.ldo + (n0 + c < N ? c : 0));
-          }
-        };
-        ask(0);
+    for (int bn = 0; bn < TN; ++bn)
 #pragma unroll
-        for (int bm = 0; bm < TM; ++bm) {
-          if (bm + 1 < TM) ask(bm + 1);
-#pragma unroll
-          for (int bn = 0; bn < TN; ++bn) *reinterpret_cast<floatx4*>(scratch + i16 * PITCH + (bn * 16 + g * 4) * 4) = acc[bn][bm];
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's accesses of LDS are served in order)
-#pragma unroll
-          for (int t = 0; t < TN; ++t) {
-            int r;
-            const int c = at(t, r), m = m0 + bm * 16 + r;
-            const floatx4 sum = *reinterpret_cast<const floatx4*>(scratch + r * PITCH + c * 4) + old[bm & 1][t];
-            if (m < M && n0 + c < N) *reinterpret_cast<floatx4*>(first + (int64_t)m * e.ldo + c) = sum;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        }
-        return;
-      }
-#pragma unroll
-      for (int bm = 0; bm < TM; ++bm) {
-        const int m = m0 + bm * 16 + i16;
-        if (m >= M) continue;
-#pragma unroll
-        for (int bn = 0; bn < TN; ++bn) {
-          const int c = bn * 16 + g * 4;
-          if (n0 + c < N) *reinterpret_cast<floatx4*>(first + (int64_t)m * e.ldo + c) = acc[bn][bm];
-        }
-      }
-      return;
-    }
-    if (e.mode == EPI_ACT) {                           // (one choice for all values)
-      auto all = [&](auto act) {
-#pragma unroll
-        for (int bn = 0; bn < TN; ++bn)
-#pragma unroll
-          for (int bm = 0; bm < TM; ++bm)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[bn][bm][r] = activate_as<T, decltype(act)::value>(acc[bn][bm][r]);
+      for (int bm = 0; bm < TM; ++bm) acc[bn][bm] += b[bn];
+  }
+  if (f32) {
+    float* const first = static_cast<float*>(e.out) + (e.mode == EPI_F32 ? (int64_t)split * e.split_stride : 0) + (n0 < N ? n0 : 0);
+    if (e.mode == EPI_RESIDUAL) {
+      // Through LDS, sixteen rows at a time, so that neighbouring lanes ask for neighbouring pieces of the stream's rows.  Asked for by the
+      // lanes that hold the sums, the pieces of neighbouring lanes are of sixteen rows, and the address unit, which takes sixteen lanes at a time,
+      // had 64 requests of every load (us, so / through LDS: 2048 x 1600 x 1600 in tiles of 128 x 128 24.4 / 22.7, 1959 x 1600 x 6400 55.5 / 54.2, 3072 x 1600 x
+      // 1600 in 128 x 160 27.2 / 25.7, 2048 x 1024 x 1024 in 128 x 64 12.9 / 12.1).  Stores, which nothing waits for, gain nothing by it, nor did 128 bytes of a
+      // row with every instruction (two neighbouring blocks' halves swapped) or the stream asked for before the bias.
+      constexpr int PITCH = COLUMNS * 4 + 16;
+      floatx4 old[2][TN];
+      auto at = [&](int t, int& r) {                 // the column of a lane's t-th piece of sixteen rows; its row in r
+        const int i = lane + 64 * t;
+        r = i / (4 * TN);
+        return 4 * (i - r * (4 * TN));
       };
-      if (e.act == ACT_GELU_TANH) all(Constant<ACT_GELU_TANH>());
-      else if (e.act == ACT_SQUARED_RELU) all(Constant<ACT_SQUARED_RELU>());
-      else all(Constant<ACT_GELU_ERF>());
-    }
-    typedef __attribute__((__vector_size__(8))) int int2v;
-    auto packed = [&](floatx4 v) {
-      const bf16x4 p = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
-      return __builtin_bit_cast(int2v, p);
-    };
-    if (!scatters) {
-      T* const out = static_cast<T*>(e.out) + n0;
+      auto ask = [&](int bm) {
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+          int r;
+          const int c = at(t, r), m = m0 + bm * 16 + r;
+          old[bm & 1][t] = *reinterpret_cast<const floatx4*>(first + (int64_t)(m < M ? m : M - 1) * e.ldo + (n0 + c < N ? c : 0));
+        }
+      };
+      ask(0);
 #pragma unroll
       for (int bm = 0; bm < TM; ++bm) {
-        const int m = m0 + bm * 16 + i16;
-        T* const row = out + (int64_t)m * e.ldo;
+        if (bm + 1 < TM) ask(bm + 1);
 #pragma unroll
-        for (int bn = 0; bn < TN; bn += 2) {
-          if (bn + 1 < TN) {
-            const int c = (bn + (g & 1)) * 16 + 8 * (g >> 1);
-            const int4v v = neighbours_joined(packed(acc[bn][bm]), packed(acc[bn + 1 < TN ? bn + 1 : bn][bm]));
-            if (m < M && n0 + c < N) *reinterpret_cast<int4v*>(row + c) = v;
-          } else {
-            const int c = bn * 16 + 4 * g;
-            if (m < M && n0 + c < N) *reinterpret_cast<int2v*>(row + c) = packed(acc[bn][bm]);
-          }
+        for (int bn = 0; bn < TN; ++bn) *reinterpret_cast<floatx4*>(scratch + i16 * PITCH + (bn * 16 + g * 4) * 4) = acc[bn][bm];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's accesses of LDS are served in order)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+          int r;
+          const int c = at(t, r), m = m0 + bm * 16 + r;
+          const floatx4 sum = *reinterpret_cast<const floatx4*>(scratch + r * PITCH + c * 4) + old[bm & 1][t];
+          if (m < M && n0 + c < N) *reinterpret_cast<floatx4*>(first + (int64_t)m * e.ldo + c) = sum;
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
       return;
     }
-    // An element's place is what its row gives (of queries, keys and values) and what its block of columns gives, which is the same for
-    // the whole wave: both worked out here, once.  (A head's number and channel divided out at every store: 2048 x 4800 x 1600 38.4 us,
-    // so 32.7.)
-    const int hd = e.kv.head_dim;
-    int64_t key_row[TM], value_row[TM];
-    uint64_t leads = 0, follows = 0;                   // rows whose position and the three behind it lie interleaved, all of them this wave's
-    auto before = [&](const int (&of)[TM], int bm) {   // of the row before (of the wave's first row: not used)
-      const int here = lane_moved<0x121>(of[bm]), last = lane_moved<0x121>(of[bm > 0 ? bm - 1 : 0]);     // (row_ror:1)
-      return i16 == 0 ? last : here;
-    };
-#pragma unroll
-    for (int bm = 0; bm < TM; ++bm) {
-      const bool here = m0 + bm * 16 + i16 < M;
-      const int seq_before = before(seq, bm), pos_before = before(pos, bm);      // (by all lanes: one that is switched off passes nothing on)
-      leads |= (__ballot(here && pos[bm] % 4 == 0) & 0xffff) << (16 * bm);
-      follows |= (__ballot(here && seq[bm] == seq_before && pos[bm] == pos_before + 1) & 0xffff) << (16 * bm);
-    }
-    leads &= follows >> 1 & follows >> 2 & follows >> 3;
-#pragma unroll
-    for (int bm = 0; bm < TM; ++bm) {
-      const int64_t plane = (int64_t)e.kv.blocks[(int64_t)seq[bm] * e.kv.max_blocks + pos[bm] / BT_KV_BLOCK] * e.kv.block_stride;
-      key_row[bm] = plane + key_offset(hd, pos[bm], 0);
-      value_row[bm] = plane + value_offset(hd, pos[bm], 0);
-    }
-    const uint64_t together = leads | leads << 1 | leads << 2 | leads << 3;
-    int64_t* const value_rows = reinterpret_cast<int64_t*>(scratch);
-    bf16_t* const turned = reinterpret_cast<bf16_t*>(scratch + TM * 16 * 8);
-    if (n0 + COLUMNS > e.n_q + e.n_kv && g == 0) {
-#pragma unroll
-      for (int bm = 0; bm < TM; ++bm) value_rows[bm * 16 + i16] = value_row[bm];
-    }
-    int64_t column[TN];                                // of queries: the column; of keys and values: the head's plane and the channel (of values times 4)
-    int kind[TN];                                      // 0 queries, 1 keys, 2 values, 3 beyond the columns
-    {
-      const int first = n0 - e.n_q;                    // (below zero: so many columns of queries come first)
-      int k = first < 0 ? 0 : first >= e.n_kv ? first - e.n_kv : first;
-      int head = k / hd, channel = k - head * hd;
-#pragma unroll
-      for (int bn = 0; bn < TN; ++bn) {
-        const int n = n0 + bn * 16;
-        kind[bn] = n < e.n_q ? 0 : n < e.n_q + e.n_kv ? 1 : n < N ? 2 : 3;
-        if (n == e.n_q || n == e.n_q + e.n_kv) head = channel = 0;
-        column[bn] = kind[bn] == 0 ? n : head * e.kv.head_stride + (kind[bn] == 1 ? channel : 4 * channel);
-        if (n >= e.n_q) {
-          channel += 16;
-          if (channel == hd) { channel = 0; ++head; }
-        }
-      }
-    }
-    T *const out = static_cast<T*>(e.out), *const keys = static_cast<T*>(e.kv.keys), *const values = static_cast<T*>(e.kv.values);
 #pragma unroll
     for (int bm = 0; bm < TM; ++bm) {
       const int m = m0 + bm * 16 + i16;
-      T *const out_row = out + (int64_t)m * e.ldo, *const keys_row = keys + key_row[bm];
+      if (m >= M) continue;
+#pragma unroll
+      for (int bn = 0; bn < TN; ++bn) {
+        const int c = bn * 16 + g * 4;
+        if (n0 + c < N) *reinterpret_cast<floatx4*>(first + (int64_t)m * e.ldo + c) = acc[bn][bm];
+      }
+    }
+    return;
+  }
+  if (e.mode == EPI_ACT) {                           // (one choice for all values)
+    auto all = [&](auto act) {
+#pragma unroll
+      for (int bn = 0; bn < TN; ++bn)
+#pragma unroll
+        for (int bm = 0; bm < TM; ++bm)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[bn][bm][r] = activate_as<T, decltype(act)::value>(acc[bn][bm][r]);
+    };
+    if (e.act == ACT_GELU_TANH) all(Constant<ACT_GELU_TANH>());
+    else if (e.act == ACT_SQUARED_RELU) all(Constant<ACT_SQUARED_RELU>());
+    else all(Constant<ACT_GELU_ERF>());
+  }
+  typedef __attribute__((__vector_size__(8))) int int2v;
+  auto packed = [&](floatx4 v) {
+    const bf16x4 p = {(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+    return __builtin_bit_cast(int2v, p);
+  };
+  if (!scatters) {
+    T* const out = static_cast<T*>(e.out) + n0;
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm) {
+      const int m = m0 + bm * 16 + i16;
+      T* const row = out + (int64_t)m * e.ldo;
 #pragma unroll
       for (int bn = 0; bn < TN; bn += 2) {
-        const int next = bn + 1 < TN ? bn + 1 : bn;
-        if (next > bn && kind[next] < 2) {             // (the kinds come in order)
-          const int4v v = neighbours_joined(packed(acc[bn][bm]), packed(acc[next][bm]));
-          const bool second = g & 1, is_key = second ? kind[next] == 1 : kind[bn] == 1;
-          if (m < M) *reinterpret_cast<int4v*>((is_key ? keys_row : out_row) + (second ? column[next] : column[bn]) + 8 * (g >> 1)) = v;
-          continue;
+        if (bn + 1 < TN) {
+          const int c = (bn + (g & 1)) * 16 + 8 * (g >> 1);
+          const int4v v = neighbours_joined(packed(acc[bn][bm]), packed(acc[bn + 1 < TN ? bn + 1 : bn][bm]));
+          if (m < M && n0 + c < N) *reinterpret_cast<int4v*>(row + c) = v;
+        } else {
+          const int c = bn * 16 + 4 * g;
+          if (m < M && n0 + c < N) *reinterpret_cast<int2v*>(row + c) = packed(acc[bn][bm]);
         }
+      }
+    }
+    return;
+  }
+  // An element's place is what its row gives (of queries, keys and values) and what its block of columns gives, which is the same for
+  // the whole wave: both worked out here, once.  (A head's number and channel divided out at every store: 2048 x 4800 x 1600 38.4 us,
+  // so 32.7.)
+  const int hd = e.kv.head_dim;
+  int64_t key_row[TM], value_row[TM];
+  uint64_t leads = 0, follows = 0;                   // rows whose position and the three behind it lie interleaved, all of them this wave's
+  auto before = [&](const int (&of)[TM], int bm) {   // of the row before (of the wave's first row: not used)
+    const int here = lane_moved<0x121>(of[bm]), last = lane_moved<0x121>(of[bm > 0 ? bm - 1 : 0]);     // (row_ror:1)
+    return i16 == 0 ? last : here;
+  };
 #pragma unroll
-        for (int b = bn; b <= next; ++b)
-          if (kind[b] < 2 && m < M) *reinterpret_cast<int2v*>((kind[b] == 1 ? keys_row : out_row) + column[b] + 4 * g) = packed(acc[b][bm]);
+  for (int bm = 0; bm < TM; ++bm) {
+    const bool here = m0 + bm * 16 + i16 < M;
+    const int seq_before = before(seq, bm), pos_before = before(pos, bm);      // (by all lanes: one that is switched off passes nothing on)
+    leads |= (__ballot(here && pos[bm] % 4 == 0) & 0xffff) << (16 * bm);
+    follows |= (__ballot(here && seq[bm] == seq_before && pos[bm] == pos_before + 1) & 0xffff) << (16 * bm);
+  }
+  leads &= follows >> 1 & follows >> 2 & follows >> 3;
+#pragma unroll
+  for (int bm = 0; bm < TM; ++bm) {
+    const int64_t plane = (int64_t)e.kv.blocks[(int64_t)seq[bm] * e.kv.max_blocks + pos[bm] / BT_KV_BLOCK] * e.kv.block_stride;
+    key_row[bm] = plane + key_offset(hd, pos[bm], 0);
+    value_row[bm] = plane + value_offset(hd, pos[bm], 0);
+  }
+  const uint64_t together = leads | leads << 1 | leads << 2 | leads << 3;
+  int64_t* const value_rows = reinterpret_cast<int64_t*>(scratch);
+  bf16_t* const turned = reinterpret_cast<bf16_t*>(scratch + TM * 16 * 8);
+  if (n0 + COLUMNS > e.n_q + e.n_kv && g == 0) {
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm) value_rows[bm * 16 + i16] = value_row[bm];
+  }
+  int64_t column[TN];                                // of queries: the column; of keys and values: the head's plane and the channel (of values times 4)
+  int kind[TN];                                      // 0 queries, 1 keys, 2 values, 3 beyond the columns
+  {
+    const int first = n0 - e.n_q;                    // (below zero: so many columns of queries come first)
+    int k = first < 0 ? 0 : first >= e.n_kv ? first - e.n_kv : first;
+    int head = k / hd, channel = k - head * hd;
+#pragma unroll
+    for (int bn = 0; bn < TN; ++bn) {
+      const int n = n0 + bn * 16;
+      kind[bn] = n < e.n_q ? 0 : n < e.n_q + e.n_kv ? 1 : n < N ? 2 : 3;
+      if (n == e.n_q || n == e.n_q + e.n_kv) head = channel = 0;
+      column[bn] = kind[bn] == 0 ? n : head * e.kv.head_stride + (kind[bn] == 1 ? channel : 4 * channel);
+      if (n >= e.n_q) {
+        channel += 16;
+        if (channel == hd) { channel = 0; ++head; }
+      }
+    }
+  }
+  T *const out = static_cast<T*>(e.out), *const keys = static_cast<T*>(e.kv.keys), *const values = static_cast<T*>(e.kv.values);
+#pragma unroll
+  for (int bm = 0; bm < TM; ++bm) {
+    const int m = m0 + bm * 16 + i16;
+    T *const out_row = out + (int64_t)m * e.ldo, *const keys_row = keys + key_row[bm];
+#pragma unroll
+    for (int bn = 0; bn < TN; bn += 2) {
+      const int next = bn + 1 < TN ? bn + 1 : bn;
+      if (next > bn && kind[next] < 2) {             // (the kinds come in order)
+        const int4v v = neighbours_joined(packed(acc[bn][bm]), packed(acc[next][bm]));
+        const bool second = g & 1, is_key = second ? kind[next] == 1 : kind[bn] == 1;
+        if (m < M) *reinterpret_cast<int4v*>((is_key ? keys_row : out_row) + (second ? column[next] : column[bn]) + 8 * (g >> 1)) = v;
+        continue;
+      }
+#pragma unroll
+      for (int b = bn; b <= next; ++b)
+        if (kind[b] < 2 && m < M) *reinterpret_cast<int2v*>((kind[b] == 1 ? keys_row : out_row) + column[b] + 4 * g) = packed(acc[b][bm]);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < TN; ++b) {
+    if (kind[b] != 2) continue;
+#pragma unroll
+    for (int bm = 0; bm < TM; ++bm) *reinterpret_cast<int2v*>(turned + (bm * 16 + i16) * 16 + 4 * g) = packed(acc[b][bm]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (a wave's accesses of LDS are served in order)
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {                   // of every four rows one leads at most; a lane takes a channel
+      const int window = 4 * t + g, lead = (int)(leads >> (4 * window)) & 15;
+      if (lead) {
+        const int r = 4 * window + __builtin_ctz(lead);
+        const bf16_t* const from = turned + r * 16 + i16;
+        const bf16x4 four = {from[0], from[16], from[32], from[48]};
+        *reinterpret_cast<bf16x4*>(values + value_rows[r] + column[b] + 4 * i16) = four;
       }
     }
 #pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      if (kind[b] != 2) continue;
+    for (int bm = 0; bm < TM; ++bm)
+      if (m0 + bm * 16 + i16 < M && !(together >> (16 * bm + i16) & 1)) {
+        T* const dst = values + value_row[bm] + column[b] + 16 * g;
 #pragma unroll
-      for (int bm = 0; bm < TM; ++bm) *reinterpret_cast<int2v*>(turned + (bm * 16 + i16) * 16 + 4 * g) = packed(acc[b][bm]);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (a wave's accesses of LDS are served in order)
-#pragma unroll
-      for (int t = 0; t < TM; ++t) {                   // of every four rows one leads at most; a lane takes a channel
-        const int window = 4 * t + g, lead = (int)(leads >> (4 * window)) & 15;
-        if (lead) {
-          const int r = 4 * window + __builtin_ctz(lead);
-          const bf16_t* const from = turned + r * 16 + i16;
-          const bf16x4 four = {from[0], from[16], from[32], from[48]};
-          *reinterpret_cast<bf16x4*>(values + value_rows[r] + column[b] + 4 * i16) = four;
-        }
+        for (int r = 0; r < 4; ++r) dst[4 * r] = from_float<T>(acc[b][bm][r]);
       }
-#pragma unroll
-      for (int bm = 0; bm < TM; ++bm)
-        if (m0 + bm * 16 + i16 < M && !(together >> (16 * bm + i16) & 1)) {
-          T* const dst = values + value_row[bm] + column[b] + 16 * g;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) dst[4 * r] = from_float<T>(acc[b][bm][r]);
-        }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
 }

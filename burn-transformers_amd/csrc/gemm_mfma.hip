@@ -906,9 +906,9 @@ static int launch_form(hipStream_t s, int variant, const bf16_t* a, int64_t lda,
     case 5:
       if (alone) return launch_pipe<64, 64, 2, 2, 8>(s, a, lda, w, M, N, K, epi, splits);
       return launch_pipe<64, 64, 2, 2, 4>(s, a, lda, w, M, N, K, epi, splits);
-    case 6: return launch_blocks<64, 128, 2, 4, 8, 5>(s, a, lda, w, M, N, K, epi, splits);
     case 7: return launch_blocks<128, 256, 2, 4, 4, 3>(s, a, lda, w, M, N, K, epi, splits);
     case 8: return launch_blocks<64, 96, 4, 2, 8, 6>(s, a, lda, w, M, N, K, epi, splits);
+    case 6:                                            // (64 x 128, which are nowhere the fastest, are 128 x 64)
     case 9: return launch_blocks<128, 64, 4, 2, 5, 8>(s, a, lda, w, M, N, K, epi, splits);
     case 10: return launch_blocks<128, 96, 4, 2, 5, 6>(s, a, lda, w, M, N, K, epi, splits);
     case 11: return launch_blocks<128, 160, 4, 2, 4, 4>(s, a, lda, w, M, N, K, epi, splits);
