@@ -21,8 +21,8 @@ One JSON line is printed:
   spread      milliseconds per step of the fastest, median and slowest repetition
   prefill     one step of 2 x 1,024 prompt tokens: tokens/s, ms, fraction of the MFMA peak;
               `own` is the same step with every product on this package's kernels (the default
-              hands products of many tiles to hipBLASLt, `kernels.library.own_tiles` says which, as
-              the reference hands its products to its backend's library)
+              hands products of many tiles to hipBLASLt, `kernels.library.tile_kernel_takes` says which,
+              as the reference hands its products to its backend's library)
   roofline    bytes a decode step has to read (every weight once + the live cache) / its time,
               against 8 TB/s
   points      decoded tokens per second at batch 1 and 64, at batch 8 from prompts of 896 tokens

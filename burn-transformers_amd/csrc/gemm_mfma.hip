@@ -191,10 +191,11 @@ gemm_tile_pipe_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict_
 
 // Tiles of BM x BN on BlockPipe (tile.h), which take a compute unit whole.  A tile is as large as leaves most units one: what bounds
 // it is what a unit can pull, 32 KiB under way at a time, so 256 x 160 x 64 takes 0.8 us where the matrix instructions alone need 0.72 and 128 x 128
-// x 64 0.45 where they need 0.31; around that 5 to 11 us of first loads (2), last stores (1 to 4) and launch, the epilogue
-// straight out of registers.  Measured with operands from memory (us, in brackets TilePipe's best form and the vendor's library):
-// 2048 x 4800 x 1600 with keys and values into the cache 34 (50, 47); 1295 x 3072 x 1024 likewise 16.6 (20, 24.7); 1959 x 1024 x 4096 into
-// the residual stream 27 (28, 30); 1295 x 4096 x 1024 with a GELU 20.3 (23, 23.8); 4096 x 1600 x 6400 87 (99, 95).
+// x 64 0.45 where they need 0.31 (busy for 0.51 and 0.36 of a unit's time in 2048 x 4800 x 1600 and 2048 x 1600 x 1600); around that 5 to 11 us of
+// first loads (2), last stores (1 to 4) and launch.  Measured with operands from memory (us, in brackets TilePipe's best form and the vendor's library):
+// 2048 x 4800 x 1600 with keys and values into the cache 35 (50, 47 with their copy); 1295 x 3072 x 1024 likewise 17.6 (20, 24.7); into the residual stream
+// 1959 x 1024 x 4096 27 (28, 31), 1959 x 1600 x 6400 54 (56, 61), 2048 x 1600 x 1600 22.7 (22.6, 24.3); 1295 x 4096 x 1024 with a GELU 22 (23, 25); 4096 x 1600 x
+// 6400 87 (99, 95).
 // Tried: tiles of 256 x 208 and 256 x 256 (2048 x 6400 x 1600 42 us without an epilogue, the library 37, with one 164 registers spilled); a ninth wave that
 // asks for lines some turns ahead (55.8 -> 55.7 at 2048 x 1600 x 6400: requests bound it); W packed by tiles (2 to 8 % faster, a third copy of the weights).
 template <typename T, int BM, int BN, int WM, int WN, int SA, int SW>

@@ -976,7 +976,9 @@ __global__ void __launch_bounds__(256, 2) keyed_blocks_walk_kernel(KeyedScanCall
 // to end, token by token or in spans / in blocks): forget gate, 2 heads of 16 x 16, 4,000 tokens 36 / 90, 4 of 64 x 64 68 / 106, 8 of 128 x 128
 // 246 / 167; delta rule with one decay a head, 8 heads of 128 x 128, 40 tokens and 63 single ones 33 / 54, 100 and 63 46 / 55, 500 and 63
 // 192 / 61, 1,000 and 200 375 / 149; 16 heads, 64 and 31 36 / 55; 2 heads of 16 x 16, 40 tokens 11 / 15.  With the walk as it is
-// now the forget gate in blocks, 4 heads of 64 x 64, 1,000 tokens 33 / 25; 2 of 16 x 16, 4,000 35 / 82.
+// now the forget gate in blocks, 4 heads of 64 x 64, 1,000 tokens 33 / 25; 2 of 16 x 16, 4,000 35 / 82.  (Of blocks that would be cut into spans the
+// time of whole sequences is weighed, which is more than they take: small states with long sequences stay token by token in spans, 4 heads of 64 x
+// 64, 4,000 tokens 64, where the blocks were not measured in spans.)
 static bool blocks_pay(const KeyedScanCall& c) {
   const float r = c.dim / 16, longest = c.max_count;
   const int span = keyed_span(c);

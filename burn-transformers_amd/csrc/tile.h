@@ -169,7 +169,8 @@ struct TilePipe {
 //             compiler knows: with reads in front of them it waited for those as well (lgkmcnt(0)), a trip to LDS every half
 //   loads     of the tile after the last one in LDS stand between the matrix instructions of the half behind the barrier: eight
 //             waves that ask for all theirs at once wait for the address unit (33.7 -> 32.3 us)
-//   stages    two of A and three of W in 160 KiB where three of both do not fit (46.9 -> 42.2 us)
+//   stages    A's and W's counted by themselves (256 x 256, two of A and three of W where three of both do not fit, 46.9 -> 42.2 us; the forms that
+//             are used have three to five of A and three to eight of W, eight of A for 64 rows)
 // What a compute unit has asked for and not got is 32 KiB at most, however many stages there are: 150 GB/s out of L2, 95 from the
 // memory-side cache and 65 from memory, so a tile wants 2 * BM * BN / (BM + BN) operations a byte and one round of tiles over the
 // chip (figures of the forms with the kernels).

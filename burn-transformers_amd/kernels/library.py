@@ -933,7 +933,9 @@ def deep_form_rows(m, k, lda, n, sliced=False, scatters=False):
 
 
 def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=False):
-    """Whether a bfloat16 product of more than 64 rows is the tile kernel's; the others are the vendor's library's.  By its rows
+    """Whether a bfloat16 product of more than 64 rows is the tile kernel's without weighing its forms beside the library (``tile_kernel_takes``
+    does that with the others).  The lines stand where they were drawn with tiles of 32 x 32 blocks, as the figures here were; on the forms of today the
+    tile kernel is as fast inside them as it was, or faster.  By its rows
     alone (``deep_form_rows``), or while a tile of 64 x 128 of it finds a compute unit of its own: measured (us, tile kernel /
     library) at K = 1,024 610 x 3072 9.4 / 10.4, 1024 x 2048 9.3 / 10.6, 1500 x 1024 9.1 / 9.9, with more tiles 610 x 4096 12.5 / 12.0, 768 x
     3072 12.3 / 12.0, 1500 x 2048 12.8 / 11.7; K = 1,600 450 x 4096 12.3 / 13.9, 610 x 4096 15.9 / 15.1.  With a
@@ -953,8 +955,7 @@ def own_tiles(m, n, k, lda, sliced=False, scatters=False, residual=False, gelu=F
     1600 9.3 / 12.0, 1024 x 1024 x 1024 7.4 / 9.4).  That line was drawn when every value of a lane went through the code of all activations; with one choice
     for a tile the tile kernel is the faster way beyond it too, while a tile of 64 x 128 finds a unit (400 x 3072 x 768 8.8 / 9.8, 640 rows 9.3 / 9.8, 300 x 4096 x 1024
     12.0 / 13.6, 512 rows 12.3 / 13.9, 300 x 6400 x 1600 16.8 / 19.0, 1600 x 1024 x 1024 10.2 / 11.0) and no longer with more tiles than that (768 x 3072 x 768 12.3 / 11.1, 610 x 4096 x 1024 15.4 / 15.0,
-    384 x 6400 x 1600 21.6 / 20.9, 1295 x 4096 x 1024 26.4 / 24.0).  The line stays all the same: the two add a product up in different orders, and steps of these
-    rows keep the results that they have.  A K below 512 (not measured) and columns that are no multiple of
+    384 x 6400 x 1600 21.6 / 20.9, 1295 x 4096 x 1024 26.4 / 24.0); such products are ``tile_kernel_takes``' to weigh.  A K below 512 (not measured) and columns that are no multiple of
     eight (not stored in whole rows) are the library's.  Rows count in whole tiles of 64 and 128 only: steps of one class (``engine.step.token_capacity``)
     choose alike."""
     if deep_form_rows(m, k, lda, n, sliced, scatters):
