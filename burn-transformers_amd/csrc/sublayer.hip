@@ -565,7 +565,7 @@ __global__ void __launch_bounds__(256) group_norm_kernel(GroupNormCall c) {
 // LDS, a wave a part, in one order however the row was read.  What bounds it with many rows is memory: a row's 14 bytes a column take
 // 6 us of 2,048 rows of 1,024 at the copy's rate.  Measured (us, 2 parts, one partial sum; a column a load and absent operands' places read too / quads):
 // 2,048 rows of 1,024 8.3 / 6.5, of 2,048 13.9 / 11.2; 512 of 1,024 4.5 / 3.7; 8 of 2,048 with two 4.9 / 3.8, one of 1,024 3.5 / 2.9.
-template <typename T, int KMAX, bool QUADS>
+template <typename T, int KMAX, bool QUADS, int READS>
 __global__ void __launch_bounds__(256) group_norm_small_kernel(GroupNormCall c) {
   typedef RowColumns<KMAX, QUADS> Columns;
   extern __shared__ __attribute__((aligned(16))) float row_buf[];       // [width], then [groups] reciprocal roots
@@ -639,12 +639,12 @@ __global__ void __launch_bounds__(256) group_norm_small_kernel(GroupNormCall c) 
   for (int p = wave; p < c.groups; p += waves) {
     const float* from = row_buf + p * per;
     float squares = 0.f;
-    for (int i = lane; i < per; i += 512) {   // (eight reads at a time, added up one after the other)
-      float x[8];
+    for (int i = lane; i < per; i += 64 * READS) {       // (so many reads at a time, added up one after the other)
+      float x[READS];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = i + 64 * u < per ? from[i + 64 * u] : 0.f;
+      for (int u = 0; u < READS; ++u) x[u] = i + 64 * u < per ? from[i + 64 * u] : 0.f;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) squares = fmaf(x[u], x[u], squares);
+      for (int u = 0; u < READS; ++u) squares = fmaf(x[u], x[u], squares);
     }
     squares = wave_sum(squares);
     if (lane == 0) rstd[p] = 1.0f / sqrtf(squares / (float)per + c.eps);
@@ -666,6 +666,114 @@ __global__ void __launch_bounds__(256) group_norm_small_kernel(GroupNormCall c) 
   }
 }
 
+// The same a column a load, for more rows than units hold at once of the kernel above, which takes 204 registers for 2,048 columns read so and 104 for
+// 1,024 (512 and 1,024 rows at once): the places of operands that are not there are read too (those of the scale) and the second
+// term's sums come behind the first's, in 88 and 44.  Measured (us, the one above / this one): 512 rows of 2,030 6.2 / 6.8, 700 9.6 / 8.0, 2,048 of 1,030 with
+// two terms 18.6 / 13.5; 1,024 of 1,022 5.8 / 6.2, 2,048 of 1,020 9.7 / 8.8.
+template <typename T, int KMAX>
+__global__ void __launch_bounds__(256) group_norm_lean_kernel(GroupNormCall c) {
+  extern __shared__ float row_buf[];          // [width], then [groups] reciprocal roots
+  float* rstd = row_buf + c.width;
+  const int t = blockIdx.x;
+  const bool from_stream = c.n_delta == 0;
+  const int source = from_stream && c.rows ? c.rows[t] : t;
+  float* xr = c.x + (int64_t)source * c.width;
+  float v[KMAX], w[KMAX], xv[KMAX], g[KMAX], gt[KMAX];
+  int cc[KMAX];
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int col = threadIdx.x + 256 * k;
+    cc[k] = col < c.width ? col : 0;
+  }
+  const float* bias = c.bias ? c.bias : c.gamma;           // (read in any case, used only where there is one)
+  const float* bias2 = c.bias2 ? c.bias2 : c.gamma;
+  const float* gate = c.gate ? c.gate + (int64_t)t * c.ld_gate : c.gamma;
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    g[k] = c.gamma[cc[k]];
+    xv[k] = xr[cc[k]];
+    v[k] = bias[cc[k]];
+    w[k] = bias2[cc[k]];
+    gt[k] = gate[cc[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    v[k] = c.bias ? v[k] : 0.f;
+    w[k] = c.bias2 ? w[k] : 0.f;
+  }
+  if (from_stream) {
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) v[k] = xv[k];
+  } else {
+    const float* row = c.delta + (int64_t)t * c.ldd;
+    for (int s0 = 0; s0 < c.n_delta; s0 += 4) {            // four partial sums at a time, all their loads together
+      float part[4][KMAX];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int sc = s0 + u < c.n_delta ? s0 + u : c.n_delta - 1;
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k) part[u][k] = row[sc * c.delta_stride + cc[k]];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k) v[k] += s0 + u < c.n_delta ? part[u][k] : 0.f;
+    }
+    const float* row2 = c.delta2 + (int64_t)t * c.ldd2;
+    for (int s0 = 0; s0 < c.n_delta2; s0 += 4) {
+      float part[4][KMAX];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int sc = s0 + u < c.n_delta2 ? s0 + u : c.n_delta2 - 1;
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k) part[u][k] = row2[sc * c.delta2_stride + cc[k]];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < KMAX; ++k) w[k] += s0 + u < c.n_delta2 ? part[u][k] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) {
+      v[k] *= c.scale;
+      if (c.n_delta2 > 0) v[k] = fmaf(c.scale2, w[k], v[k]);
+      if (c.gate) v[k] *= 1.0f / (1.0f + expf(-gt[k]));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int col = threadIdx.x + 256 * k;
+    if (col < c.width) row_buf[col] = v[k];
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int per = c.width / c.groups;
+  for (int part = wave; part < c.groups; part += waves) {
+    float squares = 0.f;
+    for (int i = lane; i < per; i += 64) squares = fmaf(row_buf[part * per + i], row_buf[part * per + i], squares);
+    squares = wave_sum(squares);
+    if (lane == 0) rstd[part] = 1.0f / sqrtf(squares / (float)per + c.eps);
+  }
+  __syncthreads();
+  T* cast = static_cast<T*>(c.cast);
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int col = threadIdx.x + 256 * k;
+    if (col < c.width) {
+      float y = v[k] * rstd[col / per] * g[k];
+      if (!from_stream) {
+        y *= c.mult;
+        if (c.accumulate) y += xv[k];
+        xr[col] = y;
+      }
+      if (cast) cast[(int64_t)t * c.ld_cast + col] = from_float<T>(y);
+    }
+  }
+  if (cast)
+    for (int col = c.width + threadIdx.x; col < c.cast_cols; col += blockDim.x)
+      cast[(int64_t)t * c.ld_cast + col] = from_float<T>(0.f);
+}
+
 template <typename T>
 static void launch_group_norm(hipStream_t stream, const GroupNormCall& c) {
   const size_t lds = (size_t)(c.width + c.groups) * sizeof(float);
@@ -675,14 +783,25 @@ static void launch_group_norm(hipStream_t stream, const GroupNormCall& c) {
   const bool quads = c.width / c.groups % 4 == 0 && (floats & 15) == 0 && c.ldd % 4 == 0 && c.delta_stride % 4 == 0 && c.ldd2 % 4 == 0 &&
                      c.delta2_stride % 4 == 0 && c.ld_gate % 4 == 0 &&
                      (!c.cast || (c.ld_cast % 4 == 0 && ((uintptr_t)c.cast & (4 * sizeof(T) - 1)) == 0));
-  if (c.width <= 1024 && quads)
-    hipLaunchKernelGGL((group_norm_small_kernel<T, 4, true>), grid, block, lds, stream, c);
-  else if (c.width <= 1024)
-    hipLaunchKernelGGL((group_norm_small_kernel<T, 4, false>), grid, block, lds, stream, c);
-  else if (c.width <= 2048 && quads)
-    hipLaunchKernelGGL((group_norm_small_kernel<T, 8, true>), grid, block, lds, stream, c);
+  // no more reads together than a part has (eight for each of 64 parts of 16 columns took 2,048 rows of 1,024 22.1 us, one 17.1;
+  // for 16 parts of 64 9.5 / 8.2, for 8 of 128 7.6, four 7.2)
+  const int per = c.width / c.groups;
+  auto small = [&](auto columns) {
+    constexpr int KMAX = decltype(columns)::value;
+    auto launch = [&](auto reads) {
+      constexpr int READS = decltype(reads)::value;
+      if (quads) hipLaunchKernelGGL((group_norm_small_kernel<T, KMAX, true, READS>), grid, block, lds, stream, c);
+      else hipLaunchKernelGGL((group_norm_small_kernel<T, KMAX, false, READS>), grid, block, lds, stream, c);
+    };
+    if (!quads && c.tokens > 4096 / KMAX) hipLaunchKernelGGL((group_norm_lean_kernel<T, KMAX>), grid, block, lds, stream, c);
+    else if (per <= 64) launch(Constant<1>());
+    else if (per <= 256) launch(Constant<4>());
+    else launch(Constant<8>());
+  };
+  if (c.width <= 1024)
+    small(Constant<4>());
   else if (c.width <= 2048)
-    hipLaunchKernelGGL((group_norm_small_kernel<T, 8, false>), grid, block, lds, stream, c);
+    small(Constant<8>());
   else
     hipLaunchKernelGGL(group_norm_kernel<T>, grid, block, lds, stream, c);
 }

@@ -221,6 +221,25 @@ def test_norm_in_parts_reads_rows_either_way(width, groups, n1, n2, gated, biase
         assert torch.equal(xs, results[0][0]) and torch.equal(cast, results[0][1])
 
 
+# rows that are read a column a load, few and more than the units hold at once: the same numbers; parts of up to 64, 256 and more columns, quads too
+@pytest.mark.parametrize("width,groups,few,many,n2,gated", [(1030, 5, 512, 513, 1, True), (2030, 2, 100, 530, 0, False), (1022, 2, 1024, 1025, 2, False),
+                                                            (102, 2, 64, 1100, 1, True), (1024, 64, 9, 70, 1, False), (1024, 16, 9, 70, 0, True), (2048, 8, 9, 70, 0, False)])
+def test_norm_in_parts_of_few_rows_and_many(width, groups, few, many, n2, gated):
+    gen = torch.Generator().manual_seed(width)
+    on = lambda *shape: torch.randn(*shape, generator=gen).to(DEV)
+    x, d1, d2, gate, gamma, bias = on(many, width), on(2, many, width), on(max(n2, 1), many, width), on(many, width), on(width), on(width)
+    v = 0.7 * (d1.double().sum(0) + bias.double()) + (1.3 * d2.double().sum(0) if n2 else 0.0)
+    v = v * torch.sigmoid(gate.double()) if gated else v
+    want = x.double().cpu() + 0.5 * plain.group_norm(v.cpu(), gamma.double().cpu(), groups, 1e-4)
+    results = []
+    for rows in (many, few):
+        xs, cast = x[:rows].clone(), torch.full((rows, width + 6), float("nan"), dtype=torch.bfloat16, device=DEV)
+        K.group_norm_output(xs, gamma, groups, 1e-4, d1[:, :rows], bias, 0.7, d2[:, :rows] if n2 else None, None, 1.3, gate=gate[:rows] if gated else None, mult=0.5, cast=cast)
+        results.append((xs, cast))
+    assert rel_err(results[0][0], want) < 2e-6 and float(results[0][1][:, width:].abs().max()) == 0.0
+    assert torch.equal(results[0][0][:few], results[1][0]) and torch.equal(results[0][1][:few], results[1][1])
+
+
 def test_capped_logits():
     gen = torch.Generator().manual_seed(0)
     logits = torch.randn(5, 3001, generator=gen) * 40.0
