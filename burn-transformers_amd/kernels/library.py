@@ -729,6 +729,8 @@ def epilogue_residual(x, bias=None):
 
 
 def epilogue_qkv(q_out, n_q, n_kv, kv_view, tok_seq, tok_pos, bias=None):
+    """Columns [0, ``n_q``) into ``q_out``, the next ``n_kv`` into the cache's keys and those behind into its values, each row's at its own place
+    (``tok_seq``, ``tok_pos``); rows come in any order (four neighbouring positions behind one another are the fastest)."""
     return Epilogue(mode=EPI_QKV, bias=_ptr(bias), out=q_out.data_ptr(), ldo=q_out.stride(0), n_q=n_q,
                     n_kv=n_kv, tok_seq=tok_seq.data_ptr(), tok_pos=tok_pos.data_ptr(), kv=kv_view)
 
